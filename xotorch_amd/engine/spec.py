@@ -61,6 +61,12 @@ class SpeculativeDecoder:
         raise ValueError(f"{cfg.model_id}: speculative decoding rewinds positions, which a recurrent state cannot")
     th, tk, tv = target_cfg.kv_cache_dims()
     dh, dk, dv = draft_cfg.kv_cache_dims()
+    for model in (target, draft):
+      # proposals are made one row at a time and verified several at a time: sums in
+      # the same order for either keep equal logits equal
+      for m in model.modules():
+        if hasattr(m, "few_rows"):
+          m.few_rows = False
     self.t_cache = ShardKVCache(target_cfg.n_layers, 1, th, self.max_seq, tk, dtype, device, v_dim=tv)
     self.d_cache = ShardKVCache(draft_cfg.n_layers, 1, dh, self.max_seq, dk, dtype, device, v_dim=dv)
 

@@ -61,6 +61,7 @@ class XotLinear(nn.Linear):
   identical to nn.Linear."""
 
   weight_packed: Optional[torch.Tensor]
+  few_rows = True  # up to ops.FEW_ROWS rows have kernels of their own, whose sums are in another order
 
   def __init__(self, *a, **kw):
     super().__init__(*a, **kw)
@@ -135,6 +136,8 @@ class XotLinear(nn.Linear):
           y = hip.skinny_gemm_fp8(x8, sx, wp8, self.weight_scale, 1, N, self.bias)
           sizes = list(x.shape[:-1]) + [N]
           return y.view(sizes)
+    if x.numel() <= ops.FEW_ROWS * self.in_features and self.few_rows and ops.few_rows(x, self.weight) and (self.bias is None or self.bias.dtype == torch.bfloat16):
+      return ops.rows_linear(x, self.weight, self.bias)
     if self.weight_packed is not None and x.is_cuda and x.dtype == torch.bfloat16:
       N, K = self.weight.shape
       M = x.numel() // K
@@ -227,7 +230,12 @@ class Attention(nn.Module):
   def forward(self, x, cos, sin, positions, kv, start_pos: int, is_decode: bool, seq_lens=None):
     if kv is None:
       return self._forward_nocache(x, cos, sin, positions)
-    B, S, _ = x.shape
+    qkv = self.qkv_proj(x)  # [B, S, (H+2KVH)*hd]
+    return self.o_proj(self.attend(qkv, cos, sin, positions, kv, start_pos, is_decode, seq_lens))
+
+  def attend(self, qkv, cos, sin, positions, kv, start_pos: int, is_decode: bool, seq_lens=None):
+    """What lies between the projections: qkv [B, S, (H+2KVH)*hd] -> [B, S, H*hd]."""
+    B, S, _ = qkv.shape
     cfg = self.cfg
     H, hd = cfg.n_heads, cfg.head_dim
     k_cache, v_cache = kv[0], kv[1]
@@ -235,7 +243,6 @@ class Attention(nn.Module):
     vp = kv[3] if len(kv) > 3 else None
     ksc = kv[4] if len(kv) > 4 else None  # fp8-KV mode scales
     vsc = kv[5] if len(kv) > 5 else None
-    qkv = self.qkv_proj(x)  # [B, S, (H+2KVH)*hd]
     qn = self.q_norm if cfg.qk_norm else None
     kn = self.k_norm if cfg.qk_norm else None
     ops.rope_qkv_append(qkv, cos, sin, positions, k_cache, v_cache, H, cfg.n_kv_heads, hd, kp, vp,
@@ -246,7 +253,7 @@ class Attention(nn.Module):
       out = ops.attn_decode(q, k_cache, v_cache, sl, kp, vp, k_scale=ksc, v_scale=vsc)
     else:
       out = ops.attn_prefill(q, k_cache, v_cache, start_pos, S, kp, vp)
-    return self.o_proj(out.reshape(B, S, H * hd))
+    return out.reshape(B, S, H * hd)
 
 
 class MLP(nn.Module):
@@ -477,7 +484,23 @@ class DecoderLayer(nn.Module):
     self.mlp = MoEMLP(cfg) if cfg.n_experts > 0 else MLP(cfg)
     self.eps = cfg.norm_eps
 
+  def _few_rows(self, x) -> bool:
+    """Whether all products of this layer are a few rows' (ops.few_rows)."""
+    a, m = self.self_attn, self.mlp
+    mods = (a.qkv_proj, a.o_proj, m.gate_up_proj, m.down_proj) if type(m) is MLP else ()
+    norms = (self.input_layernorm.weight, self.post_attention_layernorm.weight)
+    return (len(mods) > 0 and all(type(p) is XotLinear and p.few_rows for p in mods)
+            and ops.few_rows_normed(x, norms, *(p.weight for p in mods)))
+
   def forward(self, x, cos, sin, positions, kv, start_pos, is_decode, seq_lens=None):
+    if x.shape[0] * x.shape[1] <= ops.FEW_ROWS and kv is not None and self._few_rows(x):
+      # norms, activation and residual sums are part of the products
+      a, m = self.self_attn, self.mlp
+      qkv = ops.rows_norm_linear(x, self.input_layernorm.weight, self.eps, a.qkv_proj.weight, a.qkv_proj.bias)
+      out = a.attend(qkv, cos, sin, positions, kv, start_pos, is_decode, seq_lens)
+      h = ops.rows_add_linear(out, a.o_proj.weight, x)
+      act = ops.rows_norm_swiglu(h, self.post_attention_layernorm.weight, self.eps, m.gate_up_proj.weight)
+      return ops.rows_add_linear(act, m.down_proj.weight, h)
     attn_out = self.self_attn(
       self.input_layernorm(x), cos, sin, positions, kv, start_pos, is_decode, seq_lens
     )
@@ -488,6 +511,8 @@ class DecoderLayer(nn.Module):
 
 class ShardedModel(nn.Module):
   """The layer range [shard.start_layer .. shard.end_layer] of one model."""
+
+  few_rows = True  # XotLinear.few_rows, for a head that is the embedding
 
   def __init__(self, cfg: ModelConfig, shard: Shard):
     super().__init__()
@@ -631,6 +656,11 @@ class ShardedModel(nn.Module):
       return h
     if last_only and h.shape[1] > 1:
       h = h[:, -1:, :].contiguous()  # kernels require contiguous rows
+    head = self.head_weight()
+    if (type(self.lm_head) is XotLinear and self.lm_head.few_rows if hasattr(self, "lm_head") else self.few_rows) and (
+        ops.few_rows_normed(h, (self.norm.weight,), head)):
+      logits = ops.rows_norm_linear(h, self.norm.weight, self.norm.eps, head)
+      return logits[:, -1, :] if is_decode or last_only else logits
     h = self.norm(h)
     if hasattr(self, "lm_head"):
       logits = self.lm_head(h)  # XotLinear: packed decode kernel when prepacked

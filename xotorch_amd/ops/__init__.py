@@ -202,6 +202,57 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
   return torch.nn.functional.linear(x, weight, bias)
 
 
+# rows that the kernels of hip/rows_ops.hip take
+FEW_ROWS = 4
+_rows_ext = None
+
+
+def _rows():
+  global _rows_ext
+  if _rows_ext is None:
+    import importlib
+    _rows_ext = importlib.import_module("xotorch_amd.ops._hip_rows")
+  return _rows_ext
+
+
+def few_rows(x: torch.Tensor, *weights: torch.Tensor) -> bool:
+  """Whether the products of x with these weights ([N, K], bf16) are a few rows'
+  (hip/rows_ops.hip): inference on the GPU, up to FEW_ROWS rows, 16-byte rows."""
+  if not x.is_cuda or x.dtype != torch.bfloat16 or torch.is_grad_enabled() or not x.is_contiguous():
+    return False
+  if not 0 < x.numel() <= FEW_ROWS * x.shape[-1] or x.data_ptr() % 16 or not _use_hip(x):
+    return False
+  return all(w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[1] % 8 == 0 and w.is_contiguous()
+             and w.data_ptr() % 16 == 0 and 0 < w.shape[0] <= 1 << 26 for w in weights)
+
+
+def few_rows_normed(x: torch.Tensor, norms, *weights: torch.Tensor) -> bool:
+  """The same where rows like x are normed first, with these weights: they have to fit into LDS."""
+  D = x.shape[-1]
+  return (few_rows(x, *weights) and (x.numel() // D) * (-(-D // 512) * 1024) <= 128 * 1024
+          and all(n.is_cuda and n.dtype == torch.bfloat16 and n.is_contiguous() and n.data_ptr() % 16 == 0 for n in norms))
+
+
+def rows_linear(x, weight, bias=None):
+  return _rows().rows_linear(x, weight, bias)
+
+
+def rows_norm_linear(x, norm, eps: float, weight, bias=None, w_bias: float = 0.0):
+  """rmsnorm(x) @ weight^T + bias"""
+  return _rows().rows_norm_linear(x, norm, eps, w_bias, weight, bias)
+
+
+def rows_norm_swiglu(x, norm, eps: float, gate_up, w_bias: float = 0.0):
+  """silu(n @ gate^T) * (n @ up^T) with n = rmsnorm(x), x fp32, products as bf16"""
+  return _rows().rows_norm_swiglu(x, norm, eps, w_bias, gate_up)
+
+
+def rows_add_linear(x, weight, residual):
+  """residual + x @ weight^T: an fp32 sum if the residual is bf16, a bf16 one if it
+  is fp32 (both addends as bf16)."""
+  return _rows().rows_add_linear(x, weight, residual)
+
+
 def softmax_sample(logits, temperature: float = 0.0, top_k: int = 0, generator=None,
                    top_p: float = 0.0):
   # torch ops here are graph-capturable (argmax / exponential+argmax)

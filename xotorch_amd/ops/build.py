@@ -18,6 +18,7 @@ PKG_DIR = Path(__file__).resolve().parent
 # extension module -> its source
 EXTENSIONS = {
   "_hip_ops": PKG_DIR / "hip" / "hip_ops.hip",
+  "_hip_rows": PKG_DIR / "hip" / "rows_ops.hip",
   "_hip_mixers": PKG_DIR / "hip" / "mixer_ops.hip",
   "_hip_attn": PKG_DIR / "hip" / "attn_rows.hip",
   "_hip_rotary": PKG_DIR / "hip" / "rotary_attn.hip",
