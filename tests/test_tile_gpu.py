@@ -1,0 +1,67 @@
+"""Products by weight tiles (hip/tile_ops.hip) against 64 bits: rows at the edges of
+16, 32, 64 and 128, weight rows past a tile, k with and without a split."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(1, 8, 64), (16, 72, 320), (17, 130, 1536), (32, 2048, 2048), (33, 136, 512), (64, 3584, 3584), (65, 129, 128),
+         (128, 520, 18944), (129, 2056, 640), (256, 28680, 192)]
+
+
+def _inputs(m, N, K):
+  g = torch.Generator(device="cuda").manual_seed(m)
+  return [torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16) for s in ((m, K), (N, K), (N,))]
+
+
+@pytest.mark.parametrize("m,N,K", SIZES)
+def test_products(m, N, K):
+  """Sums of K products in fp32 are off by less than K 2^-24 of the products' sizes;
+  what is stored as bf16 by 2^-8 of itself."""
+  from xotorch_amd import ops
+  x, w, b = _inputs(m, N, K)
+  ref, terms = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t() * (K * 2.0 ** -24)
+  with torch.no_grad():
+    assert ops.tile_rows(x, w)
+    parts = ops.tile_parts(x, w)
+    assert parts.shape[1:] == ref.shape and bool(((parts.double().sum(0) - ref).abs() <= terms).all())
+    for bias in (None, b):
+      want = ref if bias is None else ref + b.double()
+      y = ops.tile_linear(x, w, bias)
+      assert bool(((y.double() - want).abs() <= terms + want.abs() * 2.0 ** -8 + 1e-30).all())
+    if N % 8 == 0:
+      (g, u), (tg, tu) = ref.chunk(2, -1), (terms + ref.abs() * 2.0 ** -8).chunk(2, -1)
+      act = torch.nn.functional.silu(g)
+      bound = 1.1 * tg * (u.abs() + tu) + act.abs() * tu + (act * u).abs() * 2.0 ** -8
+      assert bool(((ops.tile_swiglu(x, w).double() - act * u).abs() <= bound + 1e-30).all())
+
+
+@pytest.mark.parametrize("N,K", [(72, 320), (3584, 3584), (28680, 192), (520, 18944)])
+def test_rows_do_not_depend_on_their_batch(N, K):
+  from xotorch_amd import ops
+  x, w, b = _inputs(256, N, K)
+  with torch.no_grad():
+    whole = ops.tile_linear(x, w, b), ops.tile_swiglu(x, w)
+    for lo, hi in ((0, 1), (3, 19), (40, 72), (100, 164), (7, 135), (20, 200)):
+      some = x[lo:hi].contiguous()
+      assert torch.equal(ops.tile_linear(some, w, b), whole[0][lo:hi]) and torch.equal(ops.tile_swiglu(some, w), whole[1][lo:hi])
+
+
+@pytest.mark.parametrize("m,D,parts", [(1, 8, 1), (3, 2048, 4), (5, 2056, 16), (256, 8192, 3), (2, 16384, 2)])
+def test_sum_and_norm(m, D, parts):
+  from xotorch_amd import ops
+  g = torch.Generator(device="cuda").manual_seed(D)
+  p = torch.randn(parts, m, D, generator=g, device="cuda")
+  x, w = (torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16) for s in ((m, D), (D,)))
+  total = p[0]
+  for q in p[1:]:
+    total = total + q
+  f = x.float() + total.to(torch.bfloat16).float()
+  for rounded in (False, True):
+    h, n = ops.parts_add_norm(p, x, w, 1e-5, 1.0, rounded)
+    assert torch.equal(h, f.to(torch.bfloat16))
+    v = (h if rounded else f).double()
+    ref = v * torch.rsqrt(v.square().mean(-1, keepdim=True) + 1e-5) * (w.double() + 1)
+    # bf16 once, and fp32 sums of D squares
+    assert bool(((n.double() - ref).abs() <= ref.abs() * (2.0 ** -8 + D * 2.0 ** -24) + 1e-30).all())
+  assert torch.equal(ops.parts_add_norm(p, x)[0], f.to(torch.bfloat16))

@@ -138,6 +138,9 @@ class XotLinear(nn.Linear):
           return y.view(sizes)
     if x.numel() <= ops.FEW_ROWS * self.in_features and self.few_rows and ops.few_rows(x, self.weight) and (self.bias is None or self.bias.dtype == torch.bfloat16):
       return ops.rows_linear(x, self.weight, self.bias)
+    if x.numel() <= ops.TILE_ROWS * self.in_features and ops.tile_rows(x, self.weight) and (
+        ops.tile_wins(x.numel() // self.in_features, self.weight) and (self.bias is None or self.bias.dtype == torch.bfloat16)):
+      return ops.tile_linear(x, self.weight, self.bias)
     if self.weight_packed is not None and x.is_cuda and x.dtype == torch.bfloat16:
       N, K = self.weight.shape
       M = x.numel() // K
@@ -270,6 +273,20 @@ class MLP(nn.Module):
   @staticmethod
   def act(gu):
     return ops.swiglu_packed(gu)
+
+  def by_tiles(self, x) -> bool:
+    gu, dp = self.gate_up_proj, self.down_proj
+    return (type(gu) is XotLinear and type(dp) is XotLinear and gu.bias is None and dp.bias is None
+            and getattr(gu, "weight_packed_fp8", None) is None and getattr(dp, "weight_packed_fp8", None) is None
+            and gu.weight.shape[0] % 8 == 0 and ops.tile_rows(x, gu.weight, dp.weight)
+            and ops.tile_wins(x.numel() // x.shape[-1], dp.weight))
+
+  def gated(self, x):
+    """The gated activation of x (by_tiles)."""
+    gu = self.gate_up_proj
+    if ops.tile_wins(x.numel() // x.shape[-1], gu.weight):
+      return ops.tile_swiglu(x, gu.weight)
+    return self.act(gu(x))
 
   def forward(self, x):
     gu = self.gate_up_proj(x)
@@ -492,6 +509,35 @@ class DecoderLayer(nn.Module):
     return (len(mods) > 0 and all(type(p) is XotLinear and p.few_rows for p in mods)
             and ops.few_rows_normed(x, norms, *(p.weight for p in mods)))
 
+  def by_tiles(self, x) -> bool:
+    """Whether `step` takes this layer: products by weight tiles (ops.tile_rows)."""
+    a, m = self.self_attn, self.mlp
+    mods = (a.qkv_proj, a.o_proj)
+    if not all(type(p) is XotLinear and getattr(p, "weight_packed_fp8", None) is None for p in mods):
+      return False
+    rows = x.shape[0] * x.shape[1]
+    return (x.shape[-1] % 8 == 0 and x.shape[-1] <= 16384 and ops.tile_rows(x, *(p.weight for p in mods))
+            and all(ops.tile_wins(rows, p.weight) for p in mods)
+            and ops.plain_norms(self.input_layernorm.weight, self.post_attention_layernorm.weight))
+
+  def step(self, x, normed, cos, sin, positions, kv, start_pos, is_decode, seq_lens, after):
+    """The layer with sums that the next norm finishes: (stream, that norm of it).
+    `after`: the module of that norm, or None; normed: this layer's, None: not made yet."""
+    a, m = self.self_attn, self.mlp
+    if normed is None:
+      normed = self.input_layernorm(x)
+    out = a.attend(a.qkv_proj(normed), cos, sin, positions, kv, start_pos, is_decode, seq_lens)
+    post = self.post_attention_layernorm
+    x, normed = ops.parts_add_norm(ops.tile_parts(out, a.o_proj.weight), x, post.weight, post.eps)
+    if type(m) is MLP and m.by_tiles(normed):
+      parts = ops.tile_parts(m.gated(normed), m.down_proj.weight)
+    else:
+      parts = m(normed).float()
+    parts = parts.view(-1, x.numel() // x.shape[-1], x.shape[-1])
+    if after is None or not ops.plain_norms(after.weight):
+      return ops.parts_add_norm(parts, x)[0], None
+    return ops.parts_add_norm(parts, x, after.weight, after.eps, rounded=True)
+
   def forward(self, x, cos, sin, positions, kv, start_pos, is_decode, seq_lens=None):
     if x.shape[0] * x.shape[1] <= ops.FEW_ROWS and kv is not None and self._few_rows(x):
       # norms, activation and residual sums are part of the products
@@ -643,9 +689,20 @@ class ShardedModel(nn.Module):
     # per-layer activation residency for a recompute in backward
     use_ckpt = (caches is None and self.training and torch.is_grad_enabled()
                 and os.getenv("XOT_ACT_CKPT", "0") == "1")
-    for idx, lid in enumerate(self.local_layer_ids):
-      layer = self.layers[str(lid)]
+    layers = [self.layers[str(lid)] for lid in self.local_layer_ids]
+    # few enough rows for weight tiles, but not so few that the layers fuse more (ops.few_rows)
+    tiles = (caches is not None and h.is_cuda and h.shape[0] * h.shape[1] <= ops.TILE_ROWS
+             and not (h.shape[0] * h.shape[1] <= ops.FEW_ROWS and layers[0]._few_rows(h)))
+    normed = None
+    for idx, layer in enumerate(layers):
       kv = caches[idx] if caches is not None else None
+      if tiles and layer.by_tiles(h):
+        after = layers[idx + 1].input_layernorm if idx + 1 < len(layers) else None
+        if after is None and self.shard.is_last_layer and (h.shape[1] == 1 or not last_only):
+          after = self.norm
+        h, normed = layer.step(h, normed, cos, sin, positions, kv, start_pos, is_decode, seq_lens, after)
+        continue
+      normed = None
       if use_ckpt:
         h = torch.utils.checkpoint.checkpoint(
           layer, h, cos, sin, positions, kv, start_pos, is_decode, seq_lens,
@@ -656,16 +713,20 @@ class ShardedModel(nn.Module):
       return h
     if last_only and h.shape[1] > 1:
       h = h[:, -1:, :].contiguous()  # kernels require contiguous rows
+      normed = None
     head = self.head_weight()
-    if (type(self.lm_head) is XotLinear and self.lm_head.few_rows if hasattr(self, "lm_head") else self.few_rows) and (
+    own = self.lm_head if hasattr(self, "lm_head") else None
+    if normed is None and (type(own) is XotLinear and own.few_rows if own is not None else self.few_rows) and (
         ops.few_rows_normed(h, (self.norm.weight,), head)):
       logits = ops.rows_norm_linear(h, self.norm.weight, self.norm.eps, head)
       return logits[:, -1, :] if is_decode or last_only else logits
-    h = self.norm(h)
-    if hasattr(self, "lm_head"):
-      logits = self.lm_head(h)  # XotLinear: packed decode kernel when prepacked
+    h = self.norm(h) if normed is None else normed
+    if own is not None:
+      logits = own(h)  # XotLinear: packed decode kernel when prepacked
+    elif h.numel() <= ops.TILE_ROWS * h.shape[-1] and ops.tile_rows(h, head) and ops.tile_wins(h.numel() // h.shape[-1], head):
+      logits = ops.tile_linear(h, head)
     else:
-      logits = ops.linear(h, self.head_weight().to(h.dtype))
+      logits = ops.linear(h, head.to(h.dtype))
     if is_decode or last_only:
       return logits[:, -1, :]
     return logits

@@ -226,11 +226,16 @@ def few_rows(x: torch.Tensor, *weights: torch.Tensor) -> bool:
              and w.data_ptr() % 16 == 0 and 0 < w.shape[0] <= 1 << 26 for w in weights)
 
 
+def plain_norms(*norms: torch.Tensor) -> bool:
+  """Whether kernels that end or begin with a norm can read these weights."""
+  return all(n.is_cuda and n.dtype == torch.bfloat16 and n.is_contiguous() and n.data_ptr() % 16 == 0 for n in norms)
+
+
 def few_rows_normed(x: torch.Tensor, norms, *weights: torch.Tensor) -> bool:
   """The same where rows like x are normed first, with these weights: they have to fit into LDS."""
   D = x.shape[-1]
   return (few_rows(x, *weights) and (x.numel() // D) * (-(-D // 512) * 1024) <= 128 * 1024
-          and all(n.is_cuda and n.dtype == torch.bfloat16 and n.is_contiguous() and n.data_ptr() % 16 == 0 for n in norms))
+          and plain_norms(*norms))
 
 
 def rows_linear(x, weight, bias=None):
@@ -251,6 +256,57 @@ def rows_add_linear(x, weight, residual):
   """residual + x @ weight^T: an fp32 sum if the residual is bf16, a bf16 one if it
   is fp32 (both addends as bf16)."""
   return _rows().rows_add_linear(x, weight, residual)
+
+
+# rows that the kernels of hip/tile_ops.hip take
+TILE_ROWS = 256
+_tile_ext = None
+
+
+def _tile():
+  global _tile_ext
+  if _tile_ext is None:
+    import importlib
+    _tile_ext = importlib.import_module("xotorch_amd.ops._hip_tile")
+  return _tile_ext
+
+
+def tile_rows(x: torch.Tensor, *weights: torch.Tensor) -> bool:
+  """Whether the products of x with these weights ([N, K], bf16) go by weight tiles
+  (hip/tile_ops.hip): inference on the GPU, up to TILE_ROWS rows, k in steps of 64."""
+  if not x.is_cuda or x.dtype != torch.bfloat16 or torch.is_grad_enabled() or not x.is_contiguous():
+    return False
+  if not 0 < x.numel() <= TILE_ROWS * x.shape[-1] or x.data_ptr() % 16 or not _use_hip(x):
+    return False
+  return all(w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[1] % 64 == 0 and w.is_contiguous()
+             and w.data_ptr() % 16 == 0 and 0 < w.shape[0] <= 1 << 26 and 0 < w.shape[1] <= 1 << 26 for w in weights)
+
+
+def tile_wins(rows: int, weight: torch.Tensor) -> bool:
+  """Above 128 rows two blocks share a weight tile, and the library is as fast where
+  the weight rows fill the chip without a split of k: [37888, 3584] with 256 rows
+  112 us and 82, [8192, 8192] 46 and 78, [8192, 28672] 153 and 313."""
+  return rows <= 128 or _tile().tile_splits(*weight.shape) > 1
+
+
+def tile_linear(x, weight, bias=None):
+  return _tile().tile_linear(x, weight, bias)
+
+
+def tile_swiglu(x, gate_up):
+  """silu(x @ gate^T) * (x @ up^T), products as bf16"""
+  return _tile().tile_swiglu(x, gate_up)
+
+
+def tile_parts(x, weight):
+  """x @ weight^T as fp32 sums over parts of k [parts, rows, N]"""
+  return _tile().tile_parts(x, weight)
+
+
+def parts_add_norm(parts, x, norm=None, eps: float = 0.0, w_bias: float = 0.0, rounded: bool = False):
+  """(h, rmsnorm(h)) with h = x + the parts' sum as bf16; (h,) without a norm.
+  rounded: the norm reads h as bf16."""
+  return _tile().parts_add_norm(parts, x, norm, eps, w_bias, rounded)
 
 
 def softmax_sample(logits, temperature: float = 0.0, top_k: int = 0, generator=None,

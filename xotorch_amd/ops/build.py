@@ -19,6 +19,7 @@ PKG_DIR = Path(__file__).resolve().parent
 EXTENSIONS = {
   "_hip_ops": PKG_DIR / "hip" / "hip_ops.hip",
   "_hip_rows": PKG_DIR / "hip" / "rows_ops.hip",
+  "_hip_tile": PKG_DIR / "hip" / "tile_ops.hip",
   "_hip_mixers": PKG_DIR / "hip" / "mixer_ops.hip",
   "_hip_attn": PKG_DIR / "hip" / "attn_rows.hip",
   "_hip_rotary": PKG_DIR / "hip" / "rotary_attn.hip",

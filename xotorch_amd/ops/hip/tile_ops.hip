@@ -1,0 +1,422 @@
+// Products of up to 256 rows (decode batches, prompt chunks) with bf16 weights as
+// they lie in the checkpoint, [N, K] row-major, and what follows them:
+//   y = x W^T + bias; silu(x Wg^T) (x Wu^T); r + x W^T and the norm of it.
+// (The reference runs these as separate modules, general_mha.py:83-102,
+// llm_utils.py:465-500.)
+//
+// What bounds them is the weights' way from memory, for which every CU wants some
+// 48 KB on its way; library tiles leave that to few blocks. A block owns 64 or 128
+// weight rows and all rows of x (128 at most, else two blocks), and walks its part of
+// k in steps of 64 through a ring of LDS buffers that are filled by direct loads: rows of 128
+// bytes, so whole lines, the 16-byte pieces of row r permuted by r & 7 in the global
+// address, which spreads fragment reads over the banks. Where the weight rows alone
+// make too few blocks, k is split; the parts' fp32 sums are added by the kernel that
+// follows anyway (norm, activation).
+//
+// us, library beside: [3584, 18944] m 8 23 (48), m 32 23 (110), m 128 33 (99);
+// [8192, 28672] m 128 97 (199); [8192, 8192] m 128 35 (48); [4608, 3584] m 256 18 (36).
+//
+// How k is split depends on the weights' shape alone, and the order of the sums within
+// a part on nothing: a row's result does not depend on what it is batched with.
+#include "common.h"
+
+struct TileArgs {
+  const bf16_t *x, *w, *bias;
+  void* y;  // bf16 [m, N], or fp32 [splits, m, N]
+  int m, N, K, steps, splits;  // steps of 64 in all; N: output features
+};
+
+// STORE: bf16 with bias; PART: fp32 sums of a part of k; GATED: weight rows [2 N, K],
+// gate first, bf16 of the gated activation
+enum TileEnd { STORE, PART, GATED };
+
+// A value as a bf16 tensor holds it
+DEVINL float rounded(float f) {
+  const bf16_t b = f2b(f);
+  return ld(&b);
+}
+
+typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(1))) const void glb_void;
+
+// R fragments from a on and C from b on, 16 rows (2 KB) apart; waits for them
+template <int R, int C>
+DEVINL void read_frags(unsigned a, unsigned b, bf16x8* r, bf16x8* c) {
+#define RD(D, A, O) "ds_read_b128 %" #D ", %" #A " offset:" #O "\n\t"
+#define DONE "s_waitcnt lgkmcnt(0)"
+  if constexpr (R == 1 && C == 1)
+    asm volatile(RD(0, 2, 0) RD(1, 3, 0) DONE : "=&v"(r[0]), "=&v"(c[0]) : "v"(a), "v"(b));
+  else if constexpr (R == 1 && C == 2)
+    asm volatile(RD(0, 3, 0) RD(1, 4, 0) RD(2, 4, 2048) DONE : "=&v"(r[0]), "=&v"(c[0]), "=&v"(c[1]) : "v"(a), "v"(b));
+  else if constexpr (R == 2 && C == 1)
+    asm volatile(RD(0, 3, 0) RD(1, 3, 2048) RD(2, 4, 0) DONE : "=&v"(r[0]), "=&v"(r[1]), "=&v"(c[0]) : "v"(a), "v"(b));
+  else if constexpr (R == 2 && C == 2)
+    asm volatile(RD(0, 4, 0) RD(1, 4, 2048) RD(2, 5, 0) RD(3, 5, 2048) DONE
+                 : "=&v"(r[0]), "=&v"(r[1]), "=&v"(c[0]), "=&v"(c[1]) : "v"(a), "v"(b));
+  else if constexpr (R == 4 && C == 2)
+    asm volatile(RD(0, 6, 0) RD(1, 6, 2048) RD(2, 6, 4096) RD(3, 6, 6144) RD(4, 7, 0) RD(5, 7, 2048) DONE
+                 : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(c[0]), "=&v"(c[1]) : "v"(a), "v"(b));
+  else {
+    static_assert(R == 4 && C == 4, "");
+    asm volatile(RD(0, 8, 0) RD(1, 8, 2048) RD(2, 8, 4096) RD(3, 8, 6144)
+                 RD(4, 9, 0) RD(5, 9, 2048) RD(6, 9, 4096) RD(7, 9, 6144) DONE
+                 : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(c[0]), "=&v"(c[1]), "=&v"(c[2]), "=&v"(c[3])
+                 : "v"(a), "v"(b));
+  }
+#undef RD
+#undef DONE
+}
+
+template <int BN, int BM, int BUFS>
+struct TileShape {
+  static constexpr int ROWS = BN + BM, BUF = ROWS * 64;  // elements of a buffer
+  static constexpr int WL = BN / 32, XL = BM >= 32 ? BM / 32 : 1;  // loads of a wave and stage
+  static constexpr int LDS = BUFS * BUF * 2;
+  // waves along x: the weight rows are split over all four for few rows of x
+  static constexpr int WX = BM >= 64 ? 2 : 1, R = BN * WX / 64, C = BM / WX / 16;
+};
+
+template <int BN, int BM, int BUFS, int END>
+__global__ __launch_bounds__(256) void tile_kernel(TileArgs a) {
+  typedef TileShape<BN, BM, BUFS> Sh;
+  constexpr int R = Sh::R, C = Sh::C, LOADS = Sh::WL + Sh::XL;
+  extern __shared__ __attribute__((aligned(16))) bf16_t buf[];  // [BUFS][weights [BN][64], x [BM][64]]
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int col = lane & 15, quad = lane >> 4;
+  // blocks go round the eight dies: two blocks of the same weights are neighbours on one
+  const int mts = (a.m + BM - 1) / BM, tiles = (a.N + (END == GATED ? BN / 2 : BN) - 1) / (END == GATED ? BN / 2 : BN);
+  const int local = blockIdx.x >> 3, mt = local % mts, unit = (local / mts << 3) + (blockIdx.x & 7);
+  if (unit >= tiles * a.splits) return;
+  const int tile = unit % tiles, split = unit / tiles;
+  const int s0 = (int)((long long)a.steps * split / a.splits), s1 = (int)((long long)a.steps * (split + 1) / a.splits);
+  const int m0 = mt * BM;
+  const bf16_t *wsrc[Sh::WL], *xsrc[Sh::XL];
+  const int sub = lane >> 3;
+  // GATED: 16 gate rows and the same 16 up rows in turn
+  auto weight_row = [&](int r) -> size_t {
+    if (END == GATED) return (size_t)min(tile * (BN / 2) + (r >> 5) * 16 + (r & 15), a.N - 1) + ((r >> 4) & 1 ? (size_t)a.N : 0);
+    return min(tile * BN + r, a.N - 1);
+  };
+#pragma unroll
+  for (int i = 0; i < Sh::WL; ++i) {
+    const int r = (wave * Sh::WL + i) * 8 + sub;
+    wsrc[i] = a.w + weight_row(r) * a.K + ((lane & 7) ^ (r & 7)) * 8;
+  }
+#pragma unroll
+  for (int i = 0; i < Sh::XL; ++i) {
+    const int r = BM >= 32 ? (wave * Sh::XL + i) * 8 + sub : wave * 4 + (sub & 3);
+    xsrc[i] = a.x + (size_t)min(m0 + r, a.m - 1) * a.K + ((lane & 7) ^ (r & 7)) * 8;
+  }
+  auto stage = [&](int s) {
+    bf16_t* dst = buf + ((s - s0) % BUFS) * Sh::BUF;
+#pragma unroll
+    for (int i = 0; i < Sh::WL; ++i)
+      __builtin_amdgcn_global_load_lds((glb_void*)(wsrc[i] + s * 64), (lds_void*)(dst + (wave * Sh::WL + i) * 512), 16, 0, 2);
+#pragma unroll
+    for (int i = 0; i < Sh::XL; ++i) {
+      bf16_t* to = dst + BN * 64 + (BM >= 32 ? (wave * Sh::XL + i) * 512 : wave * 256);
+      if (BM >= 32 || lane < 32)
+        __builtin_amdgcn_global_load_lds((glb_void*)(xsrc[i] + s * 64), (lds_void*)to, 16, 0, 0);
+    }
+  };
+  floatx4 acc[R][C];
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int j = 0; j < C; ++j) acc[i][j] = (floatx4)(0.f);
+#pragma unroll
+  for (int i = 0; i < BUFS - 1; ++i)
+    if (s0 + i < s1) stage(s0 + i);
+  const int wr = Sh::WX == 2 ? (wave >> 1) * (BN / 2) : wave * (BN / 4), wx = Sh::WX == 2 ? (wave & 1) * (BM / 2) : 0;
+  // this lane's first fragments, as LDS byte addresses within a buffer
+  const unsigned base = (unsigned)(size_t)(lds_void*)buf;
+  const unsigned wl = base + (wr + col) * 128, xl = base + (BN + wx + col) * 128;
+  const unsigned place[2] = {(unsigned)((quad ^ (col & 7)) * 16), (unsigned)(((4 + quad) ^ (col & 7)) * 16)};
+  for (int s = s0; s < s1; ++s) {
+    // this step is in LDS, up to BUFS - 2 later ones are on their way; the buffer of
+    // the step before is free
+    const int left = min(BUFS - 2, s1 - 1 - s);
+    if (left >= 2) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(2 * LOADS) : "memory");
+    else if (left == 1) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(LOADS) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    if (s + BUFS - 1 < s1) stage(s + BUFS - 1);
+    const unsigned at = (unsigned)((s - s0) % BUFS) * (Sh::BUF * 2);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      bf16x8 wf[R], xf[C];
+      read_frags<R, C>(wl + at + place[h], xl + at + place[h], wf, xf);
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int j = 0; j < C; ++j) acc[i][j] = mma(wf[i], xf[j], acc[i][j]);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < C; ++j) {
+    const int m = m0 + wx + j * 16 + col;
+    if (m >= a.m) continue;
+    if (END == GATED) {
+#pragma unroll
+      for (int i = 0; i + 1 < R; i += 2) {
+        const int n = tile * (BN / 2) + (wr + i * 16) / 2 + quad * 4;
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = siluf(rounded(acc[i][j][r])) * rounded(acc[i + 1][j][r]);
+        bf16_t* dst = (bf16_t*)a.y + (size_t)m * a.N + n;
+        if (n + 3 < a.N && (a.N & 3) == 0) st4(dst, v);
+        else
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (n + r < a.N) st(dst + r, v[r]);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        const int n = tile * BN + wr + i * 16 + quad * 4;
+        const bool whole = n + 3 < a.N && (a.N & 3) == 0;
+        if (END == PART) {
+          float* dst = (float*)a.y + ((size_t)split * a.m + m) * a.N + n;
+          if (whole) *(floatx4*)dst = acc[i][j];
+          else
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (n + r < a.N) dst[r] = acc[i][j][r];
+        } else {
+          float v[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = acc[i][j][r] + (a.bias && n + r < a.N ? ld(a.bias + n + r) : 0.f);
+          bf16_t* dst = (bf16_t*)a.y + (size_t)m * a.N + n;
+          if (whole) st4(dst, v);
+          else
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (n + r < a.N) st(dst + r, v[r]);
+        }
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// what follows a product whose k was split: the parts' sums, in order
+// ---------------------------------------------------------------------------
+
+DEVINL floatx4 sum_parts(const float* p, size_t at, size_t stride, int splits) {
+  floatx4 v = *(const floatx4*)(p + at);
+  for (int s = 1; s < splits; ++s) v += *(const floatx4*)(p + s * stride + at);
+  return v;
+}
+
+// y = bf16 of the sums + bias; GATE: [m, 2 N] -> silu(gate) up [m, N]. N % 4 == 0.
+template <bool GATE>
+__global__ __launch_bounds__(256) void finish_kernel(const float* __restrict__ part, const bf16_t* __restrict__ bias,
+                                                     bf16_t* __restrict__ y, int m, int N, int splits) {
+  const int at = (blockIdx.x * 256 + threadIdx.x) * 4, wide = GATE ? 2 * N : N;
+  if (at >= N) return;
+  const size_t row = blockIdx.y, stride = (size_t)m * wide;
+  const floatx4 g = sum_parts(part, row * wide + at, stride, splits);
+  float v[4];
+  if (GATE) {
+    const floatx4 u = sum_parts(part, row * wide + N + at, stride, splits);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = siluf(rounded(g[r])) * rounded(u[r]);
+  } else {
+    float b[4] = {};
+    if (bias) ld4(bias + at, b);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = g[r] + b[r];
+  }
+  st4(y + row * N + at, v);
+}
+
+// h = x + bf16 of the sums (bf16), n = norm(x + ..) w. One block a row, which stays
+// in registers. ROUND: the norm reads h as it is stored.
+template <int NC>
+__global__ __launch_bounds__(256) void add_norm_kernel(const float* __restrict__ part, const bf16_t* __restrict__ x,
+                                                       const bf16_t* __restrict__ w, bf16_t* __restrict__ h,
+                                                       bf16_t* __restrict__ n, int m, int D, int splits, float eps,
+                                                       float add, bool round) {
+  __shared__ float red[4];
+  const size_t row = (size_t)blockIdx.x * D, stride = (size_t)m * D;
+  float v[NC][4], ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int at = (c * 256 + threadIdx.x) * 4;
+    if (at >= D) break;
+    const floatx4 p = sum_parts(part, row + at, stride, splits);
+    ld4(x + row + at, v[c]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[c][r] += rounded(p[r]);
+    st4(h + row + at, v[c]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if (round) v[c][r] = rounded(v[c][r]);
+      ss += v[c][r] * v[c][r];
+    }
+  }
+  if (!w) return;
+  const float inv = rsqrtf(block_sum(ss, red) / (float)D + eps);
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int at = (c * 256 + threadIdx.x) * 4;
+    if (at >= D) break;
+    float by[4];
+    ld4(w + at, by);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[c][r] *= inv * (by[r] + add);
+    st4(n + row + at, v[c]);
+  }
+}
+
+// ===========================================================================
+// host side
+// ===========================================================================
+template <int BN, int BM, int BUFS, int END>
+static void launch_tile(const TileArgs& a) {
+  typedef TileShape<BN, BM, BUFS> Sh;
+  if (Sh::LDS > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute((const void*)tile_kernel<BN, BM, BUFS, END>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, Sh::LDS);
+    TORCH_CHECK(e == hipSuccess, "no LDS for weight tiles");
+  }
+  const int per = END == GATED ? BN / 2 : BN;
+  const int units = (a.N + per - 1) / per * a.splits, mts = (a.m + BM - 1) / BM;
+  hipLaunchKernelGGL((tile_kernel<BN, BM, BUFS, END>), dim3((units + 7) / 8 * 8 * mts), dim3(256), Sh::LDS, cur_stream(), a);
+}
+
+// Tile and depth by the rows of x and by the blocks that 128 weight rows make. us at
+// [N, K], 64-row or (deeper, fewer to a CU) first:
+//   m 32: [2048, 2048] in 128 blocks 4.4, 5.0; [3584, 18944] in 224 25.6, 22.9
+//   m 64: [2048, 2048] 5.0, 6.0; [28672 -> 8192] 89.7, 76.1
+//   m 128, 3 and 2 buffers: [8192, 8192] in 256 35.4, 39.6; [57344, 8192] in 448 203, 194
+template <int END>
+static void run_tile(const TileArgs& a) {
+  const int rows = END == GATED ? 2 * a.N : a.N, units = (rows + 127) / 128 * a.splits;
+  if (a.m <= 16) launch_tile<(END == GATED ? 128 : 64), 16, 4, END>(a);
+  else if (a.m <= 32) {
+    if (END == GATED || units >= 200) launch_tile<128, 32, 4, END>(a);
+    else launch_tile<64, 32, 4, (END == GATED ? STORE : END)>(a);
+  } else if (a.m <= 64) {
+    if (units >= 200) launch_tile<128, 64, 3, END>(a);
+    else launch_tile<64, 64, 4, END>(a);
+  } else if (units * ((a.m + 127) / 128) > 288) launch_tile<128, 128, 2, END>(a);
+  else launch_tile<128, 128, 3, END>(a);
+}
+
+static TileArgs tile_args(const Tensor& x, const Tensor& w) {
+  check_io(x, torch::kBFloat16);
+  check_io(w, torch::kBFloat16);
+  TileArgs a{};
+  CHK(w.dim() == 2 && w.size(1) % 64 == 0 && w.size(1) > 0 && x.size(-1) == w.size(1));
+  CHK(w.size(0) >= 1 && w.size(0) <= 1 << 26 && w.size(1) <= 1 << 26);
+  a.K = (int)w.size(1);
+  const int64_t m = x.numel() / a.K;
+  CHK(m >= 1 && m <= 256);
+  CHK(((size_t)x.data_ptr() & 15) == 0 && ((size_t)w.data_ptr() & 15) == 0);
+  a.m = (int)m;
+  a.N = (int)w.size(0);
+  a.steps = a.K / 64;
+  a.x = P<bf16_t>(x);
+  a.w = P<bf16_t>(w);
+  return a;
+}
+
+// Parts of k: as few as give some 450 blocks of 64 weight rows, of 4 steps at least
+static int splits_of(int rows, int steps) {
+  const int tiles = (rows + 63) / 64;
+  return std::max(1, std::min({(448 + tiles - 1) / tiles, steps / 4, 16}));
+}
+
+static Tensor sized(const Tensor& x, int64_t n) {
+  auto shape = x.sizes().vec();
+  shape.back() = n;
+  return torch::empty(shape, x.options());
+}
+
+// fp32 [splits, m, N]
+Tensor tile_parts(Tensor x, Tensor w) {
+  auto a = tile_args(x, w);
+  a.splits = splits_of(a.N, a.steps);
+  auto part = torch::empty({a.splits, a.m, a.N}, x.options().dtype(torch::kFloat32));
+  a.y = part.data_ptr();
+  run_tile<PART>(a);
+  return part;
+}
+
+Tensor tile_linear(Tensor x, Tensor w, OptT bias) {
+  auto a = tile_args(x, w);
+  if (bias) {
+    check_io(*bias, torch::kBFloat16);
+    CHK(bias->numel() == a.N);
+    a.bias = P<bf16_t>(*bias);
+  }
+  auto y = sized(x, a.N);
+  a.splits = a.N % 4 ? 1 : splits_of(a.N, a.steps);
+  if (a.splits == 1) {
+    a.y = y.data_ptr();
+    run_tile<STORE>(a);
+    return y;
+  }
+  auto part = torch::empty({a.splits, a.m, a.N}, x.options().dtype(torch::kFloat32));
+  a.y = part.data_ptr();
+  run_tile<PART>(a);
+  hipLaunchKernelGGL((finish_kernel<false>), dim3((a.N + 1023) / 1024, a.m), dim3(256), 0, cur_stream(),
+                     part.data_ptr<float>(), a.bias, M<bf16_t>(y), a.m, a.N, a.splits);
+  return y;
+}
+
+Tensor tile_swiglu(Tensor x, Tensor w) {
+  auto a = tile_args(x, w);
+  CHK(a.N % 8 == 0);
+  const int I = a.N / 2;
+  auto y = sized(x, I);
+  a.splits = splits_of(a.N, a.steps);
+  if (a.splits == 1) {
+    a.N = I;
+    a.y = y.data_ptr();
+    run_tile<GATED>(a);
+    return y;
+  }
+  auto part = torch::empty({a.splits, a.m, a.N}, x.options().dtype(torch::kFloat32));
+  a.y = part.data_ptr();
+  run_tile<PART>(a);
+  hipLaunchKernelGGL((finish_kernel<true>), dim3((I + 1023) / 1024, a.m), dim3(256), 0, cur_stream(),
+                     part.data_ptr<float>(), nullptr, M<bf16_t>(y), a.m, I, a.splits);
+  return y;
+}
+
+// (h, norm(h) w) with h = x + sum of the parts; w none: h alone
+std::vector<Tensor> parts_add_norm(Tensor part, Tensor x, OptT w, double eps, double add, bool round) {
+  check_io(part, torch::kFloat32);
+  check_io(x, torch::kBFloat16);
+  CHK(part.dim() == 3 && part.numel() == x.numel() * part.size(0) && part.size(2) == x.size(-1));
+  const int D = (int)x.size(-1), m = (int)part.size(1);
+  CHK(D % 4 == 0 && D <= 16384 && ((size_t)x.data_ptr() & 7) == 0);
+  auto h = torch::empty_like(x);
+  Tensor n;
+  const bf16_t* wp = nullptr;
+  if (w) {
+    check_io(*w, torch::kBFloat16);
+    CHK(w->numel() == D && ((size_t)w->data_ptr() & 7) == 0);
+    n = torch::empty_like(x);
+    wp = P<bf16_t>(*w);
+  }
+  bf16_t* np = w ? M<bf16_t>(n) : nullptr;
+#define GO(NC_) hipLaunchKernelGGL((add_norm_kernel<NC_>), dim3(m), dim3(256), 0, cur_stream(), part.data_ptr<float>(), \
+                                   P<bf16_t>(x), wp, M<bf16_t>(h), np, m, D, (int)part.size(0), (float)eps, (float)add, round)
+  if (D <= 2048) GO(2);
+  else if (D <= 4096) GO(4);
+  else if (D <= 8192) GO(8);
+  else GO(16);
+#undef GO
+  if (w) return {h, n};
+  return {h};
+}
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("tile_splits", [](int64_t n, int64_t k) { return splits_of((int)n, (int)(k / 64)); });
+  m.def("tile_parts", &tile_parts);
+  m.def("tile_linear", &tile_linear);
+  m.def("tile_swiglu", &tile_swiglu);
+  m.def("parts_add_norm", &parts_add_norm);
+}
