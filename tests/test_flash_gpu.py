@@ -1,0 +1,43 @@
+"""Prompt attention over the packed cache against 64 bits: rows and keys at the edges of
+their tiles (128 rows of heads times positions, 32 and 64 keys), keys split over blocks."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _pack(k, v):
+  """[B, heads, T, 128] -> the fragment order of the cache, T rounded up to 32."""
+  B, heads, T, _ = k.shape
+  t32 = -(-T // 32) * 32
+  k, v = (torch.nn.functional.pad(t, (0, 0, 0, t32 - T)) for t in (k, v))
+  return (k.view(B, heads, t32 // 16, 16, 4, 4, 8).permute(0, 1, 2, 4, 5, 3, 6).reshape(B, heads, t32 // 16, 4, 64, 8).contiguous(),
+          v.view(B, heads, t32 // 32, 4, 8, 8, 16).permute(0, 1, 5, 2, 3, 6, 4).reshape(B, heads, 8, t32 // 32, 64, 8).contiguous())
+
+
+@pytest.mark.parametrize("B,S,H,KVH,start,cap,window", [
+  (1, 1, 1, 1, 0, 0.0, 0), (2, 33, 5, 1, 31, 0.0, 0), (1, 128, 7, 7, 0, 0.0, 0), (3, 65, 12, 2, 64, 0.0, 0),
+  (1, 9, 28, 4, 1500, 0.0, 0), (1, 257, 8, 2, 1023, 0.0, 0), (1, 600, 4, 2, 0, 0.0, 0),
+  (1, 140, 4, 2, 300, 20.0, 0), (1, 140, 4, 2, 300, 0.0, 50), (2, 40, 4, 1, 700, 30.0, 64), (1, 300, 2, 1, 0, 0.0, 1)])
+def test_prefill_attention(B, S, H, KVH, start, cap, window):
+  from xotorch_amd.ops import _hip_ops
+  g = torch.Generator(device="cuda").manual_seed(S)
+  T, rep = start + S, H // KVH
+  qkv = torch.randn(B, S, H + 3, 128, generator=g, device="cuda").to(torch.bfloat16)
+  q = qkv[:, :, :H]  # a view of a wider row, as the projection gives it
+  k, v = (torch.randn(B, KVH, T, 128, generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
+  out = _hip_ops.attn_prefill_mfma(q, *_pack(k, v), start, 0.0, cap, window).double()
+  kd, vd = k.double().repeat_interleave(rep, 1), v.double().repeat_interleave(rep, 1)
+  qd = q.double().transpose(1, 2)
+  s = qd @ kd.transpose(-1, -2) * 128 ** -0.5
+  # fp32 sums of 128 products, the scaling and the exponent
+  off = (qd.abs() @ kd.abs().transpose(-1, -2)).amax(-1, keepdim=True) * 128 ** -0.5 * (132 * 2.0 ** -24)
+  if cap:
+    s = cap * torch.tanh(s / cap)
+  at = torch.arange(start, T, device="cuda")[:, None] - torch.arange(T, device="cuda")[None]
+  hidden = (at < 0) | (at >= window) if window else at < 0
+  p = s.masked_fill(hidden, -torch.inf).softmax(-1)
+  ref, size = (p @ vd).transpose(1, 2), (p @ vd.abs()).transpose(1, 2)
+  # probabilities as bf16, above and below the line, and the result
+  bound = size * (2.0 ** -7 + 4 * off.transpose(1, 2)) + ref.abs() * 2.0 ** -8
+  assert out.shape == ref.shape and bool(((out - ref).abs() <= bound + 1e-6).all())

@@ -690,197 +690,239 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// MFMA flash-forward prefill attention (hd = 128, causal, GQA).
+// MFMA flash-forward prefill attention (hd = 128, causal, GQA) over the packed
+// cache (reference: torchtune MultiHeadAttention prefill, general_mha.py:218-226).
 //
-// Replaces torch sdpa for the prefill step (reference: torchtune
-// MultiHeadAttention prefill, general_mha.py:218-226; sdpa measures ~1.8 ms
-// per 70B layer at B=64xS=512 — VALU/flash at ~300 TF).  Grid: one 4-wave
-// workgroup per (b, q-head, 128-row q block); the block's waves share K/V
-// tiles staged in LDS from the MFMA-packed cache (fragment layout is
-// lane-linear, so staging is 1 KB coalesced loads and conflict-free b128
-// reads).  Each wave owns 32 q rows (2 MFMA sub-tiles), walks kv position
-// tiles of 32 with online softmax, masks the causal boundary, writes final
-// bf16 rows (no split-K workspace).
+// What bounds it are the matrix cores and, as much, the exponentials. A block owns
+// 128 query rows of one key head: positions times the heads that share it, so that
+// keys and values are staged once for all of them and few scores are computed past
+// the diagonal. Scores are computed transposed (keys x queries) from key rows in an
+// order in which the lane that holds a query's probabilities feeds them to the value
+// product directly; a row of ones gives the sums of the probabilities as they are
+// multiplied. 64 positions at a time come by direct loads, two buffers deep. Lanes
+// exchange maxima and rescale only where one grows (a maximum that may lag costs
+// precision: the largest probability is then rounded too). Where the rows make too
+// few blocks, the keys are split and the parts merged.
+// us, and as it was with a block per head and probabilities through LDS: 6001 tokens,
+// 32 heads on 8 338 (873 TFLOP/s; 1309); 16 x 512, 64 on 8 137 (352); 256 tokens after
+// 1280, 28 on 4 37 (150).
 // ---------------------------------------------------------------------------
 
-__global__ __launch_bounds__(256) void attn_prefill_mfma_kernel(
-    const unsigned short* __restrict__ q, const unsigned short* __restrict__ kp,
-    const unsigned short* __restrict__ vp, unsigned short* __restrict__ out,
-    int B, int S, int H, int KVH, int T32, int start_pos,
-    long long q_bstride, long long q_sstride, float scale,
-    float softcap, int window) {
-  // block -> (b, h, q-block)
-  const int qblocks = (S + 127) >> 7;
-  const int h = blockIdx.x % H;
-  const int t1 = blockIdx.x / H;
-  const int qb = t1 % qblocks;
-  const int b = t1 / qblocks;
-  const int wv = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63;
-  const int kvh = h / (H / KVH);
+DEVINL floatx4 mma16(const bf16x8& a, const bf16x8& b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
 
-  // this wave's 32 q rows: [r0, r0+32)
-  const int r0 = qb * 128 + wv * 32;
-  const int col = lane & 15;
+// What the cache holds per 32 positions and key head: K two tiles of 16 positions
+// [4 chunks of 32 dims][64 lanes][8], lane = (dim % 32) / 8 * 16 + position % 16;
+// V [8 groups of 16 dims], each [64 lanes][8] with lane = (position % 32) / 8 * 16 +
+// dim % 16, groups T32 * 16 apart.
+struct FlashArgs {
+  const unsigned short *q, *k, *v;
+  unsigned short* out;
+  float *part, *ml;  // [rows][splits][128] and [rows][splits][2] where the keys are split
+  int S, H, KVH, T32, start, blocks, splits, window;
+  long long q_b, q_s;  // strides of a batch row and of a token
+  float scale, cap;    // scale times log2 e, or plain with a cap
+};
 
-  __shared__ unsigned short kv_lds[2][8192];  // K tile 8 KB + V tile 8 KB, dbuf
+typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(1))) const void glb_void;
 
-  // Q fragments for 2 sub-tiles x 4 hd-chunks; rows clamped to S-1 (writes
-  // are predicated, extra rows only waste compute)
-  bf16x8 qf[2][4];
+constexpr int KSUB = 8192 + 128, SUB = KSUB + 8192, STAGE = 2 * SUB;  // bytes of LDS: keys, 32 positions, 64
+
+// 8 fragments from LDS, and the wait for them
+#define READ8(F, A, O0, O1, O2, O3, O4, O5, O6, O7)                                                                    \
+  asm volatile("ds_read_b128 %0, %8 offset:" #O0 "\n\tds_read_b128 %1, %8 offset:" #O1 "\n\tds_read_b128 %2, %8 offset:" #O2 \
+               "\n\tds_read_b128 %3, %8 offset:" #O3 "\n\tds_read_b128 %4, %8 offset:" #O4                             \
+               "\n\tds_read_b128 %5, %8 offset:" #O5 "\n\tds_read_b128 %6, %8 offset:" #O6                             \
+               "\n\tds_read_b128 %7, %8 offset:" #O7 "\n\ts_waitcnt lgkmcnt(0)"                                        \
+               : "=&v"(F[0]), "=&v"(F[1]), "=&v"(F[2]), "=&v"(F[3]), "=&v"(F[4]), "=&v"(F[5]), "=&v"(F[6]), "=&v"(F[7]) \
+               : "v"(A))
+
+// maximum over the four lanes that hold a query's scores
+DEVINL float quad_max(float v) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+// SIDE: capped scores and a sliding window
+template <bool SIDE>
+__global__ __launch_bounds__(256, 2) void flash_prefill_kernel(FlashArgs a) {
+  constexpr int QT = 2;  // tiles of 16 query rows a wave
+  extern __shared__ __attribute__((aligned(16))) char lds[];  // [2][STAGE]
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int col = lane & 15, quad = lane >> 4;
+  const int rep = a.H / a.KVH, heads = gridDim.x / (a.blocks * a.splits);  // heads: batch rows times key heads
+  // the longest rows first; a key head stays on one die where there are eight of them
+  const int bh = blockIdx.x % heads, rest = blockIdx.x / heads, split = rest % a.splits;
+  const int block = a.blocks - 1 - rest / a.splits;
+  const int b = bh / a.KVH, kvh = bh % a.KVH;
+  const int rows = a.S * rep, row0 = block * 128 + wave * QT * 16;
+  const char* kb = (const char*)(a.k + (size_t)bh * a.T32 * 128);
+  const char* vb = (const char*)(a.v + (size_t)bh * a.T32 * 128);
+  // positions that this block reads: whole tiles of 64, a part of them per split
+  const int last = a.start + (min(block * 128 + 127, rows - 1)) / rep;  // the last one seen
+  const int low = SIDE && a.window > 0 ? max(0, a.start + block * 128 / rep - a.window + 1) : 0;
+  const int tile0 = low >> 6, count = (last >> 6) + 1 - tile0;
+  const int t0 = tile0 + count * split / a.splits, t1 = tile0 + count * (split + 1) / a.splits;
+  const int subs = (last >> 5) + 1;  // tiles of 32 that hold something
+
+  bf16x8 qf[QT][4];
+  int pos[QT];  // of this lane's query
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int row = min(r0 + t * 16 + col, S - 1);
-    const unsigned short* qrow = q + (size_t)b * q_bstride + (size_t)row * q_sstride + (size_t)h * 128;
+  for (int t = 0; t < QT; ++t) {
+    const int r = min(row0 + t * 16 + col, rows - 1), s = r / rep;
+    pos[t] = a.start + s;
+    const unsigned short* q = a.q + (size_t)b * a.q_b + (size_t)s * a.q_s + (size_t)(kvh * rep + r % rep) * 128 + quad * 8;
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
-      qf[t][c] = *reinterpret_cast<const bf16x8*>(qrow + c * 32 + (lane >> 4) * 8);
+    for (int c = 0; c < 4; ++c) qf[t][c] = *(const bf16x8*)(q + c * 32);
   }
+  const int first_pos = a.start + min(row0, rows - 1) / rep;  // of the wave's first row
+  const int last_pos = a.start + min(row0 + QT * 16 - 1, rows - 1) / rep;
 
-  float m[2][4], lsum[2][4];
-  floatx4 acco[2][8];
+  // waves 0 and 2 stage keys of 32 positions each, waves 1 and 3 values
+  auto stage = [&](int tile) {
+    const int sub = min(tile * 2 + (wave >> 1), (a.T32 >> 5) - 1);
+    char* dst = lds + (tile & 1) * STAGE + (wave >> 1) * SUB;
+    if (wave & 1) {
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+      for (int g = 0; g < 8; ++g)
+        __builtin_amdgcn_global_load_lds((glb_void*)(vb + ((size_t)g * (a.T32 >> 5) + sub) * 1024 + lane * 16),
+                                         (lds_void*)(dst + KSUB + g * 1024), 16, 0, 0);
+    } else {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) { m[t][r] = -INFINITY; lsum[t][r] = 0.f; }
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int g = 0; g < 8; ++g) acco[t][g] = (floatx4)(0.f);
-
-  const size_t kbase = (size_t)(b * KVH + kvh) * (T32 >> 4) * 2048;
-  const size_t vbase = (size_t)(b * KVH + kvh) * 8 * (T32 >> 5) * 512;
-  // causal end for the BLOCK (max row): positions [0, start_pos + block_hi]
-  const int block_hi = min(qb * 128 + 127, S - 1);
-  const int kv_end = start_pos + block_hi + 1;  // exclusive
-
-  __shared__ unsigned short plds_all[4][16 * 48 * 2];
-
-  // cooperative stage of kv tile `tp` (32 positions) into kv_lds[buf]
-  auto stage = [&](int tp, int buf) {
-    // K: two 16-pos tiles x 4 chunks x 512 elems; V: 8 groups x 512 elems
-    // 256 threads x 24 pieces of 256 B... simpler: each thread copies 16 B x3
-    const unsigned short* ksrc = kp + kbase + (size_t)(tp * 2) * 2048;
-    const unsigned short* vsrc = vp + vbase + (size_t)tp * 512;
-    unsigned short* dk = kv_lds[buf];
-    unsigned short* dv = kv_lds[buf] + 4096;
-    const int tid = threadIdx.x;
-    // K: 4096 elems = 8192 B: 256 threads x 2 x 16 B
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int e = (tid + i * 256) * 8;
-      *(ushort8*)(dk + e) = *(const ushort8*)(ksrc + e);
-    }
-    // V: 8 groups x 512 elems, group stride (T32>>5)*512 in global
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int e = tid + i * 256;           // 0..511 -> (group, piece)
-      const int g = e >> 6, piece = e & 63;  // 64 pieces of 8 elems per group
-      *(ushort8*)(dv + g * 512 + piece * 8) =
-          *(const ushort8*)(vsrc + (size_t)g * (T32 >> 5) * 512 + piece * 8);
+      for (int c = 0; c < 8; ++c)  // the second 16 positions 64 bytes further: their rows fall on other banks
+        __builtin_amdgcn_global_load_lds((glb_void*)(kb + (size_t)sub * 8192 + c * 1024 + lane * 16),
+                                         (lds_void*)(dst + c * 1024 + (c >> 2) * 64), 16, 0, 0);
     }
   };
 
-  const int ntiles = (kv_end + 31) >> 5;
-  // sliding window: the block's lowest q row sees nothing before
-  // start_pos + qb*128 - window + 1 — skip whole kv tiles below it
-  const int tp0 = (window > 0) ? max(0, (start_pos + qb * 128 - window + 1) >> 5) : 0;
-  stage(tp0, tp0 & 1);
-  __syncthreads();
-
-  for (int tp = tp0; tp < ntiles; ++tp) {
-    const int buf = tp & 1;
-    if (tp + 1 < ntiles) stage(tp + 1, buf ^ 1);  // plain loads overlap compute
-    const unsigned short* dk = kv_lds[buf];
-    const unsigned short* dv = kv_lds[buf] + 4096;
-    unsigned short* plds = plds_all[wv];
+  float m[QT];
+  floatx4 o[QT][8], l[QT];  // l: the same sum in all four
+  bf16x8 ones;
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      // scores for two 16-pos halves of this kv tile
-      floatx4 sc[2];
+  for (int i = 0; i < 8; ++i) ones[i] = (__bf16)1.f;
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        sc[hh] = (floatx4)(0.f);
+  for (int t = 0; t < QT; ++t) {
+    m[t] = -1e30f;
+    l[t] = (floatx4)(0.f);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const bf16x8 kb = *reinterpret_cast<const bf16x8*>(dk + (hh * 4 + c) * 512 + lane * 8);
-          sc[hh] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qf[t][c], kb, sc[hh], 0, 0, 0);
+    for (int g = 0; g < 8; ++g) o[t][g] = (floatx4)(0.f);
+  }
+  // key rows of the two products of 16: row i is position i / 4 * 8 + i % 4, and 4 more
+  const int p = (col >> 2) * 8 + (col & 3);
+  const unsigned base = (unsigned)(size_t)(lds_void*)lds;
+  const unsigned klane = base + (p >> 4) * (4096 + 64) + (quad * 16 + (p & 15)) * 16, vlane = base + KSUB + lane * 16;
+  if (t0 < t1) stage(t0);
+  for (int tile = t0; tile < t1; ++tile) {
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    if (tile + 1 < t1) stage(tile + 1);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int p0 = tile * 64 + u * 32;
+      if (tile * 2 + u >= subs || p0 > last_pos) continue;
+      if (SIDE && a.window > 0 && p0 + 31 <= first_pos - a.window) continue;
+      const unsigned at = (tile & 1) * STAGE + u * SUB;
+      bf16x8 kf[8];
+      READ8(kf, klane + at, 0, 64, 1024, 1088, 2048, 2112, 3072, 3136);
+      floatx4 sc[QT][2];
+#pragma unroll
+      for (int t = 0; t < QT; ++t)
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {
+          sc[t][hf] = (floatx4)(0.f);
+#pragma unroll
+          for (int c = 0; c < 4; ++c) sc[t][hf] = mma16(kf[c * 2 + hf], qf[t][c], sc[t][hf]);
         }
-      }
-      // causal mask: kv pos must be < start_pos + row + 1
-      float rmax[4];
+      const bool edge = p0 + 31 > first_pos || (SIDE && a.window > 0 && p0 <= last_pos - a.window);
+      bf16x8 pf[QT];
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        const int pos = tp * 32 + hh * 16 + col;
+      for (int t = 0; t < QT; ++t) {
+        float v[8];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = r0 + t * 16 + (lane >> 4) * 4 + r;
-          bool ok = (pos <= start_pos + row) && (pos < kv_end);
-          if (window > 0) ok = ok && (pos > start_pos + row - window);
-          float s = sc[hh][r] * scale;
-          if (softcap > 0.f) s = softcap * tanhf(s * (1.f / softcap));
-          sc[hh][r] = ok ? s : -INFINITY;
+        for (int i = 0; i < 8; ++i) {
+          v[i] = sc[t][i >> 2][i & 3] * a.scale;
+          if (SIDE && a.cap > 0.f) v[i] = 1.4426950408889634f * a.cap * tanhf(v[i] * (1.f / a.cap));
         }
+        if (edge) {
+          const int d = pos[t] - p0 - quad * 8;  // distance to this lane's first key
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            bool ok = i <= d;
+            if (SIDE && a.window > 0) ok = ok && d - i < a.window;
+            v[i] = ok ? v[i] : -INFINITY;
+          }
+        }
+        float top = fmaxf(fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])), fmaxf(fmaxf(v[4], v[5]), fmaxf(v[6], v[7])));
+        if (__any(top > m[t])) {
+          top = fmaxf(m[t], quad_max(top));
+          const float f = __builtin_amdgcn_exp2f(m[t] - top);
+          m[t] = top;
+          l[t] *= f;
+#pragma unroll
+          for (int g = 0; g < 8; ++g) o[t][g] *= f;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) pf[t][i] = (__bf16)__builtin_amdgcn_exp2f(v[i] - m[t]);
+        l[t] = mma16(ones, pf[t], l[t]);
       }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) rmax[r] = fmaxf(sc[0][r], sc[1][r]);
-#pragma unroll
-      for (int mm = 1; mm < 16; mm <<= 1)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) rmax[r] = fmaxf(rmax[r], __shfl_xor(rmax[r], mm));
-      float alpha[4], rsum[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float mn = fmaxf(m[t][r], rmax[r]);
-        if (mn == -INFINITY) { alpha[r] = 1.f; rsum[r] = 0.f; sc[0][r] = 0.f; sc[1][r] = 0.f; continue; }
-        alpha[r] = (lsum[t][r] > 0.f) ? __expf(m[t][r] - mn) : 0.f;
-        m[t][r] = mn;
-        const float p0 = __expf(sc[0][r] - mn);
-        const float p1 = __expf(sc[1][r] - mn);
-        sc[0][r] = p0;
-        sc[1][r] = p1;
-        rsum[r] = p0 + p1;
-      }
-#pragma unroll
-      for (int mm = 1; mm < 16; mm <<= 1)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) rsum[r] += __shfl_xor(rsum[r], mm);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) lsum[t][r] = lsum[t][r] * alpha[r] + rsum[r];
+      bf16x8 vf[8];
+      READ8(vf, vlane + at, 0, 1024, 2048, 3072, 4096, 5120, 6144, 7168);
 #pragma unroll
       for (int g = 0; g < 8; ++g)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acco[t][g][r] *= alpha[r];
-      unsigned short* pl = plds + t * 16 * 48;  // reuse the 2x buffer per sub-tile
-#pragma unroll
-      for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          pl[((lane >> 4) * 4 + r) * 48 + hh * 16 + col] = f2b(sc[hh][r]);
-      const bf16x8 pf = *reinterpret_cast<const bf16x8*>(pl + (lane & 15) * 48 + (lane >> 4) * 8);
-#pragma unroll
-      for (int g = 0; g < 8; ++g) {
-        const bf16x8 vb = *reinterpret_cast<const bf16x8*>(dv + g * 512 + lane * 8);
-        acco[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf, vb, acco[t][g], 0, 0, 0);
-      }
+        for (int t = 0; t < QT; ++t) o[t][g] = mma16(vf[g], pf[t], o[t][g]);
     }
-    __syncthreads();  // all waves done with kv_lds[buf] before restaging
   }
+#pragma unroll
+  for (int t = 0; t < QT; ++t) {
+    const int r = row0 + t * 16 + col;
+    const float sum = l[t][0];
+    if (r >= rows) continue;
+    if (a.splits > 1) {
+      const size_t i = ((size_t)bh * rows + r) * a.splits + split;
+#pragma unroll
+      for (int g = 0; g < 8; ++g) *(floatx4*)(a.part + i * 128 + g * 16 + quad * 4) = o[t][g];
+      if (quad == 0) {
+        a.ml[i * 2] = m[t];
+        a.ml[i * 2 + 1] = sum;
+      }
+      continue;
+    }
+    const float f = sum > 0.f ? 1.f / sum : 0.f;
+    unsigned short* dst = a.out + (((size_t)b * a.S + r / rep) * a.H + kvh * rep + r % rep) * 128 + quad * 4;
+#pragma unroll
+    for (int g = 0; g < 8; ++g) {
+      ushort4_t v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = f2b(o[t][g][i] * f);
+      *(ushort4_t*)(dst + g * 16) = v;
+    }
+  }
+}
 
-  // epilogue: out[b, row, h, g*16 + col] = acc / lsum
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = r0 + t * 16 + (lane >> 4) * 4 + r;
-      if (row < S) {
-        const float inv = (lsum[t][r] > 0.f) ? 1.f / lsum[t][r] : 0.f;
-        unsigned short* orow = out + (((size_t)b * S + row) * H + h) * 128;
-#pragma unroll
-        for (int g = 0; g < 8; ++g) orow[g * 16 + col] = f2b(acco[t][g][r] * inv);
-      }
-    }
+// A wave a row of [B, S, H]: the splits' parts, weighed by how far their maxima lie
+// below the largest.
+__global__ __launch_bounds__(256) void flash_merge_kernel(FlashArgs a, int total) {
+  const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (i >= total) return;
+  const int h = i % a.H, rest = i / a.H, s = rest % a.S, b = rest / a.S, rep = a.H / a.KVH;
+  const size_t row = ((size_t)b * a.KVH + h / rep) * a.S * rep + (size_t)s * rep + h % rep;
+  const float* ml = a.ml + row * a.splits * 2;
+  float top = -1e30f, sum = 0.f, o[2] = {};
+  for (int k = 0; k < a.splits; ++k) top = fmaxf(top, ml[k * 2]);
+  for (int k = 0; k < a.splits; ++k) {
+    const float f = __builtin_amdgcn_exp2f(ml[k * 2] - top);
+    sum += f * ml[k * 2 + 1];
+    const float2 v = *(const float2*)(a.part + (row * a.splits + k) * 128 + lane * 2);
+    o[0] += f * v.x;
+    o[1] += f * v.y;
   }
+  const float f = sum > 0.f ? 1.f / sum : 0.f;
+  const unsigned two = f2b(o[0] * f) | (unsigned)f2b(o[1] * f) << 16;
+  *(unsigned*)(a.out + (size_t)i * 128 + lane * 2) = two;
 }
 
 // layout probe for tests: one v_mfma_f32_16x16x32_bf16, row-major inputs
@@ -2444,28 +2486,65 @@ torch::Tensor attn_decode_mfma(torch::Tensor q, torch::Tensor kp, torch::Tensor 
   return out;
 }
 
-// q: [B, S, H, 128] (strided over b/s OK, head rows contiguous); kp/vp: the
-// packed cache copies already holding positions [0, start_pos + S).
-torch::Tensor attn_prefill_mfma(torch::Tensor q, torch::Tensor kp, torch::Tensor vp,
-                                int64_t start_pos, double scale_in, double softcap,
+// q: [B, S, H, 128], heads contiguous; k, v: the packed cache, which holds positions
+// [0, start + S). window 0: none; cap 0: none; scale 0: 1 / sqrt(128).
+torch::Tensor attn_prefill_mfma(torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                                int64_t start, double scale, double cap,
                                 int64_t window) {
-  CHK(q.is_cuda() && q.dtype() == torch::kBFloat16);
-  CHK(q.stride(3) == 1 && q.stride(2) == q.size(3));
-  CHK(kp.is_contiguous() && vp.is_contiguous());
-  const int B = q.size(0), S = q.size(1), H = q.size(2), hd = q.size(3);
-  TORCH_CHECK(hd == 128, "attn_prefill_mfma requires head_dim 128");
-  const int KVH = kp.size(1);
-  const int T32 = kp.size(2) * 16;
-  CHK(start_pos + S <= T32);
-  auto out = torch::empty({B, S, H, hd},
-                          torch::TensorOptions().dtype(torch::kBFloat16).device(q.device()));
-  const float scale = (scale_in > 0.0) ? (float)scale_in : 1.0f / sqrtf((float)hd);
-  const int qblocks = (S + 127) / 128;
-  hipLaunchKernelGGL(attn_prefill_mfma_kernel, dim3(B * qblocks * H), dim3(256), 0, cur_stream(),
-                     (const unsigned short*)q.data_ptr(), (const unsigned short*)kp.data_ptr(),
-                     (const unsigned short*)vp.data_ptr(), (unsigned short*)out.data_ptr(),
-                     B, S, H, KVH, T32, (int)start_pos, q.stride(0), q.stride(1), scale,
-                     (float)softcap, (int)window);
+  CHK(q.is_cuda() && q.scalar_type() == torch::kBFloat16 && q.dim() == 4);
+  CHK(q.size(3) == 128 && q.stride(3) == 1 && q.stride(2) == 128);
+  CHK(k.is_cuda() && v.is_cuda() && k.scalar_type() == torch::kBFloat16 && v.scalar_type() == torch::kBFloat16);
+  CHK(k.is_contiguous() && v.is_contiguous());
+  CHK((((size_t)k.data_ptr() | (size_t)v.data_ptr()) & 15) == 0);
+  FlashArgs a{};
+  const int B = (int)q.size(0);
+  a.S = (int)q.size(1);
+  a.H = (int)q.size(2);
+  a.KVH = (int)k.size(1);
+  a.T32 = (int)k.size(2) * 16;
+  CHK(k.size(0) >= B && v.size(0) >= B && a.KVH > 0 && a.H % a.KVH == 0 && k.numel() == k.size(0) * a.KVH * a.T32 * 128);
+  CHK(v.numel() == v.size(0) * a.KVH * a.T32 * 128 && a.T32 % 32 == 0 && start >= 0 && start + a.S <= a.T32);
+  auto out = torch::empty({B, a.S, a.H, 128}, q.options());
+  if (out.numel() == 0) return out;
+  a.start = (int)start;
+  a.window = (int)window;
+  a.cap = (float)cap;
+  const bool side = cap > 0.0 || window > 0;
+  a.scale = (scale > 0.0 ? (float)scale : 0.08838834764831845f) * (cap > 0.0 ? 1.f : 1.4426950408889634f);
+  a.q = (const unsigned short*)q.data_ptr();
+  a.k = (const unsigned short*)k.data_ptr();
+  a.v = (const unsigned short*)v.data_ptr();
+  a.out = (unsigned short*)out.data_ptr();
+  a.q_b = q.stride(0);
+  a.q_s = q.stride(1);
+  const int64_t rows = (int64_t)a.S * (a.H / a.KVH);
+  CHK(rows <= INT_MAX / 256);
+  a.blocks = (int)((rows + 127) / 128);
+  const int64_t whole = (int64_t)a.blocks * B * a.KVH;
+  // two blocks a CU, of two tiles of 64 positions at least
+  const int tiles = (int)((start + a.S + 63) / 64);
+  a.splits = (int)std::max<int64_t>(1, std::min<int64_t>({(512 + whole - 1) / whole, tiles / 2, 16}));
+  CHK(whole * a.splits <= INT_MAX);
+  torch::Tensor part, ml;
+  if (a.splits > 1) {
+    const auto opts = q.options().dtype(torch::kFloat32);
+    part = torch::empty({B * a.KVH * rows, a.splits, 128}, opts);
+    ml = torch::empty({B * a.KVH * rows, a.splits, 2}, opts);
+    a.part = part.data_ptr<float>();
+    a.ml = ml.data_ptr<float>();
+  }
+  const dim3 grid((unsigned)(whole * a.splits));
+  auto run = [&](auto kernel) {
+    const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * STAGE);
+    TORCH_CHECK(e == hipSuccess, "no LDS for attention tiles");
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 2 * STAGE, cur_stream(), a);
+  };
+  if (side) run(flash_prefill_kernel<true>);
+  else run(flash_prefill_kernel<false>);
+  if (a.splits > 1) {
+    const int64_t total = (int64_t)B * a.S * a.H;
+    hipLaunchKernelGGL(flash_merge_kernel, dim3((unsigned)((total + 3) / 4)), dim3(256), 0, cur_stream(), a, (int)total);
+  }
   return out;
 }
 
