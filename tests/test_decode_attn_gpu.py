@@ -1,0 +1,91 @@
+"""A decode step's attention from the projection on (hip/decode_attn.hip): against 64 bits,
+and its caches against the separate append. Lengths at the edges of tiles (32), rows long
+enough for several blocks, parked rows, rows that share a position."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # B, H, KVH, hd, T, lengths (the new position included), norms, shared position
+  (1, 1, 1, 64, 8, [1], False, True), (2, 8, 2, 64, 100, [32, 33], False, False), (1, 32, 8, 64, 1024, [221], False, True),
+  (3, 16, 1, 128, 70, [64, 65, 1], True, False), (2, 28, 4, 128, 4096, [3100, 7], False, False),
+  (4, 5, 1, 64, 2400, [2400, 1, 1500, 800], True, False), (70, 8, 8, 128, 96, [40] * 70, False, True),
+  (2, 12, 2, 128, 2050, [2050, 257], True, False)]
+
+
+@pytest.mark.parametrize("B,H,KVH,hd,T,lens,norms,shared", CASES)
+def test_decode_attend(B, H, KVH, hd, T, lens, norms, shared):
+  from xotorch_amd import ops
+  from xotorch_amd.engine.kvcache import ShardKVCache
+  from xotorch_amd.ops import torch_ref
+  g = torch.Generator(device="cuda").manual_seed(T)
+
+  def rand(*shape):
+    return torch.randn(*shape, generator=g, device="cuda").to(torch.bfloat16)
+
+  cos, sin = torch_ref.rope_cos_sin(hd, T, 10000.0, device="cuda")
+  caches = [ShardKVCache(1, B, KVH, T, hd, torch.bfloat16, "cuda")[0] for _ in range(2)]
+  old = rand(B, T, (H + 2 * KVH) * hd)
+  at = torch.arange(T, dtype=torch.int32, device="cuda")
+  for c in caches:
+    ops.rope_qkv_append(old.clone(), cos, sin, at, c.k, c.v, H, KVH, hd, c.kp, c.vp)
+  qkv = rand(B, 1, (H + 2 * KVH) * hd)
+  qn, kn = (rand(hd), rand(hd)) if norms else (None, None)
+  seen = torch.tensor(lens, dtype=torch.int32, device="cuda")
+  pos = (seen[:1] if shared else seen) - 1
+  assert ops.decode_attends(qkv, H, KVH, hd, caches[0].kp, qn, kn)
+  before = qkv.clone()
+  out = ops.decode_attend(qkv, cos, sin, pos, seen, *caches[0][:4], H, KVH, qn, kn, 1e-6)
+  assert torch.equal(qkv, before)
+  ops.rope_qkv_append(qkv, cos, sin, pos, caches[1].k, caches[1].v, H, KVH, hd, caches[1].kp, caches[1].vp, qn, kn, 1e-6)
+  # fp32 sums of the norm in another order: a step of bf16 at most, and that rarely
+  for a, b in zip(caches[0][:4], caches[1][:4]):
+    assert torch.equal(a, b) if not norms else bool(((a.float() - b.float()).abs() <= b.float().abs() * 2.0 ** -7).all())
+  q = qkv[:, 0, :H * hd].view(B, H, hd).double()
+  for b, n in enumerate(lens):
+    k, v = (c[b, :, :n].double().repeat_interleave(H // KVH, 0) for c in (caches[0].k, caches[0].v))
+    s = (k @ q[b, :, :, None])[..., 0] * hd ** -0.5
+    # fp32 sums of hd products; with norms a query may be a step of bf16 off as well
+    off = (k.abs() @ q[b, :, :, None].abs())[..., 0].amax(-1, keepdim=True) * hd ** -0.5 * ((hd + 4) * 2.0 ** -24 + (2.0 ** -8 if norms else 0))
+    p = s.softmax(-1)
+    ref, size = (p[:, None] @ v)[:, 0], (p[:, None] @ v.abs())[:, 0]
+    bound = size * (2.0 ** -7 + 4 * off) + ref.abs() * 2.0 ** -8
+    assert bool(((out[b, 0].view(H, hd).double() - ref).abs() <= bound + 1e-6).all())
+
+
+def test_parked_row_keeps_to_its_own_place():
+  """A row that sees less than its position appends there and reads what it sees."""
+  from xotorch_amd import ops
+  from xotorch_amd.engine.kvcache import ShardKVCache
+  from xotorch_amd.ops import torch_ref
+  cos, sin = torch_ref.rope_cos_sin(128, 256, 10000.0, device="cuda")
+  c = ShardKVCache(1, 2, 2, 256, 128, torch.bfloat16, "cuda")[0]
+  g = torch.Generator(device="cuda").manual_seed(0)
+  qkv = torch.randn(2, 1, 8 * 128, generator=g, device="cuda").to(torch.bfloat16)
+  c.v[:, :, 0] = 1.0
+  c.vp.view(2, 2, 8, 8, 64, 8)[:, :, :, 0, :16, 0] = 1.0
+  pos, seen = torch.tensor([255, 300], dtype=torch.int32, device="cuda"), torch.tensor([1, 0], dtype=torch.int32, device="cuda")
+  cos, sin = (torch.cat([t, t]) for t in (cos, sin))
+  out = ops.decode_attend(qkv, cos, sin, pos, seen, *c[:4], 4, 2)
+  assert torch.equal(out[0], torch.ones_like(out[0])) and torch.equal(out[1], torch.zeros_like(out[1]))
+  assert torch.equal(c.v[0, :, 255].flatten(), qkv[0, 0, 6 * 128:]) and not c.v[0, :, 1:255].any() and not c.v[1, :, 1:].any()
+
+
+@pytest.mark.parametrize("S,H,KVH,start", [(1, 4, 2, 0), (45, 32, 8, 0), (257, 8, 2, 1000), (130, 7, 1, 63)])
+def test_prompt_attention_of_64_channels(S, H, KVH, start):
+  from xotorch_amd import ops
+  from xotorch_amd.engine.kvcache import ShardKVCache
+  g = torch.Generator(device="cuda").manual_seed(S)
+  c = ShardKVCache(1, 2, KVH, start + S, 64, torch.bfloat16, "cuda")[0]
+  qkv = torch.randn(2, start + S, (H + 2 * KVH) * 64, generator=g, device="cuda").to(torch.bfloat16)
+  still, none = torch.ones(start + S, 32, device="cuda"), torch.zeros(start + S, 32, device="cuda")
+  ops.rope_qkv_append(qkv, still, none, torch.arange(start + S, dtype=torch.int32, device="cuda"), c.k, c.v, H, KVH, 64, c.kp, c.vp)
+  q = qkv[:, start:, :H * 64].reshape(2, S, H, 64)
+  with torch.no_grad():
+    out = ops.attn_prefill(q, c.k, c.v, start, S, c.kp, c.vp).double()
+  k, v = (t.double().repeat_interleave(H // KVH, 1) for t in (c.k, c.v))
+  s = q.double().transpose(1, 2) @ k.transpose(-1, -2) * 64 ** -0.5
+  later = torch.arange(start + S, device="cuda")[None] > torch.arange(start, start + S, device="cuda")[:, None]
+  p = s.masked_fill(later, -torch.inf).softmax(-1)
+  ref, size = (p @ v).transpose(1, 2), (p @ v.abs()).transpose(1, 2)
+  assert bool(((out - ref).abs() <= size * 2.0 ** -7 * 1.05 + ref.abs() * 2.0 ** -8 + 1e-6).all())

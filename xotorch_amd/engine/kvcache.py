@@ -4,11 +4,11 @@ Standard layout [B, KVH, T, hd]: each (b, kv_head) has T contiguous rows of
 hd elements (256 B at hd=128 bf16) — prefill attention (sdpa) and the VALU
 decode kernel stream rows with coalesced 16 B/lane loads.
 
-MFMA layout (GPU, hd=128): a second copy of K and V pre-shuffled into
+MFMA layout (GPU, hd 64 or 128): a second copy of K and V pre-shuffled into
 v_mfma_f32_16x16x32_bf16 B-fragment order so the MFMA flash-decoding kernel
 streams the cache with fully-coalesced 1 KB wave loads:
-  K_packed [B, KVH, T32/16, 4, 64, 8]   (16-position x 32-hd-chunk tiles)
-  V_packed [B, KVH, 8, T32/32, 64, 8]   (32-position x 16-hd-column tiles)
+  K_packed [B, KVH, T32/16, hd/32, 64, 8]   (16-position x 32-hd-chunk tiles)
+  V_packed [B, KVH, hd/16, T32/32, 64, 8]   (32-position x 16-hd-column tiles)
 (T32 = capacity rounded up to 32; both copies are appended by the fused
 rope_qkv_append kernel.)  The reference's equivalent is torchtune's per-layer
 cache setup (/root/reference/xotorch/inference/torch/sharded_inference_engine.py:71-82).
@@ -24,7 +24,7 @@ import torch
 class LayerKV(NamedTuple):
   k: torch.Tensor
   v: torch.Tensor
-  kp: Optional[torch.Tensor] = None  # MFMA-packed K (cuda, hd=128; bf16 or e4m3 bytes)
+  kp: Optional[torch.Tensor] = None  # MFMA-packed K (cuda, hd 64 or 128; bf16 or (128) e4m3 bytes)
   vp: Optional[torch.Tensor] = None  # MFMA-packed V
   ksc: Optional[torch.Tensor] = None  # fp8 mode: per-row K scales [B, KVH, T32]
   vsc: Optional[torch.Tensor] = None  # fp8 mode: per-row V scales
@@ -33,7 +33,7 @@ class LayerKV(NamedTuple):
 def _want_packed(device: str, head_dim: int, dtype: torch.dtype) -> bool:
   return (
     str(device).startswith("cuda")
-    and head_dim == 128
+    and head_dim in (64, 128)
     and dtype == torch.bfloat16
     and os.getenv("XOT_MFMA_ATTN", "1") == "1"
   )
@@ -53,7 +53,7 @@ class ShardKVCache:
     self.caches: List[LayerKV] = []
     vd = v_dim if v_dim is not None else head_dim
     packed = _want_packed(device, head_dim, dtype) and vd == head_dim
-    fp8_kv = packed and os.getenv("XOT_FP8_KV", "0") == "1"
+    fp8_kv = packed and head_dim == 128 and os.getenv("XOT_FP8_KV", "0") == "1"
     # MLA latent cache (k = 512-dim latent, v = 64-dim roped shared key,
     # one kv "head"): fragment-packed copies for the absorbed-MQA MFMA
     # decode kernel (18 qk chunks / 32 pv groups — hip_ops.hip MLA section)
@@ -75,8 +75,8 @@ class ShardKVCache:
         vsc = torch.ones(batch, n_kv_heads, t32, dtype=torch.float32, device=device)
         self.caches.append(LayerKV(k, v, kp, vp, ksc, vsc))
       elif packed:
-        kp = torch.zeros(batch, n_kv_heads, t32 // 16, 4, 64, 8, dtype=dtype, device=device)
-        vp = torch.zeros(batch, n_kv_heads, 8, t32 // 32, 64, 8, dtype=dtype, device=device)
+        kp = torch.zeros(batch, n_kv_heads, t32 // 16, head_dim // 32, 64, 8, dtype=dtype, device=device)
+        vp = torch.zeros(batch, n_kv_heads, head_dim // 16, t32 // 32, 64, 8, dtype=dtype, device=device)
         self.caches.append(LayerKV(k, v, kp, vp))
       elif mla_packed and os.getenv("XOT_FP8_KV", "0") == "1":
         kp = torch.zeros(batch, t32 // 16, 18, 64, 8, dtype=torch.uint8, device=device)

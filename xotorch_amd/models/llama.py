@@ -242,12 +242,16 @@ class Attention(nn.Module):
     cfg = self.cfg
     H, hd = cfg.n_heads, cfg.head_dim
     k_cache, v_cache = kv[0], kv[1]
-    kp = kv[2] if len(kv) > 2 else None  # MFMA-packed cache copies (GPU, hd=128)
+    kp = kv[2] if len(kv) > 2 else None  # MFMA-packed cache copies (GPU, hd 64 or 128)
     vp = kv[3] if len(kv) > 3 else None
     ksc = kv[4] if len(kv) > 4 else None  # fp8-KV mode scales
     vsc = kv[5] if len(kv) > 5 else None
     qn = self.q_norm if cfg.qk_norm else None
     kn = self.k_norm if cfg.qk_norm else None
+    if is_decode and ops.decode_attends(qkv, H, cfg.n_kv_heads, hd, kp, qn, kn):
+      sl = seq_lens if seq_lens is not None else start_pos + 1
+      return ops.decode_attend(qkv, cos, sin, positions, sl, k_cache, v_cache, kp, vp, H, cfg.n_kv_heads,
+                               qn, kn, cfg.norm_eps)
     ops.rope_qkv_append(qkv, cos, sin, positions, k_cache, v_cache, H, cfg.n_kv_heads, hd, kp, vp,
                         qn, kn, cfg.norm_eps, ksc, vsc)
     q = qkv[:, :, : H * hd].view(B, S, H, hd)  # strided view; kernels accept it

@@ -98,7 +98,7 @@ def rope_qkv_append(qkv, cos, sin, positions, k_cache, v_cache, n_heads: int, n_
 
 def attn_prefill(q, k_cache, v_cache, start_pos: int, s_len: int, kp=None, vp=None,
                  scale=None, softcap: float = 0.0, window: int = 0):
-  if q.is_cuda and q.dtype == torch.bfloat16 and kp is not None and q.shape[3] == 128 \
+  if q.is_cuda and q.dtype == torch.bfloat16 and kp is not None and q.shape[3] in (64, 128) \
      and kp.dtype == torch.bfloat16 \
      and os.getenv("XOT_MFMA_ATTN", "1") == "1" and _use_hip(q):
     # causal flash-forward on matrix cores, streaming the MFMA-packed cache;
@@ -134,12 +134,42 @@ def attn_decode(q, k_cache, v_cache, seq_len, kp=None, vp=None,
     if not isinstance(seq_len, torch.Tensor):
       seq_len = torch.full((q.shape[0],), int(seq_len), dtype=torch.int32, device=q.device)
     rep = q.shape[2] // k_cache.shape[1]
-    if kp is not None and rep <= 16 and os.getenv("XOT_MFMA_ATTN", "1") == "1":
+    if kp is not None and rep <= 16 and q.shape[3] == 128 and os.getenv("XOT_MFMA_ATTN", "1") == "1":
       return _hip.attn_decode_mfma(q, kp, vp, seq_len, k_cache.shape[2],
                                    scale or 0.0, softcap, window, k_scale, v_scale)
     if not softcap and not window and scale is None:
       return _hip.attn_decode(q, k_cache, v_cache, seq_len)
   return torch_ref.attn_decode(q, k_cache, v_cache, seq_len, scale, softcap, window)
+
+
+_decode_ext = None
+
+
+def _decode():
+  global _decode_ext
+  if _decode_ext is None:
+    import importlib
+    _decode_ext = importlib.import_module("xotorch_amd.ops._hip_decode")
+  return _decode_ext
+
+
+def decode_attends(qkv, n_heads: int, n_kv_heads: int, head_dim: int, kp, *norms) -> bool:
+  """Whether decode_attend takes this step: one token a row, a packed bf16 cache of
+  head dim 64 or 128, up to 16 heads on a key head."""
+  return (qkv.is_cuda and qkv.dtype == torch.bfloat16 and qkv.dim() == 3 and qkv.shape[1] == 1 and qkv.is_contiguous()
+          and qkv.data_ptr() % 16 == 0 and kp is not None and kp.dtype == torch.bfloat16 and head_dim in (64, 128)
+          and n_heads <= 16 * n_kv_heads and os.getenv("XOT_MFMA_ATTN", "1") == "1"
+          and all(n is None or n.dtype == torch.bfloat16 for n in norms) and _use_hip(qkv))
+
+
+def decode_attend(qkv, cos, sin, positions, seq_len, k_cache, v_cache, kp, vp, n_heads: int, n_kv_heads: int,
+                  q_norm=None, k_norm=None, norm_eps: float = 1e-6):
+  """rope_qkv_append and attn_decode in one: [B, 1, (H+2KVH)*hd] -> [B, 1, H*hd].
+  qkv is left as projected."""
+  if not isinstance(seq_len, torch.Tensor):
+    seq_len = torch.full((qkv.shape[0],), int(seq_len), dtype=torch.int32, device=qkv.device)
+  return _decode().decode_attend(qkv, cos, sin, positions, seq_len, k_cache, v_cache, kp, vp, n_heads, n_kv_heads,
+                                 q_norm, k_norm, norm_eps)
 
 
 def swiglu(gate, up):

@@ -126,11 +126,11 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(
 // cos/sin tables fp32 [maxT, hd/2].
 // ---------------------------------------------------------------------------
 
-// When the MFMA-packed cache copies exist (kpc/vpc non-null, hd == 128) the
+// When the MFMA-packed cache copies exist (kpc/vpc non-null, hd 64 or 128) the
 // same kernel also appends into them (decode attention then streams the
 // cache as coalesced v_mfma_f32_16x16x32_bf16 B-fragments):
-//   K_packed [B,KVH][T32/16 tile][4 hd-chunk][64 lane][8]  lane=(hd&31)/8*16 + (pos&15)
-//   V_packed [B,KVH][8 hd-group][T32/32 tile][64 lane][8]  lane=((pos&31)>>3)*16 + (hd&15)
+//   K_packed [B,KVH][T32/16 tile][hd/32 chunk][64 lane][8]  lane=(hd&31)/8*16 + (pos&15)
+//   V_packed [B,KVH][hd/16 group][T32/32 tile][64 lane][8]  lane=((pos&31)>>3)*16 + (hd&15)
 // Optional qwen3 per-head q/k RMSNorm (qn/kn weights [hd], fused before the
 // rotation): the slot's wave reduces sum-of-squares over the head row with
 // shfl_xor, then scales while rotating.
@@ -213,7 +213,7 @@ __global__ __launch_bounds__(256) void rope_qkv_append_kernel(
       if (kpc) {
         // packed K: element for hd-dim d at
         //   [(b*KVH+h)][pos>>4][d>>5][((d&31)>>3)*16 + (pos&15)][d&7]
-        const size_t base = ((size_t)(b * KVH + h) * (T32 >> 4) + (pos >> 4)) * 2048;
+        const size_t base = ((size_t)(b * KVH + h) * (T32 >> 4) + (pos >> 4)) * (size_t)(hd >> 5) * 512;
         const int d1 = lane, d2 = lane + hd2;
         kpc[base + (size_t)(d1 >> 5) * 512 + (((d1 & 31) >> 3) * 16 + (pos & 15)) * 8 + (d1 & 7)] = f2b(f1);
         kpc[base + (size_t)(d2 >> 5) * 512 + (((d2 & 31) >> 3) * 16 + (pos & 15)) * 8 + (d2 & 7)] = f2b(f2v);
@@ -244,7 +244,7 @@ __global__ __launch_bounds__(256) void rope_qkv_append_kernel(
       // packed V: element for hd-dim d at
       //   [(b*KVH+h)][d>>4][pos>>5][((pos&31)>>3)*16 + (d&15)][pos&7]
       const int tp = pos >> 5, qt = (pos & 31) >> 3, j = pos & 7;
-      const size_t gbase = (size_t)(b * KVH + h) * 8;
+      const size_t gbase = (size_t)(b * KVH + h) * (hd >> 4);
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         const int d = lane * 2 + e;
@@ -690,7 +690,7 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// MFMA flash-forward prefill attention (hd = 128, causal, GQA) over the packed
+// MFMA flash-forward prefill attention (hd 64 or 128, causal, GQA) over the packed
 // cache (reference: torchtune MultiHeadAttention prefill, general_mha.py:218-226).
 //
 // What bounds it are the matrix cores and, as much, the exponentials. A block owns
@@ -713,13 +713,13 @@ DEVINL floatx4 mma16(const bf16x8& a, const bf16x8& b, floatx4 c) {
 }
 
 // What the cache holds per 32 positions and key head: K two tiles of 16 positions
-// [4 chunks of 32 dims][64 lanes][8], lane = (dim % 32) / 8 * 16 + position % 16;
-// V [8 groups of 16 dims], each [64 lanes][8] with lane = (position % 32) / 8 * 16 +
+// [chunks of 32 dims][64 lanes][8], lane = (dim % 32) / 8 * 16 + position % 16;
+// V [groups of 16 dims], each [64 lanes][8] with lane = (position % 32) / 8 * 16 +
 // dim % 16, groups T32 * 16 apart.
 struct FlashArgs {
   const unsigned short *q, *k, *v;
   unsigned short* out;
-  float *part, *ml;  // [rows][splits][128] and [rows][splits][2] where the keys are split
+  float *part, *ml;  // [rows][splits][HD] and [rows][splits][2] where the keys are split
   int S, H, KVH, T32, start, blocks, splits, window;
   long long q_b, q_s;  // strides of a batch row and of a token
   float scale, cap;    // scale times log2 e, or plain with a cap
@@ -728,7 +728,10 @@ struct FlashArgs {
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(1))) const void glb_void;
 
-constexpr int KSUB = 8192 + 128, SUB = KSUB + 8192, STAGE = 2 * SUB;  // bytes of LDS: keys, 32 positions, 64
+// bytes of LDS: keys of 32 positions (their halves 64 bytes apart), 32 positions, 64
+template <int HD> struct FlashLds {
+  static constexpr int KSUB = HD * 64 + 128, SUB = KSUB + HD * 64, STAGE = 2 * SUB;
+};
 
 // 8 fragments from LDS, and the wait for them
 #define READ8(F, A, O0, O1, O2, O3, O4, O5, O6, O7)                                                                    \
@@ -737,6 +740,12 @@ constexpr int KSUB = 8192 + 128, SUB = KSUB + 8192, STAGE = 2 * SUB;  // bytes o
                "\n\tds_read_b128 %5, %8 offset:" #O5 "\n\tds_read_b128 %6, %8 offset:" #O6                             \
                "\n\tds_read_b128 %7, %8 offset:" #O7 "\n\ts_waitcnt lgkmcnt(0)"                                        \
                : "=&v"(F[0]), "=&v"(F[1]), "=&v"(F[2]), "=&v"(F[3]), "=&v"(F[4]), "=&v"(F[5]), "=&v"(F[6]), "=&v"(F[7]) \
+               : "v"(A))
+
+#define READ4(F, A, O0, O1, O2, O3)                                                                                    \
+  asm volatile("ds_read_b128 %0, %4 offset:" #O0 "\n\tds_read_b128 %1, %4 offset:" #O1 "\n\tds_read_b128 %2, %4 offset:" #O2 \
+               "\n\tds_read_b128 %3, %4 offset:" #O3 "\n\ts_waitcnt lgkmcnt(0)"                                       \
+               : "=&v"(F[0]), "=&v"(F[1]), "=&v"(F[2]), "=&v"(F[3])                                                    \
                : "v"(A))
 
 // maximum over the four lanes that hold a query's scores
@@ -748,9 +757,10 @@ DEVINL float quad_max(float v) {
 }
 
 // SIDE: capped scores and a sliding window
-template <bool SIDE>
+template <int HD, bool SIDE>
 __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(FlashArgs a) {
   constexpr int QT = 2;  // tiles of 16 query rows a wave
+  constexpr int KC = HD / 32, VG = HD / 16, KSUB = FlashLds<HD>::KSUB, SUB = FlashLds<HD>::SUB, STAGE = FlashLds<HD>::STAGE;
   extern __shared__ __attribute__((aligned(16))) char lds[];  // [2][STAGE]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int col = lane & 15, quad = lane >> 4;
@@ -760,8 +770,8 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(FlashArgs a) {
   const int block = a.blocks - 1 - rest / a.splits;
   const int b = bh / a.KVH, kvh = bh % a.KVH;
   const int rows = a.S * rep, row0 = block * 128 + wave * QT * 16;
-  const char* kb = (const char*)(a.k + (size_t)bh * a.T32 * 128);
-  const char* vb = (const char*)(a.v + (size_t)bh * a.T32 * 128);
+  const char* kb = (const char*)(a.k + (size_t)bh * a.T32 * HD);
+  const char* vb = (const char*)(a.v + (size_t)bh * a.T32 * HD);
   // positions that this block reads: whole tiles of 64, a part of them per split
   const int last = a.start + (min(block * 128 + 127, rows - 1)) / rep;  // the last one seen
   const int low = SIDE && a.window > 0 ? max(0, a.start + block * 128 / rep - a.window + 1) : 0;
@@ -769,15 +779,15 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(FlashArgs a) {
   const int t0 = tile0 + count * split / a.splits, t1 = tile0 + count * (split + 1) / a.splits;
   const int subs = (last >> 5) + 1;  // tiles of 32 that hold something
 
-  bf16x8 qf[QT][4];
+  bf16x8 qf[QT][KC];
   int pos[QT];  // of this lane's query
 #pragma unroll
   for (int t = 0; t < QT; ++t) {
     const int r = min(row0 + t * 16 + col, rows - 1), s = r / rep;
     pos[t] = a.start + s;
-    const unsigned short* q = a.q + (size_t)b * a.q_b + (size_t)s * a.q_s + (size_t)(kvh * rep + r % rep) * 128 + quad * 8;
+    const unsigned short* q = a.q + (size_t)b * a.q_b + (size_t)s * a.q_s + (size_t)(kvh * rep + r % rep) * HD + quad * 8;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) qf[t][c] = *(const bf16x8*)(q + c * 32);
+    for (int c = 0; c < KC; ++c) qf[t][c] = *(const bf16x8*)(q + c * 32);
   }
   const int first_pos = a.start + min(row0, rows - 1) / rep;  // of the wave's first row
   const int last_pos = a.start + min(row0 + QT * 16 - 1, rows - 1) / rep;
@@ -788,19 +798,19 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(FlashArgs a) {
     char* dst = lds + (tile & 1) * STAGE + (wave >> 1) * SUB;
     if (wave & 1) {
 #pragma unroll
-      for (int g = 0; g < 8; ++g)
+      for (int g = 0; g < VG; ++g)
         __builtin_amdgcn_global_load_lds((glb_void*)(vb + ((size_t)g * (a.T32 >> 5) + sub) * 1024 + lane * 16),
                                          (lds_void*)(dst + KSUB + g * 1024), 16, 0, 0);
     } else {
 #pragma unroll
-      for (int c = 0; c < 8; ++c)  // the second 16 positions 64 bytes further: their rows fall on other banks
-        __builtin_amdgcn_global_load_lds((glb_void*)(kb + (size_t)sub * 8192 + c * 1024 + lane * 16),
-                                         (lds_void*)(dst + c * 1024 + (c >> 2) * 64), 16, 0, 0);
+      for (int c = 0; c < 2 * KC; ++c)  // the second 16 positions 64 bytes further: their rows fall on other banks
+        __builtin_amdgcn_global_load_lds((glb_void*)(kb + (size_t)sub * (HD * 64) + c * 1024 + lane * 16),
+                                         (lds_void*)(dst + c * 1024 + c / KC * 64), 16, 0, 0);
     }
   };
 
   float m[QT];
-  floatx4 o[QT][8], l[QT];  // l: the same sum in all four
+  floatx4 o[QT][VG], l[QT];  // l: the same sum in all four
   bf16x8 ones;
 #pragma unroll
   for (int i = 0; i < 8; ++i) ones[i] = (__bf16)1.f;
@@ -809,12 +819,12 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(FlashArgs a) {
     m[t] = -1e30f;
     l[t] = (floatx4)(0.f);
 #pragma unroll
-    for (int g = 0; g < 8; ++g) o[t][g] = (floatx4)(0.f);
+    for (int g = 0; g < VG; ++g) o[t][g] = (floatx4)(0.f);
   }
   // key rows of the two products of 16: row i is position i / 4 * 8 + i % 4, and 4 more
   const int p = (col >> 2) * 8 + (col & 3);
   const unsigned base = (unsigned)(size_t)(lds_void*)lds;
-  const unsigned klane = base + (p >> 4) * (4096 + 64) + (quad * 16 + (p & 15)) * 16, vlane = base + KSUB + lane * 16;
+  const unsigned klane = base + (p >> 4) * (HD * 32 + 64) + (quad * 16 + (p & 15)) * 16, vlane = base + KSUB + lane * 16;
   if (t0 < t1) stage(t0);
   for (int tile = t0; tile < t1; ++tile) {
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
@@ -825,8 +835,9 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(FlashArgs a) {
       if (tile * 2 + u >= subs || p0 > last_pos) continue;
       if (SIDE && a.window > 0 && p0 + 31 <= first_pos - a.window) continue;
       const unsigned at = (tile & 1) * STAGE + u * SUB;
-      bf16x8 kf[8];
-      READ8(kf, klane + at, 0, 64, 1024, 1088, 2048, 2112, 3072, 3136);
+      bf16x8 kf[2 * KC];
+      if constexpr (HD == 128) READ8(kf, klane + at, 0, 64, 1024, 1088, 2048, 2112, 3072, 3136);
+      else READ4(kf, klane + at, 0, 64, 1024, 1088);
       floatx4 sc[QT][2];
 #pragma unroll
       for (int t = 0; t < QT; ++t)
@@ -834,7 +845,7 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(FlashArgs a) {
         for (int hf = 0; hf < 2; ++hf) {
           sc[t][hf] = (floatx4)(0.f);
 #pragma unroll
-          for (int c = 0; c < 4; ++c) sc[t][hf] = mma16(kf[c * 2 + hf], qf[t][c], sc[t][hf]);
+          for (int c = 0; c < KC; ++c) sc[t][hf] = mma16(kf[c * 2 + hf], qf[t][c], sc[t][hf]);
         }
       const bool edge = p0 + 31 > first_pos || (SIDE && a.window > 0 && p0 <= last_pos - a.window);
       bf16x8 pf[QT];
@@ -862,16 +873,17 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(FlashArgs a) {
           m[t] = top;
           l[t] *= f;
 #pragma unroll
-          for (int g = 0; g < 8; ++g) o[t][g] *= f;
+          for (int g = 0; g < VG; ++g) o[t][g] *= f;
         }
 #pragma unroll
         for (int i = 0; i < 8; ++i) pf[t][i] = (__bf16)__builtin_amdgcn_exp2f(v[i] - m[t]);
         l[t] = mma16(ones, pf[t], l[t]);
       }
-      bf16x8 vf[8];
-      READ8(vf, vlane + at, 0, 1024, 2048, 3072, 4096, 5120, 6144, 7168);
+      bf16x8 vf[VG];
+      if constexpr (HD == 128) READ8(vf, vlane + at, 0, 1024, 2048, 3072, 4096, 5120, 6144, 7168);
+      else READ4(vf, vlane + at, 0, 1024, 2048, 3072);
 #pragma unroll
-      for (int g = 0; g < 8; ++g)
+      for (int g = 0; g < VG; ++g)
 #pragma unroll
         for (int t = 0; t < QT; ++t) o[t][g] = mma16(vf[g], pf[t], o[t][g]);
     }
@@ -884,7 +896,7 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(FlashArgs a) {
     if (a.splits > 1) {
       const size_t i = ((size_t)bh * rows + r) * a.splits + split;
 #pragma unroll
-      for (int g = 0; g < 8; ++g) *(floatx4*)(a.part + i * 128 + g * 16 + quad * 4) = o[t][g];
+      for (int g = 0; g < VG; ++g) *(floatx4*)(a.part + i * HD + g * 16 + quad * 4) = o[t][g];
       if (quad == 0) {
         a.ml[i * 2] = m[t];
         a.ml[i * 2 + 1] = sum;
@@ -892,9 +904,9 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(FlashArgs a) {
       continue;
     }
     const float f = sum > 0.f ? 1.f / sum : 0.f;
-    unsigned short* dst = a.out + (((size_t)b * a.S + r / rep) * a.H + kvh * rep + r % rep) * 128 + quad * 4;
+    unsigned short* dst = a.out + (((size_t)b * a.S + r / rep) * a.H + kvh * rep + r % rep) * HD + quad * 4;
 #pragma unroll
-    for (int g = 0; g < 8; ++g) {
+    for (int g = 0; g < VG; ++g) {
       ushort4_t v;
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[i] = f2b(o[t][g][i] * f);
@@ -905,6 +917,7 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(FlashArgs a) {
 
 // A wave a row of [B, S, H]: the splits' parts, weighed by how far their maxima lie
 // below the largest.
+template <int HD>
 __global__ __launch_bounds__(256) void flash_merge_kernel(FlashArgs a, int total) {
   const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (i >= total) return;
@@ -916,13 +929,12 @@ __global__ __launch_bounds__(256) void flash_merge_kernel(FlashArgs a, int total
   for (int k = 0; k < a.splits; ++k) {
     const float f = __builtin_amdgcn_exp2f(ml[k * 2] - top);
     sum += f * ml[k * 2 + 1];
-    const float2 v = *(const float2*)(a.part + (row * a.splits + k) * 128 + lane * 2);
-    o[0] += f * v.x;
-    o[1] += f * v.y;
+#pragma unroll
+    for (int i = 0; i < HD / 64; ++i) o[i] += f * a.part[(row * a.splits + k) * HD + i * 64 + lane];
   }
   const float f = sum > 0.f ? 1.f / sum : 0.f;
-  const unsigned two = f2b(o[0] * f) | (unsigned)f2b(o[1] * f) << 16;
-  *(unsigned*)(a.out + (size_t)i * 128 + lane * 2) = two;
+#pragma unroll
+  for (int d = 0; d < HD / 64; ++d) a.out[(size_t)i * HD + d * 64 + lane] = f2b(o[d] * f);
 }
 
 // layout probe for tests: one v_mfma_f32_16x16x32_bf16, row-major inputs
@@ -2340,7 +2352,7 @@ void rope_qkv_append(torch::Tensor qkv, torch::Tensor cos, torch::Tensor sin,
   float* svp = nullptr;
   int T32 = 0;
   if (kp.has_value() && vp.has_value()) {
-    CHK(hd == 128 && kp->is_contiguous() && vp->is_contiguous());
+    CHK((hd == 128 || (hd == 64 && kp->dtype() != torch::kUInt8)) && kp->is_contiguous() && vp->is_contiguous());
     T32 = (int)kp->size(2) * 16;
     if (kp->dtype() == torch::kUInt8) {
       // fp8 packed mode: per-row e4m3 scales required
@@ -2486,13 +2498,15 @@ torch::Tensor attn_decode_mfma(torch::Tensor q, torch::Tensor kp, torch::Tensor 
   return out;
 }
 
-// q: [B, S, H, 128], heads contiguous; k, v: the packed cache, which holds positions
-// [0, start + S). window 0: none; cap 0: none; scale 0: 1 / sqrt(128).
+// q: [B, S, H, 64 or 128], heads contiguous; k, v: the packed cache, which holds positions
+// [0, start + S). window 0: none; cap 0: none; scale 0: 1 / sqrt of the head dim.
 torch::Tensor attn_prefill_mfma(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                                 int64_t start, double scale, double cap,
                                 int64_t window) {
   CHK(q.is_cuda() && q.scalar_type() == torch::kBFloat16 && q.dim() == 4);
-  CHK(q.size(3) == 128 && q.stride(3) == 1 && q.stride(2) == 128);
+  const int HD = (int)q.size(3);
+  TORCH_CHECK(HD == 64 || HD == 128, "attn_prefill_mfma: head_dim must be 64 or 128, got ", HD);
+  CHK(q.stride(3) == 1 && q.stride(2) == HD);
   CHK(k.is_cuda() && v.is_cuda() && k.scalar_type() == torch::kBFloat16 && v.scalar_type() == torch::kBFloat16);
   CHK(k.is_contiguous() && v.is_contiguous());
   CHK((((size_t)k.data_ptr() | (size_t)v.data_ptr()) & 15) == 0);
@@ -2502,15 +2516,15 @@ torch::Tensor attn_prefill_mfma(torch::Tensor q, torch::Tensor k, torch::Tensor 
   a.H = (int)q.size(2);
   a.KVH = (int)k.size(1);
   a.T32 = (int)k.size(2) * 16;
-  CHK(k.size(0) >= B && v.size(0) >= B && a.KVH > 0 && a.H % a.KVH == 0 && k.numel() == k.size(0) * a.KVH * a.T32 * 128);
-  CHK(v.numel() == v.size(0) * a.KVH * a.T32 * 128 && a.T32 % 32 == 0 && start >= 0 && start + a.S <= a.T32);
-  auto out = torch::empty({B, a.S, a.H, 128}, q.options());
+  CHK(k.size(0) >= B && v.size(0) >= B && a.KVH > 0 && a.H % a.KVH == 0 && k.numel() == k.size(0) * a.KVH * a.T32 * HD);
+  CHK(v.numel() == v.size(0) * a.KVH * a.T32 * HD && a.T32 % 32 == 0 && start >= 0 && start + a.S <= a.T32);
+  auto out = torch::empty({B, a.S, a.H, HD}, q.options());
   if (out.numel() == 0) return out;
   a.start = (int)start;
   a.window = (int)window;
   a.cap = (float)cap;
   const bool side = cap > 0.0 || window > 0;
-  a.scale = (scale > 0.0 ? (float)scale : 0.08838834764831845f) * (cap > 0.0 ? 1.f : 1.4426950408889634f);
+  a.scale = (scale > 0.0 ? (float)scale : 1.f / sqrtf((float)HD)) * (cap > 0.0 ? 1.f : 1.4426950408889634f);
   a.q = (const unsigned short*)q.data_ptr();
   a.k = (const unsigned short*)k.data_ptr();
   a.v = (const unsigned short*)v.data_ptr();
@@ -2528,22 +2542,30 @@ torch::Tensor attn_prefill_mfma(torch::Tensor q, torch::Tensor k, torch::Tensor 
   torch::Tensor part, ml;
   if (a.splits > 1) {
     const auto opts = q.options().dtype(torch::kFloat32);
-    part = torch::empty({B * a.KVH * rows, a.splits, 128}, opts);
+    part = torch::empty({B * a.KVH * rows, a.splits, HD}, opts);
     ml = torch::empty({B * a.KVH * rows, a.splits, 2}, opts);
     a.part = part.data_ptr<float>();
     a.ml = ml.data_ptr<float>();
   }
   const dim3 grid((unsigned)(whole * a.splits));
   auto run = [&](auto kernel) {
-    const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * STAGE);
+    const int lds = 2 * (HD == 128 ? FlashLds<128>::STAGE : FlashLds<64>::STAGE);
+    const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     TORCH_CHECK(e == hipSuccess, "no LDS for attention tiles");
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 2 * STAGE, cur_stream(), a);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), lds, cur_stream(), a);
   };
-  if (side) run(flash_prefill_kernel<true>);
-  else run(flash_prefill_kernel<false>);
+  if (HD == 128) {
+    if (side) run(flash_prefill_kernel<128, true>);
+    else run(flash_prefill_kernel<128, false>);
+  } else {
+    if (side) run(flash_prefill_kernel<64, true>);
+    else run(flash_prefill_kernel<64, false>);
+  }
   if (a.splits > 1) {
     const int64_t total = (int64_t)B * a.S * a.H;
-    hipLaunchKernelGGL(flash_merge_kernel, dim3((unsigned)((total + 3) / 4)), dim3(256), 0, cur_stream(), a, (int)total);
+    const dim3 rows4((unsigned)((total + 3) / 4));
+    if (HD == 128) hipLaunchKernelGGL((flash_merge_kernel<128>), rows4, dim3(256), 0, cur_stream(), a, (int)total);
+    else hipLaunchKernelGGL((flash_merge_kernel<64>), rows4, dim3(256), 0, cur_stream(), a, (int)total);
   }
   return out;
 }

@@ -127,7 +127,7 @@ class RingPipeline:
           self.M * 2 * shards[rank].get_layer_count() * mb_batch * self.cfg.n_kv_heads
           * self.total_len * self.cfg.head_dim * (2 if dtype == torch.bfloat16 else 4)
         )
-      if self.cfg.head_dim == 128 and dtype == torch.bfloat16 \
+      if self.cfg.head_dim in (64, 128) and dtype == torch.bfloat16 \
          and os.getenv("XOT_MFMA_ATTN", "1") == "1":
         kv_bytes *= 2  # the MFMA-packed cache copies double KV residency
       torch.cuda.empty_cache()  # release init-time cached blocks so the
