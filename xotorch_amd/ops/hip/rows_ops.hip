@@ -1,4 +1,4 @@
-// Products of a few rows (decode steps of up to 4 sequences, prompts of up to 4
+// Products of one or two rows (decode steps of so many sequences, prompts of so many
 // tokens) with bf16 weights as they lie in the checkpoint, [N, K] row-major:
 //   y = x W^T + bias, y = norm(x) W^T + bias, y = silu(norm(x) Wg^T) norm(x) Wu^T,
 //   y = r + x W^T.
@@ -9,7 +9,7 @@
 // launches around it; so the norm before and the activation or the residual sum
 // after a product belong to its kernel. A wave takes R weight rows at a time, 512
 // numbers of each (one load of 1 KB a row, whole lines) two steps deep, and
-// multiplies pairs of bf16 into fp32 sums; matrix instructions would have 12 or more
+// multiplies pairs of bf16 into fp32 sums; matrix instructions would have 14 or more
 // columns idle and want the weights in another order. Waves of a block share a row
 // group's k where there are few rows. Weights are read once: non-temporal.
 // One row, against the library (us, TB/s): [128256, 2048] 75 (7.0) and 113,
@@ -227,15 +227,12 @@ __global__ __launch_bounds__(256) void rows_kernel(RowsArgs a) {
 // ===========================================================================
 
 // Waves that share a row group: as many as it takes to have some 2000 waves that
-// each keep a few KB in flight, fewer where the sums over the wave (COUNT
-// exchanges a group and wave) and the reads of x would outweigh it. Measured at
-// [N, K] of this file's first line, us for 1, 2, 4 waves a group (library: 11-12):
-//   m 1: [2048, 8192] 10.8, 8.3, 7.6; [3584, 18944] 23.9, 23.6, 24.1; [128256, 2048] 86, 75, 74
-//   m 4: [2048, 8192] 14.0, 10.8, 11.1; [8192, 8192] 28.7, 27.7, 31.1; [128256, 2048] 109, 155, 259
-// With a norm blocks also read all of x first, so that there are at most 512 or
-// 1024 of them, which go on to further groups:
-//   m 1: [3072, 2048] 6.1, 5.5, 5.5; [37888, 3584] 43.0, 42.1, 43.5
-//   m 4: [3072, 2048] 9.9, 9.8, 12.3; [37888, 3584] 53.7, 59.9, 84.8
+// each keep a few KB in flight, fewer where the sums over the wave (4 or 8 exchanges
+// a group and wave) would outweigh it. Measured, us for 1, 2, 4 waves a group and one
+// row: [2048, 8192] 10.8, 8.3, 7.6; [3584, 18944] 23.9, 23.6, 24.1; two rows, [128256,
+// 2048] 88, 77, 89. With a norm blocks also read all of x first, so that there are at
+// most 512 or 1024 of them, which go on to further groups: one row, [3072, 2048] 6.1,
+// 5.5, 5.5; [37888, 3584] 43.0, 42.1, 43.5.
 template <int M, int KS, int SRC, int END>
 static void launch_rows(const RowsArgs& a, int most) {
   const int lds = SRC == PLAIN_X ? 0 : a.m * ((a.K + 511) / 512) * 1024;
@@ -251,11 +248,8 @@ static void launch_rows(const RowsArgs& a, int most) {
 template <int M, int SRC, int END>
 static void run_m(const RowsArgs& a) {
   if constexpr (SRC != PLAIN_X) {
-    if (M == 1 || (M == 2 && END == STORE)) launch_rows<M, 2, SRC, END>(a, END == STORE ? 1024 : 512);
+    if (M == 1 || END == STORE) launch_rows<M, 2, SRC, END>(a, END == STORE ? 1024 : 512);
     else launch_rows<M, 1, SRC, END>(a, 512);
-  } else if (M == 4) {
-    if (a.groups <= 2048) launch_rows<M, 2, SRC, END>(a, INT_MAX);
-    else launch_rows<M, 1, SRC, END>(a, INT_MAX);
   } else {
     if (a.groups <= 4096 && a.K > 1536) launch_rows<M, 4, SRC, END>(a, INT_MAX);
     else launch_rows<M, 2, SRC, END>(a, INT_MAX);
@@ -267,8 +261,7 @@ static void run_rows(RowsArgs a) {
   const int per = END == GATED_STORE ? 2 : 4;
   a.groups = (a.N + per - 1) / per;
   if (a.m == 1) run_m<1, SRC, END>(a);
-  else if (a.m == 2) run_m<2, SRC, END>(a);
-  else run_m<4, SRC, END>(a);
+  else run_m<2, SRC, END>(a);
 }
 
 static RowsArgs rows_args(const Tensor& x, const Tensor& w, int64_t n) {
@@ -278,7 +271,7 @@ static RowsArgs rows_args(const Tensor& x, const Tensor& w, int64_t n) {
   a.K = (int)w.size(1);
   CHK(a.K > 0 && a.K % 8 == 0 && x.size(-1) == a.K);
   a.m = (int)(x.numel() / a.K);
-  CHK(a.m >= 1 && a.m <= 4 && n >= 1 && n <= INT_MAX / 16);
+  CHK(a.m >= 1 && a.m <= 2 && n >= 1 && n <= INT_MAX / 16);
   a.N = (int)n;
   CHK(((size_t)x.data_ptr() & 15) == 0 && ((size_t)w.data_ptr() & 15) == 0);
   a.x = x.data_ptr();

@@ -92,9 +92,9 @@ __global__ __launch_bounds__(256) void tile_kernel(TileArgs a) {
   const int m0 = mt * BM;
   const bf16_t *wsrc[Sh::WL], *xsrc[Sh::XL];
   const int sub = lane >> 3;
-  // GATED: 16 gate rows and the same 16 up rows in turn
+  // GATED: 8 gate rows and the same 8 up rows in turn
   auto weight_row = [&](int r) -> size_t {
-    if (END == GATED) return (size_t)min(tile * (BN / 2) + (r >> 5) * 16 + (r & 15), a.N - 1) + ((r >> 4) & 1 ? (size_t)a.N : 0);
+    if (END == GATED) return (size_t)min(tile * (BN / 2) + (r >> 4) * 8 + (r & 7), a.N - 1) + ((r >> 3) & 1 ? (size_t)a.N : 0);
     return min(tile * BN + r, a.N - 1);
   };
 #pragma unroll
@@ -154,14 +154,15 @@ __global__ __launch_bounds__(256) void tile_kernel(TileArgs a) {
 #pragma unroll
   for (int j = 0; j < C; ++j) {
     const int m = m0 + wx + j * 16 + col;
-    if (m >= a.m) continue;
     if (END == GATED) {
 #pragma unroll
-      for (int i = 0; i + 1 < R; i += 2) {
+      for (int i = 0; i < R; ++i) {
+        // lanes of quads 0 and 1 hold gates, those of 2 and 3 the products of up
         const int n = tile * (BN / 2) + (wr + i * 16) / 2 + quad * 4;
         float v[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = siluf(rounded(acc[i][j][r])) * rounded(acc[i + 1][j][r]);
+        for (int r = 0; r < 4; ++r) v[r] = siluf(rounded(acc[i][j][r])) * rounded(__shfl_xor(acc[i][j][r], 32));
+        if (m >= a.m || quad > 1) continue;
         bf16_t* dst = (bf16_t*)a.y + (size_t)m * a.N + n;
         if (n + 3 < a.N && (a.N & 3) == 0) st4(dst, v);
         else
@@ -170,6 +171,7 @@ __global__ __launch_bounds__(256) void tile_kernel(TileArgs a) {
             if (n + r < a.N) st(dst + r, v[r]);
       }
     } else {
+      if (m >= a.m) continue;
 #pragma unroll
       for (int i = 0; i < R; ++i) {
         const int n = tile * BN + wr + i * 16 + quad * 4;
@@ -201,9 +203,18 @@ __global__ __launch_bounds__(256) void tile_kernel(TileArgs a) {
 // what follows a product whose k was split: the parts' sums, in order
 // ---------------------------------------------------------------------------
 
+// four at a time on their way
 DEVINL floatx4 sum_parts(const float* p, size_t at, size_t stride, int splits) {
   floatx4 v = *(const floatx4*)(p + at);
-  for (int s = 1; s < splits; ++s) v += *(const floatx4*)(p + s * stride + at);
+  int s = 1;
+  for (; s + 3 < splits; s += 4) {
+    floatx4 q[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q[i] = *(const floatx4*)(p + (s + i) * stride + at);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v += q[i];
+  }
+  for (; s < splits; ++s) v += *(const floatx4*)(p + s * stride + at);
   return v;
 }
 
@@ -230,18 +241,20 @@ __global__ __launch_bounds__(256) void finish_kernel(const float* __restrict__ p
 }
 
 // h = x + bf16 of the sums (bf16), n = norm(x + ..) w. One block a row, which stays
-// in registers. ROUND: the norm reads h as it is stored.
-template <int NC>
-__global__ __launch_bounds__(256) void add_norm_kernel(const float* __restrict__ part, const bf16_t* __restrict__ x,
+// in registers; with few rows its chain of loads is all the time there is, so that
+// threads take 4 numbers (8 of rows over 4096). ROUND: the norm reads h as it is stored.
+// 8 rows of 3584, 8 parts: 5 us (11 with 256 threads and part after part).
+template <int NC, int THREADS>
+__global__ __launch_bounds__(THREADS) void add_norm_kernel(const float* __restrict__ part, const bf16_t* __restrict__ x,
                                                        const bf16_t* __restrict__ w, bf16_t* __restrict__ h,
                                                        bf16_t* __restrict__ n, int m, int D, int splits, float eps,
                                                        float add, bool round) {
-  __shared__ float red[4];
+  __shared__ float red[THREADS / 64];
   const size_t row = (size_t)blockIdx.x * D, stride = (size_t)m * D;
   float v[NC][4], ss = 0.f;
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    const int at = (c * 256 + threadIdx.x) * 4;
+    const int at = (c * THREADS + threadIdx.x) * 4;
     if (at >= D) break;
     const floatx4 p = sum_parts(part, row + at, stride, splits);
     ld4(x + row + at, v[c]);
@@ -255,10 +268,16 @@ __global__ __launch_bounds__(256) void add_norm_kernel(const float* __restrict__
     }
   }
   if (!w) return;
-  const float inv = rsqrtf(block_sum(ss, red) / (float)D + eps);
+  ss = wave_sum(ss);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < THREADS / 64; ++i) ss += red[i];
+  const float inv = rsqrtf(ss / (float)D + eps);
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    const int at = (c * 256 + threadIdx.x) * 4;
+    const int at = (c * THREADS + threadIdx.x) * 4;
     if (at >= D) break;
     float by[4];
     ld4(w + at, by);
@@ -292,10 +311,10 @@ static void launch_tile(const TileArgs& a) {
 template <int END>
 static void run_tile(const TileArgs& a) {
   const int rows = END == GATED ? 2 * a.N : a.N, units = (rows + 127) / 128 * a.splits;
-  if (a.m <= 16) launch_tile<(END == GATED ? 128 : 64), 16, 4, END>(a);
+  if (a.m <= 16) launch_tile<64, 16, 4, END>(a);
   else if (a.m <= 32) {
-    if (END == GATED || units >= 200) launch_tile<128, 32, 4, END>(a);
-    else launch_tile<64, 32, 4, (END == GATED ? STORE : END)>(a);
+    if (units >= 200) launch_tile<128, 32, 4, END>(a);
+    else launch_tile<64, 32, 4, END>(a);
   } else if (a.m <= 64) {
     if (units >= 200) launch_tile<128, 64, 3, END>(a);
     else launch_tile<64, 64, 4, END>(a);
@@ -402,12 +421,13 @@ std::vector<Tensor> parts_add_norm(Tensor part, Tensor x, OptT w, double eps, do
     wp = P<bf16_t>(*w);
   }
   bf16_t* np = w ? M<bf16_t>(n) : nullptr;
-#define GO(NC_) hipLaunchKernelGGL((add_norm_kernel<NC_>), dim3(m), dim3(256), 0, cur_stream(), part.data_ptr<float>(), \
-                                   P<bf16_t>(x), wp, M<bf16_t>(h), np, m, D, (int)part.size(0), (float)eps, (float)add, round)
-  if (D <= 2048) GO(2);
-  else if (D <= 4096) GO(4);
-  else if (D <= 8192) GO(8);
-  else GO(16);
+#define GO(NC_, T_) hipLaunchKernelGGL((add_norm_kernel<NC_, T_>), dim3(m), dim3(T_), 0, cur_stream(), part.data_ptr<float>(), \
+                                       P<bf16_t>(x), wp, M<bf16_t>(h), np, m, D, (int)part.size(0), (float)eps, (float)add, round)
+  if (D <= 1024) GO(1, 256);
+  else if (D <= 2048) GO(1, 512);
+  else if (D <= 4096) GO(1, 1024);
+  else if (D <= 8192) GO(2, 1024);
+  else GO(4, 1024);
 #undef GO
   if (w) return {h, n};
   return {h};
