@@ -1,0 +1,39 @@
+"""Prompts through routed experts by tiles against a loop over experts in 64 bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,E,k,D,I", [(257, 8, 2, 128, 192), (300, 3, 2, 64, 64), (1500, 8, 2, 192, 320), (700, 16, 1, 64, 128),
+                                       (2000, 5, 4, 256, 448)])
+def test_prompt_by_tiles(T, E, k, D, I):
+  from xotorch_amd.models.config import ModelConfig
+  from xotorch_amd.models.llama import MoEMLP
+  g = torch.Generator(device="cuda").manual_seed(T)
+  moe = MoEMLP(ModelConfig(dim=D, n_experts=E, n_experts_per_tok=k, intermediate_dim=I)).to("cuda", torch.bfloat16)
+  x = torch.randn(1, T, D, generator=g, device="cuda").to(torch.bfloat16)
+  with torch.no_grad():
+    for p in moe.parameters():
+      p.copy_(torch.randn(p.shape, generator=g, device="cuda") * p.shape[-1] ** -0.5)
+    moe.gate.weight.mul_(4)  # decided choices: the best of the rest is rarely within rounding
+    assert moe._by_tiles(x[0])
+    out = moe(x)[0].double()
+    xd = x[0].double()
+    logits = xd @ moe.gate.weight.double().t()
+    w, chosen = logits.softmax(-1).topk(k)
+    w = w / w.sum(-1, keepdim=True)
+    ref, size = torch.zeros_like(xd), torch.zeros_like(xd)
+    for e in range(E):
+      token, place = torch.where(chosen == e)
+      gate, up = (xd[token] @ moe.experts[e].gate_up_proj.weight.double().t()).chunk(2, -1)
+      h = torch.nn.functional.silu(gate) * up
+      down = moe.experts[e].down_proj.weight.double()
+      ref.index_add_(0, token, h @ down.t() * w[token, place, None])
+      size.index_add_(0, token, h.abs() @ down.abs().t() * w[token, place, None])
+    # activations, rows and the sum are bf16 once each; the rest is fp32
+    near = logits.topk(min(k + 1, E)).values
+    sure = (near[:, k - 1] - near[:, -1] > 1e-4) if E > k else torch.ones(T, dtype=torch.bool, device="cuda")
+    assert sure.float().mean() > 0.99
+    bound = size * 2.0 ** -7 + ref.abs() * 2.0 ** -8 + 1e-6
+    assert bool(((out - ref).abs() <= bound)[sure].all())

@@ -395,6 +395,8 @@ class MoEMLP(nn.Module):
     # large-M GEMM). Instead, prefill sorts the token-expert pairs ONCE and
     # runs each expert on a contiguous slice — one argsort + one gather
     # replaces E per-expert where/eq scans over the full assignment list.
+    if x.is_cuda and not torch.is_grad_enabled() and self._by_tiles(flat):
+      return self._forward_prefill_tiles(flat).view(B, S, D)
     weights, selected = self._route(flat)
     if x.is_cuda and not torch.is_grad_enabled():
       return self._forward_prefill_sorted(flat, weights, selected).view(B, S, D).to(x.dtype)
@@ -406,6 +408,34 @@ class MoEMLP(nn.Module):
       expert_out = self.experts[e](flat[token_idx]).float()
       out.index_add_(0, token_idx, expert_out * weights[token_idx, k_idx, None])
     return out.view(B, S, D).to(x.dtype)
+
+  def _by_tiles(self, flat) -> bool:
+    """Whether a prompt goes through the experts as two grouped products by tiles: bf16
+    weights that are one tensor per expert, over 24 rows per expert (fewer leave most
+    of a tile of 128 tokens empty)."""
+    E, k = self.n_experts, self.top_k
+    if flat.dtype != torch.bfloat16 or flat.shape[0] * k <= 24 * E or E > 256 or k > 8 or flat.shape[1] % 64 \
+       or self.intermediate % 64 or not flat.is_contiguous() or flat.data_ptr() % 16 \
+       or os.getenv("XOT_FP8_PREFILL", "0") == "1" or not ops._use_hip(flat):
+      return False
+    mods = [p for e in self.experts for p in (e.gate_up_proj, e.down_proj)]
+    return (type(self.gate) is nn.Linear and all(type(e) is MLP for e in self.experts)
+            and all(type(p) is XotLinear and p.bias is None for p in mods)
+            and all(p.weight.dtype == torch.bfloat16 and p.weight.is_cuda and p.weight.is_contiguous()
+                    and p.weight.data_ptr() % 16 == 0 for p in (self.gate, *mods)))
+
+  def _forward_prefill_tiles(self, flat):
+    """Rows of all (token, expert) pairs are placed by counting, without the host; the
+    products read tokens and weights where they lie."""
+    from xotorch_amd.ops.mixer_ops import load_hip
+    hip = load_hip("_hip_experts")
+    # tiles of 256 tokens from 150 rows an expert on: 8 experts of 4096 x 14336, two of
+    # them a token, us with 128 and 256: 300 tokens 691, 750; 700 963, 851; 2100 2218, 1904
+    tile = 256 if flat.shape[0] * self.top_k >= 150 * self.n_experts else 128
+    weight, row, *places = hip.route(flat, self.gate.weight, None, self.top_k, 1, 1, 1.0, True, 0, False, False, tile)
+    h = hip.expert_product_of(flat, [e.gate_up_proj.weight for e in self.experts], *places, True)
+    y = hip.expert_product_of(h, [e.down_proj.weight for e in self.experts], *places, False)
+    return ops._load_hip().moe_combine(y, row, weight)
 
   def _forward_prefill_sorted(self, flat, weights, selected):
     T, D = flat.shape

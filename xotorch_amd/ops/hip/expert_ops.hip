@@ -261,8 +261,9 @@ DEVINL float gated(float g, float u, const Act& a) {
 
 // What a product is: of a pair's own row; of its token with gate and up weights
 // and the gated activation; of its token with one set of weights and the square
-// of what is positive.
-enum Product { PLAIN, GATED, RELU2 };
+// of what is positive; of its token with gate and up weights and silu (no limits).
+enum Product { PLAIN, GATED, RELU2, SWIGLU };
+constexpr bool has_gate(int kind) { return kind == GATED || kind == SWIGLU; }
 
 struct GroupArgs {
   int K, kp, F, E;  // valid and stored length of a weight row, output features, experts
@@ -273,6 +274,7 @@ struct GroupArgs {
 template <int KIND>
 DEVINL float activated(float by, float g, float u, const Act& a) {
   if (KIND == GATED) return gated(by * g, by * u, a);
+  if (KIND == SWIGLU) return siluf(by * g) * (by * u);
   g = by * g;
   if (KIND == RELU2) g = fmaxf(g, 0.f) * g;
   return g;
@@ -362,17 +364,28 @@ __global__ __launch_bounds__(256) void expert_stream_kernel(
 // over the banks.
 constexpr int TILE_W = 256;  // weight rows
 
+// Where an expert's weight rows lie: in one tensor, or in one tensor each
+struct Stacked {
+  const bf16_t* w;
+  DEVINL const bf16_t* of(int e, size_t expert) const { return w + e * expert; }
+};
+constexpr int MOST_LISTED = 256;
+struct Listed {
+  const bf16_t* w[MOST_LISTED];
+  DEVINL const bf16_t* of(int e, size_t) const { return w[e]; }
+};
+
 template <int TOK> struct TileShape {
   static constexpr int WAVES = TOK / 32, BUFS = TOK == 256 ? 2 : 3, BUF = (TILE_W + TOK) * 64;  // elements of a buffer
 };
 
-template <int KIND, int TOK>
+template <int KIND, int TOK, typename W>
 __global__ __launch_bounds__(TOK * 2) void expert_tile_kernel(
-    const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const int* __restrict__ first,
+    const bf16_t* __restrict__ x, W w, const int* __restrict__ first,
     const int* __restrict__ token, const int2* __restrict__ tiles, const float* __restrict__ by_row,
     bf16_t* __restrict__ y, int max_tiles, int group, GroupArgs a, Act act) {
   typedef TileShape<TOK> Sh;
-  constexpr bool TWO = KIND == GATED;  // weight rows are gate and up
+  constexpr bool TWO = has_gate(KIND);  // weight rows are gate and up
   constexpr int WL = TILE_W / Sh::WAVES / 8, XL = 4, LOADS = WL + XL;  // loads of a stage and wave
   extern __shared__ __attribute__((aligned(16))) bf16_t buf[];  // [BUFS][weights [256][64], tokens [TOK][64]]
   // blocks go round the eight dies: give a die `group` neighbouring tiles and
@@ -387,6 +400,9 @@ __global__ __launch_bounds__(TOK * 2) void expert_tile_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
   const int wf = wave & 1, wt = wave >> 1;  // which 128 weight rows, which 64 tokens
+  // an expert's last tile: waves without tokens only load (of 256 tokens; with 128 the
+  // branch costs more than it saves)
+  const bool some = TOK < 256 || r0 + wt * 64 < hi;
   const int f0 = fb * (TWO ? 128 : 256);
   // each wave stages its share of the weight rows and 32 tokens, 8 rows a load
   const bf16_t *wsrc[WL], *xsrc[XL];
@@ -397,7 +413,7 @@ __global__ __launch_bounds__(TOK * 2) void expert_tile_kernel(
     // GATED rows: [64 gate, the same 64 up] for either half of the features
     const int f = TWO ? f0 + (r >> 7) * 64 + (r & 63) : f0 + r;
     const int part = TWO ? (r >> 6) & 1 : 0;
-    wsrc[i] = w + (((size_t)tile.x * (TWO ? 2 : 1) + part) * a.F + min(f, a.F - 1)) * a.kp + piece;
+    wsrc[i] = w.of(tile.x, (size_t)(TWO ? 2 : 1) * a.F * a.kp) + ((size_t)part * a.F + min(f, a.F - 1)) * a.kp + piece;
   }
 #pragma unroll
   for (int i = 0; i < XL; ++i) {
@@ -447,9 +463,11 @@ __global__ __launch_bounds__(TOK * 2) void expert_tile_kernel(
       READ(w8[4], wa, 4); READ(w8[5], wa, 5); READ(w8[6], wa, 6); READ(w8[7], wa, 7);
 #undef READ
     };
+    if (some)
 #pragma unroll
-    for (int kk = 0; kk < SETS; ++kk) read(kk, wv[kk], xv[kk]);
+      for (int kk = 0; kk < SETS; ++kk) read(kk, wv[kk], xv[kk]);
     if (s + Sh::BUFS - 1 < steps) stage(s + Sh::BUFS - 1);
+    if (some)
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
       bf16x8 *w8 = wv[kk % SETS], *x4 = xv[kk % SETS];
@@ -551,7 +569,7 @@ __global__ __launch_bounds__(256) void add_norm_kernel(
 std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, int64_t> route(Tensor x, Tensor w, OptT correction, int64_t pick,
                                                                   int64_t groups, int64_t keep, double scale,
                                                                   bool softmax, int64_t shared, bool gate,
-                                                                  bool on_input) {
+                                                                  bool on_input, int64_t tile_of) {
   const auto dt = io_type(x);
   check_io(w, dt);
   gate = gate && shared > 0;
@@ -565,7 +583,8 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, int64_t> route(Tensor x, Tens
               "routing to ", pick, " experts of ", keep, " of ", groups, " groups of ", E, " experts");
   CHK((int64_t)T_ * top < INT_MAX);
   const int nblk = (T_ + RT - 1) / RT, pairs = T_ * (int)top;
-  const int tile = pairs >= 320 * all ? 256 : 128, max_tiles = pairs / tile + std::min(pairs, (int)all);
+  CHK(tile_of == 0 || tile_of == 128 || tile_of == 256);
+  const int tile = tile_of ? (int)tile_of : pairs >= 320 * all ? 256 : 128, max_tiles = pairs / tile + std::min(pairs, (int)all);
   const auto ints = x.options().dtype(torch::kInt32);
   auto weight = f32(x, {T_, top});
   Tensor by_row;
@@ -601,6 +620,54 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, int64_t> route(Tensor x, Tens
   return {on_input ? by_row : weight, row, token, first, tiles, tile};
 }
 
+template <typename W>
+static void launch_tiles(const W& w, const Tensor& x, const Tensor& token, const Tensor& first, const Tensor& tiles,
+                         int64_t tile, int64_t kind, const GroupArgs& a, const Act& act, const float* by_row, Tensor& y) {
+  const int width = has_gate((int)kind) ? TILE_W / 2 : TILE_W;
+  const int max_tiles = tiles.size(0), group = std::min(8, std::max(1, max_tiles / 64)), nf = (a.F + width - 1) / width;
+  const dim3 grid((max_tiles + 8 * group - 1) / (8 * group) * 8 * group * nf);
+  CHK(tile == 128 || tile == 256);
+  auto run = [&](auto kernel, int threads, int lds) {
+    static const hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    TORCH_CHECK(err == hipSuccess, "no LDS for expert tiles");
+    hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, cur_stream(), P<bf16_t>(x), w, first.data_ptr<int>(),
+                       token.data_ptr<int>(), (const int2*)tiles.data_ptr<int>(), by_row, M<bf16_t>(y), max_tiles, group, a, act);
+  };
+#define TILES(KIND, TOK) \
+  run(expert_tile_kernel<KIND, TOK, W>, TOK * 2, TileShape<TOK>::BUFS * TileShape<TOK>::BUF * (int)sizeof(bf16_t))
+#define TILES_OF(KIND) if (tile == 256) TILES(KIND, 256); else TILES(KIND, 128)
+  if constexpr (std::is_same<W, Listed>::value) {
+    if (kind == SWIGLU) { TILES_OF(SWIGLU); }
+    else { TILES_OF(PLAIN); }
+  } else {
+    if (kind == GATED) { TILES_OF(GATED); }
+    else if (kind == RELU2) { TILES_OF(RELU2); }
+    else { TILES_OF(PLAIN); }
+  }
+#undef TILES_OF
+#undef TILES
+}
+
+// The tiled form with one weight tensor per expert, bf16: SWIGLU ([2 F, K], gate rows
+// first) or PLAIN ([F, K]), K % 64 == 0.
+Tensor expert_product_of(Tensor x, std::vector<Tensor> w, Tensor token, Tensor first, Tensor tiles, int64_t tile, bool swiglu) {
+  check_io(x, torch::kBFloat16);
+  const int64_t E = w.size();
+  CHK(x.dim() == 2 && E >= 1 && E <= MOST_LISTED && ((size_t)x.data_ptr() & 15) == 0);
+  for (const Tensor& t : {token, first, tiles}) check_io(t, torch::kInt32);
+  const int K = x.size(1), pairs = token.numel(), F_ = w[0].size(0) / (swiglu ? 2 : 1);
+  CHK(first.numel() == E + 1 && K % 64 == 0 && F_ % 16 == 0 && (swiglu || x.size(0) == pairs));
+  Listed list{};
+  for (int64_t e = 0; e < E; ++e) {
+    check_io(w[e], torch::kBFloat16);
+    CHK(w[e].dim() == 2 && w[e].size(0) == F_ * (swiglu ? 2 : 1) && w[e].size(1) == K && ((size_t)w[e].data_ptr() & 15) == 0);
+    list.w[e] = P<bf16_t>(w[e]);
+  }
+  auto y = torch::empty({pairs, F_}, x.options());
+  launch_tiles(list, x, token, first, tiles, tile, swiglu ? SWIGLU : PLAIN, GroupArgs{K, K, F_, (int)E, K, F_}, Act{}, nullptr, y);
+  return y;
+}
+
 // One grouped product over all pairs: GATED (x by token, weights [E,2,F,kp]),
 // RELU2 (x by token, weights [E,F,kp]) or PLAIN (x by row, weights [E,F,kp]); kp:
 // row length padded with zeros. by_row [pairs]: scales of the product's rows.
@@ -624,25 +691,7 @@ Tensor expert_product(Tensor x, Tensor w, Tensor token, Tensor first, Tensor til
   const int *fp = first.data_ptr<int>(), *tp = token.data_ptr<int>();
   // on average more than 24 rows per expert: weights are worth tiling
   if (dt == torch::kBFloat16 && K % 8 == 0 && pairs > 24 * E) {
-    const int width = gated_ ? TILE_W / 2 : TILE_W;
-    const int max_tiles = tiles.size(0), group = std::min(8, std::max(1, max_tiles / 64)), nf = (F_ + width - 1) / width;
-    const dim3 grid((max_tiles + 8 * group - 1) / (8 * group) * 8 * group * nf);
-    const int2* tl = (const int2*)tiles.data_ptr<int>();
-    CHK(tile == 128 || tile == 256);
-    auto run = [&](auto kernel, int threads, int lds) {
-      static const hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-      TORCH_CHECK(err == hipSuccess, "no LDS for expert tiles");
-      hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, stream, P<bf16_t>(x), P<bf16_t>(w), fp, tp, tl, bp,
-                         M<bf16_t>(y), max_tiles, group, a, act);
-    };
-#define TILES(KIND, TOK) \
-  run(expert_tile_kernel<KIND, TOK>, TOK * 2, TileShape<TOK>::BUFS * TileShape<TOK>::BUF * (int)sizeof(bf16_t))
-#define TILES_OF(KIND) if (tile == 256) TILES(KIND, 256); else TILES(KIND, 128)
-    if (kind == GATED) { TILES_OF(GATED); }
-    else if (kind == RELU2) { TILES_OF(RELU2); }
-    else { TILES_OF(PLAIN); }
-#undef TILES_OF
-#undef TILES
+    launch_tiles(Stacked{P<bf16_t>(w)}, x, token, first, tiles, tile, kind, a, act, bp, y);
     return y;
   }
   const dim3 grid(F_ / 16, E);
@@ -704,10 +753,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("route", &route, "router: sigmoid scores or a softmax over the chosen, group-limited top-k, shared experts; rows of all pairs",
         py::arg("x"), py::arg("w"), py::arg("correction"), py::arg("top"), py::arg("groups"), py::arg("keep"),
         py::arg("scale"), py::arg("softmax") = false, py::arg("shared") = 0, py::arg("gate") = true,
-        py::arg("on_input") = false);
+        py::arg("on_input") = false, py::arg("tile") = 0);
   m.def("expert_product", &expert_product, "grouped product of all (token, expert) pairs, with an activation or plain",
         py::arg("x"), py::arg("w"), py::arg("token"), py::arg("first"), py::arg("tiles"), py::arg("tile"), py::arg("kind"),
         py::arg("alpha") = 0.0, py::arg("limit") = 0.0, py::arg("plus") = 0.0, py::arg("by_row") = py::none());
+  m.def("expert_product_of", &expert_product_of, "the same by tiles, with one weight tensor per expert: silu of gate and up, or plain");
   m.attr("PLAIN") = (int)PLAIN;
   m.attr("GATED") = (int)GATED;
   m.attr("RELU2") = (int)RELU2;
