@@ -1,0 +1,115 @@
+"""Differentiable operators of a training pass (hip/train_ops.hip) against 64 bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+BF, STEP = torch.bfloat16, 2.0 ** -8  # what a result rounded to bf16 may be off by, of itself
+
+
+def _rand(*shape, seed=0):
+  g = torch.Generator(device="cuda").manual_seed(seed)
+  return torch.randn(*shape, generator=g, device="cuda").to(BF)
+
+
+def _norm64(f, w, add):
+  return f * torch.rsqrt(f.square().mean(-1, keepdim=True) + 1e-5) * (w + add)
+
+
+@pytest.mark.parametrize("rows,D", [(1, 8), (3, 2048), (700, 2056), (5, 4104), (2, 8200), (513, 64), (1, 16384)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_norm(rows, D, residual):
+  from xotorch_amd import ops
+  x, r, w = _rand(2, rows, D), _rand(2, rows, D, seed=1), _rand(D, seed=2)
+  dy, ds = _rand(2, rows, D, seed=3), _rand(2, rows, D, seed=4)
+  leaves = [t.clone().requires_grad_(True) for t in (x, r, w)]
+  exact = [t.double().requires_grad_(True) for t in (x, r, w)]
+  if residual:
+    y, s = ops.rmsnorm_residual(*leaves, 1e-5, 1.0)
+    assert y.grad_fn is not None and "_NormResidual" in type(y.grad_fn).__name__
+    torch.autograd.backward([y, s], [dy, ds])
+    f = exact[0] + exact[1]
+    torch.autograd.backward([_norm64(f, exact[2], 1.0), f], [dy.double(), ds.double()])
+    assert torch.equal(leaves[0].grad, leaves[1].grad)
+  else:
+    y = ops.rmsnorm(leaves[0], leaves[2], 1e-5, 1.0)
+    assert "_Norm" in type(y.grad_fn).__name__
+    y.backward(dy)
+    _norm64(exact[0], exact[2], 1.0).backward(dy.double())
+    f = exact[0]
+  f = f.detach()
+  inv = torch.rsqrt(f.square().mean(-1, keepdim=True) + 1e-5)
+  dn = dy.double() * (w.double() + 1)
+  # fp32 sums over a row, scaled by the row
+  terms = inv * (dn.abs() + f.abs() * inv * inv * (dn * f).abs().mean(-1, keepdim=True)) + (ds.double().abs() if residual else 0)
+  ref = exact[0].grad
+  assert bool(((leaves[0].grad.double() - ref).abs() <= ref.abs() * STEP + terms * (D + 16) * 2.0 ** -24).all())
+  dw, size = exact[2].grad, (dy.double() * f * inv).abs().flatten(0, 1).sum(0)
+  assert bool(((leaves[2].grad.double() - dw).abs() <= dw.abs() * STEP + size * (2 * rows + D) * 2.0 ** -24).all())
+
+
+@pytest.mark.parametrize("rows,I", [(1, 8), (3, 1000), (257, 5632)])
+def test_swiglu(rows, I):
+  from xotorch_amd import ops
+  gu, dy = (_rand(rows, 2 * I) * 4).requires_grad_(True), _rand(rows, I, seed=1)
+  y = ops.swiglu_packed(gu)
+  assert "_SwiGLU" in type(y.grad_fn).__name__
+  y.backward(dy)
+  e = gu.detach().double().requires_grad_(True)
+  g, u = e.chunk(2, -1)
+  (torch.nn.functional.silu(g) * u).backward(dy.double())
+  # the sigmoid to a few 2^-22, in a sum with 1 that may cancel
+  slack = (dy.double().abs() * (1 + g.abs() + u.abs() * (1 + g.abs()))).repeat(1, 2) * 2.0 ** -20
+  assert bool(((gu.grad.double() - e.grad).abs() <= e.grad.abs() * STEP + slack).all())
+
+
+@pytest.mark.parametrize("B,S,H,KVH,hd,per_row", [(1, 1, 1, 1, 8, False), (2, 33, 6, 2, 64, True), (2, 40, 4, 4, 128, False), (3, 5, 8, 1, 24, True)])
+def test_heads(B, S, H, KVH, hd, per_row):
+  from xotorch_amd.ops import torch_ref, train_ops
+  cos, sin = torch_ref.rope_cos_sin(hd, 64, 10000.0, device="cuda")
+  pos = torch.arange(3, 3 + S, dtype=torch.int32, device="cuda")
+  pos = torch.stack([pos + b for b in range(B)]) if per_row else pos
+  qkv = _rand(B, S, (H + 2 * KVH) * hd).requires_grad_(True)
+  assert train_ops.takes_heads(qkv, cos, sin, pos, hd)
+  out = train_ops._SplitHeads.apply(qkv, cos, sin, pos, H, KVH, hd)
+  ref = train_ops._split(qkv.detach(), cos, sin, pos, H, KVH, hd)
+  grads = [torch.randn(t.shape, device="cuda") for t in out]
+  for a, b in zip(out, ref):  # x cos - y sin may be contracted differently: a step of bf16
+    assert a.dtype == torch.float32 and a.is_contiguous() and bool(((a - b).abs() <= b.abs() * 2.0 ** -7 + 2.0 ** -20).all())
+  torch.autograd.backward(out, grads)
+  # exactly: the sum over heads that share a key, and the rotation's transpose
+  dq, dk, dv = (g.double().view(B, -1, H // n, S, hd).sum(2).transpose(1, 2) for g, n in zip(grads, (H, KVH, KVH)))
+  c, s = (t[pos.long()].double().expand(B, S, hd // 2)[:, :, None] for t in (cos, sin))
+  def turned_back(g):
+    g1, g2 = g.chunk(2, -1)
+    return torch.cat([g1 * c + g2 * s, g2 * c - g1 * s], -1)
+  ref = torch.cat([turned_back(dq), turned_back(dk), dv], 2).flatten(2)
+  # rounded to bf16 before and after the turn; fp32 sums of H / KVH numbers
+  size = torch.cat([dq, dk, dv], 2).abs()
+  size = (size + size.roll(hd // 2, -1)).flatten(2)
+  assert bool(((qkv.grad.double() - ref).abs() <= ref.abs() * STEP + size * (STEP + 2.0 ** -18)).all())
+  o = torch.randn(B, H, S, hd, device="cuda").requires_grad_(True)
+  m, d = train_ops._MergeHeads.apply(o), _rand(B, S, H * hd, seed=5)
+  m.backward(d)
+  assert torch.equal(m, o.detach().to(BF).transpose(1, 2).flatten(2)) and torch.equal(o.grad, d.view(B, S, H, hd).transpose(1, 2).float())
+
+
+def test_second_derivatives_forward_mode_and_transforms():
+  """What the functions cannot do themselves goes by torch's operators."""
+  from xotorch_amd import ops
+  from xotorch_amd.ops import torch_ref
+  x, w, gu, dy = _rand(3, 64), _rand(64, seed=1), _rand(3, 128, seed=2), _rand(3, 64, seed=3)
+  for own, ref, at in ((lambda t: ops.rmsnorm(t, w, 1e-5), lambda t: torch_ref.rmsnorm(t, w, 1e-5), x),
+                       (lambda t: ops.rmsnorm_residual(t, dy, w, 1e-5)[0], lambda t: torch_ref.rmsnorm_residual(t, dy, w, 1e-5)[0], x),
+                       (ops.swiglu_packed, torch_ref.swiglu_packed, gu)):
+    found = []
+    for f in (own, ref):
+      t = at.clone().requires_grad_(True)
+      g, = torch.autograd.grad(f(t), t, dy, create_graph=True)
+      found.append(torch.autograd.grad(g.float().square().sum(), t)[0].float())
+    assert (found[0] - found[1]).norm() <= 0.02 * found[1].norm()  # bf16 gradients of bf16 gradients
+    assert torch.equal(torch.func.vmap(torch.func.grad(lambda t: own(t).float().sum()))(at[:, None]),
+                       torch.func.vmap(torch.func.grad(lambda t: ref(t).float().sum()))(at[:, None]))
+    t = at.clone().requires_grad_(True)
+    with torch.autograd.forward_ad.dual_level():
+      dual = torch.autograd.forward_ad.make_dual(t, torch.ones_like(t))
+      assert torch.autograd.forward_ad.unpack_dual(own(dual)).tangent is not None

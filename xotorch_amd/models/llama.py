@@ -24,6 +24,7 @@ import torch.nn as nn
 
 from xotorch_amd import ops
 from xotorch_amd.models.config import ModelConfig
+from xotorch_amd.ops import train_ops
 from xotorch_amd.ops.torch_ref import rope_cos_sin
 from xotorch_amd.shard import Shard
 
@@ -212,6 +213,8 @@ class Attention(nn.Module):
     cfg = self.cfg
     H, KVH, hd = cfg.n_heads, cfg.n_kv_heads, cfg.head_dim
     qkv = self.qkv_proj(x)
+    if not cfg.qk_norm and train_ops.takes_heads(qkv, cos, sin, positions, hd):
+      return self.o_proj(train_ops.causal_heads(qkv, cos, sin, positions, H, KVH, hd))
     q, k, v = torch.split(qkv, [H * hd, KVH * hd, KVH * hd], dim=-1)
     q = q.reshape(B, S, H, hd)
     k = k.reshape(B, S, KVH, hd)

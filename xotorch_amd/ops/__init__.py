@@ -14,7 +14,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from xotorch_amd.ops import torch_ref
+from xotorch_amd.ops import torch_ref, train_ops
 
 _hip = None
 _hip_load_error: Optional[Exception] = None
@@ -42,8 +42,8 @@ def _use_hip(*tensors: torch.Tensor) -> bool:
   if not t.is_cuda:
     return False
   if torch.is_grad_enabled() and any(x.requires_grad for x in tensors):
-    # training path: HIP kernels are inference-only (no autograd); the torch
-    # ops are differentiable. Inference runs on the HIP kernels.
+    # training path: these kernels are inference-only (no autograd); train_ops has
+    # differentiable ones for some, the torch ops are differentiable.
     return False
   if _load_hip() is not None:
     return True
@@ -61,6 +61,8 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, w_bias: float = 0
   """w_bias=1.0 gives the gemma convention (scale by 1 + w, fp32 math)."""
   if _use_hip(x, weight) and x.dtype == torch.bfloat16:
     return _hip.rmsnorm(x, weight, eps, w_bias)
+  if train_ops.takes(x, weight) and x.shape[-1] <= 16384:
+    return train_ops.rmsnorm(x, weight, eps, w_bias)
   return torch_ref.rmsnorm(x, weight, eps, w_bias)
 
 
@@ -70,6 +72,8 @@ def rmsnorm_residual(
 ) -> Tuple[torch.Tensor, torch.Tensor]:
   if _use_hip(x, residual, weight) and x.dtype == torch.bfloat16:
     return _hip.rmsnorm_residual(x, residual, weight, eps, w_bias)
+  if train_ops.takes(x, residual, weight) and x.shape[-1] <= 16384 and x.shape == residual.shape:
+    return train_ops.rmsnorm_residual(x, residual, weight, eps, w_bias)
   return torch_ref.rmsnorm_residual(x, residual, weight, eps, w_bias)
 
 
@@ -182,6 +186,8 @@ def swiglu_packed(gu):
   """silu(gate)*up on the packed [.., 2I] fused gate_up GEMM output."""
   if _use_hip(gu) and gu.dtype == torch.bfloat16:
     return _hip.swiglu_packed(gu)
+  if train_ops.takes(gu) and gu.shape[-1] % 16 == 0:
+    return train_ops.swiglu_packed(gu)
   return torch_ref.swiglu_packed(gu)
 
 

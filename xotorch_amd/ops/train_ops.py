@@ -1,0 +1,188 @@
+"""Differentiable forms of the decoder's operators for training on the GPU (bf16,
+hip/train_ops.hip): one kernel forward and one backward where separate torch operators
+pass fp32 copies through memory. What they cannot take (other types, tracing,
+functorch transforms, forward-mode) goes by torch_ref, and so does a backward pass
+that is itself differentiated."""
+from __future__ import annotations
+
+import os
+from typing import Callable, Sequence
+
+import torch
+
+from xotorch_amd.ops import torch_ref
+
+_ext = None
+
+
+def _hip():
+  global _ext
+  if _ext is None:
+    import importlib
+    _ext = importlib.import_module("xotorch_amd.ops._hip_train")
+  return _ext
+
+
+def _missing() -> bool:
+  """Whether the kernels are not built and torch's operators are asked for then."""
+  if _ext is None and os.getenv("XOT_ALLOW_EAGER", "0") == "1":
+    try:
+      _hip()
+    except ImportError:
+      return True
+  return False
+
+
+def plain_autograd() -> bool:
+  """Whether autograd alone looks on: no tracing, no functorch transform, no
+  forward-mode level, which pass such functions by."""
+  return not (torch.jit.is_tracing() or torch.jit.is_scripting() or torch.compiler.is_compiling()
+              or torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0)
+
+
+def takes(x: torch.Tensor, *others: torch.Tensor) -> bool:
+  """Whether these operands of a differentiated operator are for the kernels: plain
+  bf16 GPU tensors, rows of whole 16 bytes up to 16384 numbers."""
+  if not (x.is_cuda and torch.is_grad_enabled() and x.dim() > 0 and 0 < x.shape[-1] <= 1 << 17 and x.shape[-1] % 8 == 0 and x.numel() > 0):
+    return False
+  return (any(t.requires_grad for t in (x, *others)) and all(t.dtype == torch.bfloat16 and t.is_cuda for t in (x, *others))
+          and plain_autograd() and not _missing())
+
+
+def _rows(t: torch.Tensor) -> torch.Tensor:
+  """Contiguous, with rows on 16 bytes."""
+  t = t.contiguous()
+  return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def _again(f: Callable, inputs: Sequence[torch.Tensor], needs: Sequence[bool], grads: Sequence) -> list:
+  """Gradients of f by torch's own operators, differentiable in turn."""
+  with torch.enable_grad():
+    outs = f(*inputs)
+    outs = outs if isinstance(outs, tuple) else (outs,)
+    pairs = [(o, g) for o, g in zip(outs, grads) if g is not None]
+    wanted = [t for t, n in zip(inputs, needs) if n]
+    found = iter(torch.autograd.grad([o for o, _ in pairs], wanted, [g for _, g in pairs], create_graph=True, allow_unused=True))
+  return [next(found) if n else None for n in needs]
+
+
+class _Norm(torch.autograd.Function):
+  @staticmethod
+  def forward(ctx, x, weight, eps, w_bias):
+    from xotorch_amd import ops
+    ctx.save_for_backward(x, weight)
+    ctx.eps, ctx.w_bias = eps, w_bias
+    return ops._load_hip().rmsnorm(_rows(x), _rows(weight), eps, w_bias)
+
+  @staticmethod
+  def backward(ctx, dy):
+    x, weight = ctx.saved_tensors
+    if torch.is_grad_enabled():
+      return (*_again(lambda a, b: torch_ref.rmsnorm(a, b, ctx.eps, ctx.w_bias), (x, weight), ctx.needs_input_grad[:2], (dy,)),
+              None, None)
+    dx, *dw = _hip().norm_backward(_rows(dy), None, _rows(x), None, _rows(weight), ctx.eps, ctx.w_bias, ctx.needs_input_grad[1])
+    return dx, dw[0] if dw else None, None, None
+
+
+class _NormResidual(torch.autograd.Function):
+  @staticmethod
+  def forward(ctx, x, residual, weight, eps, w_bias):
+    from xotorch_amd import ops
+    ctx.save_for_backward(x, residual, weight)
+    ctx.eps, ctx.w_bias = eps, w_bias
+    ctx.set_materialize_grads(False)
+    return tuple(ops._load_hip().rmsnorm_residual(_rows(x), _rows(residual), _rows(weight), eps, w_bias))
+
+  @staticmethod
+  def backward(ctx, dy, ds):
+    x, residual, weight = ctx.saved_tensors
+    if dy is None and ds is None:
+      return None, None, None, None, None
+    if torch.is_grad_enabled():
+      return (*_again(lambda a, r, w: torch_ref.rmsnorm_residual(a, r, w, ctx.eps, ctx.w_bias), (x, residual, weight),
+                      ctx.needs_input_grad[:3], (dy, ds)), None, None)
+    if dy is None:
+      return ds, ds, torch.zeros_like(weight) if ctx.needs_input_grad[2] else None, None, None
+    dx, *dw = _hip().norm_backward(_rows(dy), None if ds is None else _rows(ds), _rows(x), _rows(residual), _rows(weight),
+                                   ctx.eps, ctx.w_bias, ctx.needs_input_grad[2])
+    return dx, dx, dw[0] if dw else None, None, None
+
+
+class _SwiGLU(torch.autograd.Function):
+  @staticmethod
+  def forward(ctx, gu):
+    from xotorch_amd import ops
+    ctx.save_for_backward(gu)
+    return ops._load_hip().swiglu_packed(_rows(gu))
+
+  @staticmethod
+  def backward(ctx, dy):
+    gu, = ctx.saved_tensors
+    if torch.is_grad_enabled():
+      return _again(torch_ref.swiglu_packed, (gu,), (True,), (dy,))[0]
+    return _hip().swiglu_backward(_rows(gu), _rows(dy))
+
+
+def _split(qkv, cos, sin, positions, n_heads, n_kv_heads, hd):
+  """The same as _SplitHeads by torch's operators."""
+  B, S, _ = qkv.shape
+  q, k, v = (t.reshape(B, S, -1, hd) for t in qkv.split([n_heads * hd, n_kv_heads * hd, n_kv_heads * hd], dim=-1))
+  q, k = torch_ref.rope_apply(q, k, cos, sin, positions)
+  rep = n_heads // n_kv_heads
+  return (q.transpose(1, 2).float(), k.transpose(1, 2).repeat_interleave(rep, dim=1).float(),
+          v.transpose(1, 2).repeat_interleave(rep, dim=1).float())
+
+
+class _SplitHeads(torch.autograd.Function):
+  @staticmethod
+  def forward(ctx, qkv, cos, sin, positions, n_heads, n_kv_heads, hd):
+    ctx.save_for_backward(qkv, cos, sin, positions)
+    ctx.sizes = n_heads, n_kv_heads, hd
+    return tuple(_hip().split_heads(_rows(qkv), cos, sin, positions, n_heads, n_kv_heads, hd))
+
+  @staticmethod
+  def backward(ctx, dq, dk, dv):
+    qkv, *places = ctx.saved_tensors
+    if torch.is_grad_enabled():
+      return (_again(lambda t: _split(t, *places, *ctx.sizes), (qkv,), (True,), (dq, dk, dv))[0], *[None] * 6)
+    return (_hip().split_heads_backward(_rows(dq), _rows(dk), _rows(dv), *places, ctx.sizes[1]), *[None] * 6)
+
+
+class _MergeHeads(torch.autograd.Function):
+  @staticmethod
+  def forward(ctx, out):
+    ctx.heads = out.shape[1]
+    return _hip().merge_heads(_rows(out))
+
+  @staticmethod
+  def backward(ctx, d):
+    B, S, width = d.shape
+    if torch.is_grad_enabled():
+      return d.reshape(B, S, ctx.heads, width // ctx.heads).transpose(1, 2).float()
+    return _hip().merge_heads_backward(_rows(d), ctx.heads)
+
+
+def rmsnorm(x, weight, eps: float, w_bias: float = 0.0):
+  return _Norm.apply(x, weight, eps, w_bias)
+
+
+def rmsnorm_residual(x, residual, weight, eps: float, w_bias: float = 0.0):
+  return _NormResidual.apply(x, residual, weight, eps, w_bias)
+
+
+def swiglu_packed(gu):
+  return _SwiGLU.apply(gu)
+
+
+def causal_heads(qkv, cos, sin, positions, n_heads: int, n_kv_heads: int, hd: int):
+  """Causal attention of a training pass, fp32 between projection and result:
+  [B, S, (H + 2 KVH) hd] -> [B, S, H hd]."""
+  q, k, v = _SplitHeads.apply(qkv, cos, sin, positions, n_heads, n_kv_heads, hd)
+  return _MergeHeads.apply(torch.nn.functional.scaled_dot_product_attention(q, k, v, is_causal=True))
+
+
+def takes_heads(qkv, cos, sin, positions, hd: int) -> bool:
+  B, S, _ = qkv.shape
+  return (takes(qkv) and hd % 8 == 0 and isinstance(positions, torch.Tensor) and positions.is_cuda
+          and positions.dtype == torch.int32 and positions.is_contiguous() and positions.shape in ((S,), (B, S))
+          and all(t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (cos, sin)))

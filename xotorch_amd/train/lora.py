@@ -36,6 +36,10 @@ class LoRALinear(nn.Module):
   def forward(self, x):
     out = self.base(x)
     if not self.merged:
+      if x.is_cuda and x.dtype == out.dtype == torch.bfloat16:
+        # the sum and the factor belong to the second product: no pass over [.., out] of their own
+        low = (self.dropout(x) @ self.lora_a.to(x.dtype).t()).reshape(-1, self.rank)
+        return torch.addmm(out.reshape(-1, out.shape[-1]), low, self.lora_b.to(x.dtype).t(), alpha=self.scaling).view(out.shape)
       lora = self.dropout(x) @ self.lora_a.to(x.dtype).t() @ self.lora_b.to(x.dtype).t()
       out = out + lora * self.scaling
     return out
