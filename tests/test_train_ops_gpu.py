@@ -93,6 +93,45 @@ def test_heads(B, S, H, KVH, hd, per_row):
   assert torch.equal(m, o.detach().to(BF).transpose(1, 2).flatten(2)) and torch.equal(o.grad, d.view(B, S, H, hd).transpose(1, 2).float())
 
 
+@pytest.mark.parametrize("B,S,H,KVH,hd,per_row", [(1, 1, 1, 1, 64, False), (2, 31, 6, 2, 64, True), (1, 33, 2, 2, 128, False),
+                                                  (2, 200, 8, 1, 128, True), (1, 545, 4, 2, 64, False)])
+@pytest.mark.parametrize("spread", [1.0, 4.0])
+def test_causal_heads(B, S, H, KVH, hd, per_row, spread):
+  from xotorch_amd.ops import torch_ref, train_ops
+  cos, sin = torch_ref.rope_cos_sin(hd, 1024, 10000.0, device="cuda")
+  pos = torch.arange(3, 3 + S, dtype=torch.int32, device="cuda")
+  pos = torch.stack([pos + b for b in range(B)]) if per_row else pos
+  qkv, d = (_rand(B, S, (H + 2 * KVH) * hd) * spread).requires_grad_(True), _rand(B, S, H * hd, seed=1)
+  out = train_ops.causal_heads(qkv, cos, sin, pos, H, KVH, hd)
+  assert "_CausalHeads" in type(out.grad_fn).__name__
+  out.backward(d)
+  # 64 bits from the rotated heads on (rounded to bf16, which the heads' test covers)
+  q, k, v = (t.double().detach().requires_grad_(True) for t in train_ops._SplitHeads.apply(qkv.detach(), cos, sin, pos, H, KVH, hd))
+  scores = (q @ k.transpose(-1, -2)) * hd ** -0.5
+  p = scores.masked_fill(torch.ones(S, S, dtype=torch.bool, device="cuda").triu(1), float("-inf")).softmax(-1)
+  o, do = p @ v, d.view(B, S, H, hd).transpose(1, 2).double()
+  o.backward(do)
+  merged = o.detach().transpose(1, 2).flatten(2)
+  # fp32 scores are off by their products' sizes, exponentials by as much relative to themselves
+  with torch.no_grad():
+    off = ((q.abs() @ k.abs().transpose(-1, -2)).amax(-1, keepdim=True) * hd ** -0.5 + 8) * (hd + 16) * 2.0 ** -24
+    slack = (off * (p @ v.abs())).transpose(1, 2).flatten(2)
+    assert bool(((out.double() - merged).abs() <= merged.abs() * STEP + slack).all())
+    dp, delta = do.abs() @ v.abs().transpose(-1, -2), (do.abs() * (p @ v.abs())).sum(-1, keepdim=True)
+    ds = p * (dp + delta) * (off + (hd + 16) * 2.0 ** -24) * hd ** -0.5
+    slacks = [ds @ k.abs(), ds.transpose(-1, -2) @ q.abs(), (p * off).transpose(-1, -2) @ do.abs()]
+    dq, dk, dv, sq, sk, sv = ((t.view(B, -1, H // n, S, hd).sum(2).transpose(1, 2))
+                              for t, n in zip([q.grad, k.grad, v.grad] + slacks, (H, KVH, KVH) * 2))
+    c, s = (t[pos.long()].double().expand(B, S, hd // 2)[:, :, None] for t in (cos, sin))
+    def turned_back(g):
+      g1, g2 = g.chunk(2, -1)
+      return torch.cat([g1 * c + g2 * s, g2 * c - g1 * s], -1)
+    ref = torch.cat([turned_back(dq), turned_back(dk), dv], 2).flatten(2)
+    size, slack = torch.cat([dq, dk, dv], 2).abs(), torch.cat([sq, sk, sv], 2)
+    size, slack = ((t + t.roll(hd // 2, -1)).flatten(2) for t in (size, slack))
+    assert bool(((qkv.grad.double() - ref).abs() <= ref.abs() * STEP + size * (STEP + 2.0 ** -18) + slack).all())
+
+
 def test_second_derivatives_forward_mode_and_transforms():
   """What the functions cannot do themselves goes by torch's operators."""
   from xotorch_amd import ops

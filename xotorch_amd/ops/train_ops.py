@@ -1,5 +1,5 @@
 """Differentiable forms of the decoder's operators for training on the GPU (bf16,
-hip/train_ops.hip): one kernel forward and one backward where separate torch operators
+hip/train_ops.hip, hip/attn_train.hip): one kernel forward and one backward where separate torch operators
 pass fp32 copies through memory. What they cannot take (other types, tracing,
 functorch transforms, forward-mode) goes by torch_ref, and so does a backward pass
 that is itself differentiated."""
@@ -12,7 +12,7 @@ import torch
 
 from xotorch_amd.ops import torch_ref
 
-_ext = None
+_ext = _attn = None
 
 
 def _hip():
@@ -23,11 +23,19 @@ def _hip():
   return _ext
 
 
+def _hip_attn():
+  global _attn
+  if _attn is None:
+    import importlib
+    _attn = importlib.import_module("xotorch_amd.ops._hip_attn_train")
+  return _attn
+
+
 def _missing() -> bool:
   """Whether the kernels are not built and torch's operators are asked for then."""
-  if _ext is None and os.getenv("XOT_ALLOW_EAGER", "0") == "1":
+  if (_ext is None or _attn is None) and os.getenv("XOT_ALLOW_EAGER", "0") == "1":
     try:
-      _hip()
+      _hip(), _hip_attn()
     except ImportError:
       return True
   return False
@@ -162,6 +170,31 @@ class _MergeHeads(torch.autograd.Function):
     return _hip().merge_heads_backward(_rows(d), ctx.heads)
 
 
+def _attend(qkv, cos, sin, positions, n_heads, n_kv_heads, hd):
+  """The same as _CausalHeads by torch's operators, each with a second derivative."""
+  q, k, v = _split(qkv, cos, sin, positions, n_heads, n_kv_heads, hd)
+  S = q.shape[2]
+  scores = (q * hd ** -0.5) @ k.transpose(-1, -2)
+  p = scores.masked_fill(torch.ones(S, S, dtype=torch.bool, device=q.device).triu(1), float("-inf")).softmax(-1)
+  return (p @ v).to(qkv.dtype).transpose(1, 2).flatten(2)
+
+
+class _CausalHeads(torch.autograd.Function):
+  @staticmethod
+  def forward(ctx, qkv, cos, sin, positions, n_heads, n_kv_heads, hd):
+    out, *kept = _hip_attn().train_attention(_rows(qkv), cos, sin, positions, n_heads, n_kv_heads, hd)
+    ctx.save_for_backward(qkv, cos, sin, positions, *kept)
+    ctx.sizes = n_heads, n_kv_heads, hd
+    return out
+
+  @staticmethod
+  def backward(ctx, dout):
+    qkv, cos, sin, positions, *kept = ctx.saved_tensors
+    if torch.is_grad_enabled():
+      return (_again(lambda t: _attend(t, cos, sin, positions, *ctx.sizes), (qkv,), (True,), (dout,))[0], *[None] * 6)
+    return (_hip_attn().train_attention_backward(_rows(dout), _rows(qkv), *kept, cos, sin, positions, *ctx.sizes), *[None] * 6)
+
+
 def rmsnorm(x, weight, eps: float, w_bias: float = 0.0):
   return _Norm.apply(x, weight, eps, w_bias)
 
@@ -177,6 +210,8 @@ def swiglu_packed(gu):
 def causal_heads(qkv, cos, sin, positions, n_heads: int, n_kv_heads: int, hd: int):
   """Causal attention of a training pass, fp32 between projection and result:
   [B, S, (H + 2 KVH) hd] -> [B, S, H hd]."""
+  if hd in (64, 128) and qkv.shape[0] <= 65535 and qkv.numel() // hd < 1 << 29 and n_heads + 2 * n_kv_heads <= 65535:
+    return _CausalHeads.apply(qkv, cos, sin, positions, n_heads, n_kv_heads, hd)
   q, k, v = _SplitHeads.apply(qkv, cos, sin, positions, n_heads, n_kv_heads, hd)
   return _MergeHeads.apply(torch.nn.functional.scaled_dot_product_attention(q, k, v, is_causal=True))
 
