@@ -107,6 +107,9 @@ class TraceRunner:
     return torch.stack(rows).cpu() if rows else torch.empty(0, self.worker.cfg.vocab_size)
 
 
+DECODER = ("_hip_ops", "_hip_rows", "_hip_tile", "_hip_decode", "_hip_experts")  # of models that list none
+
+
 def build_extensions(model_dir: str):
   """Compiles what is missing of the HIP extensions that the model runs on."""
   from xotorch_amd.models import config_from_hf, model_class_for
@@ -115,7 +118,7 @@ def build_extensions(model_dir: str):
   cfg = config_from_hf(Path(model_dir) / "config.json", "model")
   with torch.device("meta"):
     model = model_class_for(cfg)(cfg, Shard("model", 0, cfg.n_layers - 1, cfg.n_layers))
-  needed = model.extensions() if hasattr(model, "extensions") else ["_hip_ops"]
+  needed = model.extensions() if hasattr(model, "extensions") else DECODER
   hip_build.build(verbose=False, missing_only=True, only=needed)
 
 

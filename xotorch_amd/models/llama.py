@@ -61,6 +61,7 @@ class XotLinear(nn.Linear):
   wins). Prefill/training/CPU stay on hipBLASLt/aten. Storage/state-dict
   identical to nn.Linear."""
 
+  hip = ("_hip_rows", "_hip_tile")  # what a pass loads beside the operators
   weight_packed: Optional[torch.Tensor]
   few_rows = True  # up to ops.FEW_ROWS rows have kernels of their own, whose sums are in another order
 
