@@ -132,6 +132,40 @@ def test_causal_heads(B, S, H, KVH, hd, per_row, spread):
     assert bool(((qkv.grad.double() - ref).abs() <= ref.abs() * STEP + size * (STEP + 2.0 ** -18) + slack).all())
 
 
+@pytest.mark.parametrize("rows,K,N,rank,bias", [(1, 8, 24, 1, False), (5, 64, 40, 3, True), (130, 256, 520, 16, False)])
+def test_adapted_linear(rows, K, N, rank, bias):
+  from xotorch_amd.models.llama import XotLinear
+  from xotorch_amd.train.lora import LoRALinear
+  base = XotLinear(K, N, bias=bias).cuda().to(BF)
+  lin = LoRALinear(base, rank=rank, alpha=3.0 * rank)
+  with torch.no_grad():
+    for n, p in enumerate(lin.parameters()):
+      p.copy_(_rand(*p.shape, seed=10 + n) * 0.1)
+  x, dy = _rand(2, rows, K).requires_grad_(True), _rand(2, rows, N, seed=1)
+  y = lin(x)
+  assert "_Adapted" in type(y.grad_fn).__name__ and y.shape == dy.shape
+  y.backward(dy)
+  own = [y.detach(), x.grad, lin.lora_a.grad, lin.lora_b.grad]
+  hook = base.register_forward_hook(lambda *_: None)  # somebody looks on: by separate operators
+  x2 = x.detach().clone().requires_grad_(True)
+  lin.lora_a.grad = lin.lora_b.grad = None
+  y2 = lin(x2)
+  assert "_Adapted" not in type(y2.grad_fn).__name__
+  y2.backward(dy)
+  hook.remove()
+  w, a, b, e, d = (t.detach().double() for t in (base.weight, lin.lora_a.to(BF), lin.lora_b.to(BF), x.flatten(0, 1), dy.flatten(0, 1)))
+  low, dlow = e @ a.t(), 3.0 * d @ b
+  ref = [e @ w.t() + (base.bias.double() if bias else 0) + 3 * low @ b.t(), d @ w + dlow @ a, dlow.t() @ e, 3 * d.t() @ low]
+  size = [e.abs() @ w.abs().t() + 1 + 3 * (e.abs() @ a.abs().t()) @ b.abs().t(), d.abs() @ w.abs() + 3 * (d.abs() @ b.abs()) @ a.abs(),
+          3 * (d.abs() @ b.abs()).t() @ e.abs(), 3 * d.abs().t() @ (e.abs() @ a.abs().t())]
+  for o, o2, r, z in zip(own, [y2.detach(), x2.grad, lin.lora_a.grad, lin.lora_b.grad], ref, size):
+    # a result and its low-rank factor are rounded to bf16, as without the function
+    assert bool(((o.double().view(r.shape) - r).abs() <= r.abs() * 2 * STEP + z * STEP).all())
+    assert (o.double().view(r.shape) - r).norm() <= 1.1 * (o2.double().view(r.shape) - r).norm() + 1e-3 * r.norm()
+  twice = torch.autograd.grad(lin(x), x, dy, create_graph=True)[0]
+  twice.float().square().sum().backward()
+
+
 def test_second_derivatives_forward_mode_and_transforms():
   """What the functions cannot do themselves goes by torch's operators."""
   from xotorch_amd import ops

@@ -13,6 +13,44 @@ from typing import Iterable, List, Optional
 
 import torch
 import torch.nn as nn
+import torch.nn.functional as F
+
+from xotorch_amd.ops import train_ops
+
+
+def _scaled(a, b, factor: float):
+  """factor a @ b, rounded once."""
+  return torch.addmm(a.new_empty(()), a, b, beta=0, alpha=factor)
+
+
+class _Adapted(torch.autograd.Function):
+  """x W' + bias + scaling (x A') B' of a frozen W, bf16. The low-rank terms are added by
+  their own products onto the full ones, forward and backward: autograd's sum of the two
+  ways through and a sum into a tensor of its own each passed all of [.., out] through
+  memory once or twice more (4 layers of 4096 with 4096 tokens, rank 16: 15.6 to 15.25 ms)."""
+
+  @staticmethod
+  def forward(ctx, x, weight, bias, a, b, scaling):
+    rows = x.reshape(-1, x.shape[-1])
+    out, low = F.linear(rows, weight, bias), rows @ a.t()
+    out.addmm_(low, b.t(), alpha=scaling)
+    ctx.save_for_backward(x, weight, bias, a, b, low)
+    ctx.scaling = scaling
+    return out.view(*x.shape[:-1], weight.shape[0])
+
+  @staticmethod
+  def backward(ctx, dy):
+    x, weight, bias, a, b, low = ctx.saved_tensors
+    need_x, _, _, need_a, need_b, _ = ctx.needs_input_grad
+    if torch.is_grad_enabled():
+      dx, da, db = train_ops._again(lambda x, a, b: F.linear(x, weight, bias) + (x @ a.t() @ b.t()) * ctx.scaling, (x, a, b),
+                                    (need_x, need_a, need_b), (dy,))
+      return dx, None, None, da, db, None
+    dy = dy.reshape(-1, dy.shape[-1])
+    dlow = _scaled(dy, b, ctx.scaling) if need_x or need_a else None
+    dx = (dy @ weight).addmm_(dlow, a).view(x.shape) if need_x else None
+    return (dx, None, None, dlow.t() @ x.reshape(-1, x.shape[-1]) if need_a else None,
+            _scaled(dy.t(), low, ctx.scaling) if need_b else None, None)
 
 
 class LoRALinear(nn.Module):
@@ -33,7 +71,25 @@ class LoRALinear(nn.Module):
     if base.bias is not None:
       base.bias.requires_grad_(False)
 
+  def _takes(self, x) -> bool:
+    """Whether base and adapter are one function for autograd: plain bf16 GPU tensors, a
+    frozen linear of which nobody else sees the result."""
+    base = self.base
+    if not (x.is_cuda and x.dtype == torch.bfloat16 and torch.is_grad_enabled() and x.numel() > 0 and type(x) is torch.Tensor
+            and type(self.dropout) is nn.Identity and type(base.weight) is nn.Parameter and base.weight.dtype == torch.bfloat16):
+      return False
+    from xotorch_amd.models.llama import XotLinear
+    held = (base.weight,) if base.bias is None else (base.weight, base.bias)
+    hooks = (base._forward_hooks, base._forward_pre_hooks, base._backward_hooks, base._backward_pre_hooks,
+             self.dropout._forward_hooks, self.dropout._forward_pre_hooks)
+    return (type(base) in (nn.Linear, XotLinear) and not any(hooks) and not torch.nn.modules.module._has_any_global_hook()
+            and all(t.is_cuda and t.dtype == torch.bfloat16 and not t.requires_grad for t in held)
+            and any(t.requires_grad for t in (x, self.lora_a, self.lora_b))
+            and not torch.is_autocast_enabled("cuda") and train_ops.plain_autograd())
+
   def forward(self, x):
+    if not self.merged and self._takes(x):
+      return _Adapted.apply(x, self.base.weight, self.base.bias, self.lora_a.to(x.dtype), self.lora_b.to(x.dtype), self.scaling)
     out = self.base(x)
     if not self.merged:
       if x.is_cuda and x.dtype == out.dtype == torch.bfloat16:
