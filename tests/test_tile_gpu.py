@@ -6,7 +6,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 SIZES = [(1, 8, 64), (16, 72, 320), (17, 130, 1536), (32, 2048, 2048), (33, 136, 512), (64, 3584, 3584), (65, 129, 128),
-         (128, 520, 18944), (129, 2056, 640), (256, 28680, 192)]
+         (128, 520, 18944), (129, 2056, 640), (256, 28680, 192), (129, 28680, 64), (200, 3592, 3584)]
 
 
 def _inputs(m, N, K):

@@ -322,7 +322,7 @@ def tile_rows(x: torch.Tensor, *weights: torch.Tensor) -> bool:
 def tile_wins(rows: int, weight: torch.Tensor) -> bool:
   """Above 128 rows two blocks share a weight tile, and the library is as fast where
   the weight rows fill the chip without a split of k: [37888, 3584] with 256 rows
-  112 us and 82, [8192, 8192] 46 and 78, [8192, 28672] 153 and 313."""
+  115 us and 81, [8192, 8192] 45 and 77, [8192, 28672] 137 and 313."""
   return rows <= 128 or _tile().tile_splits(*weight.shape) > 1
 
 

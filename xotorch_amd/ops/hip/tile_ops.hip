@@ -6,7 +6,7 @@
 //
 // What bounds them is the weights' way from memory, for which every CU wants some
 // 48 KB on its way; library tiles leave that to few blocks. A block owns 64 or 128
-// weight rows and all rows of x (128 at most, else two blocks), and walks its part of
+// weight rows and all rows of x (from 129 on 128 of them, or all in 8 waves), and walks its part of
 // k in steps of 64 through a ring of LDS buffers that are filled by direct loads: rows of 128
 // bytes, so whole lines, the 16-byte pieces of row r permuted by r & 7 in the global
 // address, which spreads fragment reads over the banks. Where the weight rows alone
@@ -70,14 +70,15 @@ DEVINL void read_frags(unsigned a, unsigned b, bf16x8* r, bf16x8* c) {
 template <int BN, int BM, int BUFS>
 struct TileShape {
   static constexpr int ROWS = BN + BM, BUF = ROWS * 64;  // elements of a buffer
-  static constexpr int WL = BN / 32, XL = BM >= 32 ? BM / 32 : 1;  // loads of a wave and stage
+  static constexpr int WAVES = BM == 256 ? 8 : 4;
+  static constexpr int WL = BN / 8 / WAVES, XL = BM >= 32 ? BM / 8 / WAVES : 1;  // loads of a wave and stage
   static constexpr int LDS = BUFS * BUF * 2;
   // waves along x: the weight rows are split over all four for few rows of x
-  static constexpr int WX = BM >= 64 ? 2 : 1, R = BN * WX / 64, C = BM / WX / 16;
+  static constexpr int WX = BM == 256 ? 4 : BM >= 64 ? 2 : 1, R = BN * WX / WAVES / 16, C = BM / WX / 16;
 };
 
 template <int BN, int BM, int BUFS, int END>
-__global__ __launch_bounds__(256) void tile_kernel(TileArgs a) {
+__global__ __launch_bounds__((TileShape<BN, BM, BUFS>::WAVES * 64)) void tile_kernel(TileArgs a) {
   typedef TileShape<BN, BM, BUFS> Sh;
   constexpr int R = Sh::R, C = Sh::C, LOADS = Sh::WL + Sh::XL;
   extern __shared__ __attribute__((aligned(16))) bf16_t buf[];  // [BUFS][weights [BN][64], x [BM][64]]
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(256) void tile_kernel(TileArgs a) {
 #pragma unroll
   for (int i = 0; i < BUFS - 1; ++i)
     if (s0 + i < s1) stage(s0 + i);
-  const int wr = Sh::WX == 2 ? (wave >> 1) * (BN / 2) : wave * (BN / 4), wx = Sh::WX == 2 ? (wave & 1) * (BM / 2) : 0;
+  const int wr = wave / Sh::WX * (R * 16), wx = wave % Sh::WX * (C * 16);
   // this lane's first fragments, as LDS byte addresses within a buffer
   const unsigned base = (unsigned)(size_t)(lds_void*)buf;
   const unsigned wl = base + (wr + col) * 128, xl = base + (BN + wx + col) * 128;
@@ -300,7 +301,7 @@ static void launch_tile(const TileArgs& a) {
   }
   const int per = END == GATED ? BN / 2 : BN;
   const int units = (a.N + per - 1) / per * a.splits, mts = (a.m + BM - 1) / BM;
-  hipLaunchKernelGGL((tile_kernel<BN, BM, BUFS, END>), dim3((units + 7) / 8 * 8 * mts), dim3(256), Sh::LDS, cur_stream(), a);
+  hipLaunchKernelGGL((tile_kernel<BN, BM, BUFS, END>), dim3((units + 7) / 8 * 8 * mts), dim3(Sh::WAVES * 64), Sh::LDS, cur_stream(), a);
 }
 
 // Tile and depth by the rows of x and by the blocks that 128 weight rows make. us at
@@ -308,6 +309,11 @@ static void launch_tile(const TileArgs& a) {
 //   m 32: [2048, 2048] in 128 blocks 4.4, 5.0; [3584, 18944] in 224 25.6, 22.9
 //   m 64: [2048, 2048] 5.0, 6.0; [28672 -> 8192] 89.7, 76.1
 //   m 128, 3 and 2 buffers: [8192, 8192] in 256 35.4, 39.6; [57344, 8192] in 448 203, 194
+// and with 128 rows of x a block or all (weights read once, x's tile for twice the work):
+//   m 256: [2048, 2048] in 128 9.1, 12.0; [3072, 2048] in 192 12.9, 13.1; [4608, 3584] in
+//   252 18.6, 18.1; [3584, 18944] in 224 55.6, 47.5; [28672 -> 8192] 157, 137
+// (turns of two groups of waves, reading and multiplying, gained 2% on that: what bounds
+// these is the way from L2, 43 GB/s to a CU.)
 template <int END>
 static void run_tile(const TileArgs& a) {
   const int rows = END == GATED ? 2 * a.N : a.N, units = (rows + 127) / 128 * a.splits;
@@ -318,7 +324,8 @@ static void run_tile(const TileArgs& a) {
   } else if (a.m <= 64) {
     if (units >= 200) launch_tile<128, 64, 3, END>(a);
     else launch_tile<64, 64, 4, END>(a);
-  } else if (units * ((a.m + 127) / 128) > 288) launch_tile<128, 128, 2, END>(a);
+  } else if (a.m > 128 && units >= 200) launch_tile<128, 256, 3, END>(a);
+  else if (units * ((a.m + 127) / 128) > 288) launch_tile<128, 128, 2, END>(a);
   else launch_tile<128, 128, 3, END>(a);
 }
 
