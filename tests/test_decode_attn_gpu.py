@@ -53,6 +53,41 @@ def test_decode_attend(B, H, KVH, hd, T, lens, norms, shared):
     assert bool(((out[b, 0].view(H, hd).double() - ref).abs() <= bound + 1e-6).all())
 
 
+@pytest.mark.parametrize("B,S,H,KVH,hd,n,bias,norms", [(1, 1, 1, 1, 64, 1, False, False), (3, 1, 28, 4, 128, 7, True, False),
+                                                       (2, 1, 16, 1, 64, 16, True, True), (5, 1, 8, 8, 128, 5, False, True),
+                                                       (1, 45, 32, 8, 64, 9, False, False), (2, 33, 7, 1, 128, 4, True, True),
+                                                       (130, 1, 4, 4, 128, 2, True, False)])
+def test_sums_over_parts_of_k(B, S, H, KVH, hd, n, bias, norms):
+  """The same numbers as from the tensor that they add up to, in order, rounded."""
+  from xotorch_amd import ops
+  from xotorch_amd.engine.kvcache import ShardKVCache
+  from xotorch_amd.ops import torch_ref
+  g = torch.Generator(device="cuda").manual_seed(n)
+  T, width = 300, (H + 2 * KVH) * hd
+  cos, sin = torch_ref.rope_cos_sin(hd, T, 10000.0, device="cuda")
+  sums = torch.randn(n, B * S, width, generator=g, device="cuda")
+  b = torch.randn(width, generator=g, device="cuda").to(torch.bfloat16) if bias else None
+  qn, kn = (torch.randn(hd, generator=g, device="cuda").to(torch.bfloat16) for _ in "qk") if norms else (None, None)
+  total = sums[0].clone()
+  for s in sums[1:]:
+    total += s
+  qkv = (total + b.float() if bias else total).to(torch.bfloat16).view(B, S, width)
+  pos = torch.arange(200, 200 + S, dtype=torch.int32, device="cuda")
+  found = []
+  for parts in (False, True):
+    c = ShardKVCache(1, B, KVH, T, hd, torch.bfloat16, "cuda")[0]
+    given, more = (torch.full_like(qkv, float("nan")), (sums, b)) if parts else (qkv.clone(), ())
+    if S == 1:
+      seen = torch.full((B,), 201, dtype=torch.int32, device="cuda")
+      out = ops.decode_attend(given, cos, sin, pos, seen, *c[:4], H, KVH, qn, kn, 1e-6, *more)
+    else:
+      ops.rope_qkv_append(given, cos, sin, pos, c.k, c.v, H, KVH, hd, c.kp, c.vp, qn, kn, 1e-6, None, None, *more)
+      out = given[..., :H * hd]
+    found.append((out, *c[:4]))
+  for x, y in zip(*found):
+    assert torch.equal(x, y)
+
+
 def test_parked_row_keeps_to_its_own_place():
   """A row that sees less than its position appends there and reads what it sees."""
   from xotorch_amd import ops

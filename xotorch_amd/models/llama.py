@@ -51,6 +51,11 @@ def _time_us(fn, reps=4, rounds=3) -> float:
   return best
 
 
+def _watched(*modules) -> bool:
+  """Whether hooks wait for a call of one of these modules, whose work then is its own."""
+  return any(m._forward_hooks or m._forward_pre_hooks for m in modules) or torch.nn.modules.module._has_any_global_hook()
+
+
 class XotLinear(nn.Linear):
   """nn.Linear with an optional decode-path prepack: `pack_decode()` stores a
   second copy of the weight in MFMA A-fragment order ([N/32,K/16,64,8], see
@@ -240,7 +245,15 @@ class Attention(nn.Module):
     qkv = self.qkv_proj(x)  # [B, S, (H+2KVH)*hd]
     return self.o_proj(self.attend(qkv, cos, sin, positions, kv, start_pos, is_decode, seq_lens))
 
-  def attend(self, qkv, cos, sin, positions, kv, start_pos: int, is_decode: bool, seq_lens=None):
+  def project(self, x):
+    """qkv_proj by weight tiles; where k is split, (a place for the queries, the sums over
+    parts of k) for attend, whose first kernel adds them up."""
+    p = self.qkv_proj
+    if type(self) is Attention and ops.tile_parted(p.weight, p.bias):
+      return x.new_empty(*x.shape[:-1], p.weight.shape[0]), ops.tile_parts(x, p.weight)
+    return p(x), None
+
+  def attend(self, qkv, cos, sin, positions, kv, start_pos: int, is_decode: bool, seq_lens=None, sums=None):
     """What lies between the projections: qkv [B, S, (H+2KVH)*hd] -> [B, S, H*hd]."""
     B, S, _ = qkv.shape
     cfg = self.cfg
@@ -252,12 +265,13 @@ class Attention(nn.Module):
     vsc = kv[5] if len(kv) > 5 else None
     qn = self.q_norm if cfg.qk_norm else None
     kn = self.k_norm if cfg.qk_norm else None
+    bias = self.qkv_proj.bias if sums is not None else None
     if is_decode and ops.decode_attends(qkv, H, cfg.n_kv_heads, hd, kp, qn, kn):
       sl = seq_lens if seq_lens is not None else start_pos + 1
       return ops.decode_attend(qkv, cos, sin, positions, sl, k_cache, v_cache, kp, vp, H, cfg.n_kv_heads,
-                               qn, kn, cfg.norm_eps)
+                               qn, kn, cfg.norm_eps, sums, bias)
     ops.rope_qkv_append(qkv, cos, sin, positions, k_cache, v_cache, H, cfg.n_kv_heads, hd, kp, vp,
-                        qn, kn, cfg.norm_eps, ksc, vsc)
+                        qn, kn, cfg.norm_eps, ksc, vsc, sums, bias)
     q = qkv[:, :, : H * hd].view(B, S, H, hd)  # strided view; kernels accept it
     if is_decode:
       sl = seq_lens if seq_lens is not None else start_pos + 1
@@ -284,7 +298,8 @@ class MLP(nn.Module):
 
   def by_tiles(self, x) -> bool:
     gu, dp = self.gate_up_proj, self.down_proj
-    return (type(gu) is XotLinear and type(dp) is XotLinear and gu.bias is None and dp.bias is None
+    return (type(gu) is XotLinear and type(dp) is XotLinear and not _watched(self, gu, dp)
+            and gu.bias is None and dp.bias is None
             and getattr(gu, "weight_packed_fp8", None) is None and getattr(dp, "weight_packed_fp8", None) is None
             and gu.weight.shape[0] % 8 == 0 and ops.tile_rows(x, gu.weight, dp.weight)
             and ops.tile_wins(x.numel() // x.shape[-1], dp.weight))
@@ -545,6 +560,7 @@ class DecoderLayer(nn.Module):
     mods = (a.qkv_proj, a.o_proj, m.gate_up_proj, m.down_proj) if type(m) is MLP else ()
     norms = (self.input_layernorm.weight, self.post_attention_layernorm.weight)
     return (len(mods) > 0 and all(type(p) is XotLinear and p.few_rows for p in mods)
+            and not _watched(a, m, self.input_layernorm, self.post_attention_layernorm, *mods)
             and ops.few_rows_normed(x, norms, *(p.weight for p in mods)))
 
   def by_tiles(self, x) -> bool:
@@ -554,7 +570,8 @@ class DecoderLayer(nn.Module):
     if not all(type(p) is XotLinear and getattr(p, "weight_packed_fp8", None) is None for p in mods):
       return False
     rows = x.shape[0] * x.shape[1]
-    return (x.shape[-1] % 8 == 0 and x.shape[-1] <= 16384 and ops.tile_rows(x, *(p.weight for p in mods))
+    return (x.shape[-1] % 8 == 0 and x.shape[-1] <= 16384 and not _watched(self, a, *mods, self.post_attention_layernorm)
+            and ops.tile_rows(x, *(p.weight for p in mods))
             and all(ops.tile_wins(rows, p.weight) for p in mods)
             and ops.plain_norms(self.input_layernorm.weight, self.post_attention_layernorm.weight))
 
@@ -564,7 +581,8 @@ class DecoderLayer(nn.Module):
     a, m = self.self_attn, self.mlp
     if normed is None:
       normed = self.input_layernorm(x)
-    out = a.attend(a.qkv_proj(normed), cos, sin, positions, kv, start_pos, is_decode, seq_lens)
+    qkv, sums = a.project(normed)
+    out = a.attend(qkv, cos, sin, positions, kv, start_pos, is_decode, seq_lens, *(() if sums is None else (sums,)))
     post = self.post_attention_layernorm
     x, normed = ops.parts_add_norm(ops.tile_parts(out, a.o_proj.weight), x, post.weight, post.eps)
     if type(m) is MLP and m.by_tiles(normed):
@@ -572,7 +590,7 @@ class DecoderLayer(nn.Module):
     else:
       parts = m(normed).float()
     parts = parts.view(-1, x.numel() // x.shape[-1], x.shape[-1])
-    if after is None or not ops.plain_norms(after.weight):
+    if after is None or _watched(after) or not ops.plain_norms(after.weight):
       return ops.parts_add_norm(parts, x)[0], None
     return ops.parts_add_norm(parts, x, after.weight, after.eps, rounded=True)
 
@@ -754,7 +772,8 @@ class ShardedModel(nn.Module):
       normed = None
     head = self.head_weight()
     own = self.lm_head if hasattr(self, "lm_head") else None
-    if normed is None and (type(own) is XotLinear and own.few_rows if own is not None else self.few_rows) and (
+    if normed is None and (type(own) is XotLinear and own.few_rows if own is not None else self.few_rows) and not (
+        _watched(self.norm, *(() if own is None else (own,)))) and (
         ops.few_rows_normed(h, (self.norm.weight,), head)):
       logits = ops.rows_norm_linear(h, self.norm.weight, self.norm.eps, head)
       return logits[:, -1, :] if is_decode or last_only else logits

@@ -86,16 +86,19 @@ def rope_apply(q, k, cos, sin, positions):
 
 def rope_qkv_append(qkv, cos, sin, positions, k_cache, v_cache, n_heads: int, n_kv_heads: int,
                     head_dim: int, kp=None, vp=None, q_norm=None, k_norm=None,
-                    norm_eps: float = 1e-6, k_scale=None, v_scale=None):
+                    norm_eps: float = 1e-6, k_scale=None, v_scale=None, sums=None, bias=None):
   """Fused on the packed qkv GEMM output [B,S,(H+2KVH)*hd]: (optionally
   per-head-RMSNorm q/k — qwen3), RoPE-rotate the q heads in place, rotate k
   heads into the cache, copy v heads into the cache. When the MFMA-packed
-  cache copies (kp, vp) exist they are appended too.
+  cache copies (kp, vp) exist they are appended too. With `sums` (tile_parts) these and
+  the bias are the projection, and qkv only receives the queries.
   """
   if _use_hip(qkv) and qkv.dtype == torch.bfloat16:
     _hip.rope_qkv_append(qkv, cos, sin, positions, k_cache, v_cache, n_heads, n_kv_heads, head_dim,
-                         kp, vp, q_norm, k_norm, norm_eps, k_scale, v_scale)
+                         kp, vp, q_norm, k_norm, norm_eps, k_scale, v_scale, sums, bias)
     return
+  if sums is not None:
+    raise ValueError("sums over parts of k are the GPU kernels'")
   torch_ref.rope_qkv_append(qkv, cos, sin, positions, k_cache, v_cache, n_heads, n_kv_heads,
                             head_dim, q_norm, k_norm, norm_eps)
 
@@ -167,13 +170,14 @@ def decode_attends(qkv, n_heads: int, n_kv_heads: int, head_dim: int, kp, *norms
 
 
 def decode_attend(qkv, cos, sin, positions, seq_len, k_cache, v_cache, kp, vp, n_heads: int, n_kv_heads: int,
-                  q_norm=None, k_norm=None, norm_eps: float = 1e-6):
+                  q_norm=None, k_norm=None, norm_eps: float = 1e-6, sums=None, bias=None):
   """rope_qkv_append and attn_decode in one: [B, 1, (H+2KVH)*hd] -> [B, 1, H*hd].
-  qkv is left as projected."""
+  qkv is left as projected; with `sums` (tile_parts) these and the bias are read in its
+  place."""
   if not isinstance(seq_len, torch.Tensor):
     seq_len = torch.full((qkv.shape[0],), int(seq_len), dtype=torch.int32, device=qkv.device)
   return _decode().decode_attend(qkv, cos, sin, positions, seq_len, k_cache, v_cache, kp, vp, n_heads, n_kv_heads,
-                                 q_norm, k_norm, norm_eps)
+                                 q_norm, k_norm, norm_eps, sums, bias)
 
 
 def swiglu(gate, up):
@@ -324,6 +328,11 @@ def tile_wins(rows: int, weight: torch.Tensor) -> bool:
   the weight rows fill the chip without a split of k: [37888, 3584] with 256 rows
   115 us and 81, [8192, 8192] 45 and 77, [8192, 28672] 137 and 313."""
   return rows <= 128 or _tile().tile_splits(*weight.shape) > 1
+
+
+def tile_parted(weight, bias=None) -> bool:
+  """Whether tile_linear would split k and add its parts up in a kernel of its own."""
+  return weight.shape[0] % 4 == 0 and (bias is None or bias.dtype == torch.bfloat16) and _tile().tile_splits(*weight.shape) > 1
 
 
 def tile_linear(x, weight, bias=None):

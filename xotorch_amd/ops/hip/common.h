@@ -41,6 +41,21 @@ DEVINL void ld4(const bf16_t* p, float* o) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) { bf16_t u = v[i]; o[i] = ld(&u); }
 }
+
+// Four numbers' sum over parts `stride` apart, in order; four parts at a time on their way
+DEVINL floatx4 sum_parts(const float* p, size_t at, size_t stride, int splits) {
+  floatx4 v = *(const floatx4*)(p + at);
+  int s = 1;
+  for (; s + 3 < splits; s += 4) {
+    floatx4 q[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q[i] = *(const floatx4*)(p + (s + i) * stride + at);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v += q[i];
+  }
+  for (; s < splits; ++s) v += *(const floatx4*)(p + s * stride + at);
+  return v;
+}
 typedef __attribute__((ext_vector_type(2))) float floatx2;
 typedef __attribute__((ext_vector_type(2))) unsigned short ushort2_t;
 DEVINL void ld2(const float* p, float* o) {

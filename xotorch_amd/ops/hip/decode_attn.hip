@@ -10,6 +10,10 @@
 // computed transposed from key rows in an order in which the lane that holds a head's
 // probabilities feeds them to the value product. Parts are cut by the row's own
 // length, so that short rows of a ragged batch have as many blocks as long ones.
+//
+// The projection may come as fp32 sums over parts of k (tile_ops.hip): a block adds up
+// its heads' numbers in LDS, which saves a kernel between the two: 2.4 us of its 4.7 in
+// every layer (8 rows through 28 layers of 3584: 3285 to 3215 us).
 #include "common.h"
 
 struct DecodeArgs {
@@ -18,6 +22,9 @@ struct DecodeArgs {
   const int *positions, *lens;
   const bf16_t *qn, *kn;  // norms per head, or null
   bf16_t *kc, *vc, *kp, *vp, *out;
+  const float* sums;   // or [nsums, B, (H + 2 KVH) HD], to be added up with bias
+  const bf16_t* bias;
+  int nsums;
   float *part, *ml;  // [B H][splits][HD], [B H][splits][2]
   int B, H, KVH, T, T32, npos, splits;
   float scale, eps;  // scale times log2 e
@@ -30,11 +37,9 @@ DEVINL float lane_max(float v, int mask) { return fmaxf(v, __shfl_xor(v, mask));
 // The new key and value of a key head, by one wave: normed and rotated, to the plain
 // cache [B, KVH, T, HD] and the packed one.
 template <int HD>
-DEVINL void append(const DecodeArgs& a, int b, int kvh, int pos, int lane) {
+DEVINL void append(const DecodeArgs& a, int b, int kvh, int pos, int lane, const bf16_t* k, const bf16_t* v) {
   constexpr int HALF = HD / 2;
-  const size_t head = (size_t)b * a.KVH + kvh, width = (size_t)(a.H + 2 * a.KVH) * HD;
-  const bf16_t* k = a.qkv + b * width + (size_t)(a.H + kvh) * HD;
-  const bf16_t* v = k + (size_t)a.KVH * HD;
+  const size_t head = (size_t)b * a.KVH + kvh;
   const bool on = lane < HALF;
   float x1 = on ? ld(k + lane) : 0.f, x2 = on ? ld(k + lane + HALF) : 0.f;
   if (a.kn) {
@@ -63,11 +68,28 @@ DEVINL void append(const DecodeArgs& a, int b, int kvh, int pos, int lane) {
   }
 }
 
+// What a row's projection holds for the heads of a key head, as bf16: rep queries, key, value
 template <int HD, int WAVES>
+DEVINL void add_up(const DecodeArgs& a, int b, int kvh, int rep, bf16_t* own) {
+  const size_t width = (size_t)(a.H + 2 * a.KVH) * HD, stride = a.B * width;
+  for (int i = threadIdx.x * 4; i < (rep + 2) * HD; i += WAVES * 256) {
+    const int slot = i / HD;
+    const size_t at = (size_t)(slot < rep ? kvh * rep + slot : a.H + (slot - rep) * a.KVH + kvh) * HD + i % HD;
+    const floatx4 v = sum_parts(a.sums, b * width + at, stride, a.nsums);
+    float y[4], c[4] = {};
+    if (a.bias) ld4(a.bias + at, c);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) y[r] = v[r] + c[r];
+    st4(own + i, y);
+  }
+}
+
+template <int HD, int WAVES, bool SUMS>
 __global__ __launch_bounds__(WAVES * 64) void decode_attn_kernel(DecodeArgs a) {
   constexpr int KC = HD / 32, VG = HD / 16, HALF = HD / 2, ROW = HD + 4;
   extern __shared__ __attribute__((aligned(16))) float lds[];  // [WAVES][rep][ROW] outputs
   __shared__ float lm[WAVES][16], ll[WAVES][16];
+  __shared__ __attribute__((aligned(16))) bf16_t own_rows[SUMS ? 18 * HD : 1];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int col = lane & 15, quad = lane >> 4, rep = a.H / a.KVH;
   const int bh = blockIdx.x % (a.B * a.KVH), split = blockIdx.x / (a.B * a.KVH), b = bh / a.KVH, kvh = bh % a.KVH;
@@ -78,14 +100,26 @@ __global__ __launch_bounds__(WAVES * 64) void decode_attn_kernel(DecodeArgs a) {
   const int own = pos < len ? pos >> 5 : -1;
   const bool fits = pos >= 0 && pos < a.T;
   const bool appends = fits && (own >= t0 && own < t1 ? (own - t0) % WAVES == wave : own < 0 && split == 0 && wave == 0);
+  const bf16_t *q0, *k0, *v0;  // this key head's queries, key and value
+  if (SUMS) {
+    add_up<HD, WAVES>(a, b, kvh, rep, own_rows);
+    __syncthreads();
+    q0 = own_rows;
+    k0 = own_rows + rep * HD;
+    v0 = k0 + HD;
+  } else {
+    q0 = a.qkv + ((size_t)b * (a.H + 2 * a.KVH) + (size_t)kvh * rep) * HD;
+    k0 = a.qkv + ((size_t)b * (a.H + 2 * a.KVH) + a.H + kvh) * HD;
+    v0 = k0 + (size_t)a.KVH * HD;
+  }
   if (appends) {
-    append<HD>(a, b, kvh, pos, lane);
+    append<HD>(a, b, kvh, pos, lane, k0, v0);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
   // this lane's query head, normed and rotated: dims c * 32 + quad * 8 + 0..7
   bf16x8 qf[KC];
   {
-    const bf16_t* q = a.qkv + (size_t)b * (a.H + 2 * a.KVH) * HD + (size_t)(kvh * rep + min(col, rep - 1)) * HD + quad * 8;
+    const bf16_t* q = q0 + min(col, rep - 1) * HD + quad * 8;
     float x[KC][8], inv = 1.f;
 #pragma unroll
     for (int c = 0; c < KC; ++c) {
@@ -260,17 +294,21 @@ static void run_decode(DecodeArgs a, const Tensor& qkv) {
     TORCH_CHECK(e == hipSuccess, "no LDS for attention outputs");
     hipLaunchKernelGGL(kernel, dim3(heads * a.splits), dim3(waves * 64), lds, cur_stream(), a);
   };
-  if (waves == 8) run(decode_attn_kernel<HD, 8>);
-  else run(decode_attn_kernel<HD, 4>);
+  if (a.sums) {
+    if (waves == 8) run(decode_attn_kernel<HD, 8, true>);
+    else run(decode_attn_kernel<HD, 4, true>);
+  } else if (waves == 8) run(decode_attn_kernel<HD, 8, false>);
+  else run(decode_attn_kernel<HD, 4, false>);
   if (a.splits > 1)
     hipLaunchKernelGGL((decode_merge_kernel<HD>), dim3((a.B * a.H + 3) / 4), dim3(256), 0, cur_stream(), a);
 }
 
-// qkv [B, 1, (H + 2 KVH) HD] as projected (left as it is); kc, vc [B, KVH, T, HD];
+// qkv [B, 1, (H + 2 KVH) HD] as projected (left as it is; not read where sums
+// [n, B, (H + 2 KVH) HD], fp32, and their bias take its place); kc, vc [B, KVH, T, HD];
 // kp, vp their packed copies; lens: positions that rows see, the new one included.
 // -> [B, 1, H HD]
 Tensor decode_attend(Tensor qkv, Tensor cos, Tensor sin, Tensor positions, Tensor lens, Tensor kc, Tensor vc, Tensor kp,
-                     Tensor vp, int64_t heads, int64_t kv_heads, OptT q_norm, OptT k_norm, double eps) {
+                     Tensor vp, int64_t heads, int64_t kv_heads, OptT q_norm, OptT k_norm, double eps, OptT sums, OptT bias) {
   check_io(qkv, torch::kBFloat16);
   for (const Tensor* t : {&kc, &vc, &kp, &vp}) {
     check_io(*t, torch::kBFloat16);
@@ -300,6 +338,18 @@ Tensor decode_attend(Tensor qkv, Tensor cos, Tensor sin, Tensor positions, Tenso
   a.qn = q_norm ? P<bf16_t>(*q_norm) : nullptr;
   a.kn = k_norm ? P<bf16_t>(*k_norm) : nullptr;
   a.qkv = P<bf16_t>(qkv);
+  if (sums) {
+    check_io(*sums, torch::kFloat32);
+    CHK(sums->dim() == 3 && sums->size(0) >= 1 && sums->size(0) <= 1024 && sums->numel() == sums->size(0) * qkv.numel());
+    CHK(sums->size(1) == a.B && ((size_t)sums->data_ptr() & 15) == 0);
+    a.sums = sums->data_ptr<float>();
+    a.nsums = (int)sums->size(0);
+    if (bias) {
+      check_io(*bias, torch::kBFloat16);
+      CHK(bias->numel() == qkv.size(2) && ((size_t)bias->data_ptr() & 7) == 0);
+      a.bias = P<bf16_t>(*bias);
+    }
+  }
   a.cos = cos.data_ptr<float>();
   a.sin = sin.data_ptr<float>();
   a.positions = positions.data_ptr<int>();
@@ -317,4 +367,10 @@ Tensor decode_attend(Tensor qkv, Tensor cos, Tensor sin, Tensor positions, Tenso
   return out;
 }
 
-PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) { m.def("decode_attend", &decode_attend); }
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("decode_attend", &decode_attend, pybind11::arg("qkv"), pybind11::arg("cos"), pybind11::arg("sin"),
+        pybind11::arg("positions"), pybind11::arg("lens"), pybind11::arg("kc"), pybind11::arg("vc"), pybind11::arg("kp"),
+        pybind11::arg("vp"), pybind11::arg("heads"), pybind11::arg("kv_heads"), pybind11::arg("q_norm"),
+        pybind11::arg("k_norm"), pybind11::arg("eps"), pybind11::arg("sums") = pybind11::none(),
+        pybind11::arg("bias") = pybind11::none());
+}

@@ -137,7 +137,12 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(
 // fp8 packed mode (kp8 non-null): the packed copies are OCP e4m3 bytes with
 // per-row scales sk/sv [B*KVH*T32] — half the decode stream and ~60% of the
 // dual-cache residency (plain cache stays bf16 for prefill). XOT_FP8_KV=1.
+// SUMS: the projection comes as fp32 sums over nsums parts of k [nsums][B*S][slots*hd]
+// and a bias, which are added up here (qkv then only receives the queries): the pass
+// that would do it takes a launch and the bf16 tensor's way through memory.
+template <bool SUMS>
 __global__ __launch_bounds__(256) void rope_qkv_append_kernel(
+    const float* __restrict__ sums, const unsigned short* __restrict__ bias, int nsums,
     unsigned short* __restrict__ qkv, const float* __restrict__ cosb,
     const float* __restrict__ sinb, const int* __restrict__ positions,
     unsigned short* __restrict__ kc, unsigned short* __restrict__ vc,
@@ -160,11 +165,45 @@ __global__ __launch_bounds__(256) void rope_qkv_append_kernel(
   const int pos = positions[(npos == B * S && npos != S) ? bs : s];
   const int hd2 = hd >> 1;
   unsigned short* row = qkv + ((size_t)bs * slots + slot) * hd;
+  // the numbers d1 and d2 of this slot, as bf16 holds them
+  auto two = [&](int d1, int d2, unsigned short* out) {
+    if (!SUMS) {
+      out[0] = row[d1];
+      out[1] = row[d2];
+      return;
+    }
+    const size_t width = (size_t)slots * hd, stride = (size_t)B * S * width;
+    const float* p = sums + (size_t)bs * width + (size_t)slot * hd;
+    float v1 = p[d1], v2 = p[d2];
+    int i = 1;
+    for (; i + 3 < nsums; i += 4) {
+      float w1[4], w2[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        w1[j] = p[(i + j) * stride + d1];
+        w2[j] = p[(i + j) * stride + d2];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        v1 += w1[j];
+        v2 += w2[j];
+      }
+    }
+    for (; i < nsums; ++i) {
+      v1 += p[i * stride + d1];
+      v2 += p[i * stride + d2];
+    }
+    const unsigned short* c = bias + (size_t)slot * hd;
+    out[0] = f2b(bias ? v1 + b2f(c[d1]) : v1);
+    out[1] = f2b(bias ? v2 + b2f(c[d2]) : v2);
+  };
   if (slot < H) {
     float x1 = 0.f, x2 = 0.f;
     if (lane < hd2) {
-      x1 = b2f(row[lane]);
-      x2 = b2f(row[lane + hd2]);
+      unsigned short x[2];
+      two(lane, lane + hd2, x);
+      x1 = b2f(x[0]);
+      x2 = b2f(x[1]);
     }
     if (qn) {
       float ss = x1 * x1 + x2 * x2;
@@ -187,8 +226,10 @@ __global__ __launch_bounds__(256) void rope_qkv_append_kernel(
     unsigned short* dst = kc + (((size_t)(b * KVH + h) * T + pos) * hd);
     float kx1 = 0.f, kx2 = 0.f;
     if (lane < hd2) {
-      kx1 = b2f(row[lane]);
-      kx2 = b2f(row[lane + hd2]);
+      unsigned short x[2];
+      two(lane, lane + hd2, x);
+      kx1 = b2f(x[0]);
+      kx2 = b2f(x[1]);
     }
     if (kn) {
       float ss = kx1 * kx1 + kx2 * kx2;
@@ -238,8 +279,11 @@ __global__ __launch_bounds__(256) void rope_qkv_append_kernel(
   } else {
     const int h = slot - H - KVH;
     unsigned short* dst = vc + (((size_t)(b * KVH + h) * T + pos) * hd);
-    if (lane * 2 < hd)
-      *(unsigned int*)(dst + lane * 2) = *(const unsigned int*)(row + lane * 2);
+    unsigned short x[2] = {0, 0};
+    if (lane * 2 < hd) {
+      two(lane * 2, lane * 2 + 1, x);
+      *(unsigned int*)(dst + lane * 2) = x[0] | (unsigned)x[1] << 16;
+    }
     if (vpc && lane * 2 < hd) {
       // packed V: element for hd-dim d at
       //   [(b*KVH+h)][d>>4][pos>>5][((pos&31)>>3)*16 + (d&15)][pos&7]
@@ -248,13 +292,13 @@ __global__ __launch_bounds__(256) void rope_qkv_append_kernel(
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         const int d = lane * 2 + e;
-        vpc[((gbase + (d >> 4)) * (T32 >> 5) + tp) * 512 + (qt * 16 + (d & 15)) * 8 + j] = row[d];
+        vpc[((gbase + (d >> 4)) * (T32 >> 5) + tp) * 512 + (qt * 16 + (d & 15)) * 8 + j] = x[e];
       }
     }
     if (vp8) {
       float mx = 0.f;
       if (lane * 2 < hd) {
-        mx = fmaxf(fabsf(b2f(row[lane * 2])), fabsf(b2f(row[lane * 2 + 1])));
+        mx = fmaxf(fabsf(b2f(x[0])), fabsf(b2f(x[1])));
       }
 #pragma unroll
       for (int m = 32; m > 0; m >>= 1) mx = fmaxf(mx, __shfl_xor(mx, m));
@@ -267,7 +311,7 @@ __global__ __launch_bounds__(256) void rope_qkv_append_kernel(
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
           const int d = lane * 2 + e;
-          const unsigned short pk = (unsigned short)__builtin_amdgcn_cvt_pk_fp8_f32(b2f(row[d]) * inv, 0.f, 0, false);
+          const unsigned short pk = (unsigned short)__builtin_amdgcn_cvt_pk_fp8_f32(b2f(x[e]) * inv, 0.f, 0, false);
           vp8[((gbase + (d >> 4)) * (T32 >> 5) + tp) * 512 + (qt * 16 + (d & 15)) * 8 + j] = (unsigned char)(pk & 0xff);
         }
       }
@@ -2332,7 +2376,8 @@ void rope_qkv_append(torch::Tensor qkv, torch::Tensor cos, torch::Tensor sin,
                      c10::optional<torch::Tensor> kp, c10::optional<torch::Tensor> vp,
                      c10::optional<torch::Tensor> q_norm, c10::optional<torch::Tensor> k_norm,
                      double norm_eps,
-                     c10::optional<torch::Tensor> k_scale, c10::optional<torch::Tensor> v_scale) {
+                     c10::optional<torch::Tensor> k_scale, c10::optional<torch::Tensor> v_scale,
+                     c10::optional<torch::Tensor> sums, c10::optional<torch::Tensor> bias) {
   CHK(qkv.is_cuda() && qkv.dtype() == torch::kBFloat16 && qkv.is_contiguous());
   CHK(kc.is_contiguous() && vc.is_contiguous());
   CHK(positions.dtype() == torch::kInt32 && positions.is_cuda());
@@ -2380,7 +2425,21 @@ void rope_qkv_append(torch::Tensor qkv, torch::Tensor cos, torch::Tensor sin,
   }
   const int waves = B * S * (H + 2 * KVH);
   const int blocks = (waves + 3) / 4;
-  hipLaunchKernelGGL(rope_qkv_append_kernel, dim3(blocks), dim3(256), 0, cur_stream(),
+  const float* sp = nullptr;
+  const unsigned short* bp = nullptr;
+  int nsums = 0;
+  if (sums.has_value()) {
+    CHK(sums->is_cuda() && sums->dtype() == torch::kFloat32 && sums->is_contiguous() && sums->dim() == 3);
+    nsums = (int)sums->size(0);
+    CHK(nsums >= 1 && nsums <= 1024 && sums->numel() == nsums * qkv.numel());
+    sp = sums->data_ptr<float>();
+    if (bias.has_value()) {
+      CHK(bias->is_cuda() && bias->dtype() == torch::kBFloat16 && bias->is_contiguous() && bias->numel() == qkv.size(2));
+      bp = (const unsigned short*)bias->data_ptr();
+    }
+  }
+  auto kernel = sp ? rope_qkv_append_kernel<true> : rope_qkv_append_kernel<false>;
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, cur_stream(), sp, bp, nsums,
                      (unsigned short*)qkv.data_ptr(), cos.data_ptr<float>(), sin.data_ptr<float>(),
                      positions.data_ptr<int>(), (unsigned short*)kc.data_ptr(),
                      (unsigned short*)vc.data_ptr(), B, S, H, KVH, hd, T, kpc, vpc, T32,
@@ -3244,7 +3303,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("kp") = py::none(), py::arg("vp") = py::none(),
         py::arg("q_norm") = py::none(), py::arg("k_norm") = py::none(),
         py::arg("norm_eps") = 1e-6,
-        py::arg("k_scale") = py::none(), py::arg("v_scale") = py::none());
+        py::arg("k_scale") = py::none(), py::arg("v_scale") = py::none(),
+        py::arg("sums") = py::none(), py::arg("bias") = py::none());
   m.def("attn_decode", &attn_decode, "GQA decode attention (flash-decoding split-KV)");
   m.def("attn_decode_mfma", &attn_decode_mfma,
         "GQA decode attention on matrix cores (packed cache, hd=128); "

@@ -204,21 +204,6 @@ __global__ __launch_bounds__((TileShape<BN, BM, BUFS>::WAVES * 64)) void tile_ke
 // what follows a product whose k was split: the parts' sums, in order
 // ---------------------------------------------------------------------------
 
-// four at a time on their way
-DEVINL floatx4 sum_parts(const float* p, size_t at, size_t stride, int splits) {
-  floatx4 v = *(const floatx4*)(p + at);
-  int s = 1;
-  for (; s + 3 < splits; s += 4) {
-    floatx4 q[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) q[i] = *(const floatx4*)(p + (s + i) * stride + at);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v += q[i];
-  }
-  for (; s < splits; ++s) v += *(const floatx4*)(p + s * stride + at);
-  return v;
-}
-
 // y = bf16 of the sums + bias; GATE: [m, 2 N] -> silu(gate) up [m, N]. N % 4 == 0.
 template <bool GATE>
 __global__ __launch_bounds__(256) void finish_kernel(const float* __restrict__ part, const bf16_t* __restrict__ bias,
