@@ -37,3 +37,18 @@ def test_prompt_by_tiles(T, E, k, D, I):
     assert sure.float().mean() > 0.99
     bound = size * 2.0 ** -7 + ref.abs() * 2.0 ** -8 + 1e-6
     assert bool(((out - ref).abs() <= bound)[sure].all())
+
+
+@pytest.mark.parametrize("T,E,k,D", [(1, 8, 2, 64), (33, 5, 3, 72), (256, 128, 8, 128)])
+def test_routes_of_bf16_logits_and_wide_sums(T, E, k, D):
+  """bf16 logits go as the same numbers in fp32 do; a wide sum is one that is not rounded yet."""
+  from xotorch_amd import ops
+  hip = ops._load_hip()
+  g = torch.Generator(device="cuda").manual_seed(T)
+  logits = torch.randn(T, E, generator=g, device="cuda").to(torch.bfloat16)
+  (idx, w), (idx2, w2) = hip.moe_route(logits, None, k, 0), hip.moe_route(logits.float(), None, k, 0)
+  assert torch.equal(idx, idx2) and torch.equal(w, w2)
+  gather, place = hip.moe_build(idx, E, (T + 31) // 32 * 32)
+  y = torch.randn(gather.numel(), D, generator=g, device="cuda").to(torch.bfloat16)
+  wide, rounded = hip.moe_combine(y, place, w, True), hip.moe_combine(y, place, w)
+  assert wide.dtype == torch.float32 and torch.equal(wide.to(torch.bfloat16), rounded)

@@ -438,7 +438,7 @@ class MoEMLP(nn.Module):
        or os.getenv("XOT_FP8_PREFILL", "0") == "1" or not ops._use_hip(flat):
       return False
     mods = [p for e in self.experts for p in (e.gate_up_proj, e.down_proj)]
-    return (type(self.gate) is nn.Linear and all(type(e) is MLP for e in self.experts)
+    return (type(self.gate) is nn.Linear and all(type(e) is MLP for e in self.experts) and not _watched(self.gate, *self.experts, *mods)
             and all(type(p) is XotLinear and p.bias is None for p in mods)
             and all(p.weight.dtype == torch.bfloat16 and p.weight.is_cuda and p.weight.is_contiguous()
                     and p.weight.data_ptr() % 16 == 0 for p in (self.gate, *mods)))
@@ -478,7 +478,8 @@ class MoEMLP(nn.Module):
     out.index_add_(0, tok_sorted, y)
     return out
 
-  def _forward_decode(self, flat):
+  def _forward_decode(self, flat, wide=False):
+    """[T, D]; `wide`: fp32, not rounded yet, for a sum with the residual stream."""
     T, D = flat.shape
     E, k = self.n_experts, self.top_k
     dev = flat.device
@@ -487,7 +488,9 @@ class MoEMLP(nn.Module):
     C = max(32, -(-T // 32) * 32)                             # capacity (lossless: count_e <= T)
     if hip0 is not None and flat.is_cuda:
       # fused router (softmax-topk-renorm in one launch)
-      logits = self.gate(flat).float()
+      logits = self.gate(flat)
+      if logits.dtype != torch.bfloat16:
+        logits = logits.float()
       selected, weights = hip0.moe_route(logits.contiguous(), None, self.top_k, 0)
     else:
       weights, selected = self._route(flat)                   # [T, k]
@@ -495,7 +498,6 @@ class MoEMLP(nn.Module):
       # single-launch counting-sort + deterministic combine (replaces the
       # argsort/cumsum/index_add torch glue — measured top MoE decode cost)
       gather_tok, inv_pos = hip0.moe_build(selected.to(torch.int32).contiguous(), E, C)
-      gather_tok = gather_tok.long()
       scale = None
     else:
       A = T * k
@@ -513,7 +515,7 @@ class MoEMLP(nn.Module):
       pos_c = pos.clamp(max=A - 1)
       gather_tok = sorted_token[pos_c.reshape(-1)]            # [E*C]
       scale = torch.where(valid, sorted_w[pos_c], torch.zeros((), dtype=sorted_w.dtype, device=dev))
-    xg = flat[gather_tok]                                     # [E*C, D]
+    xg = flat.index_select(0, gather_tok)                     # [E*C, D]
     if self.wp_gate_up_fp8 is not None and not torch.is_grad_enabled():
       from xotorch_amd.ops import _load_hip
       hip = _load_hip()
@@ -539,7 +541,7 @@ class MoEMLP(nn.Module):
       y = torch.cat(outs, dim=0)
     if scale is None:
       return hip0.moe_combine(y.view(E * C, D).to(torch.bfloat16).contiguous(), inv_pos,
-                              weights.float().contiguous()).float()
+                              weights.float().contiguous(), wide)
     out = torch.zeros(T, D, dtype=torch.float32, device=dev)
     out.index_add_(0, gather_tok, y.float() * scale.reshape(-1, 1))
     return out
@@ -587,6 +589,8 @@ class DecoderLayer(nn.Module):
     x, normed = ops.parts_add_norm(ops.tile_parts(out, a.o_proj.weight), x, post.weight, post.eps)
     if type(m) is MLP and m.by_tiles(normed):
       parts = ops.tile_parts(m.gated(normed), m.down_proj.weight)
+    elif type(m) is MoEMLP and not _watched(m):
+      parts = m._forward_decode(normed.view(-1, x.shape[-1]), True).float()
     else:
       parts = m(normed).float()
     parts = parts.view(-1, x.numel() // x.shape[-1], x.shape[-1])

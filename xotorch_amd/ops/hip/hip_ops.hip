@@ -1032,8 +1032,12 @@ __global__ __launch_bounds__(128) void attn_decode_merge(
 //         scores, keep topk_group groups) -> gather sigmoid weights ->
 //         optional renorm -> routed scaling (DeepSeek V2/V3).
 // Replaces ~4-10 torch launches per MoE layer per step. E <= 256, k <= 8.
+// Logits fp32, or bf16 as a projection leaves them.
+DEVINL float logit(const float* p, size_t i) { return p[i]; }
+DEVINL float logit(const unsigned short* p, size_t i) { return b2f(p[i]); }
+template <typename L>
 __global__ __launch_bounds__(256) void moe_route_kernel(
-    const float* __restrict__ logits, const float* __restrict__ bias,
+    const L* __restrict__ logits, const float* __restrict__ bias,
     int* __restrict__ idx, float* __restrict__ w,
     int T, int E, int k, int mode, int n_group, int topk_group,
     float routed_scale, int norm_topk) {
@@ -1045,7 +1049,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int e = lane * 4 + j;
-    v[j] = (e < E) ? logits[(size_t)row * E + e] : -INFINITY;
+    v[j] = (e < E) ? logit(logits, (size_t)row * E + e) : -INFINITY;
   }
   if (mode == 0) {
     // softmax over the row
@@ -1184,10 +1188,12 @@ __global__ __launch_bounds__(256) void moe_build_kernel(
   }
 }
 
-// out[t, :] = sum_j w[t, j] * y[inv_pos[t*k + j], :]   (fp32 accumulate)
+// out[t, :] = sum_j w[t, j] * y[inv_pos[t*k + j], :]   (fp32 accumulate); O: bf16, or
+// fp32 for a kernel that adds it to the residual stream
+template <typename O>
 __global__ __launch_bounds__(256) void moe_combine_kernel(
     const unsigned short* __restrict__ y, const int* __restrict__ inv_pos,
-    const float* __restrict__ w, unsigned short* __restrict__ out,
+    const float* __restrict__ w, O* __restrict__ out,
     int T, int k, int D) {
   const long long n8 = (long long)T * (D >> 3);
   const long long stride = (long long)gridDim.x * blockDim.x;
@@ -1204,10 +1210,14 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(
 #pragma unroll
       for (int q = 0; q < 8; ++q) acc[q] += wj * b2f(v[q]);
     }
-    ushort8 o;
+    typedef __attribute__((ext_vector_type(8))) O O8;
+    O8 o;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) o[q] = f2b(acc[q]);
-    *(ushort8*)(out + (size_t)t * D + c8) = o;
+    for (int q = 0; q < 8; ++q) {
+      if constexpr (sizeof(O) == 4) o[q] = acc[q];
+      else o[q] = f2b(acc[q]);
+    }
+    *(O8*)(out + (size_t)t * D + c8) = o;
   }
 }
 
@@ -2629,11 +2639,12 @@ torch::Tensor attn_prefill_mfma(torch::Tensor q, torch::Tensor k, torch::Tensor 
   return out;
 }
 
-// logits: [T, E] fp32 gate output -> (idx int32 [T,k], w fp32 [T,k]).
+// logits: [T, E] gate output, fp32 or bf16 -> (idx int32 [T,k], w fp32 [T,k]).
 std::vector<torch::Tensor> moe_route(torch::Tensor logits, c10::optional<torch::Tensor> bias,
                                      int64_t k, int64_t mode, int64_t n_group,
                                      int64_t topk_group, double routed_scale, bool norm_topk) {
-  CHK(logits.is_cuda() && logits.dtype() == torch::kFloat32 && logits.is_contiguous() && logits.dim() == 2);
+  const bool wide = logits.dtype() == torch::kFloat32;
+  CHK(logits.is_cuda() && (wide || logits.dtype() == torch::kBFloat16) && logits.is_contiguous() && logits.dim() == 2);
   const int T = logits.size(0), E = logits.size(1);
   CHK(E <= 256 && k >= 1 && k <= 8 && n_group >= 1 && n_group <= 8);
   const float* bptr = nullptr;
@@ -2645,10 +2656,15 @@ std::vector<torch::Tensor> moe_route(torch::Tensor logits, c10::optional<torch::
   auto fopts = torch::TensorOptions().dtype(torch::kFloat32).device(logits.device());
   auto idx = torch::empty({(long)T, (long)k}, iopts);
   auto w = torch::empty({(long)T, (long)k}, fopts);
-  hipLaunchKernelGGL(moe_route_kernel, dim3((T + 3) / 4), dim3(256), 0, cur_stream(),
-                     logits.data_ptr<float>(), bptr, idx.data_ptr<int>(), w.data_ptr<float>(),
-                     T, E, (int)k, (int)mode, (int)n_group, (int)topk_group,
-                     (float)routed_scale, norm_topk ? 1 : 0);
+  auto run = [&](auto* p) {
+    typedef std::remove_const_t<std::remove_pointer_t<decltype(p)>> L;
+    hipLaunchKernelGGL(moe_route_kernel<L>, dim3((T + 3) / 4), dim3(256), 0, cur_stream(),
+                       p, bptr, idx.data_ptr<int>(), w.data_ptr<float>(),
+                       T, E, (int)k, (int)mode, (int)n_group, (int)topk_group,
+                       (float)routed_scale, norm_topk ? 1 : 0);
+  };
+  if (wide) run((const float*)logits.data_ptr());
+  else run((const unsigned short*)logits.data_ptr());
   return {idx, w};
 }
 
@@ -2669,7 +2685,7 @@ std::vector<torch::Tensor> moe_build(torch::Tensor idx, int64_t E, int64_t C) {
 
 // y: [E*C, D] bf16 expert outputs, inv_pos [T,k] int32, w [T,k] fp32 ->
 // out [T, D] bf16 (deterministic weighted combine, no atomics).
-torch::Tensor moe_combine(torch::Tensor y, torch::Tensor inv_pos, torch::Tensor w) {
+torch::Tensor moe_combine(torch::Tensor y, torch::Tensor inv_pos, torch::Tensor w, bool wide) {
   CHK(y.is_cuda() && y.dtype() == torch::kBFloat16 && y.is_contiguous());
   CHK(inv_pos.dtype() == torch::kInt32 && inv_pos.is_contiguous());
   CHK(w.dtype() == torch::kFloat32 && w.is_contiguous());
@@ -2677,12 +2693,17 @@ torch::Tensor moe_combine(torch::Tensor y, torch::Tensor inv_pos, torch::Tensor 
   const int D = y.size(-1);
   CHK(D % 8 == 0);
   auto out = torch::empty({(long)T, (long)D},
-                          torch::TensorOptions().dtype(torch::kBFloat16).device(y.device()));
+                          torch::TensorOptions().dtype(wide ? torch::kFloat32 : torch::kBFloat16).device(y.device()));
   const long long n8 = (long long)T * (D / 8);
   const int blocks = (int)std::min<long long>(1024, (n8 + 255) / 256);
-  hipLaunchKernelGGL(moe_combine_kernel, dim3(blocks), dim3(256), 0, cur_stream(),
-                     (const unsigned short*)y.data_ptr(), inv_pos.data_ptr<int>(),
-                     w.data_ptr<float>(), (unsigned short*)out.data_ptr(), T, k, D);
+  if (wide)
+    hipLaunchKernelGGL(moe_combine_kernel<float>, dim3(blocks), dim3(256), 0, cur_stream(),
+                       (const unsigned short*)y.data_ptr(), inv_pos.data_ptr<int>(),
+                       w.data_ptr<float>(), (float*)out.data_ptr(), T, k, D);
+  else
+    hipLaunchKernelGGL(moe_combine_kernel<unsigned short>, dim3(blocks), dim3(256), 0, cur_stream(),
+                       (const unsigned short*)y.data_ptr(), inv_pos.data_ptr<int>(),
+                       w.data_ptr<float>(), (unsigned short*)out.data_ptr(), T, k, D);
   return out;
 }
 
@@ -3324,7 +3345,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_build", &moe_build,
         "MoE decode routing: counting-sort token-expert pairs to padded per-expert slots");
   m.def("moe_combine", &moe_combine,
-        "MoE decode combine: out[t] = sum_j w[t,j] * y[pos(t,j)] (deterministic)");
+        "MoE decode combine: out[t] = sum_j w[t,j] * y[pos(t,j)] (deterministic)",
+        py::arg("y"), py::arg("inv_pos"), py::arg("w"), py::arg("wide") = false);
   m.def("mla_q_prep", &mla_q_prep,
         "MLA absorbed-query finisher: rope the 64-dim tail + assemble [B,H,576]; "
         "fp8=True returns (q8, per-head scales)",
