@@ -56,6 +56,7 @@ def test_decode_attend(B, H, KVH, hd, T, lens, norms, shared):
 @pytest.mark.parametrize("B,S,H,KVH,hd,n,bias,norms", [(1, 1, 1, 1, 64, 1, False, False), (3, 1, 28, 4, 128, 7, True, False),
                                                        (2, 1, 16, 1, 64, 16, True, True), (5, 1, 8, 8, 128, 5, False, True),
                                                        (1, 45, 32, 8, 64, 9, False, False), (2, 33, 7, 1, 128, 4, True, True),
+                                                       (3, 71, 32, 8, 128, 3, True, False), (2, 99, 32, 8, 64, 2, False, False),
                                                        (130, 1, 4, 4, 128, 2, True, False)])
 def test_sums_over_parts_of_k(B, S, H, KVH, hd, n, bias, norms):
   """The same numbers as from the tensor that they add up to, in order, rounded."""
@@ -86,6 +87,39 @@ def test_sums_over_parts_of_k(B, S, H, KVH, hd, n, bias, norms):
     found.append((out, *c[:4]))
   for x, y in zip(*found):
     assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("B,S,H,KVH,hd,per_row,norms", [(1, 1027, 4, 1, 128, False, True), (3, 333, 30, 2, 64, True, False),
+                                                        (2, 515, 9, 3, 128, True, True)])
+def test_rows_of_prompts_as_one_by_one(B, S, H, KVH, hd, per_row, norms):
+  """Many tokens, several to a wave, against a wave a token (few of them at a time)."""
+  from xotorch_amd import ops
+  from xotorch_amd.engine.kvcache import ShardKVCache
+  from xotorch_amd.ops import torch_ref
+  g = torch.Generator(device="cuda").manual_seed(S)
+  T = S + 70
+  cos, sin = torch_ref.rope_cos_sin(hd, T, 10000.0, device="cuda")
+  qkv = torch.randn(B, S, (H + 2 * KVH) * hd, generator=g, device="cuda").to(torch.bfloat16)
+  qn, kn = (torch.randn(hd, generator=g, device="cuda").to(torch.bfloat16) for _ in "qk") if norms else (None, None)
+  pos = torch.arange(5, 5 + S, dtype=torch.int32, device="cuda")
+  if per_row:
+    pos = torch.stack([pos + 17 * b for b in range(B)])
+  found = []
+  for step in (S, 16):
+    c = ShardKVCache(1, B, KVH, T, hd, torch.bfloat16, "cuda")[0]
+    queries = []
+    for at in range(0, S, step):
+      part = qkv[:, at:at + step].clone()
+      ops.rope_qkv_append(part, cos, sin, pos[..., at:at + step].contiguous(), c.k, c.v, H, KVH, hd, c.kp, c.vp, qn, kn, 1e-6)
+      queries.append(part[..., :H * hd])
+    found.append((torch.cat(queries, 1), *c[:4]))
+  for n, (x, y) in enumerate(zip(*found)):
+    # values as they are; x cos - y sin may be contracted either way, which is off by 2^-23 of
+    # terms up to 8 and a step of bf16 then, rarely; a norm's sums are in another order
+    if n in (2, 4):
+      assert torch.equal(x, y)
+    assert bool(((x.float() - y.float()).abs() <= y.float().abs() * 2.0 ** -7 + 2.0 ** -20).all())
+    assert (x != y).float().mean() < 0.01
 
 
 def test_parked_row_keeps_to_its_own_place():

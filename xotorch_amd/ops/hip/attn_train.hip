@@ -30,9 +30,14 @@ struct TrainArgs {
   float *o, *lse, *delta;   // fp32 [B, S, H HD]; [B][H][S32], lse to base 2
   const float *cos, *sin;
   const int* positions;
-  int B, S, S32, H, KVH, per_row;
+  int B, S, S32, H, KVH, per_row, places;  // places: rows of the rotation's tables
   float scale;
 };
+
+// where a token stands, within the tables
+DEVINL int place(const TrainArgs& a, int b, int s) {
+  return min(max(a.positions[a.per_row ? b * a.S + s : s], 0), a.places - 1);
+}
 
 // The 32 rows of one head from tile s0 on, in LDS, to both orders
 template <int HD>
@@ -67,7 +72,7 @@ __global__ __launch_bounds__(256) void pack_qkv_kernel(TrainArgs a) {
       ld4(src + HD / 2, x2);
       if (slot < a.H + a.KVH) {
         float co[4], si[4];
-        const int pos = a.positions[a.per_row ? b * a.S + s : s];
+        const int pos = place(a, b, s);
         ld4(a.cos + (size_t)pos * (HD / 2) + c, co);
         ld4(a.sin + (size_t)pos * (HD / 2) + c, si);
 #pragma unroll
@@ -275,7 +280,7 @@ __global__ __launch_bounds__(256, 2) void train_forward_kernel(TrainArgs a) {
 template <int HD>
 DEVINL void turn_back(const TrainArgs& a, floatx4* o, int b, int s, int quad, bf16_t* dst, bool turn) {
   constexpr int VG = HD / 16;
-  const size_t at = turn ? (size_t)a.positions[a.per_row ? b * a.S + s : s] * (HD / 2) + quad * 4 : 0;
+  const size_t at = turn ? (size_t)place(a, b, s) * (HD / 2) + quad * 4 : 0;
 #pragma unroll
   for (int g = 0; g < VG / 2; ++g) {
     float y1[4], y2[4];
@@ -480,7 +485,7 @@ static TrainArgs train_args(const Tensor& qkv, const Tensor& cos, const Tensor& 
   CHK((hd == 64 || hd == 128) && H >= 1 && KVH >= 1 && H % KVH == 0);
   CHK(qkv.dim() == 3 && qkv.size(2) == (H + 2 * KVH) * hd && qkv.numel() > 0);
   const int64_t B = qkv.size(0), S = qkv.size(1), S32 = (S + 31) / 32 * 32;
-  CHK(cos.size(-1) == hd / 2 && sin.sizes() == cos.sizes() && (positions.numel() == S || positions.numel() == B * S));
+  CHK(cos.size(-1) == hd / 2 && cos.numel() > 0 && cos.numel() <= INT_MAX && sin.sizes() == cos.sizes() && (positions.numel() == S || positions.numel() == B * S));
   CHK((((size_t)qkv.data_ptr() | (size_t)cos.data_ptr() | (size_t)sin.data_ptr()) & 15) == 0);
   CHK(B <= 65535 && H + 2 * KVH <= 65535 && B * S * (H + 2 * KVH) <= INT_MAX / 4);
   TrainArgs a{};
@@ -494,6 +499,7 @@ static TrainArgs train_args(const Tensor& qkv, const Tensor& cos, const Tensor& 
   a.H = (int)H;
   a.KVH = (int)KVH;
   a.per_row = positions.numel() == B * S && B > 1;
+  a.places = (int)(cos.numel() / (hd / 2));
   a.scale = 1.f / sqrtf((float)hd);
   return a;
 }

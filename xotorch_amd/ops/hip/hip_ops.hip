@@ -319,6 +319,108 @@ __global__ __launch_bounds__(256) void rope_qkv_append_kernel(
   }
 }
 
+// The same for head dims 64 and 128 without fp8 copies: a wave has 8 or 4 tokens of one
+// head, a lane 4 channels and their partners, so that rows move in pieces of 8 bytes.
+// Bound by memory and by the waves' starts: 6001 tokens of 48 heads of 128 48 us (170 MB;
+// 75 with a wave a token), 8192 of 80 89 us (171).
+struct RopeRows {
+  const float* sums;  // or null: fp32 sums over nsums parts of k [nsums][B*S][slots*HD]
+  const unsigned short* bias;
+  unsigned short* qkv;
+  const float *cosb, *sinb;
+  const int* positions;
+  unsigned short *kc, *vc, *kpc, *vpc;
+  const unsigned short *qn, *kn;
+  int nsums, B, S, H, KVH, T, T32, per_row;
+  float eps;
+};
+template <int HD, bool SUMS>
+__global__ __launch_bounds__(256) void rope_rows_kernel(RopeRows a) {
+  constexpr int HALF = HD / 2, LANES = HALF / 4, ROWS = 64 / LANES;
+  const int lane = threadIdx.x & 63, slots = a.H + 2 * a.KVH, rows = a.B * a.S;
+  const int unit = blockIdx.x * 4 + (threadIdx.x >> 6), slot = unit % slots;
+  const int bs = unit / slots * ROWS + lane / LANES, d = lane % LANES * 4;
+  if (bs >= rows) return;
+  const int b = bs / a.S, s = bs - b * a.S, pos = a.positions[a.per_row ? bs : s];
+  unsigned short* row = a.qkv + ((size_t)bs * slots + slot) * HD + d;
+  float x[2][4];
+  ushort4_t y[2];  // as projected, then rotated
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    if (SUMS) {
+      const size_t width = (size_t)slots * HD, stride = rows * width, at = (size_t)slot * HD + d + h * HALF;
+      const float* p = a.sums + bs * width + at;
+      floatx4 v = *(const floatx4*)p;
+      int i = 1;
+      for (; i + 3 < a.nsums; i += 4) {
+        floatx4 w[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] = *(const floatx4*)(p + (i + j) * stride);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v += w[j];
+      }
+      for (; i < a.nsums; ++i) v += *(const floatx4*)(p + i * stride);
+      if (a.bias) {
+        const ushort4_t c = *(const ushort4_t*)(a.bias + at);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] += b2f(c[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[h][j] = f2b(v[j]);
+    } else
+      y[h] = *(const ushort4_t*)(row + h * HALF);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[h][j] = b2f(y[h][j]);
+  }
+  if (slot < a.H + a.KVH) {
+    const unsigned short* w = slot < a.H ? a.qn : a.kn;
+    if (w) {
+      float ss = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) ss += x[0][j] * x[0][j] + x[1][j] * x[1][j];
+#pragma unroll
+      for (int m = LANES / 2; m > 0; m >>= 1) ss += __shfl_xor(ss, m);
+      const float inv = rsqrtf(ss / (float)HD + a.eps);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const ushort4_t by = *(const ushort4_t*)(w + d + h * HALF);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[h][j] *= inv * b2f(by[j]);
+      }
+    }
+    const floatx4 c = *(const floatx4*)(a.cosb + (size_t)pos * HALF + d), sn = *(const floatx4*)(a.sinb + (size_t)pos * HALF + d);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      y[0][j] = f2b(x[0][j] * c[j] - x[1][j] * sn[j]);
+      y[1][j] = f2b(x[1][j] * c[j] + x[0][j] * sn[j]);
+    }
+  }
+  if (slot < a.H) {
+    *(ushort4_t*)row = y[0];
+    *(ushort4_t*)(row + HALF) = y[1];
+    return;
+  }
+  const bool key = slot < a.H + a.KVH;
+  const size_t head = (size_t)b * a.KVH + (slot - a.H - (key ? 0 : a.KVH));
+  unsigned short* dst = (key ? a.kc : a.vc) + (head * a.T + pos) * HD + d;
+  *(ushort4_t*)dst = y[0];
+  *(ushort4_t*)(dst + HALF) = y[1];
+  if (!a.kpc) return;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int e = d + h * HALF;
+    if (key)
+      *(ushort4_t*)(a.kpc + (head * (a.T32 >> 4) + (pos >> 4)) * (HD / 32 * 512) + (e >> 5) * 512 +
+                   (((e & 31) >> 3) * 16 + (pos & 15)) * 8 + (e & 7)) = y[h];
+    else
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        a.vpc[((head * (HD / 16) + (e >> 4)) * (a.T32 >> 5) + (pos >> 5)) * 512 +
+              (((pos & 31) >> 3) * 16 + (e & 15) + j) * 8 + (pos & 7)] = y[h][j];
+  }
+}
+
+
 // ---------------------------------------------------------------------------
 // GQA decode attention (flash-decoding): split-KV partials + merge.
 //
@@ -2447,6 +2549,21 @@ void rope_qkv_append(torch::Tensor qkv, torch::Tensor cos, torch::Tensor sin,
       CHK(bias->is_cuda() && bias->dtype() == torch::kBFloat16 && bias->is_contiguous() && bias->numel() == qkv.size(2));
       bp = (const unsigned short*)bias->data_ptr();
     }
+  }
+  auto at = [](const void* p) { return (size_t)p; };
+  // a wave a token where tokens are few: with 8 parts, 45 rows of 48 heads of 64 4.6 us, by
+  // rows (288 waves) 5.8; 256 rows of 36 heads of 128 (2304 waves) 10.9 and 9.4
+  const long long units = (long long)((B * S + 512 / hd - 1) / (512 / hd)) * (H + 2 * KVH);
+  if ((hd == 64 || hd == 128) && !kp8 && units >= 1024 &&
+      ((at(qkv.data_ptr()) | at(kc.data_ptr()) | at(vc.data_ptr()) | at(kpc) | at(qnp) | at(knp) | at(bp)) & 7) == 0 &&
+      ((at(cos.data_ptr()) | at(sin.data_ptr()) | at(sp)) & 15) == 0) {
+    RopeRows a{sp, bp, (unsigned short*)qkv.data_ptr(), cos.data_ptr<float>(), sin.data_ptr<float>(), positions.data_ptr<int>(),
+               (unsigned short*)kc.data_ptr(), (unsigned short*)vc.data_ptr(), kpc, vpc, qnp, knp, nsums, B, S, H, KVH, T, T32,
+               npos == B * S && npos != S, (float)norm_eps};
+    auto rows_kernel = hd == 128 ? (sp ? rope_rows_kernel<128, true> : rope_rows_kernel<128, false>)
+                                 : (sp ? rope_rows_kernel<64, true> : rope_rows_kernel<64, false>);
+    hipLaunchKernelGGL(rows_kernel, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, cur_stream(), a);
+    return;
   }
   auto kernel = sp ? rope_qkv_append_kernel<true> : rope_qkv_append_kernel<false>;
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, cur_stream(), sp, bp, nsums,

@@ -158,7 +158,7 @@ __global__ __launch_bounds__(256) void swiglu_backward_kernel(const bf16_t* __re
 struct HeadArgs {
   const float *cos, *sin;
   const int* positions;
-  int B, S, H, KVH, hd, per_row;  // per_row: positions [B, S], else [S]
+  int B, S, H, KVH, hd, per_row, places;  // per_row: positions [B, S], else [S]; places: rows of the tables
 };
 
 __global__ __launch_bounds__(256) void split_heads_kernel(const bf16_t* __restrict__ qkv, float* __restrict__ q,
@@ -175,7 +175,7 @@ __global__ __launch_bounds__(256) void split_heads_kernel(const bf16_t* __restri
   ld4(src + half, x2);
   if (slot < a.H + a.KVH) {
     float co[4], si[4];
-    const int pos = a.positions[a.per_row ? tok : s];
+    const int pos = min(max(a.positions[a.per_row ? tok : s], 0), a.places - 1);
     ld4(a.cos + (size_t)pos * half + c, co);
     ld4(a.sin + (size_t)pos * half + c, si);
 #pragma unroll
@@ -220,7 +220,7 @@ __global__ __launch_bounds__(256) void split_heads_backward_kernel(const float* 
   }
   if (slot < a.H + a.KVH) {
     float co[4], si[4];
-    const int pos = a.positions[a.per_row ? tok : s];
+    const int pos = min(max(a.positions[a.per_row ? tok : s], 0), a.places - 1);
     ld4(a.cos + (size_t)pos * half + c, co);
     ld4(a.sin + (size_t)pos * half + c, si);
 #pragma unroll
@@ -314,11 +314,11 @@ static HeadArgs head_args(const Tensor& cos, const Tensor& sin, const Tensor& po
   check_16(cos, torch::kFloat32);
   check_16(sin, torch::kFloat32);
   check_io(positions, torch::kInt32);
-  CHK(H >= 1 && KVH >= 1 && H % KVH == 0 && hd % 8 == 0 && cos.size(-1) == hd / 2 && sin.sizes() == cos.sizes());
+  CHK(H >= 1 && KVH >= 1 && H % KVH == 0 && hd % 8 == 0 && cos.size(-1) == hd / 2 && cos.numel() > 0 && cos.numel() <= INT_MAX && sin.sizes() == cos.sizes());
   CHK(positions.numel() == S || positions.numel() == B * S);
   CHK(B <= INT_MAX && S <= INT_MAX && B * S * (H + 2 * KVH) * (hd / 8) / 256 < INT_MAX);
   return HeadArgs{cos.data_ptr<float>(), sin.data_ptr<float>(), positions.data_ptr<int>(), (int)B, (int)S, (int)H, (int)KVH,
-                  (int)hd, positions.numel() == B * S && B > 1};
+                  (int)hd, positions.numel() == B * S && B > 1, (int)(cos.numel() / (hd / 2))};
 }
 
 // -> q, k, v fp32 [B, H, S, hd]
