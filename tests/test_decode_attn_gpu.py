@@ -158,3 +158,34 @@ def test_prompt_attention_of_64_channels(S, H, KVH, start):
   p = s.masked_fill(later, -torch.inf).softmax(-1)
   ref, size = (p @ v).transpose(1, 2), (p @ v.abs()).transpose(1, 2)
   assert bool(((out - ref).abs() <= size * 2.0 ** -7 * 1.05 + ref.abs() * 2.0 ** -8 + 1e-6).all())
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("place", [300, -3])
+def test_parked_row_reads_within_the_tables(hd, place):
+  """Tables of as many rows as the cache has positions: a row that stands elsewhere is
+  not appended, and turned by the nearest row that they have."""
+  from xotorch_amd import ops
+  from xotorch_amd.engine.kvcache import ShardKVCache
+  from xotorch_amd.ops import torch_ref
+  T, H, KVH, n = 256, 4, 2, 64
+  g = torch.Generator(device="cuda").manual_seed(1)
+  cos, sin = torch_ref.rope_cos_sin(hd, T, 10000.0, device="cuda")
+  c = ShardKVCache(1, 1, KVH, T, hd, torch.bfloat16, "cuda")[0]
+  rows = torch.randn(1, n, (H + 2 * KVH) * hd, generator=g, device="cuda").to(torch.bfloat16)
+  ops.rope_qkv_append(rows, cos, sin, torch.arange(n, dtype=torch.int32, device="cuda"), c.k, c.v, H, KVH, hd, c.kp, c.vp)
+  qkv = torch.randn(1, 1, (H + 2 * KVH) * hd, generator=g, device="cuda").to(torch.bfloat16)
+  before = [t.clone() for t in c[:4]]
+  out = ops.decode_attend(qkv, cos, sin, torch.tensor([place], dtype=torch.int32, device="cuda"),
+                          torch.tensor([n], dtype=torch.int32, device="cuda"), *c[:4], H, KVH)
+  assert all(torch.equal(a, b) for a, b in zip(c[:4], before))
+  at = min(max(place, 0), T - 1)
+  q = qkv[0, 0, :H * hd].view(H, hd).double()
+  q1, q2 = q.chunk(2, -1)
+  q = torch.cat([q1 * cos[at] - q2 * sin[at], q2 * cos[at] + q1 * sin[at]], -1)
+  k, v = (t[0, :, :n].double().repeat_interleave(H // KVH, 0) for t in (c.k, c.v))
+  s = (k @ q[..., None])[..., 0] * hd ** -0.5
+  off = (k.abs() @ q.abs()[..., None])[..., 0].amax(-1, keepdim=True) * hd ** -0.5 * 2.0 ** -8  # queries are rounded
+  p = s.softmax(-1)
+  ref, size = (p[:, None] @ v)[:, 0], (p[:, None] @ v.abs())[:, 0]
+  assert bool(((out.view(H, hd).double() - ref).abs() <= size * (2.0 ** -7 + 4 * off) + ref.abs() * 2.0 ** -8).all())

@@ -26,9 +26,12 @@ struct DecodeArgs {
   const bf16_t* bias;
   int nsums;
   float *part, *ml;  // [B H][splits][HD], [B H][splits][2]
-  int B, H, KVH, T, T32, npos, splits;
+  int B, H, KVH, T, T32, npos, splits, places;  // places: rows of the rotation's tables
   float scale, eps;  // scale times log2 e
 };
+
+// Where the rotation's tables are read: a parked row may stand past their end
+DEVINL size_t angle_row(const DecodeArgs& a, int pos) { return (size_t)min(max(pos, 0), a.places - 1); }
 
 typedef __attribute__((ext_vector_type(4))) unsigned int uintx4;
 
@@ -52,7 +55,8 @@ DEVINL void append(const DecodeArgs& a, int b, int kvh, int pos, int lane, const
   bf16_t* kp = a.kp + (head * (a.T32 >> 4) + (pos >> 4)) * (HD / 32 * 512);
   bf16_t *kc = a.kc + (head * a.T + pos) * HD, *vc = a.vc + (head * a.T + pos) * HD;
   if (on) {
-    const float c = a.cos[(size_t)pos * HALF + lane], s = a.sin[(size_t)pos * HALF + lane];
+    const size_t at = angle_row(a, pos) * HALF + lane;
+    const float c = a.cos[at], s = a.sin[at];
     const bf16_t r[2] = {f2b(x1 * c - x2 * s), f2b(x2 * c + x1 * s)};
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -142,7 +146,8 @@ __global__ __launch_bounds__(WAVES * 64) void decode_attn_kernel(DecodeArgs a) {
     }
 #pragma unroll
     for (int c = 0; c < KC / 2; ++c) {
-      const float *cs = a.cos + (size_t)pos * HALF + c * 32 + quad * 8, *sn = a.sin + (size_t)pos * HALF + c * 32 + quad * 8;
+      const size_t at = angle_row(a, pos) * HALF + c * 32 + quad * 8;
+      const float *cs = a.cos + at, *sn = a.sin + at;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const float x1 = x[c][j], x2 = x[c + KC / 2][j];
@@ -329,7 +334,8 @@ Tensor decode_attend(Tensor qkv, Tensor cos, Tensor sin, Tensor positions, Tenso
   a.T32 = (int)kp.size(2) * 16;
   CHK(kc.size(1) == kv_heads && vc.sizes() == kc.sizes() && a.T <= a.T32 && a.T32 % 32 == 0);
   CHK(kp.numel() == kp.size(0) * kv_heads * a.T32 * HD && vp.numel() == vp.size(0) * kv_heads * a.T32 * HD);
-  CHK(cos.size(-1) == HD / 2 && sin.sizes() == cos.sizes());
+  CHK(cos.size(-1) == HD / 2 && cos.numel() > 0 && cos.numel() <= INT_MAX && sin.sizes() == cos.sizes());
+  a.places = (int)(cos.numel() / (HD / 2));
   a.npos = (int)positions.numel();
   CHK((a.npos == 1 || a.npos == a.B) && lens.numel() == a.B);
   CHK((int64_t)a.B * kv_heads * 64 <= INT_MAX);
