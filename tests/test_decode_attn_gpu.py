@@ -189,3 +189,18 @@ def test_parked_row_reads_within_the_tables(hd, place):
   p = s.softmax(-1)
   ref, size = (p[:, None] @ v)[:, 0], (p[:, None] @ v.abs())[:, 0]
   assert bool(((out.view(H, hd).double() - ref).abs() <= size * (2.0 ** -7 + 4 * off) + ref.abs() * 2.0 ** -8).all())
+
+
+@pytest.mark.parametrize("hd,T", [(64, 64), (64, 3000), (128, 3000)])
+def test_nan_is_seen(hd, T):
+  """A query that is not a number gives outputs that are not, in one block or several."""
+  from xotorch_amd import ops
+  from xotorch_amd.engine.kvcache import ShardKVCache
+  H, KVH = 4, 1
+  c = ShardKVCache(1, 1, KVH, T, hd, torch.bfloat16, "cuda")[0]
+  still, none = torch.ones(T, hd // 2, device="cuda"), torch.zeros(T, hd // 2, device="cuda")
+  qkv = torch.ones(1, 1, (H + 2 * KVH) * hd, device="cuda", dtype=torch.bfloat16)
+  qkv[0, 0, hd] = float("nan")
+  at = torch.tensor([T - 1], dtype=torch.int32, device="cuda")
+  out = ops.decode_attend(qkv, still, none, at, at + 1, *c[:4], H, KVH).view(H, hd)
+  assert bool(out[1].isnan().all()) and bool(torch.isfinite(out[[0, 2, 3]]).all())

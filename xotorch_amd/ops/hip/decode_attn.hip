@@ -271,7 +271,7 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeArgs a) {
     }
   }
 #pragma unroll
-  for (int i = 0; i < HD / 64; ++i) st(a.out + (size_t)row * HD + i * 64 + lane, sum > 0.f ? o[i] / sum : 0.f);
+  for (int i = 0; i < HD / 64; ++i) st(a.out + (size_t)row * HD + i * 64 + lane, sum == 0.f ? 0.f : o[i] / sum);  // NaN stays
 }
 
 // ===========================================================================
