@@ -204,3 +204,25 @@ def test_nan_is_seen(hd, T):
   at = torch.tensor([T - 1], dtype=torch.int32, device="cuda")
   out = ops.decode_attend(qkv, still, none, at, at + 1, *c[:4], H, KVH).view(H, hd)
   assert bool(out[1].isnan().all()) and bool(torch.isfinite(out[[0, 2, 3]]).all())
+
+
+@pytest.mark.parametrize("B,H,KVH,T,n", [(1, 32, 8, 256, 221), (3, 16, 1, 96, 65), (1, 8, 2, 7000, 6999)])
+def test_probabilities_of_64_channels_stay_fp32(B, H, KVH, T, n):
+  from xotorch_amd import ops
+  from xotorch_amd.engine.kvcache import ShardKVCache
+  g = torch.Generator(device="cuda").manual_seed(n)
+  c = ShardKVCache(1, B, KVH, T, 64, torch.bfloat16, "cuda")[0]
+  still, none = torch.ones(T, 32, device="cuda"), torch.zeros(T, 32, device="cuda")
+  rows = torch.randn(B, n, (H + 2 * KVH) * 64, generator=g, device="cuda").to(torch.bfloat16)
+  ops.rope_qkv_append(rows.clone(), still, none, torch.arange(n, dtype=torch.int32, device="cuda"), c.k, c.v, H, KVH, 64, c.kp, c.vp)
+  qkv = rows[:, -1:].contiguous()
+  at = torch.full((B,), n - 1, dtype=torch.int32, device="cuda")
+  out = ops.decode_attend(qkv, still, none, at, at + 1, *c[:4], H, KVH).view(B, KVH, H // KVH, 64).double()
+  q = qkv[:, 0, :H * 64].view(B, KVH, H // KVH, 64).double()
+  k, v = c.k[:, :, :n].double(), c.v[:, :, :n].double()
+  s = q @ k.transpose(-1, -2).contiguous() * 0.125
+  off = (q.abs() @ k.abs().transpose(-1, -2).contiguous()).amax(-1, keepdim=True) * 0.125 * 68 * 2.0 ** -24
+  p = s.softmax(-1)
+  ref, size = p @ v, p @ v.abs()
+  # the result's rounding, and errors of fp32 scores and sums: nothing of the size of a bf16 probability's
+  assert bool(((out - ref).abs() <= ref.abs() * 2.0 ** -8 * 1.01 + size * (4 * off + 2.0 ** -18)).all())

@@ -121,21 +121,6 @@ __global__ __launch_bounds__(256) void pack_dout_kernel(TrainArgs a) {
   pack_tile<HD>(tile, a.dr + at, a.dt + at, s0, a.S32);
 }
 
-// 8 fp32 numbers as three bf16 operands that add up to them
-DEVINL void split3(const float* v, bf16x8* p) {
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const __bf16 a = (__bf16)v[i];
-    const float r = v[i] - (float)a;
-    const __bf16 b = (__bf16)r;
-    p[0][i] = a;
-    p[1][i] = b;
-    p[2][i] = (__bf16)(r - (float)b);
-  }
-}
-// += m times the three parts, the smallest first
-DEVINL floatx4 mma3(const bf16x8& m, const bf16x8* p, floatx4 c) { return mma(m, p[0], mma(m, p[1], mma(m, p[2], c))); }
-
 // Fragments of 16 rows in order, and of 32 rows in the order for the next product
 // (row i of product hf is i / 4 * 8 + i % 4 + 4 hf)
 template <int HD>

@@ -174,6 +174,20 @@ DEVINL floatx4 mma(const floatx4& a, const floatx4& b, floatx4 c) {
   for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
   return c;
 }
+// 8 fp32 numbers as three bf16 operands that add up to them
+DEVINL void split3(const float* v, bf16x8* p) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const __bf16 a = (__bf16)v[i];
+    const float r = v[i] - (float)a;
+    const __bf16 b = (__bf16)r;
+    p[0][i] = a;
+    p[1][i] = b;
+    p[2][i] = (__bf16)(r - (float)b);
+  }
+}
+// += m times the three parts, the smallest first
+DEVINL floatx4 mma3(const bf16x8& m, const bf16x8* p, floatx4 c) { return mma(m, p[0], mma(m, p[1], mma(m, p[2], c))); }
 // a lane's elements k.. of a row of n; WHOLE: n is a multiple of the step
 template <typename T, bool WHOLE>
 DEVINL typename Frag<T>::V ld_frag(const T* row, int k, int n) {

@@ -11,6 +11,9 @@
 // probabilities feeds them to the value product. Parts are cut by the row's own
 // length, so that short rows of a ragged batch have as many blocks as long ones.
 //
+// Probabilities of 64-channel heads stay fp32, as three bf16 parts that hold all their
+// bits; those of 128-channel heads are rounded, as in the kernels of that size before.
+//
 // The projection may come as fp32 sums over parts of k (tile_ops.hip): a block adds up
 // its heads' numbers in LDS, which saves a kernel between the two: 2.4 us of its 4.7 in
 // every layer (8 rows through 28 layers of 3584: 3285 to 3215 us).
@@ -198,12 +201,22 @@ __global__ __launch_bounds__(WAVES * 64) void decode_attn_kernel(DecodeArgs a) {
 #pragma unroll
       for (int g = 0; g < VG; ++g) o[g] *= f;
     }
-    bf16x8 pf;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) pf[i] = (__bf16)__builtin_amdgcn_exp2f(v[i] - m);
-    l = mma(ones, pf, l);
+    for (int i = 0; i < 8; ++i) v[i] = __builtin_amdgcn_exp2f(v[i] - m);
+    if constexpr (HD == 64) {
+      bf16x8 pf[3];
+      split3(v, pf);
+      l = mma3(ones, pf, l);
 #pragma unroll
-    for (int g = 0; g < VG; ++g) o[g] = mma(vf[g], pf, o[g]);
+      for (int g = 0; g < VG; ++g) o[g] = mma3(vf[g], pf, o[g]);
+    } else {
+      bf16x8 pf;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) pf[i] = (__bf16)v[i];
+      l = mma(ones, pf, l);
+#pragma unroll
+      for (int g = 0; g < VG; ++g) o[g] = mma(vf[g], pf, o[g]);
+    }
   }
   if (quad == 0) {
     lm[wave][col] = m;
