@@ -598,7 +598,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, int64_t> route(Tensor x, Tens
   BY_TYPE(dt, {
     const T* cp = correction ? P<T>(*correction) : nullptr;
     auto run = [&](auto kernel, int waves) {
-      static const hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+      const hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
       TORCH_CHECK(err == hipSuccess, "no LDS for the router");
       const size_t lds = (2 * RT * E + waves * RT * 65) * sizeof(float) + RT * (top + 1) * sizeof(int);  // parts of 16 bytes
       hipLaunchKernelGGL(kernel, dim3(nblk), dim3(64 * waves), lds, stream, P<T>(x), P<T>(w), cp,
@@ -628,7 +628,7 @@ static void launch_tiles(const W& w, const Tensor& x, const Tensor& token, const
   const dim3 grid((max_tiles + 8 * group - 1) / (8 * group) * 8 * group * nf);
   CHK(tile == 128 || tile == 256);
   auto run = [&](auto kernel, int threads, int lds) {
-    static const hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    const hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     TORCH_CHECK(err == hipSuccess, "no LDS for expert tiles");
     hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, cur_stream(), P<bf16_t>(x), w, first.data_ptr<int>(),
                        token.data_ptr<int>(), (const int2*)tiles.data_ptr<int>(), by_row, M<bf16_t>(y), max_tiles, group, a, act);

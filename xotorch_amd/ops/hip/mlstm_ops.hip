@@ -769,7 +769,7 @@ static void prompt(const Tensor& proj, const Tensor& u, const Tensor& r, const T
   const bool vec = ((a.dim | a.vdim | a.N | a.q_at | a.k_at | a.v_at | a.g_at | a.K | a.out_at) & 3) == 0;
   if (!vec) { a.seg = chunks; a.nseg = 1; }
   auto run = [&](auto kernel, bool outputs) {
-    static const hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    const hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     TORCH_CHECK(err == hipSuccess, "no LDS for the memory's chunks");
     const size_t lds = Sh::lds(waves, outputs);
     TORCH_CHECK(lds <= 160 * 1024, "a memory of ", a.dim, " by ", a.vdim, " channels does not fit LDS");
