@@ -1,0 +1,50 @@
+"""Which calls go to the kernels: those that can read their operands and that nobody follows."""
+import pytest
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+
+BF = torch.bfloat16
+
+
+def test_fake_tensors_are_not_read_in_training():
+  from xotorch_amd.models.llama import XotLinear
+  from xotorch_amd.ops import train_ops
+  from xotorch_amd.train.lora import LoRALinear
+  with FakeTensorMode():
+    x = torch.empty(2, 3, 512, dtype=BF, device="cuda", requires_grad=True)
+    w = torch.nn.Parameter(torch.empty(512, dtype=BF, device="cuda"))
+    cos = torch.empty(8, 32, device="cuda")
+    at = torch.empty(3, dtype=torch.int32, device="cuda")
+    lora = LoRALinear(XotLinear(512, 64, bias=False, device="cuda", dtype=BF), rank=2)
+    assert not train_ops.takes(x) and not train_ops.takes(x, w)
+    assert not train_ops.takes_heads(x, cos, cos, at, 64)
+    assert not lora._takes(x)
+
+
+@pytest.mark.gpu
+def test_training_on_another_device_than_the_current_one(monkeypatch):
+  """Launches go to the current device's stream: other tensors are torch's."""
+  from xotorch_amd.ops import torch_ref, train_ops
+  x = torch.randn(2, 16, 512, device="cuda").to(BF).requires_grad_(True)
+  w = torch.ones(512, device="cuda", dtype=BF)
+  cos, sin = torch_ref.rope_cos_sin(64, 16, 10000.0, device="cuda")
+  at = torch.arange(16, dtype=torch.int32, device="cuda")
+  assert train_ops.takes(x, w) and train_ops.takes_heads(x, cos, sin, at, 64)
+  with monkeypatch.context() as m:
+    m.setattr(torch._C, "_cuda_getDevice", lambda: 1)
+    found = train_ops.takes(x, w), train_ops.takes_heads(x, cos, sin, at, 64)
+  assert found == (False, False)
+
+
+@pytest.mark.gpu
+def test_a_training_pass_that_is_followed():
+  """A tracer records what torch's operators do; a kernel would be a constant to it."""
+  from torch.fx.experimental.proxy_tensor import make_fx
+  from xotorch_amd import ops
+  x, w = torch.randn(4, 64, device="cuda").to(BF).requires_grad_(True), torch.ones(64, device="cuda", dtype=BF)
+
+  def f(t):
+    return ops.rmsnorm(t, w, 1e-5)
+
+  graph, other = make_fx(f)(x), torch.randn(4, 64, device="cuda").to(BF).requires_grad_(True)
+  assert (graph(other).float() - f(other).float()).abs().max() < 0.05

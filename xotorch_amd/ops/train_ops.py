@@ -13,6 +13,7 @@ import torch
 from xotorch_amd.ops import torch_ref
 
 _ext = _attn = None
+_OWN = (torch.Tensor, torch.nn.Parameter)
 
 
 def _hip():
@@ -41,20 +42,28 @@ def _missing() -> bool:
   return False
 
 
-def plain_autograd() -> bool:
-  """Whether autograd alone looks on: no tracing, no functorch transform, no
-  forward-mode level, which pass such functions by."""
-  return not (torch.jit.is_tracing() or torch.jit.is_scripting() or torch.compiler.is_compiling()
-              or torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0)
+def plain(*tensors: torch.Tensor) -> bool:
+  """Whether kernels may read these here and now: tensors with memory of their own (fake
+  and wrapped ones have none, or another) on the device whose streams launches go to, and
+  nobody who follows the operators instead: tracing, a dispatch mode, a functorch
+  transform or a forward-mode level, none of which sees a kernel."""
+  if torch.compiler.is_compiling() or type(tensors[0]) not in _OWN or not tensors[0].is_cuda:
+    return False
+  here = torch._C._cuda_getDevice()
+  for t in tensors:
+    if type(t) not in _OWN or t.get_device() != here:
+      return False
+  return not (torch._C._len_torch_dispatch_stack() or torch._C._are_functorch_transforms_active()
+              or torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state())
 
 
 def takes(x: torch.Tensor, *others: torch.Tensor) -> bool:
   """Whether these operands of a differentiated operator are for the kernels: plain
-  bf16 GPU tensors, rows of whole 16 bytes up to 16384 numbers."""
+  bf16 GPU tensors, rows of whole 16 bytes up to 2^17 numbers (norms: up to 16384)."""
   if not (x.is_cuda and torch.is_grad_enabled() and x.dim() > 0 and 0 < x.shape[-1] <= 1 << 17 and x.shape[-1] % 8 == 0 and x.numel() > 0):
     return False
-  return (any(t.requires_grad for t in (x, *others)) and all(t.dtype == torch.bfloat16 and t.is_cuda for t in (x, *others))
-          and plain_autograd() and not _missing())
+  return (any(t.requires_grad for t in (x, *others)) and all(t.dtype == torch.bfloat16 for t in (x, *others))
+          and plain(x, *others) and not _missing())
 
 
 def _rows(t: torch.Tensor) -> torch.Tensor:
@@ -218,6 +227,7 @@ def causal_heads(qkv, cos, sin, positions, n_heads: int, n_kv_heads: int, hd: in
 
 def takes_heads(qkv, cos, sin, positions, hd: int) -> bool:
   B, S, _ = qkv.shape
-  return (takes(qkv) and hd % 8 == 0 and isinstance(positions, torch.Tensor) and positions.is_cuda
+  return (takes(qkv) and hd % 8 == 0 and isinstance(positions, torch.Tensor)
           and positions.dtype == torch.int32 and positions.is_contiguous() and positions.shape in ((S,), (B, S))
-          and all(t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (cos, sin)))
+          and plain(qkv, cos, sin, positions)
+          and all(t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (cos, sin)))

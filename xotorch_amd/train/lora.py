@@ -75,7 +75,7 @@ class LoRALinear(nn.Module):
     """Whether base and adapter are one function for autograd: plain bf16 GPU tensors, a
     frozen linear of which nobody else sees the result."""
     base = self.base
-    if not (x.is_cuda and x.dtype == torch.bfloat16 and torch.is_grad_enabled() and x.numel() > 0 and type(x) is torch.Tensor
+    if not (x.is_cuda and x.dtype == torch.bfloat16 and torch.is_grad_enabled() and x.numel() > 0
             and type(self.dropout) is nn.Identity and type(base.weight) is nn.Parameter and base.weight.dtype == torch.bfloat16):
       return False
     from xotorch_amd.models.llama import XotLinear
@@ -85,7 +85,7 @@ class LoRALinear(nn.Module):
     return (type(base) in (nn.Linear, XotLinear) and not any(hooks) and not torch.nn.modules.module._has_any_global_hook()
             and all(t.is_cuda and t.dtype == torch.bfloat16 and not t.requires_grad for t in held)
             and any(t.requires_grad for t in (x, self.lora_a, self.lora_b))
-            and not torch.is_autocast_enabled("cuda") and train_ops.plain_autograd())
+            and not torch.is_autocast_enabled("cuda") and train_ops.plain(x, *held, self.lora_a, self.lora_b))
 
   def forward(self, x):
     if not self.merged and self._takes(x):
