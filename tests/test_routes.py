@@ -21,6 +21,48 @@ def test_fake_tensors_are_not_read_in_training():
     assert not lora._takes(x)
 
 
+def test_fake_tensors_are_not_read_by_linears():
+  from types import SimpleNamespace
+  from xotorch_amd import ops
+  from xotorch_amd.models.llama import MLP, MoEMLP, XotLinear
+  cfg = SimpleNamespace(dim=64, n_experts=2, n_experts_per_tok=1, moe_intermediate_dim=64, intermediate_dim=64)
+  with FakeTensorMode(), torch.no_grad(), torch.device("cuda"):
+    torch.set_default_dtype(BF)
+    lin, mlp, moe = XotLinear(64, 128), MLP(cfg), MoEMLP(cfg)
+    torch.set_default_dtype(torch.float32)
+    for rows in (1, 3, 200):
+      x = torch.empty(rows, 64, dtype=BF)
+      assert not ops.few_rows(x, lin.weight) and not ops.tile_rows(x, lin.weight) 
+      assert lin(x).shape == (rows, 128)
+    assert not moe._by_tiles(torch.empty(300, 64, dtype=BF))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 5])
+def test_a_linear_that_is_followed(rows, monkeypatch):
+  from torch.fx.experimental.proxy_tensor import make_fx
+  from xotorch_amd import ops
+  from xotorch_amd.models.llama import XotLinear
+  lin = XotLinear(64, 128).cuda().to(BF)
+  x, y = (torch.randn(rows, 64, device="cuda").to(BF) for _ in "xy")
+  plain, ad = torch.nn.functional.linear, torch.autograd.forward_ad
+  with torch.no_grad():
+    ref = plain(y, lin.weight, lin.bias).float()
+    close = {"atol": 0.02, "rtol": 2.0 ** -6}
+    assert ops.tile_rows(x, lin.weight)
+    assert torch.allclose(make_fx(lin)(x)(y).float(), ref, **close)
+    assert torch.allclose(torch.jit.trace(lin, (x,))(y).float(), ref, **close)
+    assert torch.allclose(torch.func.vmap(lin)(y[:, None])[:, 0].float(), ref, **close)
+    with ad.dual_level():
+      assert ad.unpack_dual(lin(ad.make_dual(x, y))).tangent is not None
+    with torch.autocast("cuda", torch.float16):
+      assert lin(x).dtype == torch.float16
+    with monkeypatch.context() as m:
+      m.setattr(torch._C, "_cuda_getDevice", lambda: 1)
+      found = ops.few_rows(x, lin.weight), ops.tile_rows(x, lin.weight)
+    assert found == (False, False)
+
+
 @pytest.mark.gpu
 def test_training_on_another_device_than_the_current_one(monkeypatch):
   """Launches go to the current device's stream: other tensors are torch's."""

@@ -301,7 +301,7 @@ class MLP(nn.Module):
     return (type(gu) is XotLinear and type(dp) is XotLinear and not _watched(self, gu, dp)
             and gu.bias is None and dp.bias is None
             and getattr(gu, "weight_packed_fp8", None) is None and getattr(dp, "weight_packed_fp8", None) is None
-            and gu.weight.shape[0] % 8 == 0 and ops.tile_rows(x, gu.weight, dp.weight)
+            and gu.weight.shape[0] % 8 == 0 and ops.tiled(x, gu.weight, dp.weight)
             and ops.tile_wins(x.numel() // x.shape[-1], dp.weight))
 
   def gated(self, x):
@@ -434,14 +434,14 @@ class MoEMLP(nn.Module):
     of a tile of 128 tokens empty)."""
     E, k = self.n_experts, self.top_k
     if flat.dtype != torch.bfloat16 or flat.shape[0] * k <= 24 * E or E > 256 or k > 8 or flat.shape[1] % 64 \
-       or self.intermediate % 64 or not flat.is_contiguous() or flat.data_ptr() % 16 \
-       or os.getenv("XOT_FP8_PREFILL", "0") == "1" or not ops._use_hip(flat):
+       or self.intermediate % 64 or not flat.is_contiguous() or os.getenv("XOT_FP8_PREFILL", "0") == "1":
       return False
     mods = [p for e in self.experts for p in (e.gate_up_proj, e.down_proj)]
     return (type(self.gate) is nn.Linear and all(type(e) is MLP for e in self.experts) and not _watched(self.gate, *self.experts, *mods)
             and all(type(p) is XotLinear and p.bias is None for p in mods)
-            and all(p.weight.dtype == torch.bfloat16 and p.weight.is_cuda and p.weight.is_contiguous()
-                    and p.weight.data_ptr() % 16 == 0 for p in (self.gate, *mods)))
+            and ops.alone(flat, *(p.weight for p in (self.gate, *mods))) and ops._use_hip(flat) and flat.data_ptr() % 16 == 0
+            and all(p.weight.dtype == torch.bfloat16 and p.weight.is_contiguous() and p.weight.data_ptr() % 16 == 0
+                    for p in (self.gate, *mods)))
 
   def _forward_prefill_tiles(self, flat):
     """Rows of all (token, expert) pairs are placed by counting, without the host; the
@@ -573,7 +573,7 @@ class DecoderLayer(nn.Module):
       return False
     rows = x.shape[0] * x.shape[1]
     return (x.shape[-1] % 8 == 0 and x.shape[-1] <= 16384 and not _watched(self, a, *mods, self.post_attention_layernorm)
-            and ops.tile_rows(x, *(p.weight for p in mods))
+            and ops.tiled(x, *(p.weight for p in mods))
             and all(ops.tile_wins(rows, p.weight) for p in mods)
             and ops.plain_norms(self.input_layernorm.weight, self.post_attention_layernorm.weight))
 
@@ -751,7 +751,7 @@ class ShardedModel(nn.Module):
                 and os.getenv("XOT_ACT_CKPT", "0") == "1")
     layers = [self.layers[str(lid)] for lid in self.local_layer_ids]
     # few enough rows for weight tiles, but not so few that the layers fuse more (ops.few_rows)
-    tiles = (caches is not None and h.is_cuda and h.shape[0] * h.shape[1] <= ops.TILE_ROWS
+    tiles = (caches is not None and h.is_cuda and h.shape[0] * h.shape[1] <= ops.TILE_ROWS and ops.alone(h)
              and not (h.shape[0] * h.shape[1] <= ops.FEW_ROWS and layers[0]._few_rows(h)))
     normed = None
     for idx, layer in enumerate(layers):

@@ -256,14 +256,19 @@ def _rows():
   return _rows_ext
 
 
+def alone(*tensors: torch.Tensor) -> bool:
+  """Whether a linear of these may be a kernel instead of torch's operator."""
+  return train_ops.plain(*tensors) and not torch._C._is_any_autocast_enabled()
+
+
 def few_rows(x: torch.Tensor, *weights: torch.Tensor) -> bool:
   """Whether the products of x with these weights ([N, K], bf16) are a few rows'
   (hip/rows_ops.hip): inference on the GPU, up to FEW_ROWS rows, 16-byte rows."""
   if not x.is_cuda or x.dtype != torch.bfloat16 or torch.is_grad_enabled() or not x.is_contiguous():
     return False
-  if not 0 < x.numel() <= FEW_ROWS * x.shape[-1] or x.data_ptr() % 16 or not _use_hip(x):
+  if not 0 < x.numel() <= FEW_ROWS * x.shape[-1] or not alone(x, *weights) or x.data_ptr() % 16 or not _use_hip(x):
     return False
-  return all(w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[1] % 8 == 0 and w.is_contiguous()
+  return all(w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[1] % 8 == 0 and w.is_contiguous()
              and w.data_ptr() % 16 == 0 and 0 < w.shape[0] <= 1 << 26 for w in weights)
 
 
@@ -315,12 +320,22 @@ def _tile():
 def tile_rows(x: torch.Tensor, *weights: torch.Tensor) -> bool:
   """Whether the products of x with these weights ([N, K], bf16) go by weight tiles
   (hip/tile_ops.hip): inference on the GPU, up to TILE_ROWS rows, k in steps of 64."""
-  if not x.is_cuda or x.dtype != torch.bfloat16 or torch.is_grad_enabled() or not x.is_contiguous():
+  return x.is_cuda and alone(x) and tiled(x, *weights)
+
+
+def tiled(x: torch.Tensor, *weights: torch.Tensor) -> bool:
+  """The same where the caller has asked whether x is alone."""
+  if not x.is_cuda or x.dtype is not torch.bfloat16 or torch.is_grad_enabled() or not x.is_contiguous():
     return False
   if not 0 < x.numel() <= TILE_ROWS * x.shape[-1] or x.data_ptr() % 16 or not _use_hip(x):
     return False
-  return all(w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[1] % 64 == 0 and w.is_contiguous()
-             and w.data_ptr() % 16 == 0 and 0 < w.shape[0] <= 1 << 26 and 0 < w.shape[1] <= 1 << 26 for w in weights)
+  at = x.get_device()
+  for w in weights:
+    size = w.shape
+    if w.dtype is not torch.bfloat16 or len(size) != 2 or size[1] % 64 or not (0 < size[0] <= 1 << 26 and 0 < size[1] <= 1 << 26) \
+       or type(w) not in train_ops.OWN or w.get_device() != at or not w.is_contiguous() or w.data_ptr() % 16:
+      return False
+  return True
 
 
 def tile_wins(rows: int, weight: torch.Tensor) -> bool:

@@ -13,7 +13,14 @@ import torch
 from xotorch_amd.ops import torch_ref
 
 _ext = _attn = None
-_OWN = (torch.Tensor, torch.nn.Parameter)
+OWN = (torch.Tensor, torch.nn.Parameter)
+# looked up once: a step of a small model asks some thirty times
+_is_compiling, _is_tracing, _forward_ad = torch.compiler.is_compiling, torch._C._is_tracing, torch.autograd.forward_ad
+_dispatch_modes, _transforms = torch._C._len_torch_dispatch_stack, torch._C._are_functorch_transforms_active
+
+
+def _current_device() -> int:
+  return torch._C._cuda_getDevice()
 
 
 def _hip():
@@ -47,14 +54,16 @@ def plain(*tensors: torch.Tensor) -> bool:
   and wrapped ones have none, or another) on the device whose streams launches go to, and
   nobody who follows the operators instead: tracing, a dispatch mode, a functorch
   transform or a forward-mode level, none of which sees a kernel."""
-  if torch.compiler.is_compiling() or type(tensors[0]) not in _OWN or not tensors[0].is_cuda:
+  if not tensors[0].is_cuda or _is_compiling():
     return False
-  here = torch._C._cuda_getDevice()
   for t in tensors:
-    if type(t) not in _OWN or t.get_device() != here:
+    if type(t) not in OWN:
       return False
-  return not (torch._C._len_torch_dispatch_stack() or torch._C._are_functorch_transforms_active()
-              or torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state())
+  here = _current_device()
+  for t in tensors:
+    if t.get_device() != here:
+      return False
+  return not (_dispatch_modes() or _transforms() or _forward_ad._current_level >= 0 or _is_tracing())
 
 
 def takes(x: torch.Tensor, *others: torch.Tensor) -> bool:
