@@ -90,3 +90,16 @@ def test_a_training_pass_that_is_followed():
 
   graph, other = make_fx(f)(x), torch.randn(4, 64, device="cuda").to(BF).requires_grad_(True)
   assert (graph(other).float() - f(other).float()).abs().max() < 0.05
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(1,), (3, 1, 64), (2, 3, 64), ()])
+def test_norms_with_weights_of_another_shape(shape):
+  """What torch broadcasts: a kernel would read D numbers from the first on."""
+  from xotorch_amd import ops
+  from xotorch_amd.ops import torch_ref
+  x, r = (torch.randn(2, 3, 1, 64, device="cuda").to(BF).requires_grad_(True) for _ in "xr")
+  w = torch.randn(shape, device="cuda").to(BF)
+  assert torch.equal(ops.rmsnorm(x, w, 1e-5), torch_ref.rmsnorm(x, w, 1e-5))
+  for a, b in zip(ops.rmsnorm_residual(x, r, w, 1e-5), torch_ref.rmsnorm_residual(x, r, w, 1e-5)):
+    assert torch.equal(a, b)

@@ -61,7 +61,7 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, w_bias: float = 0
   """w_bias=1.0 gives the gemma convention (scale by 1 + w, fp32 math)."""
   if _use_hip(x, weight) and x.dtype == torch.bfloat16:
     return _hip.rmsnorm(x, weight, eps, w_bias)
-  if train_ops.takes(x, weight) and x.shape[-1] <= 16384:
+  if train_ops.takes(x, weight) and x.shape[-1] <= 16384 and weight.shape == x.shape[-1:]:
     return train_ops.rmsnorm(x, weight, eps, w_bias)
   return torch_ref.rmsnorm(x, weight, eps, w_bias)
 
@@ -72,7 +72,7 @@ def rmsnorm_residual(
 ) -> Tuple[torch.Tensor, torch.Tensor]:
   if _use_hip(x, residual, weight) and x.dtype == torch.bfloat16:
     return _hip.rmsnorm_residual(x, residual, weight, eps, w_bias)
-  if train_ops.takes(x, residual, weight) and x.shape[-1] <= 16384 and x.shape == residual.shape:
+  if train_ops.takes(x, residual, weight) and x.shape[-1] <= 16384 and x.shape == residual.shape and weight.shape == x.shape[-1:]:
     return train_ops.rmsnorm_residual(x, residual, weight, eps, w_bias)
   return torch_ref.rmsnorm_residual(x, residual, weight, eps, w_bias)
 
