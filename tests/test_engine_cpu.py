@@ -70,6 +70,24 @@ def test_engine_train_last_shard():
   assert run(go())
 
 
+def test_engine_train_past_the_context():
+  """Sequences longer than the rotation's tables are refused before a pass starts."""
+  from xotorch_amd.engine.torch_engine import ContextExhausted
+
+  async def go():
+    eng = TorchEngine(device="cpu", dtype=torch.float32)
+    shard = build_full_shard("dummy", "TorchEngine")
+    await eng.ensure_shard(shard)
+    S = eng.model.rope_cos.shape[0] + 1
+    x = np.zeros((1, S), dtype=np.int64)
+    with pytest.raises(ContextExhausted):
+      await eng.train("t", shard, x, x, np.array([S]))
+    with pytest.raises(ContextExhausted):
+      await eng.evaluate("t", shard, x, x, np.array([S]))
+    return True
+  assert run(go())
+
+
 def test_engine_ring_train_back_gradient():
   """Pipeline training: last shard CE + gradient hop back to the first shard."""
   async def go():

@@ -132,6 +132,32 @@ def test_causal_heads(B, S, H, KVH, hd, per_row, spread):
     assert bool(((qkv.grad.double() - ref).abs() <= ref.abs() * STEP + size * (STEP + 2.0 ** -18) + slack).all())
 
 
+@pytest.mark.parametrize("hd", [24, 64, 128])
+def test_positions_as_torch_indexes(hd):
+  """Negative ones count from the tables' end; past it there is nothing to train with."""
+  from xotorch_amd.ops import torch_ref, train_ops
+  B, S, H, KVH, T = 2, 40, 4, 2, 64
+  cos, sin = torch_ref.rope_cos_sin(hd, T, 10000.0, device="cuda")
+  at = torch.arange(T - S, T, dtype=torch.int32, device="cuda").expand(B, S).contiguous()
+  d, found = _rand(B, S, H * hd, seed=1), []
+  for pos in (at, at - T):
+    qkv = _rand(B, S, (H + 2 * KVH) * hd).requires_grad_(True)
+    assert train_ops.takes_heads(qkv, cos, sin, pos, hd)
+    out = train_ops.causal_heads(qkv, cos, sin, pos, H, KVH, hd)
+    out.backward(d)
+    found.append((out, qkv.grad))
+  assert all(torch.equal(a, b) for a, b in zip(*found))
+  for bad in (T, -T - 1, 2 ** 31 - 1, -2 ** 31):
+    pos = at.clone()
+    pos[1, 33] = bad
+    out = train_ops.causal_heads(_rand(B, S, (H + 2 * KVH) * hd).requires_grad_(True), cos, sin, pos, H, KVH, hd)
+    assert torch.equal(out[0], found[0][0][0]) and bool(out[1, 33:].isnan().all())
+    if hd != 24:  # (torch's attention spreads it to earlier tokens as well)
+      assert torch.equal(out[1, :33], found[0][0][1, :33])
+  short = torch.arange(T + 1, dtype=torch.int32, device="cuda")
+  assert not train_ops.takes_heads(_rand(1, T + 1, (H + 2 * KVH) * hd).requires_grad_(True), cos, sin, short, hd)
+
+
 @pytest.mark.parametrize("rows,K,N,rank,bias", [(1, 8, 24, 1, False), (5, 64, 40, 3, True), (130, 256, 520, 16, False)])
 def test_adapted_linear(rows, K, N, rank, bias):
   from xotorch_amd.models.llama import XotLinear

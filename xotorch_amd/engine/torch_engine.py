@@ -255,6 +255,9 @@ class TorchEngine(InferenceEngine):
     (XOT_ACT_CKPT=1): measured 380 vs 283 ms/step on 8B LoRA B=8 — worth it
     only when activations would not fit."""
     S = x.shape[1]
+    angles = getattr(self.model, "rope_cos", None)
+    if angles is not None and S > angles.shape[0]:
+      raise ContextExhausted(f"training on sequences of {S} tokens exceeds max_seq_len {angles.shape[0]}")
     positions = torch.arange(0, S, dtype=torch.int32, device=self.device)
     return self.model(x, caches=None, positions=positions, start_pos=0, last_only=False)
 

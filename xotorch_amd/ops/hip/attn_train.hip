@@ -34,9 +34,9 @@ struct TrainArgs {
   float scale;
 };
 
-// where a token stands, within the tables
+// where a token stands in the tables
 DEVINL int place(const TrainArgs& a, int b, int s) {
-  return min(max(a.positions[a.per_row ? b * a.S + s : s], 0), a.places - 1);
+  return table_row(a.positions[a.per_row ? b * a.S + s : s], a.places);
 }
 
 // The 32 rows of one head from tile s0 on, in LDS, to both orders
@@ -73,8 +73,8 @@ __global__ __launch_bounds__(256) void pack_qkv_kernel(TrainArgs a) {
       if (slot < a.H + a.KVH) {
         float co[4], si[4];
         const int pos = place(a, b, s);
-        ld4(a.cos + (size_t)pos * (HD / 2) + c, co);
-        ld4(a.sin + (size_t)pos * (HD / 2) + c, si);
+        ld_angles(a.cos, pos, HD / 2, c, co);
+        ld_angles(a.sin, pos, HD / 2, c, si);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const float y1 = x1[j] * co[j] - x2[j] * si[j], y2 = x2[j] * co[j] + x1[j] * si[j];
@@ -265,7 +265,7 @@ __global__ __launch_bounds__(256, 2) void train_forward_kernel(TrainArgs a) {
 template <int HD>
 DEVINL void turn_back(const TrainArgs& a, floatx4* o, int b, int s, int quad, bf16_t* dst, bool turn) {
   constexpr int VG = HD / 16;
-  const size_t at = turn ? (size_t)place(a, b, s) * (HD / 2) + quad * 4 : 0;
+  const int pos = turn ? place(a, b, s) : 0;
 #pragma unroll
   for (int g = 0; g < VG / 2; ++g) {
     float y1[4], y2[4];
@@ -276,8 +276,8 @@ DEVINL void turn_back(const TrainArgs& a, floatx4* o, int b, int s, int quad, bf
     }
     if (turn) {
       float co[4], si[4];
-      ld4(a.cos + at + g * 16, co);
-      ld4(a.sin + at + g * 16, si);
+      ld_angles(a.cos, pos, HD / 2, g * 16 + quad * 4, co);
+      ld_angles(a.sin, pos, HD / 2, g * 16 + quad * 4, si);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const bf16_t r1 = f2b(y1[i]), r2 = f2b(y2[i]);

@@ -56,6 +56,19 @@ DEVINL floatx4 sum_parts(const float* p, size_t at, size_t stride, int splits) {
   for (; s < splits; ++s) v += *(const floatx4*)(p + s * stride + at);
   return v;
 }
+// Row of a rotation's tables for a position: negative ones count from the end, as an
+// index of torch's does; -1: the tables have none
+DEVINL int table_row(int pos, int rows) {
+  if (pos < 0) pos += rows;
+  return pos < 0 || pos >= rows ? -1 : pos;
+}
+// Four of its cosines or sines; not a number where there is no row, so that it is seen
+DEVINL void ld_angles(const float* table, int row, int half, int c, float* o) {
+  ld4(table + (size_t)max(row, 0) * half + c, o);
+  if (row < 0)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = __builtin_nanf("");
+}
 typedef __attribute__((ext_vector_type(2))) float floatx2;
 typedef __attribute__((ext_vector_type(2))) unsigned short ushort2_t;
 DEVINL void ld2(const float* p, float* o) {

@@ -175,9 +175,9 @@ __global__ __launch_bounds__(256) void split_heads_kernel(const bf16_t* __restri
   ld4(src + half, x2);
   if (slot < a.H + a.KVH) {
     float co[4], si[4];
-    const int pos = min(max(a.positions[a.per_row ? tok : s], 0), a.places - 1);
-    ld4(a.cos + (size_t)pos * half + c, co);
-    ld4(a.sin + (size_t)pos * half + c, si);
+    const int pos = table_row(a.positions[a.per_row ? tok : s], a.places);
+    ld_angles(a.cos, pos, half, c, co);
+    ld_angles(a.sin, pos, half, c, si);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const float y1 = x1[j] * co[j] - x2[j] * si[j], y2 = x2[j] * co[j] + x1[j] * si[j];
@@ -220,9 +220,9 @@ __global__ __launch_bounds__(256) void split_heads_backward_kernel(const float* 
   }
   if (slot < a.H + a.KVH) {
     float co[4], si[4];
-    const int pos = min(max(a.positions[a.per_row ? tok : s], 0), a.places - 1);
-    ld4(a.cos + (size_t)pos * half + c, co);
-    ld4(a.sin + (size_t)pos * half + c, si);
+    const int pos = table_row(a.positions[a.per_row ? tok : s], a.places);
+    ld_angles(a.cos, pos, half, c, co);
+    ld_angles(a.sin, pos, half, c, si);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const float y1 = rounded(g1[j]), y2 = rounded(g2[j]);

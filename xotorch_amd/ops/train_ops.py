@@ -235,8 +235,10 @@ def causal_heads(qkv, cos, sin, positions, n_heads: int, n_kv_heads: int, hd: in
 
 
 def takes_heads(qkv, cos, sin, positions, hd: int) -> bool:
+  """Whether these kernels rotate the heads: tables of a row per token at least, by which
+  a sequence longer than them stays torch's to refuse."""
   B, S, _ = qkv.shape
-  return (takes(qkv) and hd % 8 == 0 and isinstance(positions, torch.Tensor)
+  return (takes(qkv) and hd % 8 == 0 and S <= cos.shape[0] and isinstance(positions, torch.Tensor)
           and positions.dtype == torch.int32 and positions.is_contiguous() and positions.shape in ((S,), (B, S))
           and plain(qkv, cos, sin, positions)
           and all(t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (cos, sin)))
