@@ -90,3 +90,16 @@ def test_other_rows_go_the_general_way():
     assert not ops.few_rows(x.float(), w) and not ops.few_rows(x.t(), w) and not ops.few_rows(x[:, :12].contiguous(), w[:, :12])
     assert not ops.few_rows(torch.ones(33, device="cuda", dtype=torch.bfloat16)[1:].view(2, 16), w)
     assert not ops.few_rows(x[:0], w) and not ops.few_rows(x, w[:, 1:9])
+
+
+def test_one_row_summed_as_more_are():
+  from xotorch_amd import ops
+  from xotorch_amd.models.llama import XotLinear
+  lin = XotLinear(4096, 512, bias=False).cuda().to(torch.bfloat16)
+  x = torch.randn(5, 4096, generator=torch.Generator(device="cuda").manual_seed(0), device="cuda").to(torch.bfloat16)
+  with torch.inference_mode():
+    assert ops.few_rows(x[:1], lin.weight)
+    with ops.sums_of_more_rows():
+      assert not ops.few_rows(x[:1], lin.weight)
+      assert torch.equal(lin(x)[:1], lin(x[:1]))
+    assert ops.few_rows(x[:1], lin.weight)

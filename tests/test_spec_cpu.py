@@ -61,3 +61,25 @@ def test_eos_stops_generation():
   sd.reset()
   toks, _ = sd.generate(prompt, max_new=40, eos_id=eos)
   assert toks == full[: full.index(eos) + 1]
+
+
+def test_the_models_stay_as_they_were():
+  """How a step of speculation sums is no state of models that others serve as well."""
+  import threading
+  from xotorch_amd import ops
+  (t, tc), (d, dc) = _build(7), _build(8)
+  before = [{k: v for k, v in vars(m).items() if not k.startswith("_")} for model in (t, d) for m in model.modules()]
+  seen = []
+
+  def look(*_):
+    here, there = ops._sums.of_more_rows, []
+    other = threading.Thread(target=lambda: there.append(ops._sums.of_more_rows))
+    other.start()
+    other.join()
+    seen.append((here, there[0]))
+
+  hook = t.register_forward_hook(look)
+  SpeculativeDecoder(t, d, tc, dc, device="cpu", dtype=torch.float32, gamma=2, max_seq=64).generate(torch.zeros(1, 4, dtype=torch.int64), 6)
+  hook.remove()
+  assert set(seen) == {(True, False)} and not ops._sums.of_more_rows
+  assert before == [{k: v for k, v in vars(m).items() if not k.startswith("_")} for model in (t, d) for m in model.modules()]

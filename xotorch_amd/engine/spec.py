@@ -26,6 +26,7 @@ from typing import List, Optional, Tuple
 
 import torch
 
+from xotorch_amd import ops
 from xotorch_amd.engine.kvcache import ShardKVCache
 from xotorch_amd.models import model_class_for
 from xotorch_amd.models.config import ModelConfig, config_from_hf
@@ -61,12 +62,6 @@ class SpeculativeDecoder:
         raise ValueError(f"{cfg.model_id}: speculative decoding rewinds positions, which a recurrent state cannot")
     th, tk, tv = target_cfg.kv_cache_dims()
     dh, dk, dv = draft_cfg.kv_cache_dims()
-    for model in (target, draft):
-      # proposals are made one row at a time and verified several at a time: sums in
-      # the same order for either keep equal logits equal
-      for m in model.modules():
-        if hasattr(m, "few_rows"):
-          m.few_rows = False
     self.t_cache = ShardKVCache(target_cfg.n_layers, 1, th, self.max_seq, tk, dtype, device, v_dim=tv)
     self.d_cache = ShardKVCache(draft_cfg.n_layers, 1, dh, self.max_seq, dk, dtype, device, v_dim=dv)
 
@@ -102,11 +97,16 @@ class SpeculativeDecoder:
 
   def _forward(self, model, cache, tokens: torch.Tensor, pos0: int) -> torch.Tensor:
     """Run `tokens` [1, S] at positions pos0..pos0+S-1; returns logits
-    [1, S, V] (all positions)."""
+    [1, S, V] (all positions).
+
+    Proposals are made one row at a time and verified several at a time: products
+    that sum alike for either keep logits close to equal. (Attention may still cut
+    the keys of a long cache elsewhere for the two.)"""
     S = tokens.shape[1]
     pos = torch.arange(pos0, pos0 + S, dtype=torch.int32, device=self.device)
-    out = model(tokens, caches=cache.caches, positions=pos, start_pos=pos0,
-                last_only=False)
+    with ops.sums_of_more_rows():
+      out = model(tokens, caches=cache.caches, positions=pos, start_pos=pos0,
+                  last_only=False)
     if out.dim() == 2:
       out = out.unsqueeze(1)
     return out

@@ -68,7 +68,6 @@ class XotLinear(nn.Linear):
 
   hip = ("_hip_rows", "_hip_tile")  # what a pass loads beside the operators
   weight_packed: Optional[torch.Tensor]
-  few_rows = True  # up to ops.FEW_ROWS rows have kernels of their own, whose sums are in another order
 
   def __init__(self, *a, **kw):
     super().__init__(*a, **kw)
@@ -143,7 +142,7 @@ class XotLinear(nn.Linear):
           y = hip.skinny_gemm_fp8(x8, sx, wp8, self.weight_scale, 1, N, self.bias)
           sizes = list(x.shape[:-1]) + [N]
           return y.view(sizes)
-    if x.numel() <= ops.FEW_ROWS * self.in_features and self.few_rows and ops.few_rows(x, self.weight) and (self.bias is None or self.bias.dtype == torch.bfloat16):
+    if x.numel() <= ops.FEW_ROWS * self.in_features and ops.few_rows(x, self.weight) and (self.bias is None or self.bias.dtype == torch.bfloat16):
       return ops.rows_linear(x, self.weight, self.bias)
     if x.numel() <= ops.TILE_ROWS * self.in_features and ops.tile_rows(x, self.weight) and (
         ops.tile_wins(x.numel() // self.in_features, self.weight) and (self.bias is None or self.bias.dtype == torch.bfloat16)):
@@ -561,7 +560,7 @@ class DecoderLayer(nn.Module):
     a, m = self.self_attn, self.mlp
     mods = (a.qkv_proj, a.o_proj, m.gate_up_proj, m.down_proj) if type(m) is MLP else ()
     norms = (self.input_layernorm.weight, self.post_attention_layernorm.weight)
-    return (len(mods) > 0 and all(type(p) is XotLinear and p.few_rows for p in mods)
+    return (len(mods) > 0 and all(type(p) is XotLinear for p in mods)
             and not _watched(a, m, self.input_layernorm, self.post_attention_layernorm, *mods)
             and ops.few_rows_normed(x, norms, *(p.weight for p in mods)))
 
@@ -617,8 +616,6 @@ class DecoderLayer(nn.Module):
 
 class ShardedModel(nn.Module):
   """The layer range [shard.start_layer .. shard.end_layer] of one model."""
-
-  few_rows = True  # XotLinear.few_rows, for a head that is the embedding
 
   def __init__(self, cfg: ModelConfig, shard: Shard):
     super().__init__()
@@ -776,7 +773,7 @@ class ShardedModel(nn.Module):
       normed = None
     head = self.head_weight()
     own = self.lm_head if hasattr(self, "lm_head") else None
-    if normed is None and (type(own) is XotLinear and own.few_rows if own is not None else self.few_rows) and not (
+    if normed is None and (own is None or type(own) is XotLinear) and not (
         _watched(self.norm, *(() if own is None else (own,)))) and (
         ops.few_rows_normed(h, (self.norm.weight,), head)):
       logits = ops.rows_norm_linear(h, self.norm.weight, self.norm.eps, head)

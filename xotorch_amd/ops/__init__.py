@@ -9,7 +9,9 @@ debugging/ablation only).
 """
 from __future__ import annotations
 
+import contextlib
 import os
+import threading
 from typing import Optional, Tuple
 
 import torch
@@ -261,10 +263,29 @@ def alone(*tensors: torch.Tensor) -> bool:
   return train_ops.plain(*tensors) and not torch._C._is_any_autocast_enabled()
 
 
+class _Sums(threading.local):
+  of_more_rows = False
+
+
+_sums = _Sums()
+
+
+@contextlib.contextmanager
+def sums_of_more_rows():
+  """Within this, in this thread, products of one or two rows are summed as those of up to
+  16 are (hip/tile_ops.hip, where a row's sums do not depend on the rows beside it), and
+  not by the kernels of their own, whose order is another."""
+  before, _sums.of_more_rows = _sums.of_more_rows, True
+  try:
+    yield
+  finally:
+    _sums.of_more_rows = before
+
+
 def few_rows(x: torch.Tensor, *weights: torch.Tensor) -> bool:
   """Whether the products of x with these weights ([N, K], bf16) are a few rows'
   (hip/rows_ops.hip): inference on the GPU, up to FEW_ROWS rows, 16-byte rows."""
-  if not x.is_cuda or x.dtype != torch.bfloat16 or torch.is_grad_enabled() or not x.is_contiguous():
+  if not x.is_cuda or x.dtype != torch.bfloat16 or torch.is_grad_enabled() or not x.is_contiguous() or _sums.of_more_rows:
     return False
   if not 0 < x.numel() <= FEW_ROWS * x.shape[-1] or not alone(x, *weights) or x.data_ptr() % 16 or not _use_hip(x):
     return False
