@@ -61,3 +61,16 @@ def test_mfma_attention_cache_consistency():
   toks_mfma = _run(use_graphs=True, pack_mode="none")
   agree = (toks_valu == toks_mfma).float().mean().item()
   assert agree > 0.95, f"token agreement {agree}"
+
+
+def test_the_library_is_loaded_before_the_first_prompt(monkeypatch):
+  """Decode steps don't touch the GEMM library: its load belongs to the warm-up."""
+  from xotorch_amd import ops
+  from xotorch_amd.parallel.ring import RingPipeline
+  ring = RingPipeline(model_id="tiny128", rank=0, world=1, device="cuda", dtype=torch.bfloat16, mb_batch=4,
+                      prompt_len=96, max_gen=12, seed=77, cfg_override=TINY128)
+  calls, prompt, load = [], ring._prefill_forward, ops.load_library
+  monkeypatch.setattr(ops, "load_library", lambda *a: (calls.append("load"), load(*a)))
+  monkeypatch.setattr(ring, "_prefill_forward", lambda *a: (calls.append("prompt"), prompt(*a))[1])
+  ring.prefill()
+  assert calls == ["load", "prompt"]

@@ -391,6 +391,13 @@ def parts_add_norm(parts, x, norm=None, eps: float = 0.0, w_bias: float = 0.0, r
   return _tile().parts_add_norm(parts, x, norm, eps, w_bias, rounded)
 
 
+def load_library(device, dtype: torch.dtype):
+  """Has the GEMM library load its kernels of this type, which takes some 0.35 s once.
+  Decode steps don't use it: without this the first prompt would wait."""
+  a = torch.zeros(512, 512, device=device, dtype=dtype)
+  torch.nn.functional.linear(a, a)
+
+
 def softmax_sample(logits, temperature: float = 0.0, top_k: int = 0, generator=None,
                    top_p: float = 0.0):
   # torch ops here are graph-capturable (argmax / exponential+argmax)

@@ -24,6 +24,7 @@ from typing import List, Optional
 import torch
 import torch.distributed as dist
 
+from xotorch_amd import ops
 from xotorch_amd.engine.kvcache import make_cache
 from xotorch_amd.models import model_class_for
 from xotorch_amd.models.config import ModelConfig, config_from_hf
@@ -191,6 +192,7 @@ class RingPipeline:
     s.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(s):
       with torch.inference_mode():
+        ops.load_library(self.device, self.dtype)
         for mb in range(self.M):
           for _ in range(2):
             self._step_mb(mb)

@@ -46,6 +46,7 @@ if __package__ in (None, ""):  # torchrun launches this file by path
 import torch
 import torch.distributed as dist
 
+from xotorch_amd import ops
 from xotorch_amd.engine.kvcache import make_cache
 from xotorch_amd.models.config import config_from_hf
 from xotorch_amd.models.registry import builtin_config, get_repo, register_local_model
@@ -180,6 +181,7 @@ class RingSlotWorker:
     s.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(s):
       with torch.inference_mode():
+        ops.load_library(self.device, self.dtype)
         for _ in range(2):
           self._decode_forward()
     torch.cuda.current_stream().wait_stream(s)
