@@ -32,9 +32,34 @@ def test_fake_tensors_are_not_read_by_linears():
     torch.set_default_dtype(torch.float32)
     for rows in (1, 3, 200):
       x = torch.empty(rows, 64, dtype=BF)
-      assert not ops.few_rows(x, lin.weight) and not ops.tile_rows(x, lin.weight) 
+      assert not ops.few_rows(x, lin.weight) and not ops.tile_rows(x, lin.weight)
       assert lin(x).shape == (rows, 128)
     assert not moe._by_tiles(torch.empty(300, 64, dtype=BF))
+
+
+def test_products_go_where_they_are_faster():
+  """Weights too wide for one round of blocks are the library's for many rows."""
+  from xotorch_amd import ops
+  for N, K in ((12288, 12288), (14336, 12288), (18432, 16384), (16384, 53248)):
+    assert ops.parts_win(16, N, K) and ops.parts_win(17, N, K) == ops.parts_win(64, N, K) == (K != 16384)
+    assert not ops.parts_win(65, N, K) and not ops.parts_win(256, N, K)
+    assert not any(ops.tile_wins(m, N, K) for m in (17, 64, 65, 256))
+  for N, K in ((4608, 3584), (8192, 28672), (10240, 8192), (3072, 2048)):
+    assert all(ops.parts_win(m, N, K) for m in (1, 16, 17, 128, 129, 256))
+  assert ops.tile_wins(128, 4096, 4096) and not ops.tile_wins(128, 2048, 2048) and ops.tile_wins(64, 2048, 2048)
+  assert ops.tile_wins(256, 4096, 14336) and not ops.tile_wins(129, 3072, 2048)
+  assert ops.tile_wins(64, 28672, 4096) and not ops.tile_wins(65, 28672, 4096) and not ops.tile_wins(17, 17920, 1536)
+  assert not ops.tile_wins(4, 8192, 8192) and ops.tile_wins(128, 8192, 8192)
+  assert ops.gate_wins(128, 57344, 8192) and not ops.gate_wins(129, 57344, 8192)
+  assert ops.gate_wins(16, 17920, 1536) and not ops.gate_wins(17, 17920, 1536) and ops.gate_wins(128, 16384, 2048)
+
+
+@pytest.mark.gpu
+def test_the_rules_know_how_k_is_split():
+  from xotorch_amd import ops
+  for N in (1, 64, 65, 896, 1536, 4608, 8192, 9536, 9537, 14336, 14337, 28672, 28673, 151936, 1 << 26):
+    for K in (64, 192, 256, 960, 1024, 2048, 3584, 4032, 4096, 16384, 53248):
+      assert ops.tile_splits(N, K) == ops._tile().tile_splits(N, K)
 
 
 @pytest.mark.gpu

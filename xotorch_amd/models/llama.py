@@ -145,7 +145,7 @@ class XotLinear(nn.Linear):
     if x.numel() <= ops.FEW_ROWS * self.in_features and ops.few_rows(x, self.weight) and (self.bias is None or self.bias.dtype == torch.bfloat16):
       return ops.rows_linear(x, self.weight, self.bias)
     if x.numel() <= ops.TILE_ROWS * self.in_features and ops.tile_rows(x, self.weight) and (
-        ops.tile_wins(x.numel() // self.in_features, self.weight) and (self.bias is None or self.bias.dtype == torch.bfloat16)):
+        ops.tile_wins(x.numel() // self.in_features, *self.weight.shape) and (self.bias is None or self.bias.dtype == torch.bfloat16)):
       return ops.tile_linear(x, self.weight, self.bias)
     if self.weight_packed is not None and x.is_cuda and x.dtype == torch.bfloat16:
       N, K = self.weight.shape
@@ -301,12 +301,12 @@ class MLP(nn.Module):
             and gu.bias is None and dp.bias is None
             and getattr(gu, "weight_packed_fp8", None) is None and getattr(dp, "weight_packed_fp8", None) is None
             and gu.weight.shape[0] % 8 == 0 and ops.tiled(x, gu.weight, dp.weight)
-            and ops.tile_wins(x.numel() // x.shape[-1], dp.weight))
+            and ops.parts_win(x.numel() // x.shape[-1], *dp.weight.shape))
 
   def gated(self, x):
     """The gated activation of x (by_tiles)."""
     gu = self.gate_up_proj
-    if ops.tile_wins(x.numel() // x.shape[-1], gu.weight):
+    if ops.gate_wins(x.numel() // x.shape[-1], *gu.weight.shape):
       return ops.tile_swiglu(x, gu.weight)
     return self.act(gu(x))
 
@@ -570,10 +570,8 @@ class DecoderLayer(nn.Module):
     mods = (a.qkv_proj, a.o_proj)
     if not all(type(p) is XotLinear and getattr(p, "weight_packed_fp8", None) is None for p in mods):
       return False
-    rows = x.shape[0] * x.shape[1]
     return (x.shape[-1] % 8 == 0 and x.shape[-1] <= 16384 and not _watched(self, a, *mods, self.post_attention_layernorm)
-            and ops.tiled(x, *(p.weight for p in mods))
-            and all(ops.tile_wins(rows, p.weight) for p in mods)
+            and ops.tiled(x, *(p.weight for p in mods), wins=ops.parts_win)
             and ops.plain_norms(self.input_layernorm.weight, self.post_attention_layernorm.weight))
 
   def step(self, x, normed, cos, sin, positions, kv, start_pos, is_decode, seq_lens, after):
@@ -781,7 +779,7 @@ class ShardedModel(nn.Module):
     h = self.norm(h) if normed is None else normed
     if own is not None:
       logits = own(h)  # XotLinear: packed decode kernel when prepacked
-    elif h.numel() <= ops.TILE_ROWS * h.shape[-1] and ops.tile_rows(h, head) and ops.tile_wins(h.numel() // h.shape[-1], head):
+    elif h.numel() <= ops.TILE_ROWS * h.shape[-1] and ops.tile_rows(h, head) and ops.tile_wins(h.numel() // h.shape[-1], *head.shape):
       logits = ops.tile_linear(h, head)
     else:
       logits = ops.linear(h, head.to(h.dtype))

@@ -10,6 +10,7 @@ debugging/ablation only).
 from __future__ import annotations
 
 import contextlib
+import functools
 import os
 import threading
 from typing import Optional, Tuple
@@ -344,31 +345,87 @@ def tile_rows(x: torch.Tensor, *weights: torch.Tensor) -> bool:
   return x.is_cuda and alone(x) and tiled(x, *weights)
 
 
-def tiled(x: torch.Tensor, *weights: torch.Tensor) -> bool:
-  """The same where the caller has asked whether x is alone."""
+def tiled(x: torch.Tensor, *weights: torch.Tensor, wins=None) -> bool:
+  """The same where the caller has asked whether x is alone; with `wins` (one of the rules
+  below) also whether that is the faster way for each of them."""
   if not x.is_cuda or x.dtype is not torch.bfloat16 or torch.is_grad_enabled() or not x.is_contiguous():
     return False
   if not 0 < x.numel() <= TILE_ROWS * x.shape[-1] or x.data_ptr() % 16 or not _use_hip(x):
     return False
-  at = x.get_device()
+  at, rows = x.get_device(), x.numel() // x.shape[-1]
   for w in weights:
     size = w.shape
     if w.dtype is not torch.bfloat16 or len(size) != 2 or size[1] % 64 or not (0 < size[0] <= 1 << 26 and 0 < size[1] <= 1 << 26) \
-       or type(w) not in train_ops.OWN or w.get_device() != at or not w.is_contiguous() or w.data_ptr() % 16:
+       or type(w) not in train_ops.OWN or w.get_device() != at or not w.is_contiguous() or w.data_ptr() % 16 \
+       or (wins is not None and not wins(rows, size[0], size[1])):
       return False
   return True
 
 
-def tile_wins(rows: int, weight: torch.Tensor) -> bool:
-  """Above 128 rows two blocks share a weight tile, and the library is as fast where
-  the weight rows fill the chip without a split of k: [37888, 3584] with 256 rows
-  115 us and 81, [8192, 8192] 45 and 77, [8192, 28672] 137 and 313."""
-  return rows <= 128 or _tile().tile_splits(*weight.shape) > 1
+@functools.lru_cache(maxsize=1024)
+def tile_splits(N: int, K: int) -> int:
+  """Parts of k of a product by tiles: as few as give some 450 blocks of 64 weight rows,
+  of 4 steps of 64 at least (splits_of in hip/tile_ops.hip)."""
+  return max(1, min(-(-448 // -(-N // 64)), K // 256, 16))
+
+
+@functools.lru_cache(maxsize=1024)
+def _one_round(N: int, K: int) -> bool:
+  """Whether k is split in three or more and the blocks of 128 weight rows are no more than
+  the chip's 256 CUs. What is split in two has so many rows of x times weight rows that
+  fp32 sums take as long as the weights; 288 blocks take as long as 512."""
+  splits = tile_splits(N, K)
+  return splits >= 3 and -(-N // 128) * splits <= 256
+
+
+@functools.lru_cache(maxsize=1024)
+def _aligned(N: int, K: int) -> bool:
+  """Whether rows and parts of k lie a power of two apart, 16 KB or more, where blocks seem to
+  wait for the same few memory channels (1.06 to 1.27 of the library's time up to 64 rows)."""
+  splits = tile_splits(N, K)
+  return K >= 8192 and K & (K - 1) == 0 and 1 < splits and splits & (splits - 1) == 0
+
+
+# The rules below by what was measured over the library's time, for all products of the
+# registry's dense decoders with weights from memory (rows 4 to 256).
+
+@functools.lru_cache(maxsize=8192)
+def tile_wins(rows: int, N: int, K: int) -> bool:
+  """Whether tile_linear is as fast as the library."""
+  if rows <= 64 and _aligned(N, K):
+    return False
+  if rows <= 16:
+    return True  # 0.34 to 1.08
+  if _one_round(N, K):
+    # the sums' own kernel takes 3 us and more. Up to 64 rows 0.25 to 1.05; up to 128 0.27
+    # to 1.11, smaller weights to 1.59; up to 256 0.36 to 1.11, smaller ones to 1.68
+    return rows <= 64 or N * K >= (9_000_000 if rows <= 128 else 16_500_000)
+  # not split: 0.67 to 1.14 (0.95 on average) up to 64 rows, 0.75 to 1.19 (1.01) up to 128,
+  # 1.26 on average above; split, but in more than a round 1.07, 1.11 and 1.26 on average
+  return rows <= 64 and tile_splits(N, K) == 1
+
+
+@functools.lru_cache(maxsize=8192)
+def parts_win(rows: int, N: int, K: int) -> bool:
+  """The same for tile_parts, whose sums the next kernel adds up: 0.23 to 1.21 (0.7 on
+  average) up to 16 rows, then 0.23 to 1.08 in one round; in more 0.72 to 1.15 up to 64
+  rows (aligned ones to 1.21), 0.72 to 1.54 above, by which layers of mistral-large and
+  llama-3.1-405b took 1.03 to 1.14 of what they take by the library."""
+  return rows <= 16 or _one_round(N, K) or (rows <= 64 and not _aligned(N, K))
+
+
+@functools.lru_cache(maxsize=8192)
+def gate_wins(rows: int, N: int, K: int) -> bool:
+  """The same for tile_swiglu, beside the library and the activation's kernel: 0.36 to 1.16
+  (0.9 on average) up to 128 rows; split in two and in more than a round 0.74 to 1.28
+  (1.05) from 17 rows on; above 128 rows 0.93 to 1.57 (1.28)."""
+  return rows <= 16 or (rows <= 128 and (tile_splits(N, K) != 2 or -(-N // 128) * 2 <= 256))
 
 
 def tile_parted(weight, bias=None) -> bool:
   """Whether tile_linear would split k and add its parts up in a kernel of its own."""
-  return weight.shape[0] % 4 == 0 and (bias is None or bias.dtype == torch.bfloat16) and _tile().tile_splits(*weight.shape) > 1
+  N, K = weight.shape
+  return N % 4 == 0 and (bias is None or bias.dtype == torch.bfloat16) and tile_splits(N, K) > 1
 
 
 def tile_linear(x, weight, bias=None):
