@@ -8,6 +8,7 @@ size the driver measures (1/2/4/8) at a generous generation budget.
 """
 import pytest
 
+from xotorch_amd import ops
 from xotorch_amd.models.config import config_from_hf
 from xotorch_amd.models.registry import builtin_config
 from xotorch_amd.parallel.ring import equal_ring_shards
@@ -43,15 +44,14 @@ def ring_rank_bytes(model_id: str, world: int, mb_batch: int, prompt_len: int,
     if sh.is_last_layer:
       params += V * D + D       # lm_head + final norm
     weights = params * BF16
-    # --- packed decode-GEMM copies (pack_decode_weights default groups:
-    # down_proj, lm_head, gate_up — a second bf16 copy of each) ---
-    packed = L * (I * D + D * 2 * I) * BF16
-    if sh.is_last_layer:
-      packed += V * D * BF16
+    # --- packed decode-GEMM copies (pack_decode_weights: a second bf16 copy of
+    # those of down_proj, gate_up and lm_head that it pays for) ---
+    packed = sum(n * N * K for n, N, K in ((L, D, I), (L, 2 * I, D), (int(sh.is_last_layer), V, D))
+                 if ops.copy_pays(N, K)) * BF16
     # --- KV caches: M micro-batches x 2 (K,V) x L layers, [B, KVH, T, hd];
     # the MFMA fragment-packed copies double residency ---
     kv = M * 2 * L * mb_batch * KVH * T * hd * BF16
-    if packed_attn and hd == 128:
+    if packed_attn and hd in (64, 128):
       kv *= 2
     # --- static I/O + position buffers (small) + prefill activation chunk
     # (bounded by XOT_PREFILL_CHUNK=128: chunk x S x 2I bf16 gate_up out) ---

@@ -50,8 +50,50 @@ def test_products_go_where_they_are_faster():
   assert ops.tile_wins(256, 4096, 14336) and not ops.tile_wins(129, 3072, 2048)
   assert ops.tile_wins(64, 28672, 4096) and not ops.tile_wins(65, 28672, 4096) and not ops.tile_wins(17, 17920, 1536)
   assert not ops.tile_wins(4, 8192, 8192) and ops.tile_wins(128, 8192, 8192)
+  assert ops.copy_pays(57344, 8192) and ops.copy_pays(12288, 28672) and not ops.copy_pays(8192, 28672) and not ops.copy_pays(16384, 2048)
   assert ops.gate_wins(128, 57344, 8192) and not ops.gate_wins(129, 57344, 8192)
   assert ops.gate_wins(16, 17920, 1536) and not ops.gate_wins(17, 17920, 1536) and ops.gate_wins(128, 16384, 2048)
+
+
+@pytest.mark.gpu
+def test_only_copies_that_are_read():
+  """One layer of the sizes of a 70B decoder: a copy of what tiles always do is not made,
+  one that was made is among what is timed for steps of 64 rows."""
+  from xotorch_amd import ops
+  from xotorch_amd.engine.kvcache import make_cache
+  from xotorch_amd.models import llama
+  from xotorch_amd.models.config import config_from_hf
+  from xotorch_amd.models.registry import builtin_config
+  from xotorch_amd.shard import Shard
+  cfg = config_from_hf(builtin_config("llama-3-70b"), "llama-3-70b")
+  shard = Shard("llama-3-70b", 3, 3, cfg.n_layers)
+  with torch.device("meta"):
+    model = llama.ShardedModel(cfg, shard)
+  model = model.to(BF).to_empty(device="cuda").eval()
+  model.reset_rope()
+  g = torch.Generator(device="cuda").manual_seed(0)
+  with torch.inference_mode():
+    for p in model.parameters():
+      p.normal_(0, 0.02, generator=g) if p.dim() > 1 else p.fill_(1)
+    model.pack_decode_weights()
+    mlp, attn = model.layers["3"].mlp, model.layers["3"].self_attn
+    assert mlp.gate_up_proj.weight_packed is not None
+    assert all(m.weight_packed is None for m in (mlp.down_proj, attn.qkv_proj, attn.o_proj))
+    x = torch.randn(64, 1, cfg.dim, generator=g, device="cuda").to(BF)
+    found = []
+    for copies in (True, False):
+      cache = make_cache(cfg, shard, 64, 32, BF, "cuda")
+      at = torch.zeros(1, dtype=torch.int32, device="cuda")
+      if not copies:
+        mlp.gate_up_proj.unpack_decode()
+      found.append(model(x, caches=cache.caches, positions=at, start_pos=-1, is_decode=True,
+                         seq_lens=torch.ones(64, dtype=torch.int32, device="cuda")).float())
+    assert ("gate", 57344, 8192, 64) in llama._PACKED_WINS
+    assert (found[0] - found[1]).norm() <= 0.01 * found[1].norm()
+    y = mlp.gate_up_proj(x)
+    mlp.gate_up_proj.pack_decode()
+    assert (mlp.gate_up_proj(x).float() - y.float()).norm() <= 0.01 * y.float().norm()
+    assert (57344, 8192, 64) in llama._PACKED_WINS
 
 
 @pytest.mark.gpu

@@ -428,13 +428,14 @@ class DeepseekV3Model(nn.Module):
 
   def pack_decode_weights(self, reserve_bytes: int = 0) -> int:
     """MLA projections + dense/shared MLPs get the packed skinny-GEMM
-    prepack (auto-picked per shape vs hipBLASLt); MoE experts get the
+    prepack where a copy pays (ops.copy_pays; auto-picked per shape); MoE experts get the
     stacked grouped prepack; routed per-expert linears are NOT individually
     packed (the grouped copy already covers them). MLA decode attention
     runs the absorbed-latent MFMA kernel via the packed cache."""
     packed = 0
     for name, mod in self.named_modules():
-      if isinstance(mod, XotLinear) and mod.packable() and ".experts." not in name:
+      if isinstance(mod, XotLinear) and mod.packable() and ".experts." not in name and (
+          ops.fp8_gemm_enabled() or ops.copy_pays(*mod.weight.shape)):
         mod.pack_decode()
         if mod.weight_packed is not None:
           packed += mod.weight_packed.numel() * 2

@@ -17,7 +17,7 @@ from __future__ import annotations
 
 import math
 import os
-from typing import List, Optional, Tuple
+from typing import Callable, List, Optional, Tuple
 
 import torch
 import torch.nn as nn
@@ -56,15 +56,29 @@ def _watched(*modules) -> bool:
   return any(m._forward_hooks or m._forward_pre_hooks for m in modules) or torch.nn.modules.module._has_any_global_hook()
 
 
+def _fastest(key, captured: str, **ways: Callable) -> str:
+  """The fastest of these ways, timed now and kept in _PACKED_WINS. Any but the first has
+  to win by 5%: closer ones would change from run to run. While a graph is captured
+  nothing can be timed: `captured`."""
+  if torch.cuda.is_current_stream_capturing():
+    return captured
+  times = {name: _time_us(f) for name, f in ways.items()}
+  first = next(iter(ways))
+  use = _PACKED_WINS[key] = min(times, key=lambda name: times[name] * (0.95 if name == first else 1.0))
+  if os.getenv("XOT_DEBUG", "0") != "0":
+    print(f"[xot] auto-pick {key}: " + ", ".join(f"{n} {t:.1f} us" for n, t in times.items()) + f" -> {use}", flush=True)
+  return use
+
+
 class XotLinear(nn.Linear):
-  """nn.Linear with an optional decode-path prepack: `pack_decode()` stores a
-  second copy of the weight in MFMA A-fragment order ([N/32,K/16,64,8], see
-  ops.pack_decode_weight); decode-shaped (rows 32..256) bf16 GEMMs then run
-  the hand-written CDNA4 weight-streaming kernel where it measures faster
-  than hipBLASLt (auto-picked per (N,K,M) at first call: e.g. 70B down_proj
-  110 -> 84.6 us, lm_head 5.3 -> 6.2 TB/s; hipBLASLt keeps the shapes it
-  wins). Prefill/training/CPU stay on hipBLASLt/aten. Storage/state-dict
-  identical to nn.Linear."""
+  """nn.Linear whose bf16 inference products of up to 256 rows go by the kernels of
+  hip/rows_ops.hip (up to ops.FEW_ROWS rows) and hip/tile_ops.hip (ops.tile_wins), which
+  read the weight as it lies. `pack_decode()` stores a second copy in MFMA A-fragment
+  order ([N/32,K/16,64,8], see ops.pack_decode_weight); with 32, 64 .. 256 rows these
+  ways, the weight-streaming kernels that read the copy and hipBLASLt are timed at the
+  first call and the fastest is kept (lm_head of 70B, 64 rows: 0.87 of the library's time
+  by the copy, 1.07 by tiles). More rows, training and the CPU stay on hipBLASLt and
+  aten. Storage and state dict are nn.Linear's."""
 
   hip = ("_hip_rows", "_hip_tile")  # what a pass loads beside the operators
   weight_packed: Optional[torch.Tensor]
@@ -86,6 +100,10 @@ class XotLinear(nn.Linear):
           self.weight_packed_fp8, self.weight_scale = ops.pack_decode_weight_fp8(self.weight.detach())
       elif self.weight_packed is None:
         self.weight_packed = ops.pack_decode_weight(self.weight.detach())
+
+  def copied(self, rows: int) -> bool:
+    """Whether a product of so many rows can read the packed copy."""
+    return self.weight_packed is not None and 32 <= rows <= 256 and rows % 32 == 0
 
   def unpack_decode(self):
     self.weight_packed = None
@@ -144,42 +162,24 @@ class XotLinear(nn.Linear):
           return y.view(sizes)
     if x.numel() <= ops.FEW_ROWS * self.in_features and ops.few_rows(x, self.weight) and (self.bias is None or self.bias.dtype == torch.bfloat16):
       return ops.rows_linear(x, self.weight, self.bias)
-    if x.numel() <= ops.TILE_ROWS * self.in_features and ops.tile_rows(x, self.weight) and (
-        ops.tile_wins(x.numel() // self.in_features, *self.weight.shape) and (self.bias is None or self.bias.dtype == torch.bfloat16)):
-      return ops.tile_linear(x, self.weight, self.bias)
-    if self.weight_packed is not None and x.is_cuda and x.dtype == torch.bfloat16:
-      N, K = self.weight.shape
+    if x.numel() <= ops.TILE_ROWS * self.in_features and ops.tile_rows(x, self.weight) and (self.bias is None or self.bias.dtype == torch.bfloat16):
+      w, b = self.weight, self.bias
+      N, K = w.shape
       M = x.numel() // K
-      if 32 <= M <= 256 and M % 32 == 0 and x.is_contiguous() and not torch.is_grad_enabled():
+      use = "tile" if ops.tile_wins(M, N, K) else "blaslt"
+      if self.copied(M):
         from xotorch_amd.ops import _load_hip
-        hip = _load_hip()
-        if hip is not None:
-          key = (N, K, M)
-          use = _PACKED_WINS.get(key)
-          if use is None:
-            if torch.cuda.is_current_stream_capturing():
-              use = "packed"  # no timing under capture; normal warmup decides first
-            else:
-              wp, w, b = self.weight_packed, self.weight, self.bias
-              t_packed = _time_us(lambda: hip.skinny_gemm_packed(x, wp, N, b))
-              t_xreg = _time_us(lambda: hip.skinny_gemm_packed_xreg(x, wp, N, b))
-              t_blaslt = _time_us(lambda: torch.nn.functional.linear(x, w, b))
-              # require a clear (>5%) win over hipBLASLt: real wins measure
-              # 20%+ and borderline shapes would flip run-to-run with DVFS
-              use = "blaslt"
-              t_best = t_blaslt * 0.95
-              if t_packed < t_best:
-                use, t_best = "packed", t_packed
-              if t_xreg < t_best:
-                use = "xreg"
-              _PACKED_WINS[key] = use
-              if os.getenv("XOT_DEBUG", "0") != "0":
-                print(f"[xot] gemm auto-pick N={N} K={K} M={M}: packed {t_packed:.1f} us "
-                      f"/ xreg {t_xreg:.1f} us vs blaslt {t_blaslt:.1f} us -> {use}", flush=True)
-          if use == "xreg":
-            return hip.skinny_gemm_packed_xreg(x, self.weight_packed, N, self.bias)
-          if use == "packed":
-            return hip.skinny_gemm_packed(x, self.weight_packed, N, self.bias)
+        hip, wp = _load_hip(), self.weight_packed
+        use = _PACKED_WINS.get((N, K, M)) or _fastest(
+          (N, K, M), use if use == "tile" else "packed",
+          blaslt=lambda: torch.nn.functional.linear(x, w, b), tile=lambda: ops.tile_linear(x, w, b),
+          packed=lambda: hip.skinny_gemm_packed(x, wp, N, b), xreg=lambda: hip.skinny_gemm_packed_xreg(x, wp, N, b))
+        if use == "xreg":
+          return hip.skinny_gemm_packed_xreg(x, wp, N, b)
+        if use == "packed":
+          return hip.skinny_gemm_packed(x, wp, N, b)
+      if use == "tile":
+        return ops.tile_linear(x, w, b)
     return ops.linear(x, self.weight, self.bias)
 
 
@@ -296,19 +296,25 @@ class MLP(nn.Module):
     return ops.swiglu_packed(gu)
 
   def by_tiles(self, x) -> bool:
+    """Whether gated() and parts of the down projection are this MLP."""
     gu, dp = self.gate_up_proj, self.down_proj
     return (type(gu) is XotLinear and type(dp) is XotLinear and not _watched(self, gu, dp)
             and gu.bias is None and dp.bias is None
             and getattr(gu, "weight_packed_fp8", None) is None and getattr(dp, "weight_packed_fp8", None) is None
             and gu.weight.shape[0] % 8 == 0 and ops.tiled(x, gu.weight, dp.weight)
-            and ops.parts_win(x.numel() // x.shape[-1], *dp.weight.shape))
+            and ops.parts_win(x.numel() // x.shape[-1], *dp.weight.shape) and not dp.copied(x.numel() // x.shape[-1]))
 
   def gated(self, x):
     """The gated activation of x (by_tiles)."""
     gu = self.gate_up_proj
-    if ops.gate_wins(x.numel() // x.shape[-1], *gu.weight.shape):
-      return ops.tile_swiglu(x, gu.weight)
-    return self.act(gu(x))
+    N, K = gu.weight.shape
+    rows = x.numel() // K
+    tile = ops.gate_wins(rows, N, K)
+    if tile and gu.copied(rows):
+      key = "gate", N, K, rows
+      tile = (_PACKED_WINS.get(key) or _fastest(key, "tile", tile=lambda: ops.tile_swiglu(x, gu.weight),
+                                                split=lambda: self.act(gu(x)))) == "tile"
+    return ops.tile_swiglu(x, gu.weight) if tile else self.act(gu(x))
 
   def forward(self, x):
     gu = self.gate_up_proj(x)
@@ -655,12 +661,12 @@ class ShardedModel(nn.Module):
     return list(range(self.shard.start_layer, self.shard.end_layer + 1))
 
   def pack_decode_weights(self, reserve_bytes: int = 8 << 30) -> int:
-    """Prepack decode-GEMM weights (second copy in MFMA fragment order) in
-    descending measured-win order — down_proj (hipBLASLt ~3 TB/s at K=28672
-    vs 5.4 packed), lm_head, gate_up, qkv/o — greedily while at least
-    `reserve_bytes` of HBM stay free (KV caches and activations are usually
-    allocated before this is called). Returns bytes packed. Policy override:
-    XOT_PACK=none|down|all."""
+    """Packs second copies of weights in MFMA fragment order: of routed experts, whose
+    grouped decode products read them, and of what is worth the memory otherwise
+    (ops.copy_pays; with fp8 weights everything) - down_proj, lm_head, gate_up, then
+    qkv/o - greedily while at least `reserve_bytes` of HBM stay free (KV caches and
+    activations are usually allocated before this is called). Returns bytes packed.
+    XOT_PACK=none packs nothing, all whatever can be packed."""
     mode = os.getenv("XOT_PACK", "auto")
     if mode == "none" or not torch.cuda.is_available():
       return 0
@@ -668,9 +674,11 @@ class ShardedModel(nn.Module):
     for name, mod in self.named_modules():
       if not isinstance(mod, XotLinear) or not mod.packable():
         continue
+      if not ("experts." in name or mode == "all" or ops.fp8_gemm_enabled() or ops.copy_pays(*mod.weight.shape)):
+        continue
       if "down_proj" in name:
         # the packed kernel wins when the split-K grid still fills the chip
-        # (>= ~1.5 blocks/CU); small-N down projections stay on hipBLASLt.
+        # (>= ~1.5 blocks/CU); small-N down projections don't.
         # MoE experts always pack: the grouped launch fills via blockIdx.y.
         if "experts." in name or mod.weight.shape[0] // 128 * 8 >= 384 or mode == "all":
           groups[0].append(mod)
@@ -681,11 +689,8 @@ class ShardedModel(nn.Module):
       else:  # qkv_proj / o_proj / experts' projections
         groups[3].append(mod)
     if mode != "all" and not ops.fp8_gemm_enabled():
-      # default (bf16): the measured winners — down_proj (tuned hipBLASLt
-      # 110 us vs 84.6 packed at 70B decode shapes), lm_head (5.3 -> 6.2
-      # TB/s), gate_up (175.5 vs 178.9 us); qkv/o measure tied on hipBLASLt
-      # — not worth the second weight copy. In fp8 mode every group wins
-      # (half the stream bytes), so all are packed.
+      # default (bf16): qkv/o are not worth the second copy (1.0 of the library's time).
+      # In fp8 mode every group wins (half the stream bytes), so all are packed.
       groups = groups[:3]
     packed = 0
     debug = os.getenv("XOT_DEBUG", "0") != "0"
