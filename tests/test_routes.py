@@ -55,6 +55,18 @@ def test_products_go_where_they_are_faster():
   assert ops.gate_wins(16, 17920, 1536) and not ops.gate_wins(17, 17920, 1536) and ops.gate_wins(128, 16384, 2048)
 
 
+@pytest.mark.parametrize("model_id", ["llama-3-8b", "gemma2-9b", "deepseek-v2-lite"])
+def test_packing_without_a_gpu(model_id):
+  from xotorch_amd.models import model_class_for
+  from xotorch_amd.models.config import config_from_hf
+  from xotorch_amd.models.registry import builtin_config
+  from xotorch_amd.shard import Shard
+  cfg = config_from_hf(builtin_config(model_id), model_id)
+  with torch.device("meta"):
+    model = model_class_for(cfg)(cfg, Shard(model_id, 1, 1, cfg.n_layers))
+  assert model.pack_decode_weights() == 0
+
+
 @pytest.mark.gpu
 def test_only_copies_that_are_read():
   """One layer of the sizes of a 70B decoder: a copy of what tiles always do is not made,

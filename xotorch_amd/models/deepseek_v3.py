@@ -29,6 +29,7 @@ from typing import List
 import torch
 import torch.nn as nn
 
+from xotorch_amd import ops
 from xotorch_amd.models.config import ModelConfig
 from xotorch_amd.models.llama import XotLinear
 from xotorch_amd.ops.torch_ref import rope_cos_sin
