@@ -416,10 +416,10 @@ def parts_win(rows: int, N: int, K: int) -> bool:
 
 @functools.lru_cache(maxsize=8192)
 def gate_wins(rows: int, N: int, K: int) -> bool:
-  """The same for tile_swiglu, beside the library and the activation's kernel: 0.36 to 1.16
-  (0.9 on average) up to 128 rows; split in two and in more than a round 0.74 to 1.28
-  (1.05) from 17 rows on; above 128 rows 0.93 to 1.57 (1.28)."""
-  return rows <= 16 or (rows <= 128 and (tile_splits(N, K) != 2 or -(-N // 128) * 2 <= 256))
+  """The same for tile_swiglu, beside the library and the activation's kernel: 0.36 to 1.21
+  (0.88 on average) up to 64 rows, 0.75 to 1.16 (0.98) up to 128 but split in two and in
+  more than a round 0.78 to 1.28 (1.09); above 128 rows 0.93 to 1.57 (1.28)."""
+  return rows <= 64 or (rows <= 128 and (tile_splits(N, K) != 2 or -(-N // 128) * 2 <= 256))
 
 
 def copy_pays(N: int, K: int) -> bool:
