@@ -226,3 +226,35 @@ def test_probabilities_of_64_channels_stay_fp32(B, H, KVH, T, n):
   ref, size = p @ v, p @ v.abs()
   # the result's rounding, and errors of fp32 scores and sums: nothing of the size of a bf16 probability's
   assert bool(((out - ref).abs() <= ref.abs() * 2.0 ** -8 * 1.01 + size * (4 * off + 2.0 ** -18)).all())
+
+
+def test_many_short_rows_of_own_keys():
+  """Heads of 64 that share no keys, many and short: by the separate kernels, to the same result."""
+  from types import SimpleNamespace
+  from xotorch_amd import ops
+  from xotorch_amd.engine.kvcache import ShardKVCache
+  from xotorch_amd.models.llama import Attention
+  from xotorch_amd.ops import torch_ref
+  B, H, T, n = 128, 16, 100, 50
+  cos, sin = torch_ref.rope_cos_sin(64, T, 10000.0, device="cuda")
+  attn = Attention(SimpleNamespace(n_heads=H, n_kv_heads=H, head_dim=64, dim=64, attn_bias=False, qk_norm=False, norm_eps=1e-6))
+  g = torch.Generator(device="cuda").manual_seed(0)
+  rows = torch.randn(B, n, 3 * H * 64, generator=g, device="cuda").to(torch.bfloat16)
+  qkv = torch.randn(B, 1, 3 * H * 64, generator=g, device="cuda").to(torch.bfloat16)
+  at = torch.tensor([n], dtype=torch.int32, device="cuda")
+  seen = torch.full((B,), n + 1, dtype=torch.int32, device="cuda")
+  found = []
+  for own in (True, False):
+    c = ShardKVCache(1, B, H, T, 64, torch.bfloat16, "cuda")[0]
+    ops.rope_qkv_append(rows.clone(), cos, sin, torch.arange(n, dtype=torch.int32, device="cuda"), c.k, c.v, H, H, 64, c.kp, c.vp)
+    with torch.inference_mode():
+      assert not ops.decode_attends(qkv, H, H, 64, c.kp) and ops.decode_attends(qkv[:127], H, H, 64, c.kp)
+      if own:
+        out = ops.decode_attend(qkv, cos, sin, at, seen, *c[:4], H, H)
+      else:
+        out = attn.attend(qkv.clone(), cos, sin, at, c, -1, True, seen)
+    found.append((out, *c[:4]))
+  for a, b in zip(found[0][1:], found[1][1:]):
+    assert torch.equal(a, b)
+  a, b = found[0][0].float(), found[1][0].float()
+  assert bool(((a - b).abs() <= b.abs() * 2.0 ** -7 + 2.0 ** -14).all())  # both round fp32 sums in other orders
