@@ -41,3 +41,23 @@ def test_prefill_attention(B, S, H, KVH, start, cap, window):
   # probabilities as bf16, above and below the line, and the result
   bound = size * (2.0 ** -7 + 4 * off.transpose(1, 2)) + ref.abs() * 2.0 ** -8
   assert out.shape == ref.shape and bool(((out - ref).abs() <= bound + 1e-6).all())
+
+
+def test_heads_of_64_in_any_order():
+  """Queries whose heads don't lie side by side, or not on 16 bytes."""
+  from xotorch_amd import ops
+  from xotorch_amd.engine.kvcache import ShardKVCache
+  B, S, H, KVH, start = 2, 40, 4, 2, 7
+  g = torch.Generator(device="cuda").manual_seed(0)
+  c = ShardKVCache(1, B, KVH, 64, 64, torch.bfloat16, "cuda")[0]
+  rows = torch.randn(B, start + S, (H + 2 * KVH) * 64, generator=g, device="cuda").to(torch.bfloat16)
+  still, none = torch.ones(start + S, 32, device="cuda"), torch.zeros(start + S, 32, device="cuda")
+  ops.rope_qkv_append(rows, still, none, torch.arange(start + S, dtype=torch.int32, device="cuda"), c.k, c.v, H, KVH, 64, c.kp, c.vp)
+  q = torch.randn(B, S, H, 64, generator=g, device="cuda").to(torch.bfloat16)
+  odd = torch.empty(q.numel() + 4, dtype=torch.bfloat16, device="cuda")[4:].view(q.shape).copy_(q)
+  with torch.inference_mode():
+    ref = ops.attn_prefill(q, c.k, c.v, start, S, c.kp, c.vp).float()
+    for other in (q.transpose(1, 2).contiguous().transpose(1, 2), odd):
+      assert not other.is_contiguous() or other.data_ptr() % 16
+      out = ops.attn_prefill(other, c.k, c.v, start, S, c.kp, c.vp).float()
+      assert bool(((out - ref).abs() <= ref.abs() * 2.0 ** -6 + 2.0 ** -6).all())  # each rounds probabilities and results

@@ -110,8 +110,11 @@ def attn_prefill(q, k_cache, v_cache, start_pos: int, s_len: int, kp=None, vp=No
                  scale=None, softcap: float = 0.0, window: int = 0):
   if q.is_cuda and q.dtype == torch.bfloat16 and kp is not None and q.shape[3] in (64, 128) \
      and kp.dtype == torch.bfloat16 \
+     and (q.shape[3] == 128 or (q.stride(3) == 1 and q.stride(2) == 64 and (q.stride(0) | q.stride(1)) % 8 == 0
+                                and q.data_ptr() % 16 == 0)) \
      and os.getenv("XOT_MFMA_ATTN", "1") == "1" and _use_hip(q):
-    # causal flash-forward on matrix cores, streaming the MFMA-packed cache;
+    # causal flash-forward on matrix cores, streaming the MFMA-packed cache (heads of 64
+    # in any other order are torch's, as they were before they had a packed cache);
     # softcap/window run gemma2 semantics inside the same kernel (fp8-KV
     # mode keeps prefill on the plain bf16 cache via the sdpa path below)
     return _hip.attn_prefill_mfma(q, kp, vp, start_pos, scale or 0.0, softcap, window)
