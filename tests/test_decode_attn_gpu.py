@@ -258,3 +258,16 @@ def test_many_short_rows_of_own_keys():
     assert torch.equal(a, b)
   a, b = found[0][0].float(), found[1][0].float()
   assert bool(((a - b).abs() <= b.abs() * 2.0 ** -7 + 2.0 ** -14).all())  # both round fp32 sums in other orders
+
+
+def test_lengths_of_more_rows_than_the_step_has():
+  from xotorch_amd import ops
+  from xotorch_amd.engine.kvcache import ShardKVCache
+  c = ShardKVCache(1, 3, 1, 32, 128, torch.bfloat16, "cuda")[0]
+  g = torch.Generator(device="cuda").manual_seed(0)
+  qkv = torch.randn(2, 1, 4 * 128, generator=g, device="cuda").to(torch.bfloat16)
+  still, none = torch.ones(32, 64, device="cuda"), torch.zeros(32, 64, device="cuda")
+  at = torch.zeros(2, dtype=torch.int32, device="cuda")
+  seen = torch.ones(3, dtype=torch.int32, device="cuda")
+  out = [ops.decode_attend(qkv, still, none, at, n, *c[:4], 2, 1) for n in (seen, seen[:2])]
+  assert torch.equal(*out)

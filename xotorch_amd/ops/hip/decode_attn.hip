@@ -350,7 +350,7 @@ Tensor decode_attend(Tensor qkv, Tensor cos, Tensor sin, Tensor positions, Tenso
   CHK(cos.size(-1) == HD / 2 && cos.numel() > 0 && cos.numel() <= INT_MAX && sin.sizes() == cos.sizes());
   a.places = (int)(cos.numel() / (HD / 2));
   a.npos = (int)positions.numel();
-  CHK((a.npos == 1 || a.npos == a.B) && lens.numel() == a.B);
+  CHK((a.npos == 1 || a.npos == a.B) && lens.numel() >= a.B);
   CHK((int64_t)a.B * kv_heads * 64 <= INT_MAX);
   for (const OptT* n : {&q_norm, &k_norm})
     if (*n) { check_io(**n, torch::kBFloat16); CHK((*n)->numel() == HD); }
