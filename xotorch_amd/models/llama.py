@@ -52,8 +52,13 @@ def _time_us(fn, reps=4, rounds=3) -> float:
 
 
 def _watched(*modules) -> bool:
-  """Whether hooks wait for a call of one of these modules, whose work then is its own."""
-  return any(m._forward_hooks or m._forward_pre_hooks for m in modules) or torch.nn.modules.module._has_any_global_hook()
+  """Whether somebody waits for a call of one of these modules, whose work then is its own:
+  a hook, or a forward that was put in place of the class's."""
+  for m in modules:
+    own = m.__dict__
+    if own["_forward_hooks"] or own["_forward_pre_hooks"] or "forward" in own:
+      return True
+  return torch.nn.modules.module._has_any_global_hook()
 
 
 def _fastest(key, captured: str, **ways: Callable) -> str:

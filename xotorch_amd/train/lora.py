@@ -82,7 +82,7 @@ class LoRALinear(nn.Module):
     held = (base.weight,) if base.bias is None else (base.weight, base.bias)
     hooks = (base._forward_hooks, base._forward_pre_hooks, base._backward_hooks, base._backward_pre_hooks,
              self.dropout._forward_hooks, self.dropout._forward_pre_hooks)
-    return (type(base) in (nn.Linear, XotLinear) and not any(hooks) and not torch.nn.modules.module._has_any_global_hook()
+    return (type(base) in (nn.Linear, XotLinear) and not any(hooks) and "forward" not in vars(base) and not torch.nn.modules.module._has_any_global_hook()
             and all(t.is_cuda and t.dtype == torch.bfloat16 and not t.requires_grad for t in held)
             and any(t.requires_grad for t in (x, self.lora_a, self.lora_b))
             and not torch.is_autocast_enabled("cuda") and train_ops.plain(x, *held, self.lora_a, self.lora_b))
