@@ -41,6 +41,20 @@ DEVINL void ld4(const bf16_t* p, float* o) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) { bf16_t u = v[i]; o[i] = ld(&u); }
 }
+DEVINL void ld8(const bf16_t* p, float* o) {
+  const bf16x8 v = *(const bf16x8*)p;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) o[i] = (float)v[i];
+}
+DEVINL void ld8(const float* p, float* o) {
+  ld4(p, o);
+  ld4(p + 4, o + 4);
+}
+// A value as a bf16 tensor holds it
+DEVINL float rounded(float f) {
+  const bf16_t b = f2b(f);
+  return ld(&b);
+}
 
 // Four numbers' sum over parts `stride` apart, in order; four parts at a time on their way
 DEVINL floatx4 sum_parts(const float* p, size_t at, size_t stride, int splits) {

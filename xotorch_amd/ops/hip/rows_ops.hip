@@ -55,26 +55,11 @@ DEVINL float spread_sum(typename Sums<COUNT>::V v, int lane) {
   }
 }
 
-// A value as a bf16 tensor holds it. Rounded where the separate operators of many
-// rows round, a step gives the same token whatever it is batched with.
-DEVINL float rounded(float f) {
-  const bf16_t b = f2b(f);
-  return ld(&b);
-}
-
+// Values are rounded where the separate operators of many rows round; the order of the
+// sums is these kernels' own, and another for one row than for two.
 constexpr int MOST_X = 128 * 1024;  // bytes of normed rows
 
 constexpr int log2_of(int n) { return n <= 1 ? 0 : 1 + log2_of(n / 2); }
-
-DEVINL void ld8(const bf16_t* p, float* o) {
-  const bf16x8 v = *(const bf16x8*)p;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) o[i] = (float)v[i];
-}
-DEVINL void ld8(const float* p, float* o) {
-  ld4(p, o);
-  ld4(p + 4, o + 4);
-}
 
 // 16 bytes at `at` of a row of `bytes`, zeros where they lie past its end. AUX 2: read once.
 template <int AUX>

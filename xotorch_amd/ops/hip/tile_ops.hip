@@ -17,7 +17,8 @@
 // [8192, 28672] m 128 97 (199); [8192, 8192] m 128 35 (48); [4608, 3584] m 256 18 (36).
 //
 // How k is split depends on the weights' shape alone, and the order of the sums within
-// a part on nothing: a row's result does not depend on what it is batched with.
+// a part on nothing: a row of these products does not depend on the rows beside it.
+// (Whether a product is one of these does, and so does how attention cuts its keys.)
 #include "common.h"
 
 struct TileArgs {
@@ -29,12 +30,6 @@ struct TileArgs {
 // STORE: bf16 with bias; PART: fp32 sums of a part of k; GATED: weight rows [2 N, K],
 // gate first, bf16 of the gated activation
 enum TileEnd { STORE, PART, GATED };
-
-// A value as a bf16 tensor holds it
-DEVINL float rounded(float f) {
-  const bf16_t b = f2b(f);
-  return ld(&b);
-}
 
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(1))) const void glb_void;
@@ -333,6 +328,7 @@ static TileArgs tile_args(const Tensor& x, const Tensor& w) {
 }
 
 // Parts of k: as few as give some 450 blocks of 64 weight rows, of 4 steps at least
+// (ops.tile_splits says the same, for the rules of which products these are)
 static int splits_of(int rows, int steps) {
   const int tiles = (rows + 63) / 64;
   return std::max(1, std::min({(448 + tiles - 1) / tiles, steps / 4, 16}));

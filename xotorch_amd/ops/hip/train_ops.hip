@@ -7,20 +7,11 @@
 // separate operators passed fp32 copies of it through memory some ten times.
 #include "common.h"
 
-DEVINL void ld8(const bf16_t* p, float* o) {
-  const bf16x8 v = *(const bf16x8*)p;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) o[i] = (float)v[i];
-}
 DEVINL void st8(bf16_t* p, const float* o) {
   bf16x8 v;
 #pragma unroll
   for (int i = 0; i < 8; ++i) v[i] = (__bf16)o[i];
   *(bf16x8*)p = v;
-}
-DEVINL float rounded(float f) {
-  const bf16_t b = f2b(f);
-  return ld(&b);
 }
 
 // ---------------------------------------------------------------------------
