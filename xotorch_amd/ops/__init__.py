@@ -114,7 +114,7 @@ def attn_prefill(q, k_cache, v_cache, start_pos: int, s_len: int, kp=None, vp=No
                                 and q.data_ptr() % 16 == 0)) \
      and os.getenv("XOT_MFMA_ATTN", "1") == "1" and _use_hip(q):
     # causal flash-forward on matrix cores, streaming the MFMA-packed cache (heads of 64
-    # in any other order are torch's, as they were before they had a packed cache);
+    # in any other order are torch's; of 128 they are refused);
     # softcap/window run gemma2 semantics inside the same kernel (fp8-KV
     # mode keeps prefill on the plain bf16 cache via the sdpa path below)
     return _hip.attn_prefill_mfma(q, kp, vp, start_pos, scale or 0.0, softcap, window)
@@ -462,8 +462,9 @@ def parts_add_norm(parts, x, norm=None, eps: float = 0.0, w_bias: float = 0.0, r
 
 
 def load_library(device, dtype: torch.dtype):
-  """Has the GEMM library load its kernels of this type, which takes some 0.35 s once.
-  Decode steps don't use it: without this the first prompt would wait."""
+  """Has the GEMM library load its kernels of this type, which takes 0.35 s once (1.1 with
+  bench.py's table of tuned products). Decode steps don't use it: without this the first
+  prompt would wait."""
   a = torch.zeros(512, 512, device=device, dtype=dtype)
   torch.nn.functional.linear(a, a)
 

@@ -12,7 +12,8 @@
 // length, so that short rows of a ragged batch have as many blocks as long ones.
 //
 // Probabilities of 64-channel heads stay fp32, as three bf16 parts that hold all their
-// bits; those of 128-channel heads are rounded, as in the kernels of that size before.
+// bits (errors against 64 bits 0.00164, 0.00188 with rounded ones); those of 128-channel
+// heads are rounded to bf16 (0.00192 to 0.00197).
 //
 // The projection may come as fp32 sums over parts of k (tile_ops.hip): a block adds up
 // its heads' numbers in LDS, which saves a kernel between the two: 2.4 us of its 4.7 in
