@@ -50,7 +50,7 @@ def test_products_go_where_they_are_faster():
   assert ops.tile_wins(256, 4096, 14336) and not ops.tile_wins(129, 3072, 2048)
   assert ops.tile_wins(64, 28672, 4096) and not ops.tile_wins(65, 28672, 4096) and not ops.tile_wins(17, 17920, 1536)
   assert not ops.tile_wins(4, 8192, 8192) and ops.tile_wins(128, 8192, 8192)
-  assert ops.copy_pays(57344, 8192) and ops.copy_pays(12288, 28672) and not ops.copy_pays(8192, 28672) and not ops.copy_pays(16384, 2048)
+  assert ops.copy_pays(57344, 8192) and ops.copy_pays(12288, 28672) and not ops.copy_pays(8192, 28672) and not ops.copy_pays(28672, 4096)
   assert ops.gate_wins(128, 57344, 8192) and not ops.gate_wins(129, 57344, 8192)
   assert ops.gate_wins(64, 17920, 1536) and not ops.gate_wins(65, 17920, 1536) and ops.gate_wins(128, 16384, 2048)
 
