@@ -431,7 +431,7 @@ def gate_wins(rows: int, N: int, K: int) -> bool:
 def copy_pays(N: int, K: int) -> bool:
   """Whether a copy of bf16 weights in fragment order (pack_decode_weight) is worth its
   memory: products that tiles do in one round never read it, and below 2.5 10^8 numbers it
-  took 0.88 to 2.1 of the library's time with 32 and 64 rows, which the gated tile or the
+  took 0.77 to 1.31 of the library's time with 32 and 64 rows, which the gated tile or the
   plain one came close to or passed (24576 to 37888 rows of 3584 to 5120: 0.9 to 1.03 beside
   0.83 to 1.09, with the activation inside). Above, 0.65 to 1.07 with 32 to 128 rows."""
   return N * K >= 250_000_000 and not _one_round(N, K)
