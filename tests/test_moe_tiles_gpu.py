@@ -52,3 +52,40 @@ def test_routes_of_bf16_logits_and_wide_sums(T, E, k, D):
   y = torch.randn(gather.numel(), D, generator=g, device="cuda").to(torch.bfloat16)
   wide, rounded = hip.moe_combine(y, place, w, True), hip.moe_combine(y, place, w)
   assert wide.dtype == torch.float32 and torch.equal(wide.to(torch.bfloat16), rounded)
+
+
+@pytest.mark.parametrize("tile", [128, 256])
+@pytest.mark.parametrize("K,F", [(64, 16), (128, 144), (192, 272), (320, 64), (576, 528)])  # steps of k, tiles of features
+@pytest.mark.parametrize("swiglu", [False, True])
+@pytest.mark.parametrize("few", [False, True])  # on average up to 56 rows an expert, or more
+def test_rows_of_an_expert(tile, K, F, swiglu, few):
+  """Experts of all numbers of rows at which a tile's form changes, none among them."""
+  from xotorch_amd.ops.mixer_ops import load_hip
+  hip = load_hip("_hip_experts")
+  counts = [0, 1, 64, 0, 65, 129] if few else [0, 63, 128, 129, 0, 192, 193, 256, 257, 321, 513, 700, 1]
+  assert (sum(counts) <= 56 * len(counts)) == few
+  first = [0]
+  for c in counts:
+    first.append(first[-1] + c)
+  pairs = first[-1]
+  tiles = [(e, r) for e in range(len(counts)) for r in range(first[e], first[e + 1], tile)]
+  most = pairs // tile + len(counts)
+  listed = tiles + [(-1, 0)] * (most - len(tiles)) + [(-1, len(tiles))]
+  g = torch.Generator(device="cuda").manual_seed(K + F)
+  n = pairs // 2 + 1
+  x = torch.randn(n if swiglu else pairs, K, generator=g, device="cuda").to(torch.bfloat16)
+  token = torch.randint(0, n, (pairs,), generator=g, device="cuda", dtype=torch.int32)
+  w = [(torch.randn((2 if swiglu else 1) * F, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16) for _ in counts]
+  ints = dict(dtype=torch.int32, device="cuda")
+  got = hip.expert_product_of(x, w, token, torch.tensor(first, **ints), torch.tensor(listed, **ints), tile, swiglu)
+  rows = (x[token.long()] if swiglu else x).double()
+  for e in range(len(counts)):
+    r = rows[first[e]:first[e + 1]]
+    want, size = r @ w[e].double().t(), r.abs() @ w[e].double().abs().t()
+    slack = size * (K + 8) * 2.0 ** -24  # fp32 sums of K products
+    if swiglu:
+      (gate, up), (sg, su) = want.chunk(2, -1), slack.chunk(2, -1)
+      want = torch.nn.functional.silu(gate) * up
+      # silu's slope is at most 1.1; its hardware exponential and reciprocal are off by some 2^-20
+      slack = (1.1 * sg + gate.abs() * 2.0 ** -19) * up.abs() + su * gate.abs()
+    assert bool(((got[first[e]:first[e + 1]].double() - want).abs() <= slack + want.abs() * 2.0 ** -8 + 1e-30).all()), counts[e]

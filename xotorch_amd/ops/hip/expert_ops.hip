@@ -15,6 +15,7 @@
 // Two element types: bf16 and fp32 (fp32 MFMA throughout).
 
 #include "common.h"
+#include "mfma_tile.h"
 
 // ---------------------------------------------------------------------------
 // router
@@ -200,7 +201,7 @@ __global__ __launch_bounds__(256) void count_scan_kernel(int* __restrict__ count
 
 // Rows of all pairs: row[pair], token[row] and, by_row given, the pair's weight;
 // first row of every expert [E + 1]; tiles (expert, first row), expert -1 past
-// the last.
+// the last, and behind them (-1, how many there are).
 __global__ __launch_bounds__(256) void place_kernel(
     const int* __restrict__ idx, const int* __restrict__ rank, const int* __restrict__ before,
     const int* __restrict__ total, const float* __restrict__ weight, int* __restrict__ row, int* __restrict__ token,
@@ -244,7 +245,10 @@ __global__ __launch_bounds__(256) void place_kernel(
     for (int i = 0; i * a.tile < cnt[e]; ++i) tiles[tile_at[e] + i] = make_int2(e, at[e] + i * a.tile);
   }
   for (int i = ends[1] + threadIdx.x; i < max_tiles; i += 256) tiles[i] = make_int2(-1, 0);
-  if (threadIdx.x == 0) first[a.all] = ends[0];
+  if (threadIdx.x == 0) {
+    first[a.all] = ends[0];
+    tiles[max_tiles] = make_int2(-1, ends[1]);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -356,13 +360,13 @@ __global__ __launch_bounds__(256) void expert_stream_kernel(
   else if (hi > r0) round(r0, std::integral_constant<int, 1>());
 }
 
-// Many tokens per expert (bf16): TOK tokens x 256 weight rows (GATED: 128 gate
-// and the same 128 up) per block, a wave 64 x 128 of it, k in steps of 64
-// through 2 (TOK 256) or 3 LDS buffers. LDS rows hold 8 pieces of 16 bytes,
-// piece p of row r at place p ^ (r & 7): loads go straight to LDS lane by lane,
-// so the permutation sits in the global address, and fragment reads spread
-// over the banks.
-constexpr int TILE_W = 256;  // weight rows
+// Many tokens per expert (bf16): up to TOK tokens x BN weight rows (GATED: BN / 2 gate and
+// the same of up) per block, by mfma_tile.h. What bounds them is the matrix cores, and
+// rows of a tile that no token fills: an expert's rows go over its tiles evenly, in steps
+// of 64, and the fewer a tile has the more waves share the weight rows out. 8 experts of
+// 4096 x 14336, two of them a token, both products, us: 2100 tokens 1533 (with tiles of
+// 256 and what is left, each as if whole, and a barrier between reading and multiplying,
+// 1916), 4000 tokens 2495 (3102), 620 676 (833), 200 509 (640).
 
 // Where an expert's weight rows lie: in one tensor, or in one tensor each
 struct Stacked {
@@ -375,133 +379,116 @@ struct Listed {
   DEVINL const bf16_t* of(int e, size_t) const { return w[e]; }
 };
 
-template <int TOK> struct TileShape {
-  static constexpr int WAVES = TOK / 32, BUFS = TOK == 256 ? 2 : 3, BUF = (TILE_W + TOK) * 64;  // elements of a buffer
-};
+// Of 64, 128, 192 and 256 tokens: waves along the weight rows, buffers of weights and tokens
+template <int BN, int BM, int WN_, int WB, int XB> struct Shape : MfmaTile<BN, BM, WN_, WB, XB> { static constexpr int WN = WN_; };
+template <int BN, int BM> struct ExpertTile;
+template <> struct ExpertTile<256, 64> : Shape<256, 64, 8, 4, 4> {};
+template <> struct ExpertTile<256, 128> : Shape<256, 128, 4, 3, 3> {};
+template <> struct ExpertTile<256, 192> : Shape<256, 192, 4, 3, 2> {};
+template <> struct ExpertTile<256, 256> : Shape<256, 256, 2, 3, 2> {};
+template <> struct ExpertTile<128, 64> : Shape<128, 64, 4, 3, 3> {};
+template <> struct ExpertTile<128, 128> : Shape<128, 128, 2, 2, 2> {};
+template <int BN, int TOK> constexpr int expert_lds() {
+  const int few = std::max(ExpertTile<BN, 64>::LDS, ExpertTile<BN, 128>::LDS);
+  if constexpr (TOK == 128) return few;
+  else return std::max({few, ExpertTile<BN, 192>::LDS, ExpertTile<BN, 256>::LDS});
+}
 
-template <int KIND, int TOK, typename W>
-__global__ __launch_bounds__(TOK * 2) void expert_tile_kernel(
-    const bf16_t* __restrict__ x, W w, const int* __restrict__ first,
-    const int* __restrict__ token, const int2* __restrict__ tiles, const float* __restrict__ by_row,
-    bf16_t* __restrict__ y, int max_tiles, int group, GroupArgs a, Act act) {
-  typedef TileShape<TOK> Sh;
+// One tile: tokens r0 up to hi, of which there are at most BM
+template <int KIND, int BN, int BM>
+DEVINL void expert_tile(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const int* __restrict__ token,
+                        const float* __restrict__ by_row, bf16_t* __restrict__ y, const GroupArgs& a, const Act& act,
+                        int r0, int hi, int fb, bf16_t* buf) {
+  typedef ExpertTile<BN, BM> Sh;
   constexpr bool TWO = has_gate(KIND);  // weight rows are gate and up
-  constexpr int WL = TILE_W / Sh::WAVES / 8, XL = 4, LOADS = WL + XL;  // loads of a stage and wave
-  extern __shared__ __attribute__((aligned(16))) bf16_t buf[];  // [BUFS][weights [256][64], tokens [TOK][64]]
-  // blocks go round the eight dies: give a die `group` neighbouring tiles and
-  // all their features, so that its L2 serves both operands
-  const int nf = (a.F + (TWO ? 127 : 255)) / (TWO ? 128 : 256);
-  const int local = blockIdx.x >> 3, per = group * nf;
-  const int m = (local / per * 8 + (blockIdx.x & 7)) * group + local % group, fb = local % per / group;
-  if (m >= max_tiles) return;
-  const int2 tile = tiles[m];
-  if (tile.x < 0) return;
-  const int hi = first[tile.x + 1], r0 = tile.y;
+  constexpr int R = Sh::R, C = Sh::C, ROWS = R * 16;  // a wave's weight rows: gate rows, then the same of up
+  constexpr int WL = Sh::WL, XL = Sh::XL;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
-  const int wf = wave & 1, wt = wave >> 1;  // which 128 weight rows, which 64 tokens
-  // an expert's last tile: waves without tokens only load (of 256 tokens; with 128 the
-  // branch costs more than it saves)
-  const bool some = TOK < 256 || r0 + wt * 64 < hi;
-  const int f0 = fb * (TWO ? 128 : 256);
-  // each wave stages its share of the weight rows and 32 tokens, 8 rows a load
+  const int wf = wave % Sh::WN, wt = wave / Sh::WN, f0 = fb * (TWO ? BN / 2 : BN);
   const bf16_t *wsrc[WL], *xsrc[XL];
   const int piece = ((lane & 7) ^ (lane >> 3)) * 8;
+  const unsigned woff = ((lane >> 3) * a.kp + piece) * 2;
 #pragma unroll
-  for (int i = 0; i < WL; ++i) {
-    const int r = (wave * WL + i) * 8 + (lane >> 3);
-    // GATED rows: [64 gate, the same 64 up] for either half of the features
-    const int f = TWO ? f0 + (r >> 7) * 64 + (r & 63) : f0 + r;
-    const int part = TWO ? (r >> 6) & 1 : 0;
-    wsrc[i] = w.of(tile.x, (size_t)(TWO ? 2 : 1) * a.F * a.kp) + ((size_t)part * a.F + min(f, a.F - 1)) * a.kp + piece;
+  for (int i = 0; i < WL; ++i) {  // F % 16 == 0: the 8 rows of a load are there, or none of them
+    const int r = (wave * WL + i) * 8;
+    const int f = TWO ? f0 + r / ROWS * (ROWS / 2) + r % (ROWS / 2) : f0 + r;
+    const int part = TWO ? r / (ROWS / 2) & 1 : 0;
+    wsrc[i] = w + ((size_t)part * a.F + min(f, a.F - 8)) * a.kp;
   }
 #pragma unroll
   for (int i = 0; i < XL; ++i) {
-    const int t = min(r0 + wave * 32 + i * 8 + (lane >> 3), hi - 1);
+    const int t = min(r0 + (wave * XL + i) * 8 + (lane >> 3), hi - 1);
     xsrc[i] = x + (size_t)(KIND == PLAIN ? t : token[t]) * a.xs;
   }
-  auto stage = [&](int s) {
-    const int k = s * 64;
-    bf16_t* dst = buf + (s % Sh::BUFS) * Sh::BUF;
-#pragma unroll
-    for (int i = 0; i < WL; ++i)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(wsrc[i] + k),
-                                       (__attribute__((address_space(3))) void*)(dst + (wave * WL + i) * 512), 16, 0, 0);
-    // past the end of a row the weights are zero; any number of the row will do
-    const int kx = k + piece < a.K ? k + piece : 0;
-#pragma unroll
-    for (int i = 0; i < XL; ++i)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xsrc[i] + kx),
-                                       (__attribute__((address_space(3))) void*)(dst + (TILE_W + wave * 32 + i * 8) * 64), 16, 0, 0);
+  auto loadw = [&](auto number, int s, unsigned at) {
+    constexpr int i = decltype(number)::value;
+    __builtin_amdgcn_global_load_lds((glb_void*)((const char*)(wsrc[i] + s * 64) + woff), (lds_void*)((char*)buf + at + (wave * WL + i) * 1024), 16, 0, 0);
   };
-  floatx4 acc[8][4];
+  auto loadx = [&](auto number, int s, unsigned at) {
+    constexpr int i = decltype(number)::value;
+    const int k = s * 64 + piece;
+    // past the end of a row the weights are zero; any number of the row will do
+    __builtin_amdgcn_global_load_lds((glb_void*)(xsrc[i] + (k < a.K ? k : 0)), (lds_void*)((char*)buf + at + (wave * XL + i) * 1024), 16, 0, 0);
+  };
+  floatx4 acc[R][C];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < R; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = (floatx4)(0.f);
-  const int steps = (a.K + 63) / 64;
-  stage(0);
-  if (Sh::BUFS == 3 && steps > 1) stage(1);
+    for (int j = 0; j < C; ++j) acc[i][j] = (floatx4)(0.f);
   // a lane's fragments, as LDS byte addresses within a buffer
-  const unsigned wl = (unsigned)(size_t)(__attribute__((address_space(3))) bf16_t*)(buf + (wf * 128 + col) * 64);
-  const unsigned xl = (unsigned)(size_t)(__attribute__((address_space(3))) bf16_t*)(buf + (TILE_W + wt * 64 + col) * 64);
+  const unsigned base = (unsigned)(size_t)(lds_void*)buf;
+  const unsigned wl = base + (wf * ROWS + col) * 128, xl = base + Sh::XAT + (wt * C * 16 + col) * 128;
   const unsigned place[2] = {(unsigned)((quad ^ (col & 7)) * 16), (unsigned)(((4 + quad) ^ (col & 7)) * 16)};
-  for (int s = 0; s < steps; ++s) {
-    // this step is in LDS (of three buffers, the next may still be on its
-    // way); the buffer of the one before is free
-    if (Sh::BUFS == 3 && s + 1 < steps) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(LOADS) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    const unsigned at = (unsigned)(s % Sh::BUFS) * (Sh::BUF * 2);
-    // reads by hand: the compiler would make them wait for every pending load to LDS
-    constexpr int SETS = Sh::BUFS == 3 ? 2 : 1;  // halves of the step in registers at a time
-    bf16x8 wv[SETS][8], xv[SETS][4];
-    auto read = [&](int kk, bf16x8* w8, bf16x8* x4) {
-      const unsigned wa = wl + at + place[kk], xa = xl + at + place[kk];
-#define READ(D, A, I) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(D) : "v"(A), "i"((I) * 2048))
-      READ(x4[0], xa, 0); READ(x4[1], xa, 1); READ(x4[2], xa, 2); READ(x4[3], xa, 3);
-      READ(w8[0], wa, 0); READ(w8[1], wa, 1); READ(w8[2], wa, 2); READ(w8[3], wa, 3);
-      READ(w8[4], wa, 4); READ(w8[5], wa, 5); READ(w8[6], wa, 6); READ(w8[7], wa, 7);
-#undef READ
-    };
-    if (some)
+  walk<Sh>(acc, wl, xl, place, (a.K + 63) / 64, loadw, loadx);
 #pragma unroll
-      for (int kk = 0; kk < SETS; ++kk) read(kk, wv[kk], xv[kk]);
-    if (s + Sh::BUFS - 1 < steps) stage(s + Sh::BUFS - 1);
-    if (some)
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      bf16x8 *w8 = wv[kk % SETS], *x4 = xv[kk % SETS];
-      if (SETS == 1 && kk == 1) read(1, w8, x4);
-      // 12 reads of the second half may be pending while the first is used
-#define TIE(D) "+v"(D)
-#define WAIT(N)                                                                                                       \
-  asm volatile("s_waitcnt lgkmcnt(" #N ")" : TIE(x4[0]), TIE(x4[1]), TIE(x4[2]), TIE(x4[3]), TIE(w8[0]), TIE(w8[1]), \
-               TIE(w8[2]), TIE(w8[3]), TIE(w8[4]), TIE(w8[5]), TIE(w8[6]), TIE(w8[7]))
-      if (SETS == 2 && kk == 0) WAIT(12);
-      else WAIT(0);
-#undef WAIT
-#undef TIE
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = mma(w8[i], x4[j], acc[i][j]);
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int t = r0 + wt * 64 + j * 16 + col;
+  for (int j = 0; j < C; ++j) {
+    const int t = r0 + (wt * C + j) * 16 + col;
     if (t >= hi) continue;
     bf16_t* dst = y + (size_t)t * a.ys;
     const float by = KIND != PLAIN && by_row ? by_row[t] : 1.f;
-    constexpr int N = TWO ? 4 : 8;
+    constexpr int N = TWO ? R / 2 : R;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const int f = f0 + wf * 16 * N + i * 16 + quad * 4;
       float v[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = activated<KIND>(by, acc[i][j][r], acc[(i + 4) & 7][j][r], act);
+      for (int r = 0; r < 4; ++r) v[r] = activated<KIND>(by, acc[i][j][r], acc[(i + R / 2) % R][j][r], act);
       if (f < a.F) st4(dst + f, v);
     }
+  }
+}
+
+// The router's tiles, of which there are as many as the last of `tiles` says
+template <int KIND, int BN, int TOK, typename W>
+__global__ __launch_bounds__(512) void expert_tile_kernel(
+    const bf16_t* __restrict__ x, W w, const int* __restrict__ first,
+    const int* __restrict__ token, const int2* __restrict__ tiles, const float* __restrict__ by_row,
+    bf16_t* __restrict__ y, int max_tiles, int group, GroupArgs a, Act act) {
+  extern __shared__ __attribute__((aligned(16))) bf16_t buf[];
+  // blocks go round the eight dies: a die has a run of them, in panels of `group` tiles
+  // whose weight rows come one after the other, so that its L2 serves both operands
+  constexpr bool TWO = has_gate(KIND);
+  constexpr int WIDE = TWO ? BN / 2 : BN;
+  const int nf = (a.F + WIDE - 1) / WIDE, real = __builtin_amdgcn_readfirstlane(tiles[max_tiles].y);
+  const int die = blockIdx.x & 7, at = blockIdx.x >> 3, each = real * nf / 8, rest = real * nf % 8;
+  if (at >= each + (die < rest)) return;
+  const int n = die * each + min(die, rest) + at, per = group * nf, panel = n / per, in = n % per;
+  const int wide = min(group, real - panel * group), m = panel * group + in % wide, fb = in / wide;
+  const int2 tile = tiles[m];
+  const int e = __builtin_amdgcn_readfirstlane(tile.x);
+  // an expert's rows go over its tiles evenly, in steps of 64
+  const int lo = __builtin_amdgcn_readfirstlane(first[e]), end = __builtin_amdgcn_readfirstlane(first[e + 1]);
+  const int of = (end - lo + TOK - 1) / TOK, share = ((end - lo + of - 1) / of + 63) / 64 * 64;
+  const int r0 = lo + (__builtin_amdgcn_readfirstlane(tile.y) - lo) / TOK * share, hi = min(end, r0 + share);
+  const bf16_t* we = w.of(e, (size_t)(TWO ? 2 : 1) * a.F * a.kp);
+  auto go = [&](auto rows) { expert_tile<KIND, BN, decltype(rows)::value>(x, we, token, by_row, y, a, act, r0, hi, fb, buf); };
+  const int rows = hi - r0;
+  if (rows <= 64) go(std::integral_constant<int, 64>());
+  else if (rows <= 128) go(std::integral_constant<int, 128>());
+  else if constexpr (TOK == 256) {
+    if (rows <= 192) go(std::integral_constant<int, 192>());
+    else go(std::integral_constant<int, 256>());
   }
 }
 
@@ -562,7 +549,7 @@ __global__ __launch_bounds__(256) void add_norm_kernel(
 // ===========================================================================
 
 // x [.., D] -> (weights [T, top] fp32, row of every pair [T, top], token of
-// every row, first row of every expert [E + 1], tiles [max, 2], rows of a tile).
+// every row, first row of every expert [E + 1], tiles [max + 1, 2], rows of a tile).
 // `shared` experts follow the routed ones in every token's list (top counts
 // them then); their weight is the sigmoid of one more row of w (gate) or one.
 // on_input: the weights by row [T * top].
@@ -591,7 +578,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, int64_t> route(Tensor x, Tens
   if (on_input) by_row = f32(x, {pairs});
   auto idx = torch::empty({T_, top}, ints), rank = torch::empty({T_, top}, ints), row = torch::empty({T_, top}, ints);
   auto counts = torch::empty({all, nblk}, ints), total = torch::empty({all}, ints), first = torch::empty({all + 1}, ints);
-  auto token = torch::empty({pairs}, ints), tiles = torch::empty({max_tiles, 2}, ints);
+  auto token = torch::empty({pairs}, ints), tiles = torch::empty({max_tiles + 1, 2}, ints);
   const RouteArgs a{T_, D, E, (int)top, (int)groups, (int)keep, nblk, tile, (float)scale, (int)pick, (int)all, softmax, gate};
   const hipStream_t stream = cur_stream();
   CHK(groups <= 4 * 65);
@@ -623,19 +610,26 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, int64_t> route(Tensor x, Tens
 template <typename W>
 static void launch_tiles(const W& w, const Tensor& x, const Tensor& token, const Tensor& first, const Tensor& tiles,
                          int64_t tile, int64_t kind, const GroupArgs& a, const Act& act, const float* by_row, Tensor& y) {
-  const int width = has_gate((int)kind) ? TILE_W / 2 : TILE_W;
-  const int max_tiles = tiles.size(0), group = std::min(8, std::max(1, max_tiles / 64)), nf = (a.F + width - 1) / width;
-  const dim3 grid((max_tiles + 8 * group - 1) / (8 * group) * 8 * group * nf);
+  const int max_tiles = tiles.size(0) - 1, pairs = token.numel(), rows = has_gate((int)kind) ? 2 * a.F : a.F;
+  CHK(max_tiles >= 1);
   CHK(tile == 128 || tile == 256);
-  auto run = [&](auto kernel, int threads, int lds) {
+  // as many tiles as an expert has on average share its weight rows in a die's L2. us of the
+  // gated product above, 3 and 4 of them: 2100 tokens (525 rows an expert) 903, 934; 4000
+  // tokens (1000 rows) 1590, 1504
+  const int group = pairs / (a.E * (int)tile) + 1;
+  // few rows an expert: blocks of 128 weight rows, two to a CU, keep more of them on their
+  // way: 25 and 50 rows 491 and 509 us (553 and 570 with 256); from 75 on 609 (589)
+  const bool half = tile == 128 && pairs <= 56 * a.E;
+  const int bn = half ? 128 : 256, nf = (rows + bn - 1) / bn;
+  const dim3 grid((max_tiles * nf + 7) / 8 * 8);
+  auto run = [&](auto kernel, int lds) {
     const hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     TORCH_CHECK(err == hipSuccess, "no LDS for expert tiles");
-    hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, cur_stream(), P<bf16_t>(x), w, first.data_ptr<int>(),
+    hipLaunchKernelGGL(kernel, grid, dim3(512), lds, cur_stream(), P<bf16_t>(x), w, first.data_ptr<int>(),
                        token.data_ptr<int>(), (const int2*)tiles.data_ptr<int>(), by_row, M<bf16_t>(y), max_tiles, group, a, act);
   };
-#define TILES(KIND, TOK) \
-  run(expert_tile_kernel<KIND, TOK, W>, TOK * 2, TileShape<TOK>::BUFS * TileShape<TOK>::BUF * (int)sizeof(bf16_t))
-#define TILES_OF(KIND) if (tile == 256) TILES(KIND, 256); else TILES(KIND, 128)
+#define TILES(KIND, BN, TOK) run(expert_tile_kernel<KIND, BN, TOK, W>, expert_lds<BN, TOK>())
+#define TILES_OF(KIND) if (half) TILES(KIND, 128, 128); else if (tile == 256) TILES(KIND, 256, 256); else TILES(KIND, 256, 128)
   if constexpr (std::is_same<W, Listed>::value) {
     if (kind == SWIGLU) { TILES_OF(SWIGLU); }
     else { TILES_OF(PLAIN); }
