@@ -65,3 +65,20 @@ def test_sum_and_norm(m, D, parts):
     # bf16 once, and fp32 sums of D squares
     assert bool(((n.double() - ref).abs() <= ref.abs() * (2.0 ** -8 + D * 2.0 ** -24) + 1e-30).all())
   assert torch.equal(ops.parts_add_norm(p, x)[0], f.to(torch.bfloat16))
+
+
+# weight rows that make one round of tiles of 128, 160 and 256; steps of k around the buffers' number
+@pytest.mark.parametrize("m,N,K", [(65, 36872, 64), (128, 40968, 192), (104, 65536, 384), (136, 25480, 128), (193, 32768, 256),
+                                   (136, 31856, 128), (256, 40960, 320), (193, 50952, 64), (256, 65528, 192)])
+def test_gated_products_of_one_round(m, N, K):
+  from xotorch_amd import ops
+  x, w, _ = _inputs(m, N, K)
+  w = w * K ** -0.5
+  with torch.no_grad():
+    assert ops.gate_wins(m, N, K)
+    y = ops.tile_swiglu(x, w).double()
+  ref, terms = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t() * (K * 2.0 ** -24)
+  (g, u), (tg, tu) = ref.chunk(2, -1), (terms + ref.abs() * 2.0 ** -8).chunk(2, -1)  # products are stored as bf16 would be
+  act = torch.nn.functional.silu(g)
+  bound = 1.1 * tg * (u.abs() + tu) + act.abs() * tu + (act * u).abs() * 2.0 ** -8
+  assert bool(((y - act * u).abs() <= bound + 1e-30).all())

@@ -424,8 +424,14 @@ def parts_win(rows: int, N: int, K: int) -> bool:
 def gate_wins(rows: int, N: int, K: int) -> bool:
   """The same for tile_swiglu, beside the library and the activation's kernel: 0.36 to 1.21
   (0.88 on average) up to 64 rows, 0.75 to 1.16 (0.98) up to 128 but split in two and in
-  more than a round 0.78 to 1.28 (1.09); above 128 rows 0.93 to 1.57 (1.28)."""
-  return rows <= 64 or (rows <= 128 and (tile_splits(N, K) != 2 or -(-N // 128) * 2 <= 256))
+  more than a round 0.78 to 1.28 (1.09). With 136 rows and more 0.77 to 1.01 (0.88) where
+  a weight tile makes one round of the chip (gate_tile in hip/tile_ops.hip), else 0.97 to
+  1.57; from 256 weight rows a tile gains nothing on the library at 129."""
+  if rows <= 64:
+    return True
+  if rows <= 128:
+    return tile_splits(N, K) != 2 or -(-N // 128) * 2 <= 256
+  return rows >= 136 and tile_splits(N, K) == 1 and any(199 * t < N <= 256 * t for t in (128, 160, 256))
 
 
 def copy_pays(N: int, K: int) -> bool:

@@ -6,7 +6,7 @@
 //
 // What bounds them is the weights' way from memory, for which every CU wants some
 // 48 KB on its way; library tiles leave that to few blocks. A block owns 64 or 128
-// weight rows and all rows of x (from 129 on 128 of them, or all in 8 waves), and walks its part of
+// weight rows and all rows of x (up to 128, more by mfma_tile.h), and walks its part of
 // k in steps of 64 through a ring of LDS buffers that are filled by direct loads: rows of 128
 // bytes, so whole lines, the 16-byte pieces of row r permuted by r & 7 in the global
 // address, which spreads fragment reads over the banks. Where the weight rows alone
@@ -14,12 +14,13 @@
 // follows anyway (norm, activation).
 //
 // us, library beside: [3584, 18944] m 8 23 (48), m 32 23 (110), m 128 33 (99);
-// [8192, 28672] m 128 97 (199); [8192, 8192] m 128 35 (48); [4608, 3584] m 256 18 (36).
+// [8192, 28672] m 128 97 (199); [8192, 8192] m 128 35 (48); [4608, 3584] m 256 19 (37).
 //
 // How k is split depends on the weights' shape alone, and the order of the sums within
 // a part on nothing: a row of these products does not depend on the rows beside it.
 // (Whether a product is one of these does, and so does how attention cuts its keys.)
 #include "common.h"
+#include "mfma_tile.h"
 
 struct TileArgs {
   const bf16_t *x, *w, *bias;
@@ -30,9 +31,6 @@ struct TileArgs {
 // STORE: bf16 with bias; PART: fp32 sums of a part of k; GATED: weight rows [2 N, K],
 // gate first, bf16 of the gated activation
 enum TileEnd { STORE, PART, GATED };
-
-typedef __attribute__((address_space(3))) void lds_void;
-typedef __attribute__((address_space(1))) const void glb_void;
 
 // R fragments from a on and C from b on, 16 rows (2 KB) apart; waits for them
 template <int R, int C>
@@ -65,12 +63,64 @@ DEVINL void read_frags(unsigned a, unsigned b, bf16x8* r, bf16x8* c) {
 template <int BN, int BM, int BUFS>
 struct TileShape {
   static constexpr int ROWS = BN + BM, BUF = ROWS * 64;  // elements of a buffer
-  static constexpr int WAVES = BM == 256 ? 8 : 4;
+  static constexpr int WAVES = 4;
   static constexpr int WL = BN / 8 / WAVES, XL = BM >= 32 ? BM / 8 / WAVES : 1;  // loads of a wave and stage
   static constexpr int LDS = BUFS * BUF * 2;
   // waves along x: the weight rows are split over all four for few rows of x
-  static constexpr int WX = BM == 256 ? 4 : BM >= 64 ? 2 : 1, R = BN * WX / WAVES / 16, C = BM / WX / 16;
+  static constexpr int WX = BM >= 64 ? 2 : 1, R = BN * WX / WAVES / 16, C = BM / WX / 16;
 };
+
+// A wave's sums of weight rows wr .. of a tile and rows m0 .. of x
+template <int END, int BN, int R, int C>
+DEVINL void finish_tile(const TileArgs& a, const floatx4 (&acc)[R][C], int tile, int split, int m0, int wr, int lane) {
+  const int col = lane & 15, quad = lane >> 4;
+#pragma unroll
+  for (int j = 0; j < C; ++j) {
+    const int m = m0 + j * 16 + col;
+    if (END == GATED) {
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        // lanes of quads 0 and 1 hold gates, those of 2 and 3 the products of up
+        const int n = tile * (BN / 2) + (wr + i * 16) / 2 + quad * 4;
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = siluf(rounded(acc[i][j][r])) * rounded(__shfl_xor(acc[i][j][r], 32));
+        if (m >= a.m || quad > 1) continue;
+        bf16_t* dst = (bf16_t*)a.y + (size_t)m * a.N + n;
+        if (n + 3 < a.N && (a.N & 3) == 0) st4(dst, v);
+        else
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (n + r < a.N) st(dst + r, v[r]);
+      }
+    } else {
+      if (m >= a.m) continue;
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        const int n = tile * BN + wr + i * 16 + quad * 4;
+        const bool whole = n + 3 < a.N && (a.N & 3) == 0;
+        if (END == PART) {
+          float* dst = (float*)a.y + ((size_t)split * a.m + m) * a.N + n;
+          if (whole) *(floatx4*)dst = acc[i][j];
+          else
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (n + r < a.N) dst[r] = acc[i][j][r];
+        } else {
+          float v[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = acc[i][j][r] + (a.bias && n + r < a.N ? ld(a.bias + n + r) : 0.f);
+          bf16_t* dst = (bf16_t*)a.y + (size_t)m * a.N + n;
+          if (whole) st4(dst, v);
+          else
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (n + r < a.N) st(dst + r, v[r]);
+        }
+      }
+    }
+  }
+}
 
 template <int BN, int BM, int BUFS, int END>
 __global__ __launch_bounds__((TileShape<BN, BM, BUFS>::WAVES * 64)) void tile_kernel(TileArgs a) {
@@ -147,52 +197,55 @@ __global__ __launch_bounds__((TileShape<BN, BM, BUFS>::WAVES * 64)) void tile_ke
         for (int j = 0; j < C; ++j) acc[i][j] = mma(wf[i], xf[j], acc[i][j]);
     }
   }
+  finish_tile<END, BN, R, C>(a, acc, tile, split, m0 + wx, wr, lane);
+}
+
+// The same of 65 to 256 rows of x, by mfma_tile.h: all of x in a block.
+template <int BN, int BM, int WN, int WB, int XB, int END>
+__global__ __launch_bounds__(512) void wide_kernel(TileArgs a) {
+  typedef MfmaTile<BN, BM, WN, WB, XB> Sh;
+  constexpr int R = Sh::R, C = Sh::C, WL = Sh::WL, XL = Sh::XL, PER = END == GATED ? BN / 2 : BN;
+  extern __shared__ __attribute__((aligned(16))) bf16_t buf[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int col = lane & 15, quad = lane >> 4, piece = ((lane & 7) ^ (lane >> 3)) * 8;
+  // blocks go round the eight dies: a die has a run of them, so that its L2 holds few parts of x
+  const int tiles = (a.N + PER - 1) / PER, units = tiles * a.splits, die = blockIdx.x & 7, rest = units % 8;
+  if ((int)(blockIdx.x >> 3) >= units / 8 + (die < rest)) return;
+  const int unit = die * (units / 8) + min(die, rest) + (blockIdx.x >> 3), tile = unit % tiles, split = unit / tiles;
+  const int s0 = (int)((long long)a.steps * split / a.splits), s1 = (int)((long long)a.steps * (split + 1) / a.splits);
+  const bf16_t *wsrc[WL], *xsrc[XL];
+  int wto[WL];
 #pragma unroll
-  for (int j = 0; j < C; ++j) {
-    const int m = m0 + wx + j * 16 + col;
-    if (END == GATED) {
-#pragma unroll
-      for (int i = 0; i < R; ++i) {
-        // lanes of quads 0 and 1 hold gates, those of 2 and 3 the products of up
-        const int n = tile * (BN / 2) + (wr + i * 16) / 2 + quad * 4;
-        float v[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = siluf(rounded(acc[i][j][r])) * rounded(__shfl_xor(acc[i][j][r], 32));
-        if (m >= a.m || quad > 1) continue;
-        bf16_t* dst = (bf16_t*)a.y + (size_t)m * a.N + n;
-        if (n + 3 < a.N && (a.N & 3) == 0) st4(dst, v);
-        else
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (n + r < a.N) st(dst + r, v[r]);
-      }
-    } else {
-      if (m >= a.m) continue;
-#pragma unroll
-      for (int i = 0; i < R; ++i) {
-        const int n = tile * BN + wr + i * 16 + quad * 4;
-        const bool whole = n + 3 < a.N && (a.N & 3) == 0;
-        if (END == PART) {
-          float* dst = (float*)a.y + ((size_t)split * a.m + m) * a.N + n;
-          if (whole) *(floatx4*)dst = acc[i][j];
-          else
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (n + r < a.N) dst[r] = acc[i][j][r];
-        } else {
-          float v[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] = acc[i][j][r] + (a.bias && n + r < a.N ? ld(a.bias + n + r) : 0.f);
-          bf16_t* dst = (bf16_t*)a.y + (size_t)m * a.N + n;
-          if (whole) st4(dst, v);
-          else
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (n + r < a.N) st(dst + r, v[r]);
-        }
-      }
-    }
+  for (int i = 0; i < WL; ++i) {  // past the last 8 rows: the same again
+    const int g = min(wave * WL + i, BN / 8 - 1), sub = lane >> 3;
+    // GATED: 8 gate rows and the same 8 up rows in turn
+    const size_t row = END == GATED ? min(tile * PER + (g >> 1) * 8 + sub, a.N - 1) + (g & 1 ? (size_t)a.N : 0)
+                                    : min(tile * PER + g * 8 + sub, a.N - 1);
+    wsrc[i] = a.w + row * a.K + s0 * 64 + piece;
+    wto[i] = g * 1024;
   }
+#pragma unroll
+  for (int i = 0; i < XL; ++i)
+    xsrc[i] = a.x + (size_t)min((wave * XL + i) * 8 + (lane >> 3), a.m - 1) * a.K + s0 * 64 + piece;
+  auto loadw = [&](auto number, int s, unsigned at) {
+    constexpr int i = decltype(number)::value;
+    __builtin_amdgcn_global_load_lds((glb_void*)(wsrc[i] + s * 64), (lds_void*)((char*)buf + at + wto[i]), 16, 0, 2);
+  };
+  auto loadx = [&](auto number, int s, unsigned at) {
+    constexpr int i = decltype(number)::value;
+    __builtin_amdgcn_global_load_lds((glb_void*)(xsrc[i] + s * 64), (lds_void*)((char*)buf + at + (wave * XL + i) * 1024), 16, 0, 0);
+  };
+  floatx4 acc[R][C];
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int j = 0; j < C; ++j) acc[i][j] = (floatx4)(0.f);
+  const int wr = wave % WN * (R * 16), wx = wave / WN * (C * 16);
+  const unsigned base = (unsigned)(size_t)(lds_void*)buf;
+  const unsigned wl = base + (wr + col) * 128, xl = base + Sh::XAT + (wx + col) * 128;
+  const unsigned place[2] = {(unsigned)((quad ^ (col & 7)) * 16), (unsigned)(((4 + quad) ^ (col & 7)) * 16)};
+  walk<Sh>(acc, wl, xl, place, s1 - s0, loadw, loadx);
+  finish_tile<END, BN, R, C>(a, acc, tile, split, wx, wr, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -289,11 +342,32 @@ static void launch_tile(const TileArgs& a) {
 //   m 32: [2048, 2048] in 128 blocks 4.4, 5.0; [3584, 18944] in 224 25.6, 22.9
 //   m 64: [2048, 2048] 5.0, 6.0; [28672 -> 8192] 89.7, 76.1
 //   m 128, 3 and 2 buffers: [8192, 8192] in 256 35.4, 39.6; [57344, 8192] in 448 203, 194
-// and with 128 rows of x a block or all (weights read once, x's tile for twice the work):
-//   m 256: [2048, 2048] in 128 9.1, 12.0; [3072, 2048] in 192 12.9, 13.1; [4608, 3584] in
-//   252 18.6, 18.1; [3584, 18944] in 224 55.6, 47.5; [28672 -> 8192] 157, 137
-// (turns of two groups of waves, reading and multiplying, gained 2% on that: what bounds
-// these is the way from L2, 43 GB/s to a CU.)
+// From 129 rows of x on all of them in one block (wide_kernel), if k is split in enough
+// parts: m 256, and 136 by 192 rows, us, with 128 rows a block: [3584, 18944] in 224 43.3
+// and 36.2 (55.6); [28672 -> 8192] 114.9 and 97.9 (157); with fewer blocks a block's start
+// outweighs it, [2048, 2048] in 128 13.0 (9.1).
+//
+// The gated product of more than 64 rows takes the weight tile that makes one round of the
+// chip's 256 CUs, if there is one: [37888, 3584] 237 blocks of 160 rows 71 with m 256 (library
+// and activation 84; 296 of 128 108, 148 of 256 87), [57344, 8192] 224 of 256 203 (253; 448 of
+// 128 247). Up to 128 rows, whose matrix products are short, 148 blocks of 256 are enough:
+// 64 with m 128 (77; 83).
+static int gate_tile(int rows, int m) {
+  if (m <= 128) return rows > 143 * 256 && rows <= 256 * 256 ? 256 : 0;
+  for (int tile : {128, 160, 256})
+    if (rows > 199 * tile && rows <= 256 * tile) return tile;
+  return 0;
+}
+
+template <int BN, int BM, int WN, int WB, int XB, int END>
+static void launch_wide(const TileArgs& a) {
+  const auto kernel = wide_kernel<BN, BM, WN, WB, XB, END>;
+  const int lds = MfmaTile<BN, BM, WN, WB, XB>::LDS, per = END == GATED ? BN / 2 : BN;
+  const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  TORCH_CHECK(e == hipSuccess, "no LDS for weight tiles");
+  hipLaunchKernelGGL(kernel, dim3(((a.N + per - 1) / per * a.splits + 7) / 8 * 8), dim3(512), lds, cur_stream(), a);
+}
+
 template <int END>
 static void run_tile(const TileArgs& a) {
   const int rows = END == GATED ? 2 * a.N : a.N, units = (rows + 127) / 128 * a.splits;
@@ -304,9 +378,19 @@ static void run_tile(const TileArgs& a) {
   } else if (a.m <= 64) {
     if (units >= 200) launch_tile<128, 64, 3, END>(a);
     else launch_tile<64, 64, 4, END>(a);
-  } else if (a.m > 128 && units >= 200) launch_tile<128, 256, 3, END>(a);
-  else if (units * ((a.m + 127) / 128) > 288) launch_tile<128, 128, 2, END>(a);
-  else launch_tile<128, 128, 3, END>(a);
+  } else {
+    if constexpr (END == GATED) {
+      const int wide = gate_tile(rows, a.m);
+      if (wide == 256 && a.m <= 128) return launch_wide<256, 128, 4, 4, 2, END>(a);
+      if (wide == 256) return launch_wide<256, 256, 2, 3, 2, END>(a);
+      if (wide == 160) return launch_wide<160, 256, 2, 3, 3, END>(a);
+    }
+    if (a.m > 128 && units >= 200) {
+      if (a.m <= 192) launch_wide<128, 192, 2, 4, 4, END>(a);
+      else launch_wide<128, 256, 2, 3, 3, END>(a);
+    } else if (units * ((a.m + 127) / 128) > 288) launch_tile<128, 128, 2, END>(a);
+    else launch_tile<128, 128, 3, END>(a);
+  }
 }
 
 static TileArgs tile_args(const Tensor& x, const Tensor& w) {
