@@ -17,7 +17,7 @@
 // [8192, 28672] m 128 97 (199); [8192, 8192] m 128 35 (48); [4608, 3584] m 256 19 (37).
 //
 // How k is split depends on the weights' shape alone, and the order of the sums within
-// a part on nothing: a row of these products does not depend on the rows beside it.
+// a part on the shape and the weight row: a row of these products does not depend on the rows beside it.
 // (Whether a product is one of these does, and so does how attention cuts its keys.)
 #include "common.h"
 #include "mfma_tile.h"
@@ -25,12 +25,37 @@
 struct TileArgs {
   const bf16_t *x, *w, *bias;
   void* y;  // bf16 [m, N], or fp32 [splits, m, N]
-  int m, N, K, steps, splits;  // steps of 64 in all; N: output features
+  int m, N, K, splits;  // N: output features
+  bool turned, runs;    // see turns, run_tile
+  int whole, more, inv;  // steps of 64 of a part, in all parts `more` besides; 65536 / splits, and one more
 };
+
+// All that a block needs to send its first loads, read at once: the compiler would leave
+// half of it until it knows which tile this is, and wait for memory twice
+DEVINL void read_args(const TileArgs& a) {
+  asm volatile("" ::"s"(a.x), "s"(a.w), "s"(a.m), "s"(a.N), "s"(a.K), "s"(a.splits), "s"(a.whole), "s"(a.more), "s"(a.inv));
+}
+
+// A part's first step, steps * split / splits: up to 16 parts, no division
+DEVINL int part_at(const TileArgs& a, int split) { return split * a.whole + (split * a.more * a.inv >> 16); }
 
 // STORE: bf16 with bias; PART: fp32 sums of a part of k; GATED: weight rows [2 N, K],
 // gate first, bf16 of the gated activation
 enum TileEnd { STORE, PART, GATED };
+
+// Where the blocks of weight rows (or GATED features) from `row` on begin among the `len`
+// steps of their part of k. Blocks that walk k in step read the same columns of rows that
+// lie a multiple of 8 KB apart, which few memory channels hold: where rows or parts do
+// (turns), blocks begin at different places. It goes by weight rows, so that a row of x
+// is summed up as in any other batch. us, all from the start of their part first:
+// [8192, 8192] m 4 34, 23; m 128 36, 29; gate [57344, 8192] m 32 168, 143; m 128 176, 149;
+// [28672, 4096] m 4 45, 39; [4096, 14336] in 7 parts m 32 27, 21. Other lengths gain nothing
+// ([37888, 3584] m 8 47.4, 47.9); long ones lose, whose parts of x come from L2 only while
+// all blocks want the same ([8192, 28672] m 128 93, 115).
+template <int END>
+DEVINL int first_step(const TileArgs& a, int row, int len) {
+  return a.turned ? (int)((((unsigned)row / (END == GATED ? 128 : 256) * 2654435761u >> 16) * (unsigned)len) >> 16) : 0;
+}
 
 // R fragments from a on and C from b on, 16 rows (2 KB) apart; waits for them
 template <int R, int C>
@@ -129,13 +154,22 @@ __global__ __launch_bounds__((TileShape<BN, BM, BUFS>::WAVES * 64)) void tile_ke
   extern __shared__ __attribute__((aligned(16))) bf16_t buf[];  // [BUFS][weights [BN][64], x [BM][64]]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int col = lane & 15, quad = lane >> 4;
-  // blocks go round the eight dies: two blocks of the same weights are neighbours on one
+  read_args(a);
+  // blocks go round the eight dies: two blocks of the same weights are neighbours on one.
+  // The grid says which part a block has, as divisions come before all loads: a product of 7
+  // steps ([3584, 3584], 8 rows) took 7.6 us with three of them and takes 7.1
   const int mts = (a.m + BM - 1) / BM, tiles = (a.N + (END == GATED ? BN / 2 : BN) - 1) / (END == GATED ? BN / 2 : BN);
-  const int local = blockIdx.x >> 3, mt = local % mts, unit = (local / mts << 3) + (blockIdx.x & 7);
-  if (unit >= tiles * a.splits) return;
-  const int tile = unit % tiles, split = unit / tiles;
-  const int s0 = (int)((long long)a.steps * split / a.splits), s1 = (int)((long long)a.steps * (split + 1) / a.splits);
-  const int m0 = mt * BM;
+  const int die = blockIdx.x & 7, local = blockIdx.x >> 3;
+  const int mt = mts > 1 ? local % mts : 0, at = mts > 1 ? local / mts : local;
+  int split = blockIdx.y, tile = at * 8 + ((die - split * tiles) & 7);
+  if (a.runs) {  // or a die has a run of them, and so few parts of x
+    const int units = tiles * a.splits, rest = units & 7, n = at + split * ((tiles + 7) >> 3);
+    if (n >= (units >> 3) + (die < rest)) return;
+    split = (die * (units >> 3) + min(die, rest) + n) / tiles;
+    tile = die * (units >> 3) + min(die, rest) + n - split * tiles;
+  }
+  if (tile >= tiles) return;
+  const int s0 = part_at(a, split), s1 = part_at(a, split + 1), m0 = mt * BM;
   const bf16_t *wsrc[Sh::WL], *xsrc[Sh::XL];
   const int sub = lane >> 3;
   // GATED: 8 gate rows and the same 8 up rows in turn
@@ -153,16 +187,18 @@ __global__ __launch_bounds__((TileShape<BN, BM, BUFS>::WAVES * 64)) void tile_ke
     const int r = BM >= 32 ? (wave * Sh::XL + i) * 8 + sub : wave * 4 + (sub & 3);
     xsrc[i] = a.x + (size_t)min(m0 + r, a.m - 1) * a.K + ((lane & 7) ^ (r & 7)) * 8;
   }
+  const int len = s1 - s0, turn = first_step<END>(a, tile * (END == GATED ? BN / 2 : BN), len);
   auto stage = [&](int s) {
     bf16_t* dst = buf + ((s - s0) % BUFS) * Sh::BUF;
+    const int k = (s + turn < s1 ? s + turn : s + turn - len) * 64;
 #pragma unroll
     for (int i = 0; i < Sh::WL; ++i)
-      __builtin_amdgcn_global_load_lds((glb_void*)(wsrc[i] + s * 64), (lds_void*)(dst + (wave * Sh::WL + i) * 512), 16, 0, 2);
+      __builtin_amdgcn_global_load_lds((glb_void*)(wsrc[i] + k), (lds_void*)(dst + (wave * Sh::WL + i) * 512), 16, 0, 2);
 #pragma unroll
     for (int i = 0; i < Sh::XL; ++i) {
       bf16_t* to = dst + BN * 64 + (BM >= 32 ? (wave * Sh::XL + i) * 512 : wave * 256);
       if (BM >= 32 || lane < 32)
-        __builtin_amdgcn_global_load_lds((glb_void*)(xsrc[i] + s * 64), (lds_void*)to, 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((glb_void*)(xsrc[i] + k), (lds_void*)to, 16, 0, 0);
     }
   };
   floatx4 acc[R][C];
@@ -208,11 +244,12 @@ __global__ __launch_bounds__(512) void wide_kernel(TileArgs a) {
   extern __shared__ __attribute__((aligned(16))) bf16_t buf[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int col = lane & 15, quad = lane >> 4, piece = ((lane & 7) ^ (lane >> 3)) * 8;
+  read_args(a);
   // blocks go round the eight dies: a die has a run of them, so that its L2 holds few parts of x
-  const int tiles = (a.N + PER - 1) / PER, units = tiles * a.splits, die = blockIdx.x & 7, rest = units % 8;
-  if ((int)(blockIdx.x >> 3) >= units / 8 + (die < rest)) return;
-  const int unit = die * (units / 8) + min(die, rest) + (blockIdx.x >> 3), tile = unit % tiles, split = unit / tiles;
-  const int s0 = (int)((long long)a.steps * split / a.splits), s1 = (int)((long long)a.steps * (split + 1) / a.splits);
+  const int tiles = (a.N + PER - 1) / PER, units = tiles * a.splits, die = blockIdx.x & 7, rest = units & 7;
+  if ((int)(blockIdx.x >> 3) >= (units >> 3) + (die < rest)) return;
+  const int unit = die * (units >> 3) + min(die, rest) + (blockIdx.x >> 3), split = a.splits > 1 ? unit / tiles : 0;
+  const int tile = unit - split * tiles, s0 = part_at(a, split), s1 = part_at(a, split + 1);
   const bf16_t *wsrc[WL], *xsrc[XL];
   int wto[WL];
 #pragma unroll
@@ -227,13 +264,15 @@ __global__ __launch_bounds__(512) void wide_kernel(TileArgs a) {
 #pragma unroll
   for (int i = 0; i < XL; ++i)
     xsrc[i] = a.x + (size_t)min((wave * XL + i) * 8 + (lane >> 3), a.m - 1) * a.K + s0 * 64 + piece;
+  const int len = s1 - s0, turn = first_step<END>(a, tile * PER, len);
+  auto step = [&](int s) { return (s + turn < len ? s + turn : s + turn - len) * 64; };
   auto loadw = [&](auto number, int s, unsigned at) {
     constexpr int i = decltype(number)::value;
-    __builtin_amdgcn_global_load_lds((glb_void*)(wsrc[i] + s * 64), (lds_void*)((char*)buf + at + wto[i]), 16, 0, 2);
+    __builtin_amdgcn_global_load_lds((glb_void*)(wsrc[i] + step(s)), (lds_void*)((char*)buf + at + wto[i]), 16, 0, 2);
   };
   auto loadx = [&](auto number, int s, unsigned at) {
     constexpr int i = decltype(number)::value;
-    __builtin_amdgcn_global_load_lds((glb_void*)(xsrc[i] + s * 64), (lds_void*)((char*)buf + at + (wave * XL + i) * 1024), 16, 0, 0);
+    __builtin_amdgcn_global_load_lds((glb_void*)(xsrc[i] + step(s)), (lds_void*)((char*)buf + at + (wave * XL + i) * 1024), 16, 0, 0);
   };
   floatx4 acc[R][C];
 #pragma unroll
@@ -244,7 +283,7 @@ __global__ __launch_bounds__(512) void wide_kernel(TileArgs a) {
   const unsigned base = (unsigned)(size_t)(lds_void*)buf;
   const unsigned wl = base + (wr + col) * 128, xl = base + Sh::XAT + (wx + col) * 128;
   const unsigned place[2] = {(unsigned)((quad ^ (col & 7)) * 16), (unsigned)(((4 + quad) ^ (col & 7)) * 16)};
-  walk<Sh>(acc, wl, xl, place, s1 - s0, loadw, loadx);
+  walk<Sh>(acc, wl, xl, place, len, loadw, loadx);
   finish_tile<END, BN, R, C>(a, acc, tile, split, wx, wr, lane);
 }
 
@@ -333,8 +372,8 @@ static void launch_tile(const TileArgs& a) {
     TORCH_CHECK(e == hipSuccess, "no LDS for weight tiles");
   }
   const int per = END == GATED ? BN / 2 : BN;
-  const int units = (a.N + per - 1) / per * a.splits, mts = (a.m + BM - 1) / BM;
-  hipLaunchKernelGGL((tile_kernel<BN, BM, BUFS, END>), dim3((units + 7) / 8 * 8 * mts), dim3(Sh::WAVES * 64), Sh::LDS, cur_stream(), a);
+  const int tiles = (a.N + per - 1) / per, mts = (a.m + BM - 1) / BM;
+  hipLaunchKernelGGL((tile_kernel<BN, BM, BUFS, END>), dim3((tiles + 7) / 8 * 8 * mts, a.splits), dim3(Sh::WAVES * 64), Sh::LDS, cur_stream(), a);
 }
 
 // Tile and depth by the rows of x and by the blocks that 128 weight rows make. us at
@@ -368,8 +407,20 @@ static void launch_wide(const TileArgs& a) {
   hipLaunchKernelGGL(kernel, dim3(((a.N + per - 1) / per * a.splits + 7) / 8 * 8), dim3(512), lds, cur_stream(), a);
 }
 
+// Whether blocks begin at different places of k (first_step): by the weights' shape alone
+static bool turns(int K, int splits) {
+  return K <= 16384 && (K % 4096 == 0 || (splits > 1 && K % splits == 0 && K / splits % 2048 == 0));
+}
+
 template <int END>
-static void run_tile(const TileArgs& a) {
+static void run_tile(TileArgs a) {
+  a.whole = a.K / 64 / a.splits;
+  a.more = a.K / 64 % a.splits;
+  a.inv = 65536 / a.splits + 1;
+  a.turned = turns(a.K, a.splits);
+  // x larger than a die's L2 has room for: [16384, 16384] m 128 132, 96 us; [16384 -> 16384,
+  // 2048] with x of 0.5 MB 23, 27
+  a.runs = END == PART && (int64_t)a.m * a.K > 1 << 20;
   const int rows = END == GATED ? 2 * a.N : a.N, units = (rows + 127) / 128 * a.splits;
   if (a.m <= 16) launch_tile<64, 16, 4, END>(a);
   else if (a.m <= 32) {
@@ -405,7 +456,6 @@ static TileArgs tile_args(const Tensor& x, const Tensor& w) {
   CHK(((size_t)x.data_ptr() & 15) == 0 && ((size_t)w.data_ptr() & 15) == 0);
   a.m = (int)m;
   a.N = (int)w.size(0);
-  a.steps = a.K / 64;
   a.x = P<bf16_t>(x);
   a.w = P<bf16_t>(w);
   return a;
@@ -427,7 +477,7 @@ static Tensor sized(const Tensor& x, int64_t n) {
 // fp32 [splits, m, N]
 Tensor tile_parts(Tensor x, Tensor w) {
   auto a = tile_args(x, w);
-  a.splits = splits_of(a.N, a.steps);
+  a.splits = splits_of(a.N, a.K / 64);
   auto part = torch::empty({a.splits, a.m, a.N}, x.options().dtype(torch::kFloat32));
   a.y = part.data_ptr();
   run_tile<PART>(a);
@@ -442,7 +492,7 @@ Tensor tile_linear(Tensor x, Tensor w, OptT bias) {
     a.bias = P<bf16_t>(*bias);
   }
   auto y = sized(x, a.N);
-  a.splits = a.N % 4 ? 1 : splits_of(a.N, a.steps);
+  a.splits = a.N % 4 ? 1 : splits_of(a.N, a.K / 64);
   if (a.splits == 1) {
     a.y = y.data_ptr();
     run_tile<STORE>(a);
@@ -461,7 +511,7 @@ Tensor tile_swiglu(Tensor x, Tensor w) {
   CHK(a.N % 8 == 0);
   const int I = a.N / 2;
   auto y = sized(x, I);
-  a.splits = splits_of(a.N, a.steps);
+  a.splits = splits_of(a.N, a.K / 64);
   if (a.splits == 1) {
     a.N = I;
     a.y = y.data_ptr();
