@@ -1,0 +1,94 @@
+"""Products of a training pass (hip/gemm_ops.hip) against 64 bits: rows and features at the
+edges of tiles, sums of one step, of whole ones and of what is left, cut into parts or not."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# tokens, features out and in: tiles of 128 and 256 and a few past them, few tiles (parts) and many
+SIZES = [(64, 64, 64), (65, 72, 128), (127, 520, 64), (200, 128, 1032), (257, 384, 256), (666, 3072, 2048),
+         (333, 16384, 264), (100, 8192, 136), (1001, 256, 4096), (1400, 1536, 896), (70, 40960, 1024), (640, 24, 8)]
+
+
+def _random(seed, *shape):
+  g = torch.Generator(device="cuda").manual_seed(seed)
+  return torch.randn(*shape, generator=g, device="cuda").to(torch.bfloat16)
+
+
+def _near(got, a, b):
+  """got is a b^T: fp32 sums of K products, less than K 2^-24 of their sizes off, stored as bf16."""
+  want, size = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
+  assert got.shape == want.shape
+  return bool(((got.double() - want).abs() <= size * (a.shape[1] + 8) * 2.0 ** -24 + want.abs() * 2.0 ** -8 + 1e-30).all())
+
+
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_products(M, N, K):
+  from xotorch_amd.ops import train_ops
+  hip = train_ops._hip_gemm()
+  x, w, dy = _random(M, M, K), _random(N, N, K), _random(K, M, N)
+  if K % 64 == 0 and N % 4 == 0:
+    assert _near(hip.forward(x, w), x, w)
+  if N % 64 == 0:
+    assert _near(hip.input_gradient(dy, w), dy, w.t())
+  assert _near(hip.weight_gradient(dy, x), dy.t(), x.t())
+
+
+@pytest.mark.parametrize("left", [64, 65, 127, 128, 129, 1003])
+def test_what_is_left_of_a_sum_counts_once(left):
+  """Tokens past whole steps; infinities in rows that the last step has twice stay what they are."""
+  from xotorch_amd.ops import train_ops
+  x, dy = _random(1, left, 136), _random(2, left, 264)
+  assert _near(train_ops._hip_gemm().weight_gradient(dy, x), dy.t(), x.t())
+  x[left - 60, 3] = float("inf")
+  dy[left - 60] = 1.0
+  got = train_ops._hip_gemm().weight_gradient(dy, x)
+  want = dy.float().t() @ x.float()
+  assert torch.equal(got.isfinite(), want.isfinite()) and torch.equal(got.isinf(), want.isinf())
+
+
+@pytest.mark.parametrize("form", ["rows", "batch", "one", "turned", "shifted", "weight shifted", "weight turned", "spread"])
+def test_linears_of_all_forms(form):
+  """Gradients of a linear whatever the strides and alignments of what it is given."""
+  from xotorch_amd import ops
+  from xotorch_amd.ops import train_ops
+  M, N, K = (70, 128, 192) if form != "one" else (1, 128, 192)
+  x, w, dy = _random(1, M, K), _random(2, N, K), _random(3, M, N)
+  if form == "batch":
+    x, dy = x.view(7, 10, K), dy.view(7, 10, N)
+  if form == "one":
+    x, dy = x[0], dy[0]
+  if form == "turned":
+    x = x.t().contiguous().t()
+  if form == "shifted":
+    x = torch.cat([x.new_zeros(1), x.flatten()])[1:].view(M, K)
+  if form == "weight shifted":
+    w = torch.cat([w.new_zeros(1), w.flatten()])[1:].view(N, K)
+  if form == "weight turned":
+    w = w.t().contiguous().t()
+  if form == "spread":
+    dy = dy[:, :1].expand(M, N)
+  x, w = x.detach().requires_grad_(), w.detach().requires_grad_()
+  assert train_ops.takes_linear(x, w)
+  held = []
+  with torch.autograd.graph.saved_tensors_hooks(lambda t: held.append(t.shape) or t, lambda t: t):
+    y = ops.linear(x, w)
+  assert len(held) == 2 and y.shape == dy.shape
+  dx, dw = torch.autograd.grad(y, (x, w), dy)
+  rows, drows = x.detach().reshape(-1, K), dy.reshape(-1, N)
+  assert dx.shape == x.shape and dw.shape == w.shape
+  assert _near(y.detach().reshape(-1, N), rows, w.detach()) and _near(dx.reshape(-1, K), drows, w.detach().t()) and _near(dw, drows.t(), rows.t())
+
+
+def test_linears_that_others_follow():
+  """Second derivatives, functorch and forward mode are torch's operators'."""
+  from torch.func import vmap
+  from xotorch_amd import ops
+  x, w = _random(1, 70, 64).requires_grad_(), _random(2, 128, 64).requires_grad_()
+  dx, = torch.autograd.grad(ops.linear(x, w).float().square().sum(), x, create_graph=True)
+  (again,) = torch.autograd.grad(dx.float().sum(), w)
+  assert again.isfinite().all()
+  assert vmap(lambda t: ops.linear(t, w))(x[None]).shape == (1, 70, 128)
+  with torch.autograd.forward_ad.dual_level():
+    y = ops.linear(torch.autograd.forward_ad.make_dual(x.detach().float(), torch.ones_like(x).float()), w.detach().float())
+    assert torch.autograd.forward_ad.unpack_dual(y).tangent is not None

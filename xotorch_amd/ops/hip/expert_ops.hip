@@ -436,11 +436,8 @@ DEVINL void expert_tile(const bf16_t* __restrict__ x, const bf16_t* __restrict__
   for (int i = 0; i < R; ++i)
 #pragma unroll
     for (int j = 0; j < C; ++j) acc[i][j] = (floatx4)(0.f);
-  // a lane's fragments, as LDS byte addresses within a buffer
   const unsigned base = (unsigned)(size_t)(lds_void*)buf;
-  const unsigned wl = base + (wf * ROWS + col) * 128, xl = base + Sh::XAT + (wt * C * 16 + col) * 128;
-  const unsigned place[2] = {(unsigned)((quad ^ (col & 7)) * 16), (unsigned)(((4 + quad) ^ (col & 7)) * 16)};
-  walk<Sh>(acc, wl, xl, place, (a.K + 63) / 64, loadw, loadx);
+  walk<Sh>(acc, RowFrags<R>(base, wf * ROWS, lane), RowFrags<C>(base + Sh::XAT, wt * C * 16, lane), (a.K + 63) / 64, loadw, loadx);
 #pragma unroll
   for (int j = 0; j < C; ++j) {
     const int t = r0 + (wt * C + j) * 16 + col;

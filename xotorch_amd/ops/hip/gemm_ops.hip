@@ -1,0 +1,214 @@
+// Products of a training pass (bf16, fp32 sums) for some hundred to some thousand tokens:
+//   forward           y = x W^T     [M, N] = [M, K] [N, K]^T
+//   input_gradient    dx = dy W     [M, K] = [M, N] [N, K]
+//   weight_gradient   dW = dy^T x   [N, K] = [M, N]^T [M, K]
+// (The reference trains through torch's own operators, train/trainer of its engines.)
+//
+// What bounds them is the matrix cores, and how many blocks there are for them: library
+// tiles leave most of the chip idle where results are small and sums long. Tiles are
+// walked by mfma_tile.h; an operand whose rows lie along the sum is read as columns, by
+// transposing reads from LDS, so that nothing is transposed in memory. Where tiles are few
+// the sum is cut into parts, whose fp32 sums a second kernel adds up.
+//
+// us, library beside, 666 tokens: input [16384 -> 2048] 56 (111), [128256 -> 2048] 377 (870);
+// weights [16384, 2048] 58 (69), [2048, 2048] 11 (20); forward [8192 -> 2048] 34 (40). 4096
+// tokens: input [28672 -> 4096] 703 (722), weights of it 762 (844), forward 730 (662).
+#include "mfma_tile.h"
+
+struct GemmArgs {
+  const bf16_t *w, *x;  // y[m][n] = sum over k of x(m, k) w(n, k)
+  void* y;              // bf16 [M, N], or fp32 [splits, M, N]
+  int M, N, K;
+  int steps, splits, group;  // steps of 64; tiles of x that are neighbours in a run of blocks
+};
+
+// Where a wave's loads of an operand come from: rows [free, k] or, COL, columns [k, free]
+template <bool COL, int F, int COUNT>
+struct Source {
+  static constexpr int SLOTS = F / 8, ROWS = COL ? 64 / SLOTS : 8;  // of a load: pieces of 16 bytes of a row, rows
+  const char* base;     // of the wave's first load of the sum's first step
+  size_t row, next;     // bytes from a k, and from a load, to the next
+  unsigned off[COUNT];  // this lane's bytes besides
+  DEVINL Source(const bf16_t* p, int f0, int free, int K, int wave, int lane) {
+    const int load = wave * COUNT;
+    if (COL) {
+      base = (const char*)(p + (size_t)(load * ROWS) * free);
+      row = (size_t)free * 2;
+      next = ROWS * row;
+#pragma unroll
+      for (int i = 0; i < COUNT; ++i) {
+        const int slot = lane % SLOTS, f = f0 + (slot ^ col_turn((load + i) * ROWS + lane / SLOTS) << 1) * 8;
+        off[i] = (lane / SLOTS * free + min(f, free - 8)) * 2;
+      }
+    } else {
+      base = (const char*)(p + (size_t)f0 * K);
+      row = 2;
+      next = 0;
+#pragma unroll
+      for (int i = 0; i < COUNT; ++i) {
+        const int r = (load + i) * 8 + (lane >> 3);
+        off[i] = (min(r, free - 1 - f0) * K + ((lane & 7) ^ (r & 7)) * 8) * 2;
+      }
+    }
+  }
+  // number I of the step that begins at k
+  template <int I>
+  DEVINL void load(int k, char* to) const {
+    __builtin_amdgcn_global_load_lds((glb_void*)(base + k * row + I * next + off[I]), (lds_void*)to, 16, 0, 0);
+  }
+};
+
+template <bool COL, int N, int F> struct Operand { typedef RowFrags<N> Frags; };
+template <int N, int F> struct Operand<true, N, F> { typedef ColFrags<N, F> Frags; };
+
+// A block has BN of N and BM of M; WN waves along N
+template <bool WCOL, bool XCOL, int BN, int BM, int WN, int WB, int XB, bool PARTS>
+__global__ __launch_bounds__(512) void gemm_kernel(GemmArgs a) {
+  typedef MfmaTile<BN, BM, WN, WB, XB> Sh;
+  constexpr int R = Sh::R, C = Sh::C, WL = Sh::WL, XL = Sh::XL;
+  extern __shared__ __attribute__((aligned(256))) bf16_t buf[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  // blocks go round the eight dies: a die has a run of them, in panels of `group` tiles of
+  // x that read the same of w
+  const int nts = (a.N + BN - 1) / BN, mts = (a.M + BM - 1) / BM, die = blockIdx.x & 7, at = blockIdx.x >> 3;
+  const int units = nts * mts * a.splits, rest = units & 7;
+  if (at >= (units >> 3) + (die < rest)) return;
+  const int unit = die * (units >> 3) + min(die, rest) + at, split = unit / (nts * mts), in_split = unit % (nts * mts);
+  const int panel = in_split / (a.group * nts), in = in_split % (a.group * nts), wide = min(a.group, mts - panel * a.group);
+  const int m0 = (panel * a.group + in % wide) * BM, n0 = in / wide * BN;
+  const int s0 = (int)((long long)a.steps * split / a.splits), s1 = (int)((long long)a.steps * (split + 1) / a.splits);
+  const Source<WCOL, BN, WL> ws(a.w, n0, a.N, a.K, wave, lane);
+  const Source<XCOL, BM, XL> xs(a.x, m0, a.M, a.K, wave, lane);
+  // the last step of columns ends where they do: what the one before has too is left out
+  const int skip = WCOL && XCOL && s1 == a.steps ? a.steps * 64 - a.K : 0;
+  auto loadw = [&](auto number, int s, unsigned to) {
+    constexpr int i = decltype(number)::value;
+    ws.template load<i>(WCOL && XCOL ? min((s0 + s) * 64, a.K - 64) : (s0 + s) * 64, (char*)buf + to + (wave * WL + i) * 1024);
+  };
+  auto loadx = [&](auto number, int s, unsigned to) {
+    constexpr int i = decltype(number)::value;
+    xs.template load<i>(WCOL && XCOL ? min((s0 + s) * 64, a.K - 64) : (s0 + s) * 64, (char*)buf + to + (wave * XL + i) * 1024);
+  };
+  floatx4 acc[R][C];
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int j = 0; j < C; ++j) acc[i][j] = (floatx4)(0.f);
+  const int wr = wave % WN * (R * 16), wx = wave / WN * (C * 16);
+  const unsigned base = (unsigned)(size_t)(lds_void*)buf;
+  walk<Sh>(acc, typename Operand<WCOL, R, BN>::Frags(base, wr, lane), typename Operand<XCOL, C, BM>::Frags(base + Sh::XAT, wx, lane),
+           s1 - s0, loadw, loadx, skip);
+#pragma unroll
+  for (int j = 0; j < C; ++j) {
+    const int m = m0 + wx + j * 16 + (lane & 15);
+    if (m >= a.M) continue;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int n = n0 + wr + i * 16 + (lane >> 4) * 4;
+      if (n >= a.N) continue;
+      if (PARTS) {
+        *(floatx4*)((float*)a.y + ((size_t)split * a.M + m) * a.N + n) = acc[i][j];
+      } else {
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = acc[i][j][r];
+        st4((bf16_t*)a.y + (size_t)m * a.N + n, v);
+      }
+    }
+  }
+}
+
+// bf16 of the parts' sums, in order; n % 4 == 0
+__global__ __launch_bounds__(256) void parts_kernel(const float* __restrict__ part, bf16_t* __restrict__ y, size_t n, int splits) {
+  for (size_t at = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4; at < n; at += (size_t)gridDim.x * 1024) {
+    const floatx4 s = sum_parts(part, at, n, splits);
+    float v[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = s[r];
+    st4(y + at, v);
+  }
+}
+
+// ===========================================================================
+// host side
+// ===========================================================================
+template <bool WCOL, bool XCOL, int BN, int BM, int WN, int WB, int XB>
+static void launch_gemm(const GemmArgs& a) {
+  const int units = (a.N + BN - 1) / BN * ((a.M + BM - 1) / BM) * a.splits;
+  const int lds = MfmaTile<BN, BM, WN, WB, XB>::LDS;
+  auto run = [&](auto kernel) {
+    const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    TORCH_CHECK(e == hipSuccess, "no LDS for a product's tiles");
+    hipLaunchKernelGGL(kernel, dim3((units + 7) / 8 * 8), dim3(512), lds, cur_stream(), a);
+  };
+  if (a.splits > 1) run(gemm_kernel<WCOL, XCOL, BN, BM, WN, WB, XB, true>);
+  else run(gemm_kernel<WCOL, XCOL, BN, BM, WN, WB, XB, false>);
+}
+
+// Tile and parts by what a round of the chip's 256 CUs takes, us: so much for a step of 64
+// and for a block's begin and end, and the parts' sums once out and in again. Of the four
+// tiles and up to 16 parts it found one within 8% of the fastest for the products above.
+static const struct { int bn, bm; double step, ends; } TILES[4] = {{256, 256, 1.42, 11}, {128, 256, 0.8, 7.5}, {256, 128, 0.8, 7.5}, {128, 128, 0.45, 4.7}};
+struct Choice { int tile, splits; };
+static Choice choose(int64_t M, int64_t N, int steps) {
+  Choice best{0, 1};
+  double least = 1e30;
+  for (int t = 0; t < 4; ++t) {
+    const int64_t blocks = (N + TILES[t].bn - 1) / TILES[t].bn * ((M + TILES[t].bm - 1) / TILES[t].bm);
+    for (int s = 1; s <= 16 && (s == 1 || (steps / s >= 4 && M * N * s <= 1 << 27)); ++s) {
+      const int64_t rounds = (blocks * s + 255) / 256;
+      const double us = rounds * ((steps + s - 1) / s * TILES[t].step + TILES[t].ends) + (s > 1 ? M * N * 8.0 * s / 5e6 + 2.5 : 0);
+      if (us < least) least = us, best = {t, s};
+    }
+  }
+  return best;
+}
+
+// y [M, N] of x [M, K] (XCOL: [K, M]) and w [N, K] (WCOL: [K, N])
+template <bool WCOL, bool XCOL>
+static Tensor product(const Tensor& x, const Tensor& w) {
+  check_io(x, torch::kBFloat16);
+  check_io(w, torch::kBFloat16);
+  CHK(x.dim() == 2 && w.dim() == 2);
+  const int64_t m = x.size(XCOL), N = w.size(WCOL), K = x.size(!XCOL);
+  CHK(K == w.size(!WCOL) && m >= 1 && N >= 1 && K >= 1 && m <= 1 << 22 && N <= 1 << 22 && K <= 1 << 22);
+  CHK(((size_t)x.data_ptr() & 15) == 0 && ((size_t)w.data_ptr() & 15) == 0);
+  // whole pieces of 16 bytes, and steps of the sum: columns' last may begin in the one before
+  CHK(XCOL ? K >= 64 && m % 8 == 0 : K % 64 == 0);
+  CHK(WCOL ? N % 8 == 0 : N % 4 == 0);
+  GemmArgs a{};
+  a.x = P<bf16_t>(x);
+  a.w = P<bf16_t>(w);
+  a.M = (int)m;
+  a.N = (int)N;
+  a.K = (int)K;
+  a.steps = (int)((K + 63) / 64);
+  // us of [4096, 28672 x 4096], panels of 2, 4 and 8 tiles of x: 694, 675, 676; 8192 of all, 766, 733, 723
+  a.group = 4;
+  const Choice c = choose(m, N, a.steps);
+  a.splits = c.splits;
+  CHK((N / TILES[c.tile].bn + 1) * (m / TILES[c.tile].bm + 1) * a.splits <= INT_MAX / 8);
+  auto y = torch::empty({m, N}, x.options());
+  Tensor part;
+  a.y = y.data_ptr();
+  if (a.splits > 1) {
+    part = f32(x, {a.splits, m, N});
+    a.y = part.data_ptr();
+  }
+  if (c.tile == 0) launch_gemm<WCOL, XCOL, 256, 256, 2, 3, 2>(a);
+  else if (c.tile == 1) launch_gemm<WCOL, XCOL, 128, 256, 2, 3, 3>(a);
+  else if (c.tile == 2) launch_gemm<WCOL, XCOL, 256, 128, 4, 3, 3>(a);
+  else launch_gemm<WCOL, XCOL, 128, 128, 2, 4, 4>(a);
+  if (a.splits > 1) {
+    const size_t n = (size_t)m * N;
+    hipLaunchKernelGGL(parts_kernel, dim3(std::min<size_t>((n + 1023) / 1024, 4096)), dim3(256), 0, cur_stream(), part.data_ptr<float>(),
+                       M<bf16_t>(y), n, a.splits);
+  }
+  return y;
+}
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("forward", [](Tensor x, Tensor w) { return product<false, false>(x, w); }, "x w^T of x [M, K], w [N, K]");
+  m.def("input_gradient", [](Tensor dy, Tensor w) { return product<true, false>(dy, w); }, "dy w of dy [M, N], w [N, K]");
+  m.def("weight_gradient", [](Tensor dy, Tensor x) { return product<true, true>(dy, x); }, "dy^T x of dy [M, N], x [M, K]");
+}

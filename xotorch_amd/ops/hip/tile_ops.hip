@@ -243,7 +243,7 @@ __global__ __launch_bounds__(512) void wide_kernel(TileArgs a) {
   constexpr int R = Sh::R, C = Sh::C, WL = Sh::WL, XL = Sh::XL, PER = END == GATED ? BN / 2 : BN;
   extern __shared__ __attribute__((aligned(16))) bf16_t buf[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int col = lane & 15, quad = lane >> 4, piece = ((lane & 7) ^ (lane >> 3)) * 8;
+  const int piece = ((lane & 7) ^ (lane >> 3)) * 8;
   read_args(a);
   // blocks go round the eight dies: a die has a run of them, so that its L2 holds few parts of x
   const int tiles = (a.N + PER - 1) / PER, units = tiles * a.splits, die = blockIdx.x & 7, rest = units & 7;
@@ -281,9 +281,7 @@ __global__ __launch_bounds__(512) void wide_kernel(TileArgs a) {
     for (int j = 0; j < C; ++j) acc[i][j] = (floatx4)(0.f);
   const int wr = wave % WN * (R * 16), wx = wave / WN * (C * 16);
   const unsigned base = (unsigned)(size_t)(lds_void*)buf;
-  const unsigned wl = base + (wr + col) * 128, xl = base + Sh::XAT + (wx + col) * 128;
-  const unsigned place[2] = {(unsigned)((quad ^ (col & 7)) * 16), (unsigned)(((4 + quad) ^ (col & 7)) * 16)};
-  walk<Sh>(acc, wl, xl, place, len, loadw, loadx);
+  walk<Sh>(acc, RowFrags<R>(base, wr, lane), RowFrags<C>(base + Sh::XAT, wx, lane), len, loadw, loadx);
   finish_tile<END, BN, R, C>(a, acc, tile, split, wx, wr, lane);
 }
 

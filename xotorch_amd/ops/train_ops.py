@@ -1,5 +1,5 @@
 """Differentiable forms of the decoder's operators for training on the GPU (bf16,
-hip/train_ops.hip, hip/attn_train.hip): one kernel forward and one backward where separate torch operators
+hip/train_ops.hip, hip/attn_train.hip, hip/gemm_ops.hip): one kernel forward and one backward where separate torch operators
 pass fp32 copies through memory. What they cannot take (other types, tracing,
 functorch transforms, forward-mode) goes by torch_ref, and so does a backward pass
 that is itself differentiated."""
@@ -12,7 +12,7 @@ import torch
 
 from xotorch_amd.ops import torch_ref
 
-_ext = _attn = None
+_ext = _attn = _gemm = None
 OWN = (torch.Tensor, torch.nn.Parameter)
 # looked up once: a step of a small model asks some thirty times
 _is_compiling, _is_tracing, _forward_ad = torch.compiler.is_compiling, torch._C._is_tracing, torch.autograd.forward_ad
@@ -39,11 +39,19 @@ def _hip_attn():
   return _attn
 
 
+def _hip_gemm():
+  global _gemm
+  if _gemm is None:
+    import importlib
+    _gemm = importlib.import_module("xotorch_amd.ops._hip_gemm")
+  return _gemm
+
+
 def _missing() -> bool:
   """Whether the kernels are not built and torch's operators are asked for then."""
-  if (_ext is None or _attn is None) and os.getenv("XOT_ALLOW_EAGER", "0") == "1":
+  if (_ext is None or _attn is None or _gemm is None) and os.getenv("XOT_ALLOW_EAGER", "0") == "1":
     try:
-      _hip(), _hip_attn()
+      _hip(), _hip_attn(), _hip_gemm()
     except ImportError:
       return True
   return False
@@ -90,6 +98,85 @@ def _again(f: Callable, inputs: Sequence[torch.Tensor], needs: Sequence[bool], g
     wanted = [t for t, n in zip(inputs, needs) if n]
     found = iter(torch.autograd.grad([o for o, _ in pairs], wanted, [g for _, g in pairs], create_graph=True, allow_unused=True))
   return [next(found) if n else None for n in needs]
+
+
+# Where the products of hip/gemm_ops.hip are faster than the library's, by what they took of
+# its time (40 to 4096 tokens, the linears of 0.5B, 1B, 8B and 70B decoders; M tokens through
+# a weight [N, K]).
+
+def forward_wins(M: int, N: int, K: int) -> bool:
+  """x W^T: 0.40 to 1.11 (0.73 on average) for narrow results of up to 1000 tokens; wider ones
+  and more tokens 0.95 to 1.40."""
+  return M <= 1000 and N <= 4096 and K % 64 == 0 and N % 4 == 0
+
+
+def input_wins(M: int, N: int, K: int) -> bool:
+  """dy W, a sum over N: 0.25 to 1.07 (0.66 on average) where that is no shorter than the result
+  is wide, or for few tokens; with more tokens 0.46 to 0.95 where it is much longer and 0.92 to
+  1.26 else. Shorter sums: 0.85 to 1.27 from 333 tokens on."""
+  return N % 64 == 0 and K % 8 == 0 and (M <= 1400 and (N >= K or M <= 300) or (M <= 3000 and N >= 8 * K))
+
+
+def weight_wins(M: int, N: int, K: int) -> bool:
+  """dy^T x, a sum over tokens: 0.81 to 1.05 (0.89 on average) from 600 tokens on, and 0.23 to
+  0.8 for small weights; large weights and 100 to 512 tokens 0.85 to 1.16."""
+  return M >= 64 and N % 8 == 0 and K % 8 == 0 and (M >= 600 or N * K <= 7_000_000)
+
+
+_MOST = 1 << 22  # rows, features
+
+
+def product(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+  """x W^T of rows [M, K]"""
+  M, (N, K) = x.shape[0], weight.shape
+  if forward_wins(M, N, K) and weight.is_contiguous() and weight.data_ptr() % 16 == 0:
+    return _hip_gemm().forward(_rows(x), weight)
+  return torch.nn.functional.linear(x, weight)
+
+
+def input_gradient(dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+  """dy W of rows [M, N]"""
+  M, (N, K) = dy.shape[0], weight.shape
+  if input_wins(M, N, K) and weight.is_contiguous() and weight.data_ptr() % 16 == 0:
+    return _hip_gemm().input_gradient(_rows(dy), weight)
+  return dy @ weight
+
+
+def weight_gradient(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+  """dy^T x of rows [M, N] and [M, K]"""
+  if weight_wins(dy.shape[0], dy.shape[1], x.shape[1]):
+    return _hip_gemm().weight_gradient(_rows(dy), _rows(x))
+  return dy.t() @ x
+
+
+def takes_linear(x: torch.Tensor, weight: torch.Tensor) -> bool:
+  """Whether a linear of these, with a gradient, is one of these products at least."""
+  if not (x.is_cuda and torch.is_grad_enabled() and weight.dim() == 2 and 0 < x.numel() and x.shape[-1] == weight.shape[1]):
+    return False
+  (N, K), M = weight.shape, x.numel() // weight.shape[1]
+  return (max(M, N, K) <= _MOST and (forward_wins(M, N, K) or input_wins(M, N, K) or weight_wins(M, N, K)) and K % 8 == 0
+          and x.dtype == weight.dtype == torch.bfloat16 and (x.requires_grad or weight.requires_grad) and plain(x, weight)
+          and not torch._C._is_any_autocast_enabled() and not _missing())
+
+
+class _Linear(torch.autograd.Function):
+  @staticmethod
+  def forward(ctx, x, weight):
+    ctx.save_for_backward(x, weight)
+    return product(x.reshape(-1, x.shape[-1]), weight).view(*x.shape[:-1], weight.shape[0])
+
+  @staticmethod
+  def backward(ctx, dy):
+    x, weight = ctx.saved_tensors
+    if torch.is_grad_enabled():
+      return tuple(_again(torch.nn.functional.linear, (x, weight), ctx.needs_input_grad, (dy,)))
+    rows = dy.reshape(-1, dy.shape[-1])
+    dx = input_gradient(rows, weight).view(x.shape) if ctx.needs_input_grad[0] else None
+    return dx, weight_gradient(rows, x.reshape(-1, x.shape[-1])) if ctx.needs_input_grad[1] else None
+
+
+def linear(x, weight):
+  return _Linear.apply(x, weight)
 
 
 class _Norm(torch.autograd.Function):

@@ -32,7 +32,8 @@ class _Adapted(torch.autograd.Function):
   @staticmethod
   def forward(ctx, x, weight, bias, a, b, scaling):
     rows = x.reshape(-1, x.shape[-1])
-    out, low = F.linear(rows, weight, bias), rows @ a.t()
+    out = F.linear(rows, weight, bias) if bias is not None else train_ops.product(rows, weight)
+    low = rows @ a.t()
     out.addmm_(low, b.t(), alpha=scaling)
     ctx.save_for_backward(x, weight, bias, a, b, low)
     ctx.scaling = scaling
@@ -48,7 +49,7 @@ class _Adapted(torch.autograd.Function):
       return dx, None, None, da, db, None
     dy = dy.reshape(-1, dy.shape[-1])
     dlow = _scaled(dy, b, ctx.scaling) if need_x or need_a else None
-    dx = (dy @ weight).addmm_(dlow, a).view(x.shape) if need_x else None
+    dx = train_ops.input_gradient(dy, weight).addmm_(dlow, a).view(x.shape) if need_x else None
     return (dx, None, None, dlow.t() @ x.reshape(-1, x.shape[-1]) if need_a else None,
             _scaled(dy.t(), low, ctx.scaling) if need_b else None, None)
 
