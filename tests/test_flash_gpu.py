@@ -43,6 +43,27 @@ def test_prefill_attention(B, S, H, KVH, start, cap, window):
   assert out.shape == ref.shape and bool(((out - ref).abs() <= bound + 1e-6).all())
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("B,S,H,KVH,start", [(1, 5, 4, 1, 2100), (1, 7, 6, 2, 1100), (2, 33, 7, 1, 560), (3, 70, 4, 4, 200), (1, 2000, 12, 2, 0)])
+def test_merged_parts(hd, B, S, H, KVH, start):
+  """Keys in 2 to 16 parts, one of them past every position that the first tokens see."""
+  from xotorch_amd.ops import _hip_ops
+  g = torch.Generator(device="cuda").manual_seed(S)
+  T, rep = start + S, H // KVH
+  t32 = -(-T // 32) * 32
+  q, k, v = (torch.randn(*s, hd, generator=g, device="cuda").to(torch.bfloat16) for s in ((B, S, H), (B, KVH, t32), (B, KVH, t32)))
+  kp = k.view(B, KVH, t32 // 16, 16, hd // 32, 4, 8).permute(0, 1, 2, 4, 5, 3, 6).reshape(B, KVH, t32 // 16, hd // 32, 64, 8).contiguous()
+  vp = v.view(B, KVH, t32 // 32, 4, 8, hd // 16, 16).permute(0, 1, 5, 2, 3, 6, 4).reshape(B, KVH, hd // 16, t32 // 32, 64, 8).contiguous()
+  out = _hip_ops.attn_prefill_mfma(q, kp, vp, start, 0.0, 0.0, 0).double()
+  kd, vd = (t[:, :, :T].double().repeat_interleave(rep, 1) for t in (k, v))
+  s = q.double().transpose(1, 2) @ kd.transpose(-1, -2) * hd ** -0.5
+  off = (q.double().abs().transpose(1, 2) @ kd.abs().transpose(-1, -2)).amax(-1, keepdim=True) * hd ** -0.5 * ((hd + 4) * 2.0 ** -24)
+  p = s.masked_fill(torch.arange(start, T, device="cuda")[:, None] < torch.arange(T, device="cuda")[None], -torch.inf).softmax(-1)
+  ref, size = (p @ vd).transpose(1, 2), (p @ vd.abs()).transpose(1, 2)
+  bound = size * (2.0 ** -7 + 4 * off.transpose(1, 2)) + ref.abs() * 2.0 ** -8  # as above
+  assert out.shape == ref.shape and bool(((out - ref).abs() <= bound + 1e-6).all())
+
+
 def test_heads_of_64_in_any_order():
   """Queries whose heads don't lie side by side, or not on 16 bytes."""
   from xotorch_amd import ops

@@ -851,7 +851,7 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
 // few blocks, the keys are split and the parts merged.
 // us, and as it was with a block per head and probabilities through LDS: 6001 tokens,
 // 32 heads on 8 338 (873 TFLOP/s; 1309); 16 x 512, 64 on 8 137 (352); 256 tokens after
-// 1280, 28 on 4 37 (150).
+// 1280, 28 on 4 27 (150).
 // ---------------------------------------------------------------------------
 
 DEVINL floatx4 mma16(const bf16x8& a, const bf16x8& b, floatx4 c) {
@@ -1061,26 +1061,48 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(FlashArgs a) {
   }
 }
 
-// A wave a row of [B, S, H]: the splits' parts, weighed by how far their maxima lie
-// below the largest.
+// The splits' parts, weighed by how far their maxima lie below the largest: four channels a
+// lane, HD / 4 lanes a row, eight parts on their way at a time. Blocks go by key heads as
+// those do that wrote the parts, and so mostly to the die whose L2 has them. us with the
+// kernel before, and with a wave a row and part after part: 256 tokens after 1280, 28 heads
+// on 4, 9 parts 27.2 (10 parts 37.7); after 256, 64 on 8 23.2 (32.4); after 1024, 32 heads of
+// 64 on 8 16.5 (19.5; with the four channels but blocks by tokens 22.5).
 template <int HD>
-__global__ __launch_bounds__(256) void flash_merge_kernel(FlashArgs a, int total) {
-  const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (i >= total) return;
-  const int h = i % a.H, rest = i / a.H, s = rest % a.S, b = rest / a.S, rep = a.H / a.KVH;
-  const size_t row = ((size_t)b * a.KVH + h / rep) * a.S * rep + (size_t)s * rep + h % rep;
-  const float* ml = a.ml + row * a.splits * 2;
-  float top = -1e30f, sum = 0.f, o[2] = {};
-  for (int k = 0; k < a.splits; ++k) top = fmaxf(top, ml[k * 2]);
-  for (int k = 0; k < a.splits; ++k) {
-    const float f = __builtin_amdgcn_exp2f(ml[k * 2] - top);
-    sum += f * ml[k * 2 + 1];
+__global__ __launch_bounds__(256) void flash_merge_kernel(FlashArgs a, int heads) {
+  constexpr int LANES = HD / 4;
+  const int bh = blockIdx.x % heads, r = blockIdx.x / heads * (256 / LANES) + threadIdx.x / LANES, lane = threadIdx.x % LANES;
+  const int rep = a.H / a.KVH, b = bh / a.KVH, kvh = bh % a.KVH;
+  if (r >= a.S * rep) return;
+  const size_t row = (size_t)bh * a.S * rep + r;
+  const float2* ml = (const float2*)a.ml + row * a.splits;
+  const float* part = a.part + row * a.splits * HD + lane * 4;
+  floatx4 v[8], o = (floatx4)(0.f);
+  auto load = [&](int k) {
 #pragma unroll
-    for (int i = 0; i < HD / 64; ++i) o[i] += f * a.part[(row * a.splits + k) * HD + i * 64 + lane];
+    for (int j = 0; j < 8; ++j) v[j] = *(const floatx4*)(part + (size_t)min(k + j, a.splits - 1) * HD);
+  };
+  // lane k of a row has what weighs part k, of 16 at most
+  const bool in = lane < a.splits;
+  const float2 mine = in ? ml[lane] : make_float2(-1e30f, 0.f);
+  load(0);
+  float top = mine.x;
+#pragma unroll
+  for (int mask = 1; mask < LANES; mask <<= 1) top = fmaxf(top, __shfl_xor(top, mask));
+  const float by = in ? __builtin_amdgcn_exp2f(mine.x - top) : 0.f;
+  float sum = by * mine.y;
+#pragma unroll
+  for (int mask = 1; mask < LANES; mask <<= 1) sum += __shfl_xor(sum, mask);
+  for (int k = 0; k < a.splits; k += 8) {
+    if (k) load(k);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (k + j < a.splits) o += __shfl(by, k + j, LANES) * v[j];
   }
   const float f = sum > 0.f ? 1.f / sum : 0.f;
+  ushort4_t y;
 #pragma unroll
-  for (int d = 0; d < HD / 64; ++d) a.out[(size_t)i * HD + d * 64 + lane] = f2b(o[d] * f);
+  for (int j = 0; j < 4; ++j) y[j] = f2b(o[j] * f);
+  *(ushort4_t*)(a.out + (((size_t)b * a.S + r / rep) * a.H + kvh * rep + r % rep) * HD + lane * 4) = y;
 }
 
 // layout probe for tests: one v_mfma_f32_16x16x32_bf16, row-major inputs
@@ -2721,9 +2743,17 @@ torch::Tensor attn_prefill_mfma(torch::Tensor q, torch::Tensor k, torch::Tensor 
   CHK(rows <= INT_MAX / 256);
   a.blocks = (int)((rows + 127) / 128);
   const int64_t whole = (int64_t)a.blocks * B * a.KVH;
-  // two blocks a CU, of two tiles of 64 positions at least
+  // as many blocks as are on the chip at once, two a CU, of two tiles of 64 positions at
+  // least; or some more, if the last ones, which come first in the sequence, are so short
+  // that this costs less than the longest gain (a block's begin and end take as long as two
+  // tiles). us: 256 tokens after 1280, 56 blocks in 9 parts 27, in 10 33; 2000 tokens, 188
+  // blocks in 2 parts 49, in 3 42
   const int tiles = (int)((start + a.S + 63) / 64);
-  a.splits = (int)std::max<int64_t>(1, std::min<int64_t>({(512 + whole - 1) / whole, tiles / 2, 16}));
+  auto takes = [&](int64_t n) {
+    return (double)tiles / n + 2 + (whole * n > 512 ? (double)((start + 63) / 64 + 1) / n + 2 : 0.0);
+  };
+  const int64_t fit = 512 / whole, parts = fit >= 1 && (512 % whole == 0 || takes(fit) <= takes(fit + 1)) ? fit : fit + 1;
+  a.splits = (int)std::max<int64_t>(1, std::min<int64_t>({parts, tiles / 2, 16}));
   CHK(whole * a.splits <= INT_MAX);
   torch::Tensor part, ml;
   if (a.splits > 1) {
@@ -2748,10 +2778,10 @@ torch::Tensor attn_prefill_mfma(torch::Tensor q, torch::Tensor k, torch::Tensor 
     else run(flash_prefill_kernel<64, false>);
   }
   if (a.splits > 1) {
-    const int64_t total = (int64_t)B * a.S * a.H;
-    const dim3 rows4((unsigned)((total + 3) / 4));
-    if (HD == 128) hipLaunchKernelGGL((flash_merge_kernel<128>), rows4, dim3(256), 0, cur_stream(), a, (int)total);
-    else hipLaunchKernelGGL((flash_merge_kernel<64>), rows4, dim3(256), 0, cur_stream(), a, (int)total);
+    const int heads = B * a.KVH, per = 1024 / HD;
+    const dim3 grid((unsigned)((rows + per - 1) / per * heads));
+    if (HD == 128) hipLaunchKernelGGL((flash_merge_kernel<128>), grid, dim3(256), 0, cur_stream(), a, heads);
+    else hipLaunchKernelGGL((flash_merge_kernel<64>), grid, dim3(256), 0, cur_stream(), a, heads);
   }
   return out;
 }
