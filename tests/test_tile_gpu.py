@@ -83,3 +83,16 @@ def test_gated_products_of_one_round(m, N, K):
   act = torch.nn.functional.silu(g)
   bound = 1.1 * tg * (u.abs() + tu) + act.abs() * tu + (act * u).abs() * 2.0 ** -8
   assert bool(((y - act * u).abs() <= bound + 1e-30).all())
+
+
+@pytest.mark.parametrize("m,D,H,I", [(3, 64, 128, 96), (45, 2048, 2048, 8192), (200, 320, 192, 512)])
+def test_rest_of_a_layer_is_its_parts(m, D, H, I):
+  from xotorch_amd import ops
+  g = torch.Generator(device="cuda").manual_seed(m)
+  heads, x, post, after, wo, gu, down = (torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16) * s[-1] ** -0.5 for s in (
+    (1, m, H), (1, m, D), (D,), (D,), (D, H), (2 * I, D), (D, I)))
+  with torch.no_grad():
+    h, n = ops.parts_add_norm(ops.tile_parts(heads, wo), x, post, 1e-5)
+    want = ops.parts_add_norm(ops.tile_parts(ops.tile_swiglu(n, gu), down), h, after, 1e-6, rounded=True)
+    got, alone = ops.tile_rest(heads, wo, x, post, 1e-5, gu, down, after, 1e-6), ops.tile_rest(heads, wo, x, post, 1e-5, gu, down)
+  assert len(got) == 2 and len(alone) == 1 and torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]) and torch.equal(alone[0], want[0])

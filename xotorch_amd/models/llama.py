@@ -61,6 +61,13 @@ def _watched(*modules) -> bool:
   return torch.nn.modules.module._has_any_global_hook()
 
 
+def _own(module, name: str = "weight"):
+  """module.weight (or another parameter) without nn.Module's search for it, which a pass
+  through a small model makes some 700 times, a quarter of a microsecond each."""
+  held = module._parameters
+  return held[name] if name in held else getattr(module, name)
+
+
 def _fastest(key, captured: str, **ways: Callable) -> str:
   """The fastest of these ways, timed now and kept in _PACKED_WINS. Any but the first has
   to win by 5%: closer ones would change from run to run. While a graph is captured
@@ -252,9 +259,10 @@ class Attention(nn.Module):
   def project(self, x):
     """qkv_proj by weight tiles; where k is split, (a place for the queries, the sums over
     parts of k) for attend, whose first kernel adds them up."""
-    p = self.qkv_proj
-    if type(self) is Attention and ops.tile_parted(p.weight, p.bias):
-      return x.new_empty(*x.shape[:-1], p.weight.shape[0]), ops.tile_parts(x, p.weight)
+    p = self._modules["qkv_proj"]
+    w = _own(p)
+    if type(self) is Attention and ops.tile_parted(w, _own(p, "bias")):
+      return x.new_empty(*x.shape[:-1], w.shape[0]), ops.tile_parts(x, w)
     return p(x), None
 
   def attend(self, qkv, cos, sin, positions, kv, start_pos: int, is_decode: bool, seq_lens=None, sums=None):
@@ -269,7 +277,7 @@ class Attention(nn.Module):
     vsc = kv[5] if len(kv) > 5 else None
     qn = self.q_norm if cfg.qk_norm else None
     kn = self.k_norm if cfg.qk_norm else None
-    bias = self.qkv_proj.bias if sums is not None else None
+    bias = _own(self._modules["qkv_proj"], "bias") if sums is not None else None
     if is_decode and ops.decode_attends(qkv, H, cfg.n_kv_heads, hd, kp, qn, kn):
       sl = seq_lens if seq_lens is not None else start_pos + 1
       return ops.decode_attend(qkv, cos, sin, positions, sl, k_cache, v_cache, kp, vp, H, cfg.n_kv_heads,
@@ -302,12 +310,21 @@ class MLP(nn.Module):
 
   def by_tiles(self, x) -> bool:
     """Whether gated() and parts of the down projection are this MLP."""
-    gu, dp = self.gate_up_proj, self.down_proj
-    return (type(gu) is XotLinear and type(dp) is XotLinear and not _watched(self, gu, dp)
-            and gu.bias is None and dp.bias is None
-            and getattr(gu, "weight_packed_fp8", None) is None and getattr(dp, "weight_packed_fp8", None) is None
-            and gu.weight.shape[0] % 8 == 0 and ops.tiled(x, gu.weight, dp.weight)
-            and ops.parts_win(x.numel() // x.shape[-1], *dp.weight.shape) and not dp.copied(x.numel() // x.shape[-1]))
+    gu, dp = self._modules["gate_up_proj"], self._modules["down_proj"]
+    if type(gu) is not XotLinear or type(dp) is not XotLinear or _watched(self, gu, dp):
+      return False
+    up, down, rows = _own(gu), _own(dp), x.numel() // x.shape[-1]
+    return (_own(gu, "bias") is None and _own(dp, "bias") is None
+            and gu.weight_packed_fp8 is None and dp.weight_packed_fp8 is None
+            and up.shape[0] % 8 == 0 and ops.tiled(x, up, down)
+            and ops.parts_win(rows, *down.shape) and not dp.copied(rows))
+
+  def gate_is_tile(self, x) -> bool:
+    """Whether gated() is tile_swiglu without timing it."""
+    gu = self._modules["gate_up_proj"]
+    N, K = _own(gu).shape
+    rows = x.numel() // K
+    return ops.gate_wins(rows, N, K) and not gu.copied(rows)
 
   def gated(self, x):
     """The gated activation of x (by_tiles)."""
@@ -577,23 +594,31 @@ class DecoderLayer(nn.Module):
 
   def by_tiles(self, x) -> bool:
     """Whether `step` takes this layer: products by weight tiles (ops.tile_rows)."""
-    a, m = self.self_attn, self.mlp
-    mods = (a.qkv_proj, a.o_proj)
-    if not all(type(p) is XotLinear and getattr(p, "weight_packed_fp8", None) is None for p in mods):
+    mods = self._modules
+    a, before, post = mods["self_attn"], mods["input_layernorm"], mods["post_attention_layernorm"]
+    q, o = a._modules["qkv_proj"], a._modules["o_proj"]
+    if type(q) is not XotLinear or type(o) is not XotLinear or q.weight_packed_fp8 is not None or o.weight_packed_fp8 is not None:
       return False
-    return (x.shape[-1] % 8 == 0 and x.shape[-1] <= 16384 and not _watched(self, a, *mods, self.post_attention_layernorm)
-            and ops.tiled(x, *(p.weight for p in mods), wins=ops.parts_win)
-            and ops.plain_norms(self.input_layernorm.weight, self.post_attention_layernorm.weight))
+    return (x.shape[-1] % 8 == 0 and x.shape[-1] <= 16384 and not _watched(self, a, q, o, post)
+            and ops.tiled(x, _own(q), _own(o), wins=ops.parts_win)
+            and ops.plain_norms(_own(before), _own(post)))
 
   def step(self, x, normed, cos, sin, positions, kv, start_pos, is_decode, seq_lens, after):
     """The layer with sums that the next norm finishes: (stream, that norm of it).
     `after`: the module of that norm, or None; normed: this layer's, None: not made yet."""
-    a, m = self.self_attn, self.mlp
+    mods = self._modules
+    a, m, post = mods["self_attn"], mods["mlp"], mods["post_attention_layernorm"]
     if normed is None:
       normed = self.input_layernorm(x)
     qkv, sums = a.project(normed)
     out = a.attend(qkv, cos, sin, positions, kv, start_pos, is_decode, seq_lens, *(() if sums is None else (sums,)))
-    post = self.post_attention_layernorm
+    follows = after is not None and not _watched(after) and ops.plain_norms(_own(after))
+    if type(m) is MLP and m.by_tiles(x) and m.gate_is_tile(x):
+      # 45 tokens through 16 layers of 2048: the host took 1171 us a pass for these five calls
+      # and their checks, 975 so
+      found = ops.tile_rest(out, _own(a._modules["o_proj"]), x, _own(post), post.eps, _own(m._modules["gate_up_proj"]),
+                            _own(m._modules["down_proj"]), *((_own(after), after.eps) if follows else ()))
+      return found if follows else (found[0], None)
     x, normed = ops.parts_add_norm(ops.tile_parts(out, a.o_proj.weight), x, post.weight, post.eps)
     if type(m) is MLP and m.by_tiles(normed):
       parts = ops.tile_parts(m.gated(normed), m.down_proj.weight)
@@ -602,7 +627,7 @@ class DecoderLayer(nn.Module):
     else:
       parts = m(normed).float()
     parts = parts.view(-1, x.numel() // x.shape[-1], x.shape[-1])
-    if after is None or _watched(after) or not ops.plain_norms(after.weight):
+    if not follows:
       return ops.parts_add_norm(parts, x)[0], None
     return ops.parts_add_norm(parts, x, after.weight, after.eps, rounded=True)
 

@@ -472,6 +472,12 @@ def parts_add_norm(parts, x, norm=None, eps: float = 0.0, w_bias: float = 0.0, r
   return _tile().parts_add_norm(parts, x, norm, eps, w_bias, rounded)
 
 
+def tile_rest(heads, wo, x, post, post_eps: float, gate_up, down, after=None, after_eps: float = 0.0):
+  """parts_add_norm, tile_swiglu and parts_add_norm again behind a layer's attention, one
+  call from Python: (h, rmsnorm(h) as the next layer wants it), (h,) without a next norm."""
+  return _tile().tile_rest(heads, wo, x, post, post_eps, gate_up, down, after, after_eps)
+
+
 def load_library(device, dtype: torch.dtype):
   """Has the GEMM library load its kernels of this type, which takes 0.35 s once (1.1 with
   bench.py's table of tuned products). Decode steps don't use it: without this the first

@@ -553,7 +553,17 @@ std::vector<Tensor> parts_add_norm(Tensor part, Tensor x, OptT w, double eps, do
   return {h};
 }
 
+// What follows a layer's attention, in one call from Python, which a short prompt through a
+// small model waits for: h = x + heads Wo^T, its norm, the gated activation, h + that Wd^T,
+// and the next layer's norm of it (`after`; none: the stream alone)
+std::vector<Tensor> tile_rest(Tensor heads, Tensor wo, Tensor x, Tensor post, double post_eps, Tensor gate_up, Tensor down,
+                              OptT after, double after_eps) {
+  auto mid = parts_add_norm(tile_parts(heads, wo), x, post, post_eps, 0.0, false);
+  return parts_add_norm(tile_parts(tile_swiglu(mid[1], gate_up), down), mid[0], after, after_eps, 0.0, after.has_value());
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("tile_rest", &tile_rest);
   m.def("tile_splits", [](int64_t n, int64_t k) { return splits_of((int)n, (int)(k / 64)); });
   m.def("tile_parts", &tile_parts);
   m.def("tile_linear", &tile_linear);
