@@ -475,9 +475,9 @@ class MoEMLP(nn.Module):
     products read tokens and weights where they lie."""
     from xotorch_amd.ops.mixer_ops import load_hip
     hip = load_hip("_hip_experts")
-    # tiles of 256 tokens from 150 rows an expert on: 8 experts of 4096 x 14336, two of
-    # them a token, us with 128 and 256: 300 tokens 691, 750; 700 963, 851; 2100 2218, 1904
-    tile = 256 if flat.shape[0] * self.top_k >= 150 * self.n_experts else 128
+    # tiles of 256 tokens from 110 rows an expert on: 8 experts of 4096 x 14336, two of
+    # them a token, us with 128 and 256: 300 tokens 565, 577; 450 607, 602; 620 667, 578
+    tile = 256 if flat.shape[0] * self.top_k >= 110 * self.n_experts else 128
     weight, row, *places = hip.route(flat, self.gate.weight, None, self.top_k, 1, 1, 1.0, True, 0, False, False, tile)
     h = hip.expert_product_of(flat, [e.gate_up_proj.weight for e in self.experts], *places, True)
     y = hip.expert_product_of(h, [e.down_proj.weight for e in self.experts], *places, False)

@@ -364,9 +364,9 @@ __global__ __launch_bounds__(256) void expert_stream_kernel(
 // the same of up) per block, by mfma_tile.h. What bounds them is the matrix cores, and
 // rows of a tile that no token fills: an expert's rows go over its tiles evenly, in steps
 // of 64, and the fewer a tile has the more waves share the weight rows out. 8 experts of
-// 4096 x 14336, two of them a token, both products, us: 2100 tokens 1533 (with tiles of
+// 4096 x 14336, two of them a token, both products, us: 2100 tokens 1447 (with tiles of
 // 256 and what is left, each as if whole, and a barrier between reading and multiplying,
-// 1916), 4000 tokens 2495 (3102), 620 676 (833), 200 509 (640).
+// 1916), 4000 tokens 2495 (3102), 620 578 (833), 200 498 (640).
 
 // Where an expert's weight rows lie: in one tensor, or in one tensor each
 struct Stacked {
@@ -388,10 +388,14 @@ template <> struct ExpertTile<256, 192> : Shape<256, 192, 4, 3, 2> {};
 template <> struct ExpertTile<256, 256> : Shape<256, 256, 2, 3, 2> {};
 template <> struct ExpertTile<128, 64> : Shape<128, 64, 4, 3, 3> {};
 template <> struct ExpertTile<128, 128> : Shape<128, 128, 2, 2, 2> {};
+template <> struct ExpertTile<128, 192> : Shape<128, 192, 2, 4, 4> {};
+template <> struct ExpertTile<128, 256> : Shape<128, 256, 2, 3, 3> {};
+// of all forms that a kernel of BN weight rows and TOK tokens may take
 template <int BN, int TOK> constexpr int expert_lds() {
-  const int few = std::max(ExpertTile<BN, 64>::LDS, ExpertTile<BN, 128>::LDS);
-  if constexpr (TOK == 128) return few;
-  else return std::max({few, ExpertTile<BN, 192>::LDS, ExpertTile<BN, 256>::LDS});
+  int most = std::max(ExpertTile<BN, 64>::LDS, ExpertTile<BN, 128>::LDS);
+  if constexpr (TOK == 256)  // and of 128 weight rows
+    most = std::max({most, expert_lds<128, 128>(), ExpertTile<128, 192>::LDS, ExpertTile<128, 256>::LDS, ExpertTile<256, 192>::LDS, ExpertTile<256, 256>::LDS});
+  return most;
 }
 
 // One tile: tokens r0 up to hi, of which there are at most BM
@@ -456,6 +460,8 @@ DEVINL void expert_tile(const bf16_t* __restrict__ x, const bf16_t* __restrict__
   }
 }
 
+constexpr int DIE_CUS = 32;  // of one of the eight dies
+
 // The router's tiles, of which there are as many as the last of `tiles` says
 template <int KIND, int BN, int TOK, typename W>
 __global__ __launch_bounds__(512) void expert_tile_kernel(
@@ -468,8 +474,17 @@ __global__ __launch_bounds__(512) void expert_tile_kernel(
   constexpr bool TWO = has_gate(KIND);
   constexpr int WIDE = TWO ? BN / 2 : BN;
   const int nf = (a.F + WIDE - 1) / WIDE, real = __builtin_amdgcn_readfirstlane(tiles[max_tiles].y);
-  const int die = blockIdx.x & 7, at = blockIdx.x >> 3, each = real * nf / 8, rest = real * nf % 8;
-  if (at >= each + (die < rest)) return;
+  const int die = blockIdx.x & 7, each = real * nf / 8, rest = real * nf % 8, all = each + (die < rest);
+  // what no more than half of a die's 32 CUs would have left to do is cut in two: 384 blocks
+  // of the down product of 2100 tokens 578 us, so 522 (with up to 128 tokens nothing, to 3% worse)
+  constexpr bool CUT = BN == 256 && TOK == 256;
+  const int whole = CUT && all % DIE_CUS <= DIE_CUS / 2 ? all - all % DIE_CUS : all;
+  int at = blockIdx.x >> 3, half = -1;
+  if (at >= whole) {
+    half = (at - whole) & 1;
+    at = whole + ((at - whole) >> 1);
+  }
+  if (at >= all) return;
   const int n = die * each + min(die, rest) + at, per = group * nf, panel = n / per, in = n % per;
   const int wide = min(group, real - panel * group), m = panel * group + in % wide, fb = in / wide;
   const int2 tile = tiles[m];
@@ -479,7 +494,14 @@ __global__ __launch_bounds__(512) void expert_tile_kernel(
   const int of = (end - lo + TOK - 1) / TOK, share = ((end - lo + of - 1) / of + 63) / 64 * 64;
   const int r0 = lo + (__builtin_amdgcn_readfirstlane(tile.y) - lo) / TOK * share, hi = min(end, r0 + share);
   const bf16_t* we = w.of(e, (size_t)(TWO ? 2 : 1) * a.F * a.kp);
-  auto go = [&](auto rows) { expert_tile<KIND, BN, decltype(rows)::value>(x, we, token, by_row, y, a, act, r0, hi, fb, buf); };
+  auto go = [&](auto rows) {
+    if constexpr (CUT) {
+      if (half < 0) return expert_tile<KIND, BN, decltype(rows)::value>(x, we, token, by_row, y, a, act, r0, hi, fb, buf);
+      if ((fb * 2 + half) * (WIDE / 2) < a.F)
+        expert_tile<KIND, 128, decltype(rows)::value>(x, we, token, by_row, y, a, act, r0, hi, fb * 2 + half, buf);
+    } else
+      expert_tile<KIND, BN, decltype(rows)::value>(x, we, token, by_row, y, a, act, r0, hi, fb, buf);
+  };
   const int rows = hi - r0;
   if (rows <= 64) go(std::integral_constant<int, 64>());
   else if (rows <= 128) go(std::integral_constant<int, 128>());
@@ -618,7 +640,7 @@ static void launch_tiles(const W& w, const Tensor& x, const Tensor& token, const
   // way: 25 and 50 rows 491 and 509 us (553 and 570 with 256); from 75 on 609 (589)
   const bool half = tile == 128 && pairs <= 56 * a.E;
   const int bn = half ? 128 : 256, nf = (rows + bn - 1) / bn;
-  const dim3 grid((max_tiles * nf + 7) / 8 * 8);
+  const dim3 grid(((max_tiles * nf + 7) / 8 + (tile == 256 ? DIE_CUS / 2 : 0)) * 8);
   auto run = [&](auto kernel, int lds) {
     const hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     TORCH_CHECK(err == hipSuccess, "no LDS for expert tiles");
