@@ -1,4 +1,4 @@
-"""Products of a training pass (hip/gemm_ops.hip) against 64 bits: rows and features at the
+"""Products of training passes and prompts (hip/gemm_ops.hip) against 64 bits: rows and features at the
 edges of tiles, sums of one step, of whole ones and of what is left, cut into parts or not."""
 import pytest
 import torch
@@ -92,3 +92,27 @@ def test_linears_that_others_follow():
   with torch.autograd.forward_ad.dual_level():
     y = ops.linear(torch.autograd.forward_ad.make_dual(x.detach().float(), torch.ones_like(x).float()), w.detach().float())
     assert torch.autograd.forward_ad.unpack_dual(y).tangent is not None
+
+
+@pytest.mark.parametrize("M,N,K,form", [(257, 64, 64, "rows"), (300, 4096, 192, "batch"), (1000, 520, 2048, "turned"),
+                                        (512, 2048, 8192, "shifted"), (260, 72, 128, "weight shifted"), (333, 128, 64, "weight turned")])
+def test_linears_of_prompts(M, N, K, form):
+  from xotorch_amd import ops
+  from xotorch_amd.ops import train_ops
+  x, w = _random(1, M, K), _random(2, N, K)
+  if form == "batch":
+    x = x.view(M // 10, 10, K)
+  if form == "turned":
+    x = x.t().contiguous().t()
+  if form == "shifted":
+    x = torch.cat([x.new_zeros(1), x.flatten()])[1:].view(M, K)
+  if form == "weight shifted":
+    w = torch.cat([w.new_zeros(1), w.flatten()])[1:].view(N, K)
+  if form == "weight turned":
+    w = w.t().contiguous().t()
+  with torch.inference_mode():
+    assert train_ops.takes_product(x, w) and not train_ops.takes_product(x.reshape(-1, K)[:256], w)
+    y = ops.linear(x, w)
+    with torch.autocast("cuda", torch.float16):
+      assert not train_ops.takes_product(x, w)
+  assert y.shape == (*x.shape[:-1], N) and _near(y.reshape(-1, N), x.reshape(-1, K), w)

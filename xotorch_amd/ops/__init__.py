@@ -247,8 +247,11 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
   The decode hot path uses XotLinear.pack_decode() + skinny_gemm_packed (the
   hand-written CDNA4 weight-streaming MFMA kernel) instead; this is the
   library-GEMM path for prefill/training/CPU and unpacked weights. Training
-  passes have products of their own where these are faster (train_ops.linear).
+  passes, and prompts of some hundred tokens, have products of their own where these
+  are faster (train_ops.linear, product).
   """
+  if bias is None and train_ops.takes_product(x, weight):
+    return train_ops.product(x.reshape(-1, x.shape[-1]), weight).view(*x.shape[:-1], weight.shape[0])
   if bias is None and torch.is_grad_enabled() and train_ops.takes_linear(x, weight):
     return train_ops.linear(x, weight)
   return torch.nn.functional.linear(x, weight, bias)

@@ -1,4 +1,4 @@
-// Products of a training pass (bf16, fp32 sums) for some hundred to some thousand tokens:
+// Products of training passes and prompts (bf16, fp32 sums) of some hundred to some thousand tokens:
 //   forward           y = x W^T     [M, N] = [M, K] [N, K]^T
 //   input_gradient    dx = dy W     [M, K] = [M, N] [N, K]
 //   weight_gradient   dW = dy^T x   [N, K] = [M, N]^T [M, K]
