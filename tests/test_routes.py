@@ -182,3 +182,12 @@ def test_norms_with_weights_of_another_shape(shape):
   assert torch.equal(ops.rmsnorm(x, w, 1e-5), torch_ref.rmsnorm(x, w, 1e-5))
   for a, b in zip(ops.rmsnorm_residual(x, r, w, 1e-5), torch_ref.rmsnorm_residual(x, r, w, 1e-5)):
     assert torch.equal(a, b)
+
+
+def test_what_a_prompt_loads_is_built_for_it():
+  """A first run in a fresh checkout compiles what linears of prompts run on."""
+  from xotorch_amd.engine.trace import DECODER
+  from xotorch_amd.models.llama import XotLinear
+  from xotorch_amd.ops.build import EXTENSIONS
+  for needed in (DECODER, XotLinear.hip):
+    assert {"_hip_rows", "_hip_tile", "_hip_gemm"} <= set(needed) <= set(EXTENSIONS)

@@ -107,7 +107,7 @@ class TraceRunner:
     return torch.stack(rows).cpu() if rows else torch.empty(0, self.worker.cfg.vocab_size)
 
 
-DECODER = ("_hip_ops", "_hip_rows", "_hip_tile", "_hip_decode", "_hip_experts")  # of models that list none
+DECODER = ("_hip_ops", "_hip_rows", "_hip_tile", "_hip_gemm", "_hip_decode", "_hip_experts")  # of models that list none
 
 
 def build_extensions(model_dir: str):

@@ -92,7 +92,7 @@ class XotLinear(nn.Linear):
   by the copy, 1.07 by tiles). More rows, training and the CPU stay on hipBLASLt and
   aten. Storage and state dict are nn.Linear's."""
 
-  hip = ("_hip_rows", "_hip_tile")  # what a pass loads beside the operators
+  hip = ("_hip_rows", "_hip_tile", "_hip_gemm")  # what a pass loads beside the operators
   weight_packed: Optional[torch.Tensor]
 
   def __init__(self, *a, **kw):
