@@ -116,3 +116,54 @@ def test_linears_of_prompts(M, N, K, form):
     with torch.autocast("cuda", torch.float16):
       assert not train_ops.takes_product(x, w)
   assert y.shape == (*x.shape[:-1], N) and _near(y.reshape(-1, N), x.reshape(-1, K), w)
+
+
+@pytest.mark.parametrize("M,N,K,form", [(257, 32, 64, "rows"), (320, 288, 128, "batch"), (513, 4096, 192, "shifted"), (1000, 2080, 448, "turned"),
+                                        (2305, 1536, 64, "rows"), (769, 9728, 896, "rows"), (300, 512, 8192, "rows")])
+def test_gates_of_prompts(M, N, K, form):
+  """silu(x gate^T) (x up^T) against 64 bits: even shares of rows, tiles cut in two, features past a tile's."""
+  from xotorch_amd.ops import train_ops
+  x, w = _random(1, M, K), _random(2, N, K)
+  if form == "batch":
+    x = x.view(M // 10, 10, K)
+  if form == "turned":
+    x = x.t().contiguous().t()
+  if form == "shifted":
+    x = torch.cat([x.new_zeros(1), x.flatten()])[1:].view(M, K)
+  with torch.inference_mode():
+    assert train_ops.takes_gate(x, w) and not train_ops.takes_gate(x.reshape(-1, K)[:256], w) and not train_ops.takes_gate(x, w[:, :K - 8])
+    y = train_ops.gate_product(x, w)
+  assert y.shape == (*x.shape[:-1], N // 2)
+  rows = x.reshape(-1, K).double()
+  (gate, up), (by_gate, by_up) = (rows @ w.double().t()).chunk(2, 1), (rows.abs() @ w.double().abs().t() * (K + 8) * 2.0 ** -24).chunk(2, 1)
+  silu = gate * torch.sigmoid(gate)  # its slope is less than 1.1
+  bound = 1.1 * by_gate * (up.abs() + by_up) + silu.abs() * by_up + (silu * up).abs() * 2.0 ** -8
+  assert bool(((y.reshape(-1, N // 2).double() - silu * up).abs() <= bound + 1e-30).all())
+
+
+def test_gates_of_prompts_in_a_layer():
+  """One kernel where nobody waits for the product, with the module's hooks and its graph."""
+  from xotorch_amd.models.llama import MLP
+  from xotorch_amd.models.registry import builtin_config
+  from xotorch_amd.models import config_from_hf
+  m = MLP(config_from_hf(builtin_config("llama-3.2-1b"), "m"), 1024).to("cuda", torch.bfloat16)
+  x, seen = _random(3, 300, m.gate_up_proj.in_features), []
+  with torch.no_grad():
+    assert m.whole_gate(x) and not m.whole_gate(x[:256])
+    y = m(x)
+    hook = m.gate_up_proj.register_forward_hook(lambda *a: seen.append(1))
+    want = m(x)
+    hook.remove()
+    assert seen == [1]
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+      again = m(x)
+    for _ in range(3):
+      again.zero_()
+      g.replay()
+      assert torch.equal(again, y)
+  assert ((y - want).float().norm() / want.float().norm()).item() < 2.0 ** -7  # bf16 gate and up, then twice as many roundings
+  x.requires_grad_()
+  assert not m.whole_gate(x)
+  m(x).float().sum().backward()
+  assert x.grad is not None

@@ -338,7 +338,15 @@ class MLP(nn.Module):
                                                 split=lambda: self.act(gu(x)))) == "tile"
     return ops.tile_swiglu(x, gu.weight) if tile else self.act(gu(x))
 
+  def whole_gate(self, x) -> bool:
+    """Whether the gated activation of a prompt is one kernel (train_ops.takes_gate)."""
+    gu = self._modules["gate_up_proj"]
+    return (type(self) is MLP and type(gu) is XotLinear and not _watched(gu) and _own(gu, "bias") is None
+            and train_ops.takes_gate(x, _own(gu)) and os.getenv("XOT_FP8_PREFILL", "0") != "1")
+
   def forward(self, x):
+    if self.whole_gate(x):
+      return self.down_proj(train_ops.gate_product(x, self.gate_up_proj.weight))
     gu = self.gate_up_proj(x)
     dp = self.down_proj
     if (getattr(dp, "weight_packed", None) is not None and gu.is_cuda and gu.dtype == torch.bfloat16

@@ -265,9 +265,11 @@ DEVINL float gated(float g, float u, const Act& a) {
 
 // What a product is: of a pair's own row; of its token with gate and up weights
 // and the gated activation; of its token with one set of weights and the square
-// of what is positive; of its token with gate and up weights and silu (no limits).
-enum Product { PLAIN, GATED, RELU2, SWIGLU };
-constexpr bool has_gate(int kind) { return kind == GATED || kind == SWIGLU; }
+// of what is positive; of its token with gate and up weights and silu (no limits); the
+// same where there is but one expert, of all rows.
+enum Product { PLAIN, GATED, RELU2, SWIGLU, DENSE };
+constexpr bool has_gate(int kind) { return kind == GATED || kind == SWIGLU || kind == DENSE; }
+constexpr bool of_own_row(int kind) { return kind == PLAIN || kind == DENSE; }
 
 struct GroupArgs {
   int K, kp, F, E;  // valid and stored length of a weight row, output features, experts
@@ -278,7 +280,7 @@ struct GroupArgs {
 template <int KIND>
 DEVINL float activated(float by, float g, float u, const Act& a) {
   if (KIND == GATED) return gated(by * g, by * u, a);
-  if (KIND == SWIGLU) return siluf(by * g) * (by * u);
+  if (KIND == SWIGLU || KIND == DENSE) return siluf(by * g) * (by * u);
   g = by * g;
   if (KIND == RELU2) g = fmaxf(g, 0.f) * g;
   return g;
@@ -423,7 +425,7 @@ DEVINL void expert_tile(const bf16_t* __restrict__ x, const bf16_t* __restrict__
 #pragma unroll
   for (int i = 0; i < XL; ++i) {
     const int t = min(r0 + (wave * XL + i) * 8 + (lane >> 3), hi - 1);
-    xsrc[i] = x + (size_t)(KIND == PLAIN ? t : token[t]) * a.xs;
+    xsrc[i] = x + (size_t)(of_own_row(KIND) ? t : token[t]) * a.xs;
   }
   auto loadw = [&](auto number, int s, unsigned at) {
     constexpr int i = decltype(number)::value;
@@ -447,7 +449,7 @@ DEVINL void expert_tile(const bf16_t* __restrict__ x, const bf16_t* __restrict__
     const int t = r0 + (wt * C + j) * 16 + col;
     if (t >= hi) continue;
     bf16_t* dst = y + (size_t)t * a.ys;
-    const float by = KIND != PLAIN && by_row ? by_row[t] : 1.f;
+    const float by = !of_own_row(KIND) && by_row ? by_row[t] : 1.f;
     constexpr int N = TWO ? R / 2 : R;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
@@ -462,18 +464,18 @@ DEVINL void expert_tile(const bf16_t* __restrict__ x, const bf16_t* __restrict__
 
 constexpr int DIE_CUS = 32;  // of one of the eight dies
 
-// The router's tiles, of which there are as many as the last of `tiles` says
+// The router's tiles, of which there are as many as the last of `tiles` says; DENSE: max_tiles of rows_of_all rows
 template <int KIND, int BN, int TOK, typename W>
 __global__ __launch_bounds__(512) void expert_tile_kernel(
     const bf16_t* __restrict__ x, W w, const int* __restrict__ first,
     const int* __restrict__ token, const int2* __restrict__ tiles, const float* __restrict__ by_row,
-    bf16_t* __restrict__ y, int max_tiles, int group, GroupArgs a, Act act) {
+    bf16_t* __restrict__ y, int max_tiles, int group, int rows_of_all, GroupArgs a, Act act) {
   extern __shared__ __attribute__((aligned(16))) bf16_t buf[];
   // blocks go round the eight dies: a die has a run of them, in panels of `group` tiles
   // whose weight rows come one after the other, so that its L2 serves both operands
   constexpr bool TWO = has_gate(KIND);
   constexpr int WIDE = TWO ? BN / 2 : BN;
-  const int nf = (a.F + WIDE - 1) / WIDE, real = __builtin_amdgcn_readfirstlane(tiles[max_tiles].y);
+  const int nf = (a.F + WIDE - 1) / WIDE, real = KIND == DENSE ? max_tiles : __builtin_amdgcn_readfirstlane(tiles[max_tiles].y);
   const int die = blockIdx.x & 7, each = real * nf / 8, rest = real * nf % 8, all = each + (die < rest);
   // what no more than half of a die's 32 CUs would have left to do is cut in two: 384 blocks
   // of the down product of 2100 tokens 578 us, so 522 (with up to 128 tokens nothing, to 3% worse)
@@ -487,12 +489,16 @@ __global__ __launch_bounds__(512) void expert_tile_kernel(
   if (at >= all) return;
   const int n = die * each + min(die, rest) + at, per = group * nf, panel = n / per, in = n % per;
   const int wide = min(group, real - panel * group), m = panel * group + in % wide, fb = in / wide;
-  const int2 tile = tiles[m];
-  const int e = __builtin_amdgcn_readfirstlane(tile.x);
+  int e = 0, lo = 0, end = rows_of_all, nth = m;
+  if constexpr (KIND != DENSE) {
+    const int2 tile = tiles[m];
+    e = __builtin_amdgcn_readfirstlane(tile.x);
+    lo = __builtin_amdgcn_readfirstlane(first[e]), end = __builtin_amdgcn_readfirstlane(first[e + 1]);
+    nth = (__builtin_amdgcn_readfirstlane(tile.y) - lo) / TOK;
+  }
   // an expert's rows go over its tiles evenly, in steps of 64
-  const int lo = __builtin_amdgcn_readfirstlane(first[e]), end = __builtin_amdgcn_readfirstlane(first[e + 1]);
   const int of = (end - lo + TOK - 1) / TOK, share = ((end - lo + of - 1) / of + 63) / 64 * 64;
-  const int r0 = lo + (__builtin_amdgcn_readfirstlane(tile.y) - lo) / TOK * share, hi = min(end, r0 + share);
+  const int r0 = lo + nth * share, hi = min(end, r0 + share);
   const bf16_t* we = w.of(e, (size_t)(TWO ? 2 : 1) * a.F * a.kp);
   auto go = [&](auto rows) {
     if constexpr (CUT) {
@@ -645,7 +651,7 @@ static void launch_tiles(const W& w, const Tensor& x, const Tensor& token, const
     const hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     TORCH_CHECK(err == hipSuccess, "no LDS for expert tiles");
     hipLaunchKernelGGL(kernel, grid, dim3(512), lds, cur_stream(), P<bf16_t>(x), w, first.data_ptr<int>(),
-                       token.data_ptr<int>(), (const int2*)tiles.data_ptr<int>(), by_row, M<bf16_t>(y), max_tiles, group, a, act);
+                       token.data_ptr<int>(), (const int2*)tiles.data_ptr<int>(), by_row, M<bf16_t>(y), max_tiles, group, 0, a, act);
   };
 #define TILES(KIND, BN, TOK) run(expert_tile_kernel<KIND, BN, TOK, W>, expert_lds<BN, TOK>())
 #define TILES_OF(KIND) if (half) TILES(KIND, 128, 128); else if (tile == 256) TILES(KIND, 256, 256); else TILES(KIND, 256, 128)
@@ -762,6 +768,33 @@ OptT add_norm(Tensor y, OptT rows, OptT weight, Tensor x, OptT w_next, double mu
   TORCH_CHECK(false, "row of ", D, " elements is too long");
 }
 
+// silu of gate and up of all rows of x, bf16: w [2 F, K], gate rows first; K % 64 == 0. The
+// product bounds it; a library's product, with the activation's kernel behind it that reads
+// and writes what this one never stores, took, us: 320 tokens by [16384, 2048] 29 (24 so);
+// 700 by [28672, 4096] 160 (145); 3000 by [37888, 3584] 728 (591); 8192 by [17920, 1536] 452
+// (358). Whole rounds of large tiles are all a library needs: 8192 by [57344, 8192] 5168 (5390).
+Tensor gate_product(Tensor x, Tensor w) {
+  check_io(x, torch::kBFloat16);
+  check_io(w, torch::kBFloat16);
+  CHK(x.dim() == 2 && w.dim() == 2 && (((size_t)x.data_ptr() | (size_t)w.data_ptr()) & 15) == 0);
+  const int64_t rows = x.size(0), K = x.size(1), F_ = w.size(0) / 2;
+  CHK(rows >= 1 && rows <= 1 << 22 && K >= 64 && K <= 1 << 22 && K % 64 == 0 && w.size(1) == K);
+  CHK(w.size(0) >= 32 && w.size(0) <= 1 << 22 && w.size(0) % 32 == 0);
+  auto y = torch::empty({rows, F_}, x.options());
+  const int tiles = (int)((rows + 255) / 256), nf = (int)((F_ + 127) / 128);
+  // panels of 2, 4, 6 and 8 tiles, us: 1500 rows of 3584 by 37888 326, 320, 315, 312; 6001 by
+  // [28672, 4096] 1047, 1030, 1005, 1022; 3000 by [57344, 8192] 2114, 2058, 1988, 2022
+  const int group = 6;
+  auto kernel = expert_tile_kernel<DENSE, 256, 256, Stacked>;
+  constexpr int lds = expert_lds<256, 256>();
+  const hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  TORCH_CHECK(err == hipSuccess, "no LDS for gate and up");
+  hipLaunchKernelGGL(kernel, dim3(((tiles * nf + 7) / 8 + DIE_CUS / 2) * 8), dim3(512), lds, cur_stream(), P<bf16_t>(x),
+                     Stacked{P<bf16_t>(w)}, (const int*)nullptr, (const int*)nullptr, (const int2*)nullptr, (const float*)nullptr,
+                     M<bf16_t>(y), tiles, group, (int)rows, GroupArgs{(int)K, (int)K, (int)F_, 1, (int)K, (int)F_}, Act{});
+  return y;
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("route", &route, "router: sigmoid scores or a softmax over the chosen, group-limited top-k, shared experts; rows of all pairs",
         py::arg("x"), py::arg("w"), py::arg("correction"), py::arg("top"), py::arg("groups"), py::arg("keep"),
@@ -774,5 +807,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.attr("PLAIN") = (int)PLAIN;
   m.attr("GATED") = (int)GATED;
   m.attr("RELU2") = (int)RELU2;
+  m.def("gate_product", &gate_product, "silu of gate and up of all rows, by the same tiles");
   m.def("add_norm", &add_norm, "stream += mult * (output or weighted expert rows); norm of the stream");
 }
