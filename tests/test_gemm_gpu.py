@@ -95,7 +95,8 @@ def test_linears_that_others_follow():
 
 
 @pytest.mark.parametrize("M,N,K,form", [(257, 64, 64, "rows"), (300, 4096, 192, "batch"), (1000, 520, 2048, "turned"),
-                                        (512, 2048, 8192, "shifted"), (260, 72, 128, "weight shifted"), (333, 128, 64, "weight turned")])
+                                        (512, 2048, 8192, "shifted"), (260, 72, 128, "weight shifted"), (333, 128, 64, "weight turned"),
+                                        (512, 8192, 12352, "rows"), (2000, 128, 16448, "rows"), (1000, 6144, 12352, "rows")])
 def test_linears_of_prompts(M, N, K, form):
   from xotorch_amd import ops
   from xotorch_amd.ops import train_ops

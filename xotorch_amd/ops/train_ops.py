@@ -114,8 +114,16 @@ def _again(f: Callable, inputs: Sequence[torch.Tensor], needs: Sequence[bool], g
 
 def forward_wins(M: int, N: int, K: int) -> bool:
   """x W^T: 0.40 to 1.11 (0.73 on average) for narrow results of up to 1000 tokens; wider ones
-  and more tokens 0.95 to 1.40."""
-  return M <= 1000 and N <= 4096 and K % 64 == 0 and N % 4 == 0
+  and more tokens 0.95 to 1.40, but for long sums, whose library tiles fill the chip badly
+  (257 to 2000 tokens by 1536 to 12288 features of 13824 to 29568): where the result is small
+  0.46 to 1.05 (0.69), of up to 6144 features 0.65 to 0.95, narrow ones of longest sums 0.39 to
+  0.87. Above these lines 0.6 to 1.5 from one size to the next."""
+  if K % 64 or N % 4:
+    return False
+  if M <= 1000 and N <= 4096:
+    return True
+  small = M * N <= 4_300_000 and N <= 12288 or M <= 1000 and N <= 6144
+  return M > 256 and (K > 12288 and small or K > 16384 and N <= 4096 and M <= 2000)
 
 
 def input_wins(M: int, N: int, K: int) -> bool:
