@@ -94,6 +94,17 @@ def test_linears_that_others_follow():
     assert torch.autograd.forward_ad.unpack_dual(y).tangent is not None
 
 
+@pytest.mark.parametrize("M", [70, 300])
+def test_many_gradients_at_once(M):
+  from xotorch_amd import ops
+  from xotorch_amd.ops import train_ops
+  x, w, dy = _random(1, M, 192).requires_grad_(), _random(2, 128, 192).requires_grad_(), _random(3, 2, M, 128)
+  assert train_ops.takes_linear(x, w)
+  dx, dw = torch.autograd.grad(ops.linear(x, w), (x, w), dy, is_grads_batched=True)
+  for i in range(2):
+    assert _near(dx[i], dy[i], w.detach().t()) and _near(dw[i], dy[i].t(), x.detach().t())
+
+
 @pytest.mark.parametrize("M,N,K,form", [(257, 64, 64, "rows"), (300, 4096, 192, "batch"), (1000, 520, 2048, "turned"),
                                         (512, 2048, 8192, "shifted"), (260, 72, 128, "weight shifted"), (333, 128, 64, "weight turned"),
                                         (512, 8192, 12352, "rows"), (2000, 128, 16448, "rows"), (1000, 6144, 12352, "rows")])

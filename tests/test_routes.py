@@ -191,3 +191,11 @@ def test_what_a_prompt_loads_is_built_for_it():
   from xotorch_amd.ops.build import EXTENSIONS
   for needed in (DECODER, XotLinear.hip):
     assert {"_hip_rows", "_hip_tile", "_hip_gemm"} <= set(needed) <= set(EXTENSIONS)
+
+
+def test_products_of_more_rows_than_kernels_index():
+  from xotorch_amd.ops import train_ops
+  most = 1 << 22
+  assert train_ops.forward_wins(64, 64, most) and train_ops.input_wins(64, most, 64) and train_ops.weight_wins(most, 64, 64)
+  for more in (most + 8, most + 64):
+    assert not train_ops.forward_wins(300, 4, more) and not train_ops.input_wins(64, more, 64) and not train_ops.weight_wins(more, 64, 64)

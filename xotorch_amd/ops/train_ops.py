@@ -110,7 +110,9 @@ def _again(f: Callable, inputs: Sequence[torch.Tensor], needs: Sequence[bool], g
 
 # Where the products of hip/gemm_ops.hip are faster than the library's, by what they took of
 # its time (40 to 4096 tokens, the linears of 0.5B, 1B, 8B and 70B decoders; M tokens through
-# a weight [N, K]).
+# a weight [N, K]). What the kernels don't index is the library's.
+_MOST = 1 << 22  # rows, features
+
 
 def forward_wins(M: int, N: int, K: int) -> bool:
   """x W^T: 0.40 to 1.11 (0.73 on average) for narrow results of up to 1000 tokens; wider ones
@@ -118,7 +120,7 @@ def forward_wins(M: int, N: int, K: int) -> bool:
   (257 to 2000 tokens by 1536 to 12288 features of 13824 to 29568): where the result is small
   0.46 to 1.05 (0.69), of up to 6144 features 0.65 to 0.95, narrow ones of longest sums 0.39 to
   0.87. Above these lines 0.6 to 1.5 from one size to the next."""
-  if K % 64 or N % 4:
+  if K % 64 or N % 4 or max(M, N, K) > _MOST:
     return False
   if M <= 1000 and N <= 4096:
     return True
@@ -130,16 +132,13 @@ def input_wins(M: int, N: int, K: int) -> bool:
   """dy W, a sum over N: 0.25 to 1.07 (0.66 on average) where that is no shorter than the result
   is wide, or for few tokens; with more tokens 0.46 to 0.95 where it is much longer and 0.92 to
   1.26 else. Shorter sums: 0.85 to 1.27 from 333 tokens on."""
-  return N % 64 == 0 and K % 8 == 0 and (M <= 1400 and (N >= K or M <= 300) or (M <= 3000 and N >= 8 * K))
+  return N % 64 == 0 and K % 8 == 0 and max(M, N, K) <= _MOST and (M <= 1400 and (N >= K or M <= 300) or (M <= 3000 and N >= 8 * K))
 
 
 def weight_wins(M: int, N: int, K: int) -> bool:
   """dy^T x, a sum over tokens: 0.81 to 1.05 (0.89 on average) from 600 tokens on, and 0.23 to
   0.8 for small weights; large weights and 100 to 512 tokens 0.85 to 1.16."""
-  return M >= 64 and N % 8 == 0 and K % 8 == 0 and (M >= 600 or N * K <= 7_000_000)
-
-
-_MOST = 1 << 22  # rows, features
+  return M >= 64 and N % 8 == 0 and K % 8 == 0 and max(M, N, K) <= _MOST and (M >= 600 or N * K <= 7_000_000)
 
 
 def product(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
@@ -203,7 +202,7 @@ def takes_linear(x: torch.Tensor, weight: torch.Tensor) -> bool:
   if not (x.is_cuda and torch.is_grad_enabled() and weight.dim() == 2 and 0 < x.numel() and x.shape[-1] == weight.shape[1]):
     return False
   (N, K), M = weight.shape, x.numel() // weight.shape[1]
-  return (max(M, N, K) <= _MOST and (forward_wins(M, N, K) or input_wins(M, N, K) or weight_wins(M, N, K)) and K % 8 == 0
+  return ((forward_wins(M, N, K) or input_wins(M, N, K) or weight_wins(M, N, K)) and K % 8 == 0
           and x.dtype == weight.dtype == torch.bfloat16 and (x.requires_grad or weight.requires_grad) and plain(x, weight)
           and not torch._C._is_any_autocast_enabled() and not _missing())
 
@@ -220,6 +219,9 @@ class _Linear(torch.autograd.Function):
     if torch.is_grad_enabled():
       return tuple(_again(torch.nn.functional.linear, (x, weight), ctx.needs_input_grad, (dy,)))
     rows = dy.reshape(-1, dy.shape[-1])
+    if not plain(dy, x, weight):  # many gradients at once
+      dx = (rows @ weight).view(x.shape) if ctx.needs_input_grad[0] else None
+      return dx, rows.t() @ x.reshape(-1, x.shape[-1]) if ctx.needs_input_grad[1] else None
     dx = input_gradient(rows, weight).view(x.shape) if ctx.needs_input_grad[0] else None
     return dx, weight_gradient(rows, x.reshape(-1, x.shape[-1])) if ctx.needs_input_grad[1] else None
 
