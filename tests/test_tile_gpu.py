@@ -85,7 +85,7 @@ def test_gated_products_of_one_round(m, N, K):
   assert bool(((y - act * u).abs() <= bound + 1e-30).all())
 
 
-@pytest.mark.parametrize("m,D,H,I", [(3, 64, 128, 96), (45, 2048, 2048, 8192), (200, 320, 192, 512)])
+@pytest.mark.parametrize("m,D,H,I", [(3, 64, 128, 192), (45, 2048, 2048, 8192), (200, 320, 192, 512)])
 def test_rest_of_a_layer_is_its_parts(m, D, H, I):
   from xotorch_amd import ops
   g = torch.Generator(device="cuda").manual_seed(m)

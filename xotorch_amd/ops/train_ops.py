@@ -219,7 +219,7 @@ class _Linear(torch.autograd.Function):
     if torch.is_grad_enabled():
       return tuple(_again(torch.nn.functional.linear, (x, weight), ctx.needs_input_grad, (dy,)))
     rows = dy.reshape(-1, dy.shape[-1])
-    if not plain(dy, x, weight):  # many gradients at once
+    if not torch._C._has_storage(dy):  # many gradients at once, wrapped
       dx = (rows @ weight).view(x.shape) if ctx.needs_input_grad[0] else None
       return dx, rows.t() @ x.reshape(-1, x.shape[-1]) if ctx.needs_input_grad[1] else None
     dx = input_gradient(rows, weight).view(x.shape) if ctx.needs_input_grad[0] else None
