@@ -158,7 +158,9 @@ def test_positions_as_torch_indexes(hd):
   assert not train_ops.takes_heads(_rand(1, T + 1, (H + 2 * KVH) * hd).requires_grad_(True), cos, sin, short, hd)
 
 
-@pytest.mark.parametrize("rows,K,N,rank,bias", [(1, 8, 24, 1, False), (5, 64, 40, 3, True), (130, 256, 520, 16, False)])
+@pytest.mark.parametrize("rows,K,N,rank,bias", [(1, 8, 24, 1, False), (5, 64, 40, 3, True), (130, 256, 520, 16, False),
+                                                 (1, 256, 512, 1, False), (31, 512, 256, 4, True), (64, 768, 1280, 8, False),
+                                                 (33, 256, 768, 11, True), (650, 2048, 256, 16, False)])
 def test_adapted_linear(rows, K, N, rank, bias):
   from xotorch_amd.models.llama import XotLinear
   from xotorch_amd.train.lora import LoRALinear
@@ -170,6 +172,7 @@ def test_adapted_linear(rows, K, N, rank, bias):
   x, dy = _rand(2, rows, K).requires_grad_(True), _rand(2, rows, N, seed=1)
   y = lin(x)
   assert "_Adapted" in type(y.grad_fn).__name__ and y.shape == dy.shape
+  assert ("_AdaptedRows" in type(y.grad_fn).__name__) == (K % 256 == N % 256 == 0)
   y.backward(dy)
   own = [y.detach(), x.grad, lin.lora_a.grad, lin.lora_b.grad]
   hook = base.register_forward_hook(lambda *_: None)  # somebody looks on: by separate operators
@@ -193,6 +196,37 @@ def test_adapted_linear(rows, K, N, rank, bias):
     assert (o.double().view(r.shape) - r).norm() <= 1.1 * (o2.double().view(r.shape) - r).norm() + 1e-3 * r.norm()
   twice = torch.autograd.grad(lin(x), x, dy, create_graph=True)[0]
   twice.float().square().sum().backward()
+  both = torch.autograd.grad(lin(x), (x, lin.lora_a, lin.lora_b), torch.stack([dy, dy]), is_grads_batched=True)
+  for o, r, z in zip(both, ref[1:], size[1:]):
+    assert bool(((o[1].double().view(r.shape) - r).abs() <= r.abs() * 2 * STEP + z * STEP).all())
+
+
+@pytest.mark.parametrize("rank", [1, 5, 16])
+@pytest.mark.parametrize("M", [1, 63, 64, 65, 129, 1500])
+def test_narrow_sums(M, rank):
+  """Rows and columns at the edges of steps; what lies past a tensor's rows counts nowhere."""
+  from xotorch_amd.ops import train_ops
+  hip, N = train_ops._hip_lora(), 768
+  t, w, c = _rand(M, N), _rand(N, rank, seed=2).float() * 1.001, _rand(16, -(-M // 64) * 64, seed=3)
+  c[rank:], c[:, M:] = 0, 0
+  wt = w.t().contiguous()
+  low, lowt, down = hip.sums(t, wt, 0.5, c, rank, 3.0, False)
+  again, _ = hip.sums(t, wt, 0.5, None, rank, 1.0, False)
+  turned, = hip.sums(t, None, 1.0, c, rank, 3.0, True)
+  assert torch.equal(low, again) and torch.equal(turned.t(), down) and down.shape == (N, rank)
+  td, wd, cd = t.double(), w.to(BF).double(), c[:rank, :M].double()
+  rows, cols = 0.5 * td @ wd, 3.0 * td.t() @ cd.t()
+  assert bool(((low[:, :rank].double() - rows).abs() <= (td.abs() @ wd.abs()) * (N + 8) * 2.0 ** -25).all()) and not low[:, rank:].any()
+  assert bool(((down.double() - cols).abs() <= (td.abs().t() @ cd.abs().t()) * (M + 8) * 3 * 2.0 ** -24).all())
+  assert torch.equal(lowt[:rank, :M], low[:, :rank].t().to(BF)) and not lowt[rank:].any() and not lowt[:, M:].any()
+  out, by = _rand(M, N, seed=4), low[:, :rank].double() @ (2.0 * w.double().t())
+  want = out.double() + by
+  hip.add(out, low, wt, 2.0)
+  slack = (low[:, :rank].double().abs() @ (2.0 * w.double().abs().t()) + want.abs()) * (rank + 4) * 2.0 ** -24
+  assert bool(((out.double() - want).abs() <= slack + want.abs() * 2.0 ** -8).all())
+  t[M - 1, 5] = float("inf")
+  low, _, down = hip.sums(t, wt, 1.0, c, rank, 1.0, False)
+  assert low[:M - 1].isfinite().all() and torch.equal(down.isnan(), (t.float().t() @ c[:rank, :M].float().t()).isnan())
 
 
 def test_second_derivatives_forward_mode_and_transforms():

@@ -22,6 +22,7 @@ EXTENSIONS = {
   "_hip_tile": PKG_DIR / "hip" / "tile_ops.hip",
   "_hip_attn_train": PKG_DIR / "hip" / "attn_train.hip",
   "_hip_gemm": PKG_DIR / "hip" / "gemm_ops.hip",
+  "_hip_lora": PKG_DIR / "hip" / "lora_ops.hip",
   "_hip_train": PKG_DIR / "hip" / "train_ops.hip",
   "_hip_decode": PKG_DIR / "hip" / "decode_attn.hip",
   "_hip_mixers": PKG_DIR / "hip" / "mixer_ops.hip",

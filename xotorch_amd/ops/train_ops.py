@@ -12,7 +12,7 @@ import torch
 
 from xotorch_amd.ops import torch_ref
 
-_ext = _attn = _gemm = _experts = None
+_ext = _attn = _gemm = _experts = _lora = None
 OWN = (torch.Tensor, torch.nn.Parameter)
 # looked up once: a step of a small model asks some thirty times
 _is_compiling, _is_tracing, _forward_ad = torch.compiler.is_compiling, torch._C._is_tracing, torch.autograd.forward_ad
@@ -55,11 +55,19 @@ def _hip_experts():
   return _experts
 
 
+def _hip_lora():
+  global _lora
+  if _lora is None:
+    import importlib
+    _lora = importlib.import_module("xotorch_amd.ops._hip_lora")
+  return _lora
+
+
 def _missing() -> bool:
   """Whether the kernels are not built and torch's operators are asked for then."""
-  if (_ext is None or _attn is None or _gemm is None or _experts is None) and os.getenv("XOT_ALLOW_EAGER", "0") == "1":
+  if (_ext is None or _attn is None or None in (_gemm, _experts, _lora)) and os.getenv("XOT_ALLOW_EAGER", "0") == "1":
     try:
-      _hip(), _hip_attn(), _hip_gemm(), _hip_experts()
+      _hip(), _hip_attn(), _hip_gemm(), _hip_experts(), _hip_lora()
     except ImportError:
       return True
   return False
@@ -89,6 +97,11 @@ def takes(x: torch.Tensor, *others: torch.Tensor) -> bool:
     return False
   return (any(t.requires_grad for t in (x, *others)) and all(t.dtype == torch.bfloat16 for t in (x, *others))
           and plain(x, *others) and not _missing())
+
+
+def own_memory(t: torch.Tensor) -> bool:
+  """Not many gradients at once, which come to a backward pass wrapped."""
+  return torch._C._has_storage(t)
 
 
 def _rows(t: torch.Tensor) -> torch.Tensor:
@@ -185,14 +198,14 @@ def gate_product(x: torch.Tensor, gate_up: torch.Tensor) -> torch.Tensor:
 def input_gradient(dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
   """dy W of rows [M, N]"""
   M, (N, K) = dy.shape[0], weight.shape
-  if input_wins(M, N, K) and weight.is_contiguous() and weight.data_ptr() % 16 == 0:
+  if input_wins(M, N, K) and own_memory(dy) and weight.is_contiguous() and weight.data_ptr() % 16 == 0:
     return _hip_gemm().input_gradient(_rows(dy), weight)
   return dy @ weight
 
 
 def weight_gradient(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
   """dy^T x of rows [M, N] and [M, K]"""
-  if weight_wins(dy.shape[0], dy.shape[1], x.shape[1]):
+  if weight_wins(dy.shape[0], dy.shape[1], x.shape[1]) and own_memory(dy):
     return _hip_gemm().weight_gradient(_rows(dy), _rows(x))
   return dy.t() @ x
 
@@ -219,9 +232,6 @@ class _Linear(torch.autograd.Function):
     if torch.is_grad_enabled():
       return tuple(_again(torch.nn.functional.linear, (x, weight), ctx.needs_input_grad, (dy,)))
     rows = dy.reshape(-1, dy.shape[-1])
-    if not torch._C._has_storage(dy):  # many gradients at once, wrapped
-      dx = (rows @ weight).view(x.shape) if ctx.needs_input_grad[0] else None
-      return dx, rows.t() @ x.reshape(-1, x.shape[-1]) if ctx.needs_input_grad[1] else None
     dx = input_gradient(rows, weight).view(x.shape) if ctx.needs_input_grad[0] else None
     return dx, weight_gradient(rows, x.reshape(-1, x.shape[-1])) if ctx.needs_input_grad[1] else None
 

@@ -54,6 +54,43 @@ class _Adapted(torch.autograd.Function):
             _scaled(dy.t(), low, ctx.scaling) if need_b else None, None)
 
 
+class _AdaptedRows(torch.autograd.Function):
+  """The same with fp32 adapters A and B^T by hip/lora_ops.hip: a gradient is read once for both of its
+  narrow sums, nothing narrow is rounded but as an operand of the matrix cores."""
+
+  @staticmethod
+  def forward(ctx, x, weight, bias, a, bt, scaling):
+    hip, rows = train_ops._hip_lora(), train_ops._rows(x.reshape(-1, x.shape[-1]))
+    out = F.linear(rows, weight, bias) if bias is not None else train_ops.product(rows, weight)
+    low, columns = hip.sums(rows, a, 1.0, None, a.shape[0], 1.0, False)
+    hip.add(out, low, bt, scaling)
+    ctx.save_for_backward(x, weight, bias, a, bt, columns)
+    ctx.scaling = scaling
+    return out.view(*x.shape[:-1], weight.shape[0])
+
+  @staticmethod
+  def backward(ctx, dy):
+    x, weight, bias, a, bt, columns = ctx.saved_tensors
+    need_x, _, _, need_a, need_b, _ = ctx.needs_input_grad
+    if torch.is_grad_enabled() or not train_ops.own_memory(dy):
+      def whole(x, a, bt):
+        return F.linear(x, weight, bias) + (x @ a.to(x.dtype).t() @ bt.to(x.dtype)) * ctx.scaling
+      dx, da, db = train_ops._again(whole, (x, a, bt), (need_x, need_a, need_b), (dy,))
+      return dx, None, None, da, db, None
+    hip, rank = train_ops._hip_lora(), a.shape[0]
+    dy, dx, da, db = train_ops._rows(dy.reshape(-1, dy.shape[-1])), None, None, None
+    found = hip.sums(dy, bt if need_x or need_a else None, ctx.scaling, columns if need_b else None, rank, ctx.scaling, False)
+    if need_b:
+      db = found.pop().t()  # lies as B does
+    if need_x:
+      dx = train_ops.input_gradient(dy, weight)
+      hip.add(dx, found[0], a, 1.0)
+      dx = dx.view(x.shape)
+    if need_a:
+      da, = hip.sums(train_ops._rows(x.reshape(-1, x.shape[-1])), None, 1.0, found[1], rank, 1.0, True)
+    return dx, None, None, da, db, None
+
+
 class LoRALinear(nn.Module):
   def __init__(self, base: nn.Linear, rank: int = 8, alpha: float = 16.0, dropout: float = 0.0):
     super().__init__()
@@ -88,8 +125,19 @@ class LoRALinear(nn.Module):
             and any(t.requires_grad for t in (x, self.lora_a, self.lora_b))
             and not torch.is_autocast_enabled("cuda") and train_ops.plain(x, *held, self.lora_a, self.lora_b))
 
+  def _by_rows(self, x) -> bool:
+    """Whether these are for the kernels of narrow sums (_takes holds)."""
+    a, b = self.lora_a, self.lora_b
+    return (a.dtype == b.dtype == torch.float32 and a.dim() == b.dim() == 2 and 1 <= a.shape[0] == b.shape[1] <= 16
+            and x.shape[-1] == a.shape[1] == self.base.weight.shape[1] and b.shape[0] == self.base.weight.shape[0]
+            and a.shape[1] % 256 == 0 and b.shape[0] % 256 == 0
+            and max(x.numel() // x.shape[-1], a.shape[1], b.shape[0]) <= train_ops._MOST and not train_ops._missing())
+
   def forward(self, x):
     if not self.merged and self._takes(x):
+      if self._by_rows(x):  # copies: the adapters may change between the passes
+        return _AdaptedRows.apply(x, self.base.weight, self.base.bias, self.lora_a.clone(memory_format=torch.contiguous_format),
+                                  self.lora_b.t().clone(memory_format=torch.contiguous_format), self.scaling)
       return _Adapted.apply(x, self.base.weight, self.base.bias, self.lora_a.to(x.dtype), self.lora_b.to(x.dtype), self.scaling)
     out = self.base(x)
     if not self.merged:
