@@ -26,7 +26,7 @@ struct TileArgs {
   const bf16_t *x, *w, *bias;
   void* y;  // bf16 [m, N], or fp32 [splits, m, N]
   int m, N, K, splits;  // N: output features
-  bool turned, runs;    // see turns, run_tile
+  bool turned, runs, dense;  // see turns, run_tile, launch_tile
   int whole, more, inv;  // steps of 64 of a part, in all parts `more` besides; 65536 / splits, and one more
 };
 
@@ -167,8 +167,11 @@ __global__ __launch_bounds__((TileShape<BN, BM, BUFS>::WAVES * 64)) void tile_ke
     if (n >= (units >> 3) + (die < rest)) return;
     split = (die * (units >> 3) + min(die, rest) + n) / tiles;
     tile = die * (units >> 3) + min(die, rest) + n - split * tiles;
+  } else if (a.dense) {
+    split = (at * 8 + die) / tiles;
+    tile = at * 8 + die - split * tiles;
   }
-  if (tile >= tiles) return;
+  if (tile >= tiles || split >= a.splits) return;
   const int s0 = part_at(a, split), s1 = part_at(a, split + 1), m0 = mt * BM;
   const bf16_t *wsrc[Sh::WL], *xsrc[Sh::XL];
   const int sub = lane >> 3;
@@ -361,8 +364,12 @@ __global__ __launch_bounds__(THREADS) void add_norm_kernel(const float* __restri
 // ===========================================================================
 // host side
 // ===========================================================================
+// Parts of tiles that don't go round the eight dies evenly are numbered through, at a division's
+// cost: blocks without work between the others keep CUs from them, which then have two. us,
+// parts of the grid and numbered through: [4608, 3584] in 36 tiles and 7 parts, m 20 10.7, 8.2;
+// m 48 12.5, 9.3
 template <int BN, int BM, int BUFS, int END>
-static void launch_tile(const TileArgs& a) {
+static void launch_tile(TileArgs a) {
   typedef TileShape<BN, BM, BUFS> Sh;
   if (Sh::LDS > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute((const void*)tile_kernel<BN, BM, BUFS, END>,
@@ -371,7 +378,9 @@ static void launch_tile(const TileArgs& a) {
   }
   const int per = END == GATED ? BN / 2 : BN;
   const int tiles = (a.N + per - 1) / per, mts = (a.m + BM - 1) / BM;
-  hipLaunchKernelGGL((tile_kernel<BN, BM, BUFS, END>), dim3((tiles + 7) / 8 * 8 * mts, a.splits), dim3(Sh::WAVES * 64), Sh::LDS, cur_stream(), a);
+  a.dense = !a.runs && a.splits > 1 && tiles % 8;
+  const dim3 grid = a.dense ? dim3((tiles * a.splits + 7) / 8 * 8 * mts) : dim3((tiles + 7) / 8 * 8 * mts, a.splits);
+  hipLaunchKernelGGL((tile_kernel<BN, BM, BUFS, END>), grid, dim3(Sh::WAVES * 64), Sh::LDS, cur_stream(), a);
 }
 
 // Tile and depth by the rows of x and by the blocks that 128 weight rows make. us at
