@@ -193,6 +193,30 @@ def test_what_a_prompt_loads_is_built_for_it():
     assert {"_hip_rows", "_hip_tile", "_hip_gemm"} <= set(needed) <= set(EXTENSIONS)
 
 
+@pytest.mark.parametrize("needs", [(True, False), (False, True), (True, True)])
+def test_a_linear_holds_what_its_gradients_read(needs):
+  """Rows for the weight's gradient, the weight for that of the rows, as torch's operator; what is
+  not held may change between the passes."""
+  from xotorch_amd.ops import train_ops
+  x, w, dy = (torch.randn(*s).to(BF) for s in ((2, 3, 40), (24, 40), (2, 3, 24)))
+  x, w = x.requires_grad_(needs[0]), w.requires_grad_(needs[1])
+  held, leaves = [], [t for t in (x, w) if t.requires_grad]
+  with torch.autograd.graph.saved_tensors_hooks(lambda t: held.append(t.shape) or t, lambda t: t):
+    y = train_ops.linear(x, w)
+  assert sorted(held) == sorted(t.shape for t, other in ((x, w), (w, x)) if other.requires_grad)
+  want = [(dy.flatten(0, 1) @ w.detach()).view_as(x), dy.flatten(0, 1).t() @ x.detach().flatten(0, 1)]
+  first = torch.autograd.grad(y, leaves, dy.requires_grad_(), create_graph=True)
+  assert all(torch.equal(a, b) for a, b in zip(first, [g for g, n in zip(want, needs) if n]))
+  assert torch.autograd.grad(first[0].float().sum(), dy)[0].shape == dy.shape
+  y = train_ops.linear(x, w)
+  with torch.no_grad():
+    for t, other in ((x, w), (w, x)):
+      if not other.requires_grad:
+        t.zero_()
+  for a, b in zip(torch.autograd.grad(y, leaves, dy.detach()), first):
+    assert torch.equal(a, b)
+
+
 def test_products_of_more_rows_than_kernels_index():
   from xotorch_amd.ops import train_ops
   most = 1 << 22

@@ -104,6 +104,12 @@ def own_memory(t: torch.Tensor) -> bool:
   return torch._C._has_storage(t)
 
 
+def once(dy: torch.Tensor) -> bool:
+  """Whether a backward pass with this gradient is one that nobody differentiates again, and
+  may go by kernels."""
+  return not torch.is_grad_enabled() and own_memory(dy)
+
+
 def _rows(t: torch.Tensor) -> torch.Tensor:
   """Contiguous, with rows on 16 bytes."""
   t = t.contiguous()
@@ -198,14 +204,14 @@ def gate_product(x: torch.Tensor, gate_up: torch.Tensor) -> torch.Tensor:
 def input_gradient(dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
   """dy W of rows [M, N]"""
   M, (N, K) = dy.shape[0], weight.shape
-  if input_wins(M, N, K) and own_memory(dy) and weight.is_contiguous() and weight.data_ptr() % 16 == 0:
+  if input_wins(M, N, K) and once(dy) and weight.is_contiguous() and weight.data_ptr() % 16 == 0:
     return _hip_gemm().input_gradient(_rows(dy), weight)
   return dy @ weight
 
 
 def weight_gradient(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
   """dy^T x of rows [M, N] and [M, K]"""
-  if weight_wins(dy.shape[0], dy.shape[1], x.shape[1]) and own_memory(dy):
+  if weight_wins(dy.shape[0], dy.shape[1], x.shape[1]) and once(dy):
     return _hip_gemm().weight_gradient(_rows(dy), _rows(x))
   return dy.t() @ x
 
@@ -221,18 +227,21 @@ def takes_linear(x: torch.Tensor, weight: torch.Tensor) -> bool:
 
 
 class _Linear(torch.autograd.Function):
+  """As torch's operator, holds only what its gradients read: a frozen weight's input lives no
+  longer than the forward pass."""
+
   @staticmethod
   def forward(ctx, x, weight):
-    ctx.save_for_backward(x, weight)
+    need_x, need_weight = ctx.needs_input_grad
+    ctx.save_for_backward(x if need_weight else None, weight if need_x else None)
+    ctx.shape = x.shape
     return product(x.reshape(-1, x.shape[-1]), weight).view(*x.shape[:-1], weight.shape[0])
 
   @staticmethod
   def backward(ctx, dy):
     x, weight = ctx.saved_tensors
-    if torch.is_grad_enabled():
-      return tuple(_again(torch.nn.functional.linear, (x, weight), ctx.needs_input_grad, (dy,)))
     rows = dy.reshape(-1, dy.shape[-1])
-    dx = input_gradient(rows, weight).view(x.shape) if ctx.needs_input_grad[0] else None
+    dx = input_gradient(rows, weight).view(ctx.shape) if ctx.needs_input_grad[0] else None
     return dx, weight_gradient(rows, x.reshape(-1, x.shape[-1])) if ctx.needs_input_grad[1] else None
 
 
