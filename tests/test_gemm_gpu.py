@@ -94,6 +94,37 @@ def test_linears_that_others_follow():
     assert torch.autograd.forward_ad.unpack_dual(y).tangent is not None
 
 
+@pytest.mark.parametrize("rank", [0, 8, 20])
+def test_backward_passes_that_others_follow(rank):
+  """A dispatch mode around the backward pass alone sees its products."""
+  from torch.utils._python_dispatch import TorchDispatchMode
+  from xotorch_amd import ops
+  from xotorch_amd.models.llama import XotLinear
+  from xotorch_amd.train.lora import LoRALinear
+  seen = []
+
+  class Recorder(TorchDispatchMode):
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+      seen.append(func.overloadpacket)
+      return func(*args, **(kwargs or {}))
+
+  x, w, dy = _random(1, 300, 256).requires_grad_(), _random(2, 512, 256), _random(3, 300, 512)
+  if rank:
+    lin = LoRALinear(XotLinear(256, 512, bias=False).to("cuda", torch.bfloat16), rank=rank)
+    lin.base.weight.data.copy_(w)
+    y, leaves = lin(x), (x, lin.lora_a, lin.lora_b)
+  else:
+    w.requires_grad_()
+    y, leaves = ops.linear(x, w), (x, w)
+  with Recorder():
+    found = torch.autograd.grad(y, leaves, dy)
+  products = [f for f in seen if f in (torch.ops.aten.mm, torch.ops.aten.addmm, torch.ops.aten.addmm_)]
+  assert len(products) >= (4 if rank else 2)
+  assert _near(found[0], dy, w.detach().t())  # B is zero
+  if not rank:
+    assert _near(found[1], dy.t(), x.detach().t())
+
+
 @pytest.mark.parametrize("M", [70, 300])
 def test_many_gradients_at_once(M):
   from xotorch_amd import ops

@@ -99,15 +99,11 @@ def takes(x: torch.Tensor, *others: torch.Tensor) -> bool:
           and plain(x, *others) and not _missing())
 
 
-def own_memory(t: torch.Tensor) -> bool:
-  """Not many gradients at once, which come to a backward pass wrapped."""
-  return torch._C._has_storage(t)
-
-
-def once(dy: torch.Tensor) -> bool:
-  """Whether a backward pass with this gradient is one that nobody differentiates again, and
-  may go by kernels."""
-  return not torch.is_grad_enabled() and own_memory(dy)
+def once(dy: torch.Tensor, *others: torch.Tensor) -> bool:
+  """Whether kernels may take a backward pass with this gradient: nobody differentiates it
+  again or follows its operators (which need not be those that followed the forward pass),
+  and it is not many gradients at once, which come wrapped and without memory."""
+  return not torch.is_grad_enabled() and torch._C._has_storage(dy) and plain(dy, *others)
 
 
 def _rows(t: torch.Tensor) -> torch.Tensor:
@@ -204,14 +200,14 @@ def gate_product(x: torch.Tensor, gate_up: torch.Tensor) -> torch.Tensor:
 def input_gradient(dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
   """dy W of rows [M, N]"""
   M, (N, K) = dy.shape[0], weight.shape
-  if input_wins(M, N, K) and once(dy) and weight.is_contiguous() and weight.data_ptr() % 16 == 0:
+  if input_wins(M, N, K) and once(dy, weight) and weight.is_contiguous() and weight.data_ptr() % 16 == 0:
     return _hip_gemm().input_gradient(_rows(dy), weight)
   return dy @ weight
 
 
 def weight_gradient(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
   """dy^T x of rows [M, N] and [M, K]"""
-  if weight_wins(dy.shape[0], dy.shape[1], x.shape[1]) and once(dy):
+  if weight_wins(dy.shape[0], dy.shape[1], x.shape[1]) and once(dy, x):
     return _hip_gemm().weight_gradient(_rows(dy), _rows(x))
   return dy.t() @ x
 

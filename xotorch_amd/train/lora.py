@@ -72,7 +72,7 @@ class _AdaptedRows(torch.autograd.Function):
   def backward(ctx, dy):
     x, weight, bias, a, bt, columns = ctx.saved_tensors
     need_x, _, _, need_a, need_b, _ = ctx.needs_input_grad
-    if torch.is_grad_enabled() or not train_ops.own_memory(dy):
+    if not train_ops.once(dy, x, weight, a, bt):
       def whole(x, a, bt):
         return F.linear(x, weight, bias) + (x @ a.to(x.dtype).t() @ bt.to(x.dtype)) * ctx.scaling
       dx, da, db = train_ops._again(whole, (x, a, bt), (need_x, need_a, need_b), (dy,))
