@@ -229,6 +229,21 @@ def test_narrow_sums(M, rank):
   assert low[:M - 1].isfinite().all() and torch.equal(down.isnan(), (t.float().t() @ c[:rank, :M].float().t()).isnan())
 
 
+@pytest.mark.parametrize("rank", [1, 3, 4, 5, 12])
+def test_narrow_sums_of_infinities(rank):
+  """Features that fill a rank up add nothing: a row that holds an infinity is one, and not a number,
+  where fp32 says so."""
+  from xotorch_amd.ops import train_ops
+  hip, M, N = train_ops._hip_lora(), 70, 512
+  t, w, out = _rand(M, N), _rand(rank, N, seed=2).float(), _rand(M, N, seed=3)
+  t[33, 5], t[M - 1, 300] = float("inf"), -float("inf")
+  low, lowt = hip.sums(t, w, 1.0, None, rank, 1.0, False)
+  assert not low[:, rank:].any() and not lowt[rank:].any()
+  want = out.float() + sum(low[:, r:r + 1] * w[r] for r in range(rank))
+  hip.add(out, low, w, 1.0)
+  assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.isinf(), want.isinf())
+
+
 def test_second_derivatives_forward_mode_and_transforms():
   """What the functions cannot do themselves goes by torch's operators."""
   from xotorch_amd import ops

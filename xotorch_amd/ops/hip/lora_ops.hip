@@ -163,6 +163,10 @@ __global__ __launch_bounds__(256) void merge_kernel(MergeArgs a) {
 #pragma unroll
   for (int p = 1; p < 8; ++p) sum += part[p][lane];
   sum *= down ? a.col_scale : a.row_scale;
+  // what fills a rank up are products with zeros, so no numbers where t has an infinity
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (q * 4 + e >= a.r) sum[e] = 0.f;
   if (down) {
     if (i >= most) return;
 #pragma unroll
