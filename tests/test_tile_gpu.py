@@ -37,7 +37,7 @@ def test_products(m, N, K):
 
 
 @pytest.mark.parametrize("N,K", [(72, 320), (3584, 3584), (28680, 192), (520, 18944), (1048, 4096), (264, 16384),
-                                 (40968, 4096)])  # the last three begin at different places of k
+                                 (40968, 4096), (40960, 4096), (36872, 4096)])  # the last five begin at different places of k
 def test_rows_do_not_depend_on_their_batch(N, K):
   from xotorch_amd import ops
   x, w, b = _inputs(256, N, K)

@@ -26,7 +26,8 @@ struct TileArgs {
   const bf16_t *x, *w, *bias;
   void* y;  // bf16 [m, N], or fp32 [splits, m, N]
   int m, N, K, splits;  // N: output features
-  bool turned, runs, dense;  // see turns, run_tile, launch_tile
+  int turned;         // see first_step: 0, or how many features of a gated product begin together
+  bool runs, dense;   // see run_tile, launch_tile
   int whole, more, inv;  // steps of 64 of a part, in all parts `more` besides; 65536 / splits, and one more
 };
 
@@ -51,10 +52,14 @@ enum TileEnd { STORE, PART, GATED };
 // [8192, 8192] m 4 34, 23; m 128 36, 29; gate [57344, 8192] m 32 168, 143; m 128 176, 149;
 // [28672, 4096] m 4 45, 39; [4096, 14336] in 7 parts m 32 27, 21. Other lengths gain nothing
 // ([37888, 3584] m 8 47.4, 47.9); long ones lose, whose parts of x come from L2 only while
-// all blocks want the same ([8192, 28672] m 128 93, 115).
+// all blocks want the same ([8192, 28672] m 128 93, 115). Rows that begin together are
+// whole tiles of any size that the weights may meet: where one is 160 rows (gate_tile), 640
+// features.
 template <int END>
 DEVINL int first_step(const TileArgs& a, int row, int len) {
-  return a.turned ? (int)((((unsigned)row / (END == GATED ? 128 : 256) * 2654435761u >> 16) * (unsigned)len) >> 16) : 0;
+  if (!a.turned) return 0;
+  const unsigned group = END != GATED ? (unsigned)row / 256 : a.turned == 640 ? (unsigned)row / 640 : (unsigned)row / 128;
+  return (int)(((group * 2654435761u >> 16) * (unsigned)len) >> 16);
 }
 
 // R fragments from a on and C from b on, 16 rows (2 KB) apart; waits for them
@@ -424,11 +429,11 @@ static void run_tile(TileArgs a) {
   a.whole = a.K / 64 / a.splits;
   a.more = a.K / 64 % a.splits;
   a.inv = 65536 / a.splits + 1;
-  a.turned = turns(a.K, a.splits);
   // x larger than a die's L2 has room for: [16384, 16384] m 128 132, 96 us; [16384 -> 16384,
   // 2048] with x of 0.5 MB 23, 27
   a.runs = END == PART && (int64_t)a.m * a.K > 1 << 20;
   const int rows = END == GATED ? 2 * a.N : a.N, units = (rows + 127) / 128 * a.splits;
+  a.turned = !turns(a.K, a.splits) ? 0 : gate_tile(rows, 256) == 160 ? 640 : 128;
   if (a.m <= 16) launch_tile<64, 16, 4, END>(a);
   else if (a.m <= 32) {
     if (units >= 200) launch_tile<128, 32, 4, END>(a);
