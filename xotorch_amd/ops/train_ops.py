@@ -124,17 +124,22 @@ def _again(f: Callable, inputs: Sequence[torch.Tensor], needs: Sequence[bool], g
 
 
 # Where the products of hip/gemm_ops.hip are faster than the library's, by what they took of
-# its time (40 to 4096 tokens, the linears of 0.5B, 1B, 8B and 70B decoders; M tokens through
-# a weight [N, K]). What the kernels don't index is the library's.
+# its time on the GPU with weights from memory, as a pass finds them (1 to 4096 tokens, the
+# linears of decoders of 0.5B to 70B; M tokens through a weight [N, K]). Passes of few tokens or
+# short rows wait for the host, to which a call of the library is the longer one: there is no
+# lower end, and narrow products of short rows are the kernels' though they are slower by
+# themselves. 300 tokens through 28 layers of 1536 took 3070 us, and 3500 with those by the
+# library; 512 tokens 3520, and 3420 to 3660. What the kernels don't index is the library's.
 _MOST = 1 << 22  # rows, features
 
 
 def forward_wins(M: int, N: int, K: int) -> bool:
-  """x W^T: 0.40 to 1.11 (0.73 on average) for narrow results of up to 1000 tokens; wider ones
-  and more tokens 0.95 to 1.40, but for long sums, whose library tiles fill the chip badly
-  (257 to 2000 tokens by 1536 to 12288 features of 13824 to 29568): where the result is small
-  0.46 to 1.05 (0.69), of up to 6144 features 0.65 to 0.95, narrow ones of longest sums 0.39 to
-  0.87. Above these lines 0.6 to 1.5 from one size to the next."""
+  """x W^T: narrow results of up to 1000 tokens 0.28 to 1.31 (0.79 on average) for rows of 3072
+  and more; for shorter ones 0.80 to 1.30 (0.98) up to 32 tokens, 0.76 to 1.65 (1.19) from
+  there on. Wider results and more tokens 0.95 to 1.40, but for long sums, whose library tiles
+  fill the chip badly (257 to 2000 tokens by 1536 to 12288 features of 13824 to 29568): where
+  the result is small 0.46 to 1.05 (0.69), of up to 6144 features 0.65 to 0.95, narrow ones of
+  longest sums 0.39 to 0.87. Above these lines 0.6 to 1.5 from one size to the next."""
   if K % 64 or N % 4 or max(M, N, K) > _MOST:
     return False
   if M <= 1000 and N <= 4096:
@@ -144,15 +149,20 @@ def forward_wins(M: int, N: int, K: int) -> bool:
 
 
 def input_wins(M: int, N: int, K: int) -> bool:
-  """dy W, a sum over N: 0.25 to 1.07 (0.66 on average) where that is no shorter than the result
-  is wide, or for few tokens; with more tokens 0.46 to 0.95 where it is much longer and 0.92 to
-  1.26 else. Shorter sums: 0.85 to 1.27 from 333 tokens on."""
-  return N % 64 == 0 and K % 8 == 0 and max(M, N, K) <= _MOST and (M <= 1400 and (N >= K or M <= 300) or (M <= 3000 and N >= 8 * K))
+  """dy W, a sum over N: 0.20 to 1.10 (0.58 on average), weights of less than 5 10^6 numbers
+  0.72 to 1.44 (1.05). What is left to the library: 1001 to 1400 tokens by sums of less than
+  four times the result's width, 0.93 to 1.31; 257 to 300 by [8192, 28672] 1.34; 3000 by
+  [16384, 2048] 1.16; shorter sums of more tokens 0.85 to 1.27."""
+  if N % 64 or K % 8 or max(M, N, K) > _MOST:
+    return False
+  if M <= 1000:
+    return N >= K or M <= (300 if N * K <= 100_000_000 else 256)
+  return N >= 10 * K and M <= 3000 or N >= 8 * K and M <= 2000 or M <= 1400 and (N >= 4 * K or N >= K and N * K <= 8_000_000)
 
 
 def weight_wins(M: int, N: int, K: int) -> bool:
-  """dy^T x, a sum over tokens: 0.81 to 1.05 (0.89 on average) from 600 tokens on, and 0.23 to
-  0.8 for small weights; large weights and 100 to 512 tokens 0.85 to 1.16."""
+  """dy^T x, a sum over tokens: 0.61 to 1.25 (0.88 on average) from 600 tokens on; small weights
+  of fewer 0.54 to 1.20 (0.89), large ones and 100 to 512 tokens 0.85 to 1.16."""
   return M >= 64 and N % 8 == 0 and K % 8 == 0 and max(M, N, K) <= _MOST and (M >= 600 or N * K <= 7_000_000)
 
 
