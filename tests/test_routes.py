@@ -117,6 +117,16 @@ def test_the_rules_know_how_k_is_split():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", [136, 200, 256])
+def test_the_rules_know_which_gated_tiles_make_a_round(rows):
+  from xotorch_amd import ops
+  edges = [f * t + d for t in (64, 128, 160, 256, 320) for f in (143, 199, 256) for d in (-8, 0, 8)]
+  for N in (1792, 4864, 16384, 17920, 28672, 37888, 57344, 106496, *edges):
+    one_round = ops.tile_splits(N, 4096) == 1 and ops._tile().gate_tile(N, rows) > 0
+    assert ops.gate_wins(rows, N, 4096) == one_round
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows", [1, 5])
 def test_a_linear_that_is_followed(rows, monkeypatch):
   from torch.fx.experimental.proxy_tensor import make_fx

@@ -579,6 +579,7 @@ std::vector<Tensor> tile_rest(Tensor heads, Tensor wo, Tensor x, Tensor post, do
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("tile_rest", &tile_rest);
   m.def("tile_splits", [](int64_t n, int64_t k) { return splits_of((int)n, (int)(k / 64)); });
+  m.def("gate_tile", [](int64_t rows, int64_t m) { return gate_tile((int)rows, (int)m); });
   m.def("tile_parts", &tile_parts);
   m.def("tile_linear", &tile_linear);
   m.def("tile_swiglu", &tile_swiglu);
