@@ -89,8 +89,10 @@ class XotLinear(nn.Linear):
   order ([N/32,K/16,64,8], see ops.pack_decode_weight); with 32, 64 .. 256 rows these
   ways, the weight-streaming kernels that read the copy and hipBLASLt are timed at the
   first call and the fastest is kept (lm_head of 70B, 64 rows: 0.87 of the library's time
-  by the copy, 1.07 by tiles). More rows, training and the CPU stay on hipBLASLt and
-  aten. Storage and state dict are nn.Linear's."""
+  by the copy, 1.07 by tiles). More rows and training go by ops.linear: the kernels of
+  hip/gemm_ops.hip where train_ops.forward_wins, input_wins and weight_wins say so, else
+  hipBLASLt; MLP.whole_gate takes gate and up of prompts in one kernel, past this
+  forward. The CPU stays on aten. Storage and state dict are nn.Linear's."""
 
   hip = ("_hip_rows", "_hip_tile", "_hip_gemm")  # what a pass loads beside the operators
   weight_packed: Optional[torch.Tensor]

@@ -392,8 +392,11 @@ def _one_round(N: int, K: int) -> bool:
 
 @functools.lru_cache(maxsize=1024)
 def _aligned(N: int, K: int) -> bool:
-  """Whether rows and parts of k lie a power of two apart, 16 KB or more, where blocks seem to
-  wait for the same few memory channels (1.06 to 1.27 of the library's time up to 64 rows)."""
+  """Whether rows and parts of k lie a power of two apart, 16 KB or more. Where all blocks begin
+  with the same columns they wait for the same few memory channels, and such products took
+  1.06 to 1.27 of the library's time up to 64 rows. Since blocks begin at different places
+  (first_step in hip/tile_ops.hip) they take 0.48 to 1.03 (0.79 on average), parts 0.28 to 0.98
+  (0.69): the line lies where it did before that, on the side of the library."""
   splits = tile_splits(N, K)
   return K >= 8192 and K & (K - 1) == 0 and 1 < splits and splits & (splits - 1) == 0
 
@@ -421,7 +424,7 @@ def tile_wins(rows: int, N: int, K: int) -> bool:
 def parts_win(rows: int, N: int, K: int) -> bool:
   """The same for tile_parts, whose sums the next kernel adds up: 0.23 to 1.21 (0.7 on
   average) up to 16 rows, then 0.23 to 1.08 in one round; in more 0.72 to 1.15 up to 64
-  rows (aligned ones to 1.21), 0.72 to 1.54 above, by which layers of mistral-large and
+  rows, 0.72 to 1.54 above, by which layers of mistral-large and
   llama-3.1-405b took 1.03 to 1.14 of what they take by the library."""
   return rows <= 16 or _one_round(N, K) or (rows <= 64 and not _aligned(N, K))
 

@@ -10,9 +10,10 @@
 // transposing reads from LDS, so that nothing is transposed in memory. Where tiles are few
 // the sum is cut into parts, whose fp32 sums a second kernel adds up.
 //
-// us, library beside, 666 tokens: input [16384 -> 2048] 56 (111), [128256 -> 2048] 377 (870);
-// weights [16384, 2048] 58 (69), [2048, 2048] 11 (20); forward [8192 -> 2048] 34 (40). 4096
-// tokens: input [28672 -> 4096] 703 (722), weights of it 762 (844), forward 730 (662).
+// us, library beside, weights from memory, 666 tokens: input [16384 -> 2048] 56 (117),
+// [128256 -> 2048] 328 (873); weights [16384, 2048] 54 (62), [2048, 2048] 10 (16); forward
+// [8192 -> 2048] 37 (42). 4096 tokens: weights [28672, 4096] 749 (825); input and forward of
+// it, which are the library's, 703 (722) and 730 (662).
 #include "mfma_tile.h"
 
 struct GemmArgs {

@@ -7,11 +7,10 @@
 // What bounds them is t, read once, or out, read and written: library products of 8 features
 // read a gradient once for either sum. us, library beside, 4096 tokens, rank 8: both sums of
 // 28672 features 55 (126), of 4096 13 (41); the sum added to 28672 102 (132), to 14336 56 (72),
-// to 4096 14 (19). Four layers of 4096 with 8 x 512 tokens 15400 to 14300 forward and back.
-// Here a block holds a strip of
-// 256 columns of t and walks down its rows in steps of 64 through two LDS buffers; a step is
-// multiplied along its rows and, read by transposing, along its columns. Sums of strips and of
-// runs of rows are added up by another kernel, in order.
+// to 4096 14 (19). Four layers of 4096 with 8 x 512 tokens, forward and back, 14300 (15500).
+// Here a block holds a strip of 256 columns of t and walks down its rows in steps of 64 through
+// two LDS buffers; a step is multiplied along its rows and, read by transposing, along its
+// columns. Sums of strips and of runs of rows are added up by another kernel, in order.
 #include "mfma_tile.h"
 
 struct SumArgs {

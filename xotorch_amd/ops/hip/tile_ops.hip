@@ -13,11 +13,12 @@
 // make too few blocks, k is split; the parts' fp32 sums are added by the kernel that
 // follows anyway (norm, activation).
 //
-// us, library beside: [3584, 18944] m 8 23 (48), m 32 23 (110), m 128 33 (99);
-// [8192, 28672] m 128 97 (199); [8192, 8192] m 128 35 (48); [4608, 3584] m 256 19 (37).
+// us, library beside: [3584, 18944] m 8 23 (46), m 32 23 (110), m 128 33 (99);
+// [8192, 28672] m 128 89 (201); [8192, 8192] m 128 29 (47); [4608, 3584] m 256 17 (36).
 //
 // How k is split depends on the weights' shape alone, and the order of the sums within
-// a part on the shape and the weight row: a row of these products does not depend on the rows beside it.
+// a part on the shape and the weight row: a row of these products does not depend on the
+// rows beside it.
 // (Whether a product is one of these does, and so does how attention cuts its keys.)
 #include "common.h"
 #include "mfma_tile.h"
@@ -49,8 +50,8 @@ enum TileEnd { STORE, PART, GATED };
 // lie a multiple of 8 KB apart, which few memory channels hold: where rows or parts do
 // (turns), blocks begin at different places. It goes by weight rows, so that a row of x
 // is summed up as in any other batch. us, all from the start of their part first:
-// [8192, 8192] m 4 34, 23; m 128 36, 29; gate [57344, 8192] m 32 168, 143; m 128 176, 149;
-// [28672, 4096] m 4 45, 39; [4096, 14336] in 7 parts m 32 27, 21. Other lengths gain nothing
+// [8192, 8192] m 4 32, 22; m 128 35, 29; gate [57344, 8192] m 32 166, 145; [28672, 4096]
+// m 4 42, 36; [4096, 14336] in 7 parts m 32 26, 19. Other lengths gain nothing
 // ([37888, 3584] m 8 47.4, 47.9); long ones lose, whose parts of x come from L2 only while
 // all blocks want the same ([8192, 28672] m 128 93, 115). Rows that begin together are
 // whole tiles of any size that the weights may meet: where one is 160 rows (gate_tile), 640
@@ -390,19 +391,20 @@ static void launch_tile(TileArgs a) {
 
 // Tile and depth by the rows of x and by the blocks that 128 weight rows make. us at
 // [N, K], 64-row or (deeper, fewer to a CU) first:
-//   m 32: [2048, 2048] in 128 blocks 4.4, 5.0; [3584, 18944] in 224 25.6, 22.9
-//   m 64: [2048, 2048] 5.0, 6.0; [28672 -> 8192] 89.7, 76.1
-//   m 128, 3 and 2 buffers: [8192, 8192] in 256 35.4, 39.6; [57344, 8192] in 448 203, 194
+//   m 32: [2048, 2048] in 128 blocks 4.1, 4.6; [3584, 18944] in 224 25.0, 22.6
+//   m 64: [2048, 2048] 4.6, 5.6; [28672 -> 8192] 91.0, 78.3
+//   m 128, 3 and 2 buffers: [8192, 8192] in 256 29.5, 36.5; gate [57344, 8192] in 448, now
+//   in other tiles, 193, 176
 // From 129 rows of x on all of them in one block (wide_kernel), if k is split in enough
-// parts: m 256, and 136 by 192 rows, us, with 128 rows a block: [3584, 18944] in 224 43.3
-// and 36.2 (55.6); [28672 -> 8192] 114.9 and 97.9 (157); with fewer blocks a block's start
-// outweighs it, [2048, 2048] in 128 13.0 (9.1).
+// parts: m 256, and 136 by 192 rows, us, with 128 rows a block: [3584, 18944] in 224 41.7
+// and 33.9 (53.6 and 51.1); [28672 -> 8192] 119 and 98 (148 and 159); with fewer blocks a
+// block's start outweighs it, [2048, 2048] in 128 11.7 (8.8).
 //
 // The gated product of more than 64 rows takes the weight tile that makes one round of the
-// chip's 256 CUs, if there is one: [37888, 3584] 237 blocks of 160 rows 71 with m 256 (library
-// and activation 84; 296 of 128 108, 148 of 256 87), [57344, 8192] 224 of 256 203 (253; 448 of
-// 128 247). Up to 128 rows, whose matrix products are short, 148 blocks of 256 are enough:
-// 64 with m 128 (77; 83).
+// chip's 256 CUs, if there is one: [37888, 3584] 237 blocks of 160 rows 70 with m 256 (library
+// and activation 84; 296 of 128 120, 148 of 256 83), [57344, 8192] 224 of 256 211 (220; 448 of
+// 128 235). Up to 128 rows, whose matrix products are short, 148 blocks of 256 are enough:
+// 63 with m 128 (73; 78).
 static int gate_tile(int rows, int m) {
   if (m <= 128) return rows > 143 * 256 && rows <= 256 * 256 ? 256 : 0;
   for (int tile : {128, 160, 256})
@@ -429,8 +431,9 @@ static void run_tile(TileArgs a) {
   a.whole = a.K / 64 / a.splits;
   a.more = a.K / 64 % a.splits;
   a.inv = 65536 / a.splits + 1;
-  // x larger than a die's L2 has room for: [16384, 16384] m 128 132, 96 us; [16384 -> 16384,
-  // 2048] with x of 0.5 MB 23, 27
+  // x larger than a die's L2 has room for beside the weights. us, the grid's parts first:
+  // m 128 by [4096, 14336] 29.2, 28.2; by [3584, 18944] 32.7, 32.2; by [8192, 28672] 90 both;
+  // with x of 0.5 MB no matter, [16384, 2048] 17.5, 17.3
   a.runs = END == PART && (int64_t)a.m * a.K > 1 << 20;
   const int rows = END == GATED ? 2 * a.N : a.N, units = (rows + 127) / 128 * a.splits;
   a.turned = !turns(a.K, a.splits) ? 0 : gate_tile(rows, 256) == 160 ? 640 : 128;

@@ -176,9 +176,9 @@ def product(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 
 def takes_product(x: torch.Tensor, weight: torch.Tensor) -> bool:
   """Whether `product` is a linear of these without a gradient, of more rows than the
-  kernels of decode steps take. Prompts by it and by the library, us: 300 tokens through 16
-  layers of 2048 1915, 2295; 512 through 8 of 4096 2302, 2422; 400 through 28 of 3584 8300,
-  11980; 1000 through 16 of 2048 3076, 3160."""
+  kernels of decode steps take. Prompts by it and gate_product, and by the library, us: 300
+  tokens through 16 layers of 2048 1870, 2300; 512 through 28 of 3584 9350, 12430; 1000
+  through 16 of 2048 2990, 3370."""
   if not x.is_cuda or x.dtype is not torch.bfloat16 or weight.dtype is not torch.bfloat16 or torch.is_grad_enabled() or weight.dim() != 2:
     return False
   (N, K), M = weight.shape, x.numel() // max(1, weight.shape[1])
