@@ -188,8 +188,8 @@ def takes_product(x: torch.Tensor, weight: torch.Tensor) -> bool:
 
 def gate_wins(M: int, N: int, K: int) -> bool:
   """silu of gate times up in one kernel over the library's product and the activation's
-  kernel (0.5B to 70B decoders, 257 to 8192 tokens): 0.65 to 1.00 (0.88 on average), with rows
-  of 8192 0.93 to 1.02 up to 3000 tokens and 1.01 to 1.04 from 4096 on."""
+  kernel (0.5B to 70B decoders, 257 to 8192 tokens): 0.64 to 1.00 (0.86 on average), with rows
+  of 8192 to 16384 0.75 to 1.10 (0.93) up to 3000 tokens and 1.01 to 1.04 from 4096 on."""
   return M > 256 and K % 64 == 0 and N % 32 == 0 and (K <= 4096 or M <= 3000)
 
 
