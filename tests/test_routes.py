@@ -204,13 +204,15 @@ def test_what_a_prompt_loads_is_built_for_it():
 
 
 def test_gradients_of_inputs_go_where_they_are_faster():
-  """Many tokens only by long sums; a second tile of rows not by the largest weights."""
+  """Many tokens only by long sums or small weights; a second tile of rows not by the largest."""
   from xotorch_amd.ops.train_ops import input_wins
   for N, K in ((2048, 2048), (4096, 14336), (16384, 2048), (28672, 4096), (128256, 2048)):
     assert all(input_wins(m, N, K) for m in (1, 40, 256, 300)) and (N < K or all(input_wins(m, N, K) for m in (666, 1000, 1001, 1400)))
-  assert input_wins(1000, 8192, 8192) and not input_wins(1001, 8192, 8192)
+  assert input_wins(1024, 8192, 8192) and not input_wins(1025, 8192, 8192)
+  for N, K in ((4096, 4096), (6144, 4096), (5120, 3072)):
+    assert input_wins(1280, N, K) and not input_wins(1281, N, K) and not input_wins(1401, N, K)
   assert input_wins(256, 8192, 28672) and not input_wins(257, 8192, 28672) and not input_wins(301, 4096, 14336)
-  assert input_wins(2000, 16384, 2048) and not input_wins(2001, 16384, 2048) and input_wins(3000, 37888, 3584) and not input_wins(3001, 37888, 3584)
+  assert input_wins(2800, 16384, 2048) and not input_wins(2801, 16384, 2048) and input_wins(3000, 37888, 3584) and not input_wins(3001, 37888, 3584)
 
 
 @pytest.mark.parametrize("needs", [(True, False), (False, True), (True, True)])

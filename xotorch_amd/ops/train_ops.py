@@ -149,15 +149,18 @@ def forward_wins(M: int, N: int, K: int) -> bool:
 
 
 def input_wins(M: int, N: int, K: int) -> bool:
-  """dy W, a sum over N: 0.20 to 1.10 (0.58 on average), weights of less than 5 10^6 numbers
-  0.72 to 1.44 (1.05). What is left to the library: 1001 to 1400 tokens by sums of less than
-  four times the result's width, 0.93 to 1.31; 257 to 300 by [8192, 28672] 1.34; 3000 by
-  [16384, 2048] 1.16; shorter sums of more tokens 0.85 to 1.27."""
+  """dy W, a sum over N: 0.20 to 1.10 (0.6 on average), weights of less than 5 10^6 numbers
+  0.72 to 1.44 (1.05). What is left to the library: by sums of less than four times the
+  result's width 1025 to 1400 tokens and weights of 8192 by 8192 and more 1.15 to 1.38, 1281 to
+  1400 and smaller ones 0.93 to 1.11 (1.04); 257 to 300 by weights of more than 10^8
+  1.21 to 1.43; 3000 by [16384, 2048] 1.15; shorter sums of more tokens 0.85 to 1.27."""
   if N % 64 or K % 8 or max(M, N, K) > _MOST:
     return False
-  if M <= 1000:
+  if M <= 1024:
     return N >= K or M <= (300 if N * K <= 100_000_000 else 256)
-  return N >= 10 * K and M <= 3000 or N >= 8 * K and M <= 2000 or M <= 1400 and (N >= 4 * K or N >= K and N * K <= 8_000_000)
+  if M <= 1400 and N < 4 * K:
+    return N >= K and N * K <= (60_000_000 if M <= 1280 else 8_000_000)
+  return M <= 1400 and N >= K or M <= 2800 and N >= 8 * K or M <= 3000 and N >= 10 * K
 
 
 def weight_wins(M: int, N: int, K: int) -> bool:
