@@ -89,3 +89,57 @@ def test_rows_of_an_expert(tile, K, F, swiglu, few):
       # silu's slope is at most 1.1; its hardware exponential and reciprocal are off by some 2^-20
       slack = (1.1 * sg + gate.abs() * 2.0 ** -19) * up.abs() + su * gate.abs()
     assert bool(((got[first[e]:first[e + 1]].double() - want).abs() <= slack + want.abs() * 2.0 ** -8 + 1e-30).all()), counts[e]
+
+
+@pytest.mark.parametrize("rows", [[129, 160, 161, 224, 225], [150, 0, 200, 300, 450, 33], [96, 97, 320, 321, 447, 448]])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_shares_of_rows_in_steps_of_32(rows, swiglu):
+  """Tiles of 160 and 224 rows, whole and cut in two: what one row gives does not depend on its tile's form."""
+  from xotorch_amd.ops.mixer_ops import load_hip
+  hip = load_hip("_hip_experts")
+  K, F, n = 320, 528, sum(rows)
+  g = torch.Generator(device="cuda").manual_seed(n)
+  x = torch.randn(n, K, generator=g, device="cuda").to(torch.bfloat16)
+  w = [(torch.randn((2 if swiglu else 1) * F, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16) for _ in rows]
+  ints = dict(dtype=torch.int32, device="cuda")
+
+  def product(counts, some, weights, tile):
+    first = [0]
+    for c in counts:
+      first.append(first[-1] + c)
+    tiles = [(e, r) for e in range(len(counts)) for r in range(first[e], first[e + 1], tile)]
+    most = first[-1] // tile + len(counts)
+    listed = tiles + [(-1, 0)] * (most - len(tiles)) + [(-1, len(tiles))]
+    token = torch.arange(first[-1], **ints)
+    return hip.expert_product_of(some, weights, token, torch.tensor(first, **ints), torch.tensor(listed, **ints), tile, swiglu), first
+
+  got, first = product(rows, x, w, 256)
+  for e, c in enumerate(rows):
+    if c:
+      alone = product([c], x[first[e]:first[e + 1]].contiguous(), [w[e]], 128)[0]
+      assert torch.equal(got[first[e]:first[e + 1]], alone)
+  size = x.double().abs().sum(1).max() * max(t.double().abs().max() for t in w)
+  want = x[:rows[0]].double() @ w[0].double().t()
+  if swiglu:
+    gate, up = want.chunk(2, -1)
+    want = torch.nn.functional.silu(gate) * up
+  assert bool(((got[:rows[0]].double() - want).abs() <= want.abs() * 2.0 ** -8 + size * size * K * 2.0 ** -22).all())
+
+
+def test_tokens_past_four_gigabytes():
+  """Offsets of more than 32 bits, of the last tokens of all."""
+  from xotorch_amd.ops.mixer_ops import load_hip
+  hip = load_hip("_hip_experts")
+  T, K, F, n = (1 << 20) + 40, 2048, 32, 300
+  x = torch.zeros(T, K, device="cuda", dtype=torch.bfloat16)
+  g = torch.Generator(device="cuda").manual_seed(T)
+  token = torch.cat([torch.randint(0, T, (n - 2,), generator=g, device="cuda"), torch.tensor([0, T - 1], device="cuda")])
+  x[token] = torch.randn(n, K, generator=g, device="cuda").to(torch.bfloat16)
+  w = (torch.randn(2 * F, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+  ints = dict(dtype=torch.int32, device="cuda")
+  for tile in (128, 256):
+    tiles = [(0, r) for r in range(0, n, tile)]
+    listed = tiles + [(-1, 0)] * (n // tile + 1 - len(tiles)) + [(-1, len(tiles))]
+    args = torch.tensor([0, n], **ints), torch.tensor(listed, **ints), tile, True
+    near = hip.expert_product_of(x[token].contiguous(), [w], torch.arange(n, **ints), *args)
+    assert torch.equal(hip.expert_product_of(x, [w], token.to(torch.int32), *args), near)

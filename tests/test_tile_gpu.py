@@ -36,6 +36,14 @@ def test_products(m, N, K):
       assert bool(((ops.tile_swiglu(x, w).double() - act * u).abs() <= bound + 1e-30).all())
 
 
+# from 65 rows on: parts of few steps and of many, blocks for a round, for more than one and for
+# half of one, rows of x in two blocks, weight rows past a tile and off the 16 bytes of a piece
+@pytest.mark.parametrize("m,N,K", [(66, 3592, 3584), (100, 4104, 14336), (128, 1002, 8192), (128, 33000, 128), (81, 41000, 64), (150, 3084, 4096),
+                                   (192, 4104, 1536), (193, 4100, 2048), (130, 1000, 1024), (256, 1006, 512), (160, 57352, 128), (129, 65528, 64)])
+def test_products_of_more_rows(m, N, K):
+  test_products(m, N, K)
+
+
 @pytest.mark.parametrize("N,K", [(72, 320), (3584, 3584), (28680, 192), (520, 18944), (1048, 4096), (264, 16384),
                                  (40968, 4096), (40960, 4096), (36872, 4096)])  # the last five begin at different places of k
 def test_rows_do_not_depend_on_their_batch(N, K):

@@ -475,7 +475,7 @@ class MoEMLP(nn.Module):
     of a tile of 128 tokens empty)."""
     E, k = self.n_experts, self.top_k
     if flat.dtype != torch.bfloat16 or flat.shape[0] * k <= 24 * E or E > 256 or k > 8 or flat.shape[1] % 64 \
-       or self.intermediate % 64 or not flat.is_contiguous() or os.getenv("XOT_FP8_PREFILL", "0") == "1":
+       or max(flat.shape[1], self.intermediate) > 1 << 22 or self.intermediate % 64 or not flat.is_contiguous() or os.getenv("XOT_FP8_PREFILL", "0") == "1":
       return False
     mods = [p for e in self.experts for p in (e.gate_up_proj, e.down_proj)]
     return (type(self.gate) is nn.Linear and all(type(e) is MLP for e in self.experts) and not _watched(self.gate, *self.experts, *mods)

@@ -365,10 +365,9 @@ __global__ __launch_bounds__(256) void expert_stream_kernel(
 // Many tokens per expert (bf16): up to TOK tokens x BN weight rows (GATED: BN / 2 gate and
 // the same of up) per block, by mfma_tile.h. What bounds them is the matrix cores, and
 // rows of a tile that no token fills: an expert's rows go over its tiles evenly, in steps
-// of 64, and the fewer a tile has the more waves share the weight rows out. 8 experts of
-// 4096 x 14336, two of them a token, both products, us: 2100 tokens 1447 (with tiles of
-// 256 and what is left, each as if whole, and a barrier between reading and multiplying,
-// 1916), 4000 tokens 2495 (3102), 620 578 (833), 200 498 (640).
+// of 32. 8 experts of 4096 x 14336, two of them a token, both products, us: 2100 tokens 1365
+// (in steps of 64 by eight waves 1420), 1500 911 (1018), 1000 814 (852), 500 548 (590), 300 553
+// (560).
 
 // Where an expert's weight rows lie: in one tensor, or in one tensor each
 struct Stacked {
@@ -381,92 +380,103 @@ struct Listed {
   DEVINL const bf16_t* of(int e, size_t) const { return w[e]; }
 };
 
-// Of 64, 128, 192 and 256 tokens: waves along the weight rows, buffers of weights and tokens
+// Waves along the weight rows, buffers of weights and tokens
 template <int BN, int BM, int WN_, int WB, int XB> struct Shape : MfmaTile<BN, BM, WN_, WB, XB> { static constexpr int WN = WN_; };
 template <int BN, int BM> struct ExpertTile;
-template <> struct ExpertTile<256, 64> : Shape<256, 64, 8, 4, 4> {};
-template <> struct ExpertTile<256, 128> : Shape<256, 128, 4, 3, 3> {};
-template <> struct ExpertTile<256, 192> : Shape<256, 192, 4, 3, 2> {};
+template <> struct ExpertTile<256, 64> : Shape<256, 64, 4, 4, 4> {};
+template <> struct ExpertTile<256, 128> : Shape<256, 128, 2, 3, 3> {};
+template <> struct ExpertTile<256, 160> : Shape<256, 160, 2, 3, 3> {};
+template <> struct ExpertTile<256, 192> : Shape<256, 192, 2, 3, 2> {};
+template <> struct ExpertTile<256, 224> : Shape<256, 224, 2, 3, 2> {};
 template <> struct ExpertTile<256, 256> : Shape<256, 256, 2, 3, 2> {};
-template <> struct ExpertTile<128, 64> : Shape<128, 64, 4, 3, 3> {};
-template <> struct ExpertTile<128, 128> : Shape<128, 128, 2, 2, 2> {};
+template <> struct ExpertTile<128, 64> : Shape<128, 64, 2, 3, 3> {};
+template <> struct ExpertTile<128, 128> : Shape<128, 128, 2, 3, 2> {};
 template <> struct ExpertTile<128, 192> : Shape<128, 192, 2, 4, 4> {};
 template <> struct ExpertTile<128, 256> : Shape<128, 256, 2, 3, 3> {};
 // of all forms that a kernel of BN weight rows and TOK tokens may take
 template <int BN, int TOK> constexpr int expert_lds() {
   int most = std::max(ExpertTile<BN, 64>::LDS, ExpertTile<BN, 128>::LDS);
   if constexpr (TOK == 256)  // and of 128 weight rows
-    most = std::max({most, expert_lds<128, 128>(), ExpertTile<128, 192>::LDS, ExpertTile<128, 256>::LDS, ExpertTile<256, 192>::LDS, ExpertTile<256, 256>::LDS});
+    most = std::max({most, expert_lds<128, 128>(), ExpertTile<128, 192>::LDS, ExpertTile<128, 256>::LDS, ExpertTile<256, 160>::LDS,
+                     ExpertTile<256, 192>::LDS, ExpertTile<256, 224>::LDS, ExpertTile<256, 256>::LDS});
   return most;
 }
 
-// One tile: tokens r0 up to hi, of which there are at most BM
-template <int KIND, int BN, int BM>
+// One tile: tokens r0 up to hi, of which there are at most BM. TAIL: rows of x may end within
+// a step; FAR: x takes 4 GB or more
+template <int KIND, int BN, int BM, bool TAIL, bool FAR>
 DEVINL void expert_tile(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const int* __restrict__ token,
                         const float* __restrict__ by_row, bf16_t* __restrict__ y, const GroupArgs& a, const Act& act,
                         int r0, int hi, int fb, bf16_t* buf) {
   typedef ExpertTile<BN, BM> Sh;
-  constexpr bool TWO = has_gate(KIND);  // weight rows are gate and up
+  constexpr bool TWO = has_gate(KIND), OWN = of_own_row(KIND);  // TWO: weight rows are gate and up
   constexpr int R = Sh::R, C = Sh::C, ROWS = R * 16;  // a wave's weight rows: gate rows, then the same of up
   constexpr int WL = Sh::WL, XL = Sh::XL;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
   const int wf = wave % Sh::WN, wt = wave / Sh::WN, f0 = fb * (TWO ? BN / 2 : BN);
-  const bf16_t *wsrc[WL], *xsrc[XL];
-  const int piece = ((lane & 7) ^ (lane >> 3)) * 8;
-  const unsigned woff = ((lane >> 3) * a.kp + piece) * 2;
+  const int piece = ((lane & 7) ^ (lane >> 3)) * 8, up = TWO ? wave >> 1 : 0;  // two waves load gates, two up
+  const bf16_t *wsrc = w + ((size_t)up * a.F + f0) * a.kp, *xsrc = OWN ? x + (size_t)r0 * a.xs : x;
+  unsigned woff[WL], wto[WL], xoff[XL];
+  const char* xfar[FAR ? XL : 1];
 #pragma unroll
   for (int i = 0; i < WL; ++i) {  // F % 16 == 0: the 8 rows of a load are there, or none of them
-    const int r = (wave * WL + i) * 8;
-    const int f = TWO ? f0 + r / ROWS * (ROWS / 2) + r % (ROWS / 2) : f0 + r;
-    const int part = TWO ? r / (ROWS / 2) & 1 : 0;
-    wsrc[i] = w + ((size_t)part * a.F + min(f, a.F - 8)) * a.kp;
+    const int r = ((TWO ? wave & 1 : wave) * WL + i) * 8;
+    woff[i] = ((unsigned)(min(r, a.F - 8 - f0) + (lane >> 3)) * a.kp + piece) * 2;
+    wto[i] = (TWO ? r / (ROWS / 2) * ROWS + up * (ROWS / 2) + r % (ROWS / 2) : r) * 128;
   }
 #pragma unroll
   for (int i = 0; i < XL; ++i) {
     const int t = min(r0 + (wave * XL + i) * 8 + (lane >> 3), hi - 1);
-    xsrc[i] = x + (size_t)(of_own_row(KIND) ? t : token[t]) * a.xs;
+    if constexpr (FAR) xfar[i] = (const char*)(x + (size_t)token[t] * a.xs);
+    else xoff[i] = ((unsigned)(OWN ? t - r0 : token[t]) * a.xs + (TAIL ? 0 : piece)) * 2;
   }
-  auto loadw = [&](auto number, int s, unsigned at) {
+  const int steps = (a.K + 63) / 64;
+  auto stepw = [&](int s) { return StepSource(wsrc, s * 128, steps - s); };
+  auto stepx = [&](int s) { return StepSource(xsrc, s * 128, steps - s); };
+  auto loadw = [&](auto number, const StepSource& from, unsigned at) {
     constexpr int i = decltype(number)::value;
-    __builtin_amdgcn_global_load_lds((glb_void*)((const char*)(wsrc[i] + s * 64) + woff), (lds_void*)((char*)buf + at + (wave * WL + i) * 1024), 16, 0, 0);
+    from.load(woff[i], (char*)buf + at + wto[i]);
   };
-  auto loadx = [&](auto number, int s, unsigned at) {
+  auto loadx = [&](auto number, StepSource from, unsigned at) {
     constexpr int i = decltype(number)::value;
-    const int k = s * 64 + piece;
+    char* to = (char*)buf + at + (wave * XL + i) * 1024;
     // past the end of a row the weights are zero; any number of the row will do
-    __builtin_amdgcn_global_load_lds((glb_void*)(xsrc[i] + (k < a.K ? k : 0)), (lds_void*)((char*)buf + at + (wave * XL + i) * 1024), 16, 0, 0);
+    const int k = from.at / 2 + piece, in = TAIL && k >= a.K ? 0 : k * 2;
+    if constexpr (FAR) __builtin_amdgcn_global_load_lds((glb_void*)(xfar[i] + in), (lds_void*)to, 16, 0, 0);
+    else if constexpr (TAIL) {
+      from.at = 0;
+      from.load(xoff[i] + in, to);
+    } else from.load(xoff[i], to);
   };
   floatx4 acc[R][C];
-#pragma unroll
-  for (int i = 0; i < R; ++i)
-#pragma unroll
-    for (int j = 0; j < C; ++j) acc[i][j] = (floatx4)(0.f);
   const unsigned base = (unsigned)(size_t)(lds_void*)buf;
-  walk<Sh>(acc, RowFrags<R>(base, wf * ROWS, lane), RowFrags<C>(base + Sh::XAT, wt * C * 16, lane), (a.K + 63) / 64, loadw, loadx);
+  walk<Sh>(acc, RowFrags<R>(base, wf * ROWS, lane), RowFrags<C>(base + Sh::XAT, wt * C * 16, lane), steps, stepw, loadw, stepx, loadx);
+  constexpr int N = TWO ? R / 2 : R;
+  const RowsOut<bf16_t, N * 16> rows(buf, wave, lane);
 #pragma unroll
   for (int j = 0; j < C; ++j) {
-    const int t = r0 + (wt * C + j) * 16 + col;
-    if (t >= hi) continue;
-    bf16_t* dst = y + (size_t)t * a.ys;
-    const float by = !of_own_row(KIND) && by_row ? by_row[t] : 1.f;
-    constexpr int N = TWO ? R / 2 : R;
+    const int t0 = r0 + (wt * C + j) * 16;
+    const float by = !OWN && by_row ? by_row[min(t0 + col, hi - 1)] : 1.f;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-      const int f = f0 + wf * 16 * N + i * 16 + quad * 4;
-      float v[4];
+      ushort4_t v;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = activated<KIND>(by, acc[i][j][r], acc[(i + R / 2) % R][j][r], act);
-      if (f < a.F) st4(dst + f, v);
+      for (int r = 0; r < 4; ++r) v[r] = f2b(activated<KIND>(by, acc[i][j][r], acc[(i + R / 2) % R][j][r], act));
+      rows.put(col, i * 16 + quad * 4, v);
     }
+    rows.out([&](int r, int f, floatx4 v) {
+      const int to = f0 + wf * 16 * N + f;
+      if (t0 + r < hi && to < a.F) *(floatx4*)(y + (size_t)(t0 + r) * a.ys + to) = v;
+    });
   }
 }
 
 constexpr int DIE_CUS = 32;  // of one of the eight dies
 
 // The router's tiles, of which there are as many as the last of `tiles` says; DENSE: max_tiles of rows_of_all rows
-template <int KIND, int BN, int TOK, typename W>
-__global__ __launch_bounds__(512) void expert_tile_kernel(
+template <int KIND, int BN, int TOK, bool FAR, typename W>
+__global__ __launch_bounds__(256) void expert_tile_kernel(
     const bf16_t* __restrict__ x, W w, const int* __restrict__ first,
     const int* __restrict__ token, const int2* __restrict__ tiles, const float* __restrict__ by_row,
     bf16_t* __restrict__ y, int max_tiles, int group, int rows_of_all, GroupArgs a, Act act) {
@@ -496,24 +506,34 @@ __global__ __launch_bounds__(512) void expert_tile_kernel(
     lo = __builtin_amdgcn_readfirstlane(first[e]), end = __builtin_amdgcn_readfirstlane(first[e + 1]);
     nth = (__builtin_amdgcn_readfirstlane(tile.y) - lo) / TOK;
   }
-  // an expert's rows go over its tiles evenly, in steps of 64
-  const int of = (end - lo + TOK - 1) / TOK, share = ((end - lo + of - 1) / of + 63) / 64 * 64;
-  const int r0 = lo + nth * share, hi = min(end, r0 + share);
+  // an expert's rows go over its tiles evenly, in steps of 32
+  const int of = (end - lo + TOK - 1) / TOK, share = ((end - lo + of - 1) / of + 31) / 32 * 32;
+  const int r0 = lo + nth * share, hi = min(end, r0 + share), rows = hi - r0;
   const bf16_t* we = w.of(e, (size_t)(TWO ? 2 : 1) * a.F * a.kp);
-  auto go = [&](auto rows) {
-    if constexpr (CUT) {
-      if (half < 0) return expert_tile<KIND, BN, decltype(rows)::value>(x, we, token, by_row, y, a, act, r0, hi, fb, buf);
-      if ((fb * 2 + half) * (WIDE / 2) < a.F)
-        expert_tile<KIND, 128, decltype(rows)::value>(x, we, token, by_row, y, a, act, r0, hi, fb * 2 + half, buf);
-    } else
-      expert_tile<KIND, BN, decltype(rows)::value>(x, we, token, by_row, y, a, act, r0, hi, fb, buf);
+  constexpr bool TAIL = std::is_same<W, Stacked>::value && KIND != DENSE;
+  auto go = [&](auto weights, auto most) {
+    constexpr int N = decltype(weights)::value, M = decltype(most)::value;
+    expert_tile<KIND, N, M, TAIL, FAR>(x, we, token, by_row, y, a, act, r0, hi, N == BN ? fb : fb * 2 + half, buf);
   };
-  const int rows = hi - r0;
-  if (rows <= 64) go(std::integral_constant<int, 64>());
-  else if (rows <= 128) go(std::integral_constant<int, 128>());
+  typedef std::integral_constant<int, BN> All;
+  if constexpr (CUT) {
+    if (half >= 0) {
+      typedef std::integral_constant<int, 128> Half;
+      if ((fb * 2 + half) * (WIDE / 2) >= a.F) return;
+      if (rows <= 64) go(Half(), std::integral_constant<int, 64>());
+      else if (rows <= 128) go(Half(), std::integral_constant<int, 128>());
+      else if (rows <= 192) go(Half(), std::integral_constant<int, 192>());
+      else go(Half(), std::integral_constant<int, 256>());
+      return;
+    }
+  }
+  if (rows <= 64) go(All(), std::integral_constant<int, 64>());
+  else if (rows <= 128) go(All(), std::integral_constant<int, 128>());
   else if constexpr (TOK == 256) {
-    if (rows <= 192) go(std::integral_constant<int, 192>());
-    else go(std::integral_constant<int, 256>());
+    if (rows <= 160) go(All(), std::integral_constant<int, 160>());
+    else if (rows <= 192) go(All(), std::integral_constant<int, 192>());
+    else if (rows <= 224) go(All(), std::integral_constant<int, 224>());
+    else go(All(), std::integral_constant<int, 256>());
   }
 }
 
@@ -650,11 +670,17 @@ static void launch_tiles(const W& w, const Tensor& x, const Tensor& token, const
   auto run = [&](auto kernel, int lds) {
     const hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     TORCH_CHECK(err == hipSuccess, "no LDS for expert tiles");
-    hipLaunchKernelGGL(kernel, grid, dim3(512), lds, cur_stream(), P<bf16_t>(x), w, first.data_ptr<int>(),
+    hipLaunchKernelGGL(kernel, grid, dim3(256), lds, cur_stream(), P<bf16_t>(x), w, first.data_ptr<int>(),
                        token.data_ptr<int>(), (const int2*)tiles.data_ptr<int>(), by_row, M<bf16_t>(y), max_tiles, group, 0, a, act);
   };
-#define TILES(KIND, BN, TOK) run(expert_tile_kernel<KIND, BN, TOK, W>, expert_lds<BN, TOK>())
-#define TILES_OF(KIND) if (half) TILES(KIND, 128, 128); else if (tile == 256) TILES(KIND, 256, 256); else TILES(KIND, 256, 128)
+  // where x takes 4 GB, offsets of gathered rows need more than 32 bits
+  const bool far = !of_own_row((int)kind) && (uint64_t)x.numel() * 2 >= 0xffffffffull;
+#define TILES(KIND, BN, TOK)                                                                                \
+  {                                                                                                         \
+    if (far) run(expert_tile_kernel<KIND, BN, TOK, !of_own_row(KIND), W>, expert_lds<BN, TOK>());            \
+    else run(expert_tile_kernel<KIND, BN, TOK, false, W>, expert_lds<BN, TOK>());                            \
+  }
+#define TILES_OF(KIND) if (half) TILES(KIND, 128, 128) else if (tile == 256) TILES(KIND, 256, 256) else TILES(KIND, 256, 128)
   if constexpr (std::is_same<W, Listed>::value) {
     if (kind == SWIGLU) { TILES_OF(SWIGLU); }
     else { TILES_OF(PLAIN); }
@@ -675,7 +701,7 @@ Tensor expert_product_of(Tensor x, std::vector<Tensor> w, Tensor token, Tensor f
   CHK(x.dim() == 2 && E >= 1 && E <= MOST_LISTED && ((size_t)x.data_ptr() & 15) == 0);
   for (const Tensor& t : {token, first, tiles}) check_io(t, torch::kInt32);
   const int K = x.size(1), pairs = token.numel(), F_ = w[0].size(0) / (swiglu ? 2 : 1);
-  CHK(first.numel() == E + 1 && K % 64 == 0 && F_ % 16 == 0 && (swiglu || x.size(0) == pairs));
+  CHK(first.numel() == E + 1 && K % 64 == 0 && K <= 1 << 22 && F_ % 16 == 0 && (swiglu || x.size(0) == pairs));
   Listed list{};
   for (int64_t e = 0; e < E; ++e) {
     check_io(w[e], torch::kBFloat16);
@@ -709,7 +735,7 @@ Tensor expert_product(Tensor x, Tensor w, Tensor token, Tensor first, Tensor til
   const hipStream_t stream = cur_stream();
   const int *fp = first.data_ptr<int>(), *tp = token.data_ptr<int>();
   // on average more than 24 rows per expert: weights are worth tiling
-  if (dt == torch::kBFloat16 && K % 8 == 0 && pairs > 24 * E) {
+  if (dt == torch::kBFloat16 && K % 8 == 0 && kp <= 1 << 22 && pairs > 24 * E) {
     launch_tiles(Stacked{P<bf16_t>(w)}, x, token, first, tiles, tile, kind, a, act, bp, y);
     return y;
   }
@@ -785,11 +811,11 @@ Tensor gate_product(Tensor x, Tensor w) {
   // panels of 2, 4, 6 and 8 tiles, us: 1500 rows of 3584 by 37888 326, 320, 315, 312; 6001 by
   // [28672, 4096] 1047, 1030, 1005, 1022; 3000 by [57344, 8192] 2114, 2058, 1988, 2022
   const int group = 6;
-  auto kernel = expert_tile_kernel<DENSE, 256, 256, Stacked>;
+  auto kernel = expert_tile_kernel<DENSE, 256, 256, false, Stacked>;
   constexpr int lds = expert_lds<256, 256>();
   const hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   TORCH_CHECK(err == hipSuccess, "no LDS for gate and up");
-  hipLaunchKernelGGL(kernel, dim3(((tiles * nf + 7) / 8 + DIE_CUS / 2) * 8), dim3(512), lds, cur_stream(), P<bf16_t>(x),
+  hipLaunchKernelGGL(kernel, dim3(((tiles * nf + 7) / 8 + DIE_CUS / 2) * 8), dim3(256), lds, cur_stream(), P<bf16_t>(x),
                      Stacked{P<bf16_t>(w)}, (const int*)nullptr, (const int*)nullptr, (const int2*)nullptr, (const float*)nullptr,
                      M<bf16_t>(y), tiles, group, (int)rows, GroupArgs{(int)K, (int)K, (int)F_, 1, (int)K, (int)F_}, Act{});
   return y;

@@ -10,10 +10,10 @@
 // transposing reads from LDS, so that nothing is transposed in memory. Where tiles are few
 // the sum is cut into parts, whose fp32 sums a second kernel adds up.
 //
-// us, library beside, weights from memory, 666 tokens: input [16384 -> 2048] 56 (117),
-// [128256 -> 2048] 328 (873); weights [16384, 2048] 54 (62), [2048, 2048] 10 (16); forward
-// [8192 -> 2048] 37 (42). 4096 tokens: weights [28672, 4096] 749 (825); input and forward of
-// it, which are the library's, 703 (722) and 730 (662).
+// us, library beside, weights from memory, 666 tokens: input [16384 -> 2048] 53 (117),
+// [128256 -> 2048] 318 (869); weights [16384, 2048] 51 (63), [2048, 2048] 11 (20), [3584, 3584]
+// 23 (32); forward [8192 -> 2048] 41 (43). 4096 tokens: weights [28672, 4096] 731 (812); input
+// and forward of it 666 (675) and 670 (599).
 #include "mfma_tile.h"
 
 struct GemmArgs {
@@ -27,15 +27,16 @@ struct GemmArgs {
 template <bool COL, int F, int COUNT>
 struct Source {
   static constexpr int SLOTS = F / 8, ROWS = COL ? 64 / SLOTS : 8;  // of a load: pieces of 16 bytes of a row, rows
-  const char* base;     // of the wave's first load of the sum's first step
-  size_t row, next;     // bytes from a k, and from a load, to the next
+  const char* base;     // of the tile, or of the wave's first load of columns, at the sum's first step
+  size_t row;           // bytes from a k to the next
+  unsigned next;        // and from a load of columns to the next
   unsigned off[COUNT];  // this lane's bytes besides
   DEVINL Source(const bf16_t* p, int f0, int free, int K, int wave, int lane) {
     const int load = wave * COUNT;
     if (COL) {
       base = (const char*)(p + (size_t)(load * ROWS) * free);
       row = (size_t)free * 2;
-      next = ROWS * row;
+      next = ROWS * free * 2;
 #pragma unroll
       for (int i = 0; i < COUNT; ++i) {
         const int slot = lane % SLOTS, f = f0 + (slot ^ col_turn((load + i) * ROWS + lane / SLOTS) << 1) * 8;
@@ -48,14 +49,19 @@ struct Source {
 #pragma unroll
       for (int i = 0; i < COUNT; ++i) {
         const int r = (load + i) * 8 + (lane >> 3);
-        off[i] = (min(r, free - 1 - f0) * K + ((lane & 7) ^ (r & 7)) * 8) * 2;
+        off[i] = ((unsigned)min(r, free - 1 - f0) * K + ((lane & 7) ^ (r & 7)) * 8) * 2;
       }
     }
   }
-  // number I of the step that begins at k
+  // the step that begins at k, if one is left: all of columns' rows may lie more than 4 GB apart
+  DEVINL StepSource step(int k, int left) const {
+    return COL ? StepSource(base + (k & StepSource::there(left)) * row, 0, left) : StepSource(base, k * 2, left);
+  }
+  // number I of it
   template <int I>
-  DEVINL void load(int k, char* to) const {
-    __builtin_amdgcn_global_load_lds((glb_void*)(base + k * row + I * next + off[I]), (lds_void*)to, 16, 0, 0);
+  DEVINL void load(StepSource from, char* to) const {
+    if (COL) from.at = I * next & from.mask;
+    from.load(off[I], to);
   }
 };
 
@@ -63,9 +69,11 @@ template <bool COL, int N, int F> struct Operand { typedef RowFrags<N> Frags; };
 template <int N, int F> struct Operand<true, N, F> { typedef ColFrags<N, F> Frags; };
 
 // A block has BN of N and BM of M; WN waves along N
+constexpr int WAVES = 8;  // blocks are few and short: see mfma_tile.h
+
 template <bool WCOL, bool XCOL, int BN, int BM, int WN, int WB, int XB, bool PARTS>
-__global__ __launch_bounds__(512) void gemm_kernel(GemmArgs a) {
-  typedef MfmaTile<BN, BM, WN, WB, XB> Sh;
+__global__ __launch_bounds__(WAVES * 64) void gemm_kernel(GemmArgs a) {
+  typedef MfmaTile<BN, BM, WN, WB, XB, WAVES> Sh;
   constexpr int R = Sh::R, C = Sh::C, WL = Sh::WL, XL = Sh::XL;
   extern __shared__ __attribute__((aligned(256))) bf16_t buf[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -82,40 +90,37 @@ __global__ __launch_bounds__(512) void gemm_kernel(GemmArgs a) {
   const Source<XCOL, BM, XL> xs(a.x, m0, a.M, a.K, wave, lane);
   // the last step of columns ends where they do: what the one before has too is left out
   const int skip = WCOL && XCOL && s1 == a.steps ? a.steps * 64 - a.K : 0;
-  auto loadw = [&](auto number, int s, unsigned to) {
+  auto k_of = [&](int s) { return WCOL && XCOL ? min((s0 + s) * 64, a.K - 64) : (s0 + s) * 64; };
+  auto stepw = [&](int s) { return ws.step(k_of(s), s1 - s0 - s); };
+  auto stepx = [&](int s) { return xs.step(k_of(s), s1 - s0 - s); };
+  auto loadw = [&](auto number, const StepSource& from, unsigned to) {
     constexpr int i = decltype(number)::value;
-    ws.template load<i>(WCOL && XCOL ? min((s0 + s) * 64, a.K - 64) : (s0 + s) * 64, (char*)buf + to + (wave * WL + i) * 1024);
+    ws.template load<i>(from, (char*)buf + to + (wave * WL + i) * 1024);
   };
-  auto loadx = [&](auto number, int s, unsigned to) {
+  auto loadx = [&](auto number, const StepSource& from, unsigned to) {
     constexpr int i = decltype(number)::value;
-    xs.template load<i>(WCOL && XCOL ? min((s0 + s) * 64, a.K - 64) : (s0 + s) * 64, (char*)buf + to + (wave * XL + i) * 1024);
+    xs.template load<i>(from, (char*)buf + to + (wave * XL + i) * 1024);
   };
   floatx4 acc[R][C];
-#pragma unroll
-  for (int i = 0; i < R; ++i)
-#pragma unroll
-    for (int j = 0; j < C; ++j) acc[i][j] = (floatx4)(0.f);
   const int wr = wave % WN * (R * 16), wx = wave / WN * (C * 16);
   const unsigned base = (unsigned)(size_t)(lds_void*)buf;
   walk<Sh>(acc, typename Operand<WCOL, R, BN>::Frags(base, wr, lane), typename Operand<XCOL, C, BM>::Frags(base + Sh::XAT, wx, lane),
-           s1 - s0, loadw, loadx, skip);
+           s1 - s0, stepw, loadw, stepx, loadx, skip);
+  typedef typename std::conditional<PARTS, float, bf16_t>::type Out;
+  const RowsOut<Out, R * 16> rows(buf, wave, lane);
+  const bool whole = a.N % (16 / sizeof(Out)) == 0;
 #pragma unroll
   for (int j = 0; j < C; ++j) {
-    const int m = m0 + wx + j * 16 + (lane & 15);
-    if (m >= a.M) continue;
 #pragma unroll
     for (int i = 0; i < R; ++i) {
-      const int n = n0 + wr + i * 16 + (lane >> 4) * 4;
-      if (n >= a.N) continue;
-      if (PARTS) {
-        *(floatx4*)((float*)a.y + ((size_t)split * a.M + m) * a.N + n) = acc[i][j];
-      } else {
-        float v[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = acc[i][j][r];
-        st4((bf16_t*)a.y + (size_t)m * a.N + n, v);
-      }
+      const int f = i * 16 + (lane >> 4) * 4;
+      if constexpr (PARTS) rows.put(lane & 15, f, acc[i][j]);
+      else rows.put(lane & 15, f, ushort4_t{f2b(acc[i][j][0]), f2b(acc[i][j][1]), f2b(acc[i][j][2]), f2b(acc[i][j][3])});
     }
+    rows.out([&](int r, int f, floatx4 v) {
+      const int m = m0 + wx + j * 16 + r, n = n0 + wr + f;
+      if (m < a.M) st_piece((Out*)a.y + ((size_t)split * a.M + m) * a.N + n, v, a.N - n, whole);
+    });
   }
 }
 
@@ -136,11 +141,11 @@ __global__ __launch_bounds__(256) void parts_kernel(const float* __restrict__ pa
 template <bool WCOL, bool XCOL, int BN, int BM, int WN, int WB, int XB>
 static void launch_gemm(const GemmArgs& a) {
   const int units = (a.N + BN - 1) / BN * ((a.M + BM - 1) / BM) * a.splits;
-  const int lds = MfmaTile<BN, BM, WN, WB, XB>::LDS;
+  const int lds = MfmaTile<BN, BM, WN, WB, XB, WAVES>::LDS;
   auto run = [&](auto kernel) {
     const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     TORCH_CHECK(e == hipSuccess, "no LDS for a product's tiles");
-    hipLaunchKernelGGL(kernel, dim3((units + 7) / 8 * 8), dim3(512), lds, cur_stream(), a);
+    hipLaunchKernelGGL(kernel, dim3((units + 7) / 8 * 8), dim3(WAVES * 64), lds, cur_stream(), a);
   };
   if (a.splits > 1) run(gemm_kernel<WCOL, XCOL, BN, BM, WN, WB, XB, true>);
   else run(gemm_kernel<WCOL, XCOL, BN, BM, WN, WB, XB, false>);

@@ -2,19 +2,29 @@
 // through two rings of LDS buffers, one for either operand: what the kernels share that
 // are bound by the matrix cores.
 //
-// Eight waves, two a SIMD. LDS rows hold 8 pieces of 16 bytes, piece p of row r at place
-// p ^ (r & 7): loads go straight to LDS lane by lane, so the permutation sits in the global
-// address, and fragment reads spread over the banks. A wave multiplies one half of a step
-// (32 of k) while it reads the fragments of the next half, so that matrix cores do not wait
-// for LDS: a step's last reads are over in the middle of it, where its one barrier lies,
-// and the loads that take its buffers are sent behind that. Weights come from farther than
-// x does and are sent further ahead: of 256 x 256, three buffers of weights and two of x
-// are the 160 KB that a CU has.
+// LDS rows hold 8 pieces of 16 bytes, piece p of row r at place p ^ (r & 7): loads go straight
+// to LDS lane by lane, so the permutation sits in the global address, and fragment reads spread
+// over the banks. A wave multiplies one half of a step (32 of k) while it reads the fragments
+// of the next half, so that matrix cores do not wait for LDS: a step's last reads are over in
+// the middle of it, where its one barrier lies, and the loads that take its buffers are sent
+// one by one over the step's length behind that. Weights come from farther than x does and
+// are sent further ahead: of 256 x 256, three buffers of weights and two of x are the 160 KB
+// that a CU has.
 //
-// [4096, 4096] x [28672, 4096]^T, 256 x 256 a block: 1.41 PFLOP/s (two buffers of both 1.35;
-// without any loads 1.74; matrix instructions alone 2.15). Four waves of 128 x 128 read
-// less of LDS and reach 1.30. Which blocks share a die's L2 counts as much: 1.32 where 32
-// neighbours read 32 weight tiles and one of x, 1.41 to 1.43 in patches of 4 by 8.
+// Four waves, one a SIMD, or eight: the larger a wave's part of a tile, the fewer fragments it
+// reads for a product, but two waves a SIMD begin and end a block faster. 256 blocks of 256 x
+// 256, of 512, 1024 and 4096 of k, us, four first: 22.1, 21.0; 33.7, 32.4; 100, 99; of 128 x
+// 256 14.4, 13.7; 20.5, 19.6; 58.1, 56.9; where both operands are columns of 256 x 256 25.0,
+// 21.9; 37.0, 33.1; 109, 104. Four where rows of x are a multiple of 32 alone, and where they
+// took less time.
+//
+// What bounds large tiles is power: [6144, 4096] x [28672, 4096]^T, 256 x 256 a block, takes
+// 2390 to 2500 cycles a step of the 2048 that its matrix instructions need, at 1.8 GHz of 2.4
+// (matrix instructions alone run at 2.1). PFLOP/s, four waves, and as it was with eight whose
+// loads took addresses in registers and whose results went out from them: 256 x 256 1.40
+// (1.34), 256 x 192 1.33 (1.26), one round of 160 x 256 1.11 (0.95). Which blocks share a die's
+// L2 counts as much: 1.32 where 32 neighbours read 32 weight tiles and one of x, 1.41 to 1.43
+// in patches of 4 by 8.
 #pragma once
 #include "common.h"
 
@@ -31,12 +41,42 @@ DEVINL void each(F&& f) { each_of(f, std::make_integer_sequence<int, N>()); }
 
 // BN weight rows and BM rows of x, WN waves along the weights; WB and XB buffers. A wave
 // has R x C tiles of 16.
-template <int BN, int BM, int WN, int WB_, int XB_>
+template <int BN, int BM, int WN, int WB_, int XB_, int WAVES_ = 4>
 struct MfmaTile {
-  static constexpr int WAVES = 8, R = BN / WN / 16, C = BM * WN / WAVES / 16;
-  static constexpr int WB = WB_, XB = XB_, WL = (BN / 8 + WAVES - 1) / WAVES, XL = BM / 8 / WAVES;  // 8 rows a load and wave
+  static constexpr int WAVES = WAVES_, THREADS = WAVES * 64, R = BN / WN / 16, C = BM * WN / WAVES / 16;
+  static constexpr int WB = WB_, XB = XB_, WL = BN / 8 / WAVES, XL = BM / 8 / WAVES;  // 8 rows a load and wave
   static constexpr int WBYTES = BN * 128, XBYTES = BM * 128, XAT = WB * WBYTES, LDS = XAT + XB * XBYTES;
-  static_assert(BN % (WN * 16) == 0 && BM * WN % (WAVES * 16) == 0 && BM % 64 == 0 && LDS <= 160 * 1024 && WB >= XB && XB >= 2, "");
+  static_assert(BN % (WN * 16) == 0 && BM * WN % (WAVES * 16) == 0 && BN % (8 * WAVES) == 0 && BM % (8 * WAVES) == 0 && LDS <= 160 * 1024, "");
+  static_assert(WB >= XB && XB >= 2 && C >= 2 && R * C >= 8, "");
+};
+
+// Where one step's loads come from, up to 4 GB from `base` on: a lane's offset stays in a
+// register and a step's is a scalar, so that a load takes no address of its own to compute
+// (64-bit addresses in registers cost 3% of a product). A step past the last is a buffer
+// without records, of which nothing is read; its offset is 0, as the hardware asks whether a
+// lane's offset lies past the records less the scalar, which would wrap round.
+struct StepSource {
+  const void* base;
+  unsigned at;  // bytes
+  int mask;     // -1; past the last step 0
+  DEVINL StepSource(const void* base_, unsigned at_, int left) : base(base_), mask(there(left)) { at = at_ & mask; }
+  // -1 where steps are left, else 0. By hand: of a comparison the compiler makes a vector, takes
+  // the buffer for another one in every lane, and loops over the lanes around each load.
+  static DEVINL int there(int left) {
+    int mask = 0;
+#ifdef __HIP_DEVICE_COMPILE__
+    asm("s_ashr_i32 %0, %1, 31" : "=s"(mask) : "s"(-left) : "scc");
+#endif
+    return mask;
+  }
+  // 16 bytes a lane to LDS. AUX 2: of lines that nobody reads again
+  template <int AUX = 0>
+  DEVINL void load(unsigned lane_at, void* to) const {
+#ifdef __HIP_DEVICE_COMPILE__  // the host's compiler does not know the type
+    const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, mask, 0x20000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lds_void*)to, 16, lane_at, at, 0, AUX);
+#endif
+  }
 };
 
 // One operand's fragments of 32 of k, N tiles of 16 rows, and where a lane reads them. By
@@ -114,93 +154,166 @@ struct ColFrags {
 };
 DEVINL void reads_landed() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
-// acc += over `steps` steps (one at least). loadw(i, s, at): this wave's load i of WL of
-// step s, to byte `at` of LDS, loadx the same; w, x: this lane's fragments (RowFrags or
+// Sums stay in the accumulation registers they are in. By hand: the compiler gives a wave's
+// 256 of them new places and moves them there, 20 moves and 16 waits a step (2780 cycles of
+// 256 x 256 in four waves, 2500 so). A sum's next is at least 8 of them later, and none follows closely
+// on something else that writes what it reads (`written`).
+DEVINL void mul(floatx4& sum, const bf16x8& a, const bf16x8& b) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(sum) : "v"(a), "v"(b));
+}
+// Two cycles between a write of registers and the instruction above
+DEVINL void written() { asm volatile("s_nop 1" ::: "memory"); }
+
+// acc = the sum over `steps` steps (one at least). stepw(s): where step s of the weights comes
+// from, loadw(i, that, at): this wave's load i of WL of it, to byte `at` of LDS; stepx and
+// loadx the same; steps past the last count as loads but have nothing to bring, so that one
+// loop does for all steps, and sums are never moved. w, x: this lane's fragments (RowFrags or
 // ColFrags), which read from the first buffers on; skip: k of the last step that do not count.
-template <typename T, int R, int C, typename W, typename X, typename LoadW, typename LoadX>
-DEVINL void walk(floatx4 (&acc)[R][C], W w, X x, int steps, LoadW loadw, LoadX loadx, int skip = 0) {
-  constexpr int WB = T::WB, XB = T::XB, WL = T::WL, XL = T::XL, AHEAD = WB - XB;
+// All of LDS is free when it returns.
+template <typename T, int R, int C, typename W, typename X, typename StepW, typename LoadW, typename StepX, typename LoadX>
+DEVINL void walk(floatx4 (&acc)[R][C], W w, X x, int steps, StepW stepw, LoadW loadw, StepX stepx, LoadX loadx, int skip = 0) {
+  constexpr int WB = T::WB, XB = T::XB, WL = T::WL, XL = T::XL, AHEAD = WB - XB, ALL = WL + XL;
+  // loads behind a row of products, and how many of a step's are sent before the next begins
+  constexpr int LPER = (ALL + 2 * R - 1) / (2 * R), NOW = ALL < LPER * R ? ALL : LPER * R;
+  // reads behind either half of a row: all of them in the first half of the rows
+  constexpr int READS = X::COUNT + W::COUNT, PER = ((READS + (R + 1) / 2 - 1) / ((R + 1) / 2) + 1) / 2;
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int j = 0; j < C; ++j) acc[i][j] = (floatx4)(0.f);
   W wa = w, wb = w;
   X xa = x, xb = x;
   // read number k of a half: x first
   auto read = [&](auto number, auto half, W& fw, X& fx, unsigned wring, unsigned xring) {
     constexpr int k = decltype(number)::value, h = decltype(half)::value;
     if constexpr (k < X::COUNT) fx.template read<k, h>(xring);
-    else if constexpr (k < X::COUNT + W::COUNT) fw.template read<k - X::COUNT, h>(wring);
+    else if constexpr (k < READS) fw.template read<k - X::COUNT, h>(wring);
+  };
+  // load number k of those that follow a step's barrier: x of a step, then weights of AHEAD
+  // steps later
+  auto load = [&](auto number, const auto& fromw, const auto& fromx, unsigned w0, unsigned x0) {
+    constexpr int k = decltype(number)::value;
+    if constexpr (k < XL) loadx(std::integral_constant<int, k>(), fromx, x0);
+    else if constexpr (k < ALL) loadw(std::integral_constant<int, k - XL>(), fromw, w0);
   };
   const std::integral_constant<int, 0> first;
   const std::integral_constant<int, 1> second;
-  auto send_w = [&](int s, unsigned at) { each<WL>([&](auto i) { loadw(i, s, at); }); };
-  auto send_x = [&](int s, unsigned at) { each<XL>([&](auto i) { loadx(i, s, at); }); };
-  // the order of the loads is that of the loop: x of a step, then weights of AHEAD steps later
 #pragma unroll
-  for (int s = 0; s < AHEAD; ++s)
-    if (s < steps) send_w(s, s * T::WBYTES);
-#pragma unroll
-  for (int s = 0; s < XB; ++s) {
-    if (s < steps) send_x(s, T::XAT + s * T::XBYTES);
-    if (s + AHEAD < steps) send_w(s + AHEAD, (s + AHEAD) * T::WBYTES);
+  for (int s = 0; s < AHEAD; ++s) {
+    const auto from = stepw(s);
+    each<WL>([&](auto i) { loadw(i, from, s * T::WBYTES); });
   }
+#pragma unroll
+  for (int s = 0; s < XB - 1; ++s) {
+    const auto fromw = stepw(s + AHEAD);
+    const auto fromx = stepx(s);
+    each<ALL>([&](auto k) { load(k, fromw, fromx, (s + AHEAD) * T::WBYTES, T::XAT + s * T::XBYTES); });
+  }
+  // the last buffers as if a step's barrier had been: what is over goes out in the first step
+  unsigned w0 = (WB - 1) * T::WBYTES, x0 = T::XAT + (XB - 1) * T::XBYTES;
+  auto fromw = stepw(WB - 1);
+  auto fromx = stepx(XB - 1);
+  each<NOW>([&](auto k) { load(k, fromw, fromx, w0, x0); });
   // loads that may still be on their way when the next step's have to be there
-  constexpr int LATER = (AHEAD ? WL : 0) + (XB - 2) * (XL + WL);
-  if (steps >= WB) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(LATER + XL + WL) : "memory");
-  else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-  constexpr int READS = X::COUNT + W::COUNT;
+  constexpr int LATER = (AHEAD ? WL : 0) + (XB - 2) * ALL;
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(LATER + NOW) : "memory");
   each<READS>([&](auto k) { read(k, first, wa, xa, 0, 0); });
-  // behind a row of products: all reads in the first half of them, all loads in as many rows
-  constexpr int PER = (2 * READS + R - 1) / R, LPER = (WL + XL + R - 1) / R;
   unsigned wu = 0, xu = 0;  // this step's buffers
-  // more: another step follows; fill: all loads go on
-  auto step = [&](int s, auto more, auto fill) {
+  // a row of products by fragments (fw, fx), reads into (gw, gx) between them
+  auto row = [&](auto number, W& fw, X& fx, W& gw, X& gx, auto half) {
+    constexpr int i = decltype(number)::value;
+    each<C>([&](auto column) {
+      constexpr int j = decltype(column)::value;
+      mul(acc[i][j], fw[i], fx[j]);
+      if constexpr (j == C / 2 - 1 || j == C - 1)
+        each<PER>([&](auto n) { read(std::integral_constant<int, (i * 2 + (j == C - 1)) * PER + decltype(n)::value>(), half, gw, gx, wu, xu); });
+    });
+  };
+  for (int s = 0; s < steps; ++s) {
     reads_landed();
     xa.landed();
     wa.landed();
-    if (!decltype(more)::value && skip > 0) {
+    if (skip > 0 && s + 1 == steps) {
       xa.clear(skip, 0, threadIdx.x & 63);
       wa.clear(skip, 0, threadIdx.x & 63);
     }
-    each<R>([&](auto row) {
-      constexpr int i = decltype(row)::value;
-#pragma unroll
-      for (int j = 0; j < C; ++j) acc[i][j] = mma(wa[i], xa[j], acc[i][j]);
-      each<PER>([&](auto n) { read(std::integral_constant<int, i * PER + decltype(n)::value>(), second, wb, xb, wu, xu); });
+    written();
+    each<R>([&](auto i) {
+      row(i, wa, xa, wb, xb, second);
+      each<LPER>([&](auto n) { load(std::integral_constant<int, NOW + decltype(i)::value * LPER + decltype(n)::value>(), fromw, fromx, w0, x0); });
       __builtin_amdgcn_sched_barrier(0);
     });
     reads_landed();
     xb.landed();
     wb.landed();
-    if (!decltype(more)::value && skip > 0) {
+    if (skip > 0 && s + 1 == steps) {
       xb.clear(skip, 1, threadIdx.x & 63);
       wb.clear(skip, 1, threadIdx.x & 63);
     }
-    const unsigned w0 = wu, x0 = T::XAT + xu;
-    if constexpr (decltype(more)::value) {
-      // all waves have read this step, and the next one is there
-      if constexpr (decltype(fill)::value) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(LATER) : "memory");
-      else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-      wu = wu == (WB - 1) * T::WBYTES ? 0 : wu + T::WBYTES;
-      xu = xu == (XB - 1) * T::XBYTES ? 0 : xu + T::XBYTES;
-      if (!decltype(fill)::value && s + XB < steps) send_x(s + XB, x0);
-    }
-    each<R>([&](auto row) {
-      constexpr int i = decltype(row)::value;
-#pragma unroll
-      for (int j = 0; j < C; ++j) acc[i][j] = mma(wb[i], xb[j], acc[i][j]);
-      if constexpr (decltype(more)::value)
-        each<PER>([&](auto n) { read(std::integral_constant<int, i * PER + decltype(n)::value>(), first, wa, xa, wu, xu); });
-      if constexpr (decltype(fill)::value)
-        each<LPER>([&](auto n) {
-          constexpr int k = i * LPER + decltype(n)::value;
-          if constexpr (k < XL) loadx(std::integral_constant<int, k>(), s + XB, x0);
-          else if constexpr (k < XL + WL) loadw(std::integral_constant<int, k - XL>(), s + WB, w0);
-        });
+    written();
+    // all waves have read this step, and the next one is there
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(LATER) : "memory");
+    w0 = wu;
+    x0 = T::XAT + xu;
+    wu = wu == (WB - 1) * T::WBYTES ? 0 : wu + T::WBYTES;
+    xu = xu == (XB - 1) * T::XBYTES ? 0 : xu + T::XBYTES;
+    fromw = stepw(s + WB);
+    fromx = stepx(s + XB);
+    each<R>([&](auto i) {
+      row(i, wb, xb, wa, xa, first);  // behind the last step of what nobody needs
+      each<LPER>([&](auto n) {
+        constexpr int k = decltype(i)::value * LPER + decltype(n)::value;
+        if constexpr (k < NOW) load(std::integral_constant<int, k>(), fromw, fromx, w0, x0);
+      });
       __builtin_amdgcn_sched_barrier(0);
     });
-  };
-  const std::true_type yes;
-  const std::false_type no;
-  int s = 0;
-  for (; s + WB < steps; ++s) step(s, yes, yes);
-  for (; s + 1 < steps; ++s) step(s, yes, no);
-  step(s, no, no);
+  }
+  // sums are written, and nothing is on its way to registers or LDS
+  asm volatile("s_nop 15\n\ts_nop 15\n\ts_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  xa.landed();
+  wa.landed();
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int j = 0; j < C; ++j) asm volatile("" : "+a"(acc[i][j]));
+  asm volatile("s_barrier" ::: "memory");
+}
+
+// A wave's results on their way out, ROWS rows of N features at a time: a lane holds four
+// features of a row, whose stores would be pieces of lines; by way of LDS they are whole ones.
+// 256 x 256 of bf16, all CUs at once: 8.6 us from registers, 3.4 so.
+template <typename T, int N, int ROWS = 16>
+struct RowsOut {
+  typedef __attribute__((ext_vector_type(4))) T four_t;
+  static constexpr int PER = 16 / sizeof(T), PIECES = N / PER, BYTES = ROWS * (N * sizeof(T) + 16), ROW = N * sizeof(T) + 16;  // numbers of a piece, pieces of a row
+  static_assert(N % PER == 0, "");
+  char* mine;
+  int lane;
+  DEVINL RowsOut(void* lds, int wave, int lane_) : mine((char*)lds + wave * BYTES), lane(lane_) {}
+  // row `r`, features f .. f + 3
+  DEVINL void put(int r, int f, four_t v) const { *(four_t*)(mine + r * ROW + f * sizeof(T)) = v; }
+  // to(row, feature, piece) for all of the rows; LDS operations of a wave are in order
+  template <typename To>
+  DEVINL void out(To to) const {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q0 = 0; q0 < ROWS * PIECES; q0 += 64) {
+      const int q = q0 + lane, r = q / PIECES, p = q % PIECES;
+      if (ROWS * PIECES % 64 == 0 || q < ROWS * PIECES) to(r, p * PER, *(const floatx4*)(mine + r * ROW + p * 16));
+    }
+    __builtin_amdgcn_sched_barrier(0);  // (the next rows' sums stay where they are meanwhile)
+  }
+};
+
+// A piece to `dst`, where `there` of its numbers have a place (some may have none); whole: rows are on 16 bytes
+template <typename T>
+DEVINL void st_piece(T* dst, floatx4 piece, int there, bool whole) {
+  constexpr int PER = 16 / sizeof(T);
+  if (whole && there >= PER) *(floatx4*)dst = piece;
+  else {
+    union { floatx4 v; T e[PER]; } u = {piece};
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      if (i < there) dst[i] = u.e[i];
+  }
 }

@@ -13,8 +13,8 @@
 // make too few blocks, k is split; the parts' fp32 sums are added by the kernel that
 // follows anyway (norm, activation).
 //
-// us, library beside: [3584, 18944] m 8 23 (46), m 32 23 (110), m 128 33 (99);
-// [8192, 28672] m 128 89 (201); [8192, 8192] m 128 29 (47); [4608, 3584] m 256 17 (36).
+// us, library beside: [3584, 18944] m 8 23 (46), m 32 23 (110), m 128 32 (99);
+// [8192, 28672] m 128 88 (201); [8192, 8192] m 128 28 (47); [4608, 3584] m 256 16 (36).
 //
 // How k is split depends on the weights' shape alone, and the order of the sums within
 // a part on the shape and the weight row: a row of these products does not depend on the
@@ -77,15 +77,10 @@ DEVINL void read_frags(unsigned a, unsigned b, bf16x8* r, bf16x8* c) {
   else if constexpr (R == 2 && C == 2)
     asm volatile(RD(0, 4, 0) RD(1, 4, 2048) RD(2, 5, 0) RD(3, 5, 2048) DONE
                  : "=&v"(r[0]), "=&v"(r[1]), "=&v"(c[0]), "=&v"(c[1]) : "v"(a), "v"(b));
-  else if constexpr (R == 4 && C == 2)
+  else {
+    static_assert(R == 4 && C == 2, "");
     asm volatile(RD(0, 6, 0) RD(1, 6, 2048) RD(2, 6, 4096) RD(3, 6, 6144) RD(4, 7, 0) RD(5, 7, 2048) DONE
                  : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(c[0]), "=&v"(c[1]) : "v"(a), "v"(b));
-  else {
-    static_assert(R == 4 && C == 4, "");
-    asm volatile(RD(0, 8, 0) RD(1, 8, 2048) RD(2, 8, 4096) RD(3, 8, 6144)
-                 RD(4, 9, 0) RD(5, 9, 2048) RD(6, 9, 4096) RD(7, 9, 6144) DONE
-                 : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(c[0]), "=&v"(c[1]), "=&v"(c[2]), "=&v"(c[3])
-                 : "v"(a), "v"(b));
   }
 #undef RD
 #undef DONE
@@ -245,53 +240,87 @@ __global__ __launch_bounds__((TileShape<BN, BM, BUFS>::WAVES * 64)) void tile_ke
   finish_tile<END, BN, R, C>(a, acc, tile, split, m0 + wx, wr, lane);
 }
 
-// The same of 65 to 256 rows of x, by mfma_tile.h: all of x in a block.
-template <int BN, int BM, int WN, int WB, int XB, int END>
-__global__ __launch_bounds__(512) void wide_kernel(TileArgs a) {
-  typedef MfmaTile<BN, BM, WN, WB, XB> Sh;
+// The same of 65 to 256 rows of x, by mfma_tile.h. With 256 rows the weights' way from memory
+// and that of x from L2 to every CU bound it: [37888, 3584] 46 us for the former alone, 61 for
+// both without products, 65 with them.
+template <int BN, int BM, int WN, int WB, int XB, int WAVES, int END>
+__global__ __launch_bounds__((WAVES * 64)) void wide_kernel(TileArgs a) {
+  typedef MfmaTile<BN, BM, WN, WB, XB, WAVES> Sh;
   constexpr int R = Sh::R, C = Sh::C, WL = Sh::WL, XL = Sh::XL, PER = END == GATED ? BN / 2 : BN;
   extern __shared__ __attribute__((aligned(16))) bf16_t buf[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int piece = ((lane & 7) ^ (lane >> 3)) * 8;
   read_args(a);
-  // blocks go round the eight dies: a die has a run of them, so that its L2 holds few parts of x
-  const int tiles = (a.N + PER - 1) / PER, units = tiles * a.splits, die = blockIdx.x & 7, rest = units & 7;
+  // blocks go round the eight dies, or a die has a run of them (run_tile); those of the same
+  // weights are neighbours
+  const int tiles = (a.N + PER - 1) / PER, mts = a.m > BM ? (a.m + BM - 1) / BM : 1, units = tiles * a.splits * mts;
+  const int die = blockIdx.x & 7, rest = units & 7;
   if ((int)(blockIdx.x >> 3) >= (units >> 3) + (die < rest)) return;
-  const int unit = die * (units >> 3) + min(die, rest) + (blockIdx.x >> 3), split = a.splits > 1 ? unit / tiles : 0;
-  const int tile = unit - split * tiles, s0 = part_at(a, split), s1 = part_at(a, split + 1);
-  const bf16_t *wsrc[WL], *xsrc[XL];
-  int wto[WL];
+  const int n = a.runs ? die * (units >> 3) + min(die, rest) + (blockIdx.x >> 3) : blockIdx.x, unit = mts > 1 ? n / mts : n, m0 = (n - unit * mts) * BM;
+  const int split = a.splits > 1 ? unit / tiles : 0, tile = unit - split * tiles, s0 = part_at(a, split), s1 = part_at(a, split + 1);
+  // GATED: 8 gate rows and the same 8 up rows in turn, of which a wave loads either
+  const int up = END == GATED ? wave / (WAVES / 2) : 0;
+  const bf16_t *wsrc = a.w + ((size_t)tile * PER + (up ? (size_t)a.N : 0)) * a.K + s0 * 64, *xsrc = a.x + (size_t)m0 * a.K + s0 * 64;
+  unsigned woff[WL], wto[WL], xoff[XL];
 #pragma unroll
-  for (int i = 0; i < WL; ++i) {  // past the last 8 rows: the same again
-    const int g = min(wave * WL + i, BN / 8 - 1), sub = lane >> 3;
-    // GATED: 8 gate rows and the same 8 up rows in turn
-    const size_t row = END == GATED ? min(tile * PER + (g >> 1) * 8 + sub, a.N - 1) + (g & 1 ? (size_t)a.N : 0)
-                                    : min(tile * PER + g * 8 + sub, a.N - 1);
-    wsrc[i] = a.w + row * a.K + s0 * 64 + piece;
-    wto[i] = g * 1024;
+  for (int i = 0; i < WL; ++i) {
+    const int g = END == GATED ? wave % (WAVES / 2) * WL + i : wave * WL + i;
+    woff[i] = ((unsigned)min(g * 8 + (lane >> 3), a.N - 1 - tile * PER) * a.K + piece) * 2;
+    wto[i] = (END == GATED ? g * 2 + up : g) * 1024;
   }
 #pragma unroll
-  for (int i = 0; i < XL; ++i)
-    xsrc[i] = a.x + (size_t)min((wave * XL + i) * 8 + (lane >> 3), a.m - 1) * a.K + s0 * 64 + piece;
+  for (int i = 0; i < XL; ++i) xoff[i] = ((unsigned)min((wave * XL + i) * 8 + (lane >> 3), a.m - 1 - m0) * a.K + piece) * 2;
   const int len = s1 - s0, turn = first_step<END>(a, tile * PER, len);
-  auto step = [&](int s) { return (s + turn < len ? s + turn : s + turn - len) * 64; };
-  auto loadw = [&](auto number, int s, unsigned at) {
+  auto step = [&](const bf16_t* p, int s) { return StepSource(p, (s + turn < len ? s + turn : s + turn - len) * 128, len - s); };
+  auto stepw = [&](int s) { return step(wsrc, s); };
+  auto stepx = [&](int s) { return step(xsrc, s); };
+  auto loadw = [&](auto number, const StepSource& from, unsigned at) {
     constexpr int i = decltype(number)::value;
-    __builtin_amdgcn_global_load_lds((glb_void*)(wsrc[i] + step(s)), (lds_void*)((char*)buf + at + wto[i]), 16, 0, 2);
+    from.load<2>(woff[i], (char*)buf + at + wto[i]);
   };
-  auto loadx = [&](auto number, int s, unsigned at) {
+  auto loadx = [&](auto number, const StepSource& from, unsigned at) {
     constexpr int i = decltype(number)::value;
-    __builtin_amdgcn_global_load_lds((glb_void*)(xsrc[i] + step(s)), (lds_void*)((char*)buf + at + (wave * XL + i) * 1024), 16, 0, 0);
+    from.load(xoff[i], (char*)buf + at + (wave * XL + i) * 1024);
   };
   floatx4 acc[R][C];
-#pragma unroll
-  for (int i = 0; i < R; ++i)
-#pragma unroll
-    for (int j = 0; j < C; ++j) acc[i][j] = (floatx4)(0.f);
-  const int wr = wave % WN * (R * 16), wx = wave / WN * (C * 16);
+  const int wr = wave % WN * (R * 16), wx = wave / WN * (C * 16), col = lane & 15, quad = lane >> 4;
   const unsigned base = (unsigned)(size_t)(lds_void*)buf;
-  walk<Sh>(acc, RowFrags<R>(base, wr, lane), RowFrags<C>(base + Sh::XAT, wx, lane), len, loadw, loadx);
-  finish_tile<END, BN, R, C>(a, acc, tile, split, wx, wr, lane);
+  walk<Sh>(acc, RowFrags<R>(base, wr, lane), RowFrags<C>(base + Sh::XAT, wx, lane), len, stepw, loadw, stepx, loadx);
+  typedef typename std::conditional<END == PART, float, bf16_t>::type Out;
+  // GATED: two tiles of x at a time. Lanes of quads 0 and 1 hold gates, those of 2 and 3 the
+  // products of up; changed round, lanes have both, the lower half those of the first tile.
+  constexpr int N = END == GATED ? R * 8 : R * 16, PAIR = END == GATED ? 2 : 1;
+  static_assert(C % PAIR == 0, "");
+  const RowsOut<Out, N, PAIR * 16> rows(buf, wave, lane);
+  const int n0 = tile * PER + (END == GATED ? wr / 2 : wr);
+  const bool whole = a.N % (16 / sizeof(Out)) == 0;
+#pragma unroll
+  for (int j = 0; j < C; j += PAIR) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      if constexpr (END == GATED) {
+        ushort4_t v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[i][j][r]), __float_as_uint(acc[i][j + 1][r]), false, false);
+          v[r] = f2b(siluf(rounded(__uint_as_float(both[0]))) * rounded(__uint_as_float(both[1])));
+        }
+        rows.put((quad >> 1) * 16 + col, i * 8 + (quad & 1) * 4, v);
+      } else if constexpr (END == PART) {
+        rows.put(col, i * 16 + quad * 4, acc[i][j]);
+      } else {
+        const int n = n0 + i * 16 + quad * 4;
+        ushort4_t v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = f2b(acc[i][j][r] + (a.bias && n + r < a.N ? ld(a.bias + n + r) : 0.f));
+        rows.put(col, i * 16 + quad * 4, v);
+      }
+    }
+    rows.out([&](int r, int f, floatx4 v) {
+      const int m = m0 + wx + j * 16 + r;
+      if (m < a.m) st_piece((Out*)a.y + ((size_t)split * a.m + m) * a.N + n0 + f, v, a.N - n0 - f, whole);
+    });
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -393,18 +422,23 @@ static void launch_tile(TileArgs a) {
 // [N, K], 64-row or (deeper, fewer to a CU) first:
 //   m 32: [2048, 2048] in 128 blocks 4.1, 4.6; [3584, 18944] in 224 25.0, 22.6
 //   m 64: [2048, 2048] 4.6, 5.6; [28672 -> 8192] 91.0, 78.3
-//   m 128, 3 and 2 buffers: [8192, 8192] in 256 29.5, 36.5; gate [57344, 8192] in 448, now
-//   in other tiles, 193, 176
-// From 129 rows of x on all of them in one block (wide_kernel), if k is split in enough
-// parts: m 256, and 136 by 192 rows, us, with 128 rows a block: [3584, 18944] in 224 41.7
-// and 33.9 (53.6 and 51.1); [28672 -> 8192] 119 and 98 (148 and 159); with fewer blocks a
-// block's start outweighs it, [2048, 2048] in 128 11.7 (8.8).
+// From 65 rows of x on by mfma_tile.h, all rows in one block. Up to 128: where blocks make one
+// round and their sums are long, four waves and more on the way, else eight, two blocks to a
+// CU; us, the former first (and by the loop above, m 128):
+//   m 96 and 128: [8192, 28672] 79 and 87, 82 and 90 (89); gate [28672, 4096] 42 and 46, 51
+//   and 50 (49); [3584, 3584] 10.2 and 11.0, 9.7 and 10.5 (11.2); [50304, 2048] in 393 blocks
+//   m 128 58, 51 (53); gate [35840, 8192] in 280 blocks m 66 135, 129 (166)
+// More rows in eight waves where they can be (from registers and with eight waves of the loop
+// before: m 256 [3584, 3584] 15.7, now 14.4; [1536, 8960] 19.0, 14.9; [8192, 8192] 38.6,
+// 37.1); with blocks for half of the chip and less, in two blocks of 128 ([2048, 2048] 8.8,
+// in one 10.2).
 //
 // The gated product of more than 64 rows takes the weight tile that makes one round of the
-// chip's 256 CUs, if there is one: [37888, 3584] 237 blocks of 160 rows 70 with m 256 (library
-// and activation 84; 296 of 128 120, 148 of 256 83), [57344, 8192] 224 of 256 211 (220; 448 of
-// 128 235). Up to 128 rows, whose matrix products are short, 148 blocks of 256 are enough:
-// 63 with m 128 (73; 78).
+// chip's 256 CUs, if there is one: [37888, 3584] 237 blocks of 160 rows 65 with m 256, 57
+// with 136 (library and activation 84; waves of 80 by 128 68; 296 blocks of 128 120, 148 of
+// 256 77); [57344, 8192] 224 of 256 196 with m 256 (220; 448 of 128 235), 165 with 192 in
+// tiles that have no more (in those of 256 200). Up to 128 rows, whose matrix products are
+// short, 148 blocks of 256 are enough: 63 with m 128 (73; 78).
 static int gate_tile(int rows, int m) {
   if (m <= 128) return rows > 143 * 256 && rows <= 256 * 256 ? 256 : 0;
   for (int tile : {128, 160, 256})
@@ -412,13 +446,13 @@ static int gate_tile(int rows, int m) {
   return 0;
 }
 
-template <int BN, int BM, int WN, int WB, int XB, int END>
+template <int BN, int BM, int WN, int WB, int XB, int WAVES, int END>
 static void launch_wide(const TileArgs& a) {
-  const auto kernel = wide_kernel<BN, BM, WN, WB, XB, END>;
-  const int lds = MfmaTile<BN, BM, WN, WB, XB>::LDS, per = END == GATED ? BN / 2 : BN;
+  const auto kernel = wide_kernel<BN, BM, WN, WB, XB, WAVES, END>;
+  const int lds = MfmaTile<BN, BM, WN, WB, XB, WAVES>::LDS, per = END == GATED ? BN / 2 : BN;
   const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   TORCH_CHECK(e == hipSuccess, "no LDS for weight tiles");
-  hipLaunchKernelGGL(kernel, dim3(((a.N + per - 1) / per * a.splits + 7) / 8 * 8), dim3(512), lds, cur_stream(), a);
+  hipLaunchKernelGGL(kernel, dim3(((a.N + per - 1) / per * a.splits * ((a.m + BM - 1) / BM) + 7) / 8 * 8), dim3(WAVES * 64), lds, cur_stream(), a);
 }
 
 // Whether blocks begin at different places of k (first_step): by the weights' shape alone
@@ -431,12 +465,16 @@ static void run_tile(TileArgs a) {
   a.whole = a.K / 64 / a.splits;
   a.more = a.K / 64 % a.splits;
   a.inv = 65536 / a.splits + 1;
-  // x larger than a die's L2 has room for beside the weights. us, the grid's parts first:
-  // m 128 by [4096, 14336] 29.2, 28.2; by [3584, 18944] 32.7, 32.2; by [8192, 28672] 90 both;
-  // with x of 0.5 MB no matter, [16384, 2048] 17.5, 17.3
-  a.runs = END == PART && (int64_t)a.m * a.K > 1 << 20;
   const int rows = END == GATED ? 2 * a.N : a.N, units = (rows + 127) / 128 * a.splits;
   a.turned = !turns(a.K, a.splits) ? 0 : gate_tile(rows, 256) == 160 ? 640 : 128;
+  // Whether a die has a run of blocks, and so few parts of x, where x is larger than its L2 has
+  // room for beside the weights; else blocks go round the dies, which spreads what the next
+  // kernel reads. us, going round first: m 32 by [8192, 28672] 77.4, 76.3; with the norm that
+  // follows, m 256 by [3584, 3584] 21.6, 25.3; [1536, 8960] 22.9, 25.8; m 192 by [3584, 18944]
+  // 41.8, 43.6; [4096, 14336], whose blocks begin at different places, 40.0, 38.7; m 256
+  // 46.8, 42.0; [8192, 28672] 125, 120
+  const int64_t x = (int64_t)a.m * a.K;
+  a.runs = END == PART ? x > (a.m <= 64 ? 2 << 19 : a.turned ? 3 << 19 : 7 << 19) : a.m > 64;
   if (a.m <= 16) launch_tile<64, 16, 4, END>(a);
   else if (a.m <= 32) {
     if (units >= 200) launch_tile<128, 32, 4, END>(a);
@@ -444,18 +482,22 @@ static void run_tile(TileArgs a) {
   } else if (a.m <= 64) {
     if (units >= 200) launch_tile<128, 64, 3, END>(a);
     else launch_tile<64, 64, 4, END>(a);
+  } else if (a.K > 1 << 22) {  // offsets of 256 rows take more than 32 bits
+    launch_tile<128, 64, 3, END>(a);
   } else {
     if constexpr (END == GATED) {
       const int wide = gate_tile(rows, a.m);
-      if (wide == 256 && a.m <= 128) return launch_wide<256, 128, 4, 4, 2, END>(a);
-      if (wide == 256) return launch_wide<256, 256, 2, 3, 2, END>(a);
-      if (wide == 160) return launch_wide<160, 256, 2, 3, 3, END>(a);
+      if (wide == 256 && a.m <= 128) return launch_wide<256, 128, 4, 4, 2, 4, END>(a);
+      if (wide == 256 && a.m <= 192) return launch_wide<256, 192, 2, 3, 2, 4, END>(a);
+      if (wide == 256) return launch_wide<256, 256, 2, 3, 2, 4, END>(a);
+      if (wide == 160) return launch_wide<160, 256, 1, 3, 3, 4, END>(a);
     }
-    if (a.m > 128 && units >= 200) {
-      if (a.m <= 192) launch_wide<128, 192, 2, 4, 4, END>(a);
-      else launch_wide<128, 256, 2, 3, 3, END>(a);
-    } else if (units * ((a.m + 127) / 128) > 288) launch_tile<128, 128, 2, END>(a);
-    else launch_tile<128, 128, 3, END>(a);
+    if (a.m <= 128 || units < 160) {
+      if (a.m <= 128 && units <= 256 && a.whole > 24) launch_wide<128, 128, 2, 4, 3, 4, END>(a);
+      else launch_wide<128, 128, 4, 3, 2, 8, END>(a);
+    } else if (a.m > 192) launch_wide<128, 256, 2, 3, 3, 8, END>(a);
+    else if constexpr (END == GATED) launch_wide<128, 192, 2, 4, 4, 4, END>(a);
+    else launch_wide<128, 192, 2, 4, 4, 8, END>(a);
   }
 }
 
