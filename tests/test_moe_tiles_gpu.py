@@ -126,6 +126,34 @@ def test_shares_of_rows_in_steps_of_32(rows, swiglu):
   assert bool(((got[:rows[0]].double() - want).abs() <= want.abs() * 2.0 ** -8 + size * size * K * 2.0 ** -22).all())
 
 
+@pytest.mark.parametrize("experts,F", [(1, 2048), (8, 4096), (65, 272), (130, 48), (250, 16)])  # one, some or many a lane
+def test_tiles_that_the_kernel_plans(experts, F):
+  """Few rounds of blocks: whatever rows a tile has, each row is what its expert gives it alone."""
+  from xotorch_amd.ops.mixer_ops import load_hip
+  hip = load_hip("_hip_experts")
+  g, K = torch.Generator(device="cuda").manual_seed(experts), 64
+  sizes = [0, 1, 100, 128, 129, 190, 193, 256, 257, 300, 384, 385]
+  w = [(torch.randn(F, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16) for _ in range(experts)]
+  ints = dict(dtype=torch.int32, device="cuda")
+  for spread in range(4):
+    if spread == 3: counts = [sizes[(5 * e) % len(sizes)] for e in range(experts)]
+    else: counts = [(260, 390, 150)[spread] + e % 3 for e in range(experts)]
+    first = [0]
+    for c in counts:
+      first.append(first[-1] + c)
+    pairs = first[-1]
+    if pairs == 0: continue
+    x = torch.randn(pairs, K, generator=g, device="cuda").to(torch.bfloat16)
+    tiles = [(e, r) for e in range(experts) for r in range(first[e], first[e + 1], 256)]
+    listed = tiles + [(-1, 0)] * (pairs // 256 + experts - len(tiles)) + [(-1, len(tiles))]
+    got = hip.expert_product_of(x, w, torch.arange(pairs, **ints), torch.tensor(first, **ints), torch.tensor(listed, **ints), 256, False)
+    for e in range(experts):
+      rows = x[first[e]:first[e + 1]].double()
+      want, size = rows @ w[e].double().t(), rows.abs() @ w[e].double().abs().t()
+      slack = size * (K + 8) * 2.0 ** -24 + want.abs() * 2.0 ** -8 + 1e-30  # fp32 sums of K products
+      assert bool(((got[first[e]:first[e + 1]].double() - want).abs() <= slack).all()), (spread, e, counts[e])
+
+
 def test_tokens_past_four_gigabytes():
   """Offsets of more than 32 bits, of the last tokens of all."""
   from xotorch_amd.ops.mixer_ops import load_hip

@@ -365,9 +365,9 @@ __global__ __launch_bounds__(256) void expert_stream_kernel(
 // Many tokens per expert (bf16): up to TOK tokens x BN weight rows (GATED: BN / 2 gate and
 // the same of up) per block, by mfma_tile.h. What bounds them is the matrix cores, and
 // rows of a tile that no token fills: an expert's rows go over its tiles evenly, in steps
-// of 32. 8 experts of 4096 x 14336, two of them a token, both products, us: 2100 tokens 1365
-// (in steps of 64 by eight waves 1420), 1500 911 (1018), 1000 814 (852), 500 548 (590), 300 553
-// (560).
+// of 32. 8 experts of 4096 x 14336, two of them a token, both products, us: 2100 tokens 1340
+// (in steps of 64 by eight waves 1480), 1500 939 (1069), 1000 776 (855), 500 560 (598), 300 538
+// (557). Up to 700 tokens the weights bound them, at some 4.5 TB/s.
 
 // Where an expert's weight rows lie: in one tensor, or in one tensor each
 struct Stacked {
@@ -474,22 +474,72 @@ DEVINL void expert_tile(const bf16_t* __restrict__ x, const bf16_t* __restrict__
 
 constexpr int DIE_CUS = 32;  // of one of the eight dies
 
-// The router's tiles, of which there are as many as the last of `tiles` says; DENSE: max_tiles of rows_of_all rows
+// Most rows of a tile, how many tiles that makes of all experts' rows, and where this lane's
+// experts end among them
+struct Plan { int most, tiles, end; };
+DEVINL int tiles_of(unsigned rows, int most) {
+  return most == 256 ? (rows + 255) / 256 : most == 192 ? (rows + 191) / 192 : (rows + 127) / 128;
+}
+// Where the chip has few rounds of blocks, what the last of them leaves idle counts for more
+// than what smaller tiles cost: 256, 192 or 128 rows, by the time that the rounds take, of
+// which a block of n rows takes 0.4 + 0.00375 n, cut in two 0.62 of that. All blocks find
+// the same. us of the down product of 8 experts of 4096 x 14336, two of them a token, with 256
+// and so: 2100 tokens 486, 443; 1000 tokens 305, 246; 1500 and 700, which stay with 256, 301
+// and 214.
+DEVINL Plan plan_of(const int* __restrict__ first, int E, int nf, int lane) {
+  const int per = (E + 63) / 64, e0 = min(lane * per, E), e1 = min(e0 + per, E);
+  int found = 0, tiles = 0, end = 0;
+  float least = 0.f;
+#pragma unroll
+  for (int most : {256, 192, 128}) {
+    int mine = 0;
+    float tall = 0.f;
+    for (int e = e0; e < e1; ++e) {
+      const int rows = first[e + 1] - first[e], n = tiles_of(rows, most);
+      mine += n;
+      if (n) tall = fmaxf(tall, (float)rows / (float)n);
+    }
+    int sum = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int other = __shfl_up(sum, d);
+      if (lane >= d) sum += other;
+      tall = fmaxf(tall, __shfl_xor(tall, d));
+    }
+    const int all = __shfl(sum, 63);
+    const unsigned blocks = all * nf, left = blocks % 256;
+    const float each = 0.4f + 0.00375f * (float)first[E] / (float)max(all, 1), last = 0.4f + 0.00375f * tall;
+    const float time = (float)(blocks / 256) * each + (left == 0 ? 0.f : left <= 128 ? 0.62f * last : last);
+    if (most == 256 || time < 0.97f * least) found = most, tiles = all, end = sum, least = time;
+  }
+  return {found, tiles, end};
+}
+
+// The router's tiles, of which there are as many as the last of `tiles` says, or (replan) those
+// of plan_of; DENSE: max_tiles of rows_of_all rows
 template <int KIND, int BN, int TOK, bool FAR, typename W>
 __global__ __launch_bounds__(256) void expert_tile_kernel(
     const bf16_t* __restrict__ x, W w, const int* __restrict__ first,
     const int* __restrict__ token, const int2* __restrict__ tiles, const float* __restrict__ by_row,
-    bf16_t* __restrict__ y, int max_tiles, int group, int rows_of_all, GroupArgs a, Act act) {
+    bf16_t* __restrict__ y, int max_tiles, int group, int rows_of_all, bool replan, GroupArgs a, Act act) {
   extern __shared__ __attribute__((aligned(16))) bf16_t buf[];
   // blocks go round the eight dies: a die has a run of them, in panels of `group` tiles
   // whose weight rows come one after the other, so that its L2 serves both operands
   constexpr bool TWO = has_gate(KIND);
   constexpr int WIDE = TWO ? BN / 2 : BN;
-  const int nf = (a.F + WIDE - 1) / WIDE, real = KIND == DENSE ? max_tiles : __builtin_amdgcn_readfirstlane(tiles[max_tiles].y);
-  const int die = blockIdx.x & 7, each = real * nf / 8, rest = real * nf % 8, all = each + (die < rest);
+  constexpr bool CUT = BN == 256 && TOK == 256;  // (up to 128 tokens gain nothing)
+  const int nf = (a.F + WIDE - 1) / WIDE, lane = threadIdx.x & 63;
+  Plan plan{TOK, 0, 0};
+  if constexpr (KIND == DENSE) plan.tiles = max_tiles;
+  else if (CUT && replan) {
+    plan = plan_of(first, a.E, nf, lane);
+    plan.most = __builtin_amdgcn_readfirstlane(plan.most);
+    plan.tiles = __builtin_amdgcn_readfirstlane(plan.tiles);
+    group = __builtin_amdgcn_readfirstlane(first[a.E]) / (a.E * plan.most) + 1;
+  } else plan.tiles = __builtin_amdgcn_readfirstlane(tiles[max_tiles].y);
+  const int real = plan.tiles, die = blockIdx.x & 7, each = real * nf / 8, rest = real * nf % 8, all = each + (die < rest);
   // what no more than half of a die's 32 CUs would have left to do is cut in two: 384 blocks
-  // of the down product of 2100 tokens 578 us, so 522 (with up to 128 tokens nothing, to 3% worse)
-  constexpr bool CUT = BN == 256 && TOK == 256;
+  // of the down product of 2100 tokens 578 us, so 522
   const int whole = CUT && all % DIE_CUS <= DIE_CUS / 2 ? all - all % DIE_CUS : all;
   int at = blockIdx.x >> 3, half = -1;
   if (at >= whole) {
@@ -501,13 +551,25 @@ __global__ __launch_bounds__(256) void expert_tile_kernel(
   const int wide = min(group, real - panel * group), m = panel * group + in % wide, fb = in / wide;
   int e = 0, lo = 0, end = rows_of_all, nth = m;
   if constexpr (KIND != DENSE) {
-    const int2 tile = tiles[m];
-    e = __builtin_amdgcn_readfirstlane(tile.x);
-    lo = __builtin_amdgcn_readfirstlane(first[e]), end = __builtin_amdgcn_readfirstlane(first[e + 1]);
-    nth = (__builtin_amdgcn_readfirstlane(tile.y) - lo) / TOK;
+    if (CUT && replan) {
+      // the first lane whose experts' tiles end behind m, and its expert
+      const int owner = __popcll(__ballot(plan.end <= m)), of_lane = (a.E + 63) / 64;
+      nth = m - (owner ? __builtin_amdgcn_readlane(plan.end, owner - 1) : 0);
+      for (e = owner * of_lane;; ++e) {
+        lo = __builtin_amdgcn_readfirstlane(first[e]), end = __builtin_amdgcn_readfirstlane(first[e + 1]);
+        const int tiles_here = tiles_of(end - lo, plan.most);
+        if (nth < tiles_here || e + 1 >= a.E) break;
+        nth -= tiles_here;
+      }
+    } else {
+      const int2 tile = tiles[m];
+      e = __builtin_amdgcn_readfirstlane(tile.x);
+      lo = __builtin_amdgcn_readfirstlane(first[e]), end = __builtin_amdgcn_readfirstlane(first[e + 1]);
+      nth = (__builtin_amdgcn_readfirstlane(tile.y) - lo) / TOK;
+    }
   }
   // an expert's rows go over its tiles evenly, in steps of 32
-  const int of = (end - lo + TOK - 1) / TOK, share = ((end - lo + of - 1) / of + 31) / 32 * 32;
+  const int of = CUT ? tiles_of(end - lo, plan.most) : (end - lo + TOK - 1) / TOK, share = ((end - lo + of - 1) / of + 31) / 32 * 32;
   const int r0 = lo + nth * share, hi = min(end, r0 + share), rows = hi - r0;
   const bf16_t* we = w.of(e, (size_t)(TWO ? 2 : 1) * a.F * a.kp);
   constexpr bool TAIL = std::is_same<W, Stacked>::value && KIND != DENSE;
@@ -663,15 +725,21 @@ static void launch_tiles(const W& w, const Tensor& x, const Tensor& token, const
   // tokens (1000 rows) 1590, 1504
   const int group = pairs / (a.E * (int)tile) + 1;
   // few rows an expert: blocks of 128 weight rows, two to a CU, keep more of them on their
-  // way: 25 and 50 rows 491 and 509 us (553 and 570 with 256); from 75 on 609 (589)
-  const bool half = tile == 128 && pairs <= 56 * a.E;
+  // way: 25 and 50 rows 491 and 509 us (553 and 570 with 256); from 75 on 609 (589). So do as
+  // many blocks as CUs, where 256 weight rows make half of that: down of 8 experts of 4096 x
+  // 14336, 75 and 100 rows each, 200 and 208 us (216 and 229)
+  const bool half = tile == 128 && (pairs <= 56 * a.E || (int64_t)(pairs / 128 + a.E) * ((rows + 255) / 256) <= 256);
   const int bn = half ? 128 : 256, nf = (rows + bn - 1) / bn;
-  const dim3 grid(((max_tiles * nf + 7) / 8 + (tile == 256 ? DIE_CUS / 2 : 0)) * 8);
+  // up to some two rounds of the chip are planned by the kernel, which may make tiles of 128 rows
+  // of them (more of them lose by the wider grid: gate and up of 700 tokens 364, 378)
+  const bool replan = tile == 256 && (int64_t)(pairs / 256 + a.E / 2) * nf < 640;
+  const int most_tiles = replan ? pairs / 128 + std::min(pairs, a.E) : max_tiles;
+  const dim3 grid(((most_tiles * nf + 7) / 8 + (tile == 256 ? DIE_CUS / 2 : 0)) * 8);
   auto run = [&](auto kernel, int lds) {
     const hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     TORCH_CHECK(err == hipSuccess, "no LDS for expert tiles");
     hipLaunchKernelGGL(kernel, grid, dim3(256), lds, cur_stream(), P<bf16_t>(x), w, first.data_ptr<int>(),
-                       token.data_ptr<int>(), (const int2*)tiles.data_ptr<int>(), by_row, M<bf16_t>(y), max_tiles, group, 0, a, act);
+                       token.data_ptr<int>(), (const int2*)tiles.data_ptr<int>(), by_row, M<bf16_t>(y), max_tiles, group, 0, replan, a, act);
   };
   // where x takes 4 GB, offsets of gathered rows need more than 32 bits
   const bool far = !of_own_row((int)kind) && (uint64_t)x.numel() * 2 >= 0xffffffffull;
@@ -817,7 +885,7 @@ Tensor gate_product(Tensor x, Tensor w) {
   TORCH_CHECK(err == hipSuccess, "no LDS for gate and up");
   hipLaunchKernelGGL(kernel, dim3(((tiles * nf + 7) / 8 + DIE_CUS / 2) * 8), dim3(256), lds, cur_stream(), P<bf16_t>(x),
                      Stacked{P<bf16_t>(w)}, (const int*)nullptr, (const int*)nullptr, (const int2*)nullptr, (const float*)nullptr,
-                     M<bf16_t>(y), tiles, group, (int)rows, GroupArgs{(int)K, (int)K, (int)F_, 1, (int)K, (int)F_}, Act{});
+                     M<bf16_t>(y), tiles, group, (int)rows, false, GroupArgs{(int)K, (int)K, (int)F_, 1, (int)K, (int)F_}, Act{});
   return y;
 }
 
