@@ -117,6 +117,14 @@ def test_the_rules_know_how_k_is_split():
 
 
 @pytest.mark.gpu
+def test_the_rules_know_how_k_of_gates_is_split():
+  from xotorch_amd import ops
+  for N in (16, 1024, 10176, 10192, 16384, 16400, 20416, 20480, 20496, 28672, 1 << 26):
+    for K in (64, 1024, 1088, 2048, 2112, 6144, 6208, 53248):
+      assert ops.gate_splits(N, K) == ops._tile().gate_splits(N, K)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows", [136, 200, 256])
 def test_the_rules_know_which_gated_tiles_make_a_round(rows):
   from xotorch_amd import ops

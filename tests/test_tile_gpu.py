@@ -93,6 +93,28 @@ def test_gated_products_of_one_round(m, N, K):
   assert bool(((y - act * u).abs() <= bound + 1e-30).all())
 
 
+# 64 weight rows a block: a feature, a tile and a round of them less, just so and more; rows of
+# x of one tile and of several; whole rows 2 KB and 4 KB apart
+@pytest.mark.parametrize("N,K", [(16, 64), (72, 1024), (2056, 704), (10256, 2048), (16384, 2048), (16400, 128), (9728, 896)])
+def test_gated_products_of_whole_rows(N, K):
+  from xotorch_amd import ops
+  assert ops._tile().gate_splits(N, K) == 1
+  x, w, _ = _inputs(256, N, K)
+  ref = x.double() @ w.double().t()
+  size = x.double().abs() @ w.double().abs().t()
+  with torch.no_grad():
+    all_rows = ops.tile_swiglu(x, w)
+    for m in (3, 17, 33, 64, 65, 100, 128, 129, 193):
+      assert torch.equal(ops.tile_swiglu(x[:m].contiguous(), w), all_rows[:m])
+  gate, up = ref.chunk(2, -1)
+  # each product is rounded to 8 bits after fp32 sums of K; silu's slope is at most 1.1
+  by = 2.0 ** -8
+  dg, du = (p.abs() * by + s * (K + 8) * 2.0 ** -24 for p, s in zip(ref.chunk(2, -1), size.chunk(2, -1)))
+  act = torch.nn.functional.silu(gate)
+  slack = (1.1 * dg + gate.abs() * 2.0 ** -19) * (up.abs() + du) + act.abs() * du + (act * up).abs() * by
+  assert bool(((all_rows.double() - act * up).abs() <= slack + 1e-30).all())
+
+
 @pytest.mark.parametrize("m,D,H,I", [(3, 64, 128, 192), (45, 2048, 2048, 8192), (200, 320, 192, 512)])
 def test_rest_of_a_layer_is_its_parts(m, D, H, I):
   from xotorch_amd import ops

@@ -382,6 +382,14 @@ def tile_splits(N: int, K: int) -> int:
 
 
 @functools.lru_cache(maxsize=1024)
+def gate_splits(N: int, K: int) -> int:
+  """The same of the gated product of N weight rows (gate_splits in hip/tile_ops.hip)."""
+  tiles = -(-N // 64)
+  whole = K <= 1024 or (tiles >= 160 and K <= (2048 if 256 < tiles < 320 else 6144))
+  return 1 if whole else tile_splits(N, K)
+
+
+@functools.lru_cache(maxsize=1024)
 def _one_round(N: int, K: int) -> bool:
   """Whether k is split in three or more and the blocks of 128 weight rows are no more than
   the chip's 256 CUs. What is split in two has so many rows of x times weight rows that
@@ -432,14 +440,19 @@ def parts_win(rows: int, N: int, K: int) -> bool:
 @functools.lru_cache(maxsize=8192)
 def gate_wins(rows: int, N: int, K: int) -> bool:
   """The same for tile_swiglu, beside the library and the activation's kernel: 0.36 to 1.21
-  (0.88 on average) up to 64 rows, 0.75 to 1.16 (0.98) up to 128 but split in two and in
+  (0.88 on average) up to 64 rows, 0.75 to 1.16 (0.97) up to 128 but split in two and in
   more than a round 0.78 to 1.28 (1.09). With 136 rows and more 0.77 to 1.01 (0.88) where
-  a weight tile makes one round of the chip (gate_tile in hip/tile_ops.hip), else 0.97 to
-  1.57; from 256 weight rows a tile gains nothing on the library at 129."""
+  a weight tile makes one round of the chip (gate_tile in hip/tile_ops.hip), 0.66 to 0.96
+  (0.81) where rows are short and whole, but 1.03 to 1.25 of 17920, which just pass a round of
+  64 each; else 0.97 to 1.57; from 256 weight rows a tile gains nothing on the
+  library at 129."""
   if rows <= 64:
     return True
+  whole = gate_splits(N, K) == 1 and not 16384 < N < 20480
   if rows <= 128:
-    return tile_splits(N, K) != 2 or -(-N // 128) * 2 <= 256
+    return whole or tile_splits(N, K) != 2 or -(-N // 128) * 2 <= 256
+  if whole and K <= 2048 and 6144 <= N <= 24576:
+    return True
   return rows >= 136 and tile_splits(N, K) == 1 and any(199 * t < N <= 256 * t for t in (128, 160, 256))
 
 

@@ -455,9 +455,10 @@ static void launch_wide(const TileArgs& a) {
   hipLaunchKernelGGL(kernel, dim3(((a.N + per - 1) / per * a.splits * ((a.m + BM - 1) / BM) + 7) / 8 * 8), dim3(WAVES * 64), lds, cur_stream(), a);
 }
 
-// Whether blocks begin at different places of k (first_step): by the weights' shape alone
+// Whether blocks begin at different places of k (first_step): by the weights' shape alone.
+// Whole sums also over rows 4 KB apart: gate [16384, 2048] m 8 16, 13 us, m 64 17, 15
 static bool turns(int K, int splits) {
-  return K <= 16384 && (K % 4096 == 0 || (splits > 1 && K % splits == 0 && K / splits % 2048 == 0));
+  return K <= 16384 && (K % (splits > 1 ? 4096 : 2048) == 0 || (splits > 1 && K % splits == 0 && K / splits % 2048 == 0));
 }
 
 template <int END>
@@ -492,6 +493,11 @@ static void run_tile(TileArgs a) {
       if (wide == 256) return launch_wide<256, 256, 2, 3, 2, 4, END>(a);
       if (wide == 160) return launch_wide<160, 256, 1, 3, 3, 4, END>(a);
     }
+    if constexpr (END == GATED)
+      // half as many weight rows a block while those make one round: m 80 and 128 by [16384,
+      // 2048] 21 and 24 us, 18 and 19 so; [13824, 4096] 40 and 44, 31 and 35; past a round
+      // they lose: [22016, 2048] 25 and 29, 30 and 34
+      if (a.m <= 128 && rows <= 256 * 64) return launch_wide<64, 128, 2, 4, 3, 4, END>(a);
     if (a.m <= 128 || units < 160) {
       if (a.m <= 128 && units <= 256 && a.whole > 24) launch_wide<128, 128, 2, 4, 3, 4, END>(a);
       else launch_wide<128, 128, 4, 3, 2, 8, END>(a);
@@ -563,12 +569,25 @@ Tensor tile_linear(Tensor x, Tensor w, OptT bias) {
   return y;
 }
 
+// Parts of k of the gated product: one, and no kernel that sums them up, where that leaves
+// blocks enough. us, parts (and the kernel) first: [16384, 2048] m 8 15, 13, m 45 17, 14,
+// m 128 23, 19; [9728, 896] m 8 8, 7, m 64 13, 8, m 256 23, 13; [13824, 4096] m 8 25, 22, m 64
+// 36, 27; [22016, 2048] m 16 22, 20, m 256 50, 33. Fewer blocks and longer sums lose: [8192,
+// 4096] m 8 17, 23; [14336, 8192] m 8 42, 44, m 160 62, 74; and so do tiles that just pass
+// one round: [17920, 4096] m 32 40, 38, m 160 62, 76.
+// (ops.gate_splits says the same)
+static int gate_splits(int rows, int steps) {
+  const int tiles = (rows + 63) / 64;
+  if (steps <= 16 || (tiles >= 160 && steps <= (tiles > 256 && tiles < 320 ? 32 : 96))) return 1;
+  return splits_of(rows, steps);
+}
+
 Tensor tile_swiglu(Tensor x, Tensor w) {
   auto a = tile_args(x, w);
   CHK(a.N % 8 == 0);
   const int I = a.N / 2;
   auto y = sized(x, I);
-  a.splits = splits_of(a.N, a.K / 64);
+  a.splits = gate_splits(a.N, a.K / 64);
   if (a.splits == 1) {
     a.N = I;
     a.y = y.data_ptr();
@@ -624,6 +643,7 @@ std::vector<Tensor> tile_rest(Tensor heads, Tensor wo, Tensor x, Tensor post, do
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("tile_rest", &tile_rest);
   m.def("tile_splits", [](int64_t n, int64_t k) { return splits_of((int)n, (int)(k / 64)); });
+  m.def("gate_splits", [](int64_t n, int64_t k) { return gate_splits((int)n, (int)(k / 64)); });
   m.def("gate_tile", [](int64_t rows, int64_t m) { return gate_tile((int)rows, (int)m); });
   m.def("tile_parts", &tile_parts);
   m.def("tile_linear", &tile_linear);
