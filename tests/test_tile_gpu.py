@@ -44,6 +44,13 @@ def test_products_of_more_rows(m, N, K):
   test_products(m, N, K)
 
 
+# parts that make one round of blocks of 64 weight rows, for each number of rows of x
+@pytest.mark.parametrize("m", [16, 65, 128, 129, 192, 193, 256])
+@pytest.mark.parametrize("N,K", [(3584, 3584), (2044, 1536), (4600, 4288), (8192, 2432), (1024, 1088), (904, 4864), (66, 1024)])
+def test_products_in_a_round_of_parts(m, N, K):
+  test_products(m, N, K)
+
+
 @pytest.mark.parametrize("N,K", [(72, 320), (3584, 3584), (28680, 192), (520, 18944), (1048, 4096), (264, 16384),
                                  (40968, 4096), (40960, 4096), (36872, 4096)])  # the last five begin at different places of k
 def test_rows_do_not_depend_on_their_batch(N, K):

@@ -376,8 +376,9 @@ def tiled(x: torch.Tensor, *weights: torch.Tensor, wins=None) -> bool:
 
 @functools.lru_cache(maxsize=1024)
 def tile_splits(N: int, K: int) -> int:
-  """Parts of k of a product by tiles: as few as give some 450 blocks of 64 weight rows,
-  of 4 steps of 64 at least (splits_of in hip/tile_ops.hip)."""
+  """Parts of k of a product by tiles, as the rules below count them: as few as give some 450
+  blocks of 64 weight rows, of 4 steps of 64 at least (splits_of in hip/tile_ops.hip; small
+  weights take fewer, parts_of)."""
   return max(1, min(-(-448 // -(-N // 64)), K // 256, 16))
 
 
@@ -386,7 +387,10 @@ def gate_splits(N: int, K: int) -> int:
   """The same of the gated product of N weight rows (gate_splits in hip/tile_ops.hip)."""
   tiles = -(-N // 64)
   whole = K <= 1024 or (tiles >= 160 and K <= (2048 if 256 < tiles < 320 else 6144))
-  return 1 if whole else tile_splits(N, K)
+  if whole:
+    return 1
+  n, one = tile_splits(N, K), 256 // tiles
+  return one if 2 <= one < n and one * tiles >= 200 and N * (K // 64) <= 312500 else n
 
 
 @functools.lru_cache(maxsize=1024)

@@ -498,6 +498,15 @@ static void run_tile(TileArgs a) {
       // 2048] 21 and 24 us, 18 and 19 so; [13824, 4096] 40 and 44, 31 and 35; past a round
       // they lose: [22016, 2048] 25 and 29, 30 and 34
       if (a.m <= 128 && rows <= 256 * 64) return launch_wide<64, 128, 2, 4, 3, 4, END>(a);
+    if constexpr (END == PART)
+      // the same of parts (parts_of): m 100 by [896, 4864] with its norm 13.5, 12.4; [1024, 1024]
+      // 9.6, 8.3; in twice the parts [3584, 3584] m 100 17.8, now 15.3, m 192 21.8, 21.0, m 256 22.8,
+      // 22.6 (of two blocks of 128 rows of x 23.7)
+      if ((rows + 63) / 64 * a.splits <= 256 && (int64_t)rows * a.K <= 20000000) {
+        if (a.m <= 128) return launch_wide<64, 128, 2, 4, 3, 4, END>(a);
+        if (a.m <= 192) return launch_wide<64, 192, 2, 4, 3, 4, END>(a);
+        return launch_wide<64, 256, 2, 4, 3, 8, END>(a);
+      }
     if (a.m <= 128 || units < 160) {
       if (a.m <= 128 && units <= 256 && a.whole > 24) launch_wide<128, 128, 2, 4, 3, 4, END>(a);
       else launch_wide<128, 128, 4, 3, 2, 8, END>(a);
@@ -524,11 +533,22 @@ static TileArgs tile_args(const Tensor& x, const Tensor& w) {
   return a;
 }
 
-// Parts of k: as few as give some 450 blocks of 64 weight rows, of 4 steps at least
-// (ops.tile_splits says the same, for the rules of which products these are)
+// Parts of k, as the rules of which products these are count them (ops.tile_splits): as few as
+// give some 450 blocks of 64 weight rows, of 4 steps at least
 static int splits_of(int rows, int steps) {
   const int tiles = (rows + 63) / 64;
   return std::max(1, std::min({(448 + tiles - 1) / tiles, steps / 4, 16}));
+}
+
+// What k is split in: of up to 20 10^6 weights in as many as make one round of the chip, where
+// they fill it, as fewer sums are then written and read. us with the norm that reads them, splits_of
+// first: m 8 [3584, 3584] 10.4, 9.9, [1536, 8960] 11.3, 10.0; m 45 [2048, 8192] 14.6, 13.0, [3072,
+// 2048] 11.3, 9.3; m 128 [4096, 4096] 20.6, 17.7; m 256 [2048, 2048] 18.7, 17.7. Larger weights
+// gain nothing from 65 rows on: m 8 and 192 [8192, 8192] 28.8, 28.7 and 42.6, 51.3, [4096, 14336]
+// 25.6, 25.4 and 40.5, 53.7; nor do they in two thirds of a round: m 8 [6144, 4096] 14.7, 16.5.
+static int parts_of(int rows, int steps) {
+  const int tiles = (rows + 63) / 64, n = splits_of(rows, steps), one = 256 / tiles;
+  return one >= 2 && one < n && one * tiles >= 200 && (int64_t)rows * steps <= 312500 ? one : n;
 }
 
 static Tensor sized(const Tensor& x, int64_t n) {
@@ -540,7 +560,7 @@ static Tensor sized(const Tensor& x, int64_t n) {
 // fp32 [splits, m, N]
 Tensor tile_parts(Tensor x, Tensor w) {
   auto a = tile_args(x, w);
-  a.splits = splits_of(a.N, a.K / 64);
+  a.splits = parts_of(a.N, a.K / 64);
   auto part = torch::empty({a.splits, a.m, a.N}, x.options().dtype(torch::kFloat32));
   a.y = part.data_ptr();
   run_tile<PART>(a);
@@ -555,7 +575,7 @@ Tensor tile_linear(Tensor x, Tensor w, OptT bias) {
     a.bias = P<bf16_t>(*bias);
   }
   auto y = sized(x, a.N);
-  a.splits = a.N % 4 ? 1 : splits_of(a.N, a.K / 64);
+  a.splits = a.N % 4 ? 1 : parts_of(a.N, a.K / 64);
   if (a.splits == 1) {
     a.y = y.data_ptr();
     run_tile<STORE>(a);
@@ -579,7 +599,7 @@ Tensor tile_linear(Tensor x, Tensor w, OptT bias) {
 static int gate_splits(int rows, int steps) {
   const int tiles = (rows + 63) / 64;
   if (steps <= 16 || (tiles >= 160 && steps <= (tiles > 256 && tiles < 320 ? 32 : 96))) return 1;
-  return splits_of(rows, steps);
+  return parts_of(rows, steps);
 }
 
 Tensor tile_swiglu(Tensor x, Tensor w) {
