@@ -184,6 +184,12 @@ def test_gates_of_prompts(M, N, K, form):
   assert bool(((y.reshape(-1, N // 2).double() - silu * up).abs() <= bound + 1e-30).all())
 
 
+# more and fewer rows a tile than rows / 256 makes, whole and cut in two
+@pytest.mark.parametrize("M,N", [(257, 9728), (300, 17920), (513, 16384), (600, 16384), (700, 16384), (1000, 17920), (1200, 16416)])
+def test_gates_of_prompts_in_even_rounds(M, N):
+  test_gates_of_prompts(M, N, 128, "rows")
+
+
 def test_gates_of_prompts_in_a_layer():
   """One kernel where nobody waits for the product, with the module's hooks and its graph."""
   from xotorch_amd.models.llama import MLP

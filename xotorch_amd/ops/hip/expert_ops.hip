@@ -569,7 +569,7 @@ __global__ __launch_bounds__(256) void expert_tile_kernel(
     }
   }
   // an expert's rows go over its tiles evenly, in steps of 32
-  const int of = CUT ? tiles_of(end - lo, plan.most) : (end - lo + TOK - 1) / TOK, share = ((end - lo + of - 1) / of + 31) / 32 * 32;
+  const int of = KIND == DENSE ? max_tiles : CUT ? tiles_of(end - lo, plan.most) : (end - lo + TOK - 1) / TOK, share = ((end - lo + of - 1) / of + 31) / 32 * 32;
   const int r0 = lo + nth * share, hi = min(end, r0 + share), rows = hi - r0;
   const bf16_t* we = w.of(e, (size_t)(TWO ? 2 : 1) * a.F * a.kp);
   constexpr bool TAIL = std::is_same<W, Stacked>::value && KIND != DENSE;
@@ -875,7 +875,22 @@ Tensor gate_product(Tensor x, Tensor w) {
   CHK(rows >= 1 && rows <= 1 << 22 && K >= 64 && K <= 1 << 22 && K % 64 == 0 && w.size(1) == K);
   CHK(w.size(0) >= 32 && w.size(0) <= 1 << 22 && w.size(0) % 32 == 0);
   auto y = torch::empty({rows, F_}, x.options());
-  const int tiles = (int)((rows + 255) / 256), nf = (int)((F_ + 127) / 128);
+  // tiles of up to 256 rows, or, up to some ten rounds, of fewer where the rounds they make take
+  // less time by what plan_of goes by. us, least tiles first: 600 and 700 rows by [16384, 2048] 45.6
+  // and 49.4, 39.4 and 44.6; 512 by [17920, 1536] 37.2, 32.0; 300 and 1000 by [9728, 896] 13.1 and
+  // 24.0, 10.3 and 21.3; larger weights the same
+  const int nf = (int)((F_ + 127) / 128), least = (int)((rows + 255) / 256);
+  auto share_of = [&](int n) { return ((rows + n - 1) / n + 31) / 32 * 32; };
+  auto time = [&](int n) {
+    const int64_t all = ((int64_t)n * nf + 7) / 8, left = all % DIE_CUS;  // of a die
+    return ((double)(all / DIE_CUS) + (left == 0 ? 0 : left <= DIE_CUS / 2 ? 0.62 : 1)) * (0.4 + 0.00375 * std::max<int64_t>(128, share_of(n)));
+  };
+  int tiles = least;
+  if ((int64_t)least * nf < 2560)
+    for (int n = least + 1; n <= 2 * least; ++n) {
+      const int some = (int)((rows + share_of(n) - 1) / share_of(n));  // none without a row
+      if (time(some) < 0.95 * time(least) && time(some) < time(tiles)) tiles = some;
+    }
   // panels of 2, 4, 6 and 8 tiles, us: 1500 rows of 3584 by 37888 326, 320, 315, 312; 6001 by
   // [28672, 4096] 1047, 1030, 1005, 1022; 3000 by [57344, 8192] 2114, 2058, 1988, 2022
   const int group = 6;
