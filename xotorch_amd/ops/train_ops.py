@@ -139,9 +139,13 @@ def forward_wins(M: int, N: int, K: int) -> bool:
   there on. Wider results and more tokens 0.95 to 1.40, but for long sums, whose library tiles
   fill the chip badly (257 to 2000 tokens by 1536 to 12288 features of 13824 to 29568): where
   the result is small 0.46 to 1.05 (0.69), of up to 6144 features 0.65 to 0.95, narrow ones of
-  longest sums 0.39 to 0.87. Above these lines 0.6 to 1.5 from one size to the next."""
+  longest sums 0.39 to 0.87. A vocabulary's width (128256 to 152064 features of 896 to 4096), 65
+  to 1000 tokens 0.63 to 1.02 (0.86), from 1333 on 0.92 to 1.05. Above these lines 0.6 to 1.5
+  from one size to the next."""
   if K % 64 or N % 4 or max(M, N, K) > _MOST:
     return False
+  if N >= 100_000 and K <= 4096:
+    return 64 < M <= 1000
   if M <= 1000 and N <= 4096:
     return True
   small = M * N <= 4_300_000 and N <= 12288 or M <= 1000 and N <= 6144
