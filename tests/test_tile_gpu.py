@@ -122,6 +122,26 @@ def test_gated_products_of_whole_rows(N, K):
   assert bool(((all_rows.double() - act * up).abs() <= slack + 1e-30).all())
 
 
+# weight rows that blocks of four to eight waves fill rounds best with, a tile's last ones missing
+@pytest.mark.parametrize("N,waves", [(37872, 5), (17920, 5), (24560, 6), (22016, 6), (28656, 7), (49136, 4), (32752, 8), (49120, 4)])
+def test_gated_products_fill_their_rounds(N, waves):
+  from xotorch_amd import ops
+  assert waves in {ops._tile().gate_waves(N, m) or (8 if m > 16 and N > 199 * 128 else 4) for m in (16, 32, 64)}
+  for m in (1, 16, 17, 32, 33, 64):
+    test_gated_product(m, N, 192)
+
+
+def test_gated_product(m=5, N=25584, K=320):
+  """Products rounded to bf16 after fp32 sums; silu's slope is at most 1.1."""
+  from xotorch_amd import ops
+  x, w, _ = _inputs(m, N, K)
+  (g, u), (tg, tu) = (x.double() @ w.double().t()).chunk(2, -1), (x.double().abs() @ w.double().abs().t() * (K * 2.0 ** -24)).chunk(2, -1)
+  tg, tu, act = tg + g.abs() * 2.0 ** -8, tu + u.abs() * 2.0 ** -8, torch.nn.functional.silu(g)
+  bound = 1.1 * tg * (u.abs() + tu) + act.abs() * tu + (act * u).abs() * 2.0 ** -8
+  with torch.no_grad():
+    assert bool(((ops.tile_swiglu(x, w).double() - act * u).abs() <= bound + 1e-30).all())
+
+
 @pytest.mark.parametrize("m,D,H,I", [(3, 64, 128, 192), (45, 2048, 2048, 8192), (200, 320, 192, 512)])
 def test_rest_of_a_layer_is_its_parts(m, D, H, I):
   from xotorch_amd import ops

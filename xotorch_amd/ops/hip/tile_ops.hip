@@ -72,6 +72,9 @@ DEVINL void read_frags(unsigned a, unsigned b, bf16x8* r, bf16x8* c) {
     asm volatile(RD(0, 2, 0) RD(1, 3, 0) DONE : "=&v"(r[0]), "=&v"(c[0]) : "v"(a), "v"(b));
   else if constexpr (R == 1 && C == 2)
     asm volatile(RD(0, 3, 0) RD(1, 4, 0) RD(2, 4, 2048) DONE : "=&v"(r[0]), "=&v"(c[0]), "=&v"(c[1]) : "v"(a), "v"(b));
+  else if constexpr (R == 1 && C == 4)
+    asm volatile(RD(0, 5, 0) RD(1, 6, 0) RD(2, 6, 2048) RD(3, 6, 4096) RD(4, 6, 6144) DONE
+                 : "=&v"(r[0]), "=&v"(c[0]), "=&v"(c[1]), "=&v"(c[2]), "=&v"(c[3]) : "v"(a), "v"(b));
   else if constexpr (R == 2 && C == 1)
     asm volatile(RD(0, 3, 0) RD(1, 3, 2048) RD(2, 4, 0) DONE : "=&v"(r[0]), "=&v"(r[1]), "=&v"(c[0]) : "v"(a), "v"(b));
   else if constexpr (R == 2 && C == 2)
@@ -86,14 +89,14 @@ DEVINL void read_frags(unsigned a, unsigned b, bf16x8* r, bf16x8* c) {
 #undef DONE
 }
 
-template <int BN, int BM, int BUFS>
+template <int BN, int BM, int BUFS, int WAVES_ = 4>
 struct TileShape {
   static constexpr int ROWS = BN + BM, BUF = ROWS * 64;  // elements of a buffer
-  static constexpr int WAVES = 4;
-  static constexpr int WL = BN / 8 / WAVES, XL = BM >= 32 ? BM / 8 / WAVES : 1;  // loads of a wave and stage
+  static constexpr int WAVES = WAVES_;
+  static constexpr int WL = BN / 8 / WAVES, XL = BM >= 32 ? BM / 32 : 1;  // loads of a wave and stage; of x by four
   static constexpr int LDS = BUFS * BUF * 2;
-  // waves along x: the weight rows are split over all four for few rows of x
-  static constexpr int WX = BM >= 64 ? 2 : 1, R = BN * WX / WAVES / 16, C = BM / WX / 16;
+  // waves along x: the weight rows are split over all of them for few rows of x, or more than four
+  static constexpr int WX = BM >= 64 && WAVES == 4 ? 2 : 1, R = BN * WX / WAVES / 16, C = BM / WX / 16;
 };
 
 // A wave's sums of weight rows wr .. of a tile and rows m0 .. of x
@@ -148,9 +151,9 @@ DEVINL void finish_tile(const TileArgs& a, const floatx4 (&acc)[R][C], int tile,
   }
 }
 
-template <int BN, int BM, int BUFS, int END>
-__global__ __launch_bounds__((TileShape<BN, BM, BUFS>::WAVES * 64)) void tile_kernel(TileArgs a) {
-  typedef TileShape<BN, BM, BUFS> Sh;
+template <int BN, int BM, int BUFS, int END, int WAVES>
+__global__ __launch_bounds__((TileShape<BN, BM, BUFS, WAVES>::WAVES * 64)) void tile_kernel(TileArgs a) {
+  typedef TileShape<BN, BM, BUFS, WAVES> Sh;
   constexpr int R = Sh::R, C = Sh::C, LOADS = Sh::WL + Sh::XL;
   extern __shared__ __attribute__((aligned(16))) bf16_t buf[];  // [BUFS][weights [BN][64], x [BM][64]]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -188,7 +191,7 @@ __global__ __launch_bounds__((TileShape<BN, BM, BUFS>::WAVES * 64)) void tile_ke
   }
 #pragma unroll
   for (int i = 0; i < Sh::XL; ++i) {
-    const int r = BM >= 32 ? (wave * Sh::XL + i) * 8 + sub : wave * 4 + (sub & 3);
+    const int r = BM >= 32 ? ((wave & 3) * Sh::XL + i) * 8 + sub : (wave & 3) * 4 + (sub & 3);  // waves past four load the same again
     xsrc[i] = a.x + (size_t)min(m0 + r, a.m - 1) * a.K + ((lane & 7) ^ (r & 7)) * 8;
   }
   const int len = s1 - s0, turn = first_step<END>(a, tile * (END == GATED ? BN / 2 : BN), len);
@@ -200,7 +203,7 @@ __global__ __launch_bounds__((TileShape<BN, BM, BUFS>::WAVES * 64)) void tile_ke
       __builtin_amdgcn_global_load_lds((glb_void*)(wsrc[i] + k), (lds_void*)(dst + (wave * Sh::WL + i) * 512), 16, 0, 2);
 #pragma unroll
     for (int i = 0; i < Sh::XL; ++i) {
-      bf16_t* to = dst + BN * 64 + (BM >= 32 ? (wave * Sh::XL + i) * 512 : wave * 256);
+      bf16_t* to = dst + BN * 64 + (wave & 3) * (BM >= 32 ? Sh::XL * 512 : 256) + i * 512;
       if (BM >= 32 || lane < 32)
         __builtin_amdgcn_global_load_lds((glb_void*)(xsrc[i] + k), (lds_void*)to, 16, 0, 0);
     }
@@ -403,11 +406,11 @@ __global__ __launch_bounds__(THREADS) void add_norm_kernel(const float* __restri
 // cost: blocks without work between the others keep CUs from them, which then have two. us,
 // parts of the grid and numbered through: [4608, 3584] in 36 tiles and 7 parts, m 20 10.7, 8.2;
 // m 48 12.5, 9.3
-template <int BN, int BM, int BUFS, int END>
+template <int BN, int BM, int BUFS, int END, int WAVES = 4>
 static void launch_tile(TileArgs a) {
-  typedef TileShape<BN, BM, BUFS> Sh;
+  typedef TileShape<BN, BM, BUFS, WAVES> Sh;
   if (Sh::LDS > 64 * 1024) {
-    const hipError_t e = hipFuncSetAttribute((const void*)tile_kernel<BN, BM, BUFS, END>,
+    const hipError_t e = hipFuncSetAttribute((const void*)tile_kernel<BN, BM, BUFS, END, WAVES>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, Sh::LDS);
     TORCH_CHECK(e == hipSuccess, "no LDS for weight tiles");
   }
@@ -415,7 +418,7 @@ static void launch_tile(TileArgs a) {
   const int tiles = (a.N + per - 1) / per, mts = (a.m + BM - 1) / BM;
   a.dense = !a.runs && a.splits > 1 && tiles % 8;
   const dim3 grid = a.dense ? dim3((tiles * a.splits + 7) / 8 * 8 * mts) : dim3((tiles + 7) / 8 * 8 * mts, a.splits);
-  hipLaunchKernelGGL((tile_kernel<BN, BM, BUFS, END>), grid, dim3(Sh::WAVES * 64), Sh::LDS, cur_stream(), a);
+  hipLaunchKernelGGL((tile_kernel<BN, BM, BUFS, END, WAVES>), grid, dim3(Sh::WAVES * 64), Sh::LDS, cur_stream(), a);
 }
 
 // Tile and depth by the rows of x and by the blocks that 128 weight rows make. us at
@@ -444,6 +447,33 @@ static int gate_tile(int rows, int m) {
   for (int tile : {128, 160, 256})
     if (rows > 199 * tile && rows <= 256 * tile) return tile;
   return 0;
+}
+
+// Up to 64 rows: waves of a block, each of 16 weight rows, by how full the last of up to four rounds
+// of 256 blocks is, where that is more than tiles of 64 or (8, also four waves) 128 rows fill it by
+// 8%, or by 20% for more than 32 rows of x, which more waves read more often from LDS. us, by those
+// first: [37888, 3584] m 8 48.7, 43.1, m 32 59.6, 46.0, m 64 66.1, 54.1; [17920, 1536] m 8 14.6, 12.5, m 45
+// 19.1, 14.7; [49152, 3584] m 16 57.2, 57.3, m 24 67.5, 58.7. Less to fill up: [27648, 5120] m 8 49.1, 46.9,
+// m 64 58.2, 60.2
+static int gate_waves(int rows, int m) {
+  auto fill = [&](int waves) {
+    const int blocks = (rows + waves * 16 - 1) / (waves * 16);
+    return (double)blocks / ((blocks + 255) / 256 * 256);
+  };
+  const int now = m > 16 && (rows + 127) / 128 >= 200 ? 8 : 4;
+  int best = now;
+  if (rows <= 4 * 256 * 64)
+    for (int waves = 4; waves <= 8; ++waves)
+      if (fill(waves) > fill(best) * (best != now ? 1.0 : m > 32 ? 1.2 : 1.08)) best = waves;
+  return best == now ? 0 : best;
+}
+template <int BM>
+static void gate_of_waves(const TileArgs& a, int waves) {
+  if (waves == 4) launch_tile<64, BM, 4, GATED>(a);
+  else if (waves == 5) launch_tile<80, BM, 4, GATED, 5>(a);
+  else if (waves == 6) launch_tile<96, BM, 4, GATED, 6>(a);
+  else if (waves == 7) launch_tile<112, BM, 4, GATED, 7>(a);
+  else launch_tile<128, BM, 4, GATED, 8>(a);
 }
 
 template <int BN, int BM, int WN, int WB, int XB, int WAVES, int END>
@@ -476,6 +506,9 @@ static void run_tile(TileArgs a) {
   // 46.8, 42.0; [8192, 28672] 125, 120
   const int64_t x = (int64_t)a.m * a.K;
   a.runs = END == PART ? x > (a.m <= 64 ? 2 << 19 : a.turned ? 3 << 19 : 7 << 19) : a.m > 64;
+  if constexpr (END == GATED)
+    if (const int waves = a.m <= 64 && !a.turned && a.splits == 1 ? gate_waves(rows, a.m) : 0)
+      return a.m <= 16 ? gate_of_waves<16>(a, waves) : a.m <= 32 ? gate_of_waves<32>(a, waves) : gate_of_waves<64>(a, waves);
   if (a.m <= 16) launch_tile<64, 16, 4, END>(a);
   else if (a.m <= 32) {
     if (units >= 200) launch_tile<128, 32, 4, END>(a);
@@ -663,6 +696,7 @@ std::vector<Tensor> tile_rest(Tensor heads, Tensor wo, Tensor x, Tensor post, do
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("tile_rest", &tile_rest);
   m.def("tile_splits", [](int64_t n, int64_t k) { return splits_of((int)n, (int)(k / 64)); });
+  m.def("gate_waves", [](int64_t rows, int64_t m) { return gate_waves((int)rows, (int)m); });
   m.def("gate_splits", [](int64_t n, int64_t k) { return gate_splits((int)n, (int)(k / 64)); });
   m.def("gate_tile", [](int64_t rows, int64_t m) { return gate_tile((int)rows, (int)m); });
   m.def("tile_parts", &tile_parts);
