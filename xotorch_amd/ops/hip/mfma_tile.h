@@ -81,7 +81,7 @@ struct StepSource {
 
 // One operand's fragments of 32 of k, N tiles of 16 rows, and where a lane reads them. By
 // hand: the compiler would make every read wait for all pending loads to LDS. What is read
-// is used, after `landed`.
+// is used, after `landed` and `whole`.
 //
 // Rows: k lies along a row, as above.
 template <int N>
@@ -105,6 +105,7 @@ struct RowFrags {
   }
   DEVINL bf16x8 operator[](int i) const { return f[i]; }
   DEVINL void clear(int, int, int) {}
+  DEVINL void whole() { landed(); }
 };
 
 // Columns: a step is 64 rows of F numbers, k along the rows. Transposing reads give a lane
@@ -116,6 +117,7 @@ struct ColFrags {
   static constexpr int COUNT = 2 * N;
   typedef __attribute__((ext_vector_type(4))) __bf16 half_t;
   half_t lo[N], hi[N];
+  bf16x8 f[N];
   unsigned at;  // of the first tile; that of tile i differs in bits 5 to 7
   DEVINL ColFrags(unsigned base, int col, int lane) {
     const int k = (lane >> 4) * 8 + ((lane & 15) >> 2);
@@ -134,7 +136,15 @@ struct ColFrags {
       asm volatile("" : "+v"(hi[i]));
     }
   }
-  DEVINL bf16x8 operator[](int i) const { return __builtin_shufflevector(lo[i], hi[i], 0, 1, 2, 3, 4, 5, 6, 7); }
+  DEVINL bf16x8 operator[](int i) const { return f[i]; }
+  // both halves where they are multiplied, before `written`
+  DEVINL void whole() {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      f[i] = __builtin_shufflevector(lo[i], hi[i], 0, 1, 2, 3, 4, 5, 6, 7);
+      asm volatile("" : "+v"(f[i]));
+    }
+  }
   // zeros for the step's first `skip` k, of half h
   DEVINL void clear(int skip, int h, int lane) {
     typedef __attribute__((ext_vector_type(4))) short short4_t;
@@ -251,6 +261,8 @@ DEVINL void walk(floatx4 (&acc)[R][C], W w, X x, int steps, StepW stepw, LoadW l
       xa.clear(skip, 0, threadIdx.x & 63);
       wa.clear(skip, 0, threadIdx.x & 63);
     }
+    xa.whole();
+    wa.whole();
     written();
     each<R>([&](auto i) {
       row(i, wa, xa, wb, xb, second, 1);
@@ -264,6 +276,8 @@ DEVINL void walk(floatx4 (&acc)[R][C], W w, X x, int steps, StepW stepw, LoadW l
       xb.clear(skip, 1, threadIdx.x & 63);
       wb.clear(skip, 1, threadIdx.x & 63);
     }
+    xb.whole();
+    wb.whole();
     written();
     // all waves have read this step, and the next one is there
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(LATER) : "memory");
