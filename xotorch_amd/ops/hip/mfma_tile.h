@@ -320,15 +320,18 @@ struct RowsOut {
   DEVINL RowsOut(void* lds, int wave, int lane_) : mine((char*)lds + wave * BYTES), lane(lane_) {}
   // row `r`, features f .. f + 3
   DEVINL void put(int r, int f, four_t v) const { *(four_t*)(mine + r * ROW + f * sizeof(T)) = v; }
-  // to(row, feature, piece) for all of the rows; LDS operations of a wave are in order
+  // to(row, feature, piece) for all of the rows. LDS operations of a wave are in order; that lanes
+  // read what others wrote, and write what others have read, is said to the compiler by the fences
   template <typename To>
   DEVINL void out(To to) const {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int q0 = 0; q0 < ROWS * PIECES; q0 += 64) {
       const int q = q0 + lane, r = q / PIECES, p = q % PIECES;
       if (ROWS * PIECES % 64 == 0 || q < ROWS * PIECES) to(r, p * PER, *(const floatx4*)(mine + r * ROW + p * 16));
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_sched_barrier(0);  // (the next rows' sums stay where they are meanwhile)
   }
 };
