@@ -171,3 +171,26 @@ def test_tokens_past_four_gigabytes():
     args = torch.tensor([0, n], **ints), torch.tensor(listed, **ints), tile, True
     near = hip.expert_product_of(x[token].contiguous(), [w], torch.arange(n, **ints), *args)
     assert torch.equal(hip.expert_product_of(x, [w], token.to(torch.int32), *args), near)
+
+
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_rows_past_what_tiles_address(swiglu):
+  from xotorch_amd.ops.mixer_ops import load_hip
+  hip = load_hip("_hip_experts")
+  K, F, counts = (1 << 22) + 64, 16, [17, 0, 3]
+  g, n = torch.Generator(device="cuda").manual_seed(K), sum(counts)
+  x = torch.randn(n, K, generator=g, device="cuda", dtype=torch.bfloat16)
+  w = [torch.randn((2 if swiglu else 1) * F, K, generator=g, device="cuda", dtype=torch.bfloat16) * 2.0 ** -11 for _ in counts]
+  ints = dict(dtype=torch.int32, device="cuda")
+  first, tiles = torch.tensor([0, 17, 17, 20], **ints), torch.tensor([(0, 0), (2, 17), (-1, 0), (-1, 2)], **ints)
+  got = hip.expert_product_of(x, w, torch.arange(n, **ints), first, tiles, 128, swiglu).double()
+  for e, (lo, hi) in ((0, (0, 17)), (2, (17, 20))):
+    want = x[lo:hi].double() @ w[e].double().t()
+    # fp32 sums by four waves, each of K / 128 additions of 32 products; of random signs, they stay
+    # within six standard deviations
+    slack = x[lo:hi].double().norm(dim=1, keepdim=True) * w[e].double().norm(dim=1) * K ** -0.5 * 6 * (K / 128 + 8) * 2.0 ** -24
+    if swiglu:
+      (gate, up), (sg, su) = want.chunk(2, -1), slack.chunk(2, -1)
+      want = torch.nn.functional.silu(gate) * up
+      slack = (1.1 * sg + gate.abs() * 2.0 ** -19) * (up.abs() + su) + su * gate.abs()
+    assert bool(((got[lo:hi] - want).abs() <= slack + want.abs() * 2.0 ** -8).all()), e

@@ -295,7 +295,7 @@ __global__ __launch_bounds__(256) void expert_stream_kernel(
     const T* __restrict__ x, const T* __restrict__ w, const int* __restrict__ first, const int* __restrict__ token,
     const float* __restrict__ by_row, T* __restrict__ y, GroupArgs a, Act act) {
   typedef Frag<T> F;
-  constexpr int NW = KIND == GATED ? 2 : 1, MOST = 4 / NW;
+  constexpr int NW = has_gate(KIND) ? 2 : 1, MOST = 4 / NW;
   __shared__ float part[4][NW][MOST * 16][17];
   // the last experts are the ones that every token uses: the longest come first
   const int e = gridDim.y - 1 - blockIdx.y, f0 = blockIdx.x * 16;
@@ -761,7 +761,7 @@ static void launch_tiles(const W& w, const Tensor& x, const Tensor& token, const
 #undef TILES
 }
 
-// The tiled form with one weight tensor per expert, bf16: SWIGLU ([2 F, K], gate rows
+// The form with one weight tensor per expert, bf16, by tiles: SWIGLU ([2 F, K], gate rows
 // first) or PLAIN ([F, K]), K % 64 == 0.
 Tensor expert_product_of(Tensor x, std::vector<Tensor> w, Tensor token, Tensor first, Tensor tiles, int64_t tile, bool swiglu) {
   check_io(x, torch::kBFloat16);
@@ -769,7 +769,7 @@ Tensor expert_product_of(Tensor x, std::vector<Tensor> w, Tensor token, Tensor f
   CHK(x.dim() == 2 && E >= 1 && E <= MOST_LISTED && ((size_t)x.data_ptr() & 15) == 0);
   for (const Tensor& t : {token, first, tiles}) check_io(t, torch::kInt32);
   const int K = x.size(1), pairs = token.numel(), F_ = w[0].size(0) / (swiglu ? 2 : 1);
-  CHK(first.numel() == E + 1 && K % 64 == 0 && K <= 1 << 22 && F_ % 16 == 0 && (swiglu || x.size(0) == pairs));
+  CHK(first.numel() == E + 1 && K % 64 == 0 && F_ % 16 == 0 && (swiglu || x.size(0) == pairs));
   Listed list{};
   for (int64_t e = 0; e < E; ++e) {
     check_io(w[e], torch::kBFloat16);
@@ -777,7 +777,20 @@ Tensor expert_product_of(Tensor x, std::vector<Tensor> w, Tensor token, Tensor f
     list.w[e] = P<bf16_t>(w[e]);
   }
   auto y = torch::empty({pairs, F_}, x.options());
-  launch_tiles(list, x, token, first, tiles, tile, swiglu ? SWIGLU : PLAIN, GroupArgs{K, K, F_, (int)E, K, F_}, Act{}, nullptr, y);
+  const GroupArgs a{K, K, F_, (int)E, K, F_};
+  if (K <= 1 << 22) {
+    launch_tiles(list, x, token, first, tiles, tile, swiglu ? SWIGLU : PLAIN, a, Act{}, nullptr, y);
+    return y;
+  }
+  // offsets of a tile's weights have 32 bits: longer rows expert by expert, without tiles
+  CHK(tile == 128 || tile == 256);
+  auto stream = [&](auto kernel) {
+    for (int64_t e = 0; e < E; ++e)
+      hipLaunchKernelGGL(kernel, dim3(F_ / 16), dim3(256), 0, cur_stream(), P<bf16_t>(x), list.w[e], first.data_ptr<int>() + e,
+                         token.data_ptr<int>(), (const float*)nullptr, M<bf16_t>(y), a, Act{});
+  };
+  if (swiglu) stream(expert_stream_kernel<bf16_t, SWIGLU, true>);
+  else stream(expert_stream_kernel<bf16_t, PLAIN, true>);
   return y;
 }
 
