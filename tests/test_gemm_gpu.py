@@ -34,6 +34,14 @@ def test_products(M, N, K):
   assert _near(hip.weight_gradient(dy, x), dy.t(), x.t())
 
 
+# rows of 4 numbers more than pieces of 8: whole sums and parts of them, tiles of 128 and 256
+@pytest.mark.parametrize("M,N,K", [(65, 68, 128), (300, 4100, 192), (100, 260, 4096), (1001, 12, 64), (700, 18308, 128), (2048, 516, 2048)])
+def test_products_of_half_pieces(M, N, K):
+  from xotorch_amd.ops import train_ops
+  x, w = _random(M, M, K), _random(N, N, K)
+  assert _near(train_ops._hip_gemm().forward(x, w), x, w)
+
+
 @pytest.mark.parametrize("left", [64, 65, 127, 128, 129, 1003])
 def test_what_is_left_of_a_sum_counts_once(left):
   """Tokens past whole steps; infinities in rows that the last step has twice stay what they are."""

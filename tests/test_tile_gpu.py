@@ -39,7 +39,7 @@ def test_products(m, N, K):
 # from 65 rows on: parts of few steps and of many, blocks for a round, for more than one and for
 # half of one, rows of x in two blocks, weight rows past a tile and off the 16 bytes of a piece
 @pytest.mark.parametrize("m,N,K", [(66, 3592, 3584), (100, 4104, 14336), (128, 1002, 8192), (128, 33000, 128), (81, 41000, 64), (150, 3084, 4096),
-                                   (192, 4104, 1536), (193, 4100, 2048), (130, 1000, 1024), (256, 1006, 512), (160, 57352, 128), (129, 65528, 64)])
+                                   (192, 4104, 1536), (193, 4100, 2048), (219, 28364, 128), (122, 47436, 192), (130, 1000, 1024), (256, 1006, 512), (160, 57352, 128), (129, 65528, 64)])
 def test_products_of_more_rows(m, N, K):
   test_products(m, N, K)
 

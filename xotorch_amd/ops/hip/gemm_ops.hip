@@ -108,7 +108,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(GemmArgs a) {
            s1 - s0, stepw, loadw, stepx, loadx, skip);
   typedef typename std::conditional<PARTS, float, bf16_t>::type Out;
   const RowsOut<Out, R * 16> rows(buf, wave, lane);
-  const bool whole = a.N % (16 / sizeof(Out)) == 0;
 #pragma unroll
   for (int j = 0; j < C; ++j) {
 #pragma unroll
@@ -119,7 +118,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(GemmArgs a) {
     }
     rows.out([&](int r, int f, floatx4 v) {
       const int m = m0 + wx + j * 16 + r, n = n0 + wr + f;
-      if (m < a.M) st_piece((Out*)a.y + ((size_t)split * a.M + m) * a.N + n, v, a.N - n, whole);
+      if (m < a.M) st_piece((Out*)a.y + ((size_t)split * a.M + m) * a.N + n, v, a.N - n, a.N);
     });
   }
 }

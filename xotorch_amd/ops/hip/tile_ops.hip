@@ -296,7 +296,6 @@ __global__ __launch_bounds__((WAVES * 64)) void wide_kernel(TileArgs a) {
   static_assert(C % PAIR == 0, "");
   const RowsOut<Out, N, PAIR * 16> rows(buf, wave, lane);
   const int n0 = tile * PER + (END == GATED ? wr / 2 : wr);
-  const bool whole = a.N % (16 / sizeof(Out)) == 0;
 #pragma unroll
   for (int j = 0; j < C; j += PAIR) {
 #pragma unroll
@@ -321,7 +320,7 @@ __global__ __launch_bounds__((WAVES * 64)) void wide_kernel(TileArgs a) {
     }
     rows.out([&](int r, int f, floatx4 v) {
       const int m = m0 + wx + j * 16 + r;
-      if (m < a.m) st_piece((Out*)a.y + ((size_t)split * a.m + m) * a.N + n0 + f, v, a.N - n0 - f, whole);
+      if (m < a.m) st_piece((Out*)a.y + ((size_t)split * a.m + m) * a.N + n0 + f, v, a.N - n0 - f, a.N);
     });
   }
 }
