@@ -127,11 +127,11 @@ def test_shares_of_rows_in_steps_of_32(rows, swiglu):
 
 
 @pytest.mark.parametrize("experts,F", [(1, 2048), (8, 4096), (65, 272), (130, 48), (250, 16)])  # one, some or many a lane
-def test_tiles_that_the_kernel_plans(experts, F):
+def test_tiles_that_the_kernel_plans(experts, F, K=64):
   """Few rounds of blocks: whatever rows a tile has, each row is what its expert gives it alone."""
   from xotorch_amd.ops.mixer_ops import load_hip
   hip = load_hip("_hip_experts")
-  g, K = torch.Generator(device="cuda").manual_seed(experts), 64
+  g = torch.Generator(device="cuda").manual_seed(experts)
   sizes = [0, 1, 100, 128, 129, 190, 193, 256, 257, 300, 384, 385]
   w = [(torch.randn(F, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16) for _ in range(experts)]
   ints = dict(dtype=torch.int32, device="cuda")
@@ -152,6 +152,12 @@ def test_tiles_that_the_kernel_plans(experts, F):
       want, size = rows @ w[e].double().t(), rows.abs() @ w[e].double().abs().t()
       slack = size * (K + 8) * 2.0 ** -24 + want.abs() * 2.0 ** -8 + 1e-30  # fp32 sums of K products
       assert bool(((got[first[e]:first[e + 1]].double() - want).abs() <= slack).all()), (spread, e, counts[e])
+
+
+@pytest.mark.parametrize("experts,F", [(8, 4096), (65, 272), (130, 48), (250, 16)])
+def test_more_tiles_that_the_kernel_plans(experts, F):
+  """As many blocks as it plans of long rows only"""
+  test_tiles_that_the_kernel_plans(experts, F, 4224)
 
 
 def test_tokens_past_four_gigabytes():

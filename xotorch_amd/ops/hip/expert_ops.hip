@@ -480,7 +480,7 @@ struct Plan { int most, tiles, end; };
 DEVINL int tiles_of(unsigned rows, int most) {
   return most == 256 ? (rows + 255) / 256 : most == 192 ? (rows + 191) / 192 : (rows + 127) / 128;
 }
-// Where the chip has few rounds of blocks, what the last of them leaves idle counts for more
+// Where blocks are few (launch_tiles), what the last round of them leaves idle counts for more
 // than what smaller tiles cost: 256, 192 or 128 rows, by the time that the rounds take, of
 // which a block of n rows takes 0.4 + 0.00375 n, cut in two 0.62 of that. All blocks find
 // the same. us of the down product of 8 experts of 4096 x 14336, two of them a token, with 256
@@ -725,14 +725,22 @@ static void launch_tiles(const W& w, const Tensor& x, const Tensor& token, const
   // tokens (1000 rows) 1590, 1504
   const int group = pairs / (a.E * (int)tile) + 1;
   // few rows an expert: blocks of 128 weight rows, two to a CU, keep more of them on their
-  // way: 25 and 50 rows 491 and 509 us (553 and 570 with 256); from 75 on 609 (589). So do as
-  // many blocks as CUs, where 256 weight rows make half of that: down of 8 experts of 4096 x
-  // 14336, 75 and 100 rows each, 200 and 208 us (216 and 229)
-  const bool half = tile == 128 && (pairs <= 56 * a.E || (int64_t)(pairs / 128 + a.E) * ((rows + 255) / 256) <= 256);
+  // way: 25 and 50 rows 491 and 509 us (553 and 570 with 256); from 75 on 609 (589). So do those
+  // that make one round of the chip: down of 8 experts of 4096 x 14336, 75 and 88 rows each, 200
+  // and 203 us (220 and 226), but 280 (230) where uneven experts make more tiles than there are
+  // CUs. From 88 rows on average on one expert in eight is taken to have a tile more, from 112 on one
+  // in two. Experts of all sizes: 1.25 to 1.45 times as fast where that leaves half of the chip idle,
+  // 1.1 to 1.2 up to the whole of it.
+  const int64_t likely = pairs <= 88 * (int64_t)a.E ? std::min(pairs, a.E) : pairs <= 112 * (int64_t)a.E ? a.E + a.E / 8 : pairs / 128 + 1 + a.E / 2;
+  const bool half = tile == 128 && (pairs <= 56 * (int64_t)a.E || likely * ((rows + 127) / 128) <= 256);
   const int bn = half ? 128 : 256, nf = (rows + bn - 1) / bn;
-  // up to some two rounds of the chip are planned by the kernel, which may make tiles of 128 rows
-  // of them (more of them lose by the wider grid: gate and up of 700 tokens 364, 378)
-  const bool replan = tile == 256 && (int64_t)(pairs / 256 + a.E / 2) * nf < 640;
+  // blocks that leave much of the chip idle, at 256 rows a tile, are planned by the kernel, which may
+  // make tiles of 128 rows of them. The plan takes 1 to 4 us, and its grid is wider; the longer the
+  // rows, the more blocks it is good for. Time with the router's tiles over time with the plan, on
+  // average: up to 64 blocks 1.22 to 1.3 (K < 512: 1.09); to 128 0.88 (K < 512), 0.96 (< 1024), 1.0 (<
+  // 2048), 1.05 (longer); to 256 0.85, 0.94, 0.99, 1.02 (< 4096), 1.05; to 384 0.86, 0.91, 0.96, 0.98, 1.0
+  // (from 8192 on 1.01); to 512 0.99 at best
+  const bool replan = tile == 256 && (int64_t)std::max(a.E, pairs / 256 + 1) * nf <= std::max(64, std::min(a.kp / 16, 384));
   const int most_tiles = replan ? pairs / 128 + std::min(pairs, a.E) : max_tiles;
   const dim3 grid(((most_tiles * nf + 7) / 8 + (tile == 256 ? DIE_CUS / 2 : 0)) * 8);
   auto run = [&](auto kernel, int lds) {
