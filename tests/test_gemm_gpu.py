@@ -35,7 +35,8 @@ def test_products(M, N, K):
 
 
 # rows of 4 numbers more than pieces of 8: whole sums and parts of them, tiles of 128 and 256
-@pytest.mark.parametrize("M,N,K", [(65, 68, 128), (300, 4100, 192), (100, 260, 4096), (1001, 12, 64), (700, 18308, 128), (2048, 516, 2048)])
+@pytest.mark.parametrize("M,N,K", [(65, 68, 128), (300, 4100, 192), (100, 260, 4096), (1001, 12, 64), (700, 18308, 128), (2048, 516, 2048),
+                                   (65, 128256, 128), (300, 100_004, 64), (1000, 151936, 64)])  # the last three a vocabulary's
 def test_products_of_half_pieces(M, N, K):
   from xotorch_amd.ops import train_ops
   x, w = _random(M, M, K), _random(N, N, K)

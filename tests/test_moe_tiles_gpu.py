@@ -93,11 +93,12 @@ def test_rows_of_an_expert(tile, K, F, swiglu, few):
 
 @pytest.mark.parametrize("rows", [[129, 160, 161, 224, 225], [150, 0, 200, 300, 450, 33], [96, 97, 320, 321, 447, 448]])
 @pytest.mark.parametrize("swiglu", [False, True])
-def test_shares_of_rows_in_steps_of_32(rows, swiglu):
+@pytest.mark.parametrize("F", [528, 3600])  # few blocks, whose tiles the kernel plans, and the router's tiles
+def test_shares_of_rows_in_steps_of_32(rows, swiglu, F):
   """Tiles of 160 and 224 rows, whole and cut in two: what one row gives does not depend on its tile's form."""
   from xotorch_amd.ops.mixer_ops import load_hip
   hip = load_hip("_hip_experts")
-  K, F, n = 320, 528, sum(rows)
+  K, n = 320, sum(rows)
   g = torch.Generator(device="cuda").manual_seed(n)
   x = torch.randn(n, K, generator=g, device="cuda").to(torch.bfloat16)
   w = [(torch.randn((2 if swiglu else 1) * F, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16) for _ in rows]
@@ -118,12 +119,14 @@ def test_shares_of_rows_in_steps_of_32(rows, swiglu):
     if c:
       alone = product([c], x[first[e]:first[e + 1]].contiguous(), [w[e]], 128)[0]
       assert torch.equal(got[first[e]:first[e + 1]], alone)
-  size = x.double().abs().sum(1).max() * max(t.double().abs().max() for t in w)
-  want = x[:rows[0]].double() @ w[0].double().t()
-  if swiglu:
-    gate, up = want.chunk(2, -1)
-    want = torch.nn.functional.silu(gate) * up
-  assert bool(((got[:rows[0]].double() - want).abs() <= want.abs() * 2.0 ** -8 + size * size * K * 2.0 ** -22).all())
+      some, weights = x[first[e]:first[e + 1]].double(), w[e].double()
+      want, size = some @ weights.t(), some.abs() @ weights.abs().t() * (K + 8) * 2.0 ** -24  # fp32 sums of K products
+      if swiglu:
+        (gate, up), (sg, su) = want.chunk(2, -1), size.chunk(2, -1)
+        want = torch.nn.functional.silu(gate) * up
+        # silu's slope is at most 1.1; its hardware exponential and reciprocal are off by some 2^-20
+        size = (1.1 * sg + gate.abs() * 2.0 ** -19) * (up.abs() + su) + su * gate.abs()
+      assert bool(((got[first[e]:first[e + 1]].double() - want).abs() <= size + want.abs() * 2.0 ** -8 + 1e-30).all()), c
 
 
 @pytest.mark.parametrize("experts,F", [(1, 2048), (8, 4096), (65, 272), (130, 48), (250, 16)])  # one, some or many a lane
@@ -177,6 +180,28 @@ def test_tokens_past_four_gigabytes():
     args = torch.tensor([0, n], **ints), torch.tensor(listed, **ints), tile, True
     near = hip.expert_product_of(x[token].contiguous(), [w], torch.arange(n, **ints), *args)
     assert torch.equal(hip.expert_product_of(x, [w], token.to(torch.int32), *args), near)
+
+
+@pytest.mark.parametrize("kind", ["GATED", "RELU2"])
+@pytest.mark.parametrize("tile,F", [(128, 32), (128, 33024), (256, 32)])  # half blocks, whole ones, large tiles
+def test_stacked_weights_of_tokens_past_four_gigabytes(kind, tile, F):
+  """The same with rows that end within a step."""
+  from xotorch_amd.ops.mixer_ops import load_hip
+  hip = load_hip("_hip_experts")
+  T, K, kp, n = (1 << 20) + 40, 2056, 2112, 300
+  x = torch.zeros(T, K, device="cuda", dtype=torch.bfloat16)
+  g = torch.Generator(device="cuda").manual_seed(T)
+  token = torch.cat([torch.randint(0, T, (n - 2,), generator=g, device="cuda"), torch.tensor([0, T - 1], device="cuda")])
+  x[token] = torch.randn(n, K, generator=g, device="cuda").to(torch.bfloat16)
+  F = F if kind == "RELU2" else max(16, F // 32 * 16)
+  w = torch.zeros(*((1, 2, F, kp) if kind == "GATED" else (1, F, kp)), device="cuda", dtype=torch.bfloat16)
+  w[..., :K] = (torch.randn(*w.shape[:-1], K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+  ints = dict(dtype=torch.int32, device="cuda")
+  tiles = [(0, r) for r in range(0, n, tile)]
+  listed = tiles + [(-1, 0)] * (n // tile + 1 - len(tiles)) + [(-1, len(tiles))]
+  args = torch.tensor([0, n], **ints), torch.tensor(listed, **ints), tile, getattr(hip, kind), 1.0, 100.0, 0.0
+  near = hip.expert_product(x[token].contiguous(), w, torch.arange(n, **ints), *args)
+  assert torch.equal(hip.expert_product(x, w, token.to(torch.int32), *args), near) and bool(near.any())
 
 
 @pytest.mark.parametrize("swiglu", [False, True])

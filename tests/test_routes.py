@@ -117,6 +117,23 @@ def test_the_rules_know_how_k_is_split():
 
 
 @pytest.mark.gpu
+def test_small_weights_are_split_for_one_round():
+  """Parts that the kernels make, beside those that the rules count: fewer of up to 20 10^6 numbers, where
+  that fills a round of the chip, and one only where the rules say so."""
+  from xotorch_amd import ops
+  hip = ops._tile()
+  for N, K, parts in [(3584, 3584, 4), (4608, 3584, 3), (6400, 1024, 2), (6336, 1024, 4), (8192, 2432, 2), (8192, 2496, 4),
+                      (904, 4864, 16), (2044, 1536, 6), (66, 1024, 4), (28672, 4096, 1), (64, 128, 1)]:
+    assert hip.parts_of(N, K) == parts
+    if N % 4 == 0:
+      x, w = torch.zeros(3, K, device="cuda", dtype=torch.bfloat16), torch.zeros(N, K, device="cuda", dtype=torch.bfloat16)
+      assert ops.tile_parts(x, w).shape == (parts, 3, N)
+  for N in (1, 64, 65, 896, 1536, 4608, 6336, 8192, 9536, 14336, 14337, 28672, 28673, 151936, 1 << 26):
+    for K in (64, 192, 256, 448, 512, 960, 1024, 2048, 3584, 4032, 4096, 16384, 53248):
+      assert hip.parts_of(N, K) <= ops.tile_splits(N, K) and (hip.parts_of(N, K) == 1) == (ops.tile_splits(N, K) == 1)
+
+
+@pytest.mark.gpu
 def test_the_rules_know_how_k_of_gates_is_split():
   from xotorch_amd import ops
   for N in (16, 1024, 10176, 10192, 16384, 16400, 20416, 20480, 20496, 28672, 1 << 26):
@@ -253,3 +270,10 @@ def test_products_of_more_rows_than_kernels_index():
   assert train_ops.forward_wins(64, 64, most) and train_ops.input_wins(64, most, 64) and train_ops.weight_wins(most, 64, 64)
   for more in (most + 8, most + 64):
     assert not train_ops.forward_wins(300, 4, more) and not train_ops.input_wins(64, more, 64) and not train_ops.weight_wins(more, 64, 64)
+
+
+def test_products_of_a_vocabulary():
+  from xotorch_amd.ops import train_ops
+  for M, N, K, own in [(64, 128256, 2048, False), (65, 128256, 2048, True), (1000, 128256, 4096, True), (1001, 128256, 4096, False),
+                       (300, 128256, 4160, False), (300, 100_000, 896, True), (300, 99_996, 896, False), (300, 151_938, 896, False)]:
+    assert train_ops.forward_wins(M, N, K) == own, (M, N, K)

@@ -153,3 +153,20 @@ def test_rest_of_a_layer_is_its_parts(m, D, H, I):
     want = ops.parts_add_norm(ops.tile_parts(ops.tile_swiglu(n, gu), down), h, after, 1e-6, rounded=True)
     got, alone = ops.tile_rest(heads, wo, x, post, 1e-5, gu, down, after, 1e-6), ops.tile_rest(heads, wo, x, post, 1e-5, gu, down)
   assert len(got) == 2 and len(alone) == 1 and torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]) and torch.equal(alone[0], want[0])
+
+
+# rows whose offsets take 32 bits just so, and more: by mfma_tile.h, and by several blocks of 64 rows of x each
+@pytest.mark.parametrize("K", [1 << 22, (1 << 22) + 64])
+@pytest.mark.parametrize("m,N", [(65, 8), (130, 8), (130, 6)])
+def test_products_of_longest_rows(m, N, K):
+  from xotorch_amd import ops
+  g = torch.Generator(device="cuda").manual_seed(m + N)
+  x = torch.randn(m, K, generator=g, device="cuda", dtype=torch.bfloat16)
+  w = torch.randn(N, K, generator=g, device="cuda", dtype=torch.bfloat16) * 2.0 ** -11
+  want = torch.stack([w.double() @ row.double() for row in x])
+  # K / 32 additions of 32 products at most; sums of random signs stay within six standard deviations
+  slack = x.norm(dim=1, keepdim=True, dtype=torch.float64) * w.norm(dim=1, dtype=torch.float64) * K ** -0.5 * 6 * (K / 32 + 8) * 2.0 ** -24
+  with torch.no_grad():
+    assert bool(((ops.tile_linear(x, w).double() - want).abs() <= slack + want.abs() * 2.0 ** -8).all())
+    if N % 4 == 0:
+      assert bool(((ops.tile_parts(x, w).double().sum(0) - want).abs() <= slack).all())

@@ -5,8 +5,8 @@
 // llm_utils.py:465-500.)
 //
 // What bounds them is the weights' way from memory, for which every CU wants some
-// 48 KB on its way; library tiles leave that to few blocks. A block owns 64 or 128
-// weight rows and all rows of x (up to 128, more by mfma_tile.h), and walks its part of
+// 48 KB on its way; library tiles leave that to few blocks. A block owns 64 to 128
+// weight rows and all rows of x (up to 64, more by mfma_tile.h), and walks its part of
 // k in steps of 64 through a ring of LDS buffers that are filled by direct loads: rows of 128
 // bytes, so whole lines, the 16-byte pieces of row r permuted by r & 7 in the global
 // address, which spreads fragment reads over the banks. Where the weight rows alone
@@ -424,7 +424,8 @@ static void launch_tile(TileArgs a) {
 // [N, K], 64-row or (deeper, fewer to a CU) first:
 //   m 32: [2048, 2048] in 128 blocks 4.1, 4.6; [3584, 18944] in 224 25.0, 22.6
 //   m 64: [2048, 2048] 4.6, 5.6; [28672 -> 8192] 91.0, 78.3
-// From 65 rows of x on by mfma_tile.h, all rows in one block. Up to 128: where blocks make one
+// From 65 rows of x on by mfma_tile.h, all rows in one block but where that leaves half of the
+// chip idle. Up to 128: where blocks make one
 // round and their sums are long, four waves and more on the way, else eight, two blocks to a
 // CU; us, the former first (and by the loop above, m 128):
 //   m 96 and 128: [8192, 28672] 79 and 87, 82 and 90 (89); gate [28672, 4096] 42 and 46, 51
@@ -515,7 +516,7 @@ static void run_tile(TileArgs a) {
   } else if (a.m <= 64) {
     if (units >= 200) launch_tile<128, 64, 3, END>(a);
     else launch_tile<64, 64, 4, END>(a);
-  } else if (a.K > 1 << 22) {  // offsets of 256 rows take more than 32 bits
+  } else if (a.K > 1 << 22) {  // from 2^23 on offsets of 256 rows take more than 32 bits
     launch_tile<128, 64, 3, END>(a);
   } else {
     if constexpr (END == GATED) {
@@ -695,6 +696,7 @@ std::vector<Tensor> tile_rest(Tensor heads, Tensor wo, Tensor x, Tensor post, do
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("tile_rest", &tile_rest);
   m.def("tile_splits", [](int64_t n, int64_t k) { return splits_of((int)n, (int)(k / 64)); });
+  m.def("parts_of", [](int64_t n, int64_t k) { return parts_of((int)n, (int)(k / 64)); });
   m.def("gate_waves", [](int64_t rows, int64_t m) { return gate_waves((int)rows, (int)m); });
   m.def("gate_splits", [](int64_t n, int64_t k) { return gate_splits((int)n, (int)(k / 64)); });
   m.def("gate_tile", [](int64_t rows, int64_t m) { return gate_tile((int)rows, (int)m); });
