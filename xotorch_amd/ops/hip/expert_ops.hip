@@ -482,7 +482,8 @@ DEVINL int tiles_of(unsigned rows, int most) {
 }
 // Where blocks are few (launch_tiles), what the last round of them leaves idle counts for more
 // than what smaller tiles cost: 256, 192 or 128 rows, by the time that the rounds take, of
-// which a block of n rows takes 0.4 + 0.00375 n, cut in two 0.62 of that. All blocks find
+// which a block of n rows takes 0.4 + 0.00375 n, cut in two 0.62 of that (rows as they are shared
+// out, not as the form that takes them has: gate_product's plan rounds to 32). All blocks find
 // the same. us of the down product of 8 experts of 4096 x 14336, two of them a token, with 256
 // and so: 2100 tokens 486, 443; 1000 tokens 305, 246; 1500 and 700, which stay with 256, 301
 // and 214.

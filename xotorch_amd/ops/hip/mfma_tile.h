@@ -15,8 +15,14 @@
 // reads for a product, but two waves a SIMD begin and end a block faster. 256 blocks of 256 x
 // 256, of 512, 1024 and 4096 of k, us, four first: 22.1, 21.0; 33.7, 32.4; 100, 99; of 128 x
 // 256 14.4, 13.7; 20.5, 19.6; 58.1, 56.9; where both operands are columns of 256 x 256 25.0,
-// 21.9; 37.0, 33.1; 109, 104. Four where rows of x are a multiple of 32 alone, and where they
-// took less time.
+// 21.9; 37.0, 33.1; 109, 104. So where rows of x fill their tiles eight gain 1 to 5%, more of short
+// sums; but only four make tiles of any multiple of 32 rows of x, eight of 64. Experts and gates of
+// prompts, whose rows are shared out, take four: 300 and 600 rows by [28672, 4096] 70 and 137, 87 and
+// 140; 600 by [16384, 8192] 132, 152; by [16384, 2048] 38.6, 42.0; 8 experts of 4096 x 14336, 250 rows
+// each, 467 and 235, 478 and 244; from 1000 rows of 1024 and more on 0.97 to 1.02 (1500 wide 1.04 to 1.09).
+// Rows of less than 1024 lose by it: 3000 by [9728, 896] 53.0, 50.1 (600 16.7, 14.7; 2000 37.6, 41.1), by
+// [9728, 256] 25.5, 23.2; 16 experts of 1024 x 512, 250 rows each, 20.4, 18.8. One set of tiles serves
+// all, as two would double the largest kernels.
 //
 // What bounds large tiles is power: [6144, 4096] x [28672, 4096]^T, 256 x 256 a block, takes
 // 2390 to 2500 cycles a step of the 2048 that its matrix instructions need, at 1.8 GHz of 2.4
