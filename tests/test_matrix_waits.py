@@ -115,3 +115,18 @@ def test_matrix_instructions_by_hand_are_waited_for(name, tmp_path):
         i, j = found[0]
         bad[kernel] = len(found), j - i, " ".join(code[i][:2]), " ".join(code[j][:2])
   assert some and not bad, bad
+
+
+@pytest.mark.parametrize("name,kernels", [("_hip_lora", "sums_kernel"), ("_hip_gemm", "gemm_kernel")])
+def test_what_is_read_across_is_multiplied(name, kernels, tmp_path):
+  """Transposing reads from LDS are hidden from the compiler like the products, which may then be of other
+  registers: all that they bring are operands."""
+  if not (OPS / f"{name}.so").exists() or not shutil.which("objcopy") or not (ROCM / "llvm-objdump").exists():
+    pytest.skip("no built extension, or no tools to look through it")
+  some = 0
+  for kernel, code in _kernels(name, tmp_path):
+    read = set().union(*(_registers(rest.split(",")[0]) for op, rest, _ in code if op.startswith("ds_read_b64_tr")))
+    multiplied = set().union(*(_registers(",".join(re.split(r",(?![^\[]*\])", rest)[1:3])) for op, rest, _ in code if op.startswith("v_mfma")))
+    some += kernels in kernel and bool(read)
+    assert kernels not in kernel or read <= multiplied, (kernel, sorted(read - multiplied))
+  assert some

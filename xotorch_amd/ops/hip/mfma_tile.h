@@ -87,7 +87,8 @@ struct StepSource {
 
 // One operand's fragments of 32 of k, N tiles of 16 rows, and where a lane reads them. By
 // hand: the compiler would make every read wait for all pending loads to LDS. What is read
-// is used, after `landed` and `whole`.
+// is used after `landed`: fragment i as [i] by instructions that the compiler knows, as f[i],
+// behind `whole` too, by those that it does not (`mul`).
 //
 // Rows: k lies along a row, as above.
 template <int N>
@@ -142,12 +143,12 @@ struct ColFrags {
       asm volatile("" : "+v"(hi[i]));
     }
   }
-  DEVINL bf16x8 operator[](int i) const { return f[i]; }
+  DEVINL bf16x8 operator[](int i) const { return __builtin_shufflevector(lo[i], hi[i], 0, 1, 2, 3, 4, 5, 6, 7); }
   // both halves where they are multiplied, before `written`
   DEVINL void whole() {
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-      f[i] = __builtin_shufflevector(lo[i], hi[i], 0, 1, 2, 3, 4, 5, 6, 7);
+      f[i] = (*this)[i];
       asm volatile("" : "+v"(f[i]));
     }
   }
@@ -253,8 +254,8 @@ DEVINL void walk(floatx4 (&acc)[R][C], W w, X x, int steps, StepW stepw, LoadW l
     constexpr int i = decltype(number)::value;
     each<C>([&](auto column) {
       constexpr int j = decltype(column)::value;
-      if constexpr (i == R - 1 && j == C - 1 && decltype(half)::value == 0) mul_last(acc[i][j], fw[i], fx[j], more);
-      else mul(acc[i][j], fw[i], fx[j]);
+      if constexpr (i == R - 1 && j == C - 1 && decltype(half)::value == 0) mul_last(acc[i][j], fw.f[i], fx.f[j], more);
+      else mul(acc[i][j], fw.f[i], fx.f[j]);
       if constexpr (j == C / 2 - 1 || j == C - 1)
         each<PER>([&](auto n) { read(std::integral_constant<int, (i * 2 + (j == C - 1)) * PER + decltype(n)::value>(), half, gw, gx, wu, xu); });
     });
