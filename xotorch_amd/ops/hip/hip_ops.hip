@@ -849,9 +849,13 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
 // exchange maxima and rescale only where one grows (a maximum that may lag costs
 // precision: the largest probability is then rounded too). Where the rows make too
 // few blocks, the keys are split and the parts merged.
-// us, and as it was with a block per head and probabilities through LDS: 6001 tokens,
-// 32 heads on 8 338 (873 TFLOP/s; 1309); 16 x 512, 64 on 8 137 (352); 256 tokens after
-// 1280, 28 on 4 27 (150).
+// A SIMD's vector port is the narrowest: a product of 16 x 16 x 32 holds it for 8 of its 16
+// cycles, other instructions take 5, exponentials 9. So the scale is part of the exponents'
+// multiply-add, a maximum one instruction (`larger`), and what never changes stays in
+// registers. us, with 8 + 8 instructions for those, 11 for 8 numbers' maximum and 3 moves a
+// tile, and so: 6001 tokens, 32 heads on 8 327, 310 (952 TFLOP/s); 16 x 512, 64 on 8 134, 129;
+// 2000 tokens, 32 heads of 64 on 8 43, 40. (32 x 32 x 16, which hold the port half as long, take
+// more power: 324, 139 and 40.)
 // ---------------------------------------------------------------------------
 
 DEVINL floatx4 mma16(const bf16x8& a, const bf16x8& b, floatx4 c) {
@@ -893,6 +897,17 @@ template <int HD> struct FlashLds {
                "\n\tds_read_b128 %3, %4 offset:" #O3 "\n\ts_waitcnt lgkmcnt(0)"                                       \
                : "=&v"(F[0]), "=&v"(F[1]), "=&v"(F[2]), "=&v"(F[3])                                                    \
                : "v"(A))
+
+// The larger of two numbers: fmaxf() quiets what the compiler has not seen to be no signalling
+// NaN, an instruction a number. `inf` is infinity, which the compiler must not know of.
+DEVINL float larger(float x, float y, float inf) { return __builtin_amdgcn_fmed3f(x, y, inf); }
+DEVINL float hidden_inf() {
+  float inf = INFINITY;
+#ifdef __HIP_DEVICE_COMPILE__
+  asm("" : "+s"(inf));
+#endif
+  return inf;
+}
 
 // maximum over the four lanes that hold a query's scores
 DEVINL float quad_max(float v) {
@@ -955,7 +970,9 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(FlashArgs a) {
     }
   };
 
-  float m[QT];
+  // scores times `scale` are exponents of two; with a cap they are capped before
+  const float scale = SIDE && a.cap > 0.f ? 1.4426950408889634f : a.scale, by_cap = SIDE ? a.scale / a.cap : 0.f, inf = hidden_inf();
+  float m[QT], least[QT];  // largest score yet, and that times -scale
   floatx4 o[QT][VG], l[QT];  // l: the same sum in all four
   bf16x8 ones;
 #pragma unroll
@@ -963,10 +980,14 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(FlashArgs a) {
 #pragma unroll
   for (int t = 0; t < QT; ++t) {
     m[t] = -1e30f;
+    least[t] = 0.f;
     l[t] = (floatx4)(0.f);
 #pragma unroll
     for (int g = 0; g < VG; ++g) o[t][g] = (floatx4)(0.f);
   }
+#ifdef __HIP_DEVICE_COMPILE__
+  asm("" : "+v"(ones));  // else made anew for each product
+#endif
   // key rows of the two products of 16: row i is position i / 4 * 8 + i % 4, and 4 more
   const int p = (col >> 2) * 8 + (col & 3);
   const unsigned base = (unsigned)(size_t)(lds_void*)lds;
@@ -1000,8 +1021,8 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(FlashArgs a) {
         float v[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          v[i] = sc[t][i >> 2][i & 3] * a.scale;
-          if (SIDE && a.cap > 0.f) v[i] = 1.4426950408889634f * a.cap * tanhf(v[i] * (1.f / a.cap));
+          v[i] = sc[t][i >> 2][i & 3];
+          if (SIDE && a.cap > 0.f) v[i] = a.cap * tanhf(v[i] * by_cap);
         }
         if (edge) {
           const int d = pos[t] - p0 - quad * 8;  // distance to this lane's first key
@@ -1012,17 +1033,19 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(FlashArgs a) {
             v[i] = ok ? v[i] : -INFINITY;
           }
         }
-        float top = fmaxf(fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])), fmaxf(fmaxf(v[4], v[5]), fmaxf(v[6], v[7])));
+        float top = larger(larger(larger(v[0], v[1], inf), larger(v[2], v[3], inf), inf),
+                           larger(larger(v[4], v[5], inf), larger(v[6], v[7], inf), inf), inf);
         if (__any(top > m[t])) {
           top = fmaxf(m[t], quad_max(top));
-          const float f = __builtin_amdgcn_exp2f(m[t] - top);
+          const float f = __builtin_amdgcn_exp2f((m[t] - top) * scale);
           m[t] = top;
+          least[t] = -top * scale;
           l[t] *= f;
 #pragma unroll
           for (int g = 0; g < VG; ++g) o[t][g] *= f;
         }
 #pragma unroll
-        for (int i = 0; i < 8; ++i) pf[t][i] = (__bf16)__builtin_amdgcn_exp2f(v[i] - m[t]);
+        for (int i = 0; i < 8; ++i) pf[t][i] = (__bf16)__builtin_amdgcn_exp2f(__builtin_fmaf(v[i], scale, least[t]));
         l[t] = mma16(ones, pf[t], l[t]);
       }
       bf16x8 vf[VG];
@@ -1044,7 +1067,7 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(FlashArgs a) {
 #pragma unroll
       for (int g = 0; g < VG; ++g) *(floatx4*)(a.part + i * HD + g * 16 + quad * 4) = o[t][g];
       if (quad == 0) {
-        a.ml[i * 2] = m[t];
+        a.ml[i * 2] = m[t] * scale;
         a.ml[i * 2 + 1] = sum;
       }
       continue;
