@@ -82,3 +82,36 @@ def test_heads_of_64_in_any_order():
       assert not other.is_contiguous() or other.data_ptr() % 16
       out = ops.attn_prefill(other, c.k, c.v, start, S, c.kp, c.vp).float()
       assert bool(((out - ref).abs() <= ref.abs() * 2.0 ** -6 + 2.0 ** -6).all())  # each rounds probabilities and results
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("few,B,S,H,KVH,start,cap,window", [
+  # short waves: one step of 32 keys for four of them, 4 and 5 steps, last rows of a block of 32, batches, both options
+  (True, 1, 129, 1, 1, 0, 0.0, 0), (True, 1, 19, 7, 1, 108, 0.0, 0), (True, 1, 33, 4, 4, 229, 0.0, 0), (True, 3, 41, 6, 2, 200, 0.0, 0),
+  (True, 1, 256, 28, 4, 500, 0.0, 0), (True, 1, 130, 4, 1, 300, 25.0, 0), (True, 2, 140, 4, 2, 300, 0.0, 50), (True, 1, 300, 2, 1, 0, 0.0, 1),
+  (True, 1, 70, 4, 1, 600, 30.0, 64),
+  # blocks of 128 rows: keys in parts, and whole
+  (False, 1, 3, 6, 2, 4000, 0.0, 0), (False, 1, 5, 4, 2, 4000, 0.0, 100), (False, 1, 2, 4, 1, 4100, 20.0, 0),
+  (False, 5, 500, 30, 10, 0, 0.0, 0), (False, 11, 140, 40, 8, 70, 0.0, 40), (False, 11, 140, 40, 8, 70, 15.0, 0)])
+def test_either_way_of_prompts(hd, few, B, S, H, KVH, start, cap, window):
+  from xotorch_amd.ops import _hip_ops
+  assert _hip_ops.prefill_few(B, S, H, KVH, hd, start) == few
+  g = torch.Generator(device="cuda").manual_seed(S + start)
+  T, rep = start + S, H // KVH
+  t32 = -(-T // 32) * 32
+  q, k, v = (torch.randn(*s, hd, generator=g, device="cuda").to(torch.bfloat16) for s in ((B, S, H), (B, KVH, t32), (B, KVH, t32)))
+  kp = k.view(B, KVH, t32 // 16, 16, hd // 32, 4, 8).permute(0, 1, 2, 4, 5, 3, 6).reshape(B, KVH, t32 // 16, hd // 32, 64, 8).contiguous()
+  vp = v.view(B, KVH, t32 // 32, 4, 8, hd // 16, 16).permute(0, 1, 5, 2, 3, 6, 4).reshape(B, KVH, hd // 16, t32 // 32, 64, 8).contiguous()
+  out = _hip_ops.attn_prefill_mfma(q, kp, vp, start, 0.0, cap, window).double()
+  kd, vd = (t[:, :, :T].double().repeat_interleave(rep, 1) for t in (k, v))
+  qd = q.double().transpose(1, 2)
+  s = qd @ kd.transpose(-1, -2) * hd ** -0.5
+  off = (qd.abs() @ kd.abs().transpose(-1, -2)).amax(-1, keepdim=True) * hd ** -0.5 * ((hd + 4) * 2.0 ** -24)
+  if cap:
+    s = cap * torch.tanh(s / cap)
+  at = torch.arange(start, T, device="cuda")[:, None] - torch.arange(T, device="cuda")[None]
+  hidden = (at < 0) | (at >= window) if window else at < 0
+  p = s.masked_fill(hidden, -torch.inf).softmax(-1)
+  ref, size = (p @ vd).transpose(1, 2), (p @ vd.abs()).transpose(1, 2)
+  bound = size * (2.0 ** -7 + 4 * off.transpose(1, 2)) + ref.abs() * 2.0 ** -8  # as above
+  assert out.shape == ref.shape and bool(((out - ref).abs() <= bound + 1e-6).all())

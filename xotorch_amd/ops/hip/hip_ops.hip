@@ -848,7 +848,8 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
 // multiplied. 64 positions at a time come by direct loads, two buffers deep. Lanes
 // exchange maxima and rescale only where one grows (a maximum that may lag costs
 // precision: the largest probability is then rounded too). Where the rows make too
-// few blocks, the keys are split and the parts merged.
+// few blocks, the waves of one split the keys (flash_few_kernel), or blocks do and the
+// parts are merged.
 // A SIMD's vector port is the narrowest: a product of 16 x 16 x 32 holds it for 8 of its 16
 // cycles, other instructions take 5, exponentials 9. So the scale is part of the exponents'
 // multiply-add, a maximum one instruction (`larger`), and what never changes stays in
@@ -1081,6 +1082,159 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(FlashArgs a) {
       for (int i = 0; i < 4; ++i) v[i] = f2b(o[t][g][i] * f);
       *(ushort4_t*)(dst + g * 16) = v;
     }
+  }
+}
+
+// The same where rows are few (prefill_few): a block owns 32 query rows of one key head, and its
+// four waves take every fourth 32 positions each and put their parts together in LDS, so that
+// no parts go through memory and no second kernel reads them. Fragments come from L2 to
+// registers as the cache holds them, one step ahead: each is read by one wave only. That way
+// bounds it, some 100 GB/s a CU: products are 32 x 32 x 16, whose layout needs one exchange
+// of lanes for a maximum and half of the vector port, and they are short enough for power. us,
+// keys split over blocks and merged, and so: 256 tokens after 1280, 28 heads on 4 25.4, 13.8; 512
+// tokens 21.7, 10.0; 700 24.8, 15.1; 1500 43.2, 33.1; 100 after 512, 32 on 8 12.4, 8.1; 300, 32 heads
+// of 64 on 8 10.4, 5.6. Eight waves: 14.2, 14.0, 20.4, 48.2, 9.0, 7.1.
+DEVINL floatx16 mma32(const bf16x8& a, const bf16x8& b, floatx16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+constexpr int FEW_WAVES = 4, FEW_ROWS = 32;
+// LDS: a wave's results, rows 16 bytes apart, then all waves' maxima and sums
+template <int HD> struct FewLds {
+  static constexpr int ROW = HD * 4 + 16, AT = FEW_WAVES * FEW_ROWS * ROW, ALL = AT + FEW_WAVES * FEW_ROWS * 8;
+};
+template <int HD, bool SIDE>
+__global__ __launch_bounds__(FEW_WAVES * 64, 2) void flash_few_kernel(FlashArgs a) {
+  constexpr int KS = HD / 16, G = HD / 32, ROW = FewLds<HD>::ROW;
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int col = lane & 31, half = lane >> 5;
+  const int rep = a.H / a.KVH, heads = gridDim.x / a.blocks;  // heads: batch rows times key heads
+  // the longest rows first; a key head stays on one die where there are eight of them
+  const int bh = blockIdx.x % heads, block = a.blocks - 1 - blockIdx.x / heads, b = bh / a.KVH, kvh = bh % a.KVH;
+  const int rows = a.S * rep, row0 = block * FEW_ROWS, mine = min(row0 + col, rows - 1), token = mine / rep, pos = a.start + token;
+  const int first_pos = a.start + row0 / rep, last_pos = a.start + min(row0 + FEW_ROWS - 1, rows - 1) / rep;
+  // steps of 32 positions that hold something
+  const int low = SIDE && a.window > 0 ? max(0, first_pos - a.window + 1) >> 5 : 0, end = (last_pos >> 5) + 1;
+  // row i of the keys' fragment is position i with bits 2 and 3 changed round: the lane that holds a
+  // query's probabilities then has what the product with the values wants of it
+  const int p = (col & 19) | (col & 4) << 1 | (col & 8) >> 1;
+  const char* kb = (const char*)(a.k + (size_t)bh * a.T32 * HD) + (p >> 4) * (HD * 32) + (half * 16 + (p & 15)) * 16;
+  const char* vb = (const char*)(a.v + (size_t)bh * a.T32 * HD) + (size_t)(col >> 4) * a.T32 * 32 + (half * 16 + (col & 15)) * 16;
+  bf16x8 kf[KS], vf[2 * G], qf[KS];
+  auto load_k = [&](int step) {
+#pragma unroll
+    for (int c = 0; c < KS; ++c) kf[c] = *(const bf16x8*)(kb + (size_t)step * (HD * 64) + c * 512);
+  };
+  auto load_v = [&](int step) {
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int k = 0; k < 2; ++k) vf[g * 2 + k] = *(const bf16x8*)(vb + (size_t)g * a.T32 * 64 + (size_t)step * 1024 + k * 512);
+  };
+  int step = low + wave;
+  if (step < end) load_k(step);
+  const unsigned short* q = a.q + (size_t)b * a.q_b + (size_t)token * a.q_s + (size_t)(kvh * rep + mine % rep) * HD + half * 8;
+#pragma unroll
+  for (int c = 0; c < KS; ++c) qf[c] = *(const bf16x8*)(q + c * 16);
+  if (step < end) load_v(step);
+  const float scale = SIDE && a.cap > 0.f ? 1.4426950408889634f : a.scale, by_cap = SIDE ? a.scale / a.cap : 0.f, inf = hidden_inf();
+  float m = -1e30f, least = 0.f, l = 0.f;  // as above; l: of this lane's keys
+  floatx16 o[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) o[g] = (floatx16)(0.f);
+  for (; step < end; step += FEW_WAVES) {
+    const int p0 = step * 32;
+    floatx16 sc = (floatx16)(0.f);
+#pragma unroll
+    for (int c = 0; c < KS; ++c) sc = mma32(kf[c], qf[c], sc);
+    if (step + FEW_WAVES < end) load_k(step + FEW_WAVES);
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      v[i] = sc[i];
+      if (SIDE && a.cap > 0.f) v[i] = a.cap * tanhf(v[i] * by_cap);
+    }
+    if (p0 + 31 > first_pos || (SIDE && a.window > 0 && p0 <= last_pos - a.window)) {
+      const int d = pos - p0 - half * 8;  // distance to this lane's first key
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int key = (i & 7) + (i >> 3) * 16;
+        bool ok = key <= d;
+        if (SIDE && a.window > 0) ok = ok && d - key < a.window;
+        v[i] = ok ? v[i] : -INFINITY;
+      }
+    }
+    float tops[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) tops[i] = larger(v[i], v[i + 8], inf);
+#pragma unroll
+    for (int n = 4; n > 0; n /= 2)
+#pragma unroll
+      for (int i = 0; i < n; ++i) tops[i] = larger(tops[i], tops[i + n], inf);
+    if (__any(tops[0] > m)) {
+      const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(tops[0]), __float_as_uint(tops[0]), false, false);
+      const float top = fmaxf(m, fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1])));
+      const float f = __builtin_amdgcn_exp2f((m - top) * scale);
+      m = top;
+      least = -top * scale;
+      l *= f;
+#pragma unroll
+      for (int g = 0; g < G; ++g) o[g] *= f;
+    }
+    bf16x8 pf[2];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) pf[i >> 3][i & 7] = (__bf16)__builtin_amdgcn_exp2f(__builtin_fmaf(v[i], scale, least));
+    const bf16x2 ones = {(__bf16)1.f, (__bf16)1.f};  // sums of the probabilities as they are multiplied
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      l = __builtin_amdgcn_fdot2_f32_bf16((bf16x2){pf[i >> 2][(i & 3) * 2], pf[i >> 2][(i & 3) * 2 + 1]}, ones, l, false);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int g = 0; g < G; ++g) o[g] = mma32(vf[g * 2 + k], pf[k], o[g]);
+    if (step + FEW_WAVES < end) load_v(step + FEW_WAVES);
+  }
+  // the waves' parts, weighed by how far their maxima lie below the largest
+  float2* ml = (float2*)(lds + FewLds<HD>::AT);
+  const float sum = l + __shfl_xor(l, 32);
+  if (half == 0) ml[wave * FEW_ROWS + col] = make_float2(m * scale, sum);
+  __syncthreads();
+  float top = ml[col].x;
+#pragma unroll
+  for (int w = 1; w < FEW_WAVES; ++w) top = fmaxf(top, ml[w * FEW_ROWS + col].x);
+  const float by = __builtin_amdgcn_exp2f(m * scale - top);
+  char* row = lds + (wave * FEW_ROWS + col) * ROW + half * 16;
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      *(floatx4*)(row + (g * 32 + k * 8) * 4) = (floatx4){o[g][k * 4] * by, o[g][k * 4 + 1] * by, o[g][k * 4 + 2] * by, o[g][k * 4 + 3] * by};
+  __syncthreads();
+  // four channels of a row a lane
+  constexpr int LANES = HD / 4, PER = FEW_WAVES * 64 / LANES;
+#pragma unroll
+  for (int r0 = 0; r0 < FEW_ROWS; r0 += PER) {
+    const int r = r0 + threadIdx.x / LANES, c = threadIdx.x % LANES * 4;
+    float2 part[FEW_WAVES];
+    float most = -INFINITY, all = 0.f;
+#pragma unroll
+    for (int w = 0; w < FEW_WAVES; ++w) {
+      part[w] = ml[w * FEW_ROWS + r];
+      most = fmaxf(most, part[w].x);
+    }
+    floatx4 s = (floatx4)(0.f);
+#pragma unroll
+    for (int w = 0; w < FEW_WAVES; ++w) {
+      all += __builtin_amdgcn_exp2f(part[w].x - most) * part[w].y;
+      s += *(const floatx4*)(lds + (w * FEW_ROWS + r) * ROW + c * 4);
+    }
+    if (row0 + r >= rows) continue;
+    const float f = all > 0.f ? 1.f / all : 0.f;
+    ushort4_t y;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) y[i] = f2b(s[i] * f);
+    *(ushort4_t*)(a.out + (((size_t)b * a.S + (row0 + r) / rep) * a.H + kvh * rep + (row0 + r) % rep) * HD + c) = y;
   }
 }
 
@@ -2729,6 +2883,38 @@ torch::Tensor attn_decode_mfma(torch::Tensor q, torch::Tensor kp, torch::Tensor 
   return out;
 }
 
+// What the keys of a prompt are split in over blocks of 128 rows. As many blocks as are on the
+// chip at once, two a CU, of two tiles of 64 positions at
+// least; or some more, if the last ones, which come first in the sequence, are so short
+// that this costs less than the longest gain (a block's begin and end take as long as two
+// tiles). us: 256 tokens after 1280, 56 blocks in 9 parts 27, in 10 33; 2000 tokens, 188
+// blocks in 2 parts 49, in 3 42
+static int prefill_splits(int64_t whole, int64_t start, int64_t S) {
+  const int tiles = (int)((start + S + 63) / 64);
+  auto takes = [&](int64_t n) {
+    return (double)tiles / n + 2 + (whole * n > 512 ? (double)((start + 63) / 64 + 1) / n + 2 : 0.0);
+  };
+  const int64_t fit = 512 / whole, parts = fit >= 1 && (512 % whole == 0 || takes(fit) <= takes(fit + 1)) ? fit : fit + 1;
+  return (int)std::max<int64_t>(1, std::min<int64_t>({parts, tiles / 2, 16}));
+}
+
+// Whether flash_few_kernel takes a prompt: by what either way takes, us. Its own: a begin and end
+// for every 256 blocks, and the steps of 32 positions of a CU, or of one block alone; the other's: the longest
+// block's tiles, and the parts' way through memory (12 bytes a number at 6 TB/s) or how full the
+// chip is. Of 315 prompts of 9 to 4000 tokens after 0 to 7000, 1 to 32 at a time, heads of
+// 64 and 128, 1 to 8 to a key head, it takes 203, in 0.40 to 0.98 of the other's time, on average 0.64; its
+// errors against 64 bits are 0.97 to 1.05 of the other's, on average 0.999.
+static bool prefill_few(int64_t B, int64_t S, int64_t H, int64_t KVH, int64_t HD, int64_t start) {
+  const int64_t rows = S * (H / KVH), whole = (rows + 127) / 128 * B * KVH, blocks = (rows + FEW_ROWS - 1) / FEW_ROWS * B * KVH;
+  const int splits = prefill_splits(whole, start, S);
+  if (whole > 512 || (splits == 1 && rows < 128)) return false;
+  const double tiles = (double)((start + S + 63) / 64), wide = HD == 128 ? 1.0 : 0.6;
+  const double fill = blocks <= 256 ? 1.0 : std::max(2.0, (double)(blocks + 100) / 256), steps = (double)(start + S / 2) / 32;
+  const double mine = 2.8 + 2 * fill + steps * (HD == 128 ? 0.165 * fill : std::max(0.14, 0.0825 * fill));
+  return mine < (splits == 1 ? 4 + wide * (1.6 * tiles + 4.5 * whole / 512)
+                             : 6.5 + wide * 1.7 * tiles / splits + (double)rows * B * KVH * splits * HD * 2e-6);
+}
+
 // q: [B, S, H, 64 or 128], heads contiguous; k, v: the packed cache, which holds positions
 // [0, start + S). window 0: none; cap 0: none; scale 0: 1 / sqrt of the head dim.
 torch::Tensor attn_prefill_mfma(torch::Tensor q, torch::Tensor k, torch::Tensor v,
@@ -2764,19 +2950,27 @@ torch::Tensor attn_prefill_mfma(torch::Tensor q, torch::Tensor k, torch::Tensor 
   a.q_s = q.stride(1);
   const int64_t rows = (int64_t)a.S * (a.H / a.KVH);
   CHK(rows <= INT_MAX / 256);
+  auto run = [&](auto kernel, int64_t blocks, int lds) {
+    const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    TORCH_CHECK(e == hipSuccess, "no LDS for attention tiles");
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), lds, cur_stream(), a);
+  };
+  if (prefill_few(B, a.S, a.H, a.KVH, HD, start)) {
+    a.blocks = (int)((rows + FEW_ROWS - 1) / FEW_ROWS);
+    a.splits = 1;
+    const int64_t blocks = (int64_t)a.blocks * B * a.KVH;
+    if (HD == 128) {
+      if (side) run(flash_few_kernel<128, true>, blocks, FewLds<128>::ALL);
+      else run(flash_few_kernel<128, false>, blocks, FewLds<128>::ALL);
+    } else {
+      if (side) run(flash_few_kernel<64, true>, blocks, FewLds<64>::ALL);
+      else run(flash_few_kernel<64, false>, blocks, FewLds<64>::ALL);
+    }
+    return out;
+  }
   a.blocks = (int)((rows + 127) / 128);
   const int64_t whole = (int64_t)a.blocks * B * a.KVH;
-  // as many blocks as are on the chip at once, two a CU, of two tiles of 64 positions at
-  // least; or some more, if the last ones, which come first in the sequence, are so short
-  // that this costs less than the longest gain (a block's begin and end take as long as two
-  // tiles). us: 256 tokens after 1280, 56 blocks in 9 parts 27, in 10 33; 2000 tokens, 188
-  // blocks in 2 parts 49, in 3 42
-  const int tiles = (int)((start + a.S + 63) / 64);
-  auto takes = [&](int64_t n) {
-    return (double)tiles / n + 2 + (whole * n > 512 ? (double)((start + 63) / 64 + 1) / n + 2 : 0.0);
-  };
-  const int64_t fit = 512 / whole, parts = fit >= 1 && (512 % whole == 0 || takes(fit) <= takes(fit + 1)) ? fit : fit + 1;
-  a.splits = (int)std::max<int64_t>(1, std::min<int64_t>({parts, tiles / 2, 16}));
+  a.splits = prefill_splits(whole, start, a.S);
   CHK(whole * a.splits <= INT_MAX);
   torch::Tensor part, ml;
   if (a.splits > 1) {
@@ -2786,19 +2980,13 @@ torch::Tensor attn_prefill_mfma(torch::Tensor q, torch::Tensor k, torch::Tensor 
     a.part = part.data_ptr<float>();
     a.ml = ml.data_ptr<float>();
   }
-  const dim3 grid((unsigned)(whole * a.splits));
-  auto run = [&](auto kernel) {
-    const int lds = 2 * (HD == 128 ? FlashLds<128>::STAGE : FlashLds<64>::STAGE);
-    const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    TORCH_CHECK(e == hipSuccess, "no LDS for attention tiles");
-    hipLaunchKernelGGL(kernel, grid, dim3(256), lds, cur_stream(), a);
-  };
+  const int64_t blocks = whole * a.splits;
   if (HD == 128) {
-    if (side) run(flash_prefill_kernel<128, true>);
-    else run(flash_prefill_kernel<128, false>);
+    if (side) run(flash_prefill_kernel<128, true>, blocks, 2 * FlashLds<128>::STAGE);
+    else run(flash_prefill_kernel<128, false>, blocks, 2 * FlashLds<128>::STAGE);
   } else {
-    if (side) run(flash_prefill_kernel<64, true>);
-    else run(flash_prefill_kernel<64, false>);
+    if (side) run(flash_prefill_kernel<64, true>, blocks, 2 * FlashLds<64>::STAGE);
+    else run(flash_prefill_kernel<64, false>, blocks, 2 * FlashLds<64>::STAGE);
   }
   if (a.splits > 1) {
     const int heads = B * a.KVH, per = 1024 / HD;
@@ -3503,6 +3691,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("q"), py::arg("kp"), py::arg("vp"), py::arg("seq_lens"), py::arg("t_capacity"),
         py::arg("scale") = 0.0, py::arg("softcap") = 0.0, py::arg("window") = 0,
         py::arg("k_scale") = py::none(), py::arg("v_scale") = py::none());
+  m.def("prefill_few", &prefill_few, "whether short waves take a prompt of these sizes (attn_prefill_mfma)");
   m.def("attn_prefill_mfma", &attn_prefill_mfma,
         "causal GQA prefill flash attention on matrix cores (packed cache, hd=128)",
         py::arg("q"), py::arg("kp"), py::arg("vp"), py::arg("start_pos"),
