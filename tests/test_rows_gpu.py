@@ -103,3 +103,11 @@ def test_one_row_summed_as_more_are():
       assert not ops.few_rows(x[:1], lin.weight)
       assert torch.equal(lin(x)[:1], lin(x[:1]))
     assert ops.few_rows(x[:1], lin.weight)
+
+
+# blocks with several row groups, whose waves have none, one, two, three or nine steps of each, and rows about
+# as long as what a thread keeps of them (2048 and 4096 numbers)
+@pytest.mark.parametrize("m,N,K", [(1, 9000, 264), (1, 20000, 600), (2, 9000, 1032), (1, 8300, 2056), (2, 8300, 2048), (1, 4200, 4096),
+                                   (2, 8300, 4104)])
+def test_further_row_groups(m, N, K):
+  test_products_of_normed_rows(m, N, K)

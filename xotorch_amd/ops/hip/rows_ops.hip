@@ -97,16 +97,70 @@ __global__ __launch_bounds__(256) void rows_kernel(RowsArgs a) {
       for (int m = 0; m < M; ++m) p.x[m] = load_row<0>((const bf16_t*)a.x + (size_t)min(m, a.m - 1) * a.K, bytes, k);
   };
   const int n = chunks > ks ? (chunks - ks + KS - 1) / KS : 0;  // this wave's chunks
+  // Numbers of x and of the norm's weights that a thread keeps: loads come back in order, so
+  // that these go out before any weights. us, read behind the first weights, twice, and every
+  // row group waited for by itself, and so: gate [16384, 2048] m 1 13.6, 12.9, m 2 15.1, 13.4; [9728, 896]
+  // 7.2, 6.4; [4608, 3584] m 1 9.1, 8.8, m 2 11.2, 9.6
+  constexpr int KEPT = SRC == PLAIN_X ? 0 : 2, RAW = sizeof(X) / 2;
+  uintx4 kept[KEPT + 1][M][RAW], kept_by[KEPT + 1];
+#pragma unroll
+  for (int p = 0; p < KEPT; ++p) {
+    const int i = min(p * 2048 + (int)threadIdx.x * 8, a.K - 8);
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+      for (int r = 0; r < RAW; ++r) kept[p][m][r] = ((const uintx4*)(x + (size_t)min(m, a.m - 1) * a.K + i))[r];
+    kept_by[p] = *(const uintx4*)(a.norm + i);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  // row m's numbers of piece p
+  auto of_piece = [&](int p, int m, float* v) {
+    if constexpr (SRC == NORM_F32)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = __uint_as_float(kept[p][m][j / 4][j % 4]);
+    else
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        v[j * 2] = __uint_as_float(kept[p][m][0][j] << 16);
+        v[j * 2 + 1] = __uint_as_float(kept[p][m][0][j] & 0xffff0000u);
+      }
+  };
   Part A, B;
   int g = blockIdx.x * PER + wave / KS;
+  // Two chunks are on their way, with a norm, whose blocks have further row groups, also from one
+  // group to the next
+  int ahead_g = g, ahead = 0;
+  auto load_next = [&](Part& p) {
+    if (n == 0 || ahead_g - wave / KS >= a.groups) return;
+    load(p, ahead_g, ks + ahead * KS);
+    if (++ahead == n) {
+      ahead = 0;
+      ahead_g += gridDim.x * PER;
+    }
+  };
   // on their way while the rows of x are normed
-  if (n > 0) load(A, g, ks);
-  if (n > 1) load(B, g, ks + KS);
+  if (SRC != PLAIN_X) {
+    load_next(A);
+    load_next(B);
+  } else {
+    if (n > 0) load(A, g, ks);
+    if (n > 1) load(B, g, ks + KS);
+  }
   if (SRC != PLAIN_X) {
     float ss[M];
 #pragma unroll
-    for (int m = 0; m < M; ++m) ss[m] = 0.f;
-    for (int i = threadIdx.x * 8; i < a.K; i += 2048)
+    for (int m = 0; m < M; ++m) {
+      ss[m] = 0.f;
+#pragma unroll
+      for (int p = 0; p < KEPT; ++p)
+        if (p * 2048 + (int)threadIdx.x * 8 < a.K) {
+          float v[8];
+          of_piece(p, m, v);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) ss[m] += v[j] * v[j];
+        }
+    }
+    for (int i = KEPT * 2048 + threadIdx.x * 8; i < a.K; i += 2048)
 #pragma unroll
       for (int m = 0; m < M; ++m) {
         float v[8];
@@ -126,25 +180,45 @@ __global__ __launch_bounds__(256) void rows_kernel(RowsArgs a) {
 #pragma unroll
       for (int m = 0; m < M; ++m)
         if (m < a.m) *(uintx4*)(xs + m * chunks * 512 + i) = (uintx4)(0u);
-    for (int i = threadIdx.x * 8; i < a.K; i += 2048) {
+    auto put = [&](int m, int i, const float* v, const float* by) {
+      bf16x8 o;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[j] = (__bf16)(v[j] * ss[m] * (by[j] + a.norm_add));
+      *(bf16x8*)(xs + m * chunks * 512 + i) = o;
+    };
+#pragma unroll
+    for (int p = 0; p < KEPT; ++p) {
+      const int i = p * 2048 + (int)threadIdx.x * 8;
+      if (i >= a.K) break;
+      float by[8];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        by[j * 2] = __uint_as_float(kept_by[p][j] << 16);
+        by[j * 2 + 1] = __uint_as_float(kept_by[p][j] & 0xffff0000u);
+      }
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        if (m >= a.m) break;
+        float v[8];
+        of_piece(p, m, v);
+        put(m, i, v, by);
+      }
+    }
+    for (int i = KEPT * 2048 + threadIdx.x * 8; i < a.K; i += 2048) {
       float by[8];
       ld8(a.norm + i, by);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) by[j] += a.norm_add;
 #pragma unroll
       for (int m = 0; m < M; ++m) {
         if (m >= a.m) break;
         float v[8];
         ld8(x + (size_t)m * a.K + i, v);
-        bf16x8 o;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) o[j] = (__bf16)(v[j] * ss[m] * by[j]);
-        *(bf16x8*)(xs + m * chunks * 512 + i) = o;
+        put(m, i, v, by);
       }
     }
     __syncthreads();
   }
-  for (bool first = true; g - wave / KS < a.groups; first = false) {
+  // a row group, whose first chunk is in P
+  auto group = [&](Part& P, Part& Q) {
     typename Sums<COUNT>::V acc = (typename Sums<COUNT>::V)(0.f);
     auto add = [&](Part& p, int i) {
       if (SRC != PLAIN_X)
@@ -162,27 +236,36 @@ __global__ __launch_bounds__(256) void rows_kernel(RowsArgs a) {
                                                              acc[r * M + m], false);
           }
     };
-    if (!first) {
-      if (n > 0) load(A, g, ks);
-      if (n > 1) load(B, g, ks + KS);
-    }
     int i = 0;
-    for (; i + 3 < n; i += 2) {
-      add(A, i);
-      load(A, g, ks + (i + 2) * KS);
-      add(B, i + 1);
-      load(B, g, ks + (i + 3) * KS);
-    }
-    if (n - i == 3) {
-      add(A, i);
-      load(A, g, ks + (i + 2) * KS);
-      add(B, i + 1);
-      add(A, i + 2);
-    } else if (n - i == 2) {
-      add(A, i);
-      add(B, i + 1);
-    } else if (n - i == 1) {
-      add(A, i);
+    if (SRC == PLAIN_X) {
+      for (; i + 3 < n; i += 2) {
+        add(P, i);
+        load(P, g, ks + (i + 2) * KS);
+        add(Q, i + 1);
+        load(Q, g, ks + (i + 3) * KS);
+      }
+      if (n - i == 3) {
+        add(P, i);
+        load(P, g, ks + (i + 2) * KS);
+        add(Q, i + 1);
+        add(P, i + 2);
+      } else if (n - i == 2) {
+        add(P, i);
+        add(Q, i + 1);
+      } else if (n - i == 1) {
+        add(P, i);
+      }
+    } else {
+      for (; i + 1 < n; i += 2) {
+        add(P, i);
+        load_next(P);
+        add(Q, i + 1);
+        load_next(Q);
+      }
+      if (i < n) {
+        add(P, i);
+        load_next(P);
+      }
     }
     float v = spread_sum<COUNT>(acc, lane);
     if (KS > 1) {
@@ -204,6 +287,15 @@ __global__ __launch_bounds__(256) void rows_kernel(RowsArgs a) {
       if (END == ADD_F32) st((bf16_t*)a.y + o, rounded(((const float*)a.res)[o]) + rounded(v));
     }
     g += gridDim.x * PER;
+  };
+  if (SRC == PLAIN_X) {  // blocks for all groups
+    group(A, B);
+    return;
+  }
+  while (g - wave / KS < a.groups) {
+    group(A, B);
+    if (n % 2 == 0 || g - wave / KS >= a.groups) continue;
+    group(B, A);
   }
 }
 
