@@ -225,3 +225,77 @@ def test_rows_past_what_tiles_address(swiglu):
       want = torch.nn.functional.silu(gate) * up
       slack = (1.1 * sg + gate.abs() * 2.0 ** -19) * (up.abs() + su) + su * gate.abs()
     assert bool(((got[lo:hi] - want).abs() <= slack + want.abs() * 2.0 ** -8).all()), e
+
+
+@pytest.mark.parametrize("K,F", [(64, 16), (192, 272), (320, 48), (2048, 80)])  # 1, 3, 5 and 32 steps, the last begun at different places
+@pytest.mark.parametrize("swiglu", [False, True])
+@pytest.mark.parametrize("counts", [[0, 1, 16, 17, 0, 2], [33, 64, 65, 0, 128, 129, 200, 1, 32], [3]])  # 64 weight rows a block, and 128
+def test_few_rows_of_an_expert(K, F, swiglu, counts):
+  from xotorch_amd.ops.mixer_ops import load_hip
+  hip = load_hip("_hip_experts")
+  first = [0]
+  for c in counts:
+    first.append(first[-1] + c)
+  pairs = first[-1]
+  tiles = [(e, r) for e in range(len(counts)) for r in range(first[e], first[e + 1], 128)]
+  listed = tiles + [(-1, 0)] * (pairs // 128 + len(counts) - len(tiles)) + [(-1, len(tiles))]
+  g = torch.Generator(device="cuda").manual_seed(K + F)
+  n = pairs // 2 + 1
+  x = torch.randn(n if swiglu else pairs, K, generator=g, device="cuda").to(torch.bfloat16)
+  token = torch.randint(0, n, (pairs,), generator=g, device="cuda", dtype=torch.int32)
+  w = [(torch.randn((2 if swiglu else 1) * F, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16) for _ in counts]
+  ints = dict(dtype=torch.int32, device="cuda")
+  places = token, torch.tensor(first, **ints), torch.tensor(listed, **ints), 128
+  got = hip.expert_few_of(x, w, *places, swiglu)
+  rows = (x[token.long()] if swiglu else x).double()
+  for e in range(len(counts)):
+    r = rows[first[e]:first[e + 1]]
+    want, size = r @ w[e].double().t(), r.abs() @ w[e].double().abs().t()
+    slack = size * (K + 8) * 2.0 ** -24  # as above
+    if swiglu:
+      (gate, up), (sg, su) = want.chunk(2, -1), slack.chunk(2, -1)
+      want = torch.nn.functional.silu(gate) * up
+      slack = (1.1 * sg + gate.abs() * 2.0 ** -19) * (up.abs() + su) + su * gate.abs()
+    assert bool(((got[first[e]:first[e + 1]].double() - want).abs() <= slack + want.abs() * 2.0 ** -8 + 1e-30).all()), counts[e]
+
+
+@pytest.mark.parametrize("T,E,k,D,I", [(1, 8, 2, 64, 128), (16, 8, 2, 128, 64), (17, 5, 3, 192, 64), (200, 128, 8, 128, 192), (256, 16, 2, 64, 64),
+                                       (300, 64, 4, 64, 64)])
+def test_few_tokens_through_experts(T, E, k, D, I):
+  """Router blocks of 16 tokens whose counts need no scan, and more of them; rows left as they are for a wide sum."""
+  from xotorch_amd.models.config import ModelConfig
+  from xotorch_amd.models.llama import MoEMLP
+  g = torch.Generator(device="cuda").manual_seed(T)
+  moe = MoEMLP(ModelConfig(dim=D, n_experts=E, n_experts_per_tok=k, intermediate_dim=I)).to("cuda", torch.bfloat16)
+  x = torch.randn(T, D, generator=g, device="cuda").to(torch.bfloat16)
+  with torch.no_grad():
+    for p in moe.parameters():
+      p.copy_(torch.randn(p.shape, generator=g, device="cuda") * p.shape[-1] ** -0.5)
+    moe.gate.weight.mul_(4)
+    assert moe._grouped(x) is not None and not moe._by_tiles(x)
+    out, wide = moe(x[None])[0], moe._forward_decode(x, True)
+    assert wide.dtype == torch.float32 and torch.equal(wide.to(torch.bfloat16), out)
+    xd = x.double()
+    logits = xd @ moe.gate.weight.double().t()
+    w, chosen = logits.softmax(-1).topk(k)
+    w = w / w.sum(-1, keepdim=True)
+    ref, size = torch.zeros_like(xd), torch.zeros_like(xd)
+    for e in range(E):
+      token, place = torch.where(chosen == e)
+      gate, up = (xd[token] @ moe.experts[e].gate_up_proj.weight.double().t()).chunk(2, -1)
+      h = torch.nn.functional.silu(gate) * up
+      down = moe.experts[e].down_proj.weight.double()
+      ref.index_add_(0, token, h @ down.t() * w[token, place, None])
+      size.index_add_(0, token, h.abs() @ down.abs().t() * w[token, place, None])
+    # up to 256 tokens logits are bf16, each off by 2^-9 of it: a choice by less than two of these may be another, and
+    # a weight is off by as much, of itself
+    loose = logits.abs().amax(-1) * 2.0 ** -8 if T <= 256 else torch.zeros(T, dtype=torch.float64, device="cuda")
+    near = logits.topk(min(k + 1, E)).values
+    sure = near[:, k - 1] - near[:, -1] > 1e-4 + loose
+    assert sure.float().mean() > 0.8
+    # activations, rows and the sum are bf16 once each; the rest is fp32
+    assert bool(((out.double() - ref).abs() <= size * (2.0 ** -7 + 1.01 * loose[:, None]) + ref.abs() * 2.0 ** -8 + 1e-6)[sure].all())
+    # someone who waits for an expert gets its call
+    seen = []
+    moe.experts[0].register_forward_hook(lambda *a: seen.append(1))
+    assert moe._grouped(x) is None

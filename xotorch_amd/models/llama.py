@@ -388,8 +388,10 @@ class MLP(nn.Module):
 class MoEMLP(nn.Module):
   """Mixtral-class sparse MoE block (top-k routed SwiGLU experts).
 
-  Decode (<=256 tokens, GPU inference) runs a STATIC-SHAPE routed path that
-  is hipGraph-capturable: assignments are argsorted by expert, every expert
+  bf16 inference on the GPU runs as grouped products that read tokens and weights
+  where they lie (`_grouped`); shapes are static and the host sees no count, so that
+  a graph can hold them. Else decode (<=256 tokens) runs a static-shape routed path:
+  assignments are argsorted by expert, every expert
   gets a fixed token capacity C = round_up(T, 32) (top-k experts are distinct
   per token so a single expert can receive at most T assignments — lossless),
   padded slots carry weight 0, and the per-expert GEMMs run as ONE grouped
@@ -455,8 +457,10 @@ class MoEMLP(nn.Module):
     # large-M GEMM). Instead, prefill sorts the token-expert pairs ONCE and
     # runs each expert on a contiguous slice — one argsort + one gather
     # replaces E per-expert where/eq scans over the full assignment list.
-    if x.is_cuda and not torch.is_grad_enabled() and self._by_tiles(flat):
-      return self._forward_prefill_tiles(flat).view(B, S, D)
+    if x.is_cuda and not torch.is_grad_enabled():
+      found = self._grouped(flat)
+      if found is not None:
+        return self._forward_grouped(flat, found).view(B, S, D)
     weights, selected = self._route(flat)
     if x.is_cuda and not torch.is_grad_enabled():
       return self._forward_prefill_sorted(flat, weights, selected).view(B, S, D).to(x.dtype)
@@ -470,32 +474,69 @@ class MoEMLP(nn.Module):
     return out.view(B, S, D).to(x.dtype)
 
   def _by_tiles(self, flat) -> bool:
-    """Whether a prompt goes through the experts as two grouped products by tiles: bf16
-    weights that are one tensor per expert, over 24 rows per expert (fewer leave most
-    of a tile of 128 tokens empty)."""
-    E, k = self.n_experts, self.top_k
-    if flat.dtype != torch.bfloat16 or flat.shape[0] * k <= 24 * E or E > 256 or k > 8 or flat.shape[1] % 64 \
-       or max(flat.shape[1], self.intermediate) > 1 << 22 or self.intermediate % 64 or not flat.is_contiguous() or os.getenv("XOT_FP8_PREFILL", "0") == "1":
-      return False
-    mods = [p for e in self.experts for p in (e.gate_up_proj, e.down_proj)]
-    return (type(self.gate) is nn.Linear and all(type(e) is MLP for e in self.experts) and not _watched(self.gate, *self.experts, *mods)
-            and all(type(p) is XotLinear and p.bias is None for p in mods)
-            and ops.alone(flat, *(p.weight for p in (self.gate, *mods))) and ops._use_hip(flat) and flat.data_ptr() % 16 == 0
-            and all(p.weight.dtype == torch.bfloat16 and p.weight.is_contiguous() and p.weight.data_ptr() % 16 == 0
-                    for p in (self.gate, *mods)))
+    """Whether the grouped products go by tiles of 128 and 256 tokens: over 24 rows
+    per expert (fewer leave most of a tile of 128 tokens empty), up to 256 tokens over 48: 8 experts
+    of 4096 x 14336, two of them a token, us by tiles of up to 64 rows and by these: 128 tokens 460, 508;
+    192 467, 516; 256 738, 563."""
+    return self._many(flat) and self._grouped(flat) is not None
 
-  def _forward_prefill_tiles(self, flat):
+  def _many(self, flat) -> bool:
+    return flat.shape[0] * self.top_k > (24 if flat.shape[0] > 256 else 48) * self.n_experts
+
+  def _expert_weights(self):
+    """The experts' weights (gate and up of all, down of all) where grouped products may read them:
+    bf16, one tensor per expert and projection, whose modules nobody waits for. Else None.
+    Straight from where modules keep things, as a pass through 128 experts asks 256 modules in
+    every layer: 740 us by their attributes, 117 so (40 with 8 experts)."""
+    if self.n_experts > 256 or self.top_k > 8 or self.dim % 64 or self.intermediate % 64 or max(self.dim, self.intermediate) > 1 << 22:
+      return None
+    gate = self._modules["gate"]
+    if type(gate) is not nn.Linear or _watched(gate):
+      return None
+    ups, downs = [], []
+    for e in self._modules["experts"]._modules.values():
+      own = e.__dict__
+      if type(e) is not MLP or own["_forward_hooks"] or own["_forward_pre_hooks"] or "forward" in own:
+        return None
+      held = own["_modules"]
+      for p, found in ((held["gate_up_proj"], ups), (held["down_proj"], downs)):
+        own = p.__dict__
+        if type(p) is not XotLinear or own["_forward_hooks"] or own["_forward_pre_hooks"] or "forward" in own:
+          return None
+        params = own["_parameters"]
+        if params.get("bias") is not None or params.get("weight") is None:
+          return None
+        found.append(params["weight"])
+    return ups, downs
+
+  def _grouped(self, flat):
+    """The experts' weights where tokens go through them as two grouped products, or None."""
+    if flat.dtype != torch.bfloat16 or not flat.is_cuda or self.wp_gate_up_fp8 is not None or not flat.is_contiguous() or not flat.numel() \
+       or (flat.shape[0] > 256 and os.getenv("XOT_FP8_PREFILL", "0") == "1"):
+      return None
+    found = self._expert_weights()
+    if found is None:
+      return None
+    weights = [_own(self._modules["gate"]), *found[0], *found[1]]
+    if not ops.alone(flat) or not ops._use_hip(flat) or any(type(w) not in train_ops.OWN for w in weights):
+      return None
+    from xotorch_amd.ops.mixer_ops import load_hip
+    return found if load_hip("_hip_experts").readable(flat, weights) else None
+
+  def _forward_grouped(self, flat, weights, wide=False):
     """Rows of all (token, expert) pairs are placed by counting, without the host; the
-    products read tokens and weights where they lie."""
+    products read tokens and weights where they lie, of experts that have a row. `wide`: fp32."""
     from xotorch_amd.ops.mixer_ops import load_hip
     hip = load_hip("_hip_experts")
     # tiles of 256 tokens from 110 rows an expert on: 8 experts of 4096 x 14336, two of
     # them a token, us with 128 and 256: 300 tokens 565, 577; 450 607, 602; 620 667, 578
     tile = 256 if flat.shape[0] * self.top_k >= 110 * self.n_experts else 128
-    weight, row, *places = hip.route(flat, self.gate.weight, None, self.top_k, 1, 1, 1.0, True, 0, False, False, tile)
-    h = hip.expert_product_of(flat, [e.gate_up_proj.weight for e in self.experts], *places, True)
-    y = hip.expert_product_of(h, [e.down_proj.weight for e in self.experts], *places, False)
-    return ops._load_hip().moe_combine(y, row, weight)
+    # up to 256 tokens logits are rounded as those of the gate's own call, which hooks bring about
+    weight, row, *places = hip.route(flat, _own(self._modules["gate"]), None, self.top_k, 1, 1, 1.0, True, 0, False, False, tile,
+                                     flat.shape[0] <= 256)
+    product = hip.expert_product_of if self._many(flat) else hip.expert_few_of
+    y = product(product(flat, weights[0], *places, True), weights[1], *places, False)
+    return ops._load_hip().moe_combine(y, row, weight, wide)
 
   def _forward_prefill_sorted(self, flat, weights, selected):
     T, D = flat.shape
@@ -521,6 +562,9 @@ class MoEMLP(nn.Module):
 
   def _forward_decode(self, flat, wide=False):
     """[T, D]; `wide`: fp32, not rounded yet, for a sum with the residual stream."""
+    found = self._grouped(flat)
+    if found is not None:
+      return self._forward_grouped(flat, found, wide)
     T, D = flat.shape
     E, k = self.n_experts, self.top_k
     dev = flat.device
@@ -705,9 +749,9 @@ class ShardedModel(nn.Module):
     return list(range(self.shard.start_layer, self.shard.end_layer + 1))
 
   def pack_decode_weights(self, reserve_bytes: int = 8 << 30) -> int:
-    """Packs second copies of weights in MFMA fragment order: of routed experts, whose
-    grouped decode products read them, and of what is worth the memory otherwise
-    (ops.copy_pays; with fp8 weights everything) - down_proj, lm_head, gate_up, then
+    """Packs second copies of weights in MFMA fragment order: of what is worth the memory
+    (ops.copy_pays; with fp8 weights everything), and of routed experts that grouped products
+    do not read as they lie (MoEMLP._expert_weights) - down_proj, lm_head, gate_up, then
     qkv/o - greedily while at least `reserve_bytes` of HBM stay free (KV caches and
     activations are usually allocated before this is called). Returns bytes packed.
     XOT_PACK=none packs nothing, all whatever can be packed."""
@@ -715,8 +759,12 @@ class ShardedModel(nn.Module):
     if mode == "none" or not torch.cuda.is_available():
       return 0
     groups: List[List[XotLinear]] = [[], [], [], []]
+    unread = set()  # experts whose copies nothing would read
+    if mode != "all" and not ops.fp8_gemm_enabled():
+      unread = {id(p) for m in self.modules() if isinstance(m, MoEMLP) and m.gate.weight.dtype == torch.bfloat16
+                and m._expert_weights() is not None for e in m.experts for p in (e.gate_up_proj, e.down_proj)}
     for name, mod in self.named_modules():
-      if not isinstance(mod, XotLinear) or not mod.packable():
+      if not isinstance(mod, XotLinear) or not mod.packable() or id(mod) in unread:
         continue
       if not ("experts." in name or mode == "all" or ops.fp8_gemm_enabled() or ops.copy_pays(*mod.weight.shape)):
         continue

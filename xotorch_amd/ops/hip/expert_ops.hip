@@ -15,19 +15,21 @@
 // Two element types: bf16 and fp32 (fp32 MFMA throughout).
 
 #include "common.h"
-#include "mfma_tile.h"
+#include "stream_tile.h"
 
 // ---------------------------------------------------------------------------
 // router
 // ---------------------------------------------------------------------------
 
 constexpr int RT = 16;          // tokens of a router block
+constexpr int FEW_BLOCKS = 16;  // of the router, whose counts need no kernel of their own to be scanned
 constexpr int MAX_EXPERTS = 512, MAX_PICK = 16;  // shared ones among the experts
 
 // pick of E experts are chosen, then come top - pick that every token uses, all
 // in all; tile: rows of a tile
 // gate: the weight of these is the sigmoid of one more row of w, else one
-struct RouteArgs { int T, D, E, top, groups, keep, nblk, tile; float scale; int pick, all, softmax, gate; };
+// narrow: logits as bf16, as a linear of their own leaves them
+struct RouteArgs { int T, D, E, top, groups, keep, nblk, tile; float scale; int pick, all, softmax, gate, narrow; };
 
 // RW waves share k. Sixteen lanes choose for a token, J experts each.
 template <typename T, bool WHOLE, int J, int RW>
@@ -82,6 +84,7 @@ __global__ __launch_bounds__(64 * RW) void route_kernel(
         float z = 0.f;
 #pragma unroll
         for (int v = 0; v < RW; ++v) z += part[(v * RT + t) * 65 + (i & 63)];
+        if (a.narrow) z = rounded(z);
         const float s = a.softmax && e < a.E ? z : 1.f / (1.f + expf(-z));
         if (e < a.E) {
           score[t * a.E + e] = s;
@@ -207,8 +210,14 @@ __global__ __launch_bounds__(256) void place_kernel(
     const int* __restrict__ total, const float* __restrict__ weight, int* __restrict__ row, int* __restrict__ token,
     float* __restrict__ by_row, int* __restrict__ first, int2* __restrict__ tiles, int max_tiles, RouteArgs a) {
   __shared__ int at[MAX_EXPERTS], cnt[MAX_EXPERTS], tile_at[MAX_EXPERTS], ends[2];
-  // a single block of the router needs no scan: its counts are the totals
-  for (int e = threadIdx.x; e < a.all; e += 256) cnt[e] = a.nblk == 1 ? before[e] : total[e];
+  // few blocks of the router need no scan (route): their counts are added up here
+  const bool few = a.nblk <= FEW_BLOCKS;
+  for (int e = threadIdx.x; e < a.all; e += 256) {
+    int n = 0;
+    if (few)
+      for (int i = 0; i < a.nblk; ++i) n += before[(size_t)e * a.nblk + i];
+    cnt[e] = few ? n : total[e];
+  }
   __syncthreads();
   if (threadIdx.x < 64) {  // one wave scans, E/64 each
     const int per = (a.all + 63) / 64, lo = threadIdx.x * per, hi = min(lo + per, a.all);
@@ -234,7 +243,10 @@ __global__ __launch_bounds__(256) void place_kernel(
   const int pair = blockIdx.x * 256 + threadIdx.x;
   if (pair < a.T * a.top) {
     const int e = idx[pair], t = pair / a.top;
-    const int r = at[e] + (a.nblk == 1 ? 0 : before[(size_t)e * a.nblk + t / RT]) + rank[pair];
+    int r = at[e] + rank[pair];
+    if (few)
+      for (int i = 0; i < t / RT; ++i) r += before[(size_t)e * a.nblk + i];
+    else r += before[(size_t)e * a.nblk + t / RT];
     row[pair] = r;
     token[r] = t;
     if (by_row) by_row[r] = weight[pair];
@@ -600,6 +612,85 @@ __global__ __launch_bounds__(256) void expert_tile_kernel(
   }
 }
 
+// Few tokens (bf16, one weight tensor per expert; SWIGLU or PLAIN): a block owns BN weight rows of one of the
+// router's tiles and takes its rows, up to 128, by 64 and, the last, 32 or 16. Weights bound it: they stream
+// through LDS (stream_tile.h), of experts that have a row only, at 6.5 TB/s where all have. us of a whole
+// sparse feed-forward in a graph, as it was, with every expert over room for all tokens from copies in
+// fragment order and kernels for logits, choice, places, gathering and the activation, and so: 8 experts of 4096 x 14336, two
+// of them a token: 1 token 501, 157; 2 505, 210; 8 504, 400; 32 503, 438; 128 633, 460; 128 of 2048 x 768, eight of them: 1
+// token 272, 46; 8 270, 110; 32 271, 200; 128 364, 228; errors against 64 bits 0.0036 to 0.0061, 0.0023
+// to 0.0025.
+template <int BN, int BM> struct FewTile : TileShape<BN, BM, BM == 64 ? 3 : 4> {};
+template <int BN> constexpr int few_lds() { return std::max({FewTile<BN, 16>::LDS, FewTile<BN, 32>::LDS, FewTile<BN, 64>::LDS}); }
+template <int KIND, int BN, int BM>
+DEVINL void few_rows_of(const bf16_t* __restrict__ x, const bf16_t* __restrict__ we, const int* __restrict__ token,
+                        bf16_t* __restrict__ y, const GroupArgs& a, int r0, int hi, int turn, bf16_t* buf) {
+  typedef FewTile<BN, BM> Sh;
+  constexpr bool TWO = has_gate(KIND), OWN = of_own_row(KIND);
+  constexpr int PER = TWO ? BN / 2 : BN;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, sub = lane >> 3;
+  const int f0 = blockIdx.x * PER;
+  const bf16_t *wsrc[Sh::WL], *xsrc[Sh::XL];
+#pragma unroll
+  for (int i = 0; i < Sh::XL; ++i) {
+    const int r = BM >= 32 ? (wave * Sh::XL + i) * 8 + sub : wave * 4 + (sub & 3), at = min(r0 + r, hi - 1);
+    xsrc[i] = x + (size_t)(OWN ? at : token[at]) * a.xs + ((lane & 7) ^ (r & 7)) * 8;
+  }
+#pragma unroll
+  for (int i = 0; i < Sh::WL; ++i) {  // TWO: 8 gate rows and the same 8 up rows in turn
+    const int r = (wave * Sh::WL + i) * 8 + sub;
+    const size_t f = TWO ? min(f0 + (r >> 4) * 8 + (r & 7), a.F - 1) + ((r >> 3) & 1 ? (size_t)a.F : 0) : min(f0 + r, a.F - 1);
+    wsrc[i] = we + f * a.kp + ((lane & 7) ^ (r & 7)) * 8;
+  }
+  floatx4 acc[Sh::R][Sh::C];
+  stream_walk<Sh>(acc, buf, wsrc, xsrc, a.K / 64, turn, wave, lane);
+  const int col = lane & 15, quad = lane >> 4;
+#pragma unroll
+  for (int j = 0; j < Sh::C; ++j) {
+    const int row = r0 + Sh::wx(wave) + j * 16 + col;
+#pragma unroll
+    for (int i = 0; i < Sh::R; ++i) {
+      const int w0 = Sh::wr(wave) + i * 16, f = f0 + (TWO ? w0 / 2 : w0) + quad * 4;
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        // lanes of quads 0 and 1 hold gates, those of 2 and 3 the products of up
+        if (TWO) v[r] = siluf(acc[i][j][r]) * __shfl_xor(acc[i][j][r], 32);
+        else v[r] = acc[i][j][r];
+      }
+      if (row < hi && f < a.F && (!TWO || quad < 2)) st4(y + (size_t)row * a.ys + f, v);  // F % 16 == 0
+    }
+  }
+}
+template <int KIND, int BN>
+__global__ __launch_bounds__(256) void expert_few_kernel(const bf16_t* __restrict__ x, Listed w, const int* __restrict__ first,
+                                                         const int* __restrict__ token, const int2* __restrict__ tiles,
+                                                         bf16_t* __restrict__ y, bool turned, GroupArgs a) {
+  extern __shared__ __attribute__((aligned(16))) bf16_t buf[];
+  const int2 tile = tiles[blockIdx.y];
+  const int e = __builtin_amdgcn_readfirstlane(tile.x);
+  if (e < 0) return;
+  int r0 = __builtin_amdgcn_readfirstlane(tile.y);
+  const int hi = min(__builtin_amdgcn_readfirstlane(first[e + 1]), r0 + 128);
+  const bf16_t* we = w.of(e, 0);
+  // where rows lie a multiple of 4 KB apart blocks begin at different places of k (first_step of tile_ops.hip);
+  // an expert's weights begin where all others' do
+  const unsigned group = blockIdx.x * BN / 128 + e * 40503u, steps = a.K / 64;
+  const int turn = turned ? (int)(((group * 2654435761u >> 16) * steps) >> 16) : 0;
+  for (bool again = false; r0 < hi; again = true) {
+    if (again) __syncthreads();  // LDS is read no more
+    const int left = hi - r0;
+    auto go = [&](auto most) {
+      constexpr int BM = decltype(most)::value;
+      few_rows_of<KIND, BN, BM>(x, we, token, y, a, r0, hi, turn, buf);
+      r0 += BM;
+    };
+    if (left > 32) go(std::integral_constant<int, 64>());
+    else if (left > 16) go(std::integral_constant<int, 32>());
+    else go(std::integral_constant<int, 16>());
+  }
+}
+
 // ---------------------------------------------------------------------------
 // residual sum and norm
 // ---------------------------------------------------------------------------
@@ -664,7 +755,7 @@ __global__ __launch_bounds__(256) void add_norm_kernel(
 std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, int64_t> route(Tensor x, Tensor w, OptT correction, int64_t pick,
                                                                   int64_t groups, int64_t keep, double scale,
                                                                   bool softmax, int64_t shared, bool gate,
-                                                                  bool on_input, int64_t tile_of) {
+                                                                  bool on_input, int64_t tile_of, bool narrow) {
   const auto dt = io_type(x);
   check_io(w, dt);
   gate = gate && shared > 0;
@@ -687,7 +778,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, int64_t> route(Tensor x, Tens
   auto idx = torch::empty({T_, top}, ints), rank = torch::empty({T_, top}, ints), row = torch::empty({T_, top}, ints);
   auto counts = torch::empty({all, nblk}, ints), total = torch::empty({all}, ints), first = torch::empty({all + 1}, ints);
   auto token = torch::empty({pairs}, ints), tiles = torch::empty({max_tiles + 1, 2}, ints);
-  const RouteArgs a{T_, D, E, (int)top, (int)groups, (int)keep, nblk, tile, (float)scale, (int)pick, (int)all, softmax, gate};
+  const RouteArgs a{T_, D, E, (int)top, (int)groups, (int)keep, nblk, tile, (float)scale, (int)pick, (int)all, softmax, gate, narrow};
   const hipStream_t stream = cur_stream();
   CHK(groups <= 4 * 65);
   BY_TYPE(dt, {
@@ -706,7 +797,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, int64_t> route(Tensor x, Tens
     else if (E <= 256) { if (few) run(route_kernel<T, true, 16, 16>, 16); else run(route_kernel<T, true, 16, 4>, 4); }
     else run(route_kernel<T, true, MAX_EXPERTS / 16, 4>, 4);
   });
-  if (nblk > 1)
+  if (nblk > FEW_BLOCKS)
     hipLaunchKernelGGL(count_scan_kernel, dim3(all), dim3(256), 0, stream, counts.data_ptr<int>(), total.data_ptr<int>(), nblk);
   hipLaunchKernelGGL(place_kernel, dim3((pairs + 255) / 256), dim3(256), 0, stream, idx.data_ptr<int>(),
                      rank.data_ptr<int>(), counts.data_ptr<int>(), total.data_ptr<int>(), P<float>(weight),
@@ -770,23 +861,31 @@ static void launch_tiles(const W& w, const Tensor& x, const Tensor& token, const
 #undef TILES
 }
 
-// The form with one weight tensor per expert, bf16, by tiles: SWIGLU ([2 F, K], gate rows
-// first) or PLAIN ([F, K]), K % 64 == 0.
-Tensor expert_product_of(Tensor x, std::vector<Tensor> w, Tensor token, Tensor first, Tensor tiles, int64_t tile, bool swiglu) {
+// What the forms with one weight tensor per expert, bf16, take: SWIGLU ([2 F, K], gate rows
+// first; x by token) or PLAIN ([F, K]; x by row), K % 64 == 0
+static GroupArgs listed(Listed& list, const Tensor& x, const std::vector<Tensor>& w, const Tensor& token, const Tensor& first,
+                        const Tensor& tiles, bool swiglu) {
   check_io(x, torch::kBFloat16);
   const int64_t E = w.size();
   CHK(x.dim() == 2 && E >= 1 && E <= MOST_LISTED && ((size_t)x.data_ptr() & 15) == 0);
   for (const Tensor& t : {token, first, tiles}) check_io(t, torch::kInt32);
-  const int K = x.size(1), pairs = token.numel(), F_ = w[0].size(0) / (swiglu ? 2 : 1);
-  CHK(first.numel() == E + 1 && K % 64 == 0 && F_ % 16 == 0 && (swiglu || x.size(0) == pairs));
-  Listed list{};
+  const int K = x.size(1), F_ = w[0].size(0) / (swiglu ? 2 : 1);
+  CHK(first.numel() == E + 1 && K % 64 == 0 && F_ % 16 == 0 && (swiglu || x.size(0) == token.numel()));
   for (int64_t e = 0; e < E; ++e) {
     check_io(w[e], torch::kBFloat16);
     CHK(w[e].dim() == 2 && w[e].size(0) == F_ * (swiglu ? 2 : 1) && w[e].size(1) == K && ((size_t)w[e].data_ptr() & 15) == 0);
     list.w[e] = P<bf16_t>(w[e]);
   }
+  return GroupArgs{K, K, F_, (int)E, K, F_};
+}
+
+// These by tiles.
+Tensor expert_product_of(Tensor x, std::vector<Tensor> w, Tensor token, Tensor first, Tensor tiles, int64_t tile, bool swiglu) {
+  Listed list{};
+  const GroupArgs a = listed(list, x, w, token, first, tiles, swiglu);
+  const int K = a.K, F_ = a.F, pairs = token.numel();
+  const int64_t E = a.E;
   auto y = torch::empty({pairs, F_}, x.options());
-  const GroupArgs a{K, K, F_, (int)E, K, F_};
   if (K <= 1 << 22) {
     launch_tiles(list, x, token, first, tiles, tile, swiglu ? SWIGLU : PLAIN, a, Act{}, nullptr, y);
     return y;
@@ -800,6 +899,33 @@ Tensor expert_product_of(Tensor x, std::vector<Tensor> w, Tensor token, Tensor f
   };
   if (swiglu) stream(expert_stream_kernel<bf16_t, SWIGLU, true>);
   else stream(expert_stream_kernel<bf16_t, PLAIN, true>);
+  return y;
+}
+
+// The same of few tokens, tiles of 128 rows
+Tensor expert_few_of(Tensor x, std::vector<Tensor> w, Tensor token, Tensor first, Tensor tiles, int64_t tile, bool swiglu) {
+  CHK(tile == 128 && tiles.dim() == 2 && tiles.size(0) >= 2 && tiles.size(0) <= 65536);
+  Listed list{};
+  const GroupArgs a = listed(list, x, w, token, first, tiles, swiglu);
+  const int pairs = token.numel();
+  auto y = torch::empty({pairs, a.F}, x.options());
+  const bool turned = a.K <= 16384 && a.K % 2048 == 0;
+  auto run = [&](auto kernel, int lds, int per) {
+    const hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    TORCH_CHECK(err == hipSuccess, "no LDS for experts of few rows");
+    hipLaunchKernelGGL(kernel, dim3((a.F + per - 1) / per, (unsigned)tiles.size(0) - 1), dim3(256), lds, cur_stream(), P<bf16_t>(x), list,
+                       first.data_ptr<int>(), token.data_ptr<int>(), (const int2*)tiles.data_ptr<int>(), M<bf16_t>(y), turned, a);
+  };
+  // 128 weight rows a block from 16 rows an expert on, so that rows are read half as often: us with 64 and so,
+  // the experts above: 64 tokens 450, 445; 128 491, 460; 192 568, 467; 32 tokens 440, 441; the smaller ones
+  // 32 tokens 202, 208; 128 230, 232
+  if (pairs >= 16 * a.E) {
+    if (swiglu) run(expert_few_kernel<SWIGLU, 128>, few_lds<128>(), 64);
+    else run(expert_few_kernel<PLAIN, 128>, few_lds<128>(), 128);
+  } else {
+    if (swiglu) run(expert_few_kernel<SWIGLU, 64>, few_lds<64>(), 32);
+    else run(expert_few_kernel<PLAIN, 64>, few_lds<64>(), 64);
+  }
   return y;
 }
 
@@ -930,11 +1056,18 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("route", &route, "router: sigmoid scores or a softmax over the chosen, group-limited top-k, shared experts; rows of all pairs",
         py::arg("x"), py::arg("w"), py::arg("correction"), py::arg("top"), py::arg("groups"), py::arg("keep"),
         py::arg("scale"), py::arg("softmax") = false, py::arg("shared") = 0, py::arg("gate") = true,
-        py::arg("on_input") = false, py::arg("tile") = 0);
+        py::arg("on_input") = false, py::arg("tile") = 0, py::arg("narrow") = false);
   m.def("expert_product", &expert_product, "grouped product of all (token, expert) pairs, with an activation or plain",
         py::arg("x"), py::arg("w"), py::arg("token"), py::arg("first"), py::arg("tiles"), py::arg("tile"), py::arg("kind"),
         py::arg("alpha") = 0.0, py::arg("limit") = 0.0, py::arg("plus") = 0.0, py::arg("by_row") = py::none());
   m.def("expert_product_of", &expert_product_of, "the same by tiles, with one weight tensor per expert: silu of gate and up, or plain");
+  m.def("readable", [](const Tensor& x, const std::vector<Tensor>& w) {
+    for (const Tensor& t : w)
+      if (!t.is_cuda() || t.device() != x.device() || t.scalar_type() != torch::kBFloat16 || !t.is_contiguous() || ((size_t)t.data_ptr() & 15))
+        return false;
+    return ((size_t)x.data_ptr() & 15) == 0;
+  }, "whether grouped products of x may read these weights: bf16 on its device, contiguous, on 16 bytes");
+  m.def("expert_few_of", &expert_few_of, "the same of few tokens");
   m.attr("PLAIN") = (int)PLAIN;
   m.attr("GATED") = (int)GATED;
   m.attr("RELU2") = (int)RELU2;

@@ -21,7 +21,7 @@
 // rows beside it.
 // (Whether a product is one of these does, and so does how attention cuts its keys.)
 #include "common.h"
-#include "mfma_tile.h"
+#include "stream_tile.h"
 
 struct TileArgs {
   const bf16_t *x, *w, *bias;
@@ -62,42 +62,6 @@ DEVINL int first_step(const TileArgs& a, int row, int len) {
   const unsigned group = END != GATED ? (unsigned)row / 256 : a.turned == 640 ? (unsigned)row / 640 : (unsigned)row / 128;
   return (int)(((group * 2654435761u >> 16) * (unsigned)len) >> 16);
 }
-
-// R fragments from a on and C from b on, 16 rows (2 KB) apart; waits for them
-template <int R, int C>
-DEVINL void read_frags(unsigned a, unsigned b, bf16x8* r, bf16x8* c) {
-#define RD(D, A, O) "ds_read_b128 %" #D ", %" #A " offset:" #O "\n\t"
-#define DONE "s_waitcnt lgkmcnt(0)"
-  if constexpr (R == 1 && C == 1)
-    asm volatile(RD(0, 2, 0) RD(1, 3, 0) DONE : "=&v"(r[0]), "=&v"(c[0]) : "v"(a), "v"(b));
-  else if constexpr (R == 1 && C == 2)
-    asm volatile(RD(0, 3, 0) RD(1, 4, 0) RD(2, 4, 2048) DONE : "=&v"(r[0]), "=&v"(c[0]), "=&v"(c[1]) : "v"(a), "v"(b));
-  else if constexpr (R == 1 && C == 4)
-    asm volatile(RD(0, 5, 0) RD(1, 6, 0) RD(2, 6, 2048) RD(3, 6, 4096) RD(4, 6, 6144) DONE
-                 : "=&v"(r[0]), "=&v"(c[0]), "=&v"(c[1]), "=&v"(c[2]), "=&v"(c[3]) : "v"(a), "v"(b));
-  else if constexpr (R == 2 && C == 1)
-    asm volatile(RD(0, 3, 0) RD(1, 3, 2048) RD(2, 4, 0) DONE : "=&v"(r[0]), "=&v"(r[1]), "=&v"(c[0]) : "v"(a), "v"(b));
-  else if constexpr (R == 2 && C == 2)
-    asm volatile(RD(0, 4, 0) RD(1, 4, 2048) RD(2, 5, 0) RD(3, 5, 2048) DONE
-                 : "=&v"(r[0]), "=&v"(r[1]), "=&v"(c[0]), "=&v"(c[1]) : "v"(a), "v"(b));
-  else {
-    static_assert(R == 4 && C == 2, "");
-    asm volatile(RD(0, 6, 0) RD(1, 6, 2048) RD(2, 6, 4096) RD(3, 6, 6144) RD(4, 7, 0) RD(5, 7, 2048) DONE
-                 : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(c[0]), "=&v"(c[1]) : "v"(a), "v"(b));
-  }
-#undef RD
-#undef DONE
-}
-
-template <int BN, int BM, int BUFS, int WAVES_ = 4>
-struct TileShape {
-  static constexpr int ROWS = BN + BM, BUF = ROWS * 64;  // elements of a buffer
-  static constexpr int WAVES = WAVES_;
-  static constexpr int WL = BN / 8 / WAVES, XL = BM >= 32 ? BM / 32 : 1;  // loads of a wave and stage; of x by four
-  static constexpr int LDS = BUFS * BUF * 2;
-  // waves along x: the weight rows are split over all of them for few rows of x, or more than four
-  static constexpr int WX = BM >= 64 && WAVES == 4 ? 2 : 1, R = BN * WX / WAVES / 16, C = BM / WX / 16;
-};
 
 // A wave's sums of weight rows wr .. of a tile and rows m0 .. of x
 template <int END, int BN, int R, int C>
@@ -154,10 +118,9 @@ DEVINL void finish_tile(const TileArgs& a, const floatx4 (&acc)[R][C], int tile,
 template <int BN, int BM, int BUFS, int END, int WAVES>
 __global__ __launch_bounds__((TileShape<BN, BM, BUFS, WAVES>::WAVES * 64)) void tile_kernel(TileArgs a) {
   typedef TileShape<BN, BM, BUFS, WAVES> Sh;
-  constexpr int R = Sh::R, C = Sh::C, LOADS = Sh::WL + Sh::XL;
+  constexpr int R = Sh::R, C = Sh::C;
   extern __shared__ __attribute__((aligned(16))) bf16_t buf[];  // [BUFS][weights [BN][64], x [BM][64]]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int col = lane & 15, quad = lane >> 4;
   read_args(a);
   // blocks go round the eight dies: two blocks of the same weights are neighbours on one.
   // The grid says which part a block has, as divisions come before all loads: a product of 7
@@ -195,51 +158,13 @@ __global__ __launch_bounds__((TileShape<BN, BM, BUFS, WAVES>::WAVES * 64)) void 
     xsrc[i] = a.x + (size_t)min(m0 + r, a.m - 1) * a.K + ((lane & 7) ^ (r & 7)) * 8;
   }
   const int len = s1 - s0, turn = first_step<END>(a, tile * (END == GATED ? BN / 2 : BN), len);
-  auto stage = [&](int s) {
-    bf16_t* dst = buf + ((s - s0) % BUFS) * Sh::BUF;
-    const int k = (s + turn < s1 ? s + turn : s + turn - len) * 64;
-#pragma unroll
-    for (int i = 0; i < Sh::WL; ++i)
-      __builtin_amdgcn_global_load_lds((glb_void*)(wsrc[i] + k), (lds_void*)(dst + (wave * Sh::WL + i) * 512), 16, 0, 2);
-#pragma unroll
-    for (int i = 0; i < Sh::XL; ++i) {
-      bf16_t* to = dst + BN * 64 + (wave & 3) * (BM >= 32 ? Sh::XL * 512 : 256) + i * 512;
-      if (BM >= 32 || lane < 32)
-        __builtin_amdgcn_global_load_lds((glb_void*)(xsrc[i] + k), (lds_void*)to, 16, 0, 0);
-    }
-  };
   floatx4 acc[R][C];
+  const int wr = Sh::wr(wave), wx = Sh::wx(wave);
 #pragma unroll
-  for (int i = 0; i < R; ++i)
+  for (int i = 0; i < Sh::WL; ++i) wsrc[i] += s0 * 64;
 #pragma unroll
-    for (int j = 0; j < C; ++j) acc[i][j] = (floatx4)(0.f);
-#pragma unroll
-  for (int i = 0; i < BUFS - 1; ++i)
-    if (s0 + i < s1) stage(s0 + i);
-  const int wr = wave / Sh::WX * (R * 16), wx = wave % Sh::WX * (C * 16);
-  // this lane's first fragments, as LDS byte addresses within a buffer
-  const unsigned base = (unsigned)(size_t)(lds_void*)buf;
-  const unsigned wl = base + (wr + col) * 128, xl = base + (BN + wx + col) * 128;
-  const unsigned place[2] = {(unsigned)((quad ^ (col & 7)) * 16), (unsigned)(((4 + quad) ^ (col & 7)) * 16)};
-  for (int s = s0; s < s1; ++s) {
-    // this step is in LDS, up to BUFS - 2 later ones are on their way; the buffer of
-    // the step before is free
-    const int left = min(BUFS - 2, s1 - 1 - s);
-    if (left >= 2) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(2 * LOADS) : "memory");
-    else if (left == 1) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(LOADS) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    if (s + BUFS - 1 < s1) stage(s + BUFS - 1);
-    const unsigned at = (unsigned)((s - s0) % BUFS) * (Sh::BUF * 2);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      bf16x8 wf[R], xf[C];
-      read_frags<R, C>(wl + at + place[h], xl + at + place[h], wf, xf);
-#pragma unroll
-      for (int i = 0; i < R; ++i)
-#pragma unroll
-        for (int j = 0; j < C; ++j) acc[i][j] = mma(wf[i], xf[j], acc[i][j]);
-    }
-  }
+  for (int i = 0; i < Sh::XL; ++i) xsrc[i] += s0 * 64;
+  stream_walk<Sh>(acc, buf, wsrc, xsrc, len, turn, wave, lane);
   finish_tile<END, BN, R, C>(a, acc, tile, split, m0 + wx, wr, lane);
 }
 
