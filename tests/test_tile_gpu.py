@@ -51,6 +51,15 @@ def test_products_in_a_round_of_parts(m, N, K):
   test_products(m, N, K)
 
 
+# one part more than 448 blocks take, where two a CU are all there; not where seven parts turn; nor of half as many tiles
+@pytest.mark.parametrize("N,K,splits", [(3584, 5696, 9), (4090, 6208, 8), (4096, 14336, 7), (2048, 11008, 14)])
+def test_two_blocks_a_cu(N, K, splits):
+  from xotorch_amd.ops import tile_splits
+  assert tile_splits(N, K) == splits
+  for m in (3, 40, 130):
+    test_products(m, N, K)
+
+
 @pytest.mark.parametrize("N,K", [(72, 320), (3584, 3584), (28680, 192), (520, 18944), (1048, 4096), (264, 16384),
                                  (40968, 4096), (40960, 4096), (36872, 4096)])  # the last five begin at different places of k
 def test_rows_do_not_depend_on_their_batch(N, K):
