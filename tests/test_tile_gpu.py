@@ -54,8 +54,8 @@ def test_products_in_a_round_of_parts(m, N, K):
 # one part more than 448 blocks take, where two a CU are all there; not where seven parts turn; nor of half as many tiles
 @pytest.mark.parametrize("N,K,splits", [(3584, 5696, 9), (4090, 6208, 8), (4096, 14336, 7), (2048, 11008, 14)])
 def test_two_blocks_a_cu(N, K, splits):
-  from xotorch_amd.ops import tile_splits
-  assert tile_splits(N, K) == splits
+  from xotorch_amd.ops import _hip_tile
+  assert _hip_tile.parts_of(N, K) == splits
   for m in (3, 40, 130):
     test_products(m, N, K)
 

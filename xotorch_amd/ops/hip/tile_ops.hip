@@ -492,14 +492,10 @@ static TileArgs tile_args(const Tensor& x, const Tensor& w) {
 }
 
 // Parts of k, as the rules of which products these are count them (ops.tile_splits): as few as
-// give some 450 blocks of 64 weight rows, of 4 steps at least; one more where two blocks a CU then are
-// all there, unless blocks of the former begin at different places of k (turns). us with the norm that
-// reads them, 8 and 9 parts: [3584, 18944] m 8 28.1, 27.1, m 16 29.2, 26.4, m 128 37.8, 36.0, m 256 51.6, 49.0;
-// 7 and 8: [4096, 11008] m 8 22.2, 21.3, m 256 40.9, 37.2; [4096, 14336], whose 7 turn, m 8 23.8, 23.9, m 32
-// 24.4, 25.3, m 128 35.8, 34.1. Of 32 tiles and fewer 14 and 16 are the same ([2048, 11008] m 8 13.4, 13.7).
+// give some 450 blocks of 64 weight rows, of 4 steps at least
 static int splits_of(int rows, int steps) {
-  const int tiles = (rows + 63) / 64, some = (448 + tiles - 1) / tiles, all = 512 / tiles;
-  return std::max(1, std::min({all > some && tiles > 32 && !turns(steps * 64, some) ? all : some, steps / 4, 16}));
+  const int tiles = (rows + 63) / 64;
+  return std::max(1, std::min({(448 + tiles - 1) / tiles, steps / 4, 16}));
 }
 
 // What k is split in: of up to 20 10^6 weights in as many as make one round of the chip, where
@@ -508,9 +504,16 @@ static int splits_of(int rows, int steps) {
 // 2048] 11.3, 9.3; m 128 [4096, 4096] 20.6, 17.7; m 256 [2048, 2048] 18.7, 17.7. Larger weights
 // gain nothing from 65 rows on: m 8 and 192 [8192, 8192] 28.8, 28.7 and 42.6, 51.3, [4096, 14336]
 // 25.6, 25.4 and 40.5, 53.7; nor do they in two thirds of a round: m 8 [6144, 4096] 14.7, 16.5.
+//
+// Of larger ones in one more where two blocks a CU then are all there, unless blocks of the former begin
+// at different places of k (turns): 8 and 9, [3584, 18944] m 8 28.1, 27.1, m 16 29.2, 26.4, m 128
+// 37.8, 36.0, m 256 51.6, 49.0; 7 and 8, [4096, 11008] m 8 22.2, 21.3, m 256 40.9, 37.2; [4096, 14336], whose 7
+// turn, m 8 23.8, 23.9, m 32 24.4, 25.3, m 128 35.8, 34.1. Of 32 tiles and fewer 14 and 16 are the same
+// ([2048, 11008] m 8 13.4, 13.7).
 static int parts_of(int rows, int steps) {
-  const int tiles = (rows + 63) / 64, n = splits_of(rows, steps), one = 256 / tiles;
-  return one >= 2 && one < n && one * tiles >= 200 && (int64_t)rows * steps <= 312500 ? one : n;
+  const int tiles = (rows + 63) / 64, n = splits_of(rows, steps), one = 256 / tiles, two = 512 / tiles;
+  if (one >= 2 && one < n && one * tiles >= 200 && (int64_t)rows * steps <= 312500) return one;
+  return two > n && two <= 16 && tiles > 32 && steps >= 4 * two && !turns(steps * 64, n) ? two : n;
 }
 
 static Tensor sized(const Tensor& x, int64_t n) {
