@@ -389,8 +389,11 @@ def gate_splits(N: int, K: int) -> int:
   whole = K <= 1024 or (tiles >= 160 and K <= (2048 if 256 < tiles < 320 else 6144))
   if whole:
     return 1
-  n, one = tile_splits(N, K), 256 // tiles
-  return one if 2 <= one < n and one * tiles >= 200 and N * (K // 64) <= 312500 else n
+  n, one, two = tile_splits(N, K), 256 // tiles, 512 // tiles
+  if 2 <= one < n and one * tiles >= 200 and N * (K // 64) <= 312500:
+    return one
+  turned = K <= 16384 and (K % (4096 if n > 1 else 2048) == 0 or (n > 1 and K % n == 0 and K // n % 2048 == 0))
+  return two if n < two <= 16 and tiles > 32 and K >= 256 * two and not turned else n
 
 
 @functools.lru_cache(maxsize=1024)
