@@ -43,6 +43,19 @@ def test_products_of_half_pieces(M, N, K):
   assert _near(train_ops._hip_gemm().forward(x, w), x, w)
 
 
+@pytest.mark.parametrize("M,N,K", [(191, 16388, 64), (192, 16384, 64), (577, 8196, 128), (190, 2048, 16384),  # 128 x 192, then in parts
+                                   (385, 33000, 128), (450, 16388, 128), (129, 8200, 8192),  # 256 x 192
+                                   (221, 33000, 1024), (448, 24584, 1024), (666, 2048, 65536)])  # 256 x 224
+def test_tiles_between(M, N, K):
+  """Of 192 and 224 rows of x: one row short, full, a tile for a few, sums in parts."""
+  from xotorch_amd.ops import train_ops
+  hip = train_ops._hip_gemm()
+  x, w = _random(M, M, K), _random(N, N, K)
+  assert _near(hip.forward(x, w), x, w)
+  if N % 8 == 0:
+    assert _near(hip.input_gradient(x, w.t().contiguous()), x, w)
+
+
 @pytest.mark.parametrize("left", [64, 65, 127, 128, 129, 1003])
 def test_what_is_left_of_a_sum_counts_once(left):
   """Tokens past whole steps; infinities in rows that the last step has twice stay what they are."""
@@ -168,6 +181,38 @@ def test_linears_of_prompts(M, N, K, form):
     with torch.autocast("cuda", torch.float16):
       assert not train_ops.takes_product(x, w)
   assert y.shape == (*x.shape[:-1], N) and _near(y.reshape(-1, N), x.reshape(-1, K), w)
+
+
+@pytest.mark.parametrize("M,N,K,form", [(65, 4100, 8064, "rows"), (2000, 4160, 8064, "turned"), (8192, 896, 16448, "rows"), (1001, 896, 896, "batch"),
+                                        (8192, 1920, 960, "spread"), (129, 4160, 2560, "shifted"), (2000, 9028, 896, "weight shifted"),
+                                        (300, 9024, 1024, "weight turned"), (70, 8192, 3264, "rows"), (1500, 960, 904, "batch"), (1100, 896, 57344, "rows")])
+def test_linears_that_later_tiles_gained(M, N, K, form):
+  """At the ends of train_ops.forward_gains and input_gains, whatever the strides and alignments."""
+  from xotorch_amd import ops
+  from xotorch_amd.ops import train_ops
+  assert train_ops.forward_gains(M, N, K) > train_ops.forward_wins(M, N, K) or train_ops.input_gains(M, N, K) > train_ops.input_wins(M, N, K)
+  x, w, dy = _random(1, M, K), _random(2, N, K), _random(3, M, N)
+  if form == "batch":
+    x, dy = x[None], dy[None]
+  if form == "turned":
+    x = x.t().contiguous().t()
+  if form == "shifted":
+    x = torch.cat([x.new_zeros(1), x.flatten()])[1:].view(M, K)
+  if form == "weight shifted":
+    w = torch.cat([w.new_zeros(1), w.flatten()])[1:].view(N, K)
+  if form == "weight turned":
+    w = w.t().contiguous().t()
+  if form == "spread":
+    dy = dy[:, :1].expand(M, N)
+  x = x.detach().requires_grad_()
+  y = ops.linear(x, w)
+  dx, = torch.autograd.grad(y, x, dy)
+  assert y.shape == dy.shape and dx.shape == x.shape
+  rows, drows = x.detach().reshape(-1, K), dy.reshape(-1, N)
+  assert _near(y.detach().reshape(-1, N), rows, w) and _near(dx.reshape(-1, K), drows, w.t())
+  if M > 256:
+    with torch.inference_mode():
+      assert _near(ops.linear(x, w).reshape(-1, N), rows, w)
 
 
 @pytest.mark.parametrize("M,N,K,form", [(257, 32, 64, "rows"), (320, 288, 128, "batch"), (513, 4096, 192, "shifted"), (1000, 2080, 448, "turned"),

@@ -68,10 +68,11 @@ struct Source {
 template <bool COL, int N, int F> struct Operand { typedef RowFrags<N> Frags; };
 template <int N, int F> struct Operand<true, N, F> { typedef ColFrags<N, F> Frags; };
 
-// A block has BN of N and BM of M; WN waves along N
-constexpr int WAVES = 8;  // blocks are few and short: see mfma_tile.h
+// A block has BN of N and BM of M; WN waves along N. Eight waves, as blocks are few and short (mfma_tile.h), but
+// four where the rows of x do not go by eight into pieces of 16
+constexpr int waves_of(int bm) { return bm % 64 ? 4 : 8; }
 
-template <bool WCOL, bool XCOL, int BN, int BM, int WN, int WB, int XB, bool PARTS>
+template <bool WCOL, bool XCOL, int BN, int BM, int WN, int WB, int XB, bool PARTS, int WAVES = waves_of(BM)>
 __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(GemmArgs a) {
   typedef MfmaTile<BN, BM, WN, WB, XB, WAVES> Sh;
   constexpr int R = Sh::R, C = Sh::C, WL = Sh::WL, XL = Sh::XL;
@@ -140,7 +141,7 @@ __global__ __launch_bounds__(256) void parts_kernel(const float* __restrict__ pa
 template <bool WCOL, bool XCOL, int BN, int BM, int WN, int WB, int XB>
 static void launch_gemm(const GemmArgs& a) {
   const int units = (a.N + BN - 1) / BN * ((a.M + BM - 1) / BM) * a.splits;
-  const int lds = MfmaTile<BN, BM, WN, WB, XB, WAVES>::LDS;
+  constexpr int WAVES = waves_of(BM), lds = MfmaTile<BN, BM, WN, WB, XB, WAVES>::LDS;
   auto run = [&](auto kernel) {
     const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     TORCH_CHECK(e == hipSuccess, "no LDS for a product's tiles");
@@ -151,18 +152,37 @@ static void launch_gemm(const GemmArgs& a) {
 }
 
 // Tile and parts by what a round of the chip's 256 CUs takes, us: so much for a step of 64
-// and for a block's begin and end, and the parts' sums once out and in again. Of the four
-// tiles and up to 16 parts it found one within 8% of the fastest for the products above.
-static const struct { int bn, bm; double step, ends; } TILES[4] = {{256, 256, 1.42, 11}, {128, 256, 0.8, 7.5}, {256, 128, 0.8, 7.5}, {128, 128, 0.45, 4.7}};
-struct Choice { int tile, splits; };
-static Choice choose(int64_t M, int64_t N, int steps) {
+// and for a block's begin and end, and the parts' sums once out and in again.
+struct Tile {
+  int bn, bm;
+  double step, ends;
+};
+struct Costs {
+  const Tile* tiles;
+  int count;
+  double bytes_us, parts;
+};
+// Of x as rows, fitted to 168 products of 64 to 4096 rows: a tile and parts within 2.2% of the fastest
+// of these on average, 21% at most. With 256 and 128 rows of x alone it were 5%, and 13% of a tile's work
+// is for rows that are not there at 666 tokens, whose products take, us, before and now: [2048 -> 128256] 370
+// and 325, its gradient 360 and 315, [8192 -> 2048] 38.2 and 33.0, [2048 -> 2048] 18.6 and 16.6. Tiles of
+// 160 rows of x, and of 224 by 128, gave 0.4% more.
+static const Tile ROW_TILES[] = {{256, 256, 1.21, 4.4}, {128, 256, 0.7, 2.7}, {256, 128, 0.76, 2.8}, {128, 128, 0.49, 1.5},
+                                 {256, 224, 1.0, 5.9}, {256, 192, 0.98, 3.1}, {128, 192, 0.62, 2.6}};
+// As columns, of the first four tiles: within 8% of the fastest.
+static const Tile COLUMN_TILES[] = {{256, 256, 1.42, 11}, {128, 256, 0.8, 7.5}, {256, 128, 0.8, 7.5}, {128, 128, 0.45, 4.7}};
+struct Choice {
+  int tile, splits;
+};
+static Choice choose(const Costs& of, int64_t M, int64_t N, int steps) {
   Choice best{0, 1};
   double least = 1e30;
-  for (int t = 0; t < 4; ++t) {
-    const int64_t blocks = (N + TILES[t].bn - 1) / TILES[t].bn * ((M + TILES[t].bm - 1) / TILES[t].bm);
+  for (int t = 0; t < of.count; ++t) {
+    const Tile& tile = of.tiles[t];
+    const int64_t blocks = (N + tile.bn - 1) / tile.bn * ((M + tile.bm - 1) / tile.bm);
     for (int s = 1; s <= 16 && (s == 1 || (steps / s >= 4 && M * N * s <= 1 << 27)); ++s) {
       const int64_t rounds = (blocks * s + 255) / 256;
-      const double us = rounds * ((steps + s - 1) / s * TILES[t].step + TILES[t].ends) + (s > 1 ? M * N * 8.0 * s / 5e6 + 2.5 : 0);
+      const double us = rounds * ((steps + s - 1) / s * tile.step + tile.ends) + (s > 1 ? M * N * 8.0 * s / of.bytes_us + of.parts : 0);
       if (us < least) least = us, best = {t, s};
     }
   }
@@ -190,9 +210,10 @@ static Tensor product(const Tensor& x, const Tensor& w) {
   a.steps = (int)((K + 63) / 64);
   // us of [4096, 28672 x 4096], panels of 2, 4 and 8 tiles of x: 694, 675, 676; 8192 of all, 766, 733, 723
   a.group = 4;
-  const Choice c = choose(m, N, a.steps);
+  const Costs of = XCOL ? Costs{COLUMN_TILES, 4, 5e6, 2.5} : Costs{ROW_TILES, 7, 6.5e6, 5.2};
+  const Choice c = choose(of, m, N, a.steps);
   a.splits = c.splits;
-  CHK((N / TILES[c.tile].bn + 1) * (m / TILES[c.tile].bm + 1) * a.splits <= INT_MAX / 8);
+  CHK((N / of.tiles[c.tile].bn + 1) * (m / of.tiles[c.tile].bm + 1) * a.splits <= INT_MAX / 8);
   auto y = torch::empty({m, N}, x.options());
   Tensor part;
   a.y = y.data_ptr();
@@ -203,7 +224,12 @@ static Tensor product(const Tensor& x, const Tensor& w) {
   if (c.tile == 0) launch_gemm<WCOL, XCOL, 256, 256, 2, 3, 2>(a);
   else if (c.tile == 1) launch_gemm<WCOL, XCOL, 128, 256, 2, 3, 3>(a);
   else if (c.tile == 2) launch_gemm<WCOL, XCOL, 256, 128, 4, 3, 3>(a);
-  else launch_gemm<WCOL, XCOL, 128, 128, 2, 4, 4>(a);
+  else if (c.tile == 3) launch_gemm<WCOL, XCOL, 128, 128, 2, 4, 4>(a);
+  else if constexpr (!XCOL) {
+    if (c.tile == 4) launch_gemm<WCOL, XCOL, 256, 224, 2, 3, 2>(a);
+    else if (c.tile == 5) launch_gemm<WCOL, XCOL, 256, 192, 2, 3, 2>(a);
+    else launch_gemm<WCOL, XCOL, 128, 192, 2, 4, 4>(a);
+  }
   if (a.splits > 1) {
     const size_t n = (size_t)m * N;
     hipLaunchKernelGGL(parts_kernel, dim3(std::min<size_t>((n + 1023) / 1024, 4096)), dim3(256), 0, cur_stream(), part.data_ptr<float>(),
