@@ -240,6 +240,19 @@ def test_gradients_of_inputs_go_where_they_are_faster():
   assert input_wins(2800, 16384, 2048) and not input_wins(2801, 16384, 2048) and input_wins(3000, 37888, 3584) and not input_wins(3001, 37888, 3584)
 
 
+def test_products_that_later_tiles_gained():
+  """Long sums, small weights of many tokens and ordinary weights of up to 2000; gradients of inputs of up to 8192."""
+  from xotorch_amd.ops.train_ops import forward_gains, input_gains
+  for M, N, K, own in [(64, 8192, 8064, False), (65, 8192, 8064, True), (2001, 8192, 8064, False), (8192, 5120, 17408, True), (8193, 5120, 17408, False),
+                       (8192, 8192, 28672, False), (1000, 2048, 3072, False), (1001, 2048, 3072, True), (8192, 2048, 3072, True), (128, 28672, 4096, False),
+                       (129, 28672, 4096, True), (2000, 28672, 4096, True), (2001, 28672, 4096, False), (100, 6144, 4096, True), (100, 16384, 2048, False),
+                       (1500, 892, 2048, False), (1500, 2048, 832, False), (1500, 2050, 2048, False), (1500, 2048, 2056, False), (1500, 128256, 2048, False)]:
+    assert forward_gains(M, N, K) == own, (M, N, K)
+  for M, N, K, own in [(8192, 28672, 4096, True), (8193, 28672, 4096, False), (1, 896, 57344, True), (1, 896, 57352, False), (1, 832, 4096, False),
+                       (1, 960, 900, False), (1, 928, 904, False), (4096, 128256, 4096, False)]:
+    assert input_gains(M, N, K) == own, (M, N, K)
+
+
 @pytest.mark.parametrize("needs", [(True, False), (False, True), (True, True)])
 def test_a_linear_holds_what_its_gradients_read(needs):
   """Rows for the weight's gradient, the weight for that of the rows, as torch's operator; what is

@@ -131,6 +131,7 @@ def _again(f: Callable, inputs: Sequence[torch.Tensor], needs: Sequence[bool], g
 # themselves. 300 tokens through 28 layers of 1536 took 3070 us, and 3500 with those by the
 # library; 512 tokens 3520, and 3420 to 3660. What the kernels don't index is the library's.
 _MOST = 1 << 22  # rows, features
+_WIDEST = 57344  # of what was measured with tiles of 192 and 224 rows of x
 
 
 def forward_wins(M: int, N: int, K: int) -> bool:
@@ -167,6 +168,25 @@ def input_wins(M: int, N: int, K: int) -> bool:
   return M <= 1400 and N >= K or M <= 2800 and N >= 8 * K or M <= 3000 and N >= 10 * K
 
 
+def forward_gains(M: int, N: int, K: int) -> bool:
+  """What is faster of forward_wins' rest since there are tiles of 192 and 224 rows of x: long
+  sums 0.26 to 1.12 (0.82), narrow ones of the longest, of more tokens 0.58 to 1.07 (0.74); small
+  weights 0.68 to 1.09 (0.93); others up to 1000 tokens 0.62 to 1.14 (0.93), up to 2000 0.70 to
+  1.16 (0.94). What it leaves: more tokens 0.69 to 1.19 (0.99), up to 128 0.81 to 1.28 (0.98).
+  Features and rows that were not measured too."""
+  if K % 64 or N % 4 or not 896 <= N < 100_000 or not 896 <= K <= _WIDEST or not 64 < M <= 8192:
+    return False
+  if K > 8000:
+    return M <= 2000 or K > 16384 and N <= 6144
+  return 1000 < M if N * K <= 7_000_000 else M <= 2000 and (M > 128 or K > 3200 and N <= 20000)
+
+
+def input_gains(M: int, N: int, K: int) -> bool:
+  """The same of input_wins' rest: up to 2000 tokens 0.48 to 1.12 (0.87), up to 4096 0.51 to 1.10
+  (0.89), up to 8192 0.59 to 1.04 (0.90)."""
+  return N % 64 == 0 and K % 8 == 0 and 896 <= N < 100_000 and 896 <= K <= _WIDEST and M <= 8192
+
+
 def weight_wins(M: int, N: int, K: int) -> bool:
   """dy^T x, a sum over tokens: 0.61 to 1.25 (0.88 on average) from 600 tokens on; small weights
   of fewer 0.54 to 1.20 (0.89), large ones and 100 to 512 tokens 0.85 to 1.16."""
@@ -176,7 +196,7 @@ def weight_wins(M: int, N: int, K: int) -> bool:
 def product(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
   """x W^T of rows [M, K]"""
   M, (N, K) = x.shape[0], weight.shape
-  if forward_wins(M, N, K) and weight.is_contiguous() and weight.data_ptr() % 16 == 0:
+  if (forward_wins(M, N, K) or forward_gains(M, N, K)) and weight.is_contiguous() and weight.data_ptr() % 16 == 0:
     return _hip_gemm().forward(_rows(x), weight)
   return torch.nn.functional.linear(x, weight)
 
@@ -189,7 +209,7 @@ def takes_product(x: torch.Tensor, weight: torch.Tensor) -> bool:
   if not x.is_cuda or x.dtype is not torch.bfloat16 or weight.dtype is not torch.bfloat16 or torch.is_grad_enabled() or weight.dim() != 2:
     return False
   (N, K), M = weight.shape, x.numel() // max(1, weight.shape[1])
-  return (256 < M and x.shape[-1] == K and forward_wins(M, N, K) and plain(x, weight)
+  return (256 < M and x.shape[-1] == K and (forward_wins(M, N, K) or forward_gains(M, N, K)) and plain(x, weight)
           and not torch._C._is_any_autocast_enabled() and not _missing())
 
 
@@ -217,7 +237,7 @@ def gate_product(x: torch.Tensor, gate_up: torch.Tensor) -> torch.Tensor:
 def input_gradient(dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
   """dy W of rows [M, N]"""
   M, (N, K) = dy.shape[0], weight.shape
-  if input_wins(M, N, K) and once(dy, weight) and weight.is_contiguous() and weight.data_ptr() % 16 == 0:
+  if (input_wins(M, N, K) or input_gains(M, N, K)) and once(dy, weight) and weight.is_contiguous() and weight.data_ptr() % 16 == 0:
     return _hip_gemm().input_gradient(_rows(dy), weight)
   return dy @ weight
 
@@ -234,7 +254,7 @@ def takes_linear(x: torch.Tensor, weight: torch.Tensor) -> bool:
   if not (x.is_cuda and torch.is_grad_enabled() and weight.dim() == 2 and 0 < x.numel() and x.shape[-1] == weight.shape[1]):
     return False
   (N, K), M = weight.shape, x.numel() // weight.shape[1]
-  return ((forward_wins(M, N, K) or input_wins(M, N, K) or weight_wins(M, N, K)) and K % 8 == 0
+  return ((forward_wins(M, N, K) or forward_gains(M, N, K) or input_wins(M, N, K) or input_gains(M, N, K) or weight_wins(M, N, K)) and K % 8 == 0
           and x.dtype == weight.dtype == torch.bfloat16 and (x.requires_grad or weight.requires_grad) and plain(x, weight)
           and not torch._C._is_any_autocast_enabled() and not _missing())
 
