@@ -43,11 +43,14 @@ def test_products_of_half_pieces(M, N, K):
   assert _near(train_ops._hip_gemm().forward(x, w), x, w)
 
 
-@pytest.mark.parametrize("M,N,K", [(191, 16388, 64), (192, 16384, 64), (577, 8196, 128), (190, 2048, 16384),  # 128 x 192, then in parts
+@pytest.mark.parametrize("M,N,K", [(191, 16392, 2048), (385, 8200, 4096), (192, 4104, 8192),  # 128 x 192, then in parts
                                    (385, 33000, 128), (450, 16388, 128), (129, 8200, 8192),  # 256 x 192
-                                   (221, 33000, 1024), (448, 24584, 1024), (666, 2048, 65536)])  # 256 x 224
+                                   (221, 33000, 1024), (448, 24584, 1024), (666, 2048, 65536),  # 256 x 224
+                                   (95, 16392, 320), (577, 4100, 64), (129, 2048, 8192),  # 128 x 96
+                                   (65, 1032, 64), (385, 4104, 128), (192, 4104, 4096),  # 128 x 64
+                                   (570, 2052, 320), (127, 8200, 4096), (1, 68, 8192), (193, 1032, 4096)])  # 64 x 128 (and gradients by 128 x 64)
 def test_tiles_between(M, N, K):
-  """Of 192 and 224 rows of x: one row short, full, a tile for a few, sums in parts."""
+  """Tiles of other shapes than 128 and 256: one row short, full, a tile for a few, sums in parts."""
   from xotorch_amd.ops import train_ops
   hip = train_ops._hip_gemm()
   x, w = _random(M, M, K), _random(N, N, K)

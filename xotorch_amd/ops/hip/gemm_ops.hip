@@ -69,10 +69,10 @@ template <bool COL, int N, int F> struct Operand { typedef RowFrags<N> Frags; };
 template <int N, int F> struct Operand<true, N, F> { typedef ColFrags<N, F> Frags; };
 
 // A block has BN of N and BM of M; WN waves along N. Eight waves, as blocks are few and short (mfma_tile.h), but
-// four where the rows of x do not go by eight into pieces of 16
-constexpr int waves_of(int bm) { return bm % 64 ? 4 : 8; }
+// four where the rows of x do not go by eight into pieces of 16 or the tile has too few of them
+constexpr int waves_of(int bn, int bm) { return bm % 64 || bn * bm < 128 * 128 ? 4 : 8; }
 
-template <bool WCOL, bool XCOL, int BN, int BM, int WN, int WB, int XB, bool PARTS, int WAVES = waves_of(BM)>
+template <bool WCOL, bool XCOL, int BN, int BM, int WN, int WB, int XB, bool PARTS, int WAVES = waves_of(BN, BM)>
 __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(GemmArgs a) {
   typedef MfmaTile<BN, BM, WN, WB, XB, WAVES> Sh;
   constexpr int R = Sh::R, C = Sh::C, WL = Sh::WL, XL = Sh::XL;
@@ -141,7 +141,7 @@ __global__ __launch_bounds__(256) void parts_kernel(const float* __restrict__ pa
 template <bool WCOL, bool XCOL, int BN, int BM, int WN, int WB, int XB>
 static void launch_gemm(const GemmArgs& a) {
   const int units = (a.N + BN - 1) / BN * ((a.M + BM - 1) / BM) * a.splits;
-  constexpr int WAVES = waves_of(BM), lds = MfmaTile<BN, BM, WN, WB, XB, WAVES>::LDS;
+  constexpr int WAVES = waves_of(BN, BM), lds = MfmaTile<BN, BM, WN, WB, XB, WAVES>::LDS;
   auto run = [&](auto kernel) {
     const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     TORCH_CHECK(e == hipSuccess, "no LDS for a product's tiles");
@@ -162,13 +162,15 @@ struct Costs {
   int count;
   double bytes_us, parts;
 };
-// Of x as rows, fitted to 168 products of 64 to 4096 rows: a tile and parts within 2.2% of the fastest
-// of these on average, 21% at most. With 256 and 128 rows of x alone it were 5%, and 13% of a tile's work
+// Of x as rows, fitted to 243 products of 64 to 4096 rows: a tile and parts within 1.3% of the fastest
+// of these on average, 16% at most. With 256 and 128 rows of x alone it were 5%, and 13% of a tile's work
 // is for rows that are not there at 666 tokens, whose products take, us, before and now: [2048 -> 128256] 370
-// and 325, its gradient 360 and 315, [8192 -> 2048] 38.2 and 33.0, [2048 -> 2048] 18.6 and 16.6. Tiles of
-// 160 rows of x, and of 224 by 128, gave 0.4% more.
-static const Tile ROW_TILES[] = {{256, 256, 1.21, 4.4}, {128, 256, 0.7, 2.7}, {256, 128, 0.76, 2.8}, {128, 128, 0.49, 1.5},
-                                 {256, 224, 1.0, 5.9}, {256, 192, 0.98, 3.1}, {128, 192, 0.62, 2.6}};
+// and 325, its gradient 360 and 315, [8192 -> 2048] 38.2 and 33.0. Small tiles are for weights that have
+// few: blocks for all CUs without parts of the sum. [2048 -> 2048] 150, 333 and 1000 tokens 14.8 and 10.7, 15.3 and
+// 11.2, 17.7 and 12.8, its gradient 15.0 and 11.4, 16.4 and 13.8, 19.0 and 15.0. Tiles of 160 rows of x, of 224 by
+// 128 and of 64 by 64 gave less than 1% more. The last is for weights as rows alone: columns have no such form.
+static const Tile ROW_TILES[] = {{256, 256, 1.14, 4.4}, {128, 256, 0.66, 2}, {256, 128, 0.76, 2}, {128, 128, 0.47, 1.3}, {256, 224, 0.95, 5.9},
+                                 {256, 192, 0.93, 3.1}, {128, 192, 0.59, 2.9}, {128, 96, 0.44, 1.3}, {128, 64, 0.32, 1.2}, {64, 128, 0.26, 1.3}};
 // As columns, of the first four tiles: within 8% of the fastest.
 static const Tile COLUMN_TILES[] = {{256, 256, 1.42, 11}, {128, 256, 0.8, 7.5}, {256, 128, 0.8, 7.5}, {128, 128, 0.45, 4.7}};
 struct Choice {
@@ -210,7 +212,7 @@ static Tensor product(const Tensor& x, const Tensor& w) {
   a.steps = (int)((K + 63) / 64);
   // us of [4096, 28672 x 4096], panels of 2, 4 and 8 tiles of x: 694, 675, 676; 8192 of all, 766, 733, 723
   a.group = 4;
-  const Costs of = XCOL ? Costs{COLUMN_TILES, 4, 5e6, 2.5} : Costs{ROW_TILES, 7, 6.5e6, 5.2};
+  const Costs of = XCOL ? Costs{COLUMN_TILES, 4, 5e6, 2.5} : Costs{ROW_TILES, WCOL ? 9 : 10, 7.2e6, 4};
   const Choice c = choose(of, m, N, a.steps);
   a.splits = c.splits;
   CHK((N / of.tiles[c.tile].bn + 1) * (m / of.tiles[c.tile].bm + 1) * a.splits <= INT_MAX / 8);
@@ -228,7 +230,10 @@ static Tensor product(const Tensor& x, const Tensor& w) {
   else if constexpr (!XCOL) {
     if (c.tile == 4) launch_gemm<WCOL, XCOL, 256, 224, 2, 3, 2>(a);
     else if (c.tile == 5) launch_gemm<WCOL, XCOL, 256, 192, 2, 3, 2>(a);
-    else launch_gemm<WCOL, XCOL, 128, 192, 2, 4, 4>(a);
+    else if (c.tile == 6) launch_gemm<WCOL, XCOL, 128, 192, 2, 4, 4>(a);
+    else if (c.tile == 7) launch_gemm<WCOL, XCOL, 128, 96, 2, 4, 4>(a);
+    else if (c.tile == 8) launch_gemm<WCOL, XCOL, 128, 64, 2, 4, 4>(a);
+    else if constexpr (!WCOL) launch_gemm<WCOL, XCOL, 64, 128, 1, 4, 4>(a);
   }
   if (a.splits > 1) {
     const size_t n = (size_t)m * N;

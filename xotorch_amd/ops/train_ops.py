@@ -127,17 +127,17 @@ def _again(f: Callable, inputs: Sequence[torch.Tensor], needs: Sequence[bool], g
 # its time on the GPU with weights from memory, as a pass finds them (1 to 4096 tokens, the
 # linears of decoders of 0.5B to 70B; M tokens through a weight [N, K]). Passes of few tokens or
 # short rows wait for the host, to which a call of the library is the longer one: there is no
-# lower end, and narrow products of short rows are the kernels' though they are slower by
+# lower end, and narrow products of short rows are the kernels' though some are slower by
 # themselves. 300 tokens through 28 layers of 1536 took 3070 us, and 3500 with those by the
 # library; 512 tokens 3520, and 3420 to 3660. What the kernels don't index is the library's.
 _MOST = 1 << 22  # rows, features
-_WIDEST = 57344  # of what was measured with tiles of 192 and 224 rows of x
+_WIDEST = 57344  # of what was measured with tiles of 64 to 224 rows of x
 
 
 def forward_wins(M: int, N: int, K: int) -> bool:
-  """x W^T: narrow results of up to 1000 tokens 0.28 to 1.31 (0.79 on average) for rows of 3072
-  and more; for shorter ones 0.80 to 1.30 (0.98) up to 32 tokens, 0.76 to 1.65 (1.19) from
-  there on. Wider results and more tokens 0.95 to 1.40, but for long sums, whose library tiles
+  """x W^T: narrow results of up to 1000 tokens 0.34 to 1.26 (0.77 on average) for rows of 3072
+  and more, 0.74 to 1.38 (0.94) for shorter ones (0.76 to 1.65, 1.19, from 65 tokens on before
+  there were tiles of 64). By tiles of 128 and 256 alone: wider results and more tokens 0.95 to 1.40, but for long sums, whose library tiles
   fill the chip badly (257 to 2000 tokens by 1536 to 12288 features of 13824 to 29568): where
   the result is small 0.46 to 1.05 (0.69), of up to 6144 features 0.65 to 0.95, narrow ones of
   longest sums 0.39 to 0.87. A vocabulary's width (128256 to 152064 features of 896 to 4096), 65
@@ -154,8 +154,8 @@ def forward_wins(M: int, N: int, K: int) -> bool:
 
 
 def input_wins(M: int, N: int, K: int) -> bool:
-  """dy W, a sum over N: 0.20 to 1.10 (0.6 on average), weights of less than 5 10^6 numbers
-  0.72 to 1.44 (1.05). What is left to the library: by sums of less than four times the
+  """dy W, a sum over N: 0.22 to 1.11 (0.64 on average), weights of less than 5 10^6 numbers
+  0.59 to 1.23 (0.87). By tiles of 128 and 256 alone there was left to the library: by sums of less than four times the
   result's width 1025 to 1400 tokens and weights of 8192 by 8192 and more 1.15 to 1.38, 1281 to
   1400 and smaller ones 0.93 to 1.11 (1.04); 257 to 300 by weights of more than 10^8
   1.21 to 1.43; 3000 by [16384, 2048] 1.15; shorter sums of more tokens 0.85 to 1.27."""
@@ -169,11 +169,11 @@ def input_wins(M: int, N: int, K: int) -> bool:
 
 
 def forward_gains(M: int, N: int, K: int) -> bool:
-  """What is faster of forward_wins' rest since there are tiles of 192 and 224 rows of x: long
-  sums 0.26 to 1.12 (0.82), narrow ones of the longest, of more tokens 0.58 to 1.07 (0.74); small
-  weights 0.68 to 1.09 (0.93); others up to 1000 tokens 0.62 to 1.14 (0.93), up to 2000 0.70 to
-  1.16 (0.94). What it leaves: more tokens 0.69 to 1.19 (0.99), up to 128 0.81 to 1.28 (0.98).
-  Features and rows that were not measured too."""
+  """What is faster of forward_wins' rest since there are tiles of 64 to 224 rows of x: long
+  sums 0.27 to 1.15 (0.81), narrow ones of the longest, of more tokens 0.58 to 1.06 (0.74); small
+  weights 0.68 to 1.07 (0.89); others up to 1000 tokens 0.59 to 1.13 (0.92), up to 2000 0.71 to
+  1.12 (0.95). What it leaves: more tokens 0.67 to 1.18 (0.99); 65 to 128 by short sums and by
+  wide weights 0.81 to 1.22 (0.98); features and rows that were not measured."""
   if K % 64 or N % 4 or not 896 <= N < 100_000 or not 896 <= K <= _WIDEST or not 64 < M <= 8192:
     return False
   if K > 8000:
@@ -182,8 +182,8 @@ def forward_gains(M: int, N: int, K: int) -> bool:
 
 
 def input_gains(M: int, N: int, K: int) -> bool:
-  """The same of input_wins' rest: up to 2000 tokens 0.48 to 1.12 (0.87), up to 4096 0.51 to 1.10
-  (0.89), up to 8192 0.59 to 1.04 (0.90)."""
+  """The same of input_wins' rest: up to 2000 tokens 0.47 to 1.11 (0.87), up to 4096 0.48 to 1.09
+  (0.88), up to 8192 0.58 to 1.05 (0.90)."""
   return N % 64 == 0 and K % 8 == 0 and 896 <= N < 100_000 and 896 <= K <= _WIDEST and M <= 8192
 
 
