@@ -59,6 +59,26 @@ def test_tiles_between(M, N, K):
     assert _near(hip.input_gradient(x, w.t().contiguous()), x, w)
 
 
+@pytest.mark.parametrize("M,N,K,rank", [(1, 72, 64, 1), (65, 1032, 64, 4), (570, 2056, 320, 5), (193, 1032, 4096, 8), (385, 4104, 128, 9),
+                                        (95, 16392, 320, 16), (129, 2048, 8192, 8), (385, 8200, 4096, 16), (450, 16392, 128, 3), (129, 8200, 8192, 8),
+                                        (221, 33000, 1024, 8), (666, 2048, 65536, 16), (1300, 4104, 320, 8), (383, 16392, 320, 2),
+                                        (2100, 4096, 4096, 8), (95, 8200, 8192, 8), (383, 8200, 64, 8)])
+def test_low_rank_terms(M, N, K, rank):
+  """Of adapters, added inside the products, of every tile, in parts or not; numbers past the rank and the ends count
+  for nothing. Not rounded before the sum: fp32 products of K + rank numbers."""
+  from xotorch_amd.ops import train_ops
+  hip = train_ops._hip_gemm()
+  x, w = _random(M, M, K), _random(N, N, K)
+  g = torch.Generator(device="cuda").manual_seed(rank)
+  by = torch.randn(rank, N, generator=g, device="cuda")
+  low = torch.zeros(M, 4 if rank <= 4 else 8 if rank <= 8 else 16, device="cuda")
+  low[:, :rank] = torch.randn(M, rank, generator=g, device="cuda") * K ** 0.5
+  want = x.double() @ w.double().t() + 0.75 * low[:, :rank].double() @ by.double()
+  size = x.double().abs() @ w.double().abs().t() + 0.75 * low[:, :rank].double().abs() @ by.double().abs()
+  for got in (hip.forward(x, w, low, by, 0.75), hip.input_gradient(x, w.t().contiguous(), low, by, 0.75)):
+    assert bool(((got.double() - want).abs() <= size * (K + rank + 9) * 2.0 ** -24 + want.abs() * 2.0 ** -8).all())
+
+
 @pytest.mark.parametrize("left", [64, 65, 127, 128, 129, 1003])
 def test_what_is_left_of_a_sum_counts_once(left):
   """Tokens past whole steps; infinities in rows that the last step has twice stay what they are."""

@@ -21,6 +21,9 @@ struct GemmArgs {
   void* y;              // bf16 [M, N], or fp32 [splits, M, N]
   int M, N, K;
   int steps, splits, group;  // steps of 64; tiles of x that are neighbours in a run of blocks
+  const float *low, *by;     // y += scale low [M, rp] by [rank, N], or none
+  int rank, rp;
+  float scale;
 };
 
 // Where a wave's loads of an operand come from: rows [free, k] or, COL, columns [k, free]
@@ -72,6 +75,31 @@ template <int N, int F> struct Operand<true, N, F> { typedef ColFrags<N, F> Frag
 // four where the rows of x do not go by eight into pieces of 16 or the tile has too few of them
 constexpr int waves_of(int bn, int bm) { return bm % 64 || bn * bm < 128 * 128 ? 4 : 8; }
 
+// The low-rank term of an adapted linear, by fp32 products of the matrix cores (16 x 16 x 4), where a block's
+// sums are whole: results go to memory once, and a pass that adds to them there reads and writes all of them
+// again. us of 4096 tokens, rank 8, library and pass, this kernel and pass, so: [4096 -> 28672] 732, 763, 694, its
+// input's gradient 711, 699, 686; [14336 -> 4096] 322, 336, 319, its input's gradient 435, 427, 394. Operands
+// of eight features at once were 0 to 3% slower.
+template <int R, int C>
+DEVINL void add_low(floatx4 (&acc)[R][C], const GemmArgs& a, int m0, int n0, int lane) {
+  const int col = lane & 15, quad = lane >> 4;
+  for (int r0 = 0; r0 < a.rp; r0 += 4) {
+    const int r = r0 + quad;
+    const float* by = a.by + (size_t)min(r, a.rank - 1) * a.N;
+    float w[R], x[C];
+#pragma unroll
+    for (int i = 0; i < R; ++i) w[i] = by[min(n0 + i * 16 + col, a.N - 1)];
+#pragma unroll
+    for (int j = 0; j < C; ++j) x[j] = a.low[(size_t)min(m0 + j * 16 + col, a.M - 1) * a.rp + r];
+#pragma unroll
+    for (int i = 0; i < R; ++i) w[i] = r < a.rank ? w[i] * a.scale : 0.f;
+#pragma unroll
+    for (int j = 0; j < C; ++j)
+#pragma unroll
+      for (int i = 0; i < R; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i], x[j], acc[i][j], 0, 0, 0);
+  }
+}
+
 template <bool WCOL, bool XCOL, int BN, int BM, int WN, int WB, int XB, bool PARTS, int WAVES = waves_of(BN, BM)>
 __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(GemmArgs a) {
   typedef MfmaTile<BN, BM, WN, WB, XB, WAVES> Sh;
@@ -107,6 +135,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(GemmArgs a) {
   const unsigned base = (unsigned)(size_t)(lds_void*)buf;
   walk<Sh>(acc, typename Operand<WCOL, R, BN>::Frags(base, wr, lane), typename Operand<XCOL, C, BM>::Frags(base + Sh::XAT, wx, lane),
            s1 - s0, stepw, loadw, stepx, loadx, skip);
+  if constexpr (!XCOL)
+    if (a.low && split == 0) add_low(acc, a, m0 + wx, n0 + wr, lane);
   typedef typename std::conditional<PARTS, float, bf16_t>::type Out;
   const RowsOut<Out, R * 16> rows(buf, wave, lane);
 #pragma unroll
@@ -191,9 +221,9 @@ static Choice choose(const Costs& of, int64_t M, int64_t N, int steps) {
   return best;
 }
 
-// y [M, N] of x [M, K] (XCOL: [K, M]) and w [N, K] (WCOL: [K, N])
+// y [M, N] of x [M, K] (XCOL: [K, M]) and w [N, K] (WCOL: [K, N]), and scale low by if they are given
 template <bool WCOL, bool XCOL>
-static Tensor product(const Tensor& x, const Tensor& w) {
+static Tensor product(const Tensor& x, const Tensor& w, const OptT& low = {}, const OptT& by = {}, double scale = 1) {
   check_io(x, torch::kBFloat16);
   check_io(w, torch::kBFloat16);
   CHK(x.dim() == 2 && w.dim() == 2);
@@ -210,6 +240,18 @@ static Tensor product(const Tensor& x, const Tensor& w) {
   a.N = (int)N;
   a.K = (int)K;
   a.steps = (int)((K + 63) / 64);
+  if (low) {
+    CHK(by.has_value() && !XCOL);
+    check_io(*low, torch::kFloat32);
+    check_io(*by, torch::kFloat32);
+    CHK(low->dim() == 2 && by->dim() == 2 && low->size(0) == m && by->size(1) == N && by->size(0) >= 1 && by->size(0) <= 16);
+    a.rank = (int)by->size(0);
+    a.rp = a.rank <= 4 ? 4 : a.rank <= 8 ? 8 : 16;
+    CHK(low->size(1) == a.rp);
+    a.low = P<float>(*low);
+    a.by = P<float>(*by);
+    a.scale = (float)scale;
+  }
   // us of [4096, 28672 x 4096], panels of 2, 4 and 8 tiles of x: 694, 675, 676; 8192 of all, 766, 733, 723
   a.group = 4;
   const Costs of = XCOL ? Costs{COLUMN_TILES, 4, 5e6, 2.5} : Costs{ROW_TILES, WCOL ? 9 : 10, 7.2e6, 4};
@@ -244,7 +286,11 @@ static Tensor product(const Tensor& x, const Tensor& w) {
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  m.def("forward", [](Tensor x, Tensor w) { return product<false, false>(x, w); }, "x w^T of x [M, K], w [N, K]");
-  m.def("input_gradient", [](Tensor dy, Tensor w) { return product<true, false>(dy, w); }, "dy w of dy [M, N], w [N, K]");
+  m.def("forward", [](Tensor x, Tensor w, OptT low, OptT by, double scale) { return product<false, false>(x, w, low, by, scale); },
+        "x w^T of x [M, K], w [N, K], and scale low by of narrow rows and [rank, N]", py::arg("x"), py::arg("w"), py::arg("low") = py::none(),
+        py::arg("by") = py::none(), py::arg("scale") = 1.0);
+  m.def("input_gradient", [](Tensor dy, Tensor w, OptT low, OptT by, double scale) { return product<true, false>(dy, w, low, by, scale); },
+        "dy w of dy [M, N], w [N, K], and scale low by of narrow rows and [rank, K]", py::arg("dy"), py::arg("w"), py::arg("low") = py::none(),
+        py::arg("by") = py::none(), py::arg("scale") = 1.0);
   m.def("weight_gradient", [](Tensor dy, Tensor x) { return product<true, true>(dy, x); }, "dy^T x of dy [M, N], x [M, K]");
 }

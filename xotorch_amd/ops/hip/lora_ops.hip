@@ -1,13 +1,14 @@
 // The low-rank terms of adapted linears (bf16 rows; fp32 adapters A [r, K] and, turned so that
 // a wave reads whole lines of it, B [r, N]; r <= 16):
 //   sums   low [M, r] = t w^T and, of narrow rows c [M, r], t^T c
-//   add    out += low w
+//   add    out += low w, where gemm_ops.hip does not add it inside the product
 // (The reference has adapters as data only, train/data/lora.)
 //
 // What bounds them is t, read once, or out, read and written: library products of 8 features
 // read a gradient once for either sum. us, library beside, 4096 tokens, rank 8: both sums of
 // 28672 features 55 (126), of 4096 13 (41); the sum added to 28672 102 (132), to 14336 56 (72),
-// to 4096 14 (19). Four layers of 4096 with 8 x 512 tokens, forward and back, 14300 (15500).
+// to 4096 14 (19). Four layers of 4096 with 8 x 512 tokens, forward and back, 14300 (15500); 13700 with
+// terms added inside the products.
 // Here a block holds a strip of 256 columns of t and walks down its rows in steps of 64 through
 // two LDS buffers; a step is multiplied along its rows and, read by transposing, along its
 // columns. Sums of strips and of runs of rows are added up by another kernel, in order.

@@ -6,7 +6,7 @@ that is itself differentiated."""
 from __future__ import annotations
 
 import os
-from typing import Callable, Sequence
+from typing import Callable, Optional, Sequence
 
 import torch
 
@@ -201,6 +201,20 @@ def product(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
   return torch.nn.functional.linear(x, weight)
 
 
+def adapted_product(x: torch.Tensor, weight: torch.Tensor, low: torch.Tensor, by: torch.Tensor, scale: float) -> torch.Tensor:
+  """x W^T + scale low by of rows [M, K], fp32 rows [M, rp] and an adapter [rank, N] (hip/lora_ops.hip).
+  Added inside the product, the term spares a pass over its result, so that sums of up to 8000 are the
+  kernels' up to 8192 tokens: us of 4096 by [28672, 4096], rank 8, the library's product and the pass 732, so
+  694; of longer sums the pass is a smaller part: [4096, 14336] 322, 319."""
+  M, (N, K) = x.shape[0], weight.shape
+  own = forward_wins(M, N, K) or forward_gains(M, N, K) or 2000 < M <= 8192 and forward_gains(2000, N, K) and K <= 8000
+  if own and weight.is_contiguous() and weight.data_ptr() % 16 == 0:
+    return _hip_gemm().forward(_rows(x), weight, low, by, scale)
+  out = torch.nn.functional.linear(x, weight)
+  _hip_lora().add(out, low, by, scale)
+  return out
+
+
 def takes_product(x: torch.Tensor, weight: torch.Tensor) -> bool:
   """Whether `product` is a linear of these without a gradient, of more rows than the
   kernels of decode steps take. Prompts by it and gate_product, and by the library, us: 300
@@ -234,12 +248,15 @@ def gate_product(x: torch.Tensor, gate_up: torch.Tensor) -> torch.Tensor:
   return _hip_experts().gate_product(_rows(x.reshape(-1, x.shape[-1])), gate_up).view(*x.shape[:-1], gate_up.shape[0] // 2)
 
 
-def input_gradient(dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-  """dy W of rows [M, N]"""
+def input_gradient(dy: torch.Tensor, weight: torch.Tensor, low: Optional[torch.Tensor] = None, by: Optional[torch.Tensor] = None) -> torch.Tensor:
+  """dy W of rows [M, N], and low by of an adapter [rank, K]"""
   M, (N, K) = dy.shape[0], weight.shape
   if (input_wins(M, N, K) or input_gains(M, N, K)) and once(dy, weight) and weight.is_contiguous() and weight.data_ptr() % 16 == 0:
-    return _hip_gemm().input_gradient(_rows(dy), weight)
-  return dy @ weight
+    return _hip_gemm().input_gradient(_rows(dy), weight, low, by)
+  dx = dy @ weight
+  if low is not None:
+    _hip_lora().add(dx, low, by, 1.0)
+  return dx
 
 
 def weight_gradient(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:

@@ -56,14 +56,18 @@ class _Adapted(torch.autograd.Function):
 
 class _AdaptedRows(torch.autograd.Function):
   """The same with fp32 adapters A and B^T by hip/lora_ops.hip: a gradient is read once for both of its
-  narrow sums, nothing narrow is rounded but as an operand of the matrix cores."""
+  narrow sums, nothing narrow is rounded but as an operand of their matrix cores; the products of
+  hip/gemm_ops.hip add the terms before they store."""
 
   @staticmethod
   def forward(ctx, x, weight, bias, a, bt, scaling):
     hip, rows = train_ops._hip_lora(), train_ops._rows(x.reshape(-1, x.shape[-1]))
-    out = F.linear(rows, weight, bias) if bias is not None else train_ops.product(rows, weight)
     low, columns = hip.sums(rows, a, 1.0, None, a.shape[0], 1.0, False)
-    hip.add(out, low, bt, scaling)
+    if bias is None:
+      out = train_ops.adapted_product(rows, weight, low, bt, scaling)
+    else:
+      out = F.linear(rows, weight, bias)
+      hip.add(out, low, bt, scaling)
     ctx.save_for_backward(x, weight, bias, a, bt, columns)
     ctx.scaling = scaling
     return out.view(*x.shape[:-1], weight.shape[0])
@@ -83,9 +87,7 @@ class _AdaptedRows(torch.autograd.Function):
     if need_b:
       db = found.pop().t()  # lies as B does
     if need_x:
-      dx = train_ops.input_gradient(dy, weight)
-      hip.add(dx, found[0], a, 1.0)
-      dx = dx.view(x.shape)
+      dx = train_ops.input_gradient(dy, weight, found[0], a).view(x.shape)
     if need_a:
       da, = hip.sums(train_ops._rows(x.reshape(-1, x.shape[-1])), None, 1.0, found[1], rank, 1.0, True)
     return dx, None, None, da, db, None
