@@ -89,6 +89,33 @@ def test_sums_over_parts_of_k(B, S, H, KVH, hd, n, bias, norms):
     assert torch.equal(x, y)
 
 
+@pytest.mark.parametrize("start", [0, 8, 13])
+@pytest.mark.parametrize("B,S,H,KVH,hd,spread", [(1, 1027, 6, 3, 128, False), (3, 700, 7, 2, 64, False), (2, 515, 9, 3, 128, True), (20, 61, 5, 2, 128, False),
+                                                 (2, 1024, 5, 2, 64, True)])
+def test_values_turned_among_lanes(B, S, H, KVH, hd, spread, start):
+  """Eight channels a lane, values of eight positions written at once where they lie side by side, against a
+  wave a token: starts on and off a multiple of eight, sequences that end within one, shorter ones than a run has."""
+  from xotorch_amd import ops
+  from xotorch_amd.engine.kvcache import ShardKVCache
+  T = S + 70
+  g = torch.Generator(device="cuda").manual_seed(S + start)
+  ones, zeros = torch.ones(T, hd // 2, device="cuda"), torch.zeros(T, hd // 2, device="cuda")
+  qkv = torch.randn(B, S, (H + 2 * KVH) * hd, generator=g, device="cuda").to(torch.bfloat16)
+  pos = torch.arange(start, start + S, dtype=torch.int32, device="cuda")
+  if spread:
+    pos = torch.stack([pos + 8 * b + (b > 0) for b in range(B)])
+  found = []
+  for step in (S, 4):
+    c = ShardKVCache(1, B, KVH, T, hd, torch.bfloat16, "cuda")[0]
+    queries = []
+    for at in range(0, S, step):
+      part = qkv[:, at:at + step].clone()
+      ops.rope_qkv_append(part, ones, zeros, pos[..., at:at + step].contiguous(), c.k, c.v, H, KVH, hd, c.kp, c.vp)
+      queries.append(part[..., :H * hd])
+    found.append((torch.cat(queries, 1), *c[:4]))
+  assert all(torch.equal(x, y) for x, y in zip(*found))
+
+
 @pytest.mark.parametrize("B,S,H,KVH,hd,per_row,norms", [(1, 1027, 4, 1, 128, False, True), (3, 333, 30, 2, 64, True, False),
                                                         (2, 515, 9, 3, 128, True, True)])
 def test_rows_of_prompts_as_one_by_one(B, S, H, KVH, hd, per_row, norms):

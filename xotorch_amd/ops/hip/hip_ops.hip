@@ -319,10 +319,12 @@ __global__ __launch_bounds__(256) void rope_qkv_append_kernel(
   }
 }
 
-// The same for head dims 64 and 128 without fp8 copies: a wave has 8 or 4 tokens of one
-// head, a lane 4 channels and their partners, so that rows move in pieces of 8 bytes.
-// Bound by memory and by the waves' starts: 6001 tokens of 48 heads of 128 48 us (170 MB;
-// 75 with a wave a token), 8192 of 80 89 us (171).
+// The same for head dims 64 and 128 without fp8 copies: a wave has some tokens of one head, a lane
+// E channels and their partners, so that rows move in pieces of 2 E bytes. Eight tokens in a row
+// whose first is a multiple of eight turn their values among lanes, as the copy that the matrix
+// cores read has eight positions of a channel side by side: else it is written in pieces of 2 bytes.
+// Bound by memory and by the waves' starts: 6001 tokens of 48 heads of 128 36 us (170 MB; 50 with
+// E = 4, 75 with a wave a token), 8192 of 80 70 us (89; 171).
 struct RopeRows {
   const float* sums;  // or null: fp32 sums over nsums parts of k [nsums][B*S][slots*HD]
   const unsigned short* bias;
@@ -331,23 +333,53 @@ struct RopeRows {
   const int* positions;
   unsigned short *kc, *vc, *kpc, *vpc;
   const unsigned short *qn, *kn;
-  int nsums, B, S, H, KVH, T, T32, per_row;
+  int nsums, B, S, H, KVH, T, T32, per_row, run;  // waves' tokens are of one run of so many
   float eps;
 };
-template <int HD, bool SUMS>
+template <int E>
+using Channels = __attribute__((ext_vector_type(E))) unsigned short;
+
+// Rows of eight lanes, `apart` from one another, to columns: of channels 0 .. 7 of a lane's own row
+// channel `r` of all eight
+DEVINL Channels<8> turned(Channels<8> v, int r, int apart) {
+  typedef __attribute__((ext_vector_type(4))) unsigned uint4_t;
+  uint4_t d = __builtin_bit_cast(uint4_t, v);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const unsigned other = __shfl_xor(d[k], apart);
+    d[k] = r & 1 ? other >> 16 | (d[k] & 0xffff0000u) : (d[k] & 0xffffu) | other << 16;
+  }
+#pragma unroll
+  for (int k = 0; k < 4; k += 2) {  // d[k]: rows r & ~1 and after of channel 2 k + (r & 1)
+    const unsigned other = __shfl_xor(r & 2 ? d[k] : d[k + 1], apart * 2);
+    if (r & 2) d[k] = other;
+    else d[k + 1] = other;
+  }
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {  // d[k], d[k + 1]: rows r & ~3 and after of channel (r & 3) + 2 k
+    const unsigned other = __shfl_xor(r & 4 ? d[k] : d[k + 2], apart * 4);
+    if (r & 4) d[k] = other;
+    else d[k + 2] = other;
+  }
+  return __builtin_bit_cast(Channels<8>, d);
+}
+
+template <int HD, bool SUMS, int E>
 __global__ __launch_bounds__(256) void rope_rows_kernel(RopeRows a) {
-  constexpr int HALF = HD / 2, LANES = HALF / 4, ROWS = 64 / LANES;
+  constexpr int HALF = HD / 2, LANES = HALF / E, ROWS = 64 / LANES;
+  typedef Channels<E> piece_t;
   const int lane = threadIdx.x & 63, slots = a.H + 2 * a.KVH, rows = a.B * a.S;
   const int unit = blockIdx.x * 4 + (threadIdx.x >> 6), slot = unit % slots;
-  const int bs = unit / slots * ROWS + lane / LANES, d = lane % LANES * 4;
-  if (bs >= rows) return;
+  const int of_run = (a.run + ROWS - 1) / ROWS, run = unit / slots / of_run, in_run = unit / slots % of_run * ROWS + lane / LANES;
+  const int bs = run * a.run + in_run, d = lane % LANES * E;
+  if (bs >= rows || in_run >= a.run) return;
   const int b = bs / a.S, s = bs - b * a.S, pos = a.positions[a.per_row ? bs : s];
   unsigned short* row = a.qkv + ((size_t)bs * slots + slot) * HD + d;
-  float x[2][4];
-  ushort4_t y[2];  // as projected, then rotated
+  float x[2][E];
+  piece_t y[2];  // as projected, then rotated
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    if (SUMS) {
+    if constexpr (SUMS) {
       const size_t width = (size_t)slots * HD, stride = rows * width, at = (size_t)slot * HD + d + h * HALF;
       const float* p = a.sums + bs * width + at;
       floatx4 v = *(const floatx4*)p;
@@ -368,53 +400,69 @@ __global__ __launch_bounds__(256) void rope_rows_kernel(RopeRows a) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) y[h][j] = f2b(v[j]);
     } else
-      y[h] = *(const ushort4_t*)(row + h * HALF);
+      y[h] = *(const piece_t*)(row + h * HALF);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) x[h][j] = b2f(y[h][j]);
+    for (int j = 0; j < E; ++j) x[h][j] = b2f(y[h][j]);
   }
   if (slot < a.H + a.KVH) {
     const unsigned short* w = slot < a.H ? a.qn : a.kn;
     if (w) {
       float ss = 0.f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) ss += x[0][j] * x[0][j] + x[1][j] * x[1][j];
+      for (int j = 0; j < E; ++j) ss += x[0][j] * x[0][j] + x[1][j] * x[1][j];
 #pragma unroll
       for (int m = LANES / 2; m > 0; m >>= 1) ss += __shfl_xor(ss, m);
       const float inv = rsqrtf(ss / (float)HD + a.eps);
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const ushort4_t by = *(const ushort4_t*)(w + d + h * HALF);
+        const piece_t by = *(const piece_t*)(w + d + h * HALF);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) x[h][j] *= inv * b2f(by[j]);
+        for (int j = 0; j < E; ++j) x[h][j] *= inv * b2f(by[j]);
       }
     }
-    const floatx4 c = *(const floatx4*)(a.cosb + (size_t)pos * HALF + d), sn = *(const floatx4*)(a.sinb + (size_t)pos * HALF + d);
+    const float *c = a.cosb + (size_t)pos * HALF + d, *sn = a.sinb + (size_t)pos * HALF + d;
+    floatx4 cv[E / 4], sv[E / 4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      y[0][j] = f2b(x[0][j] * c[j] - x[1][j] * sn[j]);
-      y[1][j] = f2b(x[1][j] * c[j] + x[0][j] * sn[j]);
+    for (int i = 0; i < E / 4; ++i) cv[i] = *(const floatx4*)(c + i * 4), sv[i] = *(const floatx4*)(sn + i * 4);
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+      y[0][j] = f2b(x[0][j] * cv[j / 4][j % 4] - x[1][j] * sv[j / 4][j % 4]);
+      y[1][j] = f2b(x[1][j] * cv[j / 4][j % 4] + x[0][j] * sv[j / 4][j % 4]);
     }
   }
   if (slot < a.H) {
-    *(ushort4_t*)row = y[0];
-    *(ushort4_t*)(row + HALF) = y[1];
+    *(piece_t*)row = y[0];
+    *(piece_t*)(row + HALF) = y[1];
     return;
   }
   const bool key = slot < a.H + a.KVH;
   const size_t head = (size_t)b * a.KVH + (slot - a.H - (key ? 0 : a.KVH));
   unsigned short* dst = (key ? a.kc : a.vc) + (head * a.T + pos) * HD + d;
-  *(ushort4_t*)dst = y[0];
-  *(ushort4_t*)(dst + HALF) = y[1];
+  *(piece_t*)dst = y[0];
+  *(piece_t*)(dst + HALF) = y[1];
   if (!a.kpc) return;
+  if constexpr (E == 8) {
+    // all of eight rows there, of one sequence, one position after the other from a multiple of eight on
+    const int r = lane / LANES % 8, first = __shfl(pos, lane - r * LANES), b0 = __shfl(b, lane - r * LANES);
+    if (!key && __all(in_run - r + 7 < a.run && first % 8 == 0 && pos == first + r && b == b0)) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int e = d + h * HALF + r;
+        *(piece_t*)(a.vpc + ((head * (HD / 16) + (e >> 4)) * (a.T32 >> 5) + (pos >> 5)) * 512 + (((pos & 31) >> 3) * 16 + (e & 15)) * 8) =
+            turned(y[h], r, LANES);
+      }
+      return;
+    }
+  }
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int e = d + h * HALF;
     if (key)
-      *(ushort4_t*)(a.kpc + (head * (a.T32 >> 4) + (pos >> 4)) * (HD / 32 * 512) + (e >> 5) * 512 +
-                   (((e & 31) >> 3) * 16 + (pos & 15)) * 8 + (e & 7)) = y[h];
+      *(piece_t*)(a.kpc + (head * (a.T32 >> 4) + (pos >> 4)) * (HD / 32 * 512) + (e >> 5) * 512 +
+                  (((e & 31) >> 3) * 16 + (pos & 15)) * 8 + (e & 7)) = y[h];
     else
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < E; ++j)
         a.vpc[((head * (HD / 16) + (e >> 4)) * (a.T32 >> 5) + (pos >> 5)) * 512 +
               (((pos & 31) >> 3) * 16 + (e & 15) + j) * 8 + (pos & 7)] = y[h][j];
   }
@@ -2758,10 +2806,17 @@ void rope_qkv_append(torch::Tensor qkv, torch::Tensor cos, torch::Tensor sin,
       ((at(cos.data_ptr()) | at(sin.data_ptr()) | at(sp)) & 15) == 0) {
     RopeRows a{sp, bp, (unsigned short*)qkv.data_ptr(), cos.data_ptr<float>(), sin.data_ptr<float>(), positions.data_ptr<int>(),
                (unsigned short*)kc.data_ptr(), (unsigned short*)vc.data_ptr(), kpc, vpc, qnp, knp, nsums, B, S, H, KVH, T, T32,
-               npos == B * S && npos != S, (float)norm_eps};
-    auto rows_kernel = hd == 128 ? (sp ? rope_rows_kernel<128, true> : rope_rows_kernel<128, false>)
-                                 : (sp ? rope_rows_kernel<64, true> : rope_rows_kernel<64, false>);
-    hipLaunchKernelGGL(rows_kernel, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, cur_stream(), a);
+               npos == B * S && npos != S, 0, (float)norm_eps};
+    // eight channels a lane where the waves are enough still and rows lie on 16 bytes. Each sequence begins with a
+    // wave of its own, so that positions are multiples of eight where they were in the first
+    const int run = S >= 64 ? S : B * S;
+    const long long half = (long long)(B * S / run) * ((run + 1024 / hd - 1) / (1024 / hd)) * (H + 2 * KVH);
+    const bool eight = !sp && half >= 1024 &&
+                       ((at(qkv.data_ptr()) | at(kc.data_ptr()) | at(vc.data_ptr()) | at(kpc) | at(vpc) | at(qnp) | at(knp)) & 15) == 0;
+    a.run = eight ? run : B * S;
+    auto rows_kernel = hd == 128 ? (sp ? rope_rows_kernel<128, true, 4> : eight ? rope_rows_kernel<128, false, 8> : rope_rows_kernel<128, false, 4>)
+                                 : (sp ? rope_rows_kernel<64, true, 4> : eight ? rope_rows_kernel<64, false, 8> : rope_rows_kernel<64, false, 4>);
+    hipLaunchKernelGGL(rows_kernel, dim3((unsigned)(((eight ? half : units) + 3) / 4)), dim3(256), 0, cur_stream(), a);
     return;
   }
   auto kernel = sp ? rope_qkv_append_kernel<true> : rope_qkv_append_kernel<false>;
