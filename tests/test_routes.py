@@ -243,7 +243,10 @@ def test_gradients_of_inputs_go_where_they_are_faster():
 def test_products_that_later_tiles_gained():
   """Long sums, small weights of many tokens and ordinary weights of up to 2000; gradients of inputs of up to 8192."""
   from xotorch_amd.ops.train_ops import forward_gains, input_gains
-  for M, N, K, own in [(64, 8192, 8064, False), (65, 8192, 8064, True), (2001, 8192, 8064, False), (8192, 5120, 17408, True), (8193, 5120, 17408, False),
+  for M, N, K, own in [(64, 8192, 8064, False), (65, 8192, 8064, True), (1000, 8192, 8064, True), (1001, 8192, 8064, False),
+                       (2000, 6144, 8064, True), (2001, 6144, 8064, False),
+                       (1100, 8192, 28672, True), (1101, 8192, 28672, False), (1541, 8192, 28672, True), (1791, 8192, 28672, False),
+                       (8192, 5120, 17408, True), (8193, 5120, 17408, False),
                        (8192, 8192, 28672, False), (1000, 2048, 3072, False), (1001, 2048, 3072, True), (8192, 2048, 3072, True), (128, 28672, 4096, False),
                        (129, 28672, 4096, True), (2000, 28672, 4096, True), (2001, 28672, 4096, False), (100, 6144, 4096, True), (100, 16384, 2048, False),
                        (1500, 892, 2048, False), (1500, 2048, 832, False), (1500, 2050, 2048, False), (1500, 2048, 2056, False), (1500, 128256, 2048, False)]:

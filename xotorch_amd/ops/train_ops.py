@@ -170,14 +170,17 @@ def input_wins(M: int, N: int, K: int) -> bool:
 
 def forward_gains(M: int, N: int, K: int) -> bool:
   """What is faster of forward_wins' rest since there are tiles of 64 to 224 rows of x: long
-  sums 0.27 to 1.15 (0.81), narrow ones of the longest, of more tokens 0.58 to 1.06 (0.74); small
-  weights 0.68 to 1.07 (0.89); others up to 1000 tokens 0.59 to 1.13 (0.92), up to 2000 0.71 to
+  sums 0.27 to 1.15 (0.81; wide ones up to 1000 tokens), narrow ones of the longest, of more
+  tokens 0.58 to 1.06 (0.74); small weights 0.68 to 1.07 (0.89); others up to 1000 tokens 0.59 to 1.13 (0.92), up to 2000 0.71 to
   1.12 (0.95). What it leaves: more tokens 0.67 to 1.18 (0.99); 65 to 128 by short sums and by
   wide weights 0.81 to 1.22 (0.98); features and rows that were not measured."""
   if K % 64 or N % 4 or not 896 <= N < 100_000 or not 896 <= K <= _WIDEST or not 64 < M <= 8192:
     return False
   if K > 8000:
-    return M <= 2000 or K > 16384 and N <= 6144
+    if N <= 6144:
+      return M <= 2000 or K > 16384
+    # [8192, 28672] to 1100 tokens 0.62, to 1540 0.66 to 1.14 (1.0), to 1790 0.79, more 1.05: as blocks fill rounds
+    return M <= 1000 or K > 16384 and (M <= 1100 or 1540 < M <= 1790)
   return 1000 < M if N * K <= 7_000_000 else M <= 2000 and (M > 128 or K > 3200 and N <= 20000)
 
 
