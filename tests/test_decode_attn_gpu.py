@@ -116,6 +116,42 @@ def test_values_turned_among_lanes(B, S, H, KVH, hd, spread, start):
   assert all(torch.equal(x, y) for x, y in zip(*found))
 
 
+@pytest.mark.parametrize("what", ["kp as rows", "vp of fewer positions", "kp of fewer sequences", "copies of fewer positions", "caches of fewer heads",
+                                  "values of fewer positions", "scales of fewer positions", "fp32 caches"])
+def test_caches_that_kernels_would_write_past(what):
+  """Refused on the host, before anything is launched: sizes that the kernels' indexes do not fit."""
+  from xotorch_amd.ops import _hip_ops
+  B, S, H, KVH, hd, T = 2, 40, 4, 2, 128, 64
+  f8 = what.startswith("scales")
+  make = lambda *size, dtype=torch.bfloat16: torch.zeros(*size, dtype=dtype, device="cuda")
+  kc, vc = make(B, KVH, T, hd), make(B, KVH, T, hd)
+  kp, vp = (make(*size, 64, 8, dtype=torch.uint8 if f8 else torch.bfloat16) for size in ((B, KVH, T // 16, hd // 32), (B, KVH, hd // 16, T // 32)))
+  scales = [make(B, KVH, T, dtype=torch.float32) for _ in range(2)] if f8 else [None, None]
+  if what == "kp as rows":
+    kp = make(B, KVH, T, hd)
+  elif what == "vp of fewer positions":
+    vp = vp[:, :, :, :1].contiguous()
+  elif what == "kp of fewer sequences":
+    kp = kp[:1]
+  elif what == "copies of fewer positions":
+    kp, vp = kp[:, :, :2].contiguous(), vp[:, :, :, :1].contiguous()
+  elif what == "caches of fewer heads":
+    kc, vc = kc[:, :1].contiguous(), vc[:, :1].contiguous()
+  elif what == "values of fewer positions":
+    vc = vc[:, :, :48].contiguous()
+  elif what == "fp32 caches":
+    kc, vc = kc.float(), vc.float()
+  else:
+    scales[1] = scales[1][:, :, :32].contiguous()
+  qkv, at = make(B, S, (H + 2 * KVH) * hd), torch.arange(S, dtype=torch.int32, device="cuda")
+  table = make(T, hd // 2, dtype=torch.float32)
+  with pytest.raises(RuntimeError):
+    _hip_ops.rope_qkv_append(qkv, table, table, at, kc, vc, H, KVH, hd, kp, vp, k_scale=scales[0], v_scale=scales[1])
+  if what not in ("copies of fewer positions", "caches of fewer heads", "values of fewer positions", "fp32 caches"):
+    with pytest.raises(RuntimeError):
+      _hip_ops.attn_decode_mfma(make(B, 1, H, hd), kp, vp, torch.full((B,), 20, dtype=torch.int32, device="cuda"), T, k_scale=scales[0], v_scale=scales[1])
+
+
 @pytest.mark.parametrize("B,S,H,KVH,hd,per_row,norms", [(1, 1027, 4, 1, 128, False, True), (3, 333, 30, 2, 64, True, False),
                                                         (2, 515, 9, 3, 128, True, True)])
 def test_rows_of_prompts_as_one_by_one(B, S, H, KVH, hd, per_row, norms):

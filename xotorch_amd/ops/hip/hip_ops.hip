@@ -2745,6 +2745,9 @@ void rope_qkv_append(torch::Tensor qkv, torch::Tensor cos, torch::Tensor sin,
   const int T = kc.size(2);
   CHK(qkv.size(2) == (H + 2 * KVH) * hd);
   CHK(hd <= 128 && hd % 2 == 0);
+  // what the kernels index by: rows of sequences, heads and positions lie where these sizes say
+  CHK(kc.is_cuda() && kc.dtype() == torch::kBFloat16 && vc.is_cuda() && vc.dtype() == torch::kBFloat16);
+  CHK(kc.dim() == 4 && kc.size(0) >= B && kc.size(1) == KVH && kc.size(3) == hd && vc.sizes() == kc.sizes());
   const int npos = (int)positions.numel();
   CHK(npos == S || npos == B * S);
   CHK(positions.is_contiguous());
@@ -2758,16 +2761,19 @@ void rope_qkv_append(torch::Tensor qkv, torch::Tensor cos, torch::Tensor sin,
   if (kp.has_value() && vp.has_value()) {
     CHK((hd == 128 || (hd == 64 && kp->dtype() != torch::kUInt8)) && kp->is_contiguous() && vp->is_contiguous());
     T32 = (int)kp->size(2) * 16;
+    CHK(kp->is_cuda() && vp->is_cuda() && vp->dtype() == kp->dtype() && T32 % 32 == 0 && T <= T32);
+    for (const auto* p : {&*kp, &*vp}) CHK(p->size(0) >= B && p->numel() == p->size(0) * KVH * T32 * hd);
     if (kp->dtype() == torch::kUInt8) {
       // fp8 packed mode: per-row e4m3 scales required
       CHK(k_scale.has_value() && v_scale.has_value());
-      CHK(k_scale->dtype() == torch::kFloat32 && k_scale->is_contiguous());
-      CHK(v_scale->dtype() == torch::kFloat32 && v_scale->is_contiguous());
+      for (const auto* p : {&*k_scale, &*v_scale})
+        CHK(p->is_cuda() && p->dtype() == torch::kFloat32 && p->is_contiguous() && p->numel() >= (int64_t)B * KVH * T32);
       kp8 = (unsigned char*)kp->data_ptr();
       vp8 = (unsigned char*)vp->data_ptr();
       skp = k_scale->data_ptr<float>();
       svp = v_scale->data_ptr<float>();
     } else {
+      CHK(kp->dtype() == torch::kBFloat16);
       kpc = (unsigned short*)kp->data_ptr();
       vpc = (unsigned short*)vp->data_ptr();
     }
@@ -2910,6 +2916,10 @@ torch::Tensor attn_decode_mfma(torch::Tensor q, torch::Tensor kp, torch::Tensor 
   TORCH_CHECK(hd == 128, "attn_decode_mfma requires head_dim 128");
   const int KVH = kp.size(1);
   const int T32 = kp.size(2) * 16;
+  CHK(vp.dtype() == kp.dtype() && T32 % 32 == 0 && seq_lens.numel() >= B);
+  for (const auto* p : {&kp, &vp}) CHK(p->is_cuda() && p->size(0) >= B && p->numel() == p->size(0) * KVH * T32 * hd);
+  if (fp8)
+    for (const auto* p : {&*k_scale, &*v_scale}) CHK(p->is_cuda() && p->is_contiguous() && p->numel() >= (int64_t)B * KVH * T32);
   const long long q_stride = q.stride(0);
   // one wave per (b, kvh, split); target >= ~2048 waves so 16 waves/CU keep
   // the packed-cache stream deep while chunks stay >= 32 positions
