@@ -54,6 +54,30 @@ def test_routes_of_bf16_logits_and_wide_sums(T, E, k, D):
   assert wide.dtype == torch.float32 and torch.equal(wide.to(torch.bfloat16), rounded)
 
 
+@pytest.mark.parametrize("E,k,mode,groups,keep", [(8, 2, 0, 1, 1), (5, 5, 0, 1, 1), (256, 8, 0, 1, 1), (16, 4, 1, 1, 1), (16, 6, 1, 4, 1)])
+def test_every_pick_is_another_expert(E, k, mode, groups, keep):
+  """Rows that are no numbers, infinities and fewer open experts than picks: a token has one row in an expert,
+  which is what the room for its rows is made for."""
+  from xotorch_amd import ops
+  hip = ops._load_hip()
+  T = 33
+  g = torch.Generator(device="cuda").manual_seed(E)
+  logits = torch.randn(T, E, generator=g, device="cuda")
+  logits[3], logits[4], logits[5] = torch.nan, torch.inf, -torch.inf
+  logits[6, 1], logits[7, E - 1] = torch.nan, torch.inf
+  logits[8, 1:] = -torch.inf  # one expert is open
+  for given in (logits, logits.to(torch.bfloat16)):
+    idx, w = hip.moe_route(given, None, k, mode, groups, keep)
+    at = idx.long().sort(-1).values
+    assert int(at.min()) >= 0 and int(at.max()) < E and bool((at.diff(dim=-1) > 0).all())
+    assert bool(w[3].isnan().all()) and bool(w[9:].isfinite().all())
+    if mode == 0:
+      assert bool(w[6].isnan().all()) and float(w[8].max()) == 1.0 and int(idx[8, 0]) == 0
+    C = 64
+    gather, place = hip.moe_build(idx, E, C)
+    assert bool((place.long() // C == idx).all()) and place.unique().numel() == T * k and bool((gather[place.long()] == torch.arange(T, device="cuda")[:, None]).all())
+
+
 @pytest.mark.parametrize("tile", [128, 256])
 @pytest.mark.parametrize("K,F", [(64, 16), (128, 144), (192, 272), (320, 64), (576, 528)])  # steps of k, tiles of features
 @pytest.mark.parametrize("swiglu", [False, True])

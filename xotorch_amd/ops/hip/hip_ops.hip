@@ -1465,10 +1465,19 @@ __global__ __launch_bounds__(256) void moe_route_kernel(
       }
     }
   }
-  // iterative wave-wide top-k on c; weights come from s
+  // iterative wave-wide top-k on c; weights come from s. Every pick is another expert, whatever
+  // the logits are: moe_build has room for one row of a token in an expert. A row that is not a
+  // number has no choice (nor has one past the groups' own): the first that are left, in order,
+  // and its weights are NaN.
   float wsum = 0.f;
   float wk[8];
   int ik[8];
+  unsigned left = 0;  // this lane's experts that are not picked yet
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    left |= (lane * 4 + j < E ? 1u : 0u) << j;
+    if (!(c[j] == c[j])) c[j] = -INFINITY;
+  }
   for (int t = 0; t < k; ++t) {
     float mx = fmaxf(fmaxf(c[0], c[1]), fmaxf(c[2], c[3]));
 #pragma unroll
@@ -1477,7 +1486,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(
     int my = INT_MAX;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      if (c[j] == mx && lane * 4 + j < my) my = lane * 4 + j;
+      if (c[j] == mx && (left >> j & 1) && lane * 4 + j < my) my = lane * 4 + j;
 #pragma unroll
     for (int m = 32; m > 0; m >>= 1) my = min(my, __shfl_xor(my, m));
     const int owner = my >> 2, slot = my & 3;
@@ -1491,7 +1500,10 @@ __global__ __launch_bounds__(256) void moe_route_kernel(
     ik[t] = my;
     wk[t] = sv;
     wsum += sv;
-    if (lane == owner) c[slot] = -INFINITY;
+    if (lane == owner) {
+      c[slot] = -INFINITY;
+      left &= ~(1u << slot);
+    }
   }
   if (lane == 0) {
     const float inv = (mode == 0 || norm_topk) ? 1.f / (wsum + 1e-20f) : 1.f;
@@ -3069,7 +3081,7 @@ std::vector<torch::Tensor> moe_route(torch::Tensor logits, c10::optional<torch::
   const bool wide = logits.dtype() == torch::kFloat32;
   CHK(logits.is_cuda() && (wide || logits.dtype() == torch::kBFloat16) && logits.is_contiguous() && logits.dim() == 2);
   const int T = logits.size(0), E = logits.size(1);
-  CHK(E <= 256 && k >= 1 && k <= 8 && n_group >= 1 && n_group <= 8);
+  CHK(E <= 256 && k >= 1 && k <= 8 && k <= E && n_group >= 1 && n_group <= 8);
   const float* bptr = nullptr;
   if (bias.has_value()) {
     CHK(bias->is_contiguous() && bias->dtype() == torch::kFloat32 && bias->numel() == E);
