@@ -323,3 +323,56 @@ def test_few_tokens_through_experts(T, E, k, D, I):
     seen = []
     moe.experts[0].register_forward_hook(lambda *a: seen.append(1))
     assert moe._grouped(x) is None
+
+
+@pytest.mark.parametrize("T", [1, 40, 256])
+@pytest.mark.parametrize("who", ["hook", "global hook", "autocast", "dispatch mode", "module of its own"])
+def test_experts_of_a_router_with_its_own_call(T, who):
+  """A router that somebody waits for is called, and its experts still go as two grouped products: the same numbers, as
+  whole ones are summed and rounded alike by either way. More tokens have all modules called."""
+  import contextlib
+  from torch.utils._python_dispatch import TorchDispatchMode
+  from xotorch_amd.models.config import ModelConfig
+  from xotorch_amd.models.llama import MoEMLP
+
+  class Seen(TorchDispatchMode):
+    def __torch_dispatch__(self, f, types, args=(), kwargs=None):
+      return f(*args, **(kwargs or {}))
+
+  class Router(torch.nn.Linear):
+    pass
+
+  E, k, D, I = 16, 4, 128, 192
+  g = torch.Generator(device="cuda").manual_seed(T)
+  moe = MoEMLP(ModelConfig(dim=D, n_experts=E, n_experts_per_tok=k, intermediate_dim=I)).to("cuda", torch.bfloat16)
+  make = lambda n: torch.randint(-1, 2, (n, D), generator=g, device="cuda").to(torch.bfloat16)
+  x, more = make(T), make(300)
+  with torch.no_grad():
+    for p in moe.parameters():
+      p.copy_(torch.randn(p.shape, generator=g, device="cuda") * p.shape[-1] ** -0.5)
+    moe.gate.weight.copy_(make(E))  # logits are whole numbers of up to 128
+    want, many = moe(x[None]), moe(more[None])
+    if who == "module of its own":
+      router = Router(D, E, bias=False)
+      router.weight = moe.gate.weight
+      moe.gate = router
+    called = []
+    with contextlib.ExitStack() as s:
+      if who in ("hook", "module of its own"):
+        h = moe.gate.register_forward_hook(lambda m, *a: called.append(m))
+      else:
+        h = torch.nn.modules.module.register_module_forward_hook(lambda m, *a: called.append(m))
+      s.callback(h.remove)
+      if who == "autocast":
+        s.enter_context(torch.autocast("cuda", torch.bfloat16))
+      if who == "dispatch mode":
+        s.enter_context(Seen())
+      found = moe._grouped(x)
+      assert found is not None and found[2] is None and moe._grouped(more) is None
+      got = moe(x[None])
+      assert [m for m in called if m is not moe] == [moe.gate]
+      assert torch.equal(got, want)
+      after = moe(more[None])
+      assert who in ("hook", "module of its own") or len(called) > 2 * k
+    assert (after.float() - many.float()).norm() <= 0.02 * many.float().norm()
+    assert moe._forward_decode(x, True).dtype == torch.float32

@@ -485,13 +485,10 @@ class MoEMLP(nn.Module):
 
   def _expert_weights(self):
     """The experts' weights (gate and up of all, down of all) where grouped products may read them:
-    bf16, one tensor per expert and projection, whose modules nobody waits for. Else None.
+    bf16, one tensor per expert and projection, whose modules nobody waits for by a hook of their own. Else None.
     Straight from where modules keep things, as a pass through 128 experts asks 256 modules in
     every layer: 740 us by their attributes, 117 so (40 with 8 experts)."""
     if self.n_experts > 256 or self.top_k > 8 or self.dim % 64 or self.intermediate % 64 or max(self.dim, self.intermediate) > 1 << 22:
-      return None
-    gate = self._modules["gate"]
-    if type(gate) is not nn.Linear or _watched(gate):
       return None
     ups, downs = [], []
     for e in self._modules["experts"]._modules.values():
@@ -510,32 +507,52 @@ class MoEMLP(nn.Module):
     return ups, downs
 
   def _grouped(self, flat):
-    """The experts' weights where tokens go through them as two grouped products, or None."""
+    """The experts' weights where tokens go through them as two grouped products, and the router's where
+    its logits are made with the choice; or None. Up to 256 tokens a router that somebody waits for, by a hook of
+    its own or a global one, that is another module or that autocast or a dispatch mode takes, has its own call and the
+    experts none: us of a layer with 1 and 32 tokens, expert by expert and so, 8 experts of 4096 x 14336 580, 155 and
+    570, 444; 128 of 2048 x 768 4510, 148 and 4535, 203. More tokens go by the modules then."""
+    few = flat.shape[0] <= 256
     if flat.dtype != torch.bfloat16 or not flat.is_cuda or self.wp_gate_up_fp8 is not None or not flat.is_contiguous() or not flat.numel() \
-       or (flat.shape[0] > 256 and os.getenv("XOT_FP8_PREFILL", "0") == "1"):
+       or (not few and os.getenv("XOT_FP8_PREFILL", "0") == "1"):
       return None
     found = self._expert_weights()
     if found is None:
       return None
-    weights = [_own(self._modules["gate"]), *found[0], *found[1]]
-    if not ops.alone(flat) or not ops._use_hip(flat) or any(type(w) not in train_ops.OWN for w in weights):
+    gate = self._modules["gate"]
+    alone = type(gate) is nn.Linear and not _watched(gate) and ops.alone(flat)
+    if not alone and (not few or train_ops.followed() or type(flat) not in train_ops.OWN):
+      return None
+    weights = [*found[0], *found[1]]
+    if not ops._use_hip(flat) or flat.get_device() != train_ops._current_device() or any(type(w) not in train_ops.OWN for w in weights):
       return None
     from xotorch_amd.ops.mixer_ops import load_hip
-    return found if load_hip("_hip_experts").readable(flat, weights) else None
+    readable = load_hip("_hip_experts").readable
+    router = _own(gate) if alone else None
+    if alone and not (type(router) in train_ops.OWN and readable(flat, [router])):
+      if not few:
+        return None
+      router = None
+    return (*found, router) if readable(flat, weights) else None
 
-  def _forward_grouped(self, flat, weights, wide=False):
+  def _forward_grouped(self, flat, found, wide=False):
     """Rows of all (token, expert) pairs are placed by counting, without the host; the
     products read tokens and weights where they lie, of experts that have a row. `wide`: fp32."""
     from xotorch_amd.ops.mixer_ops import load_hip
     hip = load_hip("_hip_experts")
+    ups, downs, router = found
     # tiles of 256 tokens from 110 rows an expert on: 8 experts of 4096 x 14336, two of
     # them a token, us with 128 and 256: 300 tokens 565, 577; 450 607, 602; 620 667, 578
     tile = 256 if flat.shape[0] * self.top_k >= 110 * self.n_experts else 128
-    # up to 256 tokens logits are rounded as those of the gate's own call, which hooks bring about
-    weight, row, *places = hip.route(flat, _own(self._modules["gate"]), None, self.top_k, 1, 1, 1.0, True, 0, False, False, tile,
-                                     flat.shape[0] <= 256)
+    rule = None, self.top_k, 1, 1, 1.0, True, 0, False, False, tile
+    if router is not None:
+      # up to 256 tokens logits are rounded as those of the gate's own call, which hooks bring about
+      weight, row, *places = hip.route(flat, router, *rule, flat.shape[0] <= 256)
+    else:
+      logits = self.gate(flat)
+      weight, row, *places = hip.route((logits if logits.dtype == torch.bfloat16 else logits.float()).contiguous(), None, *rule)
     product = hip.expert_product_of if self._many(flat) else hip.expert_few_of
-    y = product(product(flat, weights[0], *places, True), weights[1], *places, False)
+    y = product(product(flat, ups, *places, True), downs, *places, False)
     return ops._load_hip().moe_combine(y, row, weight, wide)
 
   def _forward_prefill_sorted(self, flat, weights, selected):
@@ -761,8 +778,8 @@ class ShardedModel(nn.Module):
     groups: List[List[XotLinear]] = [[], [], [], []]
     unread = set()  # experts whose copies nothing would read
     if mode != "all" and not ops.fp8_gemm_enabled():
-      unread = {id(p) for m in self.modules() if isinstance(m, MoEMLP) and m.gate.weight.dtype == torch.bfloat16
-                and m._expert_weights() is not None for e in m.experts for p in (e.gate_up_proj, e.down_proj)}
+      unread = {id(p) for m in self.modules() if isinstance(m, MoEMLP) and m._expert_weights() is not None
+                for e in m.experts for p in (e.gate_up_proj, e.down_proj)}
     for name, mod in self.named_modules():
       if not isinstance(mod, XotLinear) or not mod.packable() or id(mod) in unread:
         continue

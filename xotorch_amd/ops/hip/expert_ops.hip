@@ -28,8 +28,8 @@ constexpr int MAX_EXPERTS = 512, MAX_PICK = 16;  // shared ones among the expert
 // pick of E experts are chosen, then come top - pick that every token uses, all
 // in all; tile: rows of a tile
 // gate: the weight of these is the sigmoid of one more row of w, else one
-// narrow: logits as bf16, as a linear of their own leaves them
-struct RouteArgs { int T, D, E, top, groups, keep, nblk, tile; float scale; int pick, all, softmax, gate, narrow; };
+// narrow: logits as bf16, as a linear of their own leaves them; given: x are the logits
+struct RouteArgs { int T, D, E, top, groups, keep, nblk, tile; float scale; int pick, all, softmax, gate, narrow, given; };
 
 // RW waves share k. Sixteen lanes choose for a token, J experts each.
 template <typename T, bool WHOLE, int J, int RW>
@@ -47,7 +47,21 @@ __global__ __launch_bounds__(64 * RW) void route_kernel(
   const int t0 = blockIdx.x * RT, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
   const T* xr = x + (size_t)min(t0 + col, a.T - 1) * a.D;
   const int steps = (a.D + F::K - 1) / F::K;
-  for (int e0 = 0; e0 < Z; e0 += 64) {
+  auto scored = [&](int t, int e, float z) {  // logit e of token t
+    const float s = a.softmax && e < a.E ? z : 1.f / (1.f + expf(-z));
+    if (e < a.E) {
+      score[t * a.E + e] = s;
+      choice[t * a.E + e] = correction ? s + ld(correction + e) : s;
+    } else open[t] = s;
+  };
+  if (a.given) {
+    for (int i = threadIdx.x; i < RT * a.E; i += 64 * RW) {
+      const int t = i / a.E, e = i - t * a.E;
+      scored(t, e, ld(x + (size_t)min(t0 + t, a.T - 1) * a.E + e));
+    }
+    __syncthreads();
+  }
+  for (int e0 = 0; e0 < Z && !a.given; e0 += 64) {
     floatx4 acc[4];
     const T* wr[4];
 #pragma unroll
@@ -84,12 +98,7 @@ __global__ __launch_bounds__(64 * RW) void route_kernel(
         float z = 0.f;
 #pragma unroll
         for (int v = 0; v < RW; ++v) z += part[(v * RT + t) * 65 + (i & 63)];
-        if (a.narrow) z = rounded(z);
-        const float s = a.softmax && e < a.E ? z : 1.f / (1.f + expf(-z));
-        if (e < a.E) {
-          score[t * a.E + e] = s;
-          choice[t * a.E + e] = correction ? s + ld(correction + e) : s;
-        } else open[t] = s;
+        scored(t, e, a.narrow ? rounded(z) : z);
       }
     }
     __syncthreads();
@@ -752,16 +761,19 @@ __global__ __launch_bounds__(256) void add_norm_kernel(
 // `shared` experts follow the routed ones in every token's list (top counts
 // them then); their weight is the sigmoid of one more row of w (gate) or one.
 // on_input: the weights by row [T * top].
-std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, int64_t> route(Tensor x, Tensor w, OptT correction, int64_t pick,
+// w: the router's weights, or none: x are logits [T, E] that a router's own call has made
+std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, int64_t> route(Tensor x, OptT w, OptT correction, int64_t pick,
                                                                   int64_t groups, int64_t keep, double scale,
                                                                   bool softmax, int64_t shared, bool gate,
                                                                   bool on_input, int64_t tile_of, bool narrow) {
   const auto dt = io_type(x);
-  check_io(w, dt);
+  const bool given = !w;
+  CHK(!given || (shared == 0 && !narrow));
+  if (!given) check_io(*w, dt);
   gate = gate && shared > 0;
-  const int D = x.size(-1), T_ = x.numel() / D, E = w.size(0) - gate;
+  const int D = x.size(-1), T_ = x.numel() / D, E = given ? D : w->size(0) - gate;
   if (correction) { check_io(*correction, dt); CHK(correction->numel() == E); }
-  CHK(w.dim() == 2 && w.size(1) == D && T_ > 0 && shared >= 0);
+  CHK((given || (w->dim() == 2 && w->size(1) == D)) && T_ > 0 && shared >= 0);
   const int64_t top = pick + shared, all = E + shared;
   TORCH_CHECK(E >= 1 && all <= MAX_EXPERTS && pick >= 1 && pick <= MAX_PICK && pick <= E, "routing to ", pick, " of ", E,
               " experts and ", shared, " shared ones");
@@ -778,7 +790,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, int64_t> route(Tensor x, Tens
   auto idx = torch::empty({T_, top}, ints), rank = torch::empty({T_, top}, ints), row = torch::empty({T_, top}, ints);
   auto counts = torch::empty({all, nblk}, ints), total = torch::empty({all}, ints), first = torch::empty({all + 1}, ints);
   auto token = torch::empty({pairs}, ints), tiles = torch::empty({max_tiles + 1, 2}, ints);
-  const RouteArgs a{T_, D, E, (int)top, (int)groups, (int)keep, nblk, tile, (float)scale, (int)pick, (int)all, softmax, gate, narrow};
+  const RouteArgs a{T_, D, E, (int)top, (int)groups, (int)keep, nblk, tile, (float)scale, (int)pick, (int)all, softmax, gate, narrow, given};
   const hipStream_t stream = cur_stream();
   CHK(groups <= 4 * 65);
   BY_TYPE(dt, {
@@ -787,12 +799,12 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, int64_t> route(Tensor x, Tens
       const hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
       TORCH_CHECK(err == hipSuccess, "no LDS for the router");
       const size_t lds = (2 * RT * E + waves * RT * 65) * sizeof(float) + RT * (top + 1) * sizeof(int);  // parts of 16 bytes
-      hipLaunchKernelGGL(kernel, dim3(nblk), dim3(64 * waves), lds, stream, P<T>(x), P<T>(w), cp,
+      hipLaunchKernelGGL(kernel, dim3(nblk), dim3(64 * waves), lds, stream, P<T>(x), given ? nullptr : P<T>(*w), cp,
                          idx.data_ptr<int>(), M<float>(weight), rank.data_ptr<int>(), counts.data_ptr<int>(), a);
     };
     // few tokens: more waves on each
     const bool few = nblk <= 256;
-    if (D % Frag<T>::K) run(route_kernel<T, false, MAX_EXPERTS / 16, 4>, 4);
+    if (!given && D % Frag<T>::K) run(route_kernel<T, false, MAX_EXPERTS / 16, 4>, 4);
     else if (E <= 64) { if (few) run(route_kernel<T, true, 4, 16>, 16); else run(route_kernel<T, true, 4, 4>, 4); }
     else if (E <= 256) { if (few) run(route_kernel<T, true, 16, 16>, 16); else run(route_kernel<T, true, 16, 4>, 4); }
     else run(route_kernel<T, true, MAX_EXPERTS / 16, 4>, 4);

@@ -90,6 +90,12 @@ def plain(*tensors: torch.Tensor) -> bool:
   return not (_dispatch_modes() or _transforms() or _forward_ad._current_level >= 0 or _is_tracing())
 
 
+def followed() -> bool:
+  """Whether somebody follows the operators whom a kernel would lead astray (`plain` without a
+  dispatch mode, which sees less then but nothing wrong)."""
+  return _is_compiling() or bool(_transforms()) or _forward_ad._current_level >= 0 or bool(_is_tracing())
+
+
 def takes(x: torch.Tensor, *others: torch.Tensor) -> bool:
   """Whether these operands of a differentiated operator are for the kernels: plain
   bf16 GPU tensors, rows of whole 16 bytes up to 2^17 numbers (norms: up to 16384)."""
