@@ -325,6 +325,30 @@ def test_few_tokens_through_experts(T, E, k, D, I):
     assert moe._grouped(x) is None
 
 
+@pytest.mark.parametrize("T", [257, 300, 500])
+def test_prompts_beside_fp8_copies(T, monkeypatch):
+  """Copies for decode leave prompts to the grouped products, which read the weights themselves."""
+  from xotorch_amd.models.config import ModelConfig
+  from xotorch_amd.models.llama import MoEMLP
+  g = torch.Generator(device="cuda").manual_seed(T)
+  moe = MoEMLP(ModelConfig(dim=256, n_experts=32, n_experts_per_tok=2, intermediate_dim=128)).to("cuda", torch.bfloat16)
+  x = torch.randn(1, T, 256, generator=g, device="cuda").to(torch.bfloat16)
+  with torch.no_grad():
+    for p in moe.parameters():
+      p.copy_(torch.randn(p.shape, generator=g, device="cuda") * p.shape[-1] ** -0.5)
+    want = moe(x)
+    monkeypatch.setenv("XOT_FP8_GEMM", "1")
+    for e in moe.experts:
+      e.gate_up_proj.pack_decode()
+      e.down_proj.pack_decode()
+    moe.pack_grouped()
+    assert moe.wp_gate_up_fp8 is not None
+    assert moe._grouped(x[0]) is not None and moe._grouped(x[0, :256]) is None
+    assert torch.equal(moe(x), want)
+    monkeypatch.setenv("XOT_FP8_PREFILL", "1")
+    assert moe._grouped(x[0]) is None
+
+
 @pytest.mark.parametrize("T", [1, 40, 256])
 @pytest.mark.parametrize("who", ["hook", "global hook", "autocast", "dispatch mode", "module of its own"])
 def test_experts_of_a_router_with_its_own_call(T, who):

@@ -513,8 +513,10 @@ class MoEMLP(nn.Module):
     experts none: us of a layer with 1 and 32 tokens, expert by expert and so, 8 experts of 4096 x 14336 580, 155 and
     570, 444; 128 of 2048 x 768 4510, 148 and 4535, 203. More tokens go by the modules then."""
     few = flat.shape[0] <= 256
-    if flat.dtype != torch.bfloat16 or not flat.is_cuda or self.wp_gate_up_fp8 is not None or not flat.is_contiguous() or not flat.numel() \
-       or (not few and os.getenv("XOT_FP8_PREFILL", "0") == "1"):
+    if flat.dtype != torch.bfloat16 or not flat.is_cuda or not flat.is_contiguous() or not flat.numel():
+      return None
+    # fp8 copies are read up to 256 tokens, fp8 products of prompts are the modules'
+    if self.wp_gate_up_fp8 is not None if few else os.getenv("XOT_FP8_PREFILL", "0") == "1":
       return None
     found = self._expert_weights()
     if found is None:
