@@ -325,6 +325,27 @@ def test_few_tokens_through_experts(T, E, k, D, I):
     assert moe._grouped(x) is None
 
 
+@pytest.mark.parametrize("mode", ["auto", "all"])
+def test_no_copies_of_experts_that_are_read_where_they_lie(mode, monkeypatch):
+  from xotorch_amd.models.config import config_from_hf
+  from xotorch_amd.models.llama import ShardedModel
+  from xotorch_amd.models.registry import builtin_config
+  from xotorch_amd.shard import Shard
+  raw = dict(builtin_config("mixtral-8x7b"))
+  raw.update(hidden_size=256, intermediate_size=512, num_attention_heads=4, num_key_value_heads=2, vocab_size=256)
+  cfg = config_from_hf(raw, "mixtral-gpu-tiny")
+  model = ShardedModel(cfg, Shard("mixtral-gpu-tiny", 1, 1, cfg.n_layers)).to("cuda", torch.bfloat16)
+  monkeypatch.setenv("XOT_PACK", mode)
+  model.pack_decode_weights()
+  layer = model.layers["1"]
+  assert layer.mlp.wp_gate_up is None and all(p.weight_packed is None for e in layer.mlp.experts for p in (e.gate_up_proj, e.down_proj))
+  assert (layer.self_attn.o_proj.weight_packed is not None) == (mode == "all")
+  # an expert with a hook has its call, which may read a copy
+  layer.mlp.experts[2].register_forward_hook(lambda *a: None)
+  model.pack_decode_weights()
+  assert layer.mlp.wp_gate_up is not None
+
+
 @pytest.mark.parametrize("T", [257, 300, 500])
 def test_prompts_beside_fp8_copies(T, monkeypatch):
   """Copies for decode leave prompts to the grouped products, which read the weights themselves."""

@@ -773,13 +773,13 @@ class ShardedModel(nn.Module):
     do not read as they lie (MoEMLP._expert_weights) - down_proj, lm_head, gate_up, then
     qkv/o - greedily while at least `reserve_bytes` of HBM stay free (KV caches and
     activations are usually allocated before this is called). Returns bytes packed.
-    XOT_PACK=none packs nothing, all whatever can be packed."""
+    XOT_PACK=none packs nothing, all whatever can be packed and is read."""
     mode = os.getenv("XOT_PACK", "auto")
     if mode == "none" or not torch.cuda.is_available():
       return 0
     groups: List[List[XotLinear]] = [[], [], [], []]
     unread = set()  # experts whose copies nothing would read
-    if mode != "all" and not ops.fp8_gemm_enabled():
+    if not ops.fp8_gemm_enabled():
       unread = {id(p) for m in self.modules() if isinstance(m, MoEMLP) and m._expert_weights() is not None
                 for e in m.experts for p in (e.gate_up_proj, e.down_proj)}
     for name, mod in self.named_modules():
