@@ -245,7 +245,11 @@ def test_products_that_later_tiles_gained():
   from xotorch_amd.ops.train_ops import forward_gains, input_gains
   for M, N, K, own in [(64, 8192, 8064, False), (65, 8192, 8064, True), (1000, 8192, 8064, True), (1001, 8192, 8064, False),
                        (2000, 6144, 8064, True), (2001, 6144, 8064, False),
-                       (1100, 8192, 28672, True), (1101, 8192, 28672, False), (1541, 8192, 28672, True), (1791, 8192, 28672, False),
+                       (1100, 8192, 28672, True), (1101, 8192, 28672, False), (1541, 8192, 28672, True), (1793, 8192, 28672, False),
+                       # as blocks of 256 rows by 224 tokens fill rounds, whatever the width
+                       (1344, 8192, 28672, False), (1345, 8192, 28672, True), (1792, 8192, 28672, True), (1600, 6400, 20480, False), (1793, 6400, 20480, True),
+                       (1344, 9216, 24576, False), (1345, 9216, 24576, True), (1569, 9216, 24576, False), (1568, 7168, 18432, False), (1569, 7168, 18432, True),
+                       (1300, 12288, 28672, True), (2000, 16384, 53248, True), (2001, 16384, 53248, False), (1001, 12288, 16384, False),
                        (8192, 5120, 17408, True), (8193, 5120, 17408, False),
                        (8192, 8192, 28672, False), (1000, 2048, 3072, False), (1001, 2048, 3072, True), (8192, 2048, 3072, True), (128, 28672, 4096, False),
                        (129, 28672, 4096, True), (2000, 28672, 4096, True), (2001, 28672, 4096, False), (100, 6144, 4096, True), (100, 16384, 2048, False),

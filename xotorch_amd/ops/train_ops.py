@@ -185,8 +185,14 @@ def forward_gains(M: int, N: int, K: int) -> bool:
   if K > 8000:
     if N <= 6144:
       return M <= 2000 or K > 16384
-    # [8192, 28672] to 1100 tokens 0.62, to 1540 0.66 to 1.14 (1.0), to 1790 0.79, more 1.05: as blocks fill rounds
-    return M <= 1000 or K > 16384 and (M <= 1100 or 1540 < M <= 1790)
+    if M <= 1000 or K <= 16384:
+      return M <= 1000
+    # the longest sums, 1001 to 2000 tokens by eight weights of 6400 to 28672 rows: from 10000 rows on 0.59
+    # to 1.08 (0.81); fewer rows and up to 1100 tokens 0.57 to 1.13 (0.75), then where blocks of 256 rows by
+    # 224 tokens leave up to an eighth of their rounds empty 0.59 to 1.01 (0.80), and 0.53 to 1.16 (0.89)
+    # where they leave more
+    blocks = -(-N // 256) * -(-M // 224)
+    return M <= 1100 or M <= 2000 and (N > 10000 or blocks >= 224 * -(-blocks // 256))
   return 1000 < M if N * K <= 7_000_000 else M <= 2000 and (M > 128 or K > 3200 and N <= 20000)
 
 
