@@ -206,16 +206,23 @@ static const Tile COLUMN_TILES[] = {{256, 256, 1.42, 11}, {128, 256, 0.8, 7.5}, 
 struct Choice {
   int tile, splits;
 };
+// At every call, and passes of few tokens wait for the host: what all tiles share is made once, and nothing
+// divides where they are compared: 0.32 us of [2048, 8192], 0.77 with divisions.
 static Choice choose(const Costs& of, int64_t M, int64_t N, int steps) {
+  double sum[16], way[16];  // by parts: steps of one, and the parts' way out and in
+  int most = 0;
+  for (int s = 1; s <= 16 && (s == 1 || (steps >= 4 * s && M * N * s <= 1 << 27)); ++s, ++most) {
+    sum[most] = (unsigned)(steps + s - 1) / (unsigned)s;
+    way[most] = s > 1 ? M * N * 8.0 * s / of.bytes_us + of.parts : 0;
+  }
   Choice best{0, 1};
   double least = 1e30;
   for (int t = 0; t < of.count; ++t) {
     const Tile& tile = of.tiles[t];
-    const int64_t blocks = (N + tile.bn - 1) / tile.bn * ((M + tile.bm - 1) / tile.bm);
-    for (int s = 1; s <= 16 && (s == 1 || (steps / s >= 4 && M * N * s <= 1 << 27)); ++s) {
-      const int64_t rounds = (blocks * s + 255) / 256;
-      const double us = rounds * ((steps + s - 1) / s * tile.step + tile.ends) + (s > 1 ? M * N * 8.0 * s / of.bytes_us + of.parts : 0);
-      if (us < least) least = us, best = {t, s};
+    const int64_t blocks = (int64_t)((unsigned)(N + tile.bn - 1) / (unsigned)tile.bn) * ((unsigned)(M + tile.bm - 1) / (unsigned)tile.bm);
+    for (int i = 0; i < most; ++i) {
+      const double us = (double)((blocks * (i + 1) + 255) >> 8) * (sum[i] * tile.step + tile.ends) + way[i];
+      if (us < least) least = us, best = {t, i + 1};
     }
   }
   return best;
