@@ -1,4 +1,6 @@
 """Which calls go to the kernels: those that can read their operands and that nobody follows."""
+import random
+
 import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
@@ -139,6 +141,21 @@ def test_the_rules_know_how_k_of_gates_is_split():
   for N in (16, 1024, 10176, 10192, 16384, 16400, 20416, 20480, 20496, 28672, 1 << 26):
     for K in (64, 1024, 1088, 2048, 2112, 6144, 6208, 53248):
       assert ops.gate_splits(N, K) == ops._tile().gate_splits(N, K)
+
+
+def test_rules_and_kernels_split_alike():
+  """What Python's rules write out of the kernels', over all that these tell apart: parts of two blocks a CU, blocks that
+  begin at different places of k, a round of small weights."""
+  hip = pytest.importorskip("xotorch_amd.ops._hip_tile")
+  from xotorch_amd import ops
+  rng = random.Random(5)
+  sizes = {(N, K) for N in (2112, 3584, 4090, 4096, 4608, 8192, 11008, 16384, 28672, 53248)
+           for K in (2048, 4096, 5696, 6144, 8192, 9600, 11008, 12288, 14336, 16384, 18432, 18944, 28672, 28736, 53248)}
+  sizes |= {(round(2 ** rng.uniform(0, 18)), 64 * round(2 ** rng.uniform(0, 10))) for _ in range(20000)}
+  for N, K in sizes:
+    assert ops.tile_splits(N, K) == hip.tile_splits(N, K), (N, K)
+    assert ops.gate_splits(N, K) == hip.gate_splits(N, K), (N, K)
+  assert len({hip.gate_splits(N, K) for N, K in sizes}) >= 12
 
 
 @pytest.mark.gpu
