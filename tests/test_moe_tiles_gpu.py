@@ -17,7 +17,7 @@ def test_prompt_by_tiles(T, E, k, D, I):
     for p in moe.parameters():
       p.copy_(torch.randn(p.shape, generator=g, device="cuda") * p.shape[-1] ** -0.5)
     moe.gate.weight.mul_(4)  # decided choices: the best of the rest is rarely within rounding
-    assert moe._by_tiles(x[0])
+    assert moe._grouped(x[0]) is not None and moe._many(x[0])
     out = moe(x)[0].double()
     xd = x[0].double()
     logits = xd @ moe.gate.weight.double().t()
@@ -296,7 +296,7 @@ def test_few_tokens_through_experts(T, E, k, D, I):
     for p in moe.parameters():
       p.copy_(torch.randn(p.shape, generator=g, device="cuda") * p.shape[-1] ** -0.5)
     moe.gate.weight.mul_(4)
-    assert moe._grouped(x) is not None and not moe._by_tiles(x)
+    assert moe._grouped(x) is not None and not moe._many(x)
     out, wide = moe(x[None])[0], moe._forward_decode(x, True)
     assert wide.dtype == torch.float32 and torch.equal(wide.to(torch.bfloat16), out)
     xd = x.double()

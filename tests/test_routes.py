@@ -36,7 +36,7 @@ def test_fake_tensors_are_not_read_by_linears():
       x = torch.empty(rows, 64, dtype=BF)
       assert not ops.few_rows(x, lin.weight) and not ops.tile_rows(x, lin.weight)
       assert lin(x).shape == (rows, 128)
-    assert not moe._by_tiles(torch.empty(300, 64, dtype=BF))
+    assert moe._grouped(torch.empty(300, 64, dtype=BF)) is None and moe._grouped(torch.empty(3, 64, dtype=BF)) is None
 
 
 def test_products_go_where_they_are_faster():

@@ -473,14 +473,11 @@ class MoEMLP(nn.Module):
       out.index_add_(0, token_idx, expert_out * weights[token_idx, k_idx, None])
     return out.view(B, S, D).to(x.dtype)
 
-  def _by_tiles(self, flat) -> bool:
+  def _many(self, flat) -> bool:
     """Whether the grouped products go by tiles of 128 and 256 tokens: over 24 rows
     per expert (fewer leave most of a tile of 128 tokens empty), up to 256 tokens over 48: 8 experts
     of 4096 x 14336, two of them a token, us by tiles of up to 64 rows and by these: 128 tokens 460, 508;
     192 467, 516; 256 738, 563."""
-    return self._many(flat) and self._grouped(flat) is not None
-
-  def _many(self, flat) -> bool:
     return flat.shape[0] * self.top_k > (24 if flat.shape[0] > 256 else 48) * self.n_experts
 
   def _expert_weights(self):
