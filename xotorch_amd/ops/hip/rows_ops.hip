@@ -292,6 +292,9 @@ __global__ __launch_bounds__(256) void rows_kernel(RowsArgs a) {
     group(A, B);
     return;
   }
+  // Waves that share k may have one an odd and one an even number of chunks, and then wait in different copies of
+  // `group` for one another. The hardware's barrier counts a block's waves wherever they are, and each comes by
+  // two of them a row group, of which all waves of a block have as many (g - wave / KS is the block's).
   while (g - wave / KS < a.groups) {
     group(A, B);
     if (n % 2 == 0 || g - wave / KS >= a.groups) continue;
