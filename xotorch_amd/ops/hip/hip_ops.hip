@@ -902,9 +902,10 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
 // cycles, other instructions take 5, exponentials 9. So the scale is part of the exponents'
 // multiply-add, a maximum one instruction (`larger`), and what never changes stays in
 // registers. us, with 8 + 8 instructions for those, 11 for 8 numbers' maximum and 3 moves a
-// tile, and so: 6001 tokens, 32 heads on 8 327, 310 (952 TFLOP/s); 16 x 512, 64 on 8 134, 129;
-// 2000 tokens, 32 heads of 64 on 8 43, 40. (32 x 32 x 16, which hold the port half as long, take
-// more power: 324, 139 and 40.)
+// tile, and so: 6001 tokens, 32 heads on 8 322, 307 (960 TFLOP/s); 16 x 512, 64 on 8 139, 137;
+// 2000 tokens, 32 heads of 64 on 8 46, 43; behind three gated products of 6001 tokens, as a pass
+// has it, whose power the clock has given way to, 378, 357 (830 TFLOP/s); 153, 149; 52, 48. (32 x
+// 32 x 16, which hold the port half as long, take more power: up to 8% slower.)
 // ---------------------------------------------------------------------------
 
 DEVINL floatx4 mma16(const bf16x8& a, const bf16x8& b, floatx4 c) {
