@@ -371,7 +371,7 @@ def test_prompts_beside_fp8_copies(T, monkeypatch):
 
 
 @pytest.mark.parametrize("T", [1, 40, 256])
-@pytest.mark.parametrize("who", ["hook", "global hook", "autocast", "dispatch mode", "module of its own"])
+@pytest.mark.parametrize("who", ["hook", "global hook", "autocast", "dispatch mode", "module of its own", "bias"])
 def test_experts_of_a_router_with_its_own_call(T, who):
   """A router that somebody waits for is called, and its experts still go as two grouped products: the same numbers, as
   whole ones are summed and rounded alike by either way. More tokens have all modules called."""
@@ -397,6 +397,24 @@ def test_experts_of_a_router_with_its_own_call(T, who):
       p.copy_(torch.randn(p.shape, generator=g, device="cuda") * p.shape[-1] ** -0.5)
     moe.gate.weight.copy_(make(E))  # logits are whole numbers of up to 128
     want, many = moe(x[None]), moe(more[None])
+    if who == "bias":  # whole numbers too, which the experts' call has to see
+      from torch.nn.functional import linear
+      bias = torch.randint(-9, 10, (E,), generator=g, device="cuda").to(torch.bfloat16)
+      direct = moe.gate.weight
+      moe.gate = torch.nn.Linear(D, E, device="cuda", dtype=torch.bfloat16)
+      moe.gate.weight, moe.gate.bias = direct, torch.nn.Parameter(bias)
+      found = moe._grouped(x)
+      assert found is not None and found[2] is None and moe._grouped(more) is None
+      w, chosen = linear(x.double(), direct.double(), bias.double()).softmax(-1).topk(k)
+      w, ref = w / w.sum(-1, keepdim=True), torch.zeros(T, D, dtype=torch.float64, device="cuda")
+      for e in range(E):
+        token, place = torch.where(chosen == e)
+        gate, up = (x.double()[token] @ moe.experts[e].gate_up_proj.weight.double().t()).chunk(2, -1)
+        h = torch.nn.functional.silu(gate) * up
+        ref.index_add_(0, token, h @ moe.experts[e].down_proj.weight.double().t() * w[token, place, None])
+      off = (moe(x[None])[0].double() - ref).norm(dim=-1) / ref.norm(dim=-1)
+      assert float(off.median()) < 1e-2  # tokens with equal logits may choose otherwise
+      return
     if who == "module of its own":
       router = Router(D, E, bias=False)
       router.weight = moe.gate.weight

@@ -506,8 +506,8 @@ class MoEMLP(nn.Module):
   def _grouped(self, flat):
     """The experts' weights where tokens go through them as two grouped products, and the router's where
     its logits are made with the choice; or None. Up to 256 tokens a router that somebody waits for, by a hook of
-    its own or a global one, that is another module or that autocast or a dispatch mode takes, has its own call and the
-    experts none: us of a layer with 1 and 32 tokens, expert by expert and so, 8 experts of 4096 x 14336 580, 155 and
+    its own or a global one, that is another module or has a bias, or that autocast or a dispatch mode takes, has its own
+    call and the experts none: us of a layer with 1 and 32 tokens, expert by expert and so, 8 experts of 4096 x 14336 580, 155 and
     570, 444; 128 of 2048 x 768 4510, 148 and 4535, 203. More tokens go by the modules then."""
     few = flat.shape[0] <= 256
     if flat.dtype != torch.bfloat16 or not flat.is_cuda or not flat.is_contiguous() or not flat.numel():
@@ -519,7 +519,7 @@ class MoEMLP(nn.Module):
     if found is None:
       return None
     gate = self._modules["gate"]
-    alone = type(gate) is nn.Linear and not _watched(gate) and ops.alone(flat)
+    alone = type(gate) is nn.Linear and _own(gate, "bias") is None and not _watched(gate) and ops.alone(flat)
     if not alone and (not few or train_ops.followed() or type(flat) not in train_ops.OWN):
       return None
     weights = [*found[0], *found[1]]
