@@ -141,7 +141,8 @@ _WIDEST = 57344  # of what was measured with tiles of 64 to 224 rows of x
 
 
 def forward_wins(M: int, N: int, K: int) -> bool:
-  """x W^T: narrow results of up to 1000 tokens 0.34 to 1.26 (0.77 on average) for rows of 3072
+  """x W^T; the kernels have what this or forward_gains is true for (gradients of inputs: input_wins or
+  input_gains). Narrow results of up to 1000 tokens 0.34 to 1.26 (0.77 on average) for rows of 3072
   and more, 0.74 to 1.38 (0.94) for shorter ones (0.76 to 1.65, 1.19, from 65 tokens on before
   there were tiles of 64). By tiles of 128 and 256 alone: wider results and more tokens 0.95 to 1.40, but for long sums, whose library tiles
   fill the chip badly (257 to 2000 tokens by 1536 to 12288 features of 13824 to 29568): where
